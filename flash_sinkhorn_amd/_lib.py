@@ -69,6 +69,9 @@ _SIGNATURES = {
     "fs_apply_mat": (ctypes.c_int, [_P] * 9 + [_I] * 4 + [_F] * 2 + [ctypes.c_int] + _TAIL),
     "fs_mat5": (ctypes.c_int, [_P] * 8 + [_I] * 3 + [_F] * 2 + _TAIL),
     "fs_c_transform": (ctypes.c_int, [_P] * 5 + [_I] * 3 + [_F] + _TAIL),
+    "fs_small_workspace_bytes": (_Z, [_P]),
+    "fs_small_solve": (ctypes.c_int, [_P, _P, _Z, _P, _P, _P, _P]),
+    "fs_small_grad": (ctypes.c_int, [_P, _P, _Z, _P, _P, _P, _P]),
 }
 EXPORTED_SYMBOLS = tuple(_SIGNATURES)
 

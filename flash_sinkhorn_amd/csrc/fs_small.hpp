@@ -1,0 +1,707 @@
+// Whole solves of small problems, one launch per step (d <= 128, fp16 planes).
+//
+// A small solve is bound by launches, not by arithmetic: at 2000 x 2000 x 3 a step of the xy
+// problem and of the two self problems of a debiased loss is a few microseconds of work, and a
+// launch costs about 3 us on the host and 2 us on the device whatever it does.  So this family
+// spends one launch per step on ALL problems of a loss (the xy pair and the two self problems, for
+// every item of a batch): a workgroup owns 32 query rows of one half-update and ALL their keys, its
+// wavefronts share the keys, merge their soft-max statistics in LDS and run the epilogue, so
+// nothing is left to a merge launch and nothing is written but the new potentials.  What used
+// to be dozens of small launches around the steps (norms, log weights, bounding boxes, plane
+// conversion, the eps schedule, the loss) is one statistics launch and one preparation launch in
+// front and one launch behind.
+//
+// The planes are kept in MFMA operand order only (per 32 rows, plane and 16-column step one
+// 1 KiB block with lane (h, row % 32)'s 16 bytes at 16 * (32 h + row % 32)): the same block
+// serves as the stationary and as the streamed operand, a wavefront reads it with one fully
+// coalesced load, and at these sizes every read hits the L2.
+//
+#pragma once
+
+#include "fs_common.hpp"
+
+namespace fs {
+
+constexpr int kSmallStatBlocks = 16;            // workgroups per matrix and item of small_stats_kernel
+constexpr int kSmallMaxD = 128;
+constexpr int kSmallStatWords = 2 + 2 * kSmallMaxD;  // absmax, weight sum, column minima, column maxima
+constexpr int kSmallTable = 512;                // longest eps schedule kept on the device
+
+// A run of small problems.  Sides: 0 f of the xy problem (rows of x against keys y), 1 g of it
+// (rows of y against keys x), 2 the self problem of x, 3 that of y.  Problems: 0 xy, 1 xx, 2 yy.
+struct SmallArgs {
+  const void* pts[2];     // x [items, n, d], y [items, m, d]
+  const float* w[2];      // weights [items, rows], null: uniform
+  int dtype;              // 0 fp32, 1 fp16, 2 bf16
+  int normalize;          // divide the weights by their sum
+  int rows[2], blocks[2];  // rows of x and y, 32-row blocks of them
+  int d, items;
+  int self;               // 1: the self problems are solved as well, 2: only they are
+  int want_values;        // value operands for small_grad_kernel are written
+  float cost_scale;
+  // eps schedule: 0 eps0 in every entry, 1 from the diameter of the clouds, 2 the table as given
+  int sched, entries, cut, extrapolate;
+  float eps0;
+  double blur, scaling;
+  float rho[2];           // <= 0: strict marginal
+  // workspace
+  float* stats;           // [items][2][kSmallStatBlocks][kSmallStatWords]
+  float* scale;           // [items][2] power-of-two scales of the planes
+  u32x4* planes[2];       // [items][blocks][2 planes][DP / 16][64]
+  u32x4* values[2];       // [items][blocks][DP / 32][2 steps][2 planes][64]
+  float* norm[2];         // [items][rows] cost_scale * |row|^2
+  float* wt[2];           // [items][rows] weights as the solve takes them
+  float* l2w[2];          // [items][rows] their base-2 logarithms
+  float* pot[4];          // [2 parities][items][rows of the side]: shifted potentials
+  float* table;           // [items][3][kSmallTable] eps of every entry
+  int* full;              // [items][3] entries of the schedules
+  int* lens;              // [items][3] those the problem runs: fewer once it has converged
+  int* host_words;        // pinned host memory, 4 words per item (see small_schedule, small_check_kernel)
+  int host_token;
+  // early stopping (threshold > 0): the potentials of the last check
+  float threshold;
+  float* prev[4];         // [items][rows of the side]
+};
+
+__device__ __forceinline__ float small_load(const void* p, size_t i, int dtype) {
+  if (dtype == 0) return static_cast<const float*>(p)[i];
+  if (dtype == 1) return (float)static_cast<const _Float16*>(p)[i];
+  return __builtin_bit_cast(float, (unsigned)static_cast<const unsigned short*>(p)[i] << 16);
+}
+
+// Entries of a problem's schedule, the number of its steps, and the eps and weight of step s
+// (the first full step at entry 0, an averaged step per entry, one full step at the last entry).
+__device__ __forceinline__ int small_entries(const SmallArgs& a, int item, int prob) {
+  return a.sched == 0 && !(a.threshold > 0.f) ? a.entries : a.lens[item * 3 + prob];
+}
+__device__ __forceinline__ int small_full_entries(const SmallArgs& a, int item, int prob) {
+  return a.sched == 0 ? a.entries : a.full[item * 3 + prob];
+}
+__device__ __forceinline__ float small_eps(const SmallArgs& a, int item, int prob, int idx) {
+  return a.sched == 0 ? a.eps0 : a.table[((size_t)item * 3 + prob) * kSmallTable + idx];
+}
+
+// Partial statistics of a slice of one matrix of one item: largest magnitude (the plane scale),
+// sum of the weights, and per column the smallest and largest value (the bounding box behind a
+// schedule by diameter).  A thread stays on one column.
+template <int T>
+__global__ __launch_bounds__(256) void small_stats_kernel(const SmallArgs a) {
+  const int mat = blockIdx.y, item = blockIdx.z, tid = threadIdx.x;
+  const int rows = a.rows[mat], d = a.d;
+  const int per = (rows + kSmallStatBlocks - 1) / kSmallStatBlocks;
+  const int r0 = min(rows, (int)blockIdx.x * per), r1 = min(rows, r0 + per);
+  const int reps = 256 / d, act = reps * d;
+  __shared__ float mn[256], mx[256];
+  float lo = 3.0e38f, hi = -3.0e38f, ws = 0.f;
+  bool nan = false;
+  if (tid < act) {
+    const size_t base = (size_t)item * rows * d;
+    for (size_t e = (size_t)r0 * d + tid; e < (size_t)r1 * d; e += act) {
+      const float v = small_load(a.pts[mat], base + e, a.dtype);
+      lo = fminf(lo, v);
+      hi = fmaxf(hi, v);
+      nan = nan || !(v == v);
+    }
+  }
+  if (a.w[mat] != nullptr && a.normalize)
+    for (int r = r0 + tid; r < r1; r += 256) ws += a.w[mat][(size_t)item * rows + r];
+  if (nan) lo = hi = __builtin_nanf("");
+  mn[tid] = lo;
+  mx[tid] = hi;
+  for (int k = reps; k > 1;) {  // columns repeat every d threads: halve the number of repeats
+    const int half = (k + 1) / 2;
+    __syncthreads();
+    if (tid < (k - half) * d) {
+      const float l = mn[tid + half * d], u = mx[tid + half * d];
+      mn[tid] = (l < mn[tid] || !(l == l)) ? l : mn[tid];
+      mx[tid] = (u > mx[tid] || !(u == u)) ? u : mx[tid];
+    }
+    k = half;
+  }
+  __syncthreads();
+  float* out = a.stats + (((size_t)item * 2 + mat) * kSmallStatBlocks + blockIdx.x) * kSmallStatWords;
+  if (tid < d) {
+    out[2 + tid] = mn[tid];
+    out[2 + kSmallMaxD + tid] = mx[tid];
+  }
+  __syncthreads();
+  // (a NaN does not reach the plane scale: fmaxf drops it, as absmax_kernel does)
+  float am = (r1 > r0 && tid < d) ? fmaxf(fabsf(mn[tid]), fabsf(mx[tid])) : 0.f;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    am = fmaxf(am, __shfl_xor(am, o, 64));
+    ws += __shfl_xor(ws, o, 64);
+  }
+  __syncthreads();
+  if ((tid & 63) == 0) {
+    mn[tid >> 6] = am;
+    mx[tid >> 6] = ws;
+  }
+  __syncthreads();
+  if (tid == 0) {
+    out[0] = fmaxf(fmaxf(mn[0], mn[1]), fmaxf(mn[2], mn[3]));
+    out[1] = (mx[0] + mx[1]) + (mx[2] + mx[3]);
+  }
+}
+
+// The schedules of one item from its bounding boxes (numpy's arange and exp in double, as the
+// host builds it for larger problems): [D^2] + exp(2 ln D + i * 2 ln scaling) while above blur^2
+// + [blur^2].  By one workgroup; diameters of the union, of x and of y.
+__device__ void small_schedule(const SmallArgs& a, int item) {
+  const int tid = threadIdx.x;
+  __shared__ float sq[3];
+  __shared__ int len[3];
+  if (a.sched == 0 && a.threshold > 0.f && tid < 3) a.lens[item * 3 + tid] = a.entries;
+  if (a.sched != 1) return;
+  if (tid < 3) sq[tid] = 0.f;
+  __syncthreads();
+  float r[3] = {0.f, 0.f, 0.f};
+  if (tid < a.d) {
+    float lo[2] = {3.0e38f, 3.0e38f}, hi[2] = {-3.0e38f, -3.0e38f};
+    for (int mat = 0; mat < 2; ++mat)
+      for (int b = 0; b < kSmallStatBlocks; ++b) {
+        const float* st = a.stats + (((size_t)item * 2 + mat) * kSmallStatBlocks + b) * kSmallStatWords;
+        const float l = st[2 + tid], u = st[2 + kSmallMaxD + tid];
+        lo[mat] = (l < lo[mat] || !(l == l)) ? l : lo[mat];
+        hi[mat] = (u > hi[mat] || !(u == u)) ? u : hi[mat];
+      }
+    const float e0 = (lo[0] < lo[1] || !(lo[0] == lo[0]) ? lo[0] : lo[1]);
+    const float e1 = (hi[0] > hi[1] || !(hi[0] == hi[0]) ? hi[0] : hi[1]);
+    r[0] = e1 - e0;
+    r[1] = hi[0] - lo[0];
+    r[2] = hi[1] - lo[1];
+  }
+#pragma unroll
+  for (int p = 0; p < 3; ++p) {
+    float s = r[p] * r[p];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+    if ((tid & 63) == 0 && tid < 128) atomicAdd(&sq[p], s);
+  }
+  __syncthreads();
+  if (tid < 3) {
+    const double D = (double)sqrtf(sq[tid]);
+    int k = -2;                      // not a number
+    if (D <= 0.0) k = -1;            // one point
+    else if (D < 3.0e38) {
+      const double start = 2.0 * log(D), stop = 2.0 * log(a.blur), step = 2.0 * log(a.scaling);
+      const double cnt = ceil((stop - start) / step);
+      const double total = 2.0 + (cnt > 0.0 ? cnt : 0.0);
+      k = total > (double)kSmallTable ? -3 : (int)total;  // -3: longer than the table
+      if (k > 0 && a.cut > 0) k = min(k, a.cut);
+    }
+    len[tid] = k;
+    a.lens[item * 3 + tid] = k;
+    a.full[item * 3 + tid] = k;
+    __hip_atomic_store(a.host_words + item * 4 + tid, k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+  __syncthreads();
+  if (tid == 0) {  // (the same wavefront wrote the three words)
+    __threadfence_system();
+    __hip_atomic_store(a.host_words + item * 4 + 3, a.host_token, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+  for (int p = 0; p < 3; ++p) {
+    const double D = (double)sqrtf(sq[p]);
+    if (len[p] <= 0) continue;
+    const double start = 2.0 * log(D), stop = 2.0 * log(a.blur), step = 2.0 * log(a.scaling);
+    const double cnt = ceil((stop - start) / step);
+    const int full = 2 + (cnt > 0.0 ? (int)cnt : 0);
+    for (int i = tid; i < len[p]; i += 256) {
+      const double e = i == 0 ? D * D : (i == full - 1 ? a.blur * a.blur : exp(start + (i - 1) * step));
+      a.table[((size_t)item * 3 + p) * kSmallTable + i] = (float)e;
+    }
+  }
+}
+
+// Everything the steps read, from one block of 32 rows: planes and (with want_values) value operands
+// in MFMA order, cost_scale * |row|^2, base-2 log weights and the initial potentials.  The last
+// workgroup column (x = blocks of the larger matrix) writes the schedules.
+template <int DP>
+__global__ __launch_bounds__(256) void small_prep_kernel(const SmallArgs a) {
+  constexpr int KK = DP / 16, NDB = (DP + 31) / 32, LDW = NDB * 32 + 1;
+  const int mat = blockIdx.y, item = blockIdx.z, tid = threadIdx.x;
+  if ((int)blockIdx.x == gridDim.x - 1) {
+    if (mat == 0) small_schedule(a, item);
+    return;
+  }
+  const int rb = blockIdx.x, rows = a.rows[mat], d = a.d;
+  if (rb >= a.blocks[mat]) return;
+  __shared__ float s[32 * LDW];
+  const float* st = a.stats + ((size_t)item * 2 + mat) * kSmallStatBlocks * kSmallStatWords;
+  float am = 0.f, ws = 0.f;
+#pragma unroll
+  for (int b = 0; b < kSmallStatBlocks; ++b) {
+    am = fmaxf(am, st[b * kSmallStatWords]);
+    ws += st[b * kSmallStatWords + 1];
+  }
+  const float sc = f16_plane_scale(am);
+  if (rb == 0 && tid == 0) a.scale[item * 2 + mat] = sc;
+  const int r0 = rb * 32;
+  if (d < NDB * 32)
+    for (int e = tid; e < 32 * LDW; e += 256) s[e] = 0.f;
+  __syncthreads();
+  const size_t base = ((size_t)item * rows + r0) * d;
+  for (int e = tid; e < 32 * d; e += 256) {
+    const int r = e / d;
+    s[r * LDW + (e - r * d)] = r0 + r < rows ? sc * small_load(a.pts[mat], base + e, a.dtype) : 0.f;
+  }
+  __syncthreads();
+  // planes
+  u32x4* po = a.planes[mat] + ((size_t)item * a.blocks[mat] + rb) * (2 * KK * 64);
+  for (int e = tid; e < KK * 64; e += 256) {
+    const int kk = e >> 6, lane = e & 63;
+    const float* v = s + (lane & 31) * LDW + 16 * kk + 8 * (lane >> 5);
+    u32x4 hi, lo;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const float v0 = v[2 * q], v1 = v[2 * q + 1];
+      const _Float16 h0 = (_Float16)v0, h1 = (_Float16)v1;
+      hi[q] = pack_f16((float)h0, (float)h1);
+      lo[q] = pack_f16(v0 - (float)h0, v1 - (float)h1);
+    }
+    po[kk * 64 + lane] = hi;
+    po[(KK + kk) * 64 + lane] = lo;
+  }
+  if (a.want_values) {
+    // lane (li, h), slot i of step t: key 16 t + (i < 4 ? 4 h + i : 4 + 4 h + i), the order in which
+    // the accumulator of a logits tile holds the keys; column 32 cb + li
+    u32x4* vo = a.values[mat] + ((size_t)item * a.blocks[mat] + rb) * (NDB * 2 * 2 * 64);
+    for (int e = tid; e < NDB * 2 * 64; e += 256) {
+      const int lane = e & 63, t = (e >> 6) & 1, cb = e >> 7;
+      const int h = lane >> 5, col = 32 * cb + (lane & 31);
+      u32x4 hi, lo;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int key = 16 * t + 4 * h + (q < 2 ? 2 * q : 4 + 2 * q);
+        const float v0 = s[key * LDW + col], v1 = s[(key + 1) * LDW + col];
+        const _Float16 h0 = (_Float16)v0, h1 = (_Float16)v1;
+        hi[q] = pack_f16((float)h0, (float)h1);
+        lo[q] = pack_f16(v0 - (float)h0, v1 - (float)h1);
+      }
+      vo[((cb * 2 + t) * 2 + 0) * 64 + lane] = hi;
+      vo[((cb * 2 + t) * 2 + 1) * 64 + lane] = lo;
+    }
+  }
+  // norms: eight threads a row
+  {
+    const int r = tid >> 3, c = tid & 7;
+    float q = 0.f;
+    for (int k = c; k < d; k += 8) q = __builtin_fmaf(s[r * LDW + k], s[r * LDW + k], q);
+    q += __shfl_xor(q, 1, 64);
+    q += __shfl_xor(q, 2, 64);
+    q += __shfl_xor(q, 4, 64);
+    const int row = r0 + r;
+    if (c == 0 && row < rows) {
+      const float inv = 1.0f / sc;
+      const float al = a.cost_scale * (q * inv * inv);
+      const size_t at = (size_t)item * rows + row;
+      a.norm[mat][at] = al;
+      float w = a.w[mat] == nullptr ? 1.0f / (float)rows : a.w[mat][at];
+      if (a.w[mat] != nullptr && a.normalize) w = w / fmaxf(ws, 1e-40f);
+      a.wt[mat][at] = w;
+      a.l2w[mat][at] = w > 0.f ? kLog2e * logf(w) : -100000.0f * kLog2e;
+      a.pot[mat][at] = -al;
+      if (a.self) a.pot[2 + mat][at] = -al;
+    }
+  }
+}
+
+// What a workgroup of the steps (and of the gradient) works on.
+struct SmallSide {
+  int side, rb, qm, km, prob;  // query and key matrix
+};
+
+__device__ __forceinline__ SmallSide small_side(const SmallArgs& a, int bid) {
+  SmallSide s;
+  s.side = 0;
+  if (a.self == 2) bid += a.blocks[0] + a.blocks[1];
+  if (bid >= a.blocks[0] + a.blocks[1]) {
+    bid -= a.blocks[0] + a.blocks[1];
+    s.side = 2;
+  }
+  if (bid >= a.blocks[0]) {
+    bid -= a.blocks[0];
+    s.side += 1;
+  }
+  s.rb = bid;
+  s.qm = s.side & 1;
+  s.km = s.side < 2 ? s.qm ^ 1 : s.qm;
+  s.prob = s.side < 2 ? 0 : s.side - 1;
+  return s;
+}
+
+__device__ __forceinline__ f32x16 small_mfma(const u32x4& x, const u32x4& y, const f32x16& c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, x), __builtin_bit_cast(f16x8, y), c, 0,
+                                                0, 0);
+}
+
+// Keys of one 32-key block: both planes and the base-2 bias of key li (in accumulator units).
+template <int KK>
+struct SmallKeys {
+  u32x4 p[2][KK];
+  float bias;
+};
+
+template <int KK>
+__device__ __forceinline__ void small_load_keys(SmallKeys<KK>& k, const u32x4* kp, const float* pot, const float* l2w,
+                                                float kc, float inv_lscale, float masked, int blk, int nk, int lane) {
+  const u32x4* b = kp + (size_t)blk * (2 * KK * 64) + lane;
+#pragma unroll
+  for (int p = 0; p < 2; ++p)
+#pragma unroll
+    for (int kk = 0; kk < KK; ++kk) k.p[p][kk] = b[(p * KK + kk) * 64];
+  const int j = blk * 32 + (lane & 31);
+  const int jc = min(j, nk - 1);
+  const float v = __builtin_fmaf(kc, pot[jc], l2w[jc]);
+  k.bias = j < nk ? fmaxf(v * inv_lscale, masked) : masked;
+}
+
+// A tile of logits in accumulator units: the three plane products from the lowest weight to
+// hi * hi, then the key bias by one fp32 MFMA.
+template <int KK>
+__device__ __forceinline__ f32x16 small_logits(const SmallKeys<KK>& k, const u32x4 (&q)[2][KK], int h) {
+  f32x16 acc;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+#pragma unroll
+  for (int kk = 0; kk < KK; ++kk) acc = small_mfma(k.p[1][kk], q[0][kk], acc);
+#pragma unroll
+  for (int kk = 0; kk < KK; ++kk) acc = small_mfma(k.p[0][kk], q[1][kk], acc);
+#pragma unroll
+  for (int kk = 0; kk < KK; ++kk) acc = small_mfma(k.p[0][kk], q[0][kk], acc);
+  return __builtin_amdgcn_mfma_f32_32x32x2f32(h ? 0.f : k.bias, h ? 0.f : 1.0f, acc, 0, 0, 0);
+}
+
+__device__ __forceinline__ float small_max16(const f32x16& a) {
+  float m = fmaxf(a[0], a[1]);
+#pragma unroll
+  for (int r = 2; r < 16; r += 2) m = fmaxf(m, fmaxf(a[r], a[r + 1]));
+  return m;
+}
+
+// Bias of a key past the last one, in accumulator units: -1e30 in base 2 where that can be held.
+// A row's maximum starts at half of it: above the masked keys, whose exponentials are then zero
+// (a wavefront may see nothing else), and below every real logit.
+__device__ __forceinline__ float small_masked(float inv_lscale) { return fmaxf(kNegBig * inv_lscale, -3.0e38f); }
+
+// One step of every problem.
+template <int DP, int W>
+__global__ __launch_bounds__(64 * W) void small_step_kernel(const SmallArgs a, int step) {
+  constexpr int KK = DP / 16;
+  const int item = blockIdx.y;
+  const SmallSide sd = small_side(a, blockIdx.x);
+  const int entries = small_entries(a, item, sd.prob);
+  if (step > entries + a.extrapolate) return;  // this problem's schedule is shorter
+  // (a problem that stopped early still extrapolates at the schedule's last eps)
+  const float eps = small_eps(a, item, sd.prob,
+                              step > entries ? small_full_entries(a, item, sd.prob) - 1 : max(step - 1, 0));
+  const float alpha = (step == 0 || step > entries) ? 1.0f : 0.5f;
+  const int nq = a.rows[sd.qm], nk = a.rows[sd.km], nkb = a.blocks[sd.km];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, li = lane & 31, h = lane >> 5;
+  const float lscale = 2.0f * a.cost_scale / eps * kLog2e / (a.scale[item * 2 + sd.qm] * a.scale[item * 2 + sd.km]);
+  const float inv_lscale = 1.0f / lscale, masked = small_masked(inv_lscale), no_max = 0.5f * masked * lscale;
+  const float kc = kLog2e / eps;
+  const int kside = sd.side < 2 ? sd.side ^ 1 : sd.side;
+  const float* kpot = a.pot[kside] + ((size_t)(step & 1) * a.items + item) * nk;
+  const float* kl2w = a.l2w[sd.km] + (size_t)item * nk;
+  const u32x4* kp = a.planes[sd.km] + (size_t)item * nkb * (2 * KK * 64);
+
+  SmallKeys<KK> kr;
+  if (wave < nkb) small_load_keys(kr, kp, kpot, kl2w, kc, inv_lscale, masked, wave, nk, lane);
+  u32x4 q[2][KK];
+  {
+    const u32x4* b = a.planes[sd.qm] + ((size_t)item * a.blocks[sd.qm] + sd.rb) * (2 * KK * 64) + lane;
+#pragma unroll
+    for (int p = 0; p < 2; ++p)
+#pragma unroll
+      for (int kk = 0; kk < KK; ++kk) q[p][kk] = b[(p * KK + kk) * 64];
+  }
+  float m = no_max, s = 0.f;
+  for (int blk = wave; blk < nkb; blk += W) {
+    const f32x16 acc = small_logits(kr, q, h);
+    if (blk + W < nkb) small_load_keys(kr, kp, kpot, kl2w, kc, inv_lscale, masked, blk + W, nk, lane);
+    const float mn = fmaxf(m, small_max16(acc) * lscale);
+    s *= fast_exp2(m - mn);
+    m = mn;
+    float p0 = 0.f, p1 = 0.f;
+#pragma unroll
+    for (int r = 0; r < 16; r += 2) {
+      p0 += fast_exp2(__builtin_fmaf(acc[r], lscale, -m));
+      p1 += fast_exp2(__builtin_fmaf(acc[r + 1], lscale, -m));
+    }
+    s += p0 + p1;
+  }
+  // ---- the row's statistics over the wavefronts and half-waves ----
+  __shared__ float2 sh[W][64];
+  sh[wave][lane] = make_float2(m, s);
+  __syncthreads();
+  const int row = sd.rb * 32 + tid;
+  if (tid >= 32 || row >= nq) return;
+  float M = no_max, S = 0.f;
+#pragma unroll
+  for (int w = 0; w < W; ++w) M = fmaxf(M, fmaxf(sh[w][tid].x, sh[w][tid + 32].x));
+#pragma unroll
+  for (int w = 0; w < W; ++w) {
+    const float2 u = sh[w][tid], v = sh[w][tid + 32];
+    S += u.y * fast_exp2(u.x - M) + v.y * fast_exp2(v.x - M);
+  }
+  const float rho = a.rho[sd.qm];
+  const float damp = rho > 0.f ? 1.0f / (1.0f + eps / rho) : 1.0f;
+  const size_t half = (size_t)a.items * nq, at = (size_t)item * nq + row;
+  float r = alpha * (-eps * damp * kLn2 * (M + log2f(fmaxf(S, 1e-40f))));
+  if (alpha != 1.0f) r += (1.0f - alpha) * a.pot[sd.side][(step & 1) * half + at];
+  if (damp < 1.0f) r -= alpha * (1.0f - damp) * a.norm[sd.qm][at];
+  a.pot[sd.side][((step & 1) ^ 1) * half + at] = r;
+}
+
+// Convergence check behind averaged step `step` (the check_every-th since the last check): a
+// problem none of whose potentials has moved by the threshold since then runs no further entries
+// (its extrapolation, if any, is the next step); the others' potentials are kept for the next
+// check.  The first check only keeps them.  One workgroup per item and problem; it leaves
+// 2 * check + converged in the problem's host word.
+template <int T>
+__global__ __launch_bounds__(1024) void small_check_kernel(const SmallArgs a, int step, int check) {
+  const int prob = blockIdx.x + (a.self == 2 ? 1 : 0), item = blockIdx.y, tid = threadIdx.x;
+  if (a.lens[item * 3 + prob] < step) return;  // stopped before, or a shorter schedule
+  const int s0 = prob == 0 ? 0 : 1 + prob, s1 = prob == 0 ? 1 : s0;
+  float change = 0.f;
+  for (int side = s0; side <= s1; ++side) {
+    const int rows = a.rows[side & 1];
+    const float* now = a.pot[side] + ((size_t)((step & 1) ^ 1) * a.items + item) * rows;
+    float* prev = a.prev[side] + (size_t)item * rows;
+    for (int i = tid; i < rows; i += 1024) {
+      const float d = fabsf(now[i] - prev[i]);
+      change = d > change || !(d == d) ? d : change;
+    }
+  }
+  __shared__ float sh[16];
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    const float d = __shfl_xor(change, o, 64);
+    change = d > change || !(d == d) ? d : change;
+  }
+  if ((tid & 63) == 0) sh[tid >> 6] = change;
+  __syncthreads();
+  bool stop = check > 0;
+  for (int w = 0; w < 16; ++w) stop = stop && sh[w] < a.threshold;
+  if (!stop)
+    for (int side = s0; side <= s1; ++side) {
+      const int rows = a.rows[side & 1];
+      const float* now = a.pot[side] + ((size_t)((step & 1) ^ 1) * a.items + item) * rows;
+      float* prev = a.prev[side] + (size_t)item * rows;
+      for (int i = tid; i < rows; i += 1024) prev[i] = now[i];
+    }
+  if (tid == 0) {
+    if (stop) a.lens[item * 3 + prob] = step;
+    __hip_atomic_store(a.host_words + item * 4 + prob, 2 * check + (stop ? 1 : 0), __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
+
+// The loss of every item, and the standard potentials (of the last step, and of the one before
+// when there was an extrapolation) of every side.  One workgroup per item.
+// pots: per side and kind (0: of the cost, 1: of the gradient) [items][rows], in that order.
+struct SmallLossArgs {
+  float* loss;        // [items] or null
+  float* pots;        // or null
+  int relaxed;        // both marginals relaxed: the other cost formula
+};
+
+template <int T>
+__global__ __launch_bounds__(1024) void small_loss_kernel(const SmallArgs a, const SmallLossArgs l) {
+  const int item = blockIdx.y, part = blockIdx.x, tid = threadIdx.x;
+  float total = 0.f;
+  size_t off = a.self == 2 ? 2 * (size_t)a.items * (a.rows[0] + a.rows[1]) : 0;
+  const int sides = a.self ? 4 : 2;
+  for (int side = a.self == 2 ? 2 : 0; side < sides; ++side) {
+    const int mat = side & 1, rows = a.rows[mat];
+    const int prob = side < 2 ? 0 : side - 1;
+    const int entries = small_entries(a, item, prob), last = entries + 1 + a.extrapolate;
+    const float eps_last = small_eps(a, item, prob, small_full_entries(a, item, prob) - 1);
+    const size_t half = (size_t)a.items * rows;
+    const float rho = a.rho[mat];
+    // (a self problem has this potential twice: its cost is 2 <a, f>)
+    const float sign = side < 2 ? 1.0f : -1.0f;
+    float sum = 0.f;
+    for (int i = part * 1024 + tid; i < rows; i += 1024 * gridDim.x) {
+      const size_t at = (size_t)item * rows + i;
+      const float al = a.norm[mat][at];
+      const float f = a.pot[side][(last & 1) * half + at] + al;
+      if (l.pots != nullptr) {
+        l.pots[off + at] = f;
+        l.pots[off + half + at] = a.extrapolate ? a.pot[side][((last & 1) ^ 1) * half + at] + al : f;
+      }
+      sum += a.wt[mat][at] * (l.relaxed ? 1.0f - expf(-f / rho) : f);
+    }
+    if (l.relaxed) sum *= rho + 0.5f * eps_last;
+    total += sign * sum;
+    off += 2 * half;
+  }
+  if (l.loss == nullptr) return;
+  __shared__ float sh[16];
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) total += __shfl_xor(total, o, 64);
+  if ((tid & 63) == 0) sh[tid >> 6] = total;
+  __syncthreads();
+  if (tid == 0) {
+    float t = 0.f;
+#pragma unroll
+    for (int w = 0; w < 16; ++w) t += sh[w];
+    l.loss[item] = t;
+  }
+}
+
+// Gradients of the loss in x and y at the potentials before the extrapolation.  A workgroup owns
+// 32 rows; with self problems it sweeps the keys of the other cloud, then its own cloud's, and
+// takes the difference of the two barycentres:
+//   xy alone   2 cs gs w_i (q_i - T_i),      with the self terms   2 cs gs w_i (T'_i - T_i).
+struct SmallGradArgs {
+  const float* grad_out;  // [items]
+  float* out[2];          // [items, rows, d] or null
+};
+
+template <int DP>
+__global__ __launch_bounds__(512, 2) void small_grad_kernel(const SmallArgs a, const SmallGradArgs g) {
+  constexpr int KK = DP / 16, NDB = (DP + 31) / 32, W = 8;
+  constexpr int LDW = NDB * 32 + 4;                 // padded row of a wavefront's partial output
+  constexpr int PER = NDB * 32 * 32 / 512;          // outputs per thread
+  __shared__ __attribute__((aligned(16))) float sh_o[W][32 * LDW];
+  __shared__ float2 sh_ms[W][32];
+  const int item = blockIdx.y, tid = threadIdx.x;
+  const int wave = tid >> 6, lane = tid & 63, li = lane & 31, h = lane >> 5;
+  int rb = blockIdx.x, qm = 0;
+  if (g.out[0] == nullptr || rb >= a.blocks[0]) {
+    rb -= g.out[0] == nullptr ? 0 : a.blocks[0];
+    qm = 1;
+  }
+  const int nq = a.rows[qm], d = a.d;
+  u32x4 q[2][KK];
+  {
+    const u32x4* b = a.planes[qm] + ((size_t)item * a.blocks[qm] + rb) * (2 * KK * 64) + lane;
+#pragma unroll
+    for (int p = 0; p < 2; ++p)
+#pragma unroll
+      for (int kk = 0; kk < KK; ++kk) q[p][kk] = b[(p * KK + kk) * 64];
+  }
+  float bary[PER];
+#pragma unroll
+  for (int i = 0; i < PER; ++i) bary[i] = 0.f;
+
+  for (int pass = 0; pass <= a.self; ++pass) {
+    const int km = pass == 0 ? qm ^ 1 : qm;
+    const int kside = pass == 0 ? km : 2 + km;
+    const int prob = pass == 0 ? 0 : 1 + km;
+    const int nk = a.rows[km], nkb = a.blocks[km];
+    const int last = small_entries(a, item, prob) + 1;  // (the step before the extrapolation)
+    const float eps = small_eps(a, item, prob, small_full_entries(a, item, prob) - 1);
+    const float lscale = 2.0f * a.cost_scale / eps * kLog2e / (a.scale[item * 2 + qm] * a.scale[item * 2 + km]);
+    const float inv_lscale = 1.0f / lscale, kc = kLog2e / eps;
+    const float masked = small_masked(inv_lscale), no_max = 0.5f * masked * lscale;
+    const float* kpot = a.pot[kside] + ((size_t)(last & 1) * a.items + item) * nk;
+    const float* kl2w = a.l2w[km] + (size_t)item * nk;
+    const u32x4* kp = a.planes[km] + (size_t)item * nkb * (2 * KK * 64);
+    const u32x4* vp = a.values[km] + (size_t)item * nkb * (NDB * 4 * 64) + lane;
+
+    float m = no_max, s = 0.f;
+    f32x16 o[NDB];
+#pragma unroll
+    for (int cb = 0; cb < NDB; ++cb)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) o[cb][r] = 0.f;
+    SmallKeys<KK> kr;
+    if (wave < nkb) small_load_keys(kr, kp, kpot, kl2w, kc, inv_lscale, masked, wave, nk, lane);
+    for (int blk = wave; blk < nkb; blk += W) {
+      const u32x4* v = vp + (size_t)blk * (NDB * 4 * 64);
+      const f32x16 acc = small_logits(kr, q, h);
+      if (blk + W < nkb) small_load_keys(kr, kp, kpot, kl2w, kc, inv_lscale, masked, blk + W, nk, lane);
+      // the two half-waves of a column feed one sum: they share its maximum
+      float mx = small_max16(acc) * lscale;
+      mx = fmaxf(mx, xor32(mx));
+      if (wave_any(mx > m)) {
+        const float mn = fmaxf(m, mx);
+        const float f = fast_exp2(m - mn);
+        m = mn;
+        s *= f;
+#pragma unroll
+        for (int cb = 0; cb < NDB; ++cb)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) o[cb][r] *= f;
+      }
+      // probabilities times 2^11, as two fp16 planes in the order of the value operands' keys
+      u32x4 ph[2], pl[2];
+      float ps = 0.f;
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          const int r = 8 * t + 2 * c;
+          const float e0 = fast_exp2(__builtin_fmaf(acc[r], lscale, 11.0f - m));
+          const float e1 = fast_exp2(__builtin_fmaf(acc[r + 1], lscale, 11.0f - m));
+          ps += e0 + e1;
+          const _Float16 h0 = (_Float16)e0, h1 = (_Float16)e1;
+          ph[t][c] = pack_f16((float)h0, (float)h1);
+          pl[t][c] = pack_f16(e0 - (float)h0, e1 - (float)h1);
+        }
+      s += ps;
+#pragma unroll
+      for (int cb = 0; cb < NDB; ++cb) {
+        u32x4 vh[2], vl[2];
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          vh[t] = v[((cb * 2 + t) * 2 + 0) * 64];
+          vl[t] = v[((cb * 2 + t) * 2 + 1) * 64];
+        }
+#pragma unroll
+        for (int t = 0; t < 2; ++t) o[cb] = small_mfma(vl[t], ph[t], o[cb]);
+#pragma unroll
+        for (int t = 0; t < 2; ++t) o[cb] = small_mfma(vh[t], pl[t], o[cb]);
+#pragma unroll
+        for (int t = 0; t < 2; ++t) o[cb] = small_mfma(vh[t], ph[t], o[cb]);
+      }
+    }
+    s += xor32(s);
+    // ---- the wavefronts' sums under a common maximum ----
+    if (h == 0) sh_ms[wave][li] = make_float2(m, s);
+    __syncthreads();
+    float M = no_max;
+#pragma unroll
+    for (int w = 0; w < W; ++w) M = fmaxf(M, sh_ms[w][li].x);
+    const float fac = fast_exp2(m - M);
+#pragma unroll
+    for (int cb = 0; cb < NDB; ++cb)
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        *reinterpret_cast<float4*>(&sh_o[wave][li * LDW + 32 * cb + 8 * c + 4 * h]) =
+            make_float4(o[cb][4 * c] * fac, o[cb][4 * c + 1] * fac, o[cb][4 * c + 2] * fac, o[cb][4 * c + 3] * fac);
+    __syncthreads();
+    const float inv_v = 1.0f / a.scale[item * 2 + km];
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int e = tid + 512 * i, row = e / (NDB * 32), col = e % (NDB * 32);
+      float mm = no_max, sum = 0.f, O = 0.f;
+#pragma unroll
+      for (int w = 0; w < W; ++w) mm = fmaxf(mm, sh_ms[w][row].x);
+#pragma unroll
+      for (int w = 0; w < W; ++w) {
+        sum += sh_ms[w][row].y * fast_exp2(sh_ms[w][row].x - mm);
+        O += sh_o[w][row * LDW + col];
+      }
+      const float t = O * inv_v / fmaxf(sum, 1e-40f);  // (2^11 is in both)
+      bary[i] = pass == 0 ? t : t - bary[i];
+    }
+    __syncthreads();  // the next pass writes the same buffers
+  }
+
+  const float coef = 2.0f * a.cost_scale * g.grad_out[item];
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const int e = tid + 512 * i, col = e % (NDB * 32), row = rb * 32 + e / (NDB * 32);
+    if (row < nq && col < d) {
+      const size_t r = (size_t)item * nq + row;
+      const float diff = a.self ? bary[i] : small_load(a.pts[qm], r * d + col, a.dtype) - bary[i];
+      g.out[qm][r * d + col] = coef * a.wt[qm][r] * diff;
+    }
+  }
+}
+
+}  // namespace fs

@@ -14,6 +14,7 @@ from typing import Optional, Sequence, Tuple, Union
 
 import torch
 
+from flash_sinkhorn_amd import _small
 from flash_sinkhorn_amd._autograd import _SinkhornConfig, _SinkhornCostFn
 from flash_sinkhorn_amd.kernels._common import epsilon_schedule, max_diameter
 from flash_sinkhorn_amd.sinkhorn_solvers import (
@@ -105,6 +106,12 @@ def _process_args(*args, normalize: bool) -> _ParsedInputs:
     if normalize:
         a, b = _normalize_weights(a), _normalize_weights(b)
     return _ParsedInputs(x, y, a, b, bool(lead), a_shape, b_shape)
+
+
+def _view_shape(args, which: int) -> Tuple[int, ...]:
+    """Shape a potential is returned in: its weights' as given, or one value per point."""
+    points, weights = (args[2 * which + 1], args[2 * which]) if len(args) == 4 else (args[which], None)
+    return points.shape[:-1] if weights is None else weights.shape
 
 
 class SamplesLoss(torch.nn.Module):
@@ -241,6 +248,15 @@ class SamplesLoss(torch.nn.Module):
 
     def forward(self, *args: Union[torch.Tensor, float], label_x: Optional[torch.Tensor] = None,
                 label_y: Optional[torch.Tensor] = None):
+        small = _small.loss_problem(self, args, label_x, label_y)
+        if small is not None:
+            try:
+                if self.potentials:
+                    f, g = _small.potentials(self, *small)
+                    return f.view(_view_shape(args, 0)), g.view(_view_shape(args, 1))
+                return _small.loss(self, *small)
+            except _small.LongSchedule:
+                pass
         parsed = _process_args(*args, normalize=self.normalize)
         if not parsed.x.is_cuda or not parsed.y.is_cuda:
             raise ValueError("flash_sinkhorn.SamplesLoss requires CUDA tensors.")

@@ -13,7 +13,7 @@ from typing import Optional, Sequence, Tuple
 
 import torch
 
-from flash_sinkhorn_amd import _graphs, _lib
+from flash_sinkhorn_amd import _graphs, _lib, _small
 from flash_sinkhorn_amd.kernels._common import (
     _f32c, augment_label_cost, dampening, epsilon_schedule, label_cost_active, log_weights,
     max_diameter,
@@ -195,6 +195,17 @@ def sinkhorn_flashstyle_symmetric(
                          "label_cost_matrix.")
     rho_x, rho_y = _resolve_rho(rho, reach, rho_x, rho_y, reach_x, reach_y)
 
+    # small clouds: the whole solve in one library call (diagnostics of the planes and warm starts
+    # are the general path's)
+    if (fused is not False and not use_labels and solve_info is None
+            and f_init is None and g_init is None
+            and _small.solver_problem(x, y, a, b, allow_tf32)):
+        out = _small_symmetric(x, y, a, b, blur, scaling, use_epsilon_scaling, last_extrapolation,
+                               cost_scale, eps, n_iters, diameter, eps_list, rho_x, rho_y,
+                               threshold, check_every, return_n_iters, return_prelast)
+        if out is not None:
+            return out
+
     if eps_list is None:
         if use_epsilon_scaling:
             if diameter is None:
@@ -354,6 +365,77 @@ def sinkhorn_flashstyle_symmetric(
     return out
 
 
+def _small_symmetric(x, y, a, b, blur, scaling, use_epsilon_scaling, last_extrapolation, cost_scale,
+                     eps, n_iters, diameter, eps_list, rho_x, rho_y, threshold, check_every,
+                     return_n_iters, return_prelast):
+    """``sinkhorn_flashstyle_symmetric`` on small clouds (``_small``); None when the schedule is not
+    one that path takes (the general one then builds it, and complains where it has to)."""
+    sched = {}
+    if threshold is not None and (check_every <= 0 or torch.cuda.is_current_stream_capturing()):
+        return None
+    if threshold is not None and not threshold > 0.0:
+        threshold = None  # never met
+    if threshold is not None and return_n_iters and eps_list is None and use_epsilon_scaling \
+            and diameter is None:
+        diameter = max_diameter(x, y)  # (the length of the schedule is asked for)
+    if eps_list is None and not use_epsilon_scaling:
+        if eps is None or n_iters is None or not eps > 0 or int(n_iters) <= 0:
+            return None
+        sched = dict(eps=float(eps), entries=int(n_iters))
+    elif eps_list is None and diameter is None:
+        if not (blur > 0 and 0.0 < scaling < 1.0) or (n_iters is not None and int(n_iters) <= 0):
+            return None
+        sched = dict(blur=float(blur), scaling=float(scaling), cut=int(n_iters or 0))
+    else:
+        if eps_list is None:
+            eps_list = epsilon_schedule(diameter, blur, scaling, p=2.0)
+        eps_list = [float(e) for e in eps_list]
+        if n_iters is not None:
+            eps_list = eps_list[: int(n_iters)]
+        if len(eps_list) == 0 or not all(e > 0 for e in eps_list):
+            return None
+        sched = dict(eps_list=eps_list)
+    try:
+        s = _small.solve(*_small.points(x, y), _f32c(a.detach()), _f32c(b.detach()), items=1, cost_scale=float(cost_scale), rho_x=rho_x,
+                         rho_y=rho_y, normalize=False, self_terms=False, want_values=False,
+                         extrapolate=last_extrapolation, want_loss=False, threshold=threshold,
+                         check_every=check_every, **sched)
+    except _small.LongSchedule:
+        return None
+    (f, f_pre), (g, g_pre) = s.potentials("f"), s.potentials("g")
+    out = (f[0], g[0])
+    if return_prelast and last_extrapolation:
+        out = out + (f_pre[0], g_pre[0])
+    if return_n_iters:
+        out = out + (s.entries + 1 + int(bool(last_extrapolation)),)
+    return out
+
+
+def _small_self_pair(x, a, y, b, blur, scaling, use_epsilon_scaling, last_extrapolation, cost_scale,
+                     eps, n_iters, rho, return_prelast):
+    """``sinkhorn_flashstyle_symmetric_self_pair`` on small clouds; None as ``_small_symmetric``."""
+    if use_epsilon_scaling:
+        if not (blur > 0 and 0.0 < scaling < 1.0) or (n_iters is not None and int(n_iters) <= 0):
+            return None
+        sched = dict(blur=float(blur), scaling=float(scaling), cut=int(n_iters or 0))
+    else:
+        if eps is None or n_iters is None or not eps > 0 or int(n_iters) <= 0:
+            return None
+        sched = dict(eps=float(eps), entries=int(n_iters))
+    try:
+        s = _small.solve(*_small.points(x, y), _f32c(a.detach()), _f32c(b.detach()), items=1,
+                         cost_scale=float(cost_scale), rho_x=rho, rho_y=rho, normalize=False,
+                         self_terms=2, want_values=False, extrapolate=last_extrapolation,
+                         want_loss=False, **sched)
+    except _small.LongSchedule:
+        return None
+    outs = []
+    for which in ("xx", "yy"):
+        f, f_pre = (t[0] for t in s.potentials(which))
+        outs.append((f, f, f_pre, f_pre) if return_prelast and last_extrapolation else (f, f))
+    return tuple(outs)
+
+
 def sinkhorn_flashstyle_symmetric_self_pair(
     x: torch.Tensor, a: torch.Tensor, y: torch.Tensor, b: torch.Tensor, *,
     blur: float = 0.05, scaling: float = 0.5, use_epsilon_scaling: bool = True,
@@ -389,6 +471,12 @@ def sinkhorn_flashstyle_symmetric_self_pair(
         if len(lst) == 0:
             raise ValueError("eps_list must be non-empty")
         return lst
+
+    if _small.pair_problem(x, y, a, b, allow_tf32):
+        out = _small_self_pair(x, a, y, b, blur, scaling, use_epsilon_scaling, last_extrapolation,
+                               cost_scale, eps, n_iters, rho, return_prelast)
+        if out is not None:
+            return out
 
     xf, yf = x.detach().float().contiguous(), y.detach().float().contiguous()
     ex, ey = schedule(xf), schedule(yf)

@@ -383,6 +383,67 @@ int fs_c_transform(const float* x, const float* y, const float* bias, float* min
                    int64_t* argmin_out, int64_t n, int64_t m, int64_t d, float coord_scale,
                    uint32_t flags, void* workspace, size_t workspace_bytes, void* stream);
 
+/*
+ * Whole solves of small problems (d <= 128, at most FS_SMALL_MAX_ROWS rows per cloud), the default
+ * operand mode: `items` independent problems of one shape (a batch; 1 otherwise), each the balanced
+ * or unbalanced symmetric problem of x [items, n, d] and y [items, m, d] and, with self_terms,
+ * its two self problems (x, x) and (y, y) (self_terms 2: these alone), all advanced by one launch per step.  What a
+ * solver needs before the first step (norms, log weights, operand planes, the eps schedule) is
+ * done on the device as well.
+ *   dtype      0 fp32, 1 fp16, 2 bf16 (x and y)
+ *   a, b       weights [items, n], [items, m] or NULL (uniform); normalize: divided by their sum
+ *   sched      0: `entries` averaged steps at `eps`; 1: the schedule of a cloud's diameter, `blur`
+ *              and `scaling` (each problem its own, cut to `cut` entries if that is > 0);
+ *              2: eps_list, a HOST array of `entries` values
+ *   extrapolate  one full step at the last eps behind them; the gradient is taken before it
+ *   rho_x, rho_y  <= 0: strict marginals
+ * Steps: one full step at the first entry, one averaged step (weight 1/2) per entry, the
+ * extrapolation.  The workspace keeps what fs_small_grad reads (want_values != 0), so it has to
+ * live until then.
+ *   threshold  > 0: a problem none of whose potentials moved by it between two checks, one every
+ *              check_every averaged steps (the first only takes a snapshot), runs no more entries
+ * host_words: sched 1 or a threshold, 4 * items ints of PINNED host memory that the device can
+ * write: the number of steps then depends on the clouds, and fs_small_solve waits for it (the one
+ * entry point that waits for the device).  It must not be in use by another call.  Afterwards
+ * word 4 * i + q holds the entries of problem q's schedule, or, with a threshold, 2 * c + 1 when
+ * the problem stopped at check c (behind (c + 1) * check_every averaged steps).
+ * loss  [items] or NULL: <a, f> + <b, g>, or (rho_x + eps/2) <a, 1 - exp(-f/rho_x)> + ... with both
+ * marginals relaxed, minus half of each self problem's cost.
+ * pots  or NULL: the standard potentials: f, f before the extrapolation ([items, n] each), g, g
+ * before it ([items, m] each), and with self_terms likewise those of (x, x) and of (y, y).
+ * Returns FS_OK, an error, or one of FS_SMALL_* (sched 1: what the diameters did not allow; no
+ * step was run).  Replaces sinkhorn_flashstyle_symmetric (sinkhorn_solvers.py:290-707) and the
+ * three solves of a debiased SamplesLoss (samples_loss.py:494-512) for these sizes.
+ */
+#define FS_SMALL_MAX_ROWS 16384
+#define FS_SMALL_NO_DIAMETER 1    /* a cloud is a single point */
+#define FS_SMALL_NOT_A_NUMBER 2   /* a coordinate is not finite */
+#define FS_SMALL_LONG_SCHEDULE 3  /* more entries than the device table holds */
+typedef struct fs_small_problem {
+  const void* x;
+  const void* y;
+  const float* a;
+  const float* b;
+  const float* eps_list;
+  int64_t n, m, d, items;
+  double blur, scaling;
+  float cost_scale, eps, rho_x, rho_y, threshold;
+  int dtype, normalize, self_terms, want_values, sched, entries, cut, extrapolate, check_every;
+} fs_small_problem;
+
+size_t fs_small_workspace_bytes(const fs_small_problem* problem);
+int fs_small_solve(const fs_small_problem* problem, void* workspace, size_t workspace_bytes,
+                   int* host_words, float* loss, float* pots, void* stream);
+
+/*
+ * Gradients of `loss` in x and y (NULL: not wanted) times grad_out [items] (device), fp32
+ * [items, n, d] and [items, m, d], from the workspace fs_small_solve left behind.
+ * Replaces sinkhorn_geomloss_online_grad_sqeuclid
+ * (kernels/sinkhorn_triton_grad_sqeuclid.py:891-1207) for these sizes.
+ */
+int fs_small_grad(const fs_small_problem* problem, void* workspace, size_t workspace_bytes,
+                  const float* grad_out, float* grad_x, float* grad_y, void* stream);
+
 #ifdef __cplusplus
 }
 #endif
