@@ -26,8 +26,8 @@ _P, _I64, _D, _F, _I = (ctypes.c_void_p, ctypes.c_int64, ctypes.c_double, ctypes
 _DTYPES = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}
 
 MAX_D = 128
-MAX_ROWS = 4096
-_TABLE = 512  # entries of a schedule the device keeps
+MAX_ROWS = 65536
+_TABLE = 511  # entries of a schedule the device keeps
 
 
 class Problem(ctypes.Structure):
@@ -72,8 +72,27 @@ class Solved:
         return tuple(self.pots[at + i * size:at + (i + 1) * size].view(p.items, rows) for i in (0, 1))
 
 
-def _rows_ok(n: int, m: int, d: int) -> bool:
-    return 0 < n <= MAX_ROWS and 0 < m <= MAX_ROWS and 0 < d <= MAX_D
+def _size_ok(n: int, m: int, d: int, fixed: bool, self_terms: int, stops: bool) -> bool:
+    """Whether a problem of this size is faster here than on the general path, launch by launch.
+
+    d <= 64 (``pair_sweep_kernel`` from 2e7 logits per step on): everywhere but where two large
+    clouds let the general path skip tiles by its coarse product, from 24,000 rows on.  At fixed
+    eps that pays from its first size on (30,000 x 64, 40 steps: 9.6 against 18 ms; 22,000 x 64, no
+    skipping: 11.3 against 10.2), on a schedule only in its last steps (30,000 x 64, both gradients:
+    8.9 against 9.6 ms; 40,000 x 16: 6.9 against 6.7), and with d <= 8 not at all (50,000 x 3: 28
+    against 19 ms).
+    d <= 128, or early stopping on a schedule: the small kernels, which go over the logits once per
+    side: up to 2e7 logits at fixed eps (3,000 x 128: 1.05 against 1.54 ms; 4,500: 2.8 against 2.4),
+    6e7 on a schedule (6,500 x 128: 1.54 against 1.94 ms; 9,000: 3.1 against 2.8).
+    """
+    if not (0 < n <= MAX_ROWS and 0 < m <= MAX_ROWS and 0 < d <= MAX_D):
+        return False
+    if d > 64 or (stops and not fixed):
+        logits = (n * m if self_terms < 2 else 0) + ((n * n + m * m) // 2 if self_terms else 0)
+        return logits <= (20_000_000 if fixed else 60_000_000)
+    if d <= 8 or min(n, m) < 24000:
+        return True
+    return not fixed and d <= 32 and n * m <= 1_600_000_000
 
 
 def _operands_ok(allow_tf32: bool) -> bool:
@@ -160,18 +179,27 @@ def points(x, y):
     return x.detach().contiguous(), y.detach().contiguous()
 
 
-def pair_problem(x, y, a, b, allow_tf32: bool) -> bool:
+def pair_problem(x, y, a, b, allow_tf32: bool, fixed: bool, self_terms: int = 0,
+                 stops: bool = False) -> bool:
     """Whether clouds and weights (any of which may need a gradient) are ones ``solve`` takes."""
     return (x.is_cuda and y.is_cuda and x.ndim == 2 and y.ndim == 2 and a.ndim == 1 and b.ndim == 1
-            and x.shape[1] == y.shape[1] and _rows_ok(x.shape[0], y.shape[0], x.shape[1])
+            and x.shape[1] == y.shape[1]
+            and _size_ok(x.shape[0], y.shape[0], x.shape[1], fixed, self_terms, stops)
+            # (a solver called by itself keeps to the tile-skipping kernels where it has them)
+            and (x.shape[1] <= 8 or min(x.shape[0], y.shape[0]) < 24000)
             and a.shape[0] == x.shape[0] and b.shape[0] == y.shape[0]
             and x.is_floating_point() and y.is_floating_point() and _operands_ok(allow_tf32)
             and x.device == y.device == a.device == b.device)
 
 
-def solver_problem(x, y, a, b, allow_tf32: bool) -> bool:
-    """Whether ``sinkhorn_flashstyle_symmetric`` may hand its clouds and weights to ``solve``."""
-    return pair_problem(x, y, a, b, allow_tf32) and not (
+def solver_problem(x, y, a, b, allow_tf32: bool, fixed: bool, stops: bool) -> bool:
+    """Whether ``sinkhorn_flashstyle_symmetric`` may hand its clouds and weights to ``solve``.  One cloud
+    against itself, on more than a few thousand points, stays with the general path: one
+    half-update per step instead of two, and f equal to g to the bit."""
+    if x.data_ptr() == y.data_ptr() and a.data_ptr() == b.data_ptr() and x.shape == y.shape \
+            and x.shape[0] ** 2 >= 20_000_000:
+        return False
+    return pair_problem(x, y, a, b, allow_tf32, fixed, 0, stops) and not (
         torch.is_grad_enabled()
         and (x.requires_grad or y.requires_grad or a.requires_grad or b.requires_grad))
 
@@ -226,7 +254,10 @@ def loss_problem(loss, args, label_x, label_y):
             or not y.is_floating_point() or not x.is_cuda or y.device != x.device:
         return None
     if x.ndim not in (2, 3) or y.ndim != x.ndim or x.shape[-1] != y.shape[-1] \
-            or x.shape[:-2] != y.shape[:-2] or not _rows_ok(x.shape[-2], y.shape[-2], x.shape[-1]):
+            or x.shape[:-2] != y.shape[:-2]:
+        return None
+    if not _size_ok(x.shape[-2], y.shape[-2], x.shape[-1], not loss.use_epsilon_scaling,
+                    int(loss.debias and not loss.potentials), loss.threshold is not None):
         return None
     lead = x.shape[:-2]
     if lead and not 0 < lead[0] <= 65535:

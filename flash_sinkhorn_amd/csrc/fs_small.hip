@@ -1,6 +1,7 @@
 // Small problems: planning, workspace and launches of the kernels in fs_small.hpp.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <atomic>
 #include <chrono>
 #include <cmath>
@@ -9,6 +10,7 @@
 #include <vector>
 
 #include "flash_sinkhorn_hip.h"
+#include "fs_pair.hpp"
 #include "fs_small.hpp"
 
 namespace fs {
@@ -21,9 +23,29 @@ struct EpsTable {
 // Schedule given by the caller: every item and problem takes the same entries.
 template <int T>
 __global__ __launch_bounds__(256) void small_table_kernel(const SmallArgs a, const EpsTable t) {
-  float* out = a.table + (size_t)blockIdx.x * kSmallTable;
-  for (int i = threadIdx.x; i < a.entries; i += 256) out[i] = t.e[i];
+  float4* out = a.table + (size_t)blockIdx.x * kSmallTable;
+  for (int i = threadIdx.x; i <= a.entries; i += 256) out[i] = small_coef(a.cost_scale, t.e[min(i, a.entries - 1)]);
   if (threadIdx.x == 0) a.lens[blockIdx.x] = a.full[blockIdx.x] = a.entries;
+}
+
+// Which kernels a problem takes.  d <= 64: both sides of a step from one sweep (fs_pair.hpp) where
+// that saves more than its second launch per step costs.  Fixed eps: from 2e7 logits per step on
+// (one problem of 4,500 points, d = 64, 40 steps: 1.19 against 1.50 ms; 3,000 points: 0.85 against
+// 0.65 ms).  A schedule rewrites the planes behind every step and has few steps: 5e7 (d = 3, 6,500 points:
+// 0.48 against 0.42 ms; 9,000: 0.67 against 0.75), 2e7 where the planes are wide (d = 64, 4,500:
+// 0.58 against 0.62 ms).  Items of a batch fill the chip without it: 12 x 2,048 x 8, debiased, 0.81
+// against 0.66 ms.  Early stopping on a schedule is only built for the small kernels.
+bool use_pair(const fs_small_problem* p) {
+  if (p->d > 64 || (p->threshold > 0.f && p->sched != 0)) return false;
+  const double n = (double)p->n, m = (double)p->m;
+  const double logits = (p->self_terms < 2 ? n * m : 0.) + (p->self_terms ? 0.5 * (n * n + m * m) : 0.);
+  return logits >= (p->sched == 0 || p->d > 32 ? 2.0e7 : 5.0e7);
+}
+
+// Workgroups over which the loss of an item is spread: one for what a workgroup does in three rounds.
+int loss_parts(const SmallArgs& a) {
+  const int rows = std::max(a.rows[0], a.rows[1]);
+  return rows <= 3072 ? 1 : std::min(64, (rows + 1023) / 1024);
 }
 
 int padded(int64_t d) { return d <= 16 ? 16 : (d <= 32 ? 32 : (d <= 64 ? 64 : 128)); }
@@ -38,7 +60,7 @@ int checked(const fs_small_problem* p) {
   if (p->sched == 1 && !(p->blur > 0.0 && p->scaling > 0.0 && p->scaling < 1.0)) return FS_ERR_BAD_ARGUMENT;
   if (p->sched == 2) {
     if (!p->eps_list) return FS_ERR_NULL_POINTER;
-    if (p->entries > kSmallTable) return FS_ERR_UNSUPPORTED;
+    if (p->entries >= kSmallTable) return FS_ERR_UNSUPPORTED;
     for (int i = 0; i < p->entries; ++i)
       if (!(p->eps_list[i] > 0.f)) return FS_ERR_BAD_ARGUMENT;
   }
@@ -46,10 +68,117 @@ int checked(const fs_small_problem* p) {
   return p->self_terms < 0 || p->self_terms > 2 ? FS_ERR_BAD_ARGUMENT : FS_OK;
 }
 
+// Work items of a medium problem's launch: 256-row groups of the stationary rows times chunks of the
+// streamed ones, one chunk length for all problems.  Two workgroups per CU run at a time, so
+// the length is the one whose last round of 512 is fullest, counting two tiles' worth of time for
+// what an item costs around its tiles.
+void plan_pair(const SmallArgs& a, PairArgs& t) {
+  t.items = a.items;
+  t.first_prob = a.self == 2 ? 1 : 0;
+  t.nprob = a.self ? 3 : 1;
+  t.sched = a.sched;
+  t.extrapolate = a.extrapolate;
+  for (int q = t.first_prob; q < t.nprob; ++q) {
+    PairProblem& pr = t.prob[q];
+    const int s = q == 2 ? 1 : 0, k = q == 0 ? 1 : s;
+    pr.self = q > 0;
+    pr.n_st = a.rows[s];
+    pr.n_str = a.rows[k];
+    pr.st_blocks = a.pblocks[s];
+    pr.str_blocks = a.pblocks[k];
+    pr.groups = (pr.n_st + 255) / 256;
+  }
+  auto items_at = [&](int tiles, PairArgs& u) {
+    int n = 0;
+    for (int q = t.first_prob; q < t.nprob; ++q) {
+      PairProblem& pr = u.prob[q];
+      pr.chunk = tiles * 64;
+      pr.chunks = (pr.n_str + pr.chunk - 1) / pr.chunk;
+      pr.first_item = n;
+      pr.n_items = 0;
+      for (int c = 0; c < pr.chunks; ++c)
+        pr.n_items += pr.self ? self_groups_of_chunk(c, pr.chunk, pr.n_str, pr.groups) : pr.groups;
+      pr.two_first = pr.groups * pr.chunks;
+      pr.two_items = pr.two_first;
+      if (!pr.self)
+        pr.two_items += (pr.n_str + 255) / 256 * ((pr.n_st + pr.chunk - 1) / pr.chunk);
+      n += pr.n_items;
+    }
+    return n;
+  };
+  int best = 4;
+  double cost = 0.0;
+  for (int tiles = 4; tiles <= 64; ++tiles) {
+    const double n = (double)items_at(tiles, t) * a.items;
+    const double c = std::ceil(n / 512.0) * (tiles + 2);
+    if (cost == 0.0 || c < cost - 1e-9) cost = c, best = tiles;
+  }
+  t.total_items = items_at(best, t);
+  for (int i = 0; i < 4; ++i) {
+    PairSide& sd = t.side[i];
+    const int mat = i & 1;
+    sd.rows = a.rows[mat];
+    sd.blocks = a.pblocks[mat];
+  }
+}
+
+// Pointers of a medium problem's kernels once the workspace is laid out; what alternates from
+// step to step is set by pair_step_args.
+void bind_pair(const SmallArgs& a, PairArgs& t) {
+  t.table = a.table;
+  t.lens = a.lens;
+  t.limits = a.limits;
+  t.reach = a.reach;
+  for (int q = t.first_prob; q < t.nprob; ++q) {
+    PairProblem& pr = t.prob[q];
+    const int s = q == 2 ? 1 : 0, k = q == 0 ? 1 : s;
+    const int ss = q == 0 ? 0 : 1 + q, ks = q == 0 ? 1 : ss;  // sides of the stationary and the streamed rows
+    auto planes = [&](int m) { return q > 0 && a.self_planes[m] ? a.self_planes[m] : a.planes[m]; };
+    pr.st_planes = planes(s);
+    pr.str_planes = planes(k);
+    pr.st_bias = t.side[ss].bias;
+    pr.str_bias = t.side[ks].bias;
+    pr.st_bias32 = t.side[ss].bias32;
+    pr.str_bias32 = t.side[ks].bias32;
+    for (int i : {ss, ks}) {
+      PairSide& sd = t.side[i];
+      const int mat = i & 1;
+      sd.part = i == ss ? pr.st_part : pr.str_part;
+      sd.parts = i == ss ? pr.chunks : pr.groups;
+      sd.col = pr.str_part;
+      sd.ms = i == ss ? pr.st_ms : pr.str_ms;
+      sd.ms_parts = i == ss ? pr.chunks : (pr.n_st + pr.chunk - 1) / pr.chunk;
+      sd.self = pr.self;
+      sd.chunk = pr.chunk;
+      sd.norm = a.norm[mat];
+      sd.l2w = a.l2w[mat];
+      sd.pts = a.pts[mat];
+      sd.dtype = a.dtype;
+      sd.d = a.d;
+      sd.rho = a.rho[mat];
+      // (where all problems share their eps, the first of them writes the planes they share)
+      sd.planes = a.self_planes[mat] ? (i < 2 ? a.planes[mat] : a.self_planes[mat])
+                                     : (i < 2 || a.self == 2 ? a.planes[mat] : nullptr);
+    }
+  }
+}
+
+void pair_step_args(const SmallArgs& a, PairArgs& t, int step) {
+  t.step = step;
+  for (int i = a.self == 2 ? 2 : 0; i < (a.self ? 4 : 2); ++i) {
+    PairSide& sd = t.side[i];
+    const size_t n = (size_t)a.items * sd.rows;
+    const int from = step < 0 ? 0 : step & 1;
+    sd.old = a.pot[i] + from * n;
+    sd.out = a.pot[i] + (from ^ 1) * n;
+  }
+}
+
 // The kernels' arguments with the workspace laid out from `ws` (null: sizes only); returns the
 // bytes the workspace takes.
-size_t layout(const fs_small_problem* p, void* ws, SmallArgs& a) {
+size_t layout(const fs_small_problem* p, void* ws, SmallArgs& a, PairArgs* pa = nullptr) {
   std::memset(&a, 0, sizeof(a));
+  a.pair = use_pair(p) ? 1 : 0;
   a.pts[0] = p->x;
   a.pts[1] = p->y;
   a.w[0] = p->a;
@@ -83,14 +212,17 @@ size_t layout(const fs_small_problem* p, void* ws, SmallArgs& a) {
   const size_t items = (size_t)p->items;
   take(a.lens, items * 3 * 4);
   take(a.full, items * 3 * 4);
-  take(a.scale, items * 2 * 4);
+  take(a.scale, items * 2 * sizeof(float2));
   take(a.stats, items * 2 * kSmallStatBlocks * kSmallStatWords * 4);
-  if (p->sched != 0) take(a.table, items * 3 * kSmallTable * 4);
+  take(a.table, items * 3 * kSmallTable * sizeof(float4));
   for (int i = 0; i < 2; ++i) {
     const size_t rows = (size_t)a.rows[i];
     a.blocks[i] = (int)((rows + 31) / 32);
-    const size_t blocks = items * (size_t)a.blocks[i];
-    take(a.planes[i], blocks * (size_t)(2 * dp / 16) * 1024);
+    // (whole 256-row groups, and the tiles that are fetched past the end)
+    a.pblocks[i] = a.pair ? (int)((rows + 255) / 256) * 8 + 8 : a.blocks[i];
+    const size_t blocks = items * (size_t)a.blocks[i], pblocks = items * (size_t)a.pblocks[i];
+    take(a.planes[i], pblocks * (size_t)(2 * dp / 16) * 1024);
+    if (a.pair && a.self && a.sched != 0) take(a.self_planes[i], pblocks * (size_t)(2 * dp / 16) * 1024);
     if (a.want_values) take(a.values[i], blocks * (size_t)(ndb * 4) * 1024);
     take(a.norm[i], items * rows * 4);
     take(a.wt[i], items * rows * 4);
@@ -101,6 +233,28 @@ size_t layout(const fs_small_problem* p, void* ws, SmallArgs& a) {
       take(a.prev[i], items * rows * 4);
       if (a.self) take(a.prev[2 + i], items * rows * 4);
     }
+  }
+  if (a.pair) {
+    take(a.limits, items * sizeof(float4));
+    take(a.reach, items * sizeof(float4));
+    PairArgs scratch;
+    PairArgs& t = pa ? *pa : scratch;
+    std::memset(&t, 0, sizeof(t));
+    plan_pair(a, t);
+    take(t.state, items * 3 * kPairStateWords * 4);
+    for (int q = t.first_prob; q < t.nprob; ++q) {
+      PairProblem& pr = t.prob[q];
+      take(pr.st_part, items * (size_t)pr.chunks * (size_t)pr.n_st * 4);
+      take(pr.str_part, items * (size_t)pr.groups * (size_t)pr.n_str * 4);
+      take(pr.st_ms, items * (size_t)pr.chunks * (size_t)pr.n_st * sizeof(float2));
+      if (!pr.self) take(pr.str_ms, items * (size_t)((pr.n_st + pr.chunk - 1) / pr.chunk) * (size_t)pr.n_str * sizeof(float2));
+    }
+    for (int i = a.self == 2 ? 2 : 0; i < (a.self ? 4 : 2); ++i) {
+      PairSide& sd = t.side[i];
+      take(sd.bias, items * (size_t)sd.blocks * 32 * sizeof(u32x4));
+      take(sd.bias32, items * (size_t)sd.blocks * 32 * 4);
+    }
+    if (pa) bind_pair(a, t);
   }
   return at;
 }
@@ -113,15 +267,65 @@ int launch_prep(const SmallArgs& a, hipStream_t st) {
   return hipGetLastError() == hipSuccess ? FS_OK : FS_ERR_LAUNCH_FAILED;
 }
 
+SmallStepArgs step_args(const SmallArgs& a, int step) {
+  SmallStepArgs t;
+  std::memset(&t, 0, sizeof(t));
+  t.scale = reinterpret_cast<const float4*>(a.scale);
+  t.step = step;
+  t.extrapolate = a.extrapolate;
+  const int first = a.self == 2 ? 2 : 0, sides = a.self == 1 ? 4 : 2;
+  for (int i = 0; i < sides; ++i) {
+    const int side = first + i, qm = side & 1, km = side < 2 ? qm ^ 1 : qm, prob = side < 2 ? 0 : side - 1;
+    SmallStepSide& s = t.side[i];
+    const size_t nq = (size_t)a.items * a.rows[qm], nk = (size_t)a.items * a.rows[km];
+    s.kplanes = a.planes[km];
+    s.qplanes = a.planes[qm];
+    s.kpot = a.pot[side < 2 ? side ^ 1 : side] + (step & 1) * nk;
+    s.kl2w = a.l2w[km];
+    // (the entry past the last repeats it, for the extrapolation)
+    s.coef = a.table + prob * kSmallTable + (a.sched == 0 ? 0 : std::min(std::max(step - 1, 0), kSmallTable - 1));
+    s.lens = a.lens + prob;
+    s.old = a.pot[side] + (step & 1) * nq;
+    s.out = a.pot[side] + ((step & 1) ^ 1) * nq;
+    s.norm = a.norm[qm];
+    s.nq = a.rows[qm];
+    s.nk = a.rows[km];
+    s.nqb = a.blocks[qm];
+    s.nkb = a.blocks[km];
+    s.rho = a.rho[qm];
+    s.qm = qm;
+    s.km = km;
+  }
+  return t;
+}
+
 template <int DP>
 int launch_step(const SmallArgs& a, int step, hipStream_t st) {
-  const int blocks = (a.blocks[0] + a.blocks[1]) * (a.self == 1 ? 2 : 1);
-#ifndef FS_SMALL_W
-#define FS_SMALL_W 8
-#endif
-  constexpr int W = FS_SMALL_W;
-  hipLaunchKernelGGL((small_step_kernel<DP, W>), dim3(blocks, a.items), dim3(64 * W), 0, st, a, step);
+  const int xb = a.blocks[0] > a.blocks[1] ? a.blocks[0] : a.blocks[1];
+  const dim3 grid(xb, a.self == 1 ? 4 : 2, a.items);
+  constexpr int W = 8;  // wavefronts that share the keys of 32 rows (16: slower from 700 points on)
+  const SmallStepArgs t = step_args(a, step);
+  hipLaunchKernelGGL((small_step_kernel<DP, W>), grid, dim3(64 * W), 0, st, t);
   return hipGetLastError() == hipSuccess ? FS_OK : FS_ERR_LAUNCH_FAILED;
+}
+
+template <int DP>
+int launch_pair_merge(const SmallArgs& a, PairArgs& t, int step, hipStream_t st) {
+  pair_step_args(a, t, step);
+  const int blocks = std::max(a.pblocks[0], a.pblocks[1]);
+  t.merge_groups = (blocks + 1) / 2;
+  // (at one eps the planes are written once, before the first step)
+  const int grid = t.merge_groups + (step < 0 || a.sched != 0 ? blocks : 0);
+  hipLaunchKernelGGL((pair_merge_kernel<DP>), dim3(grid, a.self == 1 ? 4 : 2, a.items), dim3(256), 0, st, t);
+  return hipGetLastError() == hipSuccess ? FS_OK : FS_ERR_LAUNCH_FAILED;
+}
+
+template <int DP>
+int launch_pair_step(const SmallArgs& a, PairArgs& t, int step, hipStream_t st) {
+  pair_step_args(a, t, step);
+  const int blocks = (t.total_items + 7) / 8 * 8;
+  hipLaunchKernelGGL((pair_sweep_kernel<DP>), dim3(blocks, a.items), dim3(256), 0, st, t);
+  return launch_pair_merge<DP>(a, t, step, st);
 }
 
 // Looks at pinned words until `arrived` says that what the device has to write is there (it
@@ -140,8 +344,9 @@ int wait_for_words(hipStream_t st, F&& arrived) {
 
 template <int DP>
 int launch_grad(const SmallArgs& a, const SmallGradArgs& g, hipStream_t st) {
-  const int blocks = (g.out[0] ? a.blocks[0] : 0) + (g.out[1] ? a.blocks[1] : 0);
-  hipLaunchKernelGGL((small_grad_kernel<DP>), dim3(blocks, a.items), dim3(512), 0, st, a, g);
+  const int xb = a.blocks[0] > a.blocks[1] ? a.blocks[0] : a.blocks[1];
+  const dim3 grid(!g.out[0] ? a.blocks[1] : (!g.out[1] ? a.blocks[0] : xb), g.out[0] && g.out[1] ? 2 : 1, a.items);
+  hipLaunchKernelGGL((small_grad_kernel<DP>), grid, dim3(512), 0, st, a, g);
   return hipGetLastError() == hipSuccess ? FS_OK : FS_ERR_LAUNCH_FAILED;
 }
 
@@ -174,7 +379,8 @@ int fs_small_solve(const fs_small_problem* p, void* workspace, size_t workspace_
   if (rc != FS_OK) return rc;
   if ((p->sched == 1 || p->threshold > 0.f) && !host_words) return FS_ERR_NULL_POINTER;
   SmallArgs a;
-  if (layout(p, workspace, a) > workspace_bytes || !workspace) return FS_ERR_WORKSPACE_TOO_SMALL;
+  PairArgs pa;
+  if (!workspace || layout(p, workspace, a, &pa) > workspace_bytes) return FS_ERR_WORKSPACE_TOO_SMALL;
   hipStream_t st = (hipStream_t)stream;
   int entries = a.entries;
   a.host_words = host_words;
@@ -190,7 +396,13 @@ int fs_small_solve(const fs_small_problem* p, void* workspace, size_t workspace_
     hipLaunchKernelGGL((small_table_kernel<0>), dim3(a.items * 3), dim3(256), 0, st, a, t);
     if (hipGetLastError() != hipSuccess) return FS_ERR_LAUNCH_FAILED;
   }
-  rc = by_width(p->d, [&](auto dp) { return launch_prep<decltype(dp)::value>(a, st); });
+  rc = by_width(p->d, [&](auto dp) {
+    constexpr int DP = decltype(dp)::value;
+    const int r = launch_prep<DP>(a, st);
+    if constexpr (DP <= 64)
+      if (r == FS_OK && a.pair) return launch_pair_merge<DP>(a, pa, -1, st);
+    return r;
+  });
   if (rc != FS_OK) return rc;
   const int p0 = a.self == 2 ? 1 : 0, p1 = a.self == 0 ? 1 : 3;  // the problems that are solved
   if (a.sched == 1) {
@@ -235,7 +447,12 @@ int fs_small_solve(const fs_small_problem* p, void* workspace, size_t workspace_
     });
   };
   for (int s = 0; s < n_steps && rc == FS_OK && !all_done; ++s) {
-    rc = by_width(p->d, [&](auto dp) { return launch_step<decltype(dp)::value>(a, s, st); });
+    rc = by_width(p->d, [&](auto dp) {
+      constexpr int DP = decltype(dp)::value;
+      if constexpr (DP <= 64)
+        if (a.pair) return launch_pair_step<DP>(a, pa, s, st);
+      return launch_step<DP>(a, s, st);
+    });
     if (rc != FS_OK || !early || s == 0 || s > entries || s % p->check_every != 0) continue;
     hipLaunchKernelGGL((small_check_kernel<0>), dim3(p1 - p0, a.items), dim3(1024), 0, st, a, s, checks);
     if (hipGetLastError() != hipSuccess) return FS_ERR_LAUNCH_FAILED;
@@ -249,7 +466,10 @@ int fs_small_solve(const fs_small_problem* p, void* workspace, size_t workspace_
   l.loss = loss;
   l.pots = pots;
   l.relaxed = a.rho[0] > 0.f && a.rho[1] > 0.f ? 1 : 0;
-  hipLaunchKernelGGL((small_loss_kernel<0>), dim3(1, a.items), dim3(1024), 0, st, a, l);
+  const int parts = loss_parts(a);
+  l.parts = a.stats;  // (done with since the preparation)
+  hipLaunchKernelGGL((small_loss_kernel<0>), dim3(parts, a.items), dim3(1024), 0, st, a, l);
+  if (loss && parts > 1) hipLaunchKernelGGL((small_loss_sum_kernel<0>), dim3(a.items), dim3(64), 0, st, l, parts);
   return hipGetLastError() == hipSuccess ? FS_OK : FS_ERR_LAUNCH_FAILED;
 }
 

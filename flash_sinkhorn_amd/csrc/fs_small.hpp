@@ -22,10 +22,10 @@
 
 namespace fs {
 
-constexpr int kSmallStatBlocks = 16;            // workgroups per matrix and item of small_stats_kernel
+constexpr int kSmallStatBlocks = 64;            // workgroups per matrix and item of small_stats_kernel
 constexpr int kSmallMaxD = 128;
-constexpr int kSmallStatWords = 2 + 2 * kSmallMaxD;  // absmax, weight sum, column minima, column maxima
-constexpr int kSmallTable = 512;                // longest eps schedule kept on the device
+constexpr int kSmallStatWords = 4 + 2 * kSmallMaxD;  // absmax; weights: sum, smallest, largest; column minima, maxima
+constexpr int kSmallTable = 512;                // entries of an eps schedule kept on the device
 
 // A run of small problems.  Sides: 0 f of the xy problem (rows of x against keys y), 1 g of it
 // (rows of y against keys x), 2 the self problem of x, 3 that of y.  Problems: 0 xy, 1 xx, 2 yy.
@@ -46,14 +46,15 @@ struct SmallArgs {
   float rho[2];           // <= 0: strict marginal
   // workspace
   float* stats;           // [items][2][kSmallStatBlocks][kSmallStatWords]
-  float* scale;           // [items][2] power-of-two scales of the planes
+  float2* scale;          // [items][2] power-of-two scales of the planes, and their inverses
   u32x4* planes[2];       // [items][blocks][2 planes][DP / 16][64]
   u32x4* values[2];       // [items][blocks][DP / 32][2 steps][2 planes][64]
   float* norm[2];         // [items][rows] cost_scale * |row|^2
   float* wt[2];           // [items][rows] weights as the solve takes them
   float* l2w[2];          // [items][rows] their base-2 logarithms
   float* pot[4];          // [2 parities][items][rows of the side]: shifted potentials
-  float* table;           // [items][3][kSmallTable] eps of every entry
+  float4* table;          // [items][3][kSmallTable] per entry: eps and what the kernels derive from
+                          // it (small_coef); one entry past the last repeats it
   int* full;              // [items][3] entries of the schedules
   int* lens;              // [items][3] those the problem runs: fewer once it has converged
   int* host_words;        // pinned host memory, 4 words per item (see small_schedule, small_check_kernel)
@@ -61,6 +62,13 @@ struct SmallArgs {
   // early stopping (threshold > 0): the potentials of the last check
   float threshold;
   float* prev[4];         // [items][rows of the side]
+  // medium problems (fs_pair.hpp): their planes carry the square root of the logits' scale, a set
+  // per problem where each has an eps of its own
+  int pair;
+  int pblocks[2];         // 32-row blocks of the planes of x and y, padding included
+  u32x4* self_planes[2];
+  float4* limits;
+  float4* reach;
 };
 
 __device__ __forceinline__ float small_load(const void* p, size_t i, int dtype) {
@@ -69,16 +77,20 @@ __device__ __forceinline__ float small_load(const void* p, size_t i, int dtype) 
   return __builtin_bit_cast(float, (unsigned)static_cast<const unsigned short*>(p)[i] << 16);
 }
 
-// Entries of a problem's schedule, the number of its steps, and the eps and weight of step s
-// (the first full step at entry 0, an averaged step per entry, one full step at the last entry).
-__device__ __forceinline__ int small_entries(const SmallArgs& a, int item, int prob) {
-  return a.sched == 0 && !(a.threshold > 0.f) ? a.entries : a.lens[item * 3 + prob];
+// What a step derives from its eps: eps, base-2 logit per unit of x.y, its inverse, base-2 units
+// per unit of a potential.
+__device__ __forceinline__ float4 small_coef(float cost_scale, float eps) {
+  const float qs = 2.0f * cost_scale / eps * kLog2e;
+  return make_float4(eps, qs, 1.0f / qs, kLog2e / eps);
 }
-__device__ __forceinline__ int small_full_entries(const SmallArgs& a, int item, int prob) {
-  return a.sched == 0 ? a.entries : a.full[item * 3 + prob];
+__device__ __forceinline__ const float4* small_table(const SmallArgs& a, int item, int prob) {
+  return a.table + ((size_t)item * 3 + prob) * kSmallTable;
 }
-__device__ __forceinline__ float small_eps(const SmallArgs& a, int item, int prob, int idx) {
-  return a.sched == 0 ? a.eps0 : a.table[((size_t)item * 3 + prob) * kSmallTable + idx];
+// The coefficients behind the cost and the gradient: those of the schedule's last entry (which a
+// problem that stopped early keeps).
+__device__ __forceinline__ float4 small_last_coef(const SmallArgs& a, int item, int prob) {
+  const float4* t = small_table(a, item, prob);
+  return t[a.sched == 0 ? 0 : a.full[item * 3 + prob] - 1];
 }
 
 // Partial statistics of a slice of one matrix of one item: largest magnitude (the plane scale),
@@ -96,6 +108,7 @@ __global__ __launch_bounds__(256) void small_stats_kernel(const SmallArgs a) {
   bool nan = false;
   if (tid < act) {
     const size_t base = (size_t)item * rows * d;
+#pragma unroll 8
     for (size_t e = (size_t)r0 * d + tid; e < (size_t)r1 * d; e += act) {
       const float v = small_load(a.pts[mat], base + e, a.dtype);
       lo = fminf(lo, v);
@@ -103,8 +116,14 @@ __global__ __launch_bounds__(256) void small_stats_kernel(const SmallArgs a) {
       nan = nan || !(v == v);
     }
   }
-  if (a.w[mat] != nullptr && a.normalize)
-    for (int r = r0 + tid; r < r1; r += 256) ws += a.w[mat][(size_t)item * rows + r];
+  float wl = 3.0e38f, wh = 0.f;
+  if (a.w[mat] != nullptr)
+    for (int r = r0 + tid; r < r1; r += 256) {
+      const float w = a.w[mat][(size_t)item * rows + r];
+      ws += w;
+      wl = fminf(wl, w);
+      wh = fmaxf(wh, w);
+    }
   if (nan) lo = hi = __builtin_nanf("");
   mn[tid] = lo;
   mx[tid] = hi;
@@ -121,8 +140,8 @@ __global__ __launch_bounds__(256) void small_stats_kernel(const SmallArgs a) {
   __syncthreads();
   float* out = a.stats + (((size_t)item * 2 + mat) * kSmallStatBlocks + blockIdx.x) * kSmallStatWords;
   if (tid < d) {
-    out[2 + tid] = mn[tid];
-    out[2 + kSmallMaxD + tid] = mx[tid];
+    out[4 + tid] = mn[tid];
+    out[4 + kSmallMaxD + tid] = mx[tid];
   }
   __syncthreads();
   // (a NaN does not reach the plane scale: fmaxf drops it, as absmax_kernel does)
@@ -131,17 +150,33 @@ __global__ __launch_bounds__(256) void small_stats_kernel(const SmallArgs a) {
   for (int o = 32; o > 0; o >>= 1) {
     am = fmaxf(am, __shfl_xor(am, o, 64));
     ws += __shfl_xor(ws, o, 64);
+    wl = fminf(wl, __shfl_xor(wl, o, 64));
+    wh = fmaxf(wh, __shfl_xor(wh, o, 64));
   }
   __syncthreads();
   if ((tid & 63) == 0) {
     mn[tid >> 6] = am;
     mx[tid >> 6] = ws;
+    mn[4 + (tid >> 6)] = wl;
+    mx[4 + (tid >> 6)] = wh;
   }
   __syncthreads();
   if (tid == 0) {
     out[0] = fmaxf(fmaxf(mn[0], mn[1]), fmaxf(mn[2], mn[3]));
     out[1] = (mx[0] + mx[1]) + (mx[2] + mx[3]);
+    out[2] = fminf(fminf(mn[4], mn[5]), fminf(mn[6], mn[7]));
+    out[3] = fmaxf(fmaxf(mx[4], mx[5]), fmaxf(mx[6], mx[7]));
   }
+}
+
+// log2(v) + c for positive v: the exponent joins c before the fraction's logarithm does, so that one
+// rounding is left where v is far from one or the two nearly cancel.
+__device__ __forceinline__ float small_log2(float v, float c) {
+  int e;
+  float f = frexpf(v, &e);
+  const bool low = f < 0.70710678f;
+  f = low ? 2.0f * f : f;
+  return ((float)(low ? e - 1 : e) + c) + __log2f(f);
 }
 
 // The schedules of one item from its bounding boxes (numpy's arange and exp in double, as the
@@ -151,17 +186,21 @@ __device__ void small_schedule(const SmallArgs& a, int item) {
   const int tid = threadIdx.x;
   __shared__ float sq[3];
   __shared__ int len[3];
-  if (a.sched == 0 && a.threshold > 0.f && tid < 3) a.lens[item * 3 + tid] = a.entries;
-  if (a.sched != 1) return;
+  if (a.sched == 0 && tid < 3) {  // one entry stands for all
+    a.lens[item * 3 + tid] = a.full[item * 3 + tid] = a.entries;
+    a.table[((size_t)item * 3 + tid) * kSmallTable] = small_coef(a.cost_scale, a.eps0);
+  }
+  if (a.sched != 1 && !a.pair) return;
   if (tid < 3) sq[tid] = 0.f;
   __syncthreads();
   float r[3] = {0.f, 0.f, 0.f};
   if (tid < a.d) {
     float lo[2] = {3.0e38f, 3.0e38f}, hi[2] = {-3.0e38f, -3.0e38f};
     for (int mat = 0; mat < 2; ++mat)
+#pragma unroll 16
       for (int b = 0; b < kSmallStatBlocks; ++b) {
         const float* st = a.stats + (((size_t)item * 2 + mat) * kSmallStatBlocks + b) * kSmallStatWords;
-        const float l = st[2 + tid], u = st[2 + kSmallMaxD + tid];
+        const float l = st[4 + tid], u = st[4 + kSmallMaxD + tid];
         lo[mat] = (l < lo[mat] || !(l == l)) ? l : lo[mat];
         hi[mat] = (u > hi[mat] || !(u == u)) ? u : hi[mat];
       }
@@ -179,6 +218,29 @@ __device__ void small_schedule(const SmallArgs& a, int item) {
     if ((tid & 63) == 0 && tid < 128) atomicAdd(&sq[p], s);
   }
   __syncthreads();
+  if (a.pair && tid == 0) {
+    float am = 0.f, lim[4];
+    for (int mat = 0; mat < 2; ++mat) {
+      const float* st = a.stats + ((size_t)item * 2 + mat) * kSmallStatBlocks * kSmallStatWords;
+      float ws = 0.f, wl = 3.0e38f, wh = 0.f;
+#pragma unroll 16
+      for (int b = 0; b < kSmallStatBlocks; ++b) {
+        am = fmaxf(am, st[b * kSmallStatWords]);
+        ws += st[b * kSmallStatWords + 1];
+        wl = fminf(wl, st[b * kSmallStatWords + 2]);
+        wh = fmaxf(wh, st[b * kSmallStatWords + 3]);
+      }
+      if (a.w[mat] == nullptr) wl = wh = 1.0f / (float)a.rows[mat];
+      else if (a.normalize) wl /= fmaxf(ws, 1e-40f), wh /= fmaxf(ws, 1e-40f);
+      lim[2 * mat] = wl > 0.f ? small_log2(wl, 0.f) : -100000.0f * kLog2e;
+      lim[2 * mat + 1] = wh > 0.f ? small_log2(wh, 0.f) : -100000.0f * kLog2e;
+    }
+    a.limits[item] = make_float4(lim[0], lim[1], lim[2], lim[3]);
+    // (the diagonal of the joint bounding box bounds every distance)
+    const float far = a.cost_scale * sq[0];
+    a.reach[item] = make_float4(am, far, 2.0f * (far + a.cost_scale * (float)a.d * am * am), 0.f);
+  }
+  if (a.sched != 1) return;
   if (tid < 3) {
     const double D = (double)sqrtf(sq[tid]);
     int k = -2;                      // not a number
@@ -187,7 +249,7 @@ __device__ void small_schedule(const SmallArgs& a, int item) {
       const double start = 2.0 * log(D), stop = 2.0 * log(a.blur), step = 2.0 * log(a.scaling);
       const double cnt = ceil((stop - start) / step);
       const double total = 2.0 + (cnt > 0.0 ? cnt : 0.0);
-      k = total > (double)kSmallTable ? -3 : (int)total;  // -3: longer than the table
+      k = total > (double)(kSmallTable - 1) ? -3 : (int)total;  // -3: longer than the table
       if (k > 0 && a.cut > 0) k = min(k, a.cut);
     }
     len[tid] = k;
@@ -206,9 +268,10 @@ __device__ void small_schedule(const SmallArgs& a, int item) {
     const double start = 2.0 * log(D), stop = 2.0 * log(a.blur), step = 2.0 * log(a.scaling);
     const double cnt = ceil((stop - start) / step);
     const int full = 2 + (cnt > 0.0 ? (int)cnt : 0);
-    for (int i = tid; i < len[p]; i += 256) {
-      const double e = i == 0 ? D * D : (i == full - 1 ? a.blur * a.blur : exp(start + (i - 1) * step));
-      a.table[((size_t)item * 3 + p) * kSmallTable + i] = (float)e;
+    for (int i = tid; i <= len[p]; i += 256) {
+      const int c = min(i, len[p] - 1);
+      const double e = c == 0 ? D * D : (c == full - 1 ? a.blur * a.blur : exp(start + (c - 1) * step));
+      a.table[((size_t)item * 3 + p) * kSmallTable + i] = small_coef(a.cost_scale, (float)e);
     }
   }
 }
@@ -228,14 +291,15 @@ __global__ __launch_bounds__(256) void small_prep_kernel(const SmallArgs a) {
   if (rb >= a.blocks[mat]) return;
   __shared__ float s[32 * LDW];
   const float* st = a.stats + ((size_t)item * 2 + mat) * kSmallStatBlocks * kSmallStatWords;
-  float am = 0.f, ws = 0.f;
+  static_assert(kSmallStatBlocks == 64, "one partial result per lane");
+  float am = st[(tid & 63) * kSmallStatWords], ws = st[(tid & 63) * kSmallStatWords + 1];
 #pragma unroll
-  for (int b = 0; b < kSmallStatBlocks; ++b) {
-    am = fmaxf(am, st[b * kSmallStatWords]);
-    ws += st[b * kSmallStatWords + 1];
+  for (int o = 32; o > 0; o >>= 1) {
+    am = fmaxf(am, __shfl_xor(am, o, 64));
+    ws += __shfl_xor(ws, o, 64);
   }
   const float sc = f16_plane_scale(am);
-  if (rb == 0 && tid == 0) a.scale[item * 2 + mat] = sc;
+  if (rb == 0 && tid == 0) a.scale[item * 2 + mat] = make_float2(sc, 1.0f / sc);
   const int r0 = rb * 32;
   if (d < NDB * 32)
     for (int e = tid; e < 32 * LDW; e += 256) s[e] = 0.f;
@@ -248,7 +312,7 @@ __global__ __launch_bounds__(256) void small_prep_kernel(const SmallArgs a) {
   __syncthreads();
   // planes
   u32x4* po = a.planes[mat] + ((size_t)item * a.blocks[mat] + rb) * (2 * KK * 64);
-  for (int e = tid; e < KK * 64; e += 256) {
+  for (int e = tid; e < KK * 64 && !a.pair; e += 256) {
     const int kk = e >> 6, lane = e & 63;
     const float* v = s + (lane & 31) * LDW + 16 * kk + 8 * (lane >> 5);
     u32x4 hi, lo;
@@ -299,35 +363,11 @@ __global__ __launch_bounds__(256) void small_prep_kernel(const SmallArgs a) {
       float w = a.w[mat] == nullptr ? 1.0f / (float)rows : a.w[mat][at];
       if (a.w[mat] != nullptr && a.normalize) w = w / fmaxf(ws, 1e-40f);
       a.wt[mat][at] = w;
-      a.l2w[mat][at] = w > 0.f ? kLog2e * logf(w) : -100000.0f * kLog2e;
+      a.l2w[mat][at] = w > 0.f ? small_log2(w, 0.f) : -100000.0f * kLog2e;
       a.pot[mat][at] = -al;
       if (a.self) a.pot[2 + mat][at] = -al;
     }
   }
-}
-
-// What a workgroup of the steps (and of the gradient) works on.
-struct SmallSide {
-  int side, rb, qm, km, prob;  // query and key matrix
-};
-
-__device__ __forceinline__ SmallSide small_side(const SmallArgs& a, int bid) {
-  SmallSide s;
-  s.side = 0;
-  if (a.self == 2) bid += a.blocks[0] + a.blocks[1];
-  if (bid >= a.blocks[0] + a.blocks[1]) {
-    bid -= a.blocks[0] + a.blocks[1];
-    s.side = 2;
-  }
-  if (bid >= a.blocks[0]) {
-    bid -= a.blocks[0];
-    s.side += 1;
-  }
-  s.rb = bid;
-  s.qm = s.side & 1;
-  s.km = s.side < 2 ? s.qm ^ 1 : s.qm;
-  s.prob = s.side < 2 ? 0 : s.side - 1;
-  return s;
 }
 
 __device__ __forceinline__ f32x16 small_mfma(const u32x4& x, const u32x4& y, const f32x16& c) {
@@ -335,92 +375,130 @@ __device__ __forceinline__ f32x16 small_mfma(const u32x4& x, const u32x4& y, con
                                                 0, 0);
 }
 
-// Keys of one 32-key block: both planes and the base-2 bias of key li (in accumulator units).
+// Keys of one 32-key block: both planes, and potential and log weight of key li.
 template <int KK>
 struct SmallKeys {
   u32x4 p[2][KK];
-  float bias;
+  float pot, l2w;
 };
 
+// The keys a wavefront streams: everything that does not change from block to block.
 template <int KK>
-__device__ __forceinline__ void small_load_keys(SmallKeys<KK>& k, const u32x4* kp, const float* pot, const float* l2w,
-                                                float kc, float inv_lscale, float masked, int blk, int nk, int lane) {
-  const u32x4* b = kp + (size_t)blk * (2 * KK * 64) + lane;
-#pragma unroll
-  for (int p = 0; p < 2; ++p)
-#pragma unroll
-    for (int kk = 0; kk < KK; ++kk) k.p[p][kk] = b[(p * KK + kk) * 64];
-  const int j = blk * 32 + (lane & 31);
-  const int jc = min(j, nk - 1);
-  const float v = __builtin_fmaf(kc, pot[jc], l2w[jc]);
-  k.bias = j < nk ? fmaxf(v * inv_lscale, masked) : masked;
-}
+struct SmallStream {
+  const u32x4* planes;
+  const float* pot;
+  const float* l2w;
+  int nk, nkb, lane;
+  float kc, raw, masked;  // base 2 per unit of a potential; accumulator units per base-2 unit; bias past the end
 
-// A tile of logits in accumulator units: the three plane products from the lowest weight to
-// hi * hi, then the key bias by one fp32 MFMA.
-template <int KK>
-__device__ __forceinline__ f32x16 small_logits(const SmallKeys<KK>& k, const u32x4 (&q)[2][KK], int h) {
-  f32x16 acc;
+  // (past the last block: the last one again, for nobody)
+  __device__ __forceinline__ void load(SmallKeys<KK>& k, int blk) const {
+    const int b = min(blk, nkb - 1);
+    const u32x4* at = planes + (size_t)b * (2 * KK * 64) + lane;
 #pragma unroll
-  for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+    for (int p = 0; p < 2; ++p)
 #pragma unroll
-  for (int kk = 0; kk < KK; ++kk) acc = small_mfma(k.p[1][kk], q[0][kk], acc);
+      for (int kk = 0; kk < KK; ++kk) k.p[p][kk] = at[(p * KK + kk) * 64];
+    const int j = min(b * 32 + (lane & 31), nk - 1);
+    k.pot = pot[j];
+    k.l2w = l2w[j];
+  }
+  // A tile of logits in accumulator units: the three plane products from the lowest weight to
+  // hi * hi, then the key bias by one fp32 MFMA.  Keys past the last one get a bias of -1e30 in
+  // base 2 (where that can be held); half of it is where a row's maximum starts: above the masked
+  // keys, whose exponentials are then zero (a wavefront may see nothing else), and below every
+  // real logit.
+  __device__ __forceinline__ f32x16 logits(const SmallKeys<KK>& k, const u32x4 (&q)[2][KK], int blk) const {
+    f32x16 acc;
 #pragma unroll
-  for (int kk = 0; kk < KK; ++kk) acc = small_mfma(k.p[0][kk], q[1][kk], acc);
+    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
 #pragma unroll
-  for (int kk = 0; kk < KK; ++kk) acc = small_mfma(k.p[0][kk], q[0][kk], acc);
-  return __builtin_amdgcn_mfma_f32_32x32x2f32(h ? 0.f : k.bias, h ? 0.f : 1.0f, acc, 0, 0, 0);
-}
+    for (int kk = 0; kk < KK; ++kk) acc = small_mfma(k.p[1][kk], q[0][kk], acc);
+#pragma unroll
+    for (int kk = 0; kk < KK; ++kk) acc = small_mfma(k.p[0][kk], q[1][kk], acc);
+#pragma unroll
+    for (int kk = 0; kk < KK; ++kk) acc = small_mfma(k.p[0][kk], q[0][kk], acc);
+    float v = __builtin_fmaf(kc, k.pot, k.l2w) * raw;
+    asm volatile("" : "+v"(v));  // (the loads stay ahead of the select below, which is not a branch)
+    const float bias = (blk * 32 + (lane & 31) < nk) ? fmaxf(v, masked) : masked;
+    const bool h = lane >= 32;
+    return __builtin_amdgcn_mfma_f32_32x32x2f32(h ? 0.f : bias, h ? 0.f : 1.0f, acc, 0, 0, 0);
+  }
+};
 
-__device__ __forceinline__ float small_max16(const f32x16& a) {
-  float m = fmaxf(a[0], a[1]);
+__device__ __forceinline__ float small_max16(float m, const f32x16& a) {
 #pragma unroll
-  for (int r = 2; r < 16; r += 2) m = fmaxf(m, fmaxf(a[r], a[r + 1]));
+  for (int r = 0; r < 16; r += 2) m = fmaxf(fmaxf(m, a[r]), a[r + 1]);
   return m;
 }
 
-// Bias of a key past the last one, in accumulator units: -1e30 in base 2 where that can be held.
-// A row's maximum starts at half of it: above the masked keys, whose exponentials are then zero
-// (a wavefront may see nothing else), and below every real logit.
-__device__ __forceinline__ float small_masked(float inv_lscale) { return fmaxf(kNegBig * inv_lscale, -3.0e38f); }
+// What one step of one side needs, laid out so that a workgroup has it after one round of
+// argument loads (pointers of item 0).
+struct SmallStepSide {
+  const u32x4* kplanes;
+  const u32x4* qplanes;
+  const float* kpot;   // potentials of the keys
+  const float* kl2w;
+  const float4* coef;  // of this step's entry; the items' are 3 * kSmallTable apart
+  const int* lens;     // the items' are 3 apart
+  const float* old;    // this side's potentials, before ...
+  float* out;          // ... and behind the step
+  const float* norm;
+  int nq, nk, nqb, nkb;
+  float rho;
+  int qm, km;          // which of the two matrices: query and key rows
+};
+struct SmallStepArgs {
+  SmallStepSide side[4];
+  const float4* scale;  // [items] scale of x, its inverse, scale of y, its inverse
+  int step, extrapolate;
+};
 
-// One step of every problem.
+// One step of every problem.  Grid (32-row blocks of the larger cloud, sides, items).
+// At these sizes the kernel is bound by the chain of memory round trips in front of its first
+// logits and by the vector pipe behind it, so everything the first loads need comes from the
+// kernel arguments, what the first logits need (coefficients, scales) arrives beside the keys,
+// and the products of the next block run under the exponentials of the one before.
 template <int DP, int W>
-__global__ __launch_bounds__(64 * W) void small_step_kernel(const SmallArgs a, int step) {
+__global__ __launch_bounds__(64 * W) void small_step_kernel(const SmallStepArgs a) {
   constexpr int KK = DP / 16;
-  const int item = blockIdx.y;
-  const SmallSide sd = small_side(a, blockIdx.x);
-  const int entries = small_entries(a, item, sd.prob);
-  if (step > entries + a.extrapolate) return;  // this problem's schedule is shorter
-  // (a problem that stopped early still extrapolates at the schedule's last eps)
-  const float eps = small_eps(a, item, sd.prob,
-                              step > entries ? small_full_entries(a, item, sd.prob) - 1 : max(step - 1, 0));
-  const float alpha = (step == 0 || step > entries) ? 1.0f : 0.5f;
-  const int nq = a.rows[sd.qm], nk = a.rows[sd.km], nkb = a.blocks[sd.km];
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, li = lane & 31, h = lane >> 5;
-  const float lscale = 2.0f * a.cost_scale / eps * kLog2e / (a.scale[item * 2 + sd.qm] * a.scale[item * 2 + sd.km]);
-  const float inv_lscale = 1.0f / lscale, masked = small_masked(inv_lscale), no_max = 0.5f * masked * lscale;
-  const float kc = kLog2e / eps;
-  const int kside = sd.side < 2 ? sd.side ^ 1 : sd.side;
-  const float* kpot = a.pot[kside] + ((size_t)(step & 1) * a.items + item) * nk;
-  const float* kl2w = a.l2w[sd.km] + (size_t)item * nk;
-  const u32x4* kp = a.planes[sd.km] + (size_t)item * nkb * (2 * KK * 64);
+  const SmallStepSide& sd = a.side[blockIdx.y];
+  const int rb = blockIdx.x, item = blockIdx.z;
+  const int nq = sd.nq, nk = sd.nk, nkb = sd.nkb, qm = sd.qm, km = sd.km;
+  if (rb >= sd.nqb) return;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
 
+  SmallStream<KK> ks;
+  ks.planes = sd.kplanes + (size_t)item * nkb * (2 * KK * 64);
+  ks.pot = sd.kpot + (size_t)item * nk;
+  ks.l2w = sd.kl2w + (size_t)item * nk;
+  ks.nk = nk;
+  ks.nkb = nkb;
+  ks.lane = lane;
   SmallKeys<KK> kr;
-  if (wave < nkb) small_load_keys(kr, kp, kpot, kl2w, kc, inv_lscale, masked, wave, nk, lane);
+  ks.load(kr, wave);
   u32x4 q[2][KK];
   {
-    const u32x4* b = a.planes[sd.qm] + ((size_t)item * a.blocks[sd.qm] + sd.rb) * (2 * KK * 64) + lane;
+    const u32x4* b = sd.qplanes + ((size_t)item * sd.nqb + rb) * (2 * KK * 64) + lane;
 #pragma unroll
     for (int p = 0; p < 2; ++p)
 #pragma unroll
       for (int kk = 0; kk < KK; ++kk) q[p][kk] = b[(p * KK + kk) * 64];
   }
-  float m = no_max, s = 0.f;
-  for (int blk = wave; blk < nkb; blk += W) {
-    const f32x16 acc = small_logits(kr, q, h);
-    if (blk + W < nkb) small_load_keys(kr, kp, kpot, kl2w, kc, inv_lscale, masked, blk + W, nk, lane);
-    const float mn = fmaxf(m, small_max16(acc) * lscale);
+  const int entries = sd.lens[item * 3];
+  const float4 coef = sd.coef[(size_t)item * 3 * kSmallTable];
+  const float4 sc = a.scale[item];
+  const float lscale = coef.y * (qm ? sc.w : sc.y) * (km ? sc.w : sc.y);
+  ks.kc = coef.w;
+  ks.raw = coef.z * (qm ? sc.z : sc.x) * (km ? sc.z : sc.x);
+  ks.masked = fmaxf(kNegBig * ks.raw, -3.0e38f);
+
+  float mr = 0.5f * ks.masked, m = mr * lscale, s = 0.f;  // the running maximum, raw and base 2
+  const float no_max = m;
+  auto soft = [&](const f32x16& acc) {
+    mr = small_max16(mr, acc);
+    float mn = mr * lscale;
+    asm("" : "+v"(mn));  // (rounded once: an unchanged maximum has to give a factor of exactly one)
     s *= fast_exp2(m - mn);
     m = mn;
     float p0 = 0.f, p1 = 0.f;
@@ -430,13 +508,33 @@ __global__ __launch_bounds__(64 * W) void small_step_kernel(const SmallArgs a, i
       p1 += fast_exp2(__builtin_fmaf(acc[r + 1], lscale, -m));
     }
     s += p0 + p1;
+  };
+  if (wave < nkb) {
+    f32x16 acc0 = ks.logits(kr, q, wave), acc1;
+    ks.load(kr, wave + W);
+    for (int blk = wave;; blk += 2 * W) {
+      if (blk + W < nkb) {
+        acc1 = ks.logits(kr, q, blk + W);
+        ks.load(kr, blk + 2 * W);
+      }
+      soft(acc0);
+      if (blk + W >= nkb) break;
+      if (blk + 2 * W < nkb) {
+        acc0 = ks.logits(kr, q, blk + 2 * W);
+        ks.load(kr, blk + 3 * W);
+      }
+      soft(acc1);
+      if (blk + 2 * W >= nkb) break;
+    }
   }
   // ---- the row's statistics over the wavefronts and half-waves ----
   __shared__ float2 sh[W][64];
   sh[wave][lane] = make_float2(m, s);
+  const int row = rb * 32 + tid, step = a.step;
+  const size_t at = (size_t)item * nq + min(row, nq - 1);
+  const float old = sd.old[at], shift = sd.norm[at];
   __syncthreads();
-  const int row = sd.rb * 32 + tid;
-  if (tid >= 32 || row >= nq) return;
+  if (tid >= 32 || row >= nq || step > entries + a.extrapolate) return;  // (its schedule is shorter)
   float M = no_max, S = 0.f;
 #pragma unroll
   for (int w = 0; w < W; ++w) M = fmaxf(M, fmaxf(sh[w][tid].x, sh[w][tid + 32].x));
@@ -445,13 +543,13 @@ __global__ __launch_bounds__(64 * W) void small_step_kernel(const SmallArgs a, i
     const float2 u = sh[w][tid], v = sh[w][tid + 32];
     S += u.y * fast_exp2(u.x - M) + v.y * fast_exp2(v.x - M);
   }
-  const float rho = a.rho[sd.qm];
+  const float eps = coef.x, rho = sd.rho;
   const float damp = rho > 0.f ? 1.0f / (1.0f + eps / rho) : 1.0f;
-  const size_t half = (size_t)a.items * nq, at = (size_t)item * nq + row;
-  float r = alpha * (-eps * damp * kLn2 * (M + log2f(fmaxf(S, 1e-40f))));
-  if (alpha != 1.0f) r += (1.0f - alpha) * a.pot[sd.side][(step & 1) * half + at];
-  if (damp < 1.0f) r -= alpha * (1.0f - damp) * a.norm[sd.qm][at];
-  a.pot[sd.side][((step & 1) ^ 1) * half + at] = r;
+  const float alpha = (step == 0 || step > entries) ? 1.0f : 0.5f;
+  float r = alpha * (-eps * damp * kLn2 * small_log2(fmaxf(S, 1e-40f), M));
+  if (alpha != 1.0f) r += (1.0f - alpha) * old;
+  if (damp < 1.0f) r -= alpha * (1.0f - damp) * shift;
+  sd.out[at] = r;
 }
 
 // Convergence check behind averaged step `step` (the check_every-th since the last check): a
@@ -492,17 +590,24 @@ __global__ __launch_bounds__(1024) void small_check_kernel(const SmallArgs a, in
       for (int i = tid; i < rows; i += 1024) prev[i] = now[i];
     }
   if (tid == 0) {
-    if (stop) a.lens[item * 3 + prob] = step;
+    if (stop) {
+      a.lens[item * 3 + prob] = step;
+      // (the extrapolation, next, takes the schedule's last eps)
+      if (a.sched != 0)
+        a.table[((size_t)item * 3 + prob) * kSmallTable + step] = small_last_coef(a, item, prob);
+    }
     __hip_atomic_store(a.host_words + item * 4 + prob, 2 * check + (stop ? 1 : 0), __ATOMIC_RELAXED,
                        __HIP_MEMORY_SCOPE_SYSTEM);
   }
 }
 
 // The loss of every item, and the standard potentials (of the last step, and of the one before
-// when there was an extrapolation) of every side.  One workgroup per item.
+// when there was an extrapolation) of every side.  Grid (parts, items): a part takes every
+// parts-th run of 1024 rows; several parts leave their sums to small_loss_sum_kernel.
 // pots: per side and kind (0: of the cost, 1: of the gradient) [items][rows], in that order.
 struct SmallLossArgs {
   float* loss;        // [items] or null
+  float* parts;       // [items][parts], where there are several
   float* pots;        // or null
   int relaxed;        // both marginals relaxed: the other cost formula
 };
@@ -516,8 +621,8 @@ __global__ __launch_bounds__(1024) void small_loss_kernel(const SmallArgs a, con
   for (int side = a.self == 2 ? 2 : 0; side < sides; ++side) {
     const int mat = side & 1, rows = a.rows[mat];
     const int prob = side < 2 ? 0 : side - 1;
-    const int entries = small_entries(a, item, prob), last = entries + 1 + a.extrapolate;
-    const float eps_last = small_eps(a, item, prob, small_full_entries(a, item, prob) - 1);
+    const int last = a.lens[item * 3 + prob] + 1 + a.extrapolate;
+    const float eps_last = small_last_coef(a, item, prob).x;
     const size_t half = (size_t)a.items * rows;
     const float rho = a.rho[mat];
     // (a self problem has this potential twice: its cost is 2 <a, f>)
@@ -547,8 +652,18 @@ __global__ __launch_bounds__(1024) void small_loss_kernel(const SmallArgs a, con
     float t = 0.f;
 #pragma unroll
     for (int w = 0; w < 16; ++w) t += sh[w];
-    l.loss[item] = t;
+    if (gridDim.x == 1) l.loss[item] = t;
+    else l.parts[(size_t)item * gridDim.x + part] = t;
   }
+}
+
+template <int T>
+__global__ __launch_bounds__(64) void small_loss_sum_kernel(const SmallLossArgs l, int parts) {
+  float t = 0.f;
+  for (int i = threadIdx.x; i < parts; i += 64) t += l.parts[(size_t)blockIdx.x * parts + i];
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) t += __shfl_xor(t, o, 64);
+  if (threadIdx.x == 0) l.loss[blockIdx.x] = t;
 }
 
 // Gradients of the loss in x and y at the potentials before the extrapolation.  A workgroup owns
@@ -567,22 +682,12 @@ __global__ __launch_bounds__(512, 2) void small_grad_kernel(const SmallArgs a, c
   constexpr int PER = NDB * 32 * 32 / 512;          // outputs per thread
   __shared__ __attribute__((aligned(16))) float sh_o[W][32 * LDW];
   __shared__ float2 sh_ms[W][32];
-  const int item = blockIdx.y, tid = threadIdx.x;
-  const int wave = tid >> 6, lane = tid & 63, li = lane & 31, h = lane >> 5;
-  int rb = blockIdx.x, qm = 0;
-  if (g.out[0] == nullptr || rb >= a.blocks[0]) {
-    rb -= g.out[0] == nullptr ? 0 : a.blocks[0];
-    qm = 1;
-  }
+  const int rb = blockIdx.x, item = blockIdx.z, tid = threadIdx.x;
+  const int qm = g.out[0] == nullptr ? 1 : blockIdx.y;
+  if (rb >= a.blocks[qm]) return;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, li = lane & 31, h = lane >> 5;
   const int nq = a.rows[qm], d = a.d;
   u32x4 q[2][KK];
-  {
-    const u32x4* b = a.planes[qm] + ((size_t)item * a.blocks[qm] + rb) * (2 * KK * 64) + lane;
-#pragma unroll
-    for (int p = 0; p < 2; ++p)
-#pragma unroll
-      for (int kk = 0; kk < KK; ++kk) q[p][kk] = b[(p * KK + kk) * 64];
-  }
   float bary[PER];
 #pragma unroll
   for (int i = 0; i < PER; ++i) bary[i] = 0.f;
@@ -592,14 +697,36 @@ __global__ __launch_bounds__(512, 2) void small_grad_kernel(const SmallArgs a, c
     const int kside = pass == 0 ? km : 2 + km;
     const int prob = pass == 0 ? 0 : 1 + km;
     const int nk = a.rows[km], nkb = a.blocks[km];
-    const int last = small_entries(a, item, prob) + 1;  // (the step before the extrapolation)
-    const float eps = small_eps(a, item, prob, small_full_entries(a, item, prob) - 1);
-    const float lscale = 2.0f * a.cost_scale / eps * kLog2e / (a.scale[item * 2 + qm] * a.scale[item * 2 + km]);
-    const float inv_lscale = 1.0f / lscale, kc = kLog2e / eps;
-    const float masked = small_masked(inv_lscale), no_max = 0.5f * masked * lscale;
-    const float* kpot = a.pot[kside] + ((size_t)(last & 1) * a.items + item) * nk;
-    const float* kl2w = a.l2w[km] + (size_t)item * nk;
-    const u32x4* kp = a.planes[km] + (size_t)item * nkb * (2 * KK * 64);
+    const int last = a.lens[item * 3 + prob] + 1;  // (the step before the extrapolation)
+    const float4 coef = small_last_coef(a, item, prob);
+    const float2 sq = a.scale[item * 2 + qm], sk = a.scale[item * 2 + km];
+    const u32x4* qp = pass == 0 || a.self_planes[qm] == nullptr ? a.planes[qm] : a.self_planes[qm];
+    const u32x4* kp = pass == 0 || a.self_planes[km] == nullptr ? a.planes[km] : a.self_planes[km];
+    if (pass == 0 || qp != a.planes[qm]) {
+      const u32x4* b = qp + ((size_t)item * a.pblocks[qm] + rb) * (2 * KK * 64) + lane;
+#pragma unroll
+      for (int p = 0; p < 2; ++p)
+#pragma unroll
+        for (int kk = 0; kk < KK; ++kk) q[p][kk] = b[(p * KK + kk) * 64];
+    }
+    float lscale = coef.y * sq.y * sk.y, raw = coef.z * sq.x * sk.x;
+    if (a.pair) {  // (see pair_scale)
+      const float most = a.reach[item].x, ps = f16_plane_scale(most);
+      const bool root = most * sqrtf(coef.y) < 30000.f;
+      lscale = root ? 1.0f : coef.y / (ps * ps);
+      raw = root ? 1.0f : coef.z * (ps * ps);
+    }
+    SmallStream<KK> ks;
+    ks.planes = kp + (size_t)item * a.pblocks[km] * (2 * KK * 64);
+    ks.pot = a.pot[kside] + ((size_t)(last & 1) * a.items + item) * nk;
+    ks.l2w = a.l2w[km] + (size_t)item * nk;
+    ks.nk = nk;
+    ks.nkb = nkb;
+    ks.lane = lane;
+    ks.kc = coef.w;
+    ks.raw = raw;
+    ks.masked = fmaxf(kNegBig * ks.raw, -3.0e38f);
+    const float no_max = 0.5f * ks.masked * lscale;
     const u32x4* vp = a.values[km] + (size_t)item * nkb * (NDB * 4 * 64) + lane;
 
     float m = no_max, s = 0.f;
@@ -609,13 +736,13 @@ __global__ __launch_bounds__(512, 2) void small_grad_kernel(const SmallArgs a, c
 #pragma unroll
       for (int r = 0; r < 16; ++r) o[cb][r] = 0.f;
     SmallKeys<KK> kr;
-    if (wave < nkb) small_load_keys(kr, kp, kpot, kl2w, kc, inv_lscale, masked, wave, nk, lane);
+    ks.load(kr, wave);
     for (int blk = wave; blk < nkb; blk += W) {
       const u32x4* v = vp + (size_t)blk * (NDB * 4 * 64);
-      const f32x16 acc = small_logits(kr, q, h);
-      if (blk + W < nkb) small_load_keys(kr, kp, kpot, kl2w, kc, inv_lscale, masked, blk + W, nk, lane);
+      const f32x16 acc = ks.logits(kr, q, blk);
+      if (blk + W < nkb) ks.load(kr, blk + W);
       // the two half-waves of a column feed one sum: they share its maximum
-      float mx = small_max16(acc) * lscale;
+      float mx = small_max16(ks.masked, acc) * lscale;
       mx = fmaxf(mx, xor32(mx));
       if (wave_any(mx > m)) {
         const float mn = fmaxf(m, mx);
@@ -674,7 +801,7 @@ __global__ __launch_bounds__(512, 2) void small_grad_kernel(const SmallArgs a, c
         *reinterpret_cast<float4*>(&sh_o[wave][li * LDW + 32 * cb + 8 * c + 4 * h]) =
             make_float4(o[cb][4 * c] * fac, o[cb][4 * c + 1] * fac, o[cb][4 * c + 2] * fac, o[cb][4 * c + 3] * fac);
     __syncthreads();
-    const float inv_v = 1.0f / a.scale[item * 2 + km];
+    const float inv_v = sk.y;
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
       const int e = tid + 512 * i, row = e / (NDB * 32), col = e % (NDB * 32);

@@ -199,7 +199,9 @@ def sinkhorn_flashstyle_symmetric(
     # are the general path's)
     if (fused is not False and not use_labels and solve_info is None
             and f_init is None and g_init is None
-            and _small.solver_problem(x, y, a, b, allow_tf32)):
+            and _small.solver_problem(x, y, a, b, allow_tf32,
+                                      eps_list is None and not use_epsilon_scaling,
+                                      threshold is not None and threshold > 0.0)):
         out = _small_symmetric(x, y, a, b, blur, scaling, use_epsilon_scaling, last_extrapolation,
                                cost_scale, eps, n_iters, diameter, eps_list, rho_x, rho_y,
                                threshold, check_every, return_n_iters, return_prelast)
@@ -396,8 +398,8 @@ def _small_symmetric(x, y, a, b, blur, scaling, use_epsilon_scaling, last_extrap
             return None
         sched = dict(eps_list=eps_list)
     try:
-        s = _small.solve(*_small.points(x, y), _f32c(a.detach()), _f32c(b.detach()), items=1, cost_scale=float(cost_scale), rho_x=rho_x,
-                         rho_y=rho_y, normalize=False, self_terms=False, want_values=False,
+        s = _small.solve(*_small.points(x, y), _f32c(a.detach()), _f32c(b.detach()), items=1,
+                         cost_scale=float(cost_scale), rho_x=rho_x, rho_y=rho_y, normalize=False, self_terms=False, want_values=False,
                          extrapolate=last_extrapolation, want_loss=False, threshold=threshold,
                          check_every=check_every, **sched)
     except _small.LongSchedule:
@@ -472,7 +474,7 @@ def sinkhorn_flashstyle_symmetric_self_pair(
             raise ValueError("eps_list must be non-empty")
         return lst
 
-    if _small.pair_problem(x, y, a, b, allow_tf32):
+    if _small.pair_problem(x, y, a, b, allow_tf32, not use_epsilon_scaling, self_terms=2):
         out = _small_self_pair(x, a, y, b, blur, scaling, use_epsilon_scaling, last_extrapolation,
                                cost_scale, eps, n_iters, rho, return_prelast)
         if out is not None:

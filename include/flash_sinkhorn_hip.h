@@ -415,7 +415,7 @@ int fs_c_transform(const float* x, const float* y, const float* bias, float* min
  * step was run).  Replaces sinkhorn_flashstyle_symmetric (sinkhorn_solvers.py:290-707) and the
  * three solves of a debiased SamplesLoss (samples_loss.py:494-512) for these sizes.
  */
-#define FS_SMALL_MAX_ROWS 16384
+#define FS_SMALL_MAX_ROWS 65536
 #define FS_SMALL_NO_DIAMETER 1    /* a cloud is a single point */
 #define FS_SMALL_NOT_A_NUMBER 2   /* a coordinate is not finite */
 #define FS_SMALL_LONG_SCHEDULE 3  /* more entries than the device table holds */
