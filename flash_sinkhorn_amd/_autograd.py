@@ -134,7 +134,7 @@ class _SinkhornCostFn(torch.autograd.Function):
             f_grad, g_grad = f_cost, g_cost
             balanced_formula = True
         else:
-            info = {}
+            info = {} if x.shape[1] <= 128 else None  # (wide rows: no tile tests, nothing to ask for)
             out = sinkhorn_flashstyle_symmetric(
                 x, y, a, b, solve_info=info, blur=config.blur, scaling=config.scaling,
                 use_epsilon_scaling=config.use_epsilon_scaling, eps=config.eps,
@@ -154,7 +154,7 @@ class _SinkhornCostFn(torch.autograd.Function):
             balanced_formula = config.rho_x is None or config.rho_y is None
             # the keys behind the rows' largest logits, where the solve kept them: a hint from
             # which the gradient's sweep recognises the tiles that cannot matter
-            prep = info.get("prepared")
+            prep = None if info is None else info.get("prepared")
             if prep is not None and info.get("coarse"):
                 kx, ky = prep.best_keys(0), prep.best_keys(1)
                 if kx is not None and ky is not None:

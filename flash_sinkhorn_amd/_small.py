@@ -25,8 +25,9 @@ _P, _I64, _D, _F, _I = (ctypes.c_void_p, ctypes.c_int64, ctypes.c_double, ctypes
                         ctypes.c_int)
 _DTYPES = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}
 
-MAX_D = 128
 MAX_ROWS = 65536
+WIDE_D = 128  # from here on the products of the clouds are kept (fs_dense.hpp), at most this many:
+MAX_KEPT = 1 << 28
 _TABLE = 511  # entries of a schedule the device keeps
 
 
@@ -72,8 +73,12 @@ class Solved:
         return tuple(self.pots[at + i * size:at + (i + 1) * size].view(p.items, rows) for i in (0, 1))
 
 
-def _size_ok(n: int, m: int, d: int, fixed: bool, self_terms: int, stops: bool) -> bool:
+def _size_ok(n: int, m: int, d: int, fixed: bool, self_terms: int, stops: bool,
+             items: int = 1) -> bool:
     """Whether a problem of this size is faster here than on the general path, launch by launch.
+
+    d > 128: while the kept products stay below 1 GiB; reading them beats forming them at every such
+    width (8,192 x 1,536: 0.07 against 0.5 ms a step).
 
     d <= 64 (``pair_sweep_kernel`` from 2e7 logits per step on): everywhere but where two large
     clouds let the general path skip tiles by its coarse product, from 24,000 rows on.  At fixed
@@ -85,8 +90,10 @@ def _size_ok(n: int, m: int, d: int, fixed: bool, self_terms: int, stops: bool) 
     side: up to 2e7 logits at fixed eps (3,000 x 128: 1.05 against 1.54 ms; 4,500: 2.8 against 2.4),
     6e7 on a schedule (6,500 x 128: 1.54 against 1.94 ms; 9,000: 3.1 against 2.8).
     """
-    if not (0 < n <= MAX_ROWS and 0 < m <= MAX_ROWS and 0 < d <= MAX_D):
+    if not (0 < n <= MAX_ROWS and 0 < m <= MAX_ROWS and 0 < d):
         return False
+    if d > WIDE_D:
+        return not self_terms and items * n * m <= MAX_KEPT
     if d > 64 or (stops and not fixed):
         logits = (n * m if self_terms < 2 else 0) + ((n * n + m * m) // 2 if self_terms else 0)
         return logits <= (20_000_000 if fixed else 60_000_000)
@@ -149,7 +156,8 @@ def solve(x, y, a, b, *, items: int, blur: float = 0.0, scaling: float = 0.0, ep
         _lib.check(rc, "fs_small_solve")
         return ws, out
 
-    if sched == 0 and not threshold and _graphs.eligible(n, m, entries, x.device):
+    if (sched == 0 and not threshold and _graphs.eligible(n, m, entries, x.device)
+            and (d <= WIDE_D or items * n * m <= 1 << 22)):  # (a graph keeps its products)
         # a fixed sequence of kernels on fixed shapes: replayed (1.9 instead of 3 us per launch)
         key = ("self pair" if self_terms else "symmetric", int(self_terms), x.device.index, x.dtype, items, n, m, d,
                eps, entries, cost_scale, _rho(rho_x), _rho(rho_y), a is None, b is None, normalize,
@@ -194,10 +202,10 @@ def pair_problem(x, y, a, b, allow_tf32: bool, fixed: bool, self_terms: int = 0,
 
 def solver_problem(x, y, a, b, allow_tf32: bool, fixed: bool, stops: bool) -> bool:
     """Whether ``sinkhorn_flashstyle_symmetric`` may hand its clouds and weights to ``solve``.  One cloud
-    against itself, on more than a few thousand points, stays with the general path: one
-    half-update per step instead of two, and f equal to g to the bit."""
+    against itself, with wide rows or on more than a few thousand points, stays with the general
+    path: one half-update per step instead of two, and f equal to g to the bit."""
     if x.data_ptr() == y.data_ptr() and a.data_ptr() == b.data_ptr() and x.shape == y.shape \
-            and x.shape[0] ** 2 >= 20_000_000:
+            and (x.shape[1] > WIDE_D or x.shape[0] ** 2 >= 20_000_000):
         return False
     return pair_problem(x, y, a, b, allow_tf32, fixed, 0, stops) and not (
         torch.is_grad_enabled()
@@ -257,8 +265,11 @@ def loss_problem(loss, args, label_x, label_y):
             or x.shape[:-2] != y.shape[:-2]:
         return None
     if not _size_ok(x.shape[-2], y.shape[-2], x.shape[-1], not loss.use_epsilon_scaling,
-                    int(loss.debias and not loss.potentials), loss.threshold is not None):
+                    int(loss.debias and not loss.potentials), loss.threshold is not None,
+                    x.shape[0] if x.ndim == 3 else 1):
         return None
+    if x.shape[-1] > WIDE_D and (loss.use_epsilon_scaling or not loss.potentials):
+        return None  # (by the solver alone: neither cost, gradients nor diameters are built for it)
     lead = x.shape[:-2]
     if lead and not 0 < lead[0] <= 65535:
         return None

@@ -10,6 +10,9 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+#include <utility>
+
 #include "flash_sinkhorn_hip.h"
 
 #ifndef FS_SETTLE
@@ -451,6 +454,25 @@ __device__ __forceinline__ float f16_plane_scale(float mx) {
 __device__ __forceinline__ unsigned pack_f16(float a, float b) {
   f32x2 v = {a, b};
   return __builtin_bit_cast(unsigned, __builtin_convertvector(v, f16x2));
+}
+
+// f(integral_constant<int, 0>{}), ..., f(integral_constant<int, N - 1>{}) in order
+template <int... I, class F>
+__device__ __forceinline__ void static_for_impl(std::integer_sequence<int, I...>, F&& f) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void static_for(F&& f) {
+  static_for_impl(std::make_integer_sequence<int, N>{}, f);
+}
+
+// 16 bytes from LDS at byte address addr + OFF (OFF < 65536), not visible to the compiler's
+// wait-count insertion: the consumer must sit behind an explicit wait
+template <int OFF>
+__device__ __forceinline__ u32x4 lds_read16(unsigned addr) {
+  u32x4 v;
+  asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(OFF) : "memory");
+  return v;
 }
 
 }  // namespace fs

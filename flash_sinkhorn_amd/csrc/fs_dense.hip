@@ -1,0 +1,83 @@
+// Planning and launches of the kernels in fs_dense.hpp.
+#include "fs_dense.hpp"
+
+#include <algorithm>
+#include <cmath>
+
+namespace fs {
+namespace {
+
+template <int WR, int WC, int RB, int CB>
+int launch_gemm(DenseGemmArgs& g, int items, hipStream_t st) {
+  g.row_tiles = (g.rows + 32 * WR * RB - 1) / (32 * WR * RB);
+  g.col_tiles = g.ld / (32 * WC * CB);
+  const int tiles = g.row_tiles * g.col_tiles;
+  hipLaunchKernelGGL((dense_gemm_kernel<WR, WC, RB, CB>), dim3((tiles + 7) / 8 * 8, items), dim3(64 * WR * WC), 0, st, g);
+  return hipGetLastError() == hipSuccess ? FS_OK : FS_ERR_LAUNCH_FAILED;
+}
+
+// Tiles of 256, 128 or 64 rows and columns: the one whose rounds over the chip cost least, a
+// workgroup of the smaller ones taking longer per product (operands are read more often).
+int gemm(DenseGemmArgs& g, int items, hipStream_t st) {
+  auto cost = [&](int side, int at_once, double per) {
+    const double tiles = (double)items * std::ceil(g.rows / (double)side) * std::ceil(g.ld / (double)side);
+    return std::ceil(tiles / (256.0 * at_once)) * at_once * per * side * side;
+  };
+  const double big = cost(256, 1, 1.0), mid = cost(128, 2, 1.25), tiny = cost(64, 4, 2.0);
+  if (big <= mid && big <= tiny) return launch_gemm<2, 4, 4, 2>(g, items, st);
+  if (mid <= tiny) return launch_gemm<2, 2, 2, 2>(g, items, st);
+  return launch_gemm<2, 2, 1, 1>(g, items, st);
+}
+
+}  // namespace
+
+void dense_plan(const SmallArgs& a, DenseArgs& t) {
+  t.n = a.rows[0];
+  t.m = a.rows[1];
+  t.items = a.items;
+  for (int i = 0; i < 2; ++i) t.blocks[i] = (a.rows[i] + 255) / 256 * 8;
+  t.ld = t.blocks[1] * 32;
+  t.steps = (a.d + 15) / 16;
+  // enough workgroups for two on every CU, each over as long a run of columns as that leaves;
+  // below that smaller ones, over 256 columns
+  const int iters = t.ld / 256, groups = (t.n + 63) / 64;
+  t.large = (double)a.items * groups * iters >= 512.0;
+  t.groups = t.large ? groups : (t.n + 31) / 32;
+  const int run = t.large ? (int)std::min<double>(iters, std::floor((double)a.items * groups * iters / 512.0)) : 1;
+  t.chunk = run * 256;
+  t.chunks = (iters + run - 1) / run;
+}
+
+int dense_prepare(const SmallArgs& a, const DenseArgs& t, hipStream_t st) {
+  hipLaunchKernelGGL((dense_stats_kernel<0>), dim3(kSmallStatBlocks, 2, a.items), dim3(1024), 0, st, a);
+  hipLaunchKernelGGL((dense_prep_kernel<0>), dim3(std::max(t.blocks[0], t.blocks[1]) + 1, 2, a.items), dim3(512), 0, st,
+                     a, t);
+  if (hipGetLastError() != hipSuccess) return FS_ERR_LAUNCH_FAILED;
+  DenseGemmArgs g;
+  g.a = t.planes[0];
+  g.b = t.planes[1];
+  g.a_blocks = t.blocks[0];
+  g.b_blocks = t.blocks[1];
+  g.steps = t.steps;
+  g.rows = t.n;
+  g.ld = t.ld;
+  g.scale = a.scale;
+  g.out = t.dots;
+  return gemm(g, a.items, st);
+}
+
+int dense_step(const SmallArgs& a, DenseArgs& t, int step, hipStream_t st) {
+  t.step = step;
+  for (int i = 0; i < 2; ++i) {
+    const size_t half = (size_t)a.items * a.rows[i];
+    t.pot[i] = a.pot[i] + (step & 1) * half;
+    t.out[i] = a.pot[i] + ((step & 1) ^ 1) * half;
+  }
+  const dim3 grid(t.groups, t.chunks, a.items);
+  if (t.large) hipLaunchKernelGGL((dense_sweep_kernel<8, 8>), grid, dim3(512), 0, st, t);
+  else hipLaunchKernelGGL((dense_sweep_kernel<8, 4>), grid, dim3(256), 0, st, t);
+  hipLaunchKernelGGL((dense_merge_kernel<0>), dim3((std::max(t.n, t.m) + 63) / 64, 2, a.items), dim3(256), 0, st, t);
+  return hipGetLastError() == hipSuccess ? FS_OK : FS_ERR_LAUNCH_FAILED;
+}
+
+}  // namespace fs

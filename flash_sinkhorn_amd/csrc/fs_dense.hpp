@@ -1,0 +1,424 @@
+// Symmetric steps on the kept matrix of inner products, for wide rows.
+//
+// A step evaluates n m logits.  Formed anew each costs 3 d matrix-core multiply-adds (two fp16 planes a
+// side), kept it costs reading four bytes: from a few hundred columns on reading wins, at
+// 8192 x 8192 x 1536 by six (495 us for a one-sweep step that forms them, about 70 for one that reads
+// 268 MB).  So the products x_i.y_j are formed once per solve, in the same two-plane arithmetic, and
+// kept as fp32 [n][ld]; 288 GB of HBM hold them many times over, and up to 256 MB of them stay
+// in the last-level cache between steps.  Three kernels:
+//   dense_gemm_kernel   C = A B^T on two-plane operands in MFMA order
+//   dense_sweep_kernel  both half-updates' soft-max statistics from one reading of the products
+//   dense_merge_kernel  the new potentials from them
+#pragma once
+
+#include "fs_common.hpp"
+#include "fs_small.hpp"
+
+namespace fs {
+
+// Planes in operand order, hi and lo next to each other: per 32 rows and 16 columns two blocks of
+// 64 16-byte words, word (h, row % 32) holding columns 8 h .. 8 h + 7.
+constexpr int kDenseStep = 2 * 64;
+
+struct DenseArgs {
+  float* dots;             // [items][n][ld], ld a multiple of 256, zero beyond the m-th column
+  u32x4* planes[2];        // [items][blocks][steps][2][64]
+  int blocks[2];           // 32-row blocks, a multiple of 8 (zero rows behind the last one)
+  int steps;               // 16-column steps
+  int n, m, ld, items, chunk, chunks, groups;
+  float2* part[2];         // (maximum, sum): [items][chunks][n] of the rows, [items][groups][m] of the columns
+  const float* pot[2];     // this step's potentials, log weights, norms
+  float* out[2];
+  const float* l2w[2];
+  const float* norm[2];
+  const float4* table;
+  const int* lens;
+  float rho[2];
+  int step, sched, extrapolate;
+  int large;               // the shape of dense_sweep_kernel
+};
+
+// Eight consecutive elements as floats; `wide`: by whole 16-byte words.
+__device__ __forceinline__ void dense_load8(float (&v)[8], const void* p, size_t at, int dtype, bool wide) {
+  if (wide && dtype == 0) {
+    const float4* q = reinterpret_cast<const float4*>(static_cast<const float*>(p) + at);
+    const float4 u = q[0], w = q[1];
+    v[0] = u.x, v[1] = u.y, v[2] = u.z, v[3] = u.w, v[4] = w.x, v[5] = w.y, v[6] = w.z, v[7] = w.w;
+  } else if (wide) {
+    const uint4 u = *reinterpret_cast<const uint4*>(static_cast<const unsigned short*>(p) + at);
+    const unsigned w[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const unsigned short b = (unsigned short)(w[k >> 1] >> (16 * (k & 1)));
+      v[k] = dtype == 1 ? (float)__builtin_bit_cast(_Float16, b) : __builtin_bit_cast(float, (unsigned)b << 16);
+    }
+  } else {
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = small_load(p, at + k, dtype);
+  }
+}
+// Do rows of d elements start at multiples of 16 bytes?
+__device__ __forceinline__ bool dense_wide(const void* p, int d, int dtype) {
+  return ((size_t)p & 15) == 0 && (d & (dtype == 0 ? 3 : 7)) == 0;
+}
+
+// Largest magnitude and sum of the weights of a slice of one matrix (small_stats_kernel's first two
+// words; no bounding boxes: a schedule comes as a table here).  Bound by memory.
+template <int T>
+__global__ __launch_bounds__(1024) void dense_stats_kernel(const SmallArgs a) {
+  const int mat = blockIdx.y, item = blockIdx.z, tid = threadIdx.x;
+  const size_t count = (size_t)a.rows[mat] * a.d, base = item * count;
+  const bool wide = dense_wide(a.pts[mat], a.d, a.dtype);
+  float am = 0.f, ws = 0.f;
+  const size_t stride = (size_t)gridDim.x * 1024 * 8;
+#pragma unroll 2
+  for (size_t i = ((size_t)blockIdx.x * 1024 + tid) * 8; i < count; i += stride) {
+    float v[8];
+    if (i + 8 <= count) {
+      dense_load8(v, a.pts[mat], base + i, a.dtype, wide);
+    } else {
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v[k] = i + k < count ? small_load(a.pts[mat], base + i + k, a.dtype) : 0.f;
+    }
+#pragma unroll
+    for (int k = 0; k < 8; ++k) am = fmaxf(am, fabsf(v[k]));
+  }
+  if (a.w[mat] != nullptr)
+    for (int i = blockIdx.x * 1024 + tid; i < a.rows[mat]; i += gridDim.x * 1024)
+      ws += a.w[mat][(size_t)item * a.rows[mat] + i];
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    am = fmaxf(am, __shfl_xor(am, o, 64));
+    ws += __shfl_xor(ws, o, 64);
+  }
+  __shared__ float sh[2][16];
+  if ((tid & 63) == 0) sh[0][tid >> 6] = am, sh[1][tid >> 6] = ws;
+  __syncthreads();
+  if (tid == 0) {
+    for (int w = 1; w < 16; ++w) am = fmaxf(am, sh[0][w]), ws += sh[1][w];
+    float* out = a.stats + (((size_t)item * 2 + mat) * kSmallStatBlocks + blockIdx.x) * kSmallStatWords;
+    out[0] = am;
+    out[1] = ws;
+  }
+}
+
+// Planes of 32 rows, their norms, log weights and initial potentials.  Grid (blocks of the larger
+// matrix and one more, which fills the table of a fixed eps; matrices; items).
+template <int T>
+__global__ __launch_bounds__(512) void dense_prep_kernel(const SmallArgs a, const DenseArgs t) {
+  const int mat = blockIdx.y, item = blockIdx.z, tid = threadIdx.x;
+  if ((int)blockIdx.x == gridDim.x - 1) {
+    if (mat == 0) small_schedule(a, item);
+    return;
+  }
+  const int rb = blockIdx.x, rows = a.rows[mat], d = a.d;
+  if (rb >= t.blocks[mat]) return;
+  const int wave = tid >> 6, lane = tid & 63, li = lane & 31, h = lane >> 5;
+  const float* st = a.stats + ((size_t)item * 2 + mat) * kSmallStatBlocks * kSmallStatWords;
+  float am = st[lane * kSmallStatWords], ws = st[lane * kSmallStatWords + 1];
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    am = fmaxf(am, __shfl_xor(am, o, 64));
+    ws += __shfl_xor(ws, o, 64);
+  }
+  const float sc = f16_plane_scale(am);
+  if (rb == 0 && tid == 0) a.scale[item * 2 + mat] = make_float2(sc, 1.0f / sc);
+  const int row = rb * 32 + li;
+  const bool live = row < rows, wide = dense_wide(a.pts[mat], d, a.dtype);
+  const size_t base = ((size_t)item * rows + min(row, rows - 1)) * d;
+  u32x4* po = t.planes[mat] + ((size_t)item * t.blocks[mat] + rb) * (size_t)t.steps * kDenseStep + lane;
+  float q = 0.f;
+  for (int kk = wave; kk < t.steps; kk += 8) {
+    float v[8];
+    const int c0 = 16 * kk + 8 * h;
+    if (c0 + 8 <= d) {
+      dense_load8(v, a.pts[mat], base + c0, a.dtype, wide);
+    } else {
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v[k] = c0 + k < d ? small_load(a.pts[mat], base + c0 + k, a.dtype) : 0.f;
+    }
+    u32x4 hi, lo;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const float v0 = live ? sc * v[2 * k] : 0.f, v1 = live ? sc * v[2 * k + 1] : 0.f;
+      const _Float16 h0 = (_Float16)v0, h1 = (_Float16)v1;
+      hi[k] = pack_f16((float)h0, (float)h1);
+      lo[k] = pack_f16(v0 - (float)h0, v1 - (float)h1);
+      q = __builtin_fmaf(v0, v0, __builtin_fmaf(v1, v1, q));
+    }
+    po[(size_t)kk * kDenseStep] = hi;
+    po[(size_t)kk * kDenseStep + 64] = lo;
+  }
+  __shared__ float sh[8][64];
+  sh[wave][lane] = q;
+  __syncthreads();
+  if (tid >= 32 || !live) return;
+  q = 0.f;
+#pragma unroll
+  for (int w = 0; w < 8; ++w) q += sh[w][tid] + sh[w][tid + 32];
+  const float inv = 1.0f / sc, al = a.cost_scale * (q * inv * inv);
+  const size_t at = (size_t)item * rows + row;
+  a.norm[mat][at] = al;
+  float w = a.w[mat] == nullptr ? 1.0f / (float)rows : a.w[mat][at];
+  if (a.w[mat] != nullptr && a.normalize) w = w / fmaxf(ws, 1e-40f);
+  a.wt[mat][at] = w;
+  a.l2w[mat][at] = w > 0.f ? small_log2(w, 0.f) : -100000.0f * kLog2e;
+  a.pot[mat][at] = -al;
+}
+
+// One operand's tile stream and C = A B^T: a workgroup of WR x WC wavefronts owns 32 WR RB rows and
+// 32 WC CB columns; per 16-column step both operands' blocks come into one of four LDS stages by
+// direct global -> LDS loads of 1 KiB per wavefront, three steps ahead, one barrier per step.
+// Bound by the matrix pipe: RB CB 3 MFMAs per wavefront and step against 2 (RB + CB) LDS reads.
+// LDS reads are written out by hand (the compiler would have each wait for the loads in flight).
+struct DenseGemmArgs {
+  const u32x4* a;           // rows, columns: planes
+  const u32x4* b;
+  int a_blocks, b_blocks;   // blocks per item
+  int steps, rows, ld;      // rows: of the result, per item
+  const float2* scale;      // [items][2]: the planes' scales and inverses
+  float* out;               // [items][rows][ld]
+  int row_tiles, col_tiles;
+};
+
+template <int WR, int WC, int RB, int CB>
+__global__ __launch_bounds__(64 * WR * WC, 2) void dense_gemm_kernel(const DenseGemmArgs g) {
+  constexpr int W = WR * WC, TR = WR * RB, TC = WC * CB, PIECES = 2 * (TR + TC), LOADS = PIECES / W, ST = 4;
+  static_assert(PIECES % W == 0, "every wavefront moves the same number of pieces");
+  static_assert(2 * RB * 1024 <= 65535 && 2 * CB * 1024 <= 65535, "offsets of the LDS reads");
+  __shared__ __attribute__((aligned(16))) u32x4 lds[ST * PIECES * 64];
+  // XCD x takes the x-th eighth of the tiles in the order (4 row tiles, column tile, row tile):
+  // what shares an L2 shares operands
+  const int tiles = g.row_tiles * g.col_tiles, per_xcd = (tiles + 7) / 8;
+  int item = ((int)blockIdx.x & 7) * per_xcd + ((int)blockIdx.x >> 3);
+  if (((int)blockIdx.x >> 3) >= per_xcd || item >= tiles) return;
+  const int band = item / (4 * g.col_tiles), within = item % (4 * g.col_tiles);
+  const int nb = min(4, g.row_tiles - 4 * band);
+  const int rt = 4 * band + within % nb, ct = within / nb, z = blockIdx.y;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int li = lane & 31, h = lane >> 5, wr = wave / WC, wc = wave % WC;
+
+  // piece p of a stage: block p / 2 (the rows' first), plane p % 2
+  const u32x4* src[LOADS];
+#pragma unroll
+  for (int i = 0; i < LOADS; ++i) {
+    const int p = wave * LOADS + i, blk = p / 2;
+    const bool of_a = blk < TR;
+    const int gb = of_a ? rt * TR + blk : ct * TC + blk - TR;  // (blocks are padded to whole tiles of 8)
+    src[i] = (of_a ? g.a + ((size_t)z * g.a_blocks + gb) * (size_t)g.steps * kDenseStep
+                   : g.b + ((size_t)z * g.b_blocks + gb) * (size_t)g.steps * kDenseStep) + (p & 1) * 64 + lane;
+  }
+  auto stage = [&](int k, int buf) {
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i)
+      __builtin_amdgcn_global_load_lds(
+          (const __attribute__((address_space(1))) void*)(src[i] + (size_t)min(k, g.steps - 1) * kDenseStep),
+          (__attribute__((address_space(3))) void*)(&lds[(buf * PIECES + wave * LOADS + i) * 64]), 16, 0, 0);
+  };
+  const unsigned base = (unsigned)(size_t)(const __attribute__((address_space(3))) u32x4*)&lds[0] + lane * 16;
+  const unsigned abase = base + wr * RB * 2 * 1024, bbase = base + (TR + wc * CB) * 2 * 1024;
+
+  f32x16 acc[RB][CB];
+#pragma unroll
+  for (int i = 0; i < RB; ++i)
+#pragma unroll
+    for (int j = 0; j < CB; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+
+  stage(0, 0);
+  stage(1, 1);
+  stage(2, 2);
+  for (int k = 0; k < g.steps; ++k) {
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(0x0F70 | ((2 * LOADS) & 15) | (((2 * LOADS) >> 4) << 14));  // step k has landed
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();  // for everyone, and step k - 1 has been read by everyone
+    asm volatile("" ::: "memory");
+    stage(k + 3, (k + 3) & 3);
+    const unsigned off = (k & 3) * (PIECES * 1024);
+    u32x4 x[RB][2], y[CB][2];
+    static_for<2 * RB>([&](auto i) { x[i / 2][i % 2] = lds_read16<decltype(i)::value * 1024>(abase + off); });
+    static_for<2 * CB>([&](auto i) { y[i / 2][i % 2] = lds_read16<decltype(i)::value * 1024>(bbase + off); });
+    static_for<CB>([&](auto j_) {
+      constexpr int j = decltype(j_)::value;
+      __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_s_waitcnt(0xC07F | ((2 * (CB - 1 - j)) << 8));  // this column block has been read
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int prod = 0; prod < 3; ++prod)
+#pragma unroll
+        for (int i = 0; i < RB; ++i)
+          acc[i][j] = small_mfma(x[i][prod == 0 ? 1 : 0], y[j][prod == 1 ? 1 : 0], acc[i][j]);
+    });
+  }
+  __builtin_amdgcn_s_waitcnt(0);
+  const float2 sa = g.scale[z * 2], sb = g.scale[z * 2 + 1];
+  const float inv = sa.y * sb.y;
+  float* out = g.out + (size_t)z * g.rows * g.ld;
+#pragma unroll
+  for (int i = 0; i < RB; ++i)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int row = (rt * TR + wr * RB + i) * 32 + 8 * (r / 4) + 4 * h + r % 4;
+      if (row < g.rows)
+#pragma unroll
+        for (int j = 0; j < CB; ++j) out[(size_t)row * g.ld + (ct * TC + wc * CB + j) * 32 + li] = acc[i][j][r] * inv;
+    }
+}
+
+__device__ __forceinline__ void dense_join(float& m, float& s, float m2, float s2) {
+  const float M = fmaxf(m, m2);
+  s = s * fast_exp2(m - M) + s2 * fast_exp2(m2 - M);
+  m = M;
+}
+
+// Soft-max statistics of all rows (over the columns' biases) and of all columns (over the rows').  A
+// wavefront reads RW rows of 256 columns (1 KiB a row) at a time, a lane four columns of them; the
+// rows' running statistics stay lane-private over the workgroup's run of columns and cross lanes
+// once, the columns' are lane-private over the rows and cross wavefronts through LDS.  Bound by
+// memory (HBM or last-level cache); two exponentials per product hide behind it with four
+// wavefronts per SIMD.  Both directions carry running maxima: no step needs permission.
+template <int RW, int WV>
+__global__ __launch_bounds__(64 * WV, 4) void dense_sweep_kernel(const DenseArgs a) {
+  constexpr int B = 8;  // rows in registers
+  static_assert(RW % B == 0, "");
+  __shared__ float2 sh[2][WV][256];
+  const int group = blockIdx.x, ch = blockIdx.y, item = blockIdx.z;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int entries = a.lens[item * 3];
+  if (a.step > entries + a.extrapolate) return;
+  const float4 coef = a.table[(size_t)item * 3 * kSmallTable + (a.sched == 0 ? 0 : min(max(a.step - 1, 0), kSmallTable - 1))];
+  const float qs = coef.y, kc = coef.w;
+  const int r0 = (group * WV + wave) * RW;
+  const float* dots = a.dots + (size_t)item * a.n * a.ld;
+  // the rows' biases, one per lane
+  float rb;
+  {
+    const int row = r0 + (lane & (RW - 1));
+    const size_t at = (size_t)item * a.n + min(row, a.n - 1);
+    rb = row < a.n ? fmaxf(__builtin_fmaf(kc, a.pot[0][at], a.l2w[0][at]), kNegBig) : kNegBig;
+  }
+  float rm[RW], rs[RW];
+#pragma unroll
+  for (int r = 0; r < RW; ++r) rm[r] = kNegBig, rs[r] = 0.f;
+  const int c_end = min(a.ld, (ch + 1) * a.chunk);
+  int buf = 0;
+  for (int c0 = ch * a.chunk; c0 < c_end; c0 += 256, buf ^= 1) {
+    float kb[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int col = c0 + 4 * lane + k;
+      const size_t at = (size_t)item * a.m + min(col, a.m - 1);
+      kb[k] = col < a.m ? fmaxf(__builtin_fmaf(kc, a.pot[1][at], a.l2w[1][at]), kNegBig) : kNegBig;
+    }
+    float cm[4], cs[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) cm[k] = kNegBig, cs[k] = 0.f;
+#pragma unroll
+    for (int b0 = 0; b0 < RW; b0 += B) {
+      float4 v[B];
+#pragma unroll
+      for (int r = 0; r < B; ++r)
+        v[r] = *reinterpret_cast<const float4*>(dots + (size_t)min(r0 + b0 + r, a.n - 1) * a.ld + c0 + 4 * lane);
+      float mc[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) mc[k] = cm[k];
+#pragma unroll
+      for (int r = 0; r < B; ++r) {
+        // ---- the row ----
+        v[r].x *= qs, v[r].y *= qs, v[r].z *= qs, v[r].w *= qs;
+        const float l0 = v[r].x + kb[0], l1 = v[r].y + kb[1], l2 = v[r].z + kb[2], l3 = v[r].w + kb[3];
+        float& m = rm[b0 + r];
+        float& s = rs[b0 + r];
+        const float M = fmaxf(fmaxf(fmaxf(l0, l1), fmaxf(l2, l3)), m);
+        s = s * fast_exp2(m - M) + ((fast_exp2(l0 - M) + fast_exp2(l1 - M)) + (fast_exp2(l2 - M) + fast_exp2(l3 - M)));
+        m = M;
+        // ---- the columns' maxima ----
+        const float br = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, rb), b0 + r));
+        v[r].x += br, v[r].y += br, v[r].z += br, v[r].w += br;
+        mc[0] = fmaxf(mc[0], v[r].x);
+        mc[1] = fmaxf(mc[1], v[r].y);
+        mc[2] = fmaxf(mc[2], v[r].z);
+        mc[3] = fmaxf(mc[3], v[r].w);
+      }
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        float s = cs[k] * fast_exp2(cm[k] - mc[k]);
+#pragma unroll
+        for (int r = 0; r < B; ++r) s += fast_exp2((k == 0 ? v[r].x : k == 1 ? v[r].y : k == 2 ? v[r].z : v[r].w) - mc[k]);
+        cs[k] = s;
+        cm[k] = mc[k];
+      }
+    }
+    float4* o = reinterpret_cast<float4*>(&sh[buf][wave][4 * lane]);
+    o[0] = make_float4(cm[0], cs[0], cm[1], cs[1]);
+    o[1] = make_float4(cm[2], cs[2], cm[3], cs[3]);
+    __syncthreads();  // (the other buffer is free once everyone is here)
+    for (int c = threadIdx.x; c < 256; c += 64 * WV) {
+      float m = sh[buf][0][c].x, s = sh[buf][0][c].y;
+#pragma unroll
+      for (int w = 1; w < WV; ++w) dense_join(m, s, sh[buf][w][c].x, sh[buf][w][c].y);
+      if (c0 + c < a.m) a.part[1][((size_t)item * a.groups + group) * a.m + c0 + c] = make_float2(m, s);
+    }
+  }
+  // ---- the rows' statistics over the lanes: halves of the rows change places ----
+#pragma unroll
+  for (int o = 32, n = RW / 2; n > 0; o >>= 1, n >>= 1) {
+    const bool up = lane & o;
+#pragma unroll
+    for (int r = 0; r < n; ++r) {
+      const float gm = up ? rm[r] : rm[r + n], gs = up ? rs[r] : rs[r + n];
+      float m = up ? rm[r + n] : rm[r], s = up ? rs[r + n] : rs[r];
+      dense_join(m, s, __shfl_xor(gm, o, 64), __shfl_xor(gs, o, 64));
+      rm[r] = m;
+      rs[r] = s;
+    }
+  }
+  constexpr int LEFT = 64 / RW;  // lanes that share a row
+#pragma unroll
+  for (int o = LEFT / 2; o > 0; o >>= 1) dense_join(rm[0], rs[0], __shfl_xor(rm[0], o, 64), __shfl_xor(rs[0], o, 64));
+  const int row = r0 + lane / LEFT;
+  if (lane % LEFT == 0 && row < a.n) a.part[0][((size_t)item * a.chunks + ch) * a.n + row] = make_float2(rm[0], rs[0]);
+}
+
+// The new potentials: 64 rows of one side per workgroup, its four wavefronts share the parts.
+template <int T>
+__global__ __launch_bounds__(256) void dense_merge_kernel(const DenseArgs a) {
+  const int side = blockIdx.y, item = blockIdx.z, rows = side ? a.m : a.n;
+  if ((int)blockIdx.x * 64 >= rows) return;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int entries = a.lens[item * 3];
+  if (a.step > entries + a.extrapolate) return;
+  const float eps = a.table[(size_t)item * 3 * kSmallTable + (a.sched == 0 ? 0 : min(max(a.step - 1, 0), kSmallTable - 1))].x;
+  const int row = blockIdx.x * 64 + lane, rc = min(row, rows - 1), parts = side ? a.groups : a.chunks;
+  const size_t at = (size_t)item * rows + rc;
+  const float old = a.pot[side][at], norm = a.norm[side][at];
+  const float2* p = a.part[side] + (size_t)item * parts * rows + rc;
+  float M = kNegBig, S = 0.f;
+#pragma unroll 8
+  for (int c = wave; c < parts; c += 4) {
+    const float2 v = p[(size_t)c * rows];
+    dense_join(M, S, v.x, v.y);
+  }
+  __shared__ float2 sh[4][64];
+  sh[wave][lane] = make_float2(M, S);
+  __syncthreads();
+  if (wave > 0 || row >= rows) return;
+#pragma unroll
+  for (int w = 1; w < 4; ++w) dense_join(M, S, sh[w][lane].x, sh[w][lane].y);
+  const float rho = a.rho[side], damp = rho > 0.f ? 1.0f / (1.0f + eps / rho) : 1.0f;
+  const float alpha = (a.step == 0 || a.step > entries) ? 1.0f : 0.5f;
+  float f = alpha * (-eps * damp * kLn2 * small_log2(fmaxf(S, 1e-40f), M));
+  if (alpha != 1.0f) f += (1.0f - alpha) * old;
+  if (damp < 1.0f) f -= alpha * (1.0f - damp) * norm;
+  a.out[side][at] = f;
+}
+
+// Host side (fs_dense.hip).
+void dense_plan(const SmallArgs& a, DenseArgs& t);
+int dense_prepare(const SmallArgs& a, const DenseArgs& t, hipStream_t st);
+int dense_step(const SmallArgs& a, DenseArgs& t, int step, hipStream_t st);
+
+}  // namespace fs

@@ -21,33 +21,11 @@
 // makes the ds_read_b128 of 16 consecutive rows at one piece index conflict free.
 #pragma once
 
-#include <type_traits>
-#include <utility>
-
 #include "fs_colsum.hpp"
 #include "fs_common.hpp"
 #include "fs_stream.hpp"
 
 namespace fs {
-
-// f(integral_constant<int, 0>{}), ..., f(integral_constant<int, N - 1>{}) in order
-template <int... I, class F>
-__device__ __forceinline__ void static_for_impl(std::integer_sequence<int, I...>, F&& f) {
-  (f(std::integral_constant<int, I>{}), ...);
-}
-template <int N, class F>
-__device__ __forceinline__ void static_for(F&& f) {
-  static_for_impl(std::make_integer_sequence<int, N>{}, f);
-}
-
-// 16 bytes from LDS at byte address addr + OFF (OFF < 65536), not visible to the compiler's
-// wait-count insertion: the consumer must sit behind an explicit wait
-template <int OFF>
-__device__ __forceinline__ u32x4 lds_read16(unsigned addr) {
-  u32x4 v;
-  asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(OFF) : "memory");
-  return v;
-}
 
 constexpr int kGemmRows = 256;   // query rows per workgroup = keys per tile
 constexpr int kGemmCols = 32;    // feature columns per k-step

@@ -10,6 +10,7 @@
 #include <vector>
 
 #include "flash_sinkhorn_hip.h"
+#include "fs_dense.hpp"
 #include "fs_pair.hpp"
 #include "fs_small.hpp"
 
@@ -42,6 +43,9 @@ bool use_pair(const fs_small_problem* p) {
   return logits >= (p->sched == 0 || p->d > 32 ? 2.0e7 : 5.0e7);
 }
 
+// Wide rows: the products are formed once and kept (fs_dense.hpp).
+bool use_dense(const fs_small_problem* p) { return p->d > kSmallMaxD; }
+
 // Workgroups over which the loss of an item is spread: one for what a workgroup does in three rounds.
 int loss_parts(const SmallArgs& a) {
   const int rows = std::max(a.rows[0], a.rows[1]);
@@ -53,7 +57,8 @@ int padded(int64_t d) { return d <= 16 ? 16 : (d <= 32 ? 32 : (d <= 64 ? 64 : 12
 int checked(const fs_small_problem* p) {
   if (!p || !p->x || !p->y) return FS_ERR_NULL_POINTER;
   if (p->n <= 0 || p->m <= 0 || p->d <= 0 || p->items <= 0 || p->items > 65535) return FS_ERR_BAD_SIZE;
-  if (p->d > kSmallMaxD || p->n > FS_SMALL_MAX_ROWS || p->m > FS_SMALL_MAX_ROWS) return FS_ERR_UNSUPPORTED;
+  if (p->n > FS_SMALL_MAX_ROWS || p->m > FS_SMALL_MAX_ROWS) return FS_ERR_UNSUPPORTED;
+  if (p->d > kSmallMaxD && (p->self_terms || p->want_values || p->sched == 1)) return FS_ERR_UNSUPPORTED;
   if (p->dtype < 0 || p->dtype > 2 || p->sched < 0 || p->sched > 2) return FS_ERR_BAD_ARGUMENT;
   if (p->sched != 1 && p->entries <= 0) return FS_ERR_BAD_ARGUMENT;
   if (p->sched == 0 && !(p->eps > 0.f)) return FS_ERR_BAD_ARGUMENT;
@@ -176,7 +181,7 @@ void pair_step_args(const SmallArgs& a, PairArgs& t, int step) {
 
 // The kernels' arguments with the workspace laid out from `ws` (null: sizes only); returns the
 // bytes the workspace takes.
-size_t layout(const fs_small_problem* p, void* ws, SmallArgs& a, PairArgs* pa = nullptr) {
+size_t layout(const fs_small_problem* p, void* ws, SmallArgs& a, PairArgs* pa = nullptr, DenseArgs* da = nullptr) {
   std::memset(&a, 0, sizeof(a));
   a.pair = use_pair(p) ? 1 : 0;
   a.pts[0] = p->x;
@@ -221,7 +226,7 @@ size_t layout(const fs_small_problem* p, void* ws, SmallArgs& a, PairArgs* pa = 
     // (whole 256-row groups, and the tiles that are fetched past the end)
     a.pblocks[i] = a.pair ? (int)((rows + 255) / 256) * 8 + 8 : a.blocks[i];
     const size_t blocks = items * (size_t)a.blocks[i], pblocks = items * (size_t)a.pblocks[i];
-    take(a.planes[i], pblocks * (size_t)(2 * dp / 16) * 1024);
+    if (!use_dense(p)) take(a.planes[i], pblocks * (size_t)(2 * dp / 16) * 1024);
     if (a.pair && a.self && a.sched != 0) take(a.self_planes[i], pblocks * (size_t)(2 * dp / 16) * 1024);
     if (a.want_values) take(a.values[i], blocks * (size_t)(ndb * 4) * 1024);
     take(a.norm[i], items * rows * 4);
@@ -232,6 +237,25 @@ size_t layout(const fs_small_problem* p, void* ws, SmallArgs& a, PairArgs* pa = 
     if (p->threshold > 0.f) {
       take(a.prev[i], items * rows * 4);
       if (a.self) take(a.prev[2 + i], items * rows * 4);
+    }
+  }
+  if (use_dense(p)) {
+    DenseArgs scratch;
+    DenseArgs& t = da ? *da : scratch;
+    std::memset(&t, 0, sizeof(t));
+    dense_plan(a, t);
+    take(t.dots, items * (size_t)t.n * (size_t)t.ld * 4);
+    for (int i = 0; i < 2; ++i) take(t.planes[i], items * (size_t)t.blocks[i] * (size_t)t.steps * 2048);
+    take(t.part[0], items * (size_t)t.chunks * (size_t)t.n * sizeof(float2));
+    take(t.part[1], items * (size_t)t.groups * (size_t)t.m * sizeof(float2));
+    t.table = a.table;
+    t.lens = a.lens;
+    t.sched = a.sched;
+    t.extrapolate = a.extrapolate;
+    for (int i = 0; i < 2; ++i) {
+      t.l2w[i] = a.l2w[i];
+      t.norm[i] = a.norm[i];
+      t.rho[i] = a.rho[i];
     }
   }
   if (a.pair) {
@@ -380,7 +404,8 @@ int fs_small_solve(const fs_small_problem* p, void* workspace, size_t workspace_
   if ((p->sched == 1 || p->threshold > 0.f) && !host_words) return FS_ERR_NULL_POINTER;
   SmallArgs a;
   PairArgs pa;
-  if (!workspace || layout(p, workspace, a, &pa) > workspace_bytes) return FS_ERR_WORKSPACE_TOO_SMALL;
+  DenseArgs da;
+  if (!workspace || layout(p, workspace, a, &pa, &da) > workspace_bytes) return FS_ERR_WORKSPACE_TOO_SMALL;
   hipStream_t st = (hipStream_t)stream;
   int entries = a.entries;
   a.host_words = host_words;
@@ -396,7 +421,8 @@ int fs_small_solve(const fs_small_problem* p, void* workspace, size_t workspace_
     hipLaunchKernelGGL((small_table_kernel<0>), dim3(a.items * 3), dim3(256), 0, st, a, t);
     if (hipGetLastError() != hipSuccess) return FS_ERR_LAUNCH_FAILED;
   }
-  rc = by_width(p->d, [&](auto dp) {
+  const bool dense = use_dense(p);
+  rc = dense ? dense_prepare(a, da, st) : by_width(p->d, [&](auto dp) {
     constexpr int DP = decltype(dp)::value;
     const int r = launch_prep<DP>(a, st);
     if constexpr (DP <= 64)
@@ -447,7 +473,7 @@ int fs_small_solve(const fs_small_problem* p, void* workspace, size_t workspace_
     });
   };
   for (int s = 0; s < n_steps && rc == FS_OK && !all_done; ++s) {
-    rc = by_width(p->d, [&](auto dp) {
+    rc = dense ? dense_step(a, da, s, st) : by_width(p->d, [&](auto dp) {
       constexpr int DP = decltype(dp)::value;
       if constexpr (DP <= 64)
         if (a.pair) return launch_pair_step<DP>(a, pa, s, st);

@@ -380,6 +380,8 @@ def _small_symmetric(x, y, a, b, blur, scaling, use_epsilon_scaling, last_extrap
     if threshold is not None and return_n_iters and eps_list is None and use_epsilon_scaling \
             and diameter is None:
         diameter = max_diameter(x, y)  # (the length of the schedule is asked for)
+    if x.shape[1] > _small.WIDE_D and eps_list is None and use_epsilon_scaling and diameter is None:
+        diameter = max_diameter(x, y)
     if eps_list is None and not use_epsilon_scaling:
         if eps is None or n_iters is None or not eps > 0 or int(n_iters) <= 0:
             return None
