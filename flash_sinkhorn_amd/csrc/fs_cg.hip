@@ -4,7 +4,7 @@
 // state back only when it wants to know whether to go on.
 #include <hip/hip_runtime.h>
 
-#include "flash_sinkhorn_hip.h"
+#include "fs_host.hpp"
 
 namespace fs {
 namespace {
@@ -24,12 +24,19 @@ __device__ double block_sum(double v, double* red) {
   return t;
 }
 
+__device__ void report(const float* state, float* host, int count) {
+  if (host == nullptr) return;
+  for (int i = 0; i < 7; ++i) __hip_atomic_store(&host[i], state[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  __threadfence_system();
+  __hip_atomic_store(reinterpret_cast<int*>(host) + 7, count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 __global__ __launch_bounds__(kCgThreads) void cg_init_kernel(const float* __restrict__ b,
                                                              float* __restrict__ sol,
                                                              float* __restrict__ res,
                                                              float* __restrict__ dir,
                                                              float* __restrict__ state, long long m,
-                                                             float rtol, float atol) {
+                                                             float rtol, float atol, float* host) {
   __shared__ double red[kCgThreads / 64];
   double acc = 0.0;
   for (long long i = threadIdx.x; i < m; i += kCgThreads) {
@@ -50,6 +57,7 @@ __global__ __launch_bounds__(kCgThreads) void cg_init_kernel(const float* __rest
     state[5] = 0.f;
     state[6] = 0.f;
     state[7] = 0.f;
+    report(state, host, 0);
   }
 }
 
@@ -58,14 +66,17 @@ __global__ __launch_bounds__(kCgThreads) void cg_update_kernel(const float* __re
                                                                float* __restrict__ res,
                                                                float* __restrict__ dir,
                                                                float* __restrict__ state,
-                                                               long long m) {
+                                                               long long m, float* host, int iter) {
   __shared__ double red[kCgThreads / 64];
   if (state[4] != 0.f) return;  // finished earlier: every later update leaves the vectors alone
   double acc = 0.0;
   for (long long i = threadIdx.x; i < m; i += kCgThreads) acc += (double)dir[i] * (double)a_dir[i];
   const double curvature = block_sum(acc, red);
   if (curvature == 0.0) {  // uniform: every thread holds the same sum
-    if (threadIdx.x == 0) state[4] = 1.f;
+    if (threadIdx.x == 0) {
+      state[4] = 1.f;
+      report(state, host, iter + 1);
+    }
     return;
   }
   const float rz = state[0];
@@ -86,6 +97,7 @@ __global__ __launch_bounds__(kCgThreads) void cg_update_kernel(const float* __re
       state[4] = 1.f;
       state[5] = 1.f;
       state[6] += 1.f;
+      report(state, host, iter + 1);
     }
     return;
   }
@@ -95,10 +107,24 @@ __global__ __launch_bounds__(kCgThreads) void cg_update_kernel(const float* __re
     state[0] = (float)rr;
     state[3] = rnorm;
     state[6] += 1.f;
+    report(state, host, iter + 1);
   }
 }
 
 }  // namespace
+
+int cg_init(const float* b, float* sol, float* res, float* dir, float* state, long long m, float rtol, float atol,
+            float* host, hipStream_t st) {
+  hipLaunchKernelGGL(cg_init_kernel, dim3(1), dim3(kCgThreads), 0, st, b, sol, res, dir, state, m, rtol, atol, host);
+  return hipGetLastError() == hipSuccess ? FS_OK : FS_ERR_LAUNCH_FAILED;
+}
+
+int cg_update(const float* a_dir, float* sol, float* res, float* dir, float* state, long long m, float* host, int iter,
+              hipStream_t st) {
+  hipLaunchKernelGGL(cg_update_kernel, dim3(1), dim3(kCgThreads), 0, st, a_dir, sol, res, dir, state, m, host, iter);
+  return hipGetLastError() == hipSuccess ? FS_OK : FS_ERR_LAUNCH_FAILED;
+}
+
 }  // namespace fs
 
 extern "C" {
@@ -107,18 +133,14 @@ int fs_cg_init(const float* b, float* sol, float* res, float* dir, float* state,
                float rtol, float atol, void* stream) {
   if (!b || !sol || !res || !dir || !state) return FS_ERR_NULL_POINTER;
   if (m <= 0 || m > ((int64_t)1 << 31)) return FS_ERR_BAD_SIZE;
-  hipLaunchKernelGGL(fs::cg_init_kernel, dim3(1), dim3(fs::kCgThreads), 0, (hipStream_t)stream, b,
-                     sol, res, dir, state, (long long)m, rtol, atol);
-  return hipGetLastError() == hipSuccess ? FS_OK : FS_ERR_LAUNCH_FAILED;
+  return fs::cg_init(b, sol, res, dir, state, (long long)m, rtol, atol, nullptr, (hipStream_t)stream);
 }
 
 int fs_cg_update(const float* a_dir, float* sol, float* res, float* dir, float* state, int64_t m,
                  void* stream) {
   if (!a_dir || !sol || !res || !dir || !state) return FS_ERR_NULL_POINTER;
   if (m <= 0 || m > ((int64_t)1 << 31)) return FS_ERR_BAD_SIZE;
-  hipLaunchKernelGGL(fs::cg_update_kernel, dim3(1), dim3(fs::kCgThreads), 0, (hipStream_t)stream,
-                     a_dir, sol, res, dir, state, (long long)m);
-  return hipGetLastError() == hipSuccess ? FS_OK : FS_ERR_LAUNCH_FAILED;
+  return fs::cg_update(a_dir, sol, res, dir, state, (long long)m, nullptr, 0, (hipStream_t)stream);
 }
 
 }  // extern "C"

@@ -12,24 +12,46 @@ int launch_gemm(DenseGemmArgs& g, int items, hipStream_t st) {
   g.row_tiles = (g.rows + 32 * WR * RB - 1) / (32 * WR * RB);
   g.col_tiles = g.ld / (32 * WC * CB);
   const int tiles = g.row_tiles * g.col_tiles;
-  hipLaunchKernelGGL((dense_gemm_kernel<WR, WC, RB, CB>), dim3((tiles + 7) / 8 * 8, items), dim3(64 * WR * WC), 0, st, g);
+  hipLaunchKernelGGL((dense_gemm_kernel<WR, WC, RB, CB>), dim3((tiles + 7) / 8 * 8, items, g.splits), dim3(64 * WR * WC), 0, st, g);
   return hipGetLastError() == hipSuccess ? FS_OK : FS_ERR_LAUNCH_FAILED;
 }
 
 // Tiles of 256, 128 or 64 rows and columns: the one whose rounds over the chip cost least, a
-// workgroup of the smaller ones taking longer per product (operands are read more often).
-int gemm(DenseGemmArgs& g, int items, hipStream_t st) {
-  auto cost = [&](int side, int at_once, double per) {
-    const double tiles = (double)items * std::ceil(g.rows / (double)side) * std::ceil(g.ld / (double)side);
-    return std::ceil(tiles / (256.0 * at_once)) * at_once * per * side * side;
-  };
-  const double big = cost(256, 1, 1.0), mid = cost(128, 2, 1.25), tiny = cost(64, 4, 2.0);
-  if (big <= mid && big <= tiny) return launch_gemm<2, 4, 4, 2>(g, items, st);
-  if (mid <= tiny) return launch_gemm<2, 2, 2, 2>(g, items, st);
-  return launch_gemm<2, 2, 1, 1>(g, items, st);
+// workgroup of the smaller ones taking longer per product (operands are read more often).  In units
+// of a 256 x 256 tile's step; writing and adding up a part of a split contraction counts what
+// 5 TB/s take.
+double tile_cost(const DenseGemmArgs& g, int side, int splits, int items) {
+  const int at_once = side == 256 ? 1 : (side == 128 ? 2 : 4);
+  const double per = side == 256 ? 1.0 : (side == 128 ? 1.25 / 4 : 2.0 / 16);
+  const double tiles = (double)items * splits * std::ceil(g.rows / (double)side) * (g.ld / side);
+  const double traffic = splits == 1 ? 0.0 : splits * 8.0 * g.rows * g.ld / 5e6 / 1.3;
+  return std::ceil(tiles / (256.0 * at_once)) * at_once * per * ((g.steps + splits - 1) / splits + 6) + traffic;
+}
+int best_side(const DenseGemmArgs& g, int splits, int items) {
+  int best = 64;
+  for (int side : {128, 256})
+    if (g.ld % side == 0 && tile_cost(g, side, splits, items) <= tile_cost(g, best, splits, items)) best = side;
+  return best;
 }
 
 }  // namespace
+
+// How many parts the contraction is cut into (results of few tiles leave most of the chip idle).
+void dense_gemm_plan(DenseGemmArgs& g, bool may_split) {
+  g.splits = 1;
+  if (may_split)
+    for (int s = 2; s <= 16 && g.steps / s >= 8; ++s)
+      if (tile_cost(g, best_side(g, s, 1), s, 1) < 0.95 * tile_cost(g, best_side(g, g.splits, 1), g.splits, 1)) g.splits = s;
+  g.run = (g.steps + g.splits - 1) / g.splits;
+  g.splits = (g.steps + g.run - 1) / g.run;
+}
+
+int dense_gemm(DenseGemmArgs& g, int items, hipStream_t st) {
+  const int side = best_side(g, g.splits, items);
+  if (side == 256) return launch_gemm<2, 4, 4, 2>(g, items, st);
+  if (side == 128) return launch_gemm<2, 2, 2, 2>(g, items, st);
+  return launch_gemm<2, 2, 1, 1>(g, items, st);
+}
 
 void dense_plan(const SmallArgs& a, DenseArgs& t) {
   t.n = a.rows[0];
@@ -62,8 +84,10 @@ int dense_prepare(const SmallArgs& a, const DenseArgs& t, hipStream_t st) {
   g.rows = t.n;
   g.ld = t.ld;
   g.scale = a.scale;
+  g.scale_a = nullptr;
   g.out = t.dots;
-  return gemm(g, a.items, st);
+  dense_gemm_plan(g, false);
+  return dense_gemm(g, a.items, st);
 }
 
 int dense_step(const SmallArgs& a, DenseArgs& t, int step, hipStream_t st) {

@@ -176,8 +176,10 @@ struct DenseGemmArgs {
   const u32x4* b;
   int a_blocks, b_blocks;   // blocks per item
   int steps, rows, ld;      // rows: of the result, per item
-  const float2* scale;      // [items][2]: the planes' scales and inverses
-  float* out;               // [items][rows][ld]
+  int splits, run;          // parts of the contraction (each a result of its own) and their steps
+  const float2* scale;      // [items][2]: the planes' scales and inverses; null: the result as it is
+  const float2* scale_a;    // of the rows where they are not those of the same array
+  float* out;               // [splits or items][rows][ld]
   int row_tiles, col_tiles;
 };
 
@@ -194,7 +196,8 @@ __global__ __launch_bounds__(64 * WR * WC, 2) void dense_gemm_kernel(const Dense
   if (((int)blockIdx.x >> 3) >= per_xcd || item >= tiles) return;
   const int band = item / (4 * g.col_tiles), within = item % (4 * g.col_tiles);
   const int nb = min(4, g.row_tiles - 4 * band);
-  const int rt = 4 * band + within % nb, ct = within / nb, z = blockIdx.y;
+  const int rt = 4 * band + within % nb, ct = within / nb, z = blockIdx.y, split = blockIdx.z;
+  const int k_begin = split * g.run, steps = min(g.steps - k_begin, g.run);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int li = lane & 31, h = lane >> 5, wr = wave / WC, wc = wave % WC;
 
@@ -206,13 +209,14 @@ __global__ __launch_bounds__(64 * WR * WC, 2) void dense_gemm_kernel(const Dense
     const bool of_a = blk < TR;
     const int gb = of_a ? rt * TR + blk : ct * TC + blk - TR;  // (blocks are padded to whole tiles of 8)
     src[i] = (of_a ? g.a + ((size_t)z * g.a_blocks + gb) * (size_t)g.steps * kDenseStep
-                   : g.b + ((size_t)z * g.b_blocks + gb) * (size_t)g.steps * kDenseStep) + (p & 1) * 64 + lane;
+                   : g.b + ((size_t)z * g.b_blocks + gb) * (size_t)g.steps * kDenseStep) +
+             ((size_t)k_begin * kDenseStep + (p & 1) * 64 + lane);
   }
   auto stage = [&](int k, int buf) {
 #pragma unroll
     for (int i = 0; i < LOADS; ++i)
       __builtin_amdgcn_global_load_lds(
-          (const __attribute__((address_space(1))) void*)(src[i] + (size_t)min(k, g.steps - 1) * kDenseStep),
+          (const __attribute__((address_space(1))) void*)(src[i] + (size_t)min(k, steps - 1) * kDenseStep),
           (__attribute__((address_space(3))) void*)(&lds[(buf * PIECES + wave * LOADS + i) * 64]), 16, 0, 0);
   };
   const unsigned base = (unsigned)(size_t)(const __attribute__((address_space(3))) u32x4*)&lds[0] + lane * 16;
@@ -229,7 +233,7 @@ __global__ __launch_bounds__(64 * WR * WC, 2) void dense_gemm_kernel(const Dense
   stage(0, 0);
   stage(1, 1);
   stage(2, 2);
-  for (int k = 0; k < g.steps; ++k) {
+  for (int k = 0; k < steps; ++k) {
     __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_waitcnt(0x0F70 | ((2 * LOADS) & 15) | (((2 * LOADS) >> 4) << 14));  // step k has landed
     __builtin_amdgcn_sched_barrier(0);
@@ -254,9 +258,8 @@ __global__ __launch_bounds__(64 * WR * WC, 2) void dense_gemm_kernel(const Dense
     });
   }
   __builtin_amdgcn_s_waitcnt(0);
-  const float2 sa = g.scale[z * 2], sb = g.scale[z * 2 + 1];
-  const float inv = sa.y * sb.y;
-  float* out = g.out + (size_t)z * g.rows * g.ld;
+  const float inv = g.scale == nullptr ? 1.0f : (g.scale_a ? g.scale_a[0].y : g.scale[z * 2].y) * g.scale[z * 2 + 1].y;
+  float* out = g.out + (size_t)(z + split) * g.rows * g.ld;  // (one item where the contraction is split)
 #pragma unroll
   for (int i = 0; i < RB; ++i)
 #pragma unroll
@@ -418,6 +421,8 @@ __global__ __launch_bounds__(256) void dense_merge_kernel(const DenseArgs a) {
 
 // Host side (fs_dense.hip).
 void dense_plan(const SmallArgs& a, DenseArgs& t);
+void dense_gemm_plan(DenseGemmArgs& g, bool may_split);
+int dense_gemm(DenseGemmArgs& g, int items, hipStream_t st);
 int dense_prepare(const SmallArgs& a, const DenseArgs& t, hipStream_t st);
 int dense_step(const SmallArgs& a, DenseArgs& t, int step, hipStream_t st);
 

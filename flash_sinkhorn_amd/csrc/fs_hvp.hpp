@@ -1,0 +1,425 @@
+// Hessian-vector product of the cost in x on kept products.
+//
+// With P the plan, A the direction, F_ij = A_i.(x_i - y_j), cs the cost's scale:
+//   r1 = 2 cs rowsum(P F),  r2 = 2 cs colsum(P F)
+//   (denom - P^T diag_x^-1 P) z = r2 - P^T (r1 / diag_x)                   (conjugate gradients)
+//   z1 = (r1 - P z) / diag_x
+//   H A = s_i x_i + 2 cs rowsum(P)_i A_i + sum_j V_ij y_j,
+//   s_i = (2 cs / eps)(rowsum(P)_i z1_i + (P z)_i) - lambda (2 / eps) r1_i,
+//   V_ij = P_ij (-(2 cs / eps)(z1_i + z_j) + lambda (4 cs / eps) F_ij).
+// So three contractions over the columns or the points carry everything: x.y, A.y and V.y (formed
+// plan by plan it was two matrix products and four vector products for the right-hand side, one
+// more product and the second-order term, each evaluating the plan anew: nine evaluations at
+// about 500 us and five products at 1.1 ms more at 8192 x 8192 x 1536).  Everything else reads the two kept
+// matrices once per pass and is bound by memory.
+#pragma once
+
+#include "fs_dense.hpp"
+
+namespace fs {
+
+struct HvpArgs {
+  const void* x;
+  const void* y;
+  const float* A;
+  const float* f;            // potentials with P_ij = exp((f_i + g_j - C_ij) / eps)
+  const float* g;
+  float* out;
+  int n, m, d, ld, dtype;
+  float eps, cs, lambda, fac_x, fac_y, floor, ridge;
+  float qs;                  // base-2 logit per unit of x.y
+  const float* dots;         // [n][ld] x.y
+  const float* prod;         // [n][ld] A.y
+  const float* norm_x;       // cs |x|^2, cs |y|^2, cs |A|^2
+  const float* norm_y;
+  const float* norm_a;
+  float* xa;                 // [n] x.A
+  float* ra;                 // [n] base-2 potential minus norm
+  float* cb;                 // [ld]
+  float2* row_part;          // [chunks][n]: sums of P and of P F
+  float2* col_part;          // [groups][m]
+  int chunk, chunks, groups;
+  float* mass;               // [n]
+  float* r1;
+  float* inv_diag;
+  float* w;                  // [n] r1 / diag_x
+  float* denom;              // [m]
+  float* r2;
+  float* strip_part;         // [strips][ld]
+  int strip_rows, strips;
+  float* vec;                // [m] the vector the strips multiply by
+  float* alpha;              // [n] -(2 cs / eps) z1
+  float* s;                  // [n]
+  float* limits;             // largest |z|, largest |y|
+  float* v_scale;            // [n] power-of-two scale of a row of V
+  u32x4* vplanes;            // [n blocks][ld / 16][2][64]
+  u32x4* yt;                 // [column blocks][ld / 16][2][64]
+  int yt_blocks;
+  const float2* scale;       // of x, y
+  const float* prod_out;     // [splits][n][ldo]
+  int ldo, splits;
+  float* cg;                 // state (see fs_cg.hip)
+  float* sol;
+  float* res;
+  float* a_dir;
+};
+
+// x_i.A_i and the base-2 biases: a wavefront per row, the rows of y behind those of x.
+template <int T>
+__global__ __launch_bounds__(256) void hvp_rows_kernel(const HvpArgs a) {
+  const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const float k = kLog2e / a.eps;
+  if (row < a.n) {
+    float s = 0.f;
+    for (int c = lane; c < a.d; c += 64)
+      s = __builtin_fmaf(small_load(a.x, (size_t)row * a.d + c, a.dtype), a.A[(size_t)row * a.d + c], s);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+    if (lane == 0) {
+      a.xa[row] = s;
+      a.ra[row] = k * (a.f[row] - a.norm_x[row]);
+    }
+  } else if (row - a.n < a.ld && lane == 0) {
+    const int j = row - a.n;
+    a.cb[j] = j < a.m ? k * (a.g[j] - a.norm_y[j]) : kNegBig;
+  }
+}
+
+// Sums of P and of P F along rows and columns, from one reading of both matrices: the shape of
+// dense_sweep_kernel, without maxima (the plan's entries are what they are).
+template <int WV>
+__global__ __launch_bounds__(64 * WV, 4) void hvp_mass_kernel(const HvpArgs a) {
+  constexpr int RW = 8;
+  __shared__ float2 sh[2][WV][256];
+  const int group = blockIdx.x, ch = blockIdx.y;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int r0 = (group * WV + wave) * RW;
+  const int mine = min(r0 + (lane & (RW - 1)), a.n - 1);
+  const float rb = r0 + (lane & (RW - 1)) < a.n ? a.ra[mine] : kNegBig, xa = a.xa[mine];
+  float rp[RW], rf[RW];
+#pragma unroll
+  for (int r = 0; r < RW; ++r) rp[r] = rf[r] = 0.f;
+  const int c_end = min(a.ld, (ch + 1) * a.chunk);
+  int buf = 0;
+  for (int c0 = ch * a.chunk; c0 < c_end; c0 += 256, buf ^= 1) {
+    float kb[4], cp[4], cf[4];
+    *reinterpret_cast<float4*>(kb) = *reinterpret_cast<const float4*>(a.cb + c0 + 4 * lane);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) cp[k] = cf[k] = 0.f;
+#pragma unroll
+    for (int r = 0; r < RW; ++r) {
+      const size_t at = (size_t)min(r0 + r, a.n - 1) * a.ld + c0 + 4 * lane;
+      float v[4], e[4];
+      *reinterpret_cast<float4*>(v) = *reinterpret_cast<const float4*>(a.dots + at);
+      *reinterpret_cast<float4*>(e) = *reinterpret_cast<const float4*>(a.prod + at);
+      const float br = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, rb), r));
+      const float xr = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, xa), r));
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const float p = fast_exp2(__builtin_fmaf(v[k], a.qs, br + kb[k])), t = p * (xr - e[k]);
+        rp[r] += p;
+        rf[r] += t;
+        cp[k] += p;
+        cf[k] += t;
+      }
+      if (r % 4 == 3) __builtin_amdgcn_sched_barrier(0);  // (four rows' loads at a time: registers)
+    }
+    float4* o = reinterpret_cast<float4*>(&sh[buf][wave][4 * lane]);
+    o[0] = make_float4(cp[0], cf[0], cp[1], cf[1]);
+    o[1] = make_float4(cp[2], cf[2], cp[3], cf[3]);
+    __syncthreads();  // (the other buffer is free once everyone is here)
+    for (int c = threadIdx.x; c < 256; c += 64 * WV) {
+      float2 s = sh[buf][0][c];
+#pragma unroll
+      for (int w = 1; w < WV; ++w) s.x += sh[buf][w][c].x, s.y += sh[buf][w][c].y;
+      if (c0 + c < a.m) a.col_part[(size_t)group * a.m + c0 + c] = s;
+    }
+  }
+#pragma unroll
+  for (int o = 32, n = RW / 2; n > 0; o >>= 1, n >>= 1) {
+    const bool up = lane & o;
+#pragma unroll
+    for (int r = 0; r < n; ++r) {
+      const float gp = up ? rp[r] : rp[r + n], gf = up ? rf[r] : rf[r + n];
+      rp[r] = (up ? rp[r + n] : rp[r]) + __shfl_xor(gp, o, 64);
+      rf[r] = (up ? rf[r + n] : rf[r]) + __shfl_xor(gf, o, 64);
+    }
+  }
+#pragma unroll
+  for (int o = 32 / RW; o > 0; o >>= 1) {
+    rp[0] += __shfl_xor(rp[0], o, 64);
+    rf[0] += __shfl_xor(rf[0], o, 64);
+  }
+  const int row = r0 + lane / (64 / RW);
+  if (lane % (64 / RW) == 0 && row < a.n) a.row_part[(size_t)ch * a.n + row] = make_float2(rp[0], rf[0]);
+}
+
+// Diagonals and right-hand sides from those sums: 64 rows of one side per workgroup.
+template <int T>
+__global__ __launch_bounds__(256) void hvp_merge_kernel(const HvpArgs a) {
+  const int side = blockIdx.y, rows = side ? a.m : a.n, parts = side ? a.groups : a.chunks;
+  if ((int)blockIdx.x * 64 >= rows) return;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, row = blockIdx.x * 64 + lane;
+  const float2* p = (side ? a.col_part : a.row_part) + min(row, rows - 1);
+  float mass = 0.f, t = 0.f;
+#pragma unroll 8
+  for (int c = wave; c < parts; c += 4) {
+    const float2 v = p[(size_t)c * rows];
+    mass += v.x;
+    t += v.y;
+  }
+  __shared__ float2 sh[4][64];
+  sh[wave][lane] = make_float2(mass, t);
+  __syncthreads();
+  if (wave > 0 || row >= rows) return;
+#pragma unroll
+  for (int w = 1; w < 4; ++w) mass += sh[w][lane].x, t += sh[w][lane].y;
+  const float r = 2.0f * a.cs * t, diag = (side ? a.fac_y : a.fac_x) * fmaxf(mass, a.floor);
+  if (side) {
+    a.denom[row] = diag + a.ridge;
+    a.r2[row] = r;
+  } else {
+    a.mass[row] = mass;
+    a.r1[row] = r;
+    a.inv_diag[row] = 1.0f / diag;
+    a.w[row] = r / diag;
+  }
+}
+
+// Whole rows of the plan in registers: a workgroup owns `strip_rows` rows, R at a time, its 512
+// threads 4 CP columns each.  MODE 0: column sums of P_ij w_i; 1: the same with w = P vec / diag_x, so
+// that one reading serves both products of a Schur-complement step; 2: P vec alone, and what the
+// result needs of it.  Bound by memory; the next R rows are in flight while the sums cross the workgroup.
+template <int CP, int R, int MODE>
+__global__ __launch_bounds__(512, 2) void hvp_strip_kernel(const HvpArgs a) {
+  if (MODE == 1 && a.cg[4] != 0.f) return;  // converged: what was enqueued behind it does nothing
+  __shared__ float sh[2][8][R];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int first = blockIdx.x * a.strip_rows, last = min(a.n, first + a.strip_rows);
+  float4 cb[CP], v[CP], acc[CP], p[R][CP], next[R][CP];
+  bool in[CP];
+#pragma unroll
+  for (int c = 0; c < CP; ++c) {
+    const int col = 4 * (tid + 512 * c);
+    in[c] = col < a.ld;
+    cb[c] = in[c] ? *reinterpret_cast<const float4*>(a.cb + col) : make_float4(kNegBig, kNegBig, kNegBig, kNegBig);
+    acc[c] = make_float4(0.f, 0.f, 0.f, 0.f);
+    v[c] = acc[c];
+    if (MODE > 0) {
+      v[c].x = col < a.m ? a.vec[col] : 0.f;
+      v[c].y = col + 1 < a.m ? a.vec[col + 1] : 0.f;
+      v[c].z = col + 2 < a.m ? a.vec[col + 2] : 0.f;
+      v[c].w = col + 3 < a.m ? a.vec[col + 3] : 0.f;
+    }
+  }
+  auto load = [&](int i0) {
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+      for (int c = 0; c < CP; ++c)
+        next[r][c] = *reinterpret_cast<const float4*>(a.dots + (size_t)min(i0 + r, a.n - 1) * a.ld + (in[c] ? 4 * (tid + 512 * c) : 0));
+  };
+  load(first);
+  int buf = 0;
+  for (int i0 = first; i0 < last; i0 += R, buf ^= 1) {
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+      for (int c = 0; c < CP; ++c) p[r][c] = next[r][c];
+    if (i0 + R < last) load(i0 + R);
+    float s[R], wr[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const float b = i0 + r < last ? a.ra[i0 + r] : kNegBig;
+      wr[r] = MODE == 0 ? (i0 + r < last ? a.w[i0 + r] : 0.f) : (MODE == 1 ? a.inv_diag[min(i0 + r, a.n - 1)] : 0.f);
+      s[r] = 0.f;
+#pragma unroll
+      for (int c = 0; c < CP; ++c) {
+        float4& q = p[r][c];
+        q.x = fast_exp2(__builtin_fmaf(q.x, a.qs, b + cb[c].x));
+        q.y = fast_exp2(__builtin_fmaf(q.y, a.qs, b + cb[c].y));
+        q.z = fast_exp2(__builtin_fmaf(q.z, a.qs, b + cb[c].z));
+        q.w = fast_exp2(__builtin_fmaf(q.w, a.qs, b + cb[c].w));
+        if (MODE > 0) s[r] += (q.x * v[c].x + q.y * v[c].y) + (q.z * v[c].z + q.w * v[c].w);
+      }
+    }
+    if (MODE > 0) {
+      // over the wavefront: halves of the rows change places, then over the eight of them
+#pragma unroll
+      for (int o = 32, n = R / 2; n > 0; o >>= 1, n >>= 1) {
+        const bool up = lane & o;
+#pragma unroll
+        for (int r = 0; r < n; ++r) {
+          const float g = up ? s[r] : s[r + n];
+          s[r] = (up ? s[r + n] : s[r]) + __shfl_xor(g, o, 64);
+        }
+      }
+#pragma unroll
+      for (int o = 32 / R; o > 0; o >>= 1) s[0] += __shfl_xor(s[0], o, 64);
+      if (lane % (64 / R) == 0) sh[buf][wave][lane / (64 / R)] = s[0];
+      __syncthreads();
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        float t = 0.f;
+#pragma unroll
+        for (int w = 0; w < 8; ++w) t += sh[buf][w][r];
+        s[r] = t;
+        if (MODE == 1) wr[r] *= t;
+      }
+      if (MODE == 2 && tid < R && i0 + tid < last) {
+        float pz = 0.f;
+#pragma unroll
+        for (int r = 0; r < R; ++r) pz = tid == r ? s[r] : pz;
+        const int i = i0 + tid;
+        const float z1 = a.w[i] - pz * a.inv_diag[i], k = 2.0f * a.cs / a.eps;
+        a.alpha[i] = -k * z1;
+        a.s[i] = k * (a.mass[i] * z1 + pz) - a.lambda * (2.0f / a.eps) * a.r1[i];
+      }
+    }
+    if (MODE < 2) {
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int c = 0; c < CP; ++c) {
+          acc[c].x = __builtin_fmaf(p[r][c].x, wr[r], acc[c].x);
+          acc[c].y = __builtin_fmaf(p[r][c].y, wr[r], acc[c].y);
+          acc[c].z = __builtin_fmaf(p[r][c].z, wr[r], acc[c].z);
+          acc[c].w = __builtin_fmaf(p[r][c].w, wr[r], acc[c].w);
+        }
+    }
+  }
+  if (MODE < 2)
+#pragma unroll
+    for (int c = 0; c < CP; ++c)
+      if (in[c]) *reinterpret_cast<float4*>(a.strip_part + (size_t)blockIdx.x * a.ld + 4 * (tid + 512 * c)) = acc[c];
+}
+
+// The strips' column sums: MODE 0 leaves r2 - sum in a_dir (the right-hand side), 1 the
+// Schur-complement product denom vec - sum.
+template <int MODE>
+__global__ __launch_bounds__(256) void hvp_columns_kernel(const HvpArgs a) {
+  if (MODE == 1 && a.cg[4] != 0.f) return;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, col = blockIdx.x * 64 + lane;
+  float t = 0.f;
+#pragma unroll 8
+  for (int g = wave; g < a.strips; g += 4) t += a.strip_part[(size_t)g * a.ld + col];
+  __shared__ float sh[4][64];
+  sh[wave][lane] = t;
+  __syncthreads();
+  if (wave > 0 || col >= a.m) return;
+  t = (sh[0][lane] + sh[1][lane]) + (sh[2][lane] + sh[3][lane]);
+  a.a_dir[col] = MODE == 0 ? a.r2[col] - t : __builtin_fmaf(a.denom[col], a.vec[col], -t);
+}
+
+// Largest |z| and |y_j|, for the scales of V's rows.
+template <int T>
+__global__ __launch_bounds__(1024) void hvp_limits_kernel(const HvpArgs a) {
+  float z = 0.f, y = 0.f;
+  for (int j = threadIdx.x; j < a.m; j += 1024) z = fmaxf(z, fabsf(a.sol[j])), y = fmaxf(y, a.norm_y[j]);
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) z = fmaxf(z, __shfl_xor(z, o, 64)), y = fmaxf(y, __shfl_xor(y, o, 64));
+  __shared__ float sh[2][16];
+  if ((threadIdx.x & 63) == 0) sh[0][threadIdx.x >> 6] = z, sh[1][threadIdx.x >> 6] = y;
+  __syncthreads();
+  if (threadIdx.x > 0) return;
+  for (int w = 1; w < 16; ++w) z = fmaxf(z, sh[0][w]), y = fmaxf(y, sh[1][w]);
+  a.limits[0] = z;
+  a.limits[1] = sqrtf(y / a.cs);
+}
+
+// Power of two that takes a row of V below 2^15 (f16_plane_scale without its clamp at 2^40: the
+// plan of a cloud with many points is small).
+__device__ __forceinline__ float hvp_scale(float most) {
+  const int e = (int)((__builtin_bit_cast(unsigned, most) >> 23) & 255u);
+  if (e == 0 || e == 255) return 1.0f;
+  return __builtin_bit_cast(float, (unsigned)max(1, min(253, 127 + 14 - (e - 127))) << 23);
+}
+
+// Planes of V, 32 rows x 256 columns per workgroup: read in rows of 1 KiB, turned into operand order in
+// LDS (units of one plane, 16-column step and half-wave, 512 + 16 bytes apart so that the eight
+// units that 64 lanes write at a time lie on different banks).  Bound by memory.
+template <int T>
+__global__ __launch_bounds__(256) void hvp_v_kernel(const HvpArgs a) {
+  constexpr int UNIT = 528;
+  __shared__ __attribute__((aligned(16))) unsigned char lds[2 * 32 * UNIT];
+  const int blk = blockIdx.x, c0 = blockIdx.y * 256;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const float k2 = 2.0f * a.cs / a.eps, k4 = a.lambda * 4.0f * a.cs / a.eps;
+  const float zmax = a.limits[0], ymax = a.limits[1];
+  float kb[4], z[4];
+  *reinterpret_cast<float4*>(kb) = *reinterpret_cast<const float4*>(a.cb + c0 + 4 * lane);
+#pragma unroll
+  for (int k = 0; k < 4; ++k) z[k] = c0 + 4 * lane + k < a.m ? k2 * a.sol[c0 + 4 * lane + k] : 0.f;
+#pragma unroll
+  for (int r = 0; r < 8; ++r) {
+    const int i = wave * 8 + r, row = blk * 32 + i, rc = min(row, a.n - 1);
+    const size_t at = (size_t)rc * a.ld + c0 + 4 * lane;
+    float v[4], e[4];
+    *reinterpret_cast<float4*>(v) = *reinterpret_cast<const float4*>(a.dots + at);
+    *reinterpret_cast<float4*>(e) = *reinterpret_cast<const float4*>(a.prod + at);
+    const float b = row < a.n ? a.ra[rc] : kNegBig, al = a.alpha[rc], xa = a.xa[rc];
+    // |F_ij| <= |x_i.A_i| + |A_i| |y_j|, P_ij <= the row's sum
+    const float most = a.mass[rc] * (fabsf(al) + k2 * zmax + fabsf(k4) * (fabsf(xa) + sqrtf(a.norm_a[rc] / a.cs) * ymax));
+    const float sc = hvp_scale(most);
+    if (c0 == 0 && lane == 0 && row < a.n) a.v_scale[row] = sc;
+    _Float16 hi[4], lo[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const float p = fast_exp2(__builtin_fmaf(v[k], a.qs, b + kb[k]));
+      const float t = sc * p * (al - z[k] + k4 * (xa - e[k]));
+      hi[k] = (_Float16)t;
+      lo[k] = (_Float16)(t - (float)hi[k]);
+    }
+    // columns 4 lane .. 4 lane + 3: step lane / 4, half-wave lane / 2 % 2, half of its 16 bytes
+    unsigned char* o = lds + (lane >> 1) * UNIT + i * 16 + (lane & 1) * 8;
+    *reinterpret_cast<uint2*>(o) = make_uint2(pack_f16((float)hi[0], (float)hi[1]), pack_f16((float)hi[2], (float)hi[3]));
+    *reinterpret_cast<uint2*>(o + 32 * UNIT) =
+        make_uint2(pack_f16((float)lo[0], (float)lo[1]), pack_f16((float)lo[2], (float)lo[3]));
+  }
+  __syncthreads();
+  u32x4* out = a.vplanes + ((size_t)blk * (a.ld / 16) + c0 / 16) * kDenseStep;
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    const int w = threadIdx.x + 256 * q;  // 16-byte word: [step][plane][half-wave][row]
+    const int kk = w >> 7, plane = (w >> 6) & 1, half = (w >> 5) & 1, i = w & 31;
+    out[w] = *reinterpret_cast<const u32x4*>(lds + (plane * 32 + kk * 2 + half) * UNIT + i * 16);
+  }
+}
+
+// Planes of y^T: the rows are y's columns.  A wavefront per 32 columns and 16 points.
+template <int T>
+__global__ __launch_bounds__(256) void hvp_yt_kernel(const HvpArgs a) {
+  const int blk = blockIdx.y, kk = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (kk >= a.ld / 16) return;
+  const int col = blk * 32 + (lane & 31), j0 = 16 * kk + 8 * (lane >> 5);
+  const float sc = a.scale[1].x;
+  float v[8];
+#pragma unroll
+  for (int q = 0; q < 8; ++q)
+    v[q] = col < a.d && j0 + q < a.m ? sc * small_load(a.y, (size_t)(j0 + q) * a.d + col, a.dtype) : 0.f;
+  u32x4 hi, lo;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const _Float16 h0 = (_Float16)v[2 * q], h1 = (_Float16)v[2 * q + 1];
+    hi[q] = pack_f16((float)h0, (float)h1);
+    lo[q] = pack_f16(v[2 * q] - (float)h0, v[2 * q + 1] - (float)h1);
+  }
+  u32x4* out = a.yt + ((size_t)blk * (a.ld / 16) + kk) * kDenseStep + lane;
+  out[0] = hi;
+  out[64] = lo;
+}
+
+// The result.
+template <int T>
+__global__ __launch_bounds__(256) void hvp_result_kernel(const HvpArgs a) {
+  const size_t count = (size_t)a.n * a.d;
+  for (size_t e = (size_t)blockIdx.x * 256 + threadIdx.x; e < count; e += (size_t)gridDim.x * 256) {
+    const int row = (int)(e / a.d), col = (int)(e - (size_t)row * a.d);
+    float v = 0.f;
+    for (int s = 0; s < a.splits; ++s) v += a.prod_out[((size_t)s * a.n + row) * a.ldo + col];
+    v *= a.scale[1].y / a.v_scale[row];
+    a.out[e] = a.s[row] * small_load(a.x, e, a.dtype) + 2.0f * a.cs * a.mass[row] * a.A[e] + v;
+  }
+}
+
+}  // namespace fs

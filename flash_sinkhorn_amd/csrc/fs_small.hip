@@ -3,7 +3,6 @@
 
 #include <algorithm>
 #include <atomic>
-#include <chrono>
 #include <cmath>
 #include <cstring>
 #include <type_traits>
@@ -11,6 +10,7 @@
 
 #include "flash_sinkhorn_hip.h"
 #include "fs_dense.hpp"
+#include "fs_host.hpp"
 #include "fs_pair.hpp"
 #include "fs_small.hpp"
 
@@ -350,20 +350,6 @@ int launch_pair_step(const SmallArgs& a, PairArgs& t, int step, hipStream_t st) 
   const int blocks = (t.total_items + 7) / 8 * 8;
   hipLaunchKernelGGL((pair_sweep_kernel<DP>), dim3(blocks, a.items), dim3(256), 0, st, t);
   return launch_pair_merge<DP>(a, t, step, st);
-}
-
-// Looks at pinned words until `arrived` says that what the device has to write is there (it
-// arrives a few microseconds after the kernel wrote it); after two milliseconds waits for the
-// stream instead.
-template <typename F>
-int wait_for_words(hipStream_t st, F&& arrived) {
-  const auto t0 = std::chrono::steady_clock::now();
-  for (int looks = 1; !arrived(); ++looks)
-    if (looks % 64 == 0 && std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(2)) {
-      if (hipStreamSynchronize(st) != hipSuccess) return FS_ERR_LAUNCH_FAILED;
-      return arrived() ? FS_OK : FS_ERR_LAUNCH_FAILED;
-    }
-  return FS_OK;
 }
 
 template <int DP>

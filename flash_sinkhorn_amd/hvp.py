@@ -15,7 +15,9 @@ torch.compile, batched, fused two-phase matvec) are not built.
 """
 from __future__ import annotations
 
+import ctypes
 import math
+import threading
 from dataclasses import dataclass
 from typing import Optional, Sequence, Tuple
 
@@ -70,6 +72,54 @@ def sinkhorn_prelast_potentials_sqeuclid(
     return f_grad, g_grad
 
 
+_P, _I64, _F, _I = ctypes.c_void_p, ctypes.c_int64, ctypes.c_float, ctypes.c_int
+
+
+class _Problem(ctypes.Structure):
+    """``fs_hvp_problem``."""
+    _fields_ = [("x", _P), ("y", _P), ("A", _P), ("f", _P), ("g", _P), ("n", _I64), ("m", _I64),
+                ("d", _I64), ("eps", _F), ("cost_scale", _F), ("rho_x", _F), ("rho_y", _F),
+                ("tau2", _F), ("lambda_indef", _F), ("rtol", _F), ("atol", _F), ("dtype", _I),
+                ("max_iter", _I)]
+
+
+_DTYPES = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}
+_KEPT_MAX_COLUMNS = 8192
+_KEPT_MAX = 1 << 26  # entries of the plan
+_state = threading.local()
+
+
+def _kept_ok(n: int, m: int, d: int, allow_tf32: bool) -> bool:
+    """Whether the product is taken on kept matrices (``fs_hvp``): they stay below 1 GiB together."""
+    return (0 < n <= 65536 and 0 < m <= _KEPT_MAX_COLUMNS and d > 0 and n * m <= _KEPT_MAX
+            and (allow_tf32 or _lib.STRICT_OPERANDS == "fp16x2")
+            and not torch.cuda.is_current_stream_capturing())
+
+
+def _kept(x, y, f_hat, g_hat, A, *, eps, cost_scale, rho_x, rho_y, tau2, lambda_indef, rtol, atol,
+          max_iter):
+    """One library call: three contractions, the rest passes over kept matrices."""
+    if x.dtype not in _DTYPES or y.dtype is not x.dtype:
+        x, y = x.float(), y.float()
+    x, y, A, f, g = x.detach().contiguous(), y.detach().contiguous(), *(
+        t.detach().float().contiguous() for t in (A, f_hat, g_hat))
+    host = getattr(_state, "words", None)
+    if host is None:
+        host = _state.words = torch.empty(8, dtype=torch.float32, pin_memory=True)
+    (n, d), m = x.shape, y.shape[0]
+    p = _Problem(x.data_ptr(), y.data_ptr(), A.data_ptr(), f.data_ptr(), g.data_ptr(), n, m, d,
+                 eps, cost_scale, 0.0 if rho_x is None else float(rho_x),
+                 0.0 if rho_y is None else float(rho_y), tau2, lambda_indef, rtol, atol,
+                 _DTYPES[x.dtype], max(0, max_iter))
+    L = _lib.lib()
+    ws = torch.empty(L.fs_hvp_workspace_bytes(ctypes.byref(p)), dtype=torch.uint8, device=x.device)
+    out = torch.empty((n, d), dtype=torch.float32, device=x.device)
+    _lib.check(L.fs_hvp(ctypes.byref(p), ws.data_ptr(), ws.numel(), out.data_ptr(),
+                        host.data_ptr(), _lib.stream_of(x)), "fs_hvp")
+    r0, r, converged, iters = (float(host[i]) for i in (1, 3, 5, 6))
+    return out, HvpInfo(converged != 0.0, int(iters) if converged else max_iter, r, r0)
+
+
 def hvp_x_sqeuclid_from_potentials(
     x: torch.Tensor, y: torch.Tensor, f_hat: torch.Tensor, g_hat: torch.Tensor, A: torch.Tensor, *,
     eps: float, rho_x: Optional[float] = None, rho_y: Optional[float] = None,
@@ -109,6 +159,11 @@ def hvp_x_sqeuclid_from_potentials(
 
     e = float(eps)
     cs = float(cost_scale)
+    if (mode == "none" and cg_x0 is None and not cg_stabilise_every and not return_components
+            and _kept_ok(n, m, d, allow_tf32) and e > 0.0 and cs > 0.0):
+        return _kept(x, y, f_hat, g_hat, A, eps=e, cost_scale=cs, rho_x=rho_x, rho_y=rho_y,
+                     tau2=float(tau2), lambda_indef=float(lambda_indef), rtol=float(cg_rtol),
+                     atol=float(cg_atol), max_iter=int(max_cg_iter))
     xf, yf, Af = x.float().contiguous(), y.float().contiguous(), A.float().contiguous()
     x_sq = (xf * xf).sum(dim=1).contiguous()
     y_sq = (yf * yf).sum(dim=1).contiguous()

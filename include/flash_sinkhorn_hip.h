@@ -444,6 +444,32 @@ int fs_small_solve(const fs_small_problem* problem, void* workspace, size_t work
 int fs_small_grad(const fs_small_problem* problem, void* workspace, size_t workspace_bytes,
                   const float* grad_out, float* grad_x, float* grad_y, void* stream);
 
+/*
+ * out [n, d] = H A, the Hessian of the cost in x times A [n, d] (fp32), at potentials f [n], g [m] with
+ * P_ij = exp((f_i + g_j - cost_scale |x_i - y_j|^2) / eps); x, y of `dtype` (0 fp32, 1 fp16, 2 bf16).
+ * rho_x, rho_y <= 0: strict marginals; tau2 then regularises the Schur complement (eps * tau2).
+ * lambda_indef weighs the indefinite part.  Conjugate gradients without preconditioner, stopped
+ * at max(atol, rtol * |r0|).  Keeps two n x m matrices and a pair of planes of one (12 n m bytes of workspace);
+ * at most FS_HVP_MAX_COLUMNS rows of y.  host_state: 8 words of PINNED host memory; the call waits
+ * for the device.  Afterwards [1] |r0|, [3] |r|, [5] converged, [6] iterations.
+ * Replaces hvp_x_sqeuclid_from_potentials (hvp.py:164-623) for these sizes.
+ */
+#define FS_HVP_MAX_COLUMNS 8192
+typedef struct fs_hvp_problem {
+  const void* x;
+  const void* y;
+  const float* A;
+  const float* f;
+  const float* g;
+  int64_t n, m, d;
+  float eps, cost_scale, rho_x, rho_y, tau2, lambda_indef, rtol, atol;
+  int dtype, max_iter;
+} fs_hvp_problem;
+
+size_t fs_hvp_workspace_bytes(const fs_hvp_problem* problem);
+int fs_hvp(const fs_hvp_problem* problem, void* workspace, size_t workspace_bytes, float* out, float* host_state,
+           void* stream);
+
 #ifdef __cplusplus
 }
 #endif
