@@ -337,10 +337,10 @@ template <int DP>
 int launch_pair_merge(const SmallArgs& a, PairArgs& t, int step, hipStream_t st) {
   pair_step_args(a, t, step);
   const int blocks = std::max(a.pblocks[0], a.pblocks[1]);
-  t.merge_groups = (blocks + 1) / 2;
+  t.merge_groups = (blocks + 7) / 8;
   // (at one eps the planes are written once, before the first step)
-  const int grid = t.merge_groups + (step < 0 || a.sched != 0 ? blocks : 0);
-  hipLaunchKernelGGL((pair_merge_kernel<DP>), dim3(grid, a.self == 1 ? 4 : 2, a.items), dim3(256), 0, st, t);
+  const int grid = t.merge_groups + (step < 0 || a.sched != 0 ? (blocks + 3) / 4 : 0);
+  hipLaunchKernelGGL((pair_merge_kernel<DP>), dim3(grid, a.self == 1 ? 4 : 2, a.items), dim3(1024), 0, st, t);
   return hipGetLastError() == hipSuccess ? FS_OK : FS_ERR_LAUNCH_FAILED;
 }
 
