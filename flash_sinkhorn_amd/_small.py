@@ -39,7 +39,7 @@ class Problem(ctypes.Structure):
                 ("cost_scale", _F), ("eps", _F), ("rho_x", _F), ("rho_y", _F), ("threshold", _F),
                 ("dtype", _I), ("normalize", _I), ("self_terms", _I), ("want_values", _I),
                 ("sched", _I), ("entries", _I), ("cut", _I), ("extrapolate", _I),
-                ("check_every", _I)]
+                ("check_every", _I), ("alternating", _I)]
 
 
 class LongSchedule(Exception):
@@ -113,7 +113,8 @@ def _rho(rho: Optional[float]) -> float:
 def solve(x, y, a, b, *, items: int, blur: float = 0.0, scaling: float = 0.0, eps: float = 0.0,
           entries: int = 0, cut: int = 0, eps_list=None, cost_scale: float, rho_x, rho_y,
           normalize: bool, self_terms: int, want_values: bool, extrapolate: bool,
-          want_loss: bool, threshold: Optional[float] = None, check_every: int = 1) -> Solved:
+          want_loss: bool, threshold: Optional[float] = None, check_every: int = 1,
+          alternating: bool = False) -> Solved:
     """Enqueue one run of small problems: contiguous x [items, n, d] and y [items, m, d] of one dtype,
     weights as contiguous fp32 or None.  ``eps_list`` (host floats), ``eps`` with ``entries``, or
     a schedule by diameter, in that order."""
@@ -133,7 +134,7 @@ def solve(x, y, a, b, *, items: int, blur: float = 0.0, scaling: float = 0.0, ep
             None if table is None else ctypes.addressof(table), n, m, d, items, blur, scaling,
             cost_scale, eps, _rho(rho_x), _rho(rho_y), threshold or 0.0, _DTYPES[x.dtype],
             int(normalize), int(self_terms), int(want_values), sched, entries, cut,
-            int(extrapolate), int(check_every))
+            int(extrapolate), int(check_every), int(alternating))
 
     rows = (n + m) * items * (4 if self_terms else 2)
 
@@ -159,7 +160,8 @@ def solve(x, y, a, b, *, items: int, blur: float = 0.0, scaling: float = 0.0, ep
     if (sched == 0 and not threshold and _graphs.eligible(n, m, entries, x.device)
             and (d <= WIDE_D or items * n * m <= 1 << 22)):  # (a graph keeps its products)
         # a fixed sequence of kernels on fixed shapes: replayed (1.9 instead of 3 us per launch)
-        key = ("self pair" if self_terms else "symmetric", int(self_terms), x.device.index, x.dtype, items, n, m, d,
+        key = ("self pair" if self_terms else "alternating" if alternating else "symmetric",
+               int(self_terms), x.device.index, x.dtype, items, n, m, d,
                eps, entries, cost_scale, _rho(rho_x), _rho(rho_y), a is None, b is None, normalize,
                want_values, extrapolate, want_loss)
         ws, out = _graphs.run(key, enqueue, [x, y, a, b])
@@ -188,28 +190,41 @@ def points(x, y):
 
 
 def pair_problem(x, y, a, b, allow_tf32: bool, fixed: bool, self_terms: int = 0,
-                 stops: bool = False) -> bool:
+                 stops: bool = False, any_size: bool = False) -> bool:
     """Whether clouds and weights (any of which may need a gradient) are ones ``solve`` takes."""
     return (x.is_cuda and y.is_cuda and x.ndim == 2 and y.ndim == 2 and a.ndim == 1 and b.ndim == 1
             and x.shape[1] == y.shape[1]
-            and _size_ok(x.shape[0], y.shape[0], x.shape[1], fixed, self_terms, stops)
-            # (a solver called by itself keeps to the tile-skipping kernels where it has them)
-            and (x.shape[1] <= 8 or min(x.shape[0], y.shape[0]) < 24000)
+            and (0 < x.shape[1] <= WIDE_D if any_size else
+                 _size_ok(x.shape[0], y.shape[0], x.shape[1], fixed, self_terms, stops)
+                 # (a solver called by itself keeps to the tile-skipping kernels where it has them)
+                 and (x.shape[1] <= 8 or min(x.shape[0], y.shape[0]) < 24000))
+            and x.shape[0] > 0 and y.shape[0] > 0
             and a.shape[0] == x.shape[0] and b.shape[0] == y.shape[0]
             and x.is_floating_point() and y.is_floating_point() and _operands_ok(allow_tf32)
             and x.device == y.device == a.device == b.device)
 
 
-def solver_problem(x, y, a, b, allow_tf32: bool, fixed: bool, stops: bool) -> bool:
+def solver_problem(x, y, a, b, allow_tf32: bool, fixed: bool, stops: bool,
+                   any_size: bool = False) -> bool:
     """Whether ``sinkhorn_flashstyle_symmetric`` may hand its clouds and weights to ``solve``.  One cloud
     against itself, with wide rows or on more than a few thousand points, stays with the general
     path: one half-update per step instead of two, and f equal to g to the bit."""
-    if x.data_ptr() == y.data_ptr() and a.data_ptr() == b.data_ptr() and x.shape == y.shape \
+    if not any_size and x.data_ptr() == y.data_ptr() and a.data_ptr() == b.data_ptr() and x.shape == y.shape \
             and (x.shape[1] > WIDE_D or x.shape[0] ** 2 >= 20_000_000):
         return False
-    return pair_problem(x, y, a, b, allow_tf32, fixed, 0, stops) and not (
+    return pair_problem(x, y, a, b, allow_tf32, fixed, 0, stops, any_size) and not (
         torch.is_grad_enabled()
         and (x.requires_grad or y.requires_grad or a.requires_grad or b.requires_grad))
+
+
+def alternating_problem(x, y, a, b, allow_tf32: bool) -> bool:
+    """Whether ``sinkhorn_flashstyle_alternating`` may hand its clouds and weights to ``solve``: a
+    half-update is one launch of the small kernels, faster than the streaming kernels' two and
+    what PyTorch does around them up to 1.4e8 logits (12,000 x 12,000 x 16: 44 against 48 us a
+    half-update; 6,206 x 5,067 x 37: 25 against 35), 6.5e7 on 33 .. 64 columns, 3.6e7 on more."""
+    n, m, d = x.shape[0], y.shape[0], x.shape[-1]
+    return (solver_problem(x, y, a, b, allow_tf32, True, False, any_size=True)
+            and n * m <= (140_000_000 if d <= 32 else 65_000_000 if d <= 64 else 36_000_000))
 
 
 def _weights(w, lead, count, device, normalize):

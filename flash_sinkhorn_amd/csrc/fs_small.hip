@@ -37,7 +37,7 @@ __global__ __launch_bounds__(256) void small_table_kernel(const SmallArgs a, con
 // 0.58 against 0.62 ms).  Items of a batch fill the chip without it: 12 x 2,048 x 8, debiased, 0.81
 // against 0.66 ms.  Early stopping on a schedule is only built for the small kernels.
 bool use_pair(const fs_small_problem* p) {
-  if (p->d > 64 || (p->threshold > 0.f && p->sched != 0)) return false;
+  if (p->alternating || p->d > 64 || (p->threshold > 0.f && p->sched != 0)) return false;
   const double n = (double)p->n, m = (double)p->m;
   const double logits = (p->self_terms < 2 ? n * m : 0.) + (p->self_terms ? 0.5 * (n * n + m * m) : 0.);
   return logits >= (p->sched == 0 || p->d > 32 ? 2.0e7 : 5.0e7);
@@ -70,6 +70,7 @@ int checked(const fs_small_problem* p) {
       if (!(p->eps_list[i] > 0.f)) return FS_ERR_BAD_ARGUMENT;
   }
   if (p->threshold > 0.f && p->check_every <= 0) return FS_ERR_BAD_ARGUMENT;
+  if (p->alternating && (p->sched != 0 || p->self_terms || p->want_values || p->d > kSmallMaxD)) return FS_ERR_UNSUPPORTED;
   return p->self_terms < 0 || p->self_terms > 2 ? FS_ERR_BAD_ARGUMENT : FS_OK;
 }
 
@@ -201,7 +202,8 @@ size_t layout(const fs_small_problem* p, void* ws, SmallArgs& a, PairArgs* pa = 
   a.sched = p->sched;
   a.entries = p->entries;
   a.cut = p->cut;
-  a.extrapolate = p->extrapolate ? 1 : 0;
+  a.alternating = p->alternating ? 1 : 0;
+  a.extrapolate = p->extrapolate || p->alternating ? 1 : 0;  // (the parity of the last potentials)
   a.eps0 = p->eps;
   a.blur = p->blur;
   a.scaling = p->scaling;
@@ -323,14 +325,41 @@ SmallStepArgs step_args(const SmallArgs& a, int step) {
   return t;
 }
 
+// Wavefronts that share the keys of 32 rows: sixteen where eight would leave the chip half empty and
+// there are keys for them (3,001 x 4,567 x 33: 326 against 424 us a solve; from 257 workgroups on, and
+// at 128 columns, where they cost registers, eight are faster).
+template <int DP>
+int launch_small(const SmallStepArgs& t, dim3 grid, int64_t working, int key_blocks, hipStream_t st) {
+  if constexpr (DP <= 64)
+    if (working <= 256 && key_blocks >= 48) {
+      hipLaunchKernelGGL((small_step_kernel<DP, 16>), grid, dim3(1024), 0, st, t);
+      return hipGetLastError() == hipSuccess ? FS_OK : FS_ERR_LAUNCH_FAILED;
+    }
+  hipLaunchKernelGGL((small_step_kernel<DP, 8>), grid, dim3(512), 0, st, t);
+  return hipGetLastError() == hipSuccess ? FS_OK : FS_ERR_LAUNCH_FAILED;
+}
+
 template <int DP>
 int launch_step(const SmallArgs& a, int step, hipStream_t st) {
-  const int xb = a.blocks[0] > a.blocks[1] ? a.blocks[0] : a.blocks[1];
-  const dim3 grid(xb, a.self == 1 ? 4 : 2, a.items);
-  constexpr int W = 8;  // wavefronts that share the keys of 32 rows (16: slower from 700 points on)
-  const SmallStepArgs t = step_args(a, step);
-  hipLaunchKernelGGL((small_step_kernel<DP, W>), grid, dim3(64 * W), 0, st, t);
-  return hipGetLastError() == hipSuccess ? FS_OK : FS_ERR_LAUNCH_FAILED;
+  const int xb = std::max(a.blocks[0], a.blocks[1]);
+  return launch_small<DP>(step_args(a, step), dim3(xb, a.self == 1 ? 4 : 2, a.items),
+                          (int64_t)(a.blocks[0] + a.blocks[1]) * (a.self == 1 ? 2 : 1) * a.items, xb, st);
+}
+
+// One alternating iteration: f from the newest g, then g from that f.
+template <int DP>
+int launch_alternating(const SmallArgs& a, int it, hipStream_t st) {
+  for (int side = 0; side < 2; ++side) {
+    SmallStepArgs t = step_args(a, it);
+    t.side[0] = t.side[side];
+    t.full = 1;
+    t.extrapolate = -1;  // (iteration `it` is one of the first lens)
+    if (side == 1) t.side[0].kpot = a.pot[0] + ((it & 1) ^ 1) * (size_t)a.items * a.rows[0];
+    const int rc = launch_small<DP>(t, dim3(a.blocks[side], 1, a.items), (int64_t)a.blocks[side] * a.items,
+                                    a.blocks[side ^ 1], st);
+    if (rc != FS_OK) return rc;
+  }
+  return FS_OK;
 }
 
 template <int DP>
@@ -433,7 +462,7 @@ int fs_small_solve(const fs_small_problem* p, void* workspace, size_t workspace_
         if (k > entries) entries = k;
       }
   }
-  const int n_steps = entries + 1 + a.extrapolate;
+  const int n_steps = a.alternating ? entries : entries + 1 + a.extrapolate;
   const bool early = a.threshold > 0.f;
   std::vector<int> length;  // early stopping: entries of every problem's schedule
   if (early)
@@ -461,12 +490,14 @@ int fs_small_solve(const fs_small_problem* p, void* workspace, size_t workspace_
   for (int s = 0; s < n_steps && rc == FS_OK && !all_done; ++s) {
     rc = dense ? dense_step(a, da, s, st) : by_width(p->d, [&](auto dp) {
       constexpr int DP = decltype(dp)::value;
+      if (a.alternating) return launch_alternating<DP>(a, s, st);
       if constexpr (DP <= 64)
         if (a.pair) return launch_pair_step<DP>(a, pa, s, st);
       return launch_step<DP>(a, s, st);
     });
-    if (rc != FS_OK || !early || s == 0 || s > entries || s % p->check_every != 0) continue;
-    hipLaunchKernelGGL((small_check_kernel<0>), dim3(p1 - p0, a.items), dim3(1024), 0, st, a, s, checks);
+    const int done = a.alternating ? s + 1 : s;  // averaged steps or iterations
+    if (rc != FS_OK || !early || done == 0 || done > entries || done % p->check_every != 0) continue;
+    hipLaunchKernelGGL((small_check_kernel<0>), dim3(p1 - p0, a.items), dim3(1024), 0, st, a, done, checks);
     if (hipGetLastError() != hipSuccess) return FS_ERR_LAUNCH_FAILED;
     // (asked for with one more stretch of steps enqueued, so that the device does not wait)
     if (checks > 0) rc = check_result(checks - 1);

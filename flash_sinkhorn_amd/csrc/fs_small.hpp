@@ -59,6 +59,7 @@ struct SmallArgs {
   int* lens;              // [items][3] those the problem runs: fewer once it has converged
   int* host_words;        // pinned host memory, 4 words per item (see small_schedule, small_check_kernel)
   int host_token;
+  int alternating;        // full steps, one side after the other, from the newest potentials
   // early stopping (threshold > 0): the potentials of the last check
   float threshold;
   float* prev[4];         // [items][rows of the side]
@@ -452,6 +453,7 @@ struct SmallStepArgs {
   SmallStepSide side[4];
   const float4* scale;  // [items] scale of x, its inverse, scale of y, its inverse
   int step, extrapolate;
+  int full;             // alternating: full steps, the whole shifted potential is damped
 };
 
 // One step of every problem.  Grid (32-row blocks of the larger cloud, sides, items).
@@ -545,10 +547,10 @@ __global__ __launch_bounds__(64 * W) void small_step_kernel(const SmallStepArgs 
   }
   const float eps = coef.x, rho = sd.rho;
   const float damp = rho > 0.f ? 1.0f / (1.0f + eps / rho) : 1.0f;
-  const float alpha = (step == 0 || step > entries) ? 1.0f : 0.5f;
+  const float alpha = (a.full || step == 0 || step > entries) ? 1.0f : 0.5f;
   float r = alpha * (-eps * damp * kLn2 * small_log2(fmaxf(S, 1e-40f), M));
   if (alpha != 1.0f) r += (1.0f - alpha) * old;
-  if (damp < 1.0f) r -= alpha * (1.0f - damp) * shift;
+  if (damp < 1.0f && !a.full) r -= alpha * (1.0f - damp) * shift;
   sd.out[at] = r;
 }
 
@@ -561,14 +563,17 @@ template <int T>
 __global__ __launch_bounds__(1024) void small_check_kernel(const SmallArgs a, int step, int check) {
   const int prob = blockIdx.x + (a.self == 2 ? 1 : 0), item = blockIdx.y, tid = threadIdx.x;
   if (a.lens[item * 3 + prob] < step) return;  // stopped before, or a shorter schedule
+  const int newest = a.alternating ? step & 1 : (step & 1) ^ 1;
   const int s0 = prob == 0 ? 0 : 1 + prob, s1 = prob == 0 ? 1 : s0;
   float change = 0.f;
   for (int side = s0; side <= s1; ++side) {
     const int rows = a.rows[side & 1];
-    const float* now = a.pot[side] + ((size_t)((step & 1) ^ 1) * a.items + item) * rows;
+    const float* now = a.pot[side] + ((size_t)newest * a.items + item) * rows;
     float* prev = a.prev[side] + (size_t)item * rows;
     for (int i = tid; i < rows; i += 1024) {
-      const float d = fabsf(now[i] - prev[i]);
+      // (alternating: the first check compares with the initial potentials)
+      const float before = a.alternating && check == 0 ? -a.norm[side & 1][(size_t)item * rows + i] : prev[i];
+      const float d = fabsf(now[i] - before);
       change = d > change || !(d == d) ? d : change;
     }
   }
@@ -580,12 +585,12 @@ __global__ __launch_bounds__(1024) void small_check_kernel(const SmallArgs a, in
   }
   if ((tid & 63) == 0) sh[tid >> 6] = change;
   __syncthreads();
-  bool stop = check > 0;
+  bool stop = check > 0 || a.alternating;
   for (int w = 0; w < 16; ++w) stop = stop && sh[w] < a.threshold;
   if (!stop)
     for (int side = s0; side <= s1; ++side) {
       const int rows = a.rows[side & 1];
-      const float* now = a.pot[side] + ((size_t)((step & 1) ^ 1) * a.items + item) * rows;
+      const float* now = a.pot[side] + ((size_t)newest * a.items + item) * rows;
       float* prev = a.prev[side] + (size_t)item * rows;
       for (int i = tid; i < rows; i += 1024) prev[i] = now[i];
     }

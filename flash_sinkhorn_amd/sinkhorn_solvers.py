@@ -118,6 +118,19 @@ def sinkhorn_flashstyle_alternating(
     rho_x, rho_y = _resolve_rho(rho, reach, rho_x, rho_y, reach_x, reach_y)
     damp_f, damp_g = dampening(eps, rho_x), dampening(eps, rho_y)
     _require_cuda(x, y)
+    stops = threshold is not None and threshold > 0.0
+    if (not ott_convention and eps > 0.0 and int(n_iters) > 0
+            and not (stops and (check_every <= 0 or torch.cuda.is_current_stream_capturing()))
+            and (rho_x is None or rho_x > 0.0) and (rho_y is None or rho_y > 0.0)
+            and _small.alternating_problem(x, y, a, b, allow_tf32)):
+        s = _small.solve(*_small.points(x, y), _f32c(a.detach()), _f32c(b.detach()), items=1,
+                         eps=float(eps), entries=int(n_iters), cost_scale=float(cost_scale),
+                         rho_x=rho_x, rho_y=rho_y, normalize=False, self_terms=0,
+                         want_values=False, extrapolate=False, want_loss=False,
+                         threshold=threshold if stops else None, check_every=check_every,
+                         alternating=True)
+        f, g = s.potentials("f")[0][0], s.potentials("g")[0][0]
+        return (f, g, s.entries) if return_n_iters else (f, g)
     xf, yf = x.float().contiguous(), y.float().contiguous()
     alpha = cost_scale * (xf * xf).sum(dim=1)
     beta = cost_scale * (yf * yf).sum(dim=1)

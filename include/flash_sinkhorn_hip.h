@@ -402,6 +402,10 @@ int fs_c_transform(const float* x, const float* y, const float* bias, float* min
  * live until then.
  *   threshold  > 0: a problem none of whose potentials moved by it between two checks, one every
  *              check_every averaged steps (the first only takes a snapshot), runs no more entries
+ *   alternating  (sched 0, d <= 128, no self problems or values) `entries` iterations of f from the newest
+ *              g, then g from that f, in full steps, the whole shifted potential damped; the first check
+ *              compares with the initial potentials (sinkhorn_flashstyle_alternating,
+ *              sinkhorn_solvers.py:94-287)
  * host_words: sched 1 or a threshold, 4 * items ints of PINNED host memory that the device can
  * write: the number of steps then depends on the clouds, and fs_small_solve waits for it (the one
  * entry point that waits for the device).  It must not be in use by another call.  Afterwards
@@ -429,6 +433,7 @@ typedef struct fs_small_problem {
   double blur, scaling;
   float cost_scale, eps, rho_x, rho_y, threshold;
   int dtype, normalize, self_terms, want_values, sched, entries, cut, extrapolate, check_every;
+  int alternating;
 } fs_small_problem;
 
 size_t fs_small_workspace_bytes(const fs_small_problem* problem);
