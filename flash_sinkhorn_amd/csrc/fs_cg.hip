@@ -28,7 +28,8 @@ __device__ void report(const float* state, float* host, int count) {
   if (host == nullptr) return;
   for (int i = 0; i < 7; ++i) __hip_atomic_store(&host[i], state[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   __threadfence_system();
-  __hip_atomic_store(reinterpret_cast<int*>(host) + 7, count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  __hip_atomic_store(reinterpret_cast<int*>(host) + 7, 2 * count + (state[4] != 0.f ? 1 : 0), __ATOMIC_RELAXED,
+                     __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 __global__ __launch_bounds__(kCgThreads) void cg_init_kernel(const float* __restrict__ b,

@@ -25,7 +25,8 @@ int wait_for_words(hipStream_t st, F&& arrived) {
 }
 
 // The launches behind fs_cg_init / fs_cg_update.  host: 8 pinned words that receive the state, the
-// last of them, an int, the number of iterations done (0: initialised); or null.
+// last of them, an int written behind the others, twice the number of iterations done (0: initialised)
+// plus one where there is nothing left to do; or null.
 int cg_init(const float* b, float* sol, float* res, float* dir, float* state, long long m, float rtol, float atol,
             float* host, hipStream_t st);
 int cg_update(const float* a_dir, float* sol, float* res, float* dir, float* state, long long m, float* host, int iter,

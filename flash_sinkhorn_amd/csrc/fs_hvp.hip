@@ -181,15 +181,18 @@ int fs_hvp(const fs_hvp_problem* p, void* workspace, size_t workspace_bytes, flo
   // ---- conjugate gradients: the host looks one iteration behind the one it enqueues, and what it
   // enqueued behind the last one does nothing ----
   int* count = reinterpret_cast<int*>(host_state) + 7;
-  auto seen = [&](int k) { return __atomic_load_n(count, __ATOMIC_ACQUIRE) >= k; };
+  bool done = false;  // (from the word that arrives last: the report is then whole)
+  auto seen = [&](int k) {
+    const int c = __atomic_load_n(count, __ATOMIC_ACQUIRE);
+    done = c >= 0 && (c & 1);
+    return done || c >= 2 * k;
+  };
   __atomic_store_n(count, -1, __ATOMIC_RELEASE);
   if ((rc = cg_init(a.a_dir, a.sol, a.res, a.vec, a.cg, a.m, p->rtol, p->atol, host_state, st)) != FS_OK) return rc;
-  bool done = false;
   for (int k = 0; k < p->max_iter && !done; ++k) {
     if ((rc = strips<1>(a, st)) != FS_OK) return rc;
     if ((rc = cg_update(a.a_dir, a.sol, a.res, a.vec, a.cg, a.m, host_state, k, st)) != FS_OK) return rc;
     if ((rc = wait_for_words(st, [&]() { return seen(k); })) != FS_OK) return rc;
-    done = host_state[4] != 0.f;
   }
   a.vec = a.sol;
   if ((rc = strips<2>(a, st)) != FS_OK) return rc;
@@ -201,7 +204,7 @@ int fs_hvp(const fs_hvp_problem* p, void* workspace, size_t workspace_bytes, flo
   hipLaunchKernelGGL((hvp_result_kernel<0>), dim3(blocks), dim3(256), 0, st, a);
   if (hipGetLastError() != hipSuccess) return FS_ERR_LAUNCH_FAILED;
   // (the last iteration's state, for the caller's report)
-  return done ? FS_OK : wait_for_words(st, [&]() { return seen(p->max_iter) || host_state[4] != 0.f; });
+  return done ? FS_OK : wait_for_words(st, [&]() { return seen(p->max_iter); });
 }
 
 }  // extern "C"

@@ -1,0 +1,219 @@
+"""Whole solves in one library call (small, medium and wide problems) and kept Hessian-vector products,
+at the edges of their tiles and dispatch rules, against the fp64 oracle.
+
+Tolerances: logits are formed from two fp16 planes a side (22 bits), so an inner product is off by
+about 2^-21 |x| |y|, a potential by 2^-21 of the largest cost per step at most, which averaged
+steps contract: 1e-5 of the largest potential.  A gradient multiplies the error of a logit (2^-21 of
+the largest cost over eps, a few hundred here at most) with the spread of the cloud: 1e-4."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from tests.golden.recipe import inputs
+
+pytestmark = pytest.mark.gpu
+POT, GRAD = 1e-5, 1e-4
+
+
+def dev(*arrs):
+    return [torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in arrs]
+
+
+def rel_err(got, want):
+    got = got.detach().cpu().numpy().astype(np.float64)
+    want = np.asarray(want, dtype=np.float64)
+    return float(np.abs(got - want).max() / max(np.abs(want).max(), 1e-30))
+
+
+def check_symmetric(x, y, a, b, tol=POT, **kw):
+    from flash_sinkhorn_amd.kernels import sinkhorn_flashstyle_symmetric as solve
+    got = solve(*dev(x, y, a, b), return_prelast=True, **kw)
+    want = oracle.sinkhorn_symmetric(x, y, a, b, return_prelast=True, **kw)
+    for g, w in zip(got, want):
+        assert rel_err(g, w) < tol
+
+
+# ---- one launch per step: 32-row blocks, 16-column steps, eight or sixteen wavefronts ----
+@pytest.mark.parametrize("n,m,d", [(1, 1, 1), (1, 40, 3), (31, 33, 16), (32, 32, 17), (33, 257, 32),
+                                   (255, 64, 33), (300, 1536, 64), (1537, 1505, 65),
+                                   (70, 2100, 128), (4100, 100, 5)])
+def test_small_steps(n, m, d):
+    x, y, a, b = inputs(n + d, n, m, d, scale=0.5)
+    check_symmetric(x, y, a, b, use_epsilon_scaling=False, eps=0.3, n_iters=4)
+    check_symmetric(x, y, a, b, use_epsilon_scaling=False, eps=0.1, n_iters=3, rho_x=0.7, rho_y=2.0)
+
+
+# schedules shorter than the steps that are enqueued before their length is known, and longer ones
+@pytest.mark.parametrize("n,m,d", [(200, 300, 16), (130, 90, 100), (7100, 7050, 6)])
+@pytest.mark.parametrize("cut", [1, 2, 3, 4, 5, 6, None])
+def test_schedules_of_every_length(n, m, d, cut):
+    if n > 1000 and cut not in (1, 5):
+        pytest.skip("the long ones cost the oracle seconds each")
+    x, y, a, b = inputs(3, n, m, d, scale=0.5)
+    for extrapolate in (True, False):
+        from flash_sinkhorn_amd.kernels import sinkhorn_flashstyle_symmetric as solve
+        kw = dict(blur=0.3, scaling=0.6, n_iters=cut, last_extrapolation=extrapolate)
+        f, g = solve(*dev(x, y, a, b), **kw)
+        wf, wg = oracle.sinkhorn_symmetric(x, y, a, b, **kw)
+        assert rel_err(f, wf) < POT and rel_err(g, wg) < POT
+
+
+# ---- both half-updates from one sweep (from 2e7 logits per step on): 256-row groups, chunks of
+# 64-row tiles; eps at which steps go without running maxima, and at which the first ones may not ----
+@pytest.mark.parametrize("n,m,d,eps", [(4481, 4703, 3, 0.5), (4608, 4352, 16, 0.01),
+                                       (21000, 970, 33, 0.2), (900, 22400, 64, 0.002)])
+def test_one_sweep_steps(n, m, d, eps):
+    x, y, a, b = inputs(n + d, n, m, d, scale=0.5)
+    a[::7] = 0.0 if eps == 0.01 else a[::7]  # (rows without weight)
+    check_symmetric(x, y, a, b, use_epsilon_scaling=False, eps=eps, n_iters=3)
+
+
+@pytest.mark.parametrize("n,m,d,eps", [(4700, 4650, 7, 0.05), (5100, 4209, 40, 0.01)])
+def test_one_sweep_self_problems(n, m, d, eps):
+    from flash_sinkhorn_amd.sinkhorn_solvers import sinkhorn_flashstyle_symmetric_self_pair as pair
+    x, y, a, b = inputs(n, n, m, d, scale=0.5)
+    X, Y, A, B = dev(x, y, a, b)
+    kw = dict(use_epsilon_scaling=False, eps=eps, n_iters=3)
+    px, py = pair(X, A, Y, B, return_prelast=True, **kw)
+    for got, (u, w) in ((px, (x, a)), (py, (y, b))):
+        want = oracle.sinkhorn_symmetric(u, u, w, w, return_prelast=True, **kw)
+        # (the potentials of a cloud against itself are far smaller than the costs, whose rounding is
+        # what is left in them: absolute, 2^-21 of the largest cost in each of two sums)
+        for p, q in ((got[0], want[0]), (got[2], want[2])):
+            assert np.abs(p.cpu().numpy() - q).max() < 2.0 ** -20 * 4.0 * (u * u).sum(axis=1).max()
+
+
+# ---- kept products: 256-column strips, tiles of 64, 128 and 256, both shapes of the sweep ----
+@pytest.mark.parametrize("n,m,d", [(1, 1, 129), (63, 257, 130), (256, 255, 144), (1000, 1000, 784),
+                                   (2100, 4099, 200), (513, 2049, 1536)])
+@pytest.mark.parametrize("dtype", ["float32", "float16"])
+def test_kept_products(n, m, d, dtype):
+    from flash_sinkhorn_amd.kernels import sinkhorn_flashstyle_symmetric as solve
+    x, y, a, b = inputs(n + d, n, m, d, scale=1.0 / np.sqrt(d))
+    x, y = x.astype(dtype), y.astype(dtype)
+    kw = dict(use_epsilon_scaling=False, eps=0.1, n_iters=4, rho_y=1.5)
+    f, g = solve(*dev(x, y, a, b), **kw)
+    wf, wg = oracle.sinkhorn_symmetric(x.astype(np.float64), y.astype(np.float64), a, b, **kw)
+    assert rel_err(f, wf) < POT and rel_err(g, wg) < POT
+
+
+# rows that do not start at multiples of 16 bytes take the narrow loads
+def test_kept_products_of_unaligned_rows():
+    from flash_sinkhorn_amd.kernels import sinkhorn_flashstyle_symmetric as solve
+    x, y, a, b = inputs(5, 300, 200, 160, scale=0.1)
+    kw = dict(use_epsilon_scaling=False, eps=0.1, n_iters=3)
+    X, Y, A, B = dev(x, y, a, b)
+    buf = torch.empty(X.numel() + 1, device="cuda")
+    U = buf[1:].view(X.shape)
+    U.copy_(X)
+    assert all(torch.equal(p, q) for p, q in zip(solve(U, Y, A, B, **kw), solve(X, Y, A, B, **kw)))
+
+
+# ---- early stopping on the device ----
+@pytest.mark.parametrize("n,m,d", [(300, 200, 20), (400, 300, 200), (4700, 4500, 8)])
+def test_early_stopping(n, m, d):
+    from flash_sinkhorn_amd.kernels import sinkhorn_flashstyle_symmetric as solve
+    x, y, a, b = inputs(9, n, m, d, scale=1.0 / np.sqrt(d))
+    kw = dict(use_epsilon_scaling=False, eps=0.5, n_iters=60, threshold=1e-3, check_every=4,
+              return_n_iters=True)
+    *got, used = solve(*dev(x, y, a, b), **kw)
+    *want, wused = oracle.sinkhorn_symmetric(x, y, a, b, **kw)
+    assert used == wused < 62
+    assert all(rel_err(p, q) < POT for p, q in zip(got, want))
+
+
+@pytest.mark.parametrize("n,m,d", [(1, 5, 2), (333, 65, 16), (200, 1600, 40), (2100, 2000, 128)])
+@pytest.mark.parametrize("threshold", [None, 1e-3])
+def test_alternating(n, m, d, threshold):
+    from flash_sinkhorn_amd.kernels import sinkhorn_flashstyle_alternating as solve
+    x, y, a, b = inputs(n + d, n, m, d, scale=1.0 / np.sqrt(d))
+    kw = dict(eps=0.3, n_iters=7 if threshold is None else 50, rho_x=0.8, threshold=threshold,
+              check_every=3, return_n_iters=True)
+    *got, used = solve(*dev(x, y, a, b * 1.2), **kw)
+    *want, wused = oracle.sinkhorn_alternating(x, y, a, b * 1.2, **kw)
+    assert used == wused
+    assert all(rel_err(p, q) < POT for p, q in zip(got, want))
+
+
+# ---- the loss, its gradients, and what a training program does with them ----
+def expected(x, y, a, b, debias, eps, n_iters):
+    def one(u, v, wu, wv):
+        f, g, fp, gp = oracle.sinkhorn_symmetric(u, v, wu, wv, use_epsilon_scaling=False, eps=eps,
+                                                 n_iters=n_iters, return_prelast=True)
+        gu, gv = oracle.grad_barycentric(u, v, wu, wv, fp, gp, eps)
+        return oracle.sinkhorn_cost(wu, wv, f, g, eps), gu, gv
+    c, gx, gy = one(x, y, a, b)
+    if debias:
+        cx, g1, g2 = one(x, x, a, a)
+        cy, h1, h2 = one(y, y, b, b)
+        c, gx, gy = c - 0.5 * (cx + cy), gx - 0.5 * (g1 + g2), gy - 0.5 * (h1 + h2)
+    return c, gx, gy
+
+
+@pytest.mark.parametrize("n,m,d", [(1, 3, 1), (33, 31, 16), (100, 129, 33), (257, 64, 65), (90, 1700, 128),
+                                   (4600, 4400, 10)])
+@pytest.mark.parametrize("debias", [False, True])
+def test_loss_and_gradients(n, m, d, debias):
+    from flash_sinkhorn_amd import SamplesLoss
+    x, y, a, b = inputs(n + d, n, m, d, scale=0.5, y_shift=0.5)
+    X, Y, A, B = dev(x, y, a, b)
+    X.requires_grad_(), Y.requires_grad_()
+    steps = 4 if n < 1000 else 1
+    fn = SamplesLoss("sinkhorn", use_epsilon_scaling=False, eps=0.2, n_iters=steps, debias=debias,
+                     half_cost=False)
+    loss = fn(A, X, B, Y)
+    assert loss.shape == ()
+    gx, gy = torch.autograd.grad(loss, [X, Y])
+    c, wx, wy = expected(x, y, a, b, debias, 0.2, steps)
+    # (a debiased loss or gradient is a difference: its error is that of the parts)
+    _, px, py = expected(x, y, a, b, False, 0.2, steps)
+    assert abs(loss.item() - c) < 1e-4 * (abs(c) + (0.5 * d if debias else 0.0))
+    for g, w, p in ((gx, wx, px), (gy, wy, py)):
+        assert np.abs(g.cpu().numpy() - w).max() < GRAD * np.abs(p).max()
+
+
+def test_batch_equals_its_items():
+    from flash_sinkhorn_amd import SamplesLoss
+    rng = np.random.default_rng(4)
+    x, y = (rng.standard_normal((5, k, 6)).astype(np.float32) * s for k, s in ((150, 0.5), (97, 0.7)))
+    X, Y = dev(x, y)
+    X.requires_grad_()
+    fn = SamplesLoss("sinkhorn", debias=True, blur=0.1)  # items have schedules of their own
+    loss = fn(X, Y)
+    gx, = torch.autograd.grad(loss.sum(), X)
+    for i in range(5):
+        Xi = X[i].detach().clone().requires_grad_()
+        li = fn(Xi, Y[i])
+        gi, = torch.autograd.grad(li, Xi)
+        assert abs(loss[i].item() - li.item()) < 1e-6 * 6
+        assert rel_err(gx[i], gi.cpu().numpy()) < GRAD
+
+
+# ---- Hessian-vector products: whole rows in registers (2,048, 4,096, 8,192 columns) ----
+@pytest.mark.parametrize("n,m,d", [(1, 1, 1), (37, 2048, 64), (300, 2049, 5), (65, 4097, 130), (257, 200, 129),
+                                   (40, 8192, 20)])
+@pytest.mark.parametrize("rho", [None, 1.5])
+def test_kept_hvp(n, m, d, rho):
+    from flash_sinkhorn_amd.hvp import hvp_x_sqeuclid_from_potentials as hvp
+    x, y, a, b = inputs(n + d, n, m, d, scale=1.0 / np.sqrt(d))
+    eps = 0.25
+    f, g = oracle.sinkhorn_symmetric(x, y, a, b, use_epsilon_scaling=False, eps=eps, n_iters=20, rho_x=rho)
+    f, g = oracle.geomloss_to_ott_potentials(f, g, a, b, eps)
+    A = np.random.default_rng(1).standard_normal((n, d)).astype(np.float32)
+    f, g = f.astype(np.float32), g.astype(np.float32)
+    for iters in (0, 1, 200):
+        kw = dict(eps=eps, rho_x=rho, max_cg_iter=iters, cg_rtol=1e-5, cg_atol=1e-12,
+                  preconditioner="none")
+        got, info = hvp(*dev(x, y, f, g, A), **kw)
+        want, winfo = oracle.hvp_x_from_potentials(x, y, f, g, A, **kw)
+        # conjugate gradients to 1e-5 of a right-hand side whose Schur complement is no smaller than
+        # the gap of the plan (above 1e-1 at this eps): 1e-4 of the result
+        assert rel_err(got, want) < 2e-4
+        assert info.cg_iters <= iters and np.isfinite(info.cg_residual)
+        if iters == 200:
+            # (one point: the right-hand side is zero, and nothing is iterated)
+            assert info.cg_converged or info.cg_initial_residual == 0.0
+            assert info.cg_residual <= max(1e-5 * info.cg_initial_residual, 1e-12)
+        elif not info.cg_converged and info.cg_initial_residual > 0.0:
+            assert info.cg_iters == iters
