@@ -161,7 +161,7 @@ def solve(x, y, a, b, *, items: int, blur: float = 0.0, scaling: float = 0.0, ep
             and (d <= WIDE_D or items * n * m <= 1 << 22)):  # (a graph keeps its products)
         # a fixed sequence of kernels on fixed shapes: replayed (1.9 instead of 3 us per launch)
         key = ("self pair" if self_terms else "alternating" if alternating else "symmetric",
-               int(self_terms), x.device.index, x.dtype, items, n, m, d,
+               int(self_terms), x.device.index, x.dtype, x.shape, y.shape,
                eps, entries, cost_scale, _rho(rho_x), _rho(rho_y), a is None, b is None, normalize,
                want_values, extrapolate, want_loss)
         ws, out = _graphs.run(key, enqueue, [x, y, a, b])

@@ -190,6 +190,16 @@ def test_batch_equals_its_items():
         assert rel_err(gx[i], gi.cpu().numpy()) < GRAD
 
 
+def test_a_batch_of_one_and_a_single_problem_keep_graphs_of_their_own():
+    from flash_sinkhorn_amd import SamplesLoss
+    x, y, _, _ = inputs(8, 61, 50, 4)
+    X, Y = dev(x, y)
+    fn = SamplesLoss("sinkhorn", use_epsilon_scaling=False, eps=0.1, n_iters=10)
+    for _ in range(3):  # (eager, captured, replayed)
+        one, batch = fn(X, Y), fn(X[None], Y[None])
+        assert one.shape == () and batch.shape == (1,) and one.item() == batch.item()
+
+
 # ---- Hessian-vector products: whole rows in registers (2,048, 4,096, 8,192 columns) ----
 @pytest.mark.parametrize("n,m,d", [(1, 1, 1), (37, 2048, 64), (300, 2049, 5), (65, 4097, 130), (257, 200, 129),
                                    (40, 8192, 20)])
