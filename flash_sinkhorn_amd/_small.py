@@ -59,13 +59,29 @@ def _host_words(items: int) -> torch.Tensor:
 
 
 class Solved:
-    """A solve that has been enqueued: its workspace (planes, log weights, potentials in the form the
-    gradient kernel reads), the loss per item, and the standard potentials."""
-    __slots__ = ("problem", "table", "x", "y", "a", "b", "ws", "loss", "pots", "entries")
+    """A solve that has been enqueued: what it read, its workspace (planes, log weights, potentials in
+    the form the gradient kernel reads), the loss per item, and the standard potentials."""
+    __slots__ = ("form", "x", "y", "a", "b", "ws", "loss", "pots", "entries")
+
+    def problem(self) -> Problem:
+        p = Problem.from_buffer_copy(self.form)
+        p.x, p.y, p.a, p.b = self.x.data_ptr(), self.y.data_ptr(), _lib.ptr(self.a), _lib.ptr(self.b)
+        return p
+
+    def tensors(self):
+        """What a backward pass needs, in the order ``restored`` takes it."""
+        return self.x, self.y, self.a, self.b, self.ws, self.pots
+
+    @classmethod
+    def restored(cls, form: Problem, tensors) -> "Solved":
+        s = cls()
+        s.form, s.loss, s.entries = form, None, None
+        s.x, s.y, s.a, s.b, s.ws, s.pots = tensors
+        return s
 
     def potentials(self, which: str):
         """("f" | "g" | "xx" | "yy") -> (of the cost, of the gradient), each [items, rows]."""
-        p = self.problem
+        p = self.form
         n, m, k = p.n * p.items, p.m * p.items, ("f", "g", "xx", "yy").index(which)
         at = [0, 2 * n, 2 * (n + m), 2 * (2 * n + m)][k]
         size = n if k % 2 == 0 else m
@@ -128,26 +144,29 @@ def solve(x, y, a, b, *, items: int, blur: float = 0.0, scaling: float = 0.0, ep
             raise LongSchedule
         table = (ctypes.c_float * entries)(*eps_list)
 
-    def problem(x, y, a, b):
-        return Problem(
-            x.data_ptr(), y.data_ptr(), _lib.ptr(a), _lib.ptr(b),
-            None if table is None else ctypes.addressof(table), n, m, d, items, blur, scaling,
-            cost_scale, eps, _rho(rho_x), _rho(rho_y), threshold or 0.0, _DTYPES[x.dtype],
-            int(normalize), int(self_terms), int(want_values), sched, entries, cut,
-            int(extrapolate), int(check_every), int(alternating))
+    form = Problem(
+        None, None, None, None, None, n, m, d, items, blur, scaling, cost_scale, eps, _rho(rho_x),
+        _rho(rho_y), threshold or 0.0, _DTYPES[x.dtype], int(normalize), int(self_terms),
+        int(want_values), sched, entries, cut, int(extrapolate), int(check_every),
+        int(alternating))
 
     rows = (n + m) * items * (4 if self_terms else 2)
 
     def enqueue(x, y, a, b):
-        p = problem(x, y, a, b)
+        p = Problem.from_buffer_copy(form)
+        p.x, p.y, p.a, p.b = x.data_ptr(), y.data_ptr(), _lib.ptr(a), _lib.ptr(b)
+        if table is not None:
+            p.eps_list = ctypes.addressof(table)
         L = _lib.lib()
         ws = torch.empty(L.fs_small_workspace_bytes(ctypes.byref(p)), dtype=torch.uint8,
                          device=x.device)
-        out = torch.empty(rows + items, dtype=torch.float32, device=x.device)
+        pots = torch.empty(rows, dtype=torch.float32, device=x.device)
+        # (a tensor of its own: a caller may change the loss in place)
+        loss = (torch.empty(x.shape[:-2], dtype=torch.float32, device=x.device) if want_loss
+                else None)
         words = _host_words(items).data_ptr() if sched == 1 or threshold else None
-        rc = L.fs_small_solve(ctypes.byref(p), ws.data_ptr(), ws.numel(), words,
-                              out.data_ptr() + 4 * rows if want_loss else None, out.data_ptr(),
-                              _lib.stream_of(x))
+        rc = L.fs_small_solve(ctypes.byref(p), ws.data_ptr(), ws.numel(), words, _lib.ptr(loss),
+                              pots.data_ptr(), _lib.stream_of(x))
         if rc > 0:
             if rc == 1:
                 raise ValueError("diameter must be > 0.")
@@ -155,7 +174,7 @@ def solve(x, y, a, b, *, items: int, blur: float = 0.0, scaling: float = 0.0, ep
                 raise ValueError("the diameter of the clouds is not a number.")
             raise LongSchedule
         _lib.check(rc, "fs_small_solve")
-        return ws, out
+        return (ws, pots, loss) if want_loss else (ws, pots)
 
     if (sched == 0 and not threshold and _graphs.eligible(n, m, entries, x.device)
             and (d <= WIDE_D or items * n * m <= 1 << 22)):  # (a graph keeps its products)
@@ -164,12 +183,12 @@ def solve(x, y, a, b, *, items: int, blur: float = 0.0, scaling: float = 0.0, ep
                int(self_terms), x.device.index, x.dtype, x.shape, y.shape,
                eps, entries, cost_scale, _rho(rho_x), _rho(rho_y), a is None, b is None, normalize,
                want_values, extrapolate, want_loss)
-        ws, out = _graphs.run(key, enqueue, [x, y, a, b])
+        out = _graphs.run(key, enqueue, [x, y, a, b])
     else:
-        ws, out = enqueue(x, y, a, b)
+        out = enqueue(x, y, a, b)
     s = Solved()
-    s.problem, s.x, s.y, s.a, s.b, s.ws = problem(x, y, a, b), x, y, a, b, ws
-    s.pots, s.loss, s.table = out[:rows], out[rows:], table
+    s.form, s.x, s.y, s.a, s.b = form, x, y, a, b
+    s.ws, s.pots, s.loss = out if want_loss else out + (None,)
     s.entries = entries
     if threshold:  # averaged steps of the first problem
         word = int(_host_words(items)[0])
@@ -315,7 +334,7 @@ def potentials(loss, x, y, a, b, normalize):
 
 
 def _gradients(s: Solved, grad_out, want_x: bool, want_y: bool):
-    p, L = s.problem, _lib.lib()
+    p, L = s.problem(), _lib.lib()
     gx = torch.empty(s.x.shape, dtype=torch.float32, device=s.x.device) if want_x else None
     gy = torch.empty(s.y.shape, dtype=torch.float32, device=s.x.device) if want_y else None
     gs = grad_out.float().contiguous()
@@ -330,28 +349,28 @@ class _SmallGrad(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, y, grad_out, solved, config, want_x, want_y):
         gx, gy = _gradients(solved, grad_out, want_x, want_y)
-        ctx.save_for_backward(x, y, grad_out)
-        ctx.solved, ctx.config = solved, config
+        ctx.save_for_backward(x, y, grad_out, *solved.tensors())
+        ctx.form, ctx.config = solved.form, config
         return gx, gy
 
     @staticmethod
     def backward(ctx, grad_grad_x, grad_grad_y):
-        x, y, grad_out = ctx.saved_tensors
+        x, y, grad_out = ctx.saved_tensors[:3]
         from flash_sinkhorn_amd.hvp import (geomloss_to_ott_potentials,
                                             hvp_x_sqeuclid_from_potentials)
-        cfg, s = ctx.config, ctx.solved
-        if grad_grad_y is not None or s.problem.self_terms:
+        cfg, s = ctx.config, Solved.restored(ctx.form, ctx.saved_tensors[3:])
+        if grad_grad_y is not None or s.form.self_terms:
             raise NotImplementedError("Double backward w.r.t y is not implemented yet.")
         if grad_grad_x is None:
             return (None,) * 7
-        items, f, g = s.problem.items, s.potentials("f")[1], s.potentials("g")[1]
+        items, f, g = s.form.items, s.potentials("f")[1], s.potentials("g")[1]
         outs = []
         with torch.no_grad():
             gs = grad_out.reshape(-1)
             for i in range(items):
                 xi, yi, v = (t if t.ndim == 2 else t[i] for t in (x, y, grad_grad_x))
-                a, b = (_item_weights(w, rows, i, s.problem.normalize, x.device)
-                        for w, rows in ((s.a, s.problem.n), (s.b, s.problem.m)))
+                a, b = (_item_weights(w, rows, i, s.form.normalize, x.device)
+                        for w, rows in ((s.a, s.form.n), (s.b, s.form.m)))
                 eps = _last_eps(cfg, xi, yi)
                 f_ott, g_ott = geomloss_to_ott_potentials(f[i], g[i], a, b, eps=eps)
                 hvp, _ = hvp_x_sqeuclid_from_potentials(
@@ -390,14 +409,14 @@ class _SmallLoss(torch.autograd.Function):
         need = ctx.needs_input_grad
         s = _solve_for(loss, x, y, a, b, normalize, self_terms=int(loss.debias),
                        want_values=need[0] or need[1], want_loss=True)
-        ctx.save_for_backward(x, y)
-        ctx.solved, ctx.config = s, loss._make_config()
-        return s.loss if x.ndim == 3 else s.loss.view(())
+        ctx.save_for_backward(x, y, *s.tensors())
+        ctx.form, ctx.config = s.form, loss._make_config()
+        return s.loss
 
     @staticmethod
     def backward(ctx, grad_out):
-        x, y = ctx.saved_tensors
-        s, cfg, need = ctx.solved, ctx.config, ctx.needs_input_grad
+        x, y, *solved = ctx.saved_tensors
+        s, cfg, need = Solved.restored(ctx.form, solved), ctx.config, ctx.needs_input_grad
         gx = gy = ga = gb = None
         if need[0] or need[1]:
             if torch.is_grad_enabled():  # create_graph
@@ -406,10 +425,10 @@ class _SmallLoss(torch.autograd.Function):
                 gx, gy = _gradients(s, grad_out, need[0], need[1])
         scale = grad_out if x.ndim == 2 else grad_out[:, None]
         if need[2]:
-            f = s.potentials("f")[0] - s.potentials("xx")[0] if s.problem.self_terms else s.potentials("f")[0]
+            f = s.potentials("f")[0] - s.potentials("xx")[0] if s.form.self_terms else s.potentials("f")[0]
             ga = scale * (f if x.ndim == 3 else f[0])
         if need[3]:
-            g = s.potentials("g")[0] - s.potentials("yy")[0] if s.problem.self_terms else s.potentials("g")[0]
+            g = s.potentials("g")[0] - s.potentials("yy")[0] if s.form.self_terms else s.potentials("g")[0]
             gb = scale * (g if x.ndim == 3 else g[0])
         return gx, gy, ga, gb, None, None
 

@@ -200,6 +200,43 @@ def test_a_batch_of_one_and_a_single_problem_keep_graphs_of_their_own():
         assert one.shape == () and batch.shape == (1,) and one.item() == batch.item()
 
 
+@pytest.mark.parametrize("batched", [False, True])
+@pytest.mark.parametrize("fixed", [False, True])
+def test_the_loss_may_be_changed_in_place(batched, fixed):
+    from flash_sinkhorn_amd import SamplesLoss
+    x, y, _, _ = inputs(8, 64, 50, 4)
+    X, Y = dev(x, y) if not batched else dev(x[None], y[None])
+    X.requires_grad_()
+    fn = SamplesLoss("sinkhorn", **(dict(use_epsilon_scaling=False, eps=0.1, n_iters=10) if fixed else {}))
+    for _ in range(3):  # (eager, captured, replayed)
+        want, = torch.autograd.grad(fn(X, Y).sum(), X)
+        loss = fn(X, Y)
+        loss += 1.0
+        loss *= 2.0
+        got, = torch.autograd.grad(loss.sum(), X)
+        assert torch.equal(got, 2.0 * want)
+
+
+def test_saved_tensors_pass_through_hooks_and_version_checks():
+    from flash_sinkhorn_amd import SamplesLoss
+    x, y, a, b = inputs(8, 90, 50, 4)
+    X, Y, A, B = dev(x, y, a, b)
+    X.requires_grad_()
+    fn = SamplesLoss("sinkhorn", normalize=False)
+    want, = torch.autograd.grad(fn(A, X, B, Y), X)
+    with torch.autograd.graph.save_on_cpu():
+        loss = fn(A, X, B, Y)
+    got, = torch.autograd.grad(loss, X, create_graph=True)
+    assert torch.equal(got, want)
+    assert torch.isfinite(torch.autograd.grad((got * Y[:1]).sum(), X)[0]).all()
+    for t in (A, Y):  # changed between the passes: refused
+        loss = fn(A, X, B, Y)
+        with torch.no_grad():
+            t.mul_(1.0)
+        with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+            loss.backward()
+
+
 # ---- Hessian-vector products: whole rows in registers (2,048, 4,096, 8,192 columns) ----
 @pytest.mark.parametrize("n,m,d", [(1, 1, 1), (37, 2048, 64), (300, 2049, 5), (65, 4097, 130), (257, 200, 129),
                                    (40, 8192, 20)])
