@@ -541,8 +541,8 @@ int run_lse_gemm(int mode, Side* sides, int nsides, int64_t d, const LseConfig& 
     hipLaunchKernelGGL((finish_argmax_kernel<0>), dim3(ceil_div(items0, 256)), dim3(256), 0, st, a);
     return hipGetLastError() == hipSuccess ? FS_OK : FS_ERR_LAUNCH_FAILED;
   }
-  hipLaunchKernelGGL((finish_kernel<false>), dim3(ceil_div(items0 + items1, 256)), dim3(256), 0, st,
-                     a, cfg.dp, items0, items1);
+  hipLaunchKernelGGL((finish_kernel<false>), dim3(ceil_div(items0 + items1, kFinishRows)), dim3(finish_threads(false)),
+                     0, st, a, cfg.dp, items0, items1);
   return hipGetLastError() == hipSuccess ? FS_OK : FS_ERR_LAUNCH_FAILED;
 }
 
@@ -892,7 +892,7 @@ int run_plan_tile(int mode, Side* sides, int nsides, int64_t d, const LseConfig&
     if (has_o)
       hipLaunchKernelGGL((finish_kernel<true>), dim3(grid), dim3(256), 0, st, f, dpk, items[0], items[1]);
     else
-      hipLaunchKernelGGL((finish_kernel<false>), dim3(grid), dim3(256), 0, st, f, dpk, items[0], items[1]);
+      hipLaunchKernelGGL((finish_kernel<false>), dim3(grid), dim3(finish_threads(false)), 0, st, f, dpk, items[0], items[1]);
     if (hipGetLastError() != hipSuccess) return FS_ERR_LAUNCH_FAILED;
   }
   return FS_OK;
@@ -1239,7 +1239,7 @@ int run_stream(int mode, bool sepv, Side* sides, int nsides, int64_t d, void* ws
     if (has_o)
       hipLaunchKernelGGL((finish_kernel<true>), dim3(grid), dim3(256), 0, st, f, dp, items[0], items[1]);
     else
-      hipLaunchKernelGGL((finish_kernel<false>), dim3(grid), dim3(256), 0, st, f, dp, items[0], items[1]);
+      hipLaunchKernelGGL((finish_kernel<false>), dim3(grid), dim3(finish_threads(false)), 0, st, f, dp, items[0], items[1]);
     if (hipGetLastError() != hipSuccess) return FS_ERR_LAUNCH_FAILED;
   }
   return FS_OK;

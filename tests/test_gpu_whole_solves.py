@@ -264,3 +264,19 @@ def test_kept_hvp(n, m, d, rho):
             assert info.cg_residual <= max(1e-5 * info.cg_initial_residual, 1e-12)
         elif not info.cg_converged and info.cg_initial_residual > 0.0:
             assert info.cg_iters == iters
+
+
+# ---- the merge of the key splits: four wavefronts share them, two, four or eight at a time ----
+@pytest.mark.parametrize("n,m", [(1, 40000), (63, 9000), (257, 20000), (1000, 3000), (5000, 5100), (20000, 700)])
+def test_merge_of_key_splits(n, m):
+    from flash_sinkhorn_amd.kernels import apply_plan_vec_flashstyle as apply
+    rng = np.random.default_rng(n)
+    x, y, a, b = inputs(n, n, m, 12, scale=0.3)
+    f, g = (0.1 * rng.standard_normal(k).astype(np.float32) for k in (n, m))
+    la, lb = np.log(a), np.log(b)
+    for axis, k in ((1, m), (0, n)):
+        v = rng.random(k).astype(np.float32)
+        got = apply(*dev(x, y, f, g, la, lb, v), eps=0.2, axis=axis)
+        want = oracle.apply_plan_vec(x, y, f, g, la, lb, v, 0.2, axis)
+        # (positive terms: the error of a logit, 2^-21 of the largest cost over eps, is the whole error)
+        assert rel_err(got, want) < GRAD
