@@ -362,14 +362,13 @@ int launch_plane_set(const PlaneSet& ps, const LseConfig& c, int64_t d, void* ws
     const bool two = ps.n > 1;
     rc = launch_absmax(ps.src[0], (long long)ps.rows[0] * d, two ? ps.src[1] : ps.src[0],
                        two ? (long long)ps.rows[1] * d : 0, partial, st);
-    for (int i = 0; i < ps.n && rc == FS_OK; ++i)
-      rc = launch_split_planes_f16(ps.src[i], reinterpret_cast<unsigned*>(base + ps.off[i]),
-                                   ps.rows[i], (int)d, c.dp, partial + 256 * i, scales + i,
-                                   two ? nullptr : scales + 1, c.gemm ? 1 : 0,
-                                   i == 0 ? select_state(ps, ws) : nullptr,
-                                   best_keys_of(ps, c, ws, ps.src[i], ps.rows[i]),
-                                   keep ? tiled_of(ps, c, ws, ps.src[i], ps.rows[i]) : nullptr, st,
-                                   start_plain ? 1 : 0);
+    SplitArgs s{{}, ps.n, (int)d, c.dp, c.gemm ? 1 : 0, start_plain ? 1 : 0};
+    for (int i = 0; i < ps.n; ++i)
+      s.m[i] = {ps.src[i], reinterpret_cast<unsigned*>(base + ps.off[i]), ps.rows[i], partial + 256 * i,
+                scales + i, two ? nullptr : scales + 1, i == 0 ? select_state(ps, ws) : nullptr,
+                best_keys_of(ps, c, ws, ps.src[i], ps.rows[i]),
+                keep ? tiled_of(ps, c, ws, ps.src[i], ps.rows[i]) : nullptr};
+    if (rc == FS_OK) rc = launch_split_planes_f16(s, st);
   }
   return rc;
 }
@@ -713,8 +712,9 @@ int run_plan_gemm(int mode, Side* sides, int nsides, int64_t d, const LseConfig&
     float* partial = reinterpret_cast<float*>(base + q2_off + plane_bytes(sd.nq, cfg));
     rc = launch_absmax(sd.q2, (long long)sd.nq * d, sd.q2, 0, partial, st);
     if (rc == FS_OK)
-      rc = launch_split_planes_f16(sd.q2, reinterpret_cast<unsigned*>(base + q2_off), sd.nq, (int)d,
-                                   cfg.dp, partial, partial + 2 * 256, nullptr, 1, nullptr, nullptr, nullptr, st);
+      rc = launch_split_planes_f16({{{sd.q2, reinterpret_cast<unsigned*>(base + q2_off), sd.nq, partial,
+                                      partial + 2 * 256, nullptr, nullptr, nullptr, nullptr}},
+                                    1, (int)d, cfg.dp, 1, 0}, st);
   }
   if (rc == FS_OK) rc = launch_plan_gemm(a, mat5, cb, total, st);
   if (rc != FS_OK) return rc;
@@ -859,8 +859,9 @@ int run_plan_tile(int mode, Side* sides, int nsides, int64_t d, const LseConfig&
     rc = launch_mat5_bounds(sd.q2, sd.nq, (int)d, sd.kb1, sd.nk, bounds + 64, bounds, st);
     if (rc == FS_OK) rc = launch_absmax(sd.q2, (long long)sd.nq * d, sd.q2, 0, partial, st);
     if (rc == FS_OK)
-      rc = launch_split_planes_f16(sd.q2, reinterpret_cast<unsigned*>(base + q2_off), sd.nq, (int)d,
-                                   cfg.dp, partial, partial + 2 * 256, nullptr, 0, nullptr, nullptr, nullptr, st);
+      rc = launch_split_planes_f16({{{sd.q2, reinterpret_cast<unsigned*>(base + q2_off), sd.nq, partial,
+                                      partial + 2 * 256, nullptr, nullptr, nullptr, nullptr}},
+                                    1, (int)d, cfg.dp, 0, 0}, st);
   }
   for (int s = 0; s < nsides && rc == FS_OK && has_o; ++s) {
     const Side& sd = sides[s];

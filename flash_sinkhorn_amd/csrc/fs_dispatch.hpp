@@ -10,10 +10,10 @@ int launch_sliced(int mode, const LaunchArgs& a, int nw, int nsl, int blocks, hi
 
 // Software-pipelined LSE kernel for d <= 128 with 16-byte aligned rows (dp in {16,32,64,128});
 // prec: 0 fp32 operands, 3 two scaled fp16 planes (3 products).
-// fp16 planes: absmax over the (at most two) operand matrices -> partial[2][256]; then one
-// split per matrix, which also writes the matrix's power-of-two scale to *scale_out and clears
-// the variant-choice state at clear_state (kSelWords words; may be null) and resets best_keys
-// (one int per row; may be null) to -1.
+// fp16 planes: absmax over the (at most two) operand matrices -> partial[2][256]; then the split of
+// all of them (one launch: 5 us less per operation than one each), which also writes a matrix's
+// power-of-two scale to *scale_out and clears the variant-choice state at clear_state (kSelWords
+// words; may be null) and resets best_keys (one int per row; may be null) to -1.
 // n 32-bit words at p (16-byte aligned) set to zero by a kernel (graph-capture safe).
 int launch_fill_zero(unsigned* p, long long n, hipStream_t st);
 int launch_absmax(const float* a, long long na, const float* b, long long nb, float* partial,
@@ -21,10 +21,22 @@ int launch_absmax(const float* a, long long na, const float* b, long long nb, fl
 // The seed part of coarse_bias_kernel alone: per side with Side::seed set, where each query row's
 // running maximum starts (its logit at the key Side::best_key names).
 int launch_row_seeds(const LaunchArgs& a, int dp, int nsides, hipStream_t st);
-int launch_split_planes_f16(const float* src, unsigned* dst, int rows, int d, int dp,
-                            const float* partial_max, float* scale_out, float* scale_out2,
-                            int chunked, unsigned* clear_state, int* best_keys, unsigned* tiled,
-                            hipStream_t st, int start_plain = 0);
+struct SplitMatrix {
+  const float* src;
+  unsigned* dst;
+  int rows;
+  const float* partial_max;
+  float* scale_out;
+  float* scale_out2;       // or null
+  unsigned* clear_state;   // or null
+  int* best_keys;          // or null
+  unsigned* tiled;         // or null
+};
+struct SplitArgs {
+  SplitMatrix m[2];
+  int n, d, dp, chunked, start_plain;
+};
+int launch_split_planes_f16(const SplitArgs& a, hipStream_t st);
 // GEMM-style LSE kernel for 128 < d <= 1536 on chunked fp16 planes; Side::splits counts
 // partial rows (twice the workgroup-level key splits).
 int launch_lse_gemm(const LaunchArgs& a, int mode, int blocks, hipStream_t st);  // kLse, kVec, kArgmax

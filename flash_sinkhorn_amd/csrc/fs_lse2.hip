@@ -47,14 +47,11 @@ int launch_fill_zero(unsigned* p, long long n, hipStream_t st) {
   return hipGetLastError() == hipSuccess ? FS_OK : FS_ERR_LAUNCH_FAILED;
 }
 
-int launch_split_planes_f16(const float* src, unsigned* dst, int rows, int d, int dp,
-                            const float* partial_max, float* scale_out, float* scale_out2,
-                            int chunked, unsigned* clear_state, int* best_keys, unsigned* tiled,
-                            hipStream_t st, int start_plain) {
-  const long long items = (long long)(rows + kPlanePadRows) * (dp / 4);
+int launch_split_planes_f16(const SplitArgs& a, hipStream_t st) {
+  const int rows = a.n > 1 && a.m[1].rows > a.m[0].rows ? a.m[1].rows : a.m[0].rows;
+  const long long items = (long long)(rows + kPlanePadRows) * (a.dp / 4);
   const int grid = (int)((items + 255) / 256);
-  hipLaunchKernelGGL(split_planes_f16_kernel, dim3(grid), dim3(256), 0, st, src, dst, rows, d, dp,
-                     partial_max, scale_out, scale_out2, chunked, clear_state, best_keys, tiled, start_plain);
+  hipLaunchKernelGGL(split_planes_f16_kernel, dim3(grid, a.n), dim3(256), 0, st, a);
   return hipGetLastError() == hipSuccess ? FS_OK : FS_ERR_LAUNCH_FAILED;
 }
 

@@ -37,6 +37,7 @@
 #include <type_traits>
 
 #include "fs_common.hpp"
+#include "fs_dispatch.hpp"
 #include "fs_stream.hpp"
 
 namespace fs {
@@ -106,11 +107,18 @@ __global__ __launch_bounds__(256) void fill_zero_kernel(unsigned* __restrict__ p
   }
 }
 
-__global__ __launch_bounds__(256) void split_planes_f16_kernel(
-    const float* __restrict__ src, unsigned* __restrict__ dst, int rows, int d, int dp,
-    const float* __restrict__ partial_max, float* __restrict__ scale_out,
-    float* __restrict__ scale_out2, int chunked, unsigned* __restrict__ clear_state,
-    int* __restrict__ best_keys, unsigned* __restrict__ tiled, int start_plain) {
+// Grid (256 items, matrices): the matrices of an operation go in one launch.
+__global__ __launch_bounds__(256) void split_planes_f16_kernel(const SplitArgs args) {
+  const SplitMatrix& mat = args.m[blockIdx.y];
+  const float* __restrict__ src = mat.src;
+  unsigned* __restrict__ dst = mat.dst;
+  const float* __restrict__ partial_max = mat.partial_max;
+  float* __restrict__ scale_out = mat.scale_out;
+  float* __restrict__ scale_out2 = mat.scale_out2;
+  unsigned* __restrict__ clear_state = mat.clear_state;
+  int* __restrict__ best_keys = mat.best_keys;
+  unsigned* __restrict__ tiled = mat.tiled;
+  const int rows = mat.rows, d = args.d, dp = args.dp, chunked = args.chunked, start_plain = args.start_plain;
   __shared__ float red[4];
   float m = partial_max[threadIdx.x];  // kAbsmaxBlocks == blockDim.x
 #pragma unroll
@@ -195,7 +203,7 @@ struct SoftmaxStage {
   float v[2][4];  // VEC: two groups of four v values in flight
 };
 
-// VEC: the plan-vector product (kVec) on the same pipeline: next to the row sums the kernel
+// VEC: the plan-vector product (kVec) on the same pipeline: in place of the row sums the kernel
 // keeps o_i = sum_j p_ij v_j, with v staged through LDS beside the key bias.  Two-plane modes
 // at d <= 64 only (the bias-as-accumulator-start variants).
 template <int DP, int RB, int PREC, bool VEC = false>
@@ -421,13 +429,16 @@ __global__ __launch_bounds__(256, 2) void lse2_kernel(const LaunchArgs args) {
     for (int r = 0; r < 16; r += 2) {
       const float e0 = fast_exp2(__builtin_fmaf(acc[r], lscale, c_new));
       const float e1 = fast_exp2(__builtin_fmaf(acc[r + 1], lscale, c_new));
-      ps0 += e0;
-      ps1 += e1;
-      if constexpr (VEC) po = __builtin_fmaf(e0, v16[r], __builtin_fmaf(e1, v16[r + 1], po));
+      if constexpr (VEC) {
+        po = __builtin_fmaf(e0, v16[r], __builtin_fmaf(e1, v16[r + 1], po));
+      } else {
+        ps0 += e0;
+        ps1 += e1;
+      }
     }
     const float resc = fast_exp2(c_new - run_c[rb]);
-    run_s[rb] = run_s[rb] * resc + (ps0 + ps1);
     if constexpr (VEC) run_o[rb] = run_o[rb] * resc + po;
+    else run_s[rb] = run_s[rb] * resc + (ps0 + ps1);
     run_m[rb] = m_new;
     run_c[rb] = c_new;
   };
@@ -439,8 +450,8 @@ __global__ __launch_bounds__(256, 2) void lse2_kernel(const LaunchArgs args) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       const float e = fast_exp2(__builtin_fmaf(acc[r], lscale, c));
-      ps += e;
       if constexpr (VEC) po = __builtin_fmaf(e, v16[r], po);
+      else ps += e;
     }
     if constexpr (VEC) run_o[rb] = po;
     run_s[rb] = ps;
@@ -505,9 +516,10 @@ __global__ __launch_bounds__(256, 2) void lse2_kernel(const LaunchArgs args) {
       }
     }
     if (q >= 2 && q < 10) {
-      s.ps0 += s.e[2 * q - 4];
-      s.ps1 += s.e[2 * q - 3];
-      if constexpr (VEC) {
+      if constexpr (!VEC) {
+        s.ps0 += s.e[2 * q - 4];
+        s.ps1 += s.e[2 * q - 3];
+      } else {
         const int r = 2 * q - 4;  // values r, r + 1 of group r / 4
         s.po = __builtin_fmaf(s.e[r], s.v[(r / 4) & 1][r % 4],
                               __builtin_fmaf(s.e[r + 1], s.v[(r / 4) & 1][r % 4 + 1], s.po));
@@ -515,11 +527,12 @@ __global__ __launch_bounds__(256, 2) void lse2_kernel(const LaunchArgs args) {
     }
   };
   auto softmax_tail = [&](SoftmaxStage& s, int rb) {  // what pieces 0..11 left undone
-    s.ps0 += s.e[14];
-    s.ps1 += s.e[15];
     const float resc = fast_exp2(s.c);
-    run_s[rb] = run_s[rb] * resc + (s.ps0 + s.ps1);
-    if constexpr (VEC) {
+    if constexpr (!VEC) {
+      s.ps0 += s.e[14];
+      s.ps1 += s.e[15];
+      run_s[rb] = run_s[rb] * resc + (s.ps0 + s.ps1);
+    } else {
       s.po = __builtin_fmaf(s.e[14], s.v[1][2], __builtin_fmaf(s.e[15], s.v[1][3], s.po));
       run_o[rb] = run_o[rb] * resc + s.po;
     }
