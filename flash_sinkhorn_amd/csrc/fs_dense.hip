@@ -60,12 +60,21 @@ void dense_plan(const SmallArgs& a, DenseArgs& t) {
   for (int i = 0; i < 2; ++i) t.blocks[i] = (a.rows[i] + 255) / 256 * 8;
   t.ld = t.blocks[1] * 32;
   t.steps = (a.d + 15) / 16;
-  // enough workgroups for two on every CU, each over as long a run of columns as that leaves;
-  // below that smaller ones, over 256 columns
+  // Two workgroups of 64 rows run on a CU at a time, each over a run of columns: the length whose rounds
+  // over the chip cost least, counting a 256-column piece's time for what a workgroup does around
+  // its run.  (With the longest run that still gives 512 workgroups the last round ran nearly empty
+  // at most sizes: 6,000 x 6,000, 564 workgroups, 46.7 us a step against 39.5; 9,000 points 109
+  // against 88; 12,000 169 against 145; 4,000 x 5,000 29.6 against 28.5.)
+  // Where there is no work for 512, smaller ones, over 256 columns.
   const int iters = t.ld / 256, groups = (t.n + 63) / 64;
   t.large = (double)a.items * groups * iters >= 512.0;
   t.groups = t.large ? groups : (t.n + 31) / 32;
-  const int run = t.large ? (int)std::min<double>(iters, std::floor((double)a.items * groups * iters / 512.0)) : 1;
+  int run = 1;
+  double cost = 0.0;
+  for (int r = 1; t.large && r <= iters; ++r) {
+    const double c = std::ceil((double)a.items * groups * ((iters + r - 1) / r) / 512.0) * (r + 1);
+    if (cost == 0.0 || c < cost) cost = c, run = r;
+  }
   t.chunk = run * 256;
   t.chunks = (iters + run - 1) / run;
 }
