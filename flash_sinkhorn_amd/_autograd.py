@@ -113,10 +113,12 @@ class _SinkhornCostFn(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, y, a, b, eps_list: Tuple[float, ...], config: _SinkhornConfig,
-                label_x, label_y, label_cost_matrix, presolved=None):
+                label_x, label_y, label_cost_matrix, presolved=None, schedule_of_points=False):
         """``presolved``: the tuple ``sinkhorn_flashstyle_symmetric`` would return for this
         problem (with ``return_prelast=config.last_extrapolation``), when the caller has already
-        run the solve (the two self terms of a debiased loss are solved together)."""
+        run the solve (the two self terms of a debiased loss are solved together).
+        ``schedule_of_points``: ``eps_list`` is the schedule by the diameter of x and y, which the
+        solver need not find out again (two passes over the clouds and a wait for the device)."""
         eps_last = float(eps_list[-1])
         seed_keys = None
         if presolved is not None:
@@ -136,7 +138,8 @@ class _SinkhornCostFn(torch.autograd.Function):
         else:
             info = {} if x.shape[1] <= 128 else None  # (wide rows: no tile tests, nothing to ask for)
             out = sinkhorn_flashstyle_symmetric(
-                x, y, a, b, solve_info=info, blur=config.blur, scaling=config.scaling,
+                x, y, a, b, solve_info=info, eps_list=eps_list if schedule_of_points else None,
+                blur=config.blur, scaling=config.scaling,
                 use_epsilon_scaling=config.use_epsilon_scaling, eps=config.eps,
                 n_iters=config.n_iters, allow_tf32=config.allow_tf32, use_exp2=config.use_exp2,
                 cost_scale=config.cost_scale, rho_x=config.rho_x, rho_y=config.rho_y,
@@ -187,4 +190,4 @@ class _SinkhornCostFn(torch.autograd.Function):
             grad_a = grad_out * f_cost
         if b.requires_grad:
             grad_b = grad_out * g_cost
-        return grad_x, grad_y, grad_a, grad_b, None, None, None, None, None, None
+        return grad_x, grad_y, grad_a, grad_b, None, None, None, None, None, None, None

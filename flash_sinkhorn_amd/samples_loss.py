@@ -264,8 +264,10 @@ class SamplesLoss(torch.nn.Module):
 
         def ot(xb, yb, ab, bb, lx, ly, presolved=None):
             sched = tuple(self._eps_list_for_inputs(xb, yb))
+            of_points = (self.use_epsilon_scaling and self.diameter is None
+                         and self.eps_list is None)
             return _SinkhornCostFn.apply(xb, yb, ab, bb, sched, config, lx, ly,
-                                         self.label_cost_matrix, presolved)
+                                         self.label_cost_matrix, presolved, of_points)
 
         # The self terms are independent solves; without early stopping, labels or an
         # asymmetric relaxation they advance together, one launch per step for both.
