@@ -67,11 +67,12 @@ static int launch_coarse_dp(const LaunchArgs& a, int blocks, hipStream_t st) {
 }
 
 int launch_row_seeds(const LaunchArgs& a, int dp, int nsides, hipStream_t st) {
-  const int sb0 = (a.side[0].nq + 7) / 8;
-  const int sb1 = nsides > 1 ? (a.side[1].nq + 7) / 8 : 0;
+  const int sb0 = (a.side[0].nq + kSeedRows - 1) / kSeedRows;
+  const int sb1 = nsides > 1 ? (a.side[1].nq + kSeedRows - 1) / kSeedRows : 0;
   LaunchArgs b = a;
   b.sel_pred = 0;
-  hipLaunchKernelGGL((coarse_bias_kernel<0>), dim3(sb0 + sb1), dim3(64), 0, st, b, 0, 0, sb0, dp);
+  hipLaunchKernelGGL((coarse_bias_kernel<0>), dim3((sb0 + sb1 + kBiasWaves - 1) / kBiasWaves), dim3(64 * kBiasWaves), 0,
+                     st, b, 0, 0, sb0, sb0 + sb1, dp);
   return hipGetLastError() == hipSuccess ? FS_OK : FS_ERR_LAUNCH_FAILED;
 }
 
@@ -80,12 +81,13 @@ static int launch_coarse(const LaunchArgs& a, int dp, int rb, int blocks, hipStr
   // the per-tile records of the key bias, for both sides (tiles past the last key included)
   const int tiles0 = (a.side[0].nk + 63) / 64 + kAuxPadTiles;
   const int tiles1 = blocks > a.blocks0 ? (a.side[1].nk + 63) / 64 + kAuxPadTiles : 0;
-  // behind them, per 8 query rows one block that computes where the rows' maxima start
+  // behind them, per kSeedRows query rows one wavefront that computes where the rows' maxima start
   const bool seeds = a.side[0].seed != nullptr;
-  const int sb0 = seeds ? (a.side[0].nq + 7) / 8 : 0;
-  const int sb1 = seeds && blocks > a.blocks0 ? (a.side[1].nq + 7) / 8 : 0;
-  hipLaunchKernelGGL((coarse_bias_kernel<0>), dim3(tiles0 + tiles1 + sb0 + sb1), dim3(64), 0, st, a,
-                     tiles0, tiles0 + tiles1, sb0, dp);
+  const int sb0 = seeds ? (a.side[0].nq + kSeedRows - 1) / kSeedRows : 0;
+  const int sb1 = seeds && blocks > a.blocks0 ? (a.side[1].nq + kSeedRows - 1) / kSeedRows : 0;
+  const int groups = (tiles0 + tiles1 + kBiasWaves - 1) / kBiasWaves + (sb0 + sb1 + kBiasWaves - 1) / kBiasWaves;
+  hipLaunchKernelGGL((coarse_bias_kernel<0>), dim3(groups), dim3(64 * kBiasWaves), 0, st, a, tiles0,
+                     tiles0 + tiles1, sb0, sb0 + sb1, dp);
   if (hipGetLastError() != hipSuccess) return FS_ERR_LAUNCH_FAILED;
   switch (dp) {
     case 16: return launch_coarse_dp<16>(a, blocks, st);

@@ -62,7 +62,7 @@ namespace fs {
 // sub-tile.  Keys past the end of the key set get a bias that masks them.  T only makes this a
 // template (header-defined kernel).
 //
-// The blocks behind the tiles (8 query rows each, side 0 first: seed_blocks0 of them) compute
+// The wavefronts behind the tiles (kSeedRows query rows each, side 0 first: seed_blocks0 of them) compute
 // where the rows' running maxima start.  A row whose largest logit of the last launch sat at key
 // j starts from its current logit at j, computed on the vector pipe from the same planes:
 // whatever the potentials did since, this is a logit of the row, hence a lower bound of its new
@@ -70,78 +70,105 @@ namespace fs {
 // result exact; a stale one only costs tests that pass.)  The sum of the fp32 roundings of the
 // two routes to a logit is far below 1/64 of the row's bound on its cross products, which is taken
 // off together with one base-2 unit.  A row without a key gets -3e38.
+//
+// Bound by the chain of loads behind best_key, and before that by the atomic maxima of the carried
+// margins, which all go to one cache line: a workgroup combines those of its sixteen tiles (one atomic
+// per tile: 21 against 11 us a launch at 50,000 x 64).  A wavefront takes 16 rows' starts, two chains at once.
+constexpr int kBiasWaves = 16, kSeedRows = 16;
 template <int T>
-__global__ __launch_bounds__(64) void coarse_bias_kernel(const LaunchArgs args, int tiles0, int tiles_all,
-                                                         int seed_blocks0, int dp) {
+__global__ __launch_bounds__(64 * kBiasWaves) void coarse_bias_kernel(const LaunchArgs args, int tiles0, int tiles_all,
+                                                                      int seed_blocks0, int seed_blocks, int dp) {
   // variant chosen on the device: nothing reads the records when the plain kernel runs
   if (args.sel_pred && args.sel[kSelWord] != 0u) return;
   if (args.sweep && blockIdx.x == 0 && threadIdx.x == 0) args.sel[kSelRan] = 0u;
   if (args.queue != nullptr)  // lse_sparse_kernel's work queues start empty
-    for (int i = blockIdx.x * 64 + threadIdx.x; i < 2 * 8 * kQueueWords; i += gridDim.x * 64)
+    for (int i = blockIdx.x * (64 * kBiasWaves) + threadIdx.x; i < 2 * 8 * kQueueWords; i += gridDim.x * (64 * kBiasWaves))
       args.queue[i] = 0u;
-  if ((int)blockIdx.x >= tiles_all) {
-    int blk = blockIdx.x - tiles_all;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int tile_groups = (tiles_all + kBiasWaves - 1) / kBiasWaves;
+  if ((int)blockIdx.x >= tile_groups) {
+    int blk = ((int)blockIdx.x - tile_groups) * kBiasWaves + wave;
+    if (blk >= seed_blocks) return;
     const bool second_s = blk >= seed_blocks0;
     if (second_s) blk -= seed_blocks0;
     const Side& ss = second_s ? args.side[1] : args.side[0];
     if (ss.seed == nullptr) return;
     // eight lanes per row, 16 bytes of each plane per lane and 64-column piece of the row (whole
-    // cache lines per row); one short wavefront per eight rows, so that the launch is as long as
-    // one chain of loads
-    const int lane = threadIdx.x, piece = lane & 7, sub = lane >> 3;
+    // cache lines per row)
+    constexpr int U = kSeedRows / 8;
+    const int piece = lane & 7, sub = lane >> 3;
     const float inv_ls = ss.plane_scale[ss.ps_q] * ss.plane_scale[ss.ps_k] / ss.qscale;
-    {
-      const int row = blk * 8 + sub;
-      const int rc = min(row, ss.nq - 1);
-      const int j = ss.best_key[rc];
-      const int jc = min(max(j, 0), ss.nk - 1);
-      float b = ss.kc0 * ss.kb0[jc];  // (every lane of the row: the loads go out with the planes')
-      if (ss.kb1) b += ss.kc1 * ss.kb1[jc];
-      if (ss.kb2) b += ss.kc2 * ss.kb2[jc];
-      float dot = 0.f, l1 = 0.f;
-      // words [w0, w0 + 4) of each plane: rows wider than 64 columns take more than one round
-      for (int w0 = piece * 4; w0 < dp / 2; w0 += 32) {
-        const unsigned* q = ss.qplanes + (size_t)rc * (size_t)dp + w0;
-        const unsigned* k = ss.kplanes + (size_t)jc * (size_t)dp + w0;
-        const u32x4 qh4 = *reinterpret_cast<const u32x4*>(q);
-        const u32x4 ql4 = *reinterpret_cast<const u32x4*>(q + dp / 2);
-        const u32x4 kh4 = *reinterpret_cast<const u32x4*>(k);
-        const u32x4 kl4 = *reinterpret_cast<const u32x4*>(k + dp / 2);
+    int j[U], rc[U], jc[U];
+    float b[U], dot[U], l1[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      rc[u] = min(blk * kSeedRows + 8 * u + sub, ss.nq - 1);
+      j[u] = ss.best_key[rc[u]];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      jc[u] = min(max(j[u], 0), ss.nk - 1);
+      b[u] = ss.kc0 * ss.kb0[jc[u]];  // (every lane of the row: the loads go out with the planes')
+      if (ss.kb1) b[u] += ss.kc1 * ss.kb1[jc[u]];
+      if (ss.kb2) b[u] += ss.kc2 * ss.kb2[jc[u]];
+      dot[u] = l1[u] = 0.f;
+    }
+    // words [w0, w0 + 4) of each plane: rows wider than 64 columns take more than one round
+    for (int w0 = piece * 4; w0 < dp / 2; w0 += 32) {
+      u32x4 qh4[U], ql4[U], kh4[U], kl4[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const unsigned* q = ss.qplanes + (size_t)rc[u] * (size_t)dp + w0;
+        const unsigned* k = ss.kplanes + (size_t)jc[u] * (size_t)dp + w0;
+        qh4[u] = *reinterpret_cast<const u32x4*>(q);
+        ql4[u] = *reinterpret_cast<const u32x4*>(q + dp / 2);
+        kh4[u] = *reinterpret_cast<const u32x4*>(k);
+        kl4[u] = *reinterpret_cast<const u32x4*>(k + dp / 2);
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           // (words copied out first: a bit cast applied to a vector element reads element 0)
-          const unsigned qhw = qh4[e], qlw = ql4[e], khw = kh4[e], klw = kl4[e];
+          const unsigned qhw = qh4[u][e], qlw = ql4[u][e], khw = kh4[u][e], klw = kl4[u][e];
           const f16x2 qh = __builtin_bit_cast(f16x2, qhw), ql = __builtin_bit_cast(f16x2, qlw);
           const f16x2 kh = __builtin_bit_cast(f16x2, khw), kl = __builtin_bit_cast(f16x2, klw);
-          dot = __builtin_amdgcn_fdot2(kh, qh, dot, false);
-          dot = __builtin_amdgcn_fdot2(kh, ql, dot, false);
-          dot = __builtin_amdgcn_fdot2(kl, qh, dot, false);
-          l1 += fabsf((float)qh[0]) + fabsf((float)qh[1]);
+          dot[u] = __builtin_amdgcn_fdot2(kh, qh, dot[u], false);
+          dot[u] = __builtin_amdgcn_fdot2(kh, ql, dot[u], false);
+          dot[u] = __builtin_amdgcn_fdot2(kl, qh, dot[u], false);
+          l1[u] += fabsf((float)qh[0]) + fabsf((float)qh[1]);
         }
-      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
 #pragma unroll
       for (int o = 4; o > 0; o >>= 1) {
-        dot += __shfl_xor(dot, o, 64);
-        l1 += __shfl_xor(l1, o, 64);
+        dot[u] += __shfl_xor(dot[u], o, 64);
+        l1[u] += __shfl_xor(l1[u], o, 64);
       }
+      const int row = blk * kSeedRows + 8 * u + sub;
       if (piece == 0 && row < ss.nq) {
         float w = -3.0e38f;
         // a key that is masked out (bias at the stand-in for -inf) says nothing about the row
-        if (j >= 0 && b > 0.5f * kNegBig) {
-          const float corr = 24.5f * l1 + (float)dp * 0x1p-9f + inv_ls;  // as in lse_coarse_kernel
-          b = fmaxf(fmaxf(b, kNegBig) * inv_ls, -3.0e38f);
-          w = fmaxf(dot + b - (corr * 0x1p-6f + inv_ls), -3.0e38f);
+        if (j[u] >= 0 && b[u] > 0.5f * kNegBig) {
+          const float corr = 24.5f * l1[u] + (float)dp * 0x1p-9f + inv_ls;  // as in lse_coarse_kernel
+          const float bias = fmaxf(fmaxf(b[u], kNegBig) * inv_ls, -3.0e38f);
+          w = fmaxf(dot[u] + bias - (corr * 0x1p-6f + inv_ls), -3.0e38f);
         }
         ss.seed[row] = w;
       }
     }
     return;
   }
-  int tile = blockIdx.x;
+  __shared__ float sh_change[2][kBiasWaves];  // [role][wavefront] largest change of a key's bias; -1: none
+  if (lane < 2) sh_change[lane][wave] = -1.f;
+  int tile = blockIdx.x * kBiasWaves + wave;
+  const bool in = tile < tiles_all;  // (else the last tile again, for nobody)
+  tile = min(tile, tiles_all - 1);
   const bool second = tile >= tiles0;
   if (second) tile -= tiles0;
   const Side& sd = second ? args.side[1] : args.side[0];
-  const int lane = threadIdx.x, li = lane & 31, h = lane >> 5;
+  const int li = lane & 31, h = lane >> 5;
   const int j = tile * 64 + lane;
   const float lscale = sd.qscale / (sd.plane_scale[sd.ps_q] * sd.plane_scale[sd.ps_k]);
   const float inv_lscale = 1.0f / lscale;
@@ -163,15 +190,17 @@ __global__ __launch_bounds__(64) void coarse_bias_kernel(const LaunchArgs args, 
     ah = __builtin_bit_cast(_Float16, (unsigned short)(__builtin_bit_cast(unsigned short, ah) - 1));
   const unsigned aw = (unsigned)__builtin_bit_cast(unsigned short, ah) * 0x00010001u;
   unsigned* rec = sd.key_aux + (size_t)tile * kAuxWords;
-  *reinterpret_cast<u32x4*>(rec + kAuxA + lane * 4) = u32x4{aw, aw, aw, aw};
-  rec[kAuxB + lane] = __builtin_bit_cast(unsigned, b - (float)ah * 0x1p18f);
   const float mx_sub = __shfl(mx, (lane & 1) * 32, 64);  // lanes 0 and 1: the two sub-tiles' maxima
-  rec[kAuxMax + lane] = lane < 2 ? __builtin_bit_cast(unsigned, mx_sub) : 0u;
+  if (in) {
+    *reinterpret_cast<u32x4*>(rec + kAuxA + lane * 4) = u32x4{aw, aw, aw, aw};
+    rec[kAuxB + lane] = __builtin_bit_cast(unsigned, b - (float)ah * 0x1p18f);
+    rec[kAuxMax + lane] = lane < 2 ? __builtin_bit_cast(unsigned, mx_sub) : 0u;
+  }
 
   // Carried margins: the largest change of a key's bias since the last launch with this side
   // (raw units), and the generation of the margins: a launch whose tag differs from the one the
   // margins were taken under (other operands, eps, coefficients) starts a new one.
-  if (sd.bias_prev != nullptr && args.sel != nullptr) {
+  if (in && sd.bias_prev != nullptr && args.sel != nullptr) {
     const int side = sd.ps_q;  // the margins' state goes with the matrix that holds the query rows
     float dch = 0.f;
     if (j < sd.nk) {
@@ -182,10 +211,7 @@ __global__ __launch_bounds__(64) void coarse_bias_kernel(const LaunchArgs args, 
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) dch = fmaxf(dch, __shfl_xor(dch, o, 64));
     if (lane == 0) {
-      // (most wavefronts find a larger value already there; a stale read only costs an atomic)
-      const unsigned dbits = __builtin_bit_cast(unsigned, dch);
-      unsigned* dslot = &args.sel[kSelDmax + side * kDmaxSlots + (tile & (kDmaxSlots - 1))];
-      if (dbits > *dslot) atomicMax(dslot, dbits);
+      sh_change[side][wave] = dch;
       if (tile == 0 && args.sel[kSelTag + side] != args.tag[second ? 1 : 0]) {
         args.sel[kSelTag + side] = args.tag[second ? 1 : 0];
         // entries carry the generation in 8 bits and are cleared only with the planes: after 255
@@ -193,6 +219,17 @@ __global__ __launch_bounds__(64) void coarse_bias_kernel(const LaunchArgs args, 
         args.sel[kSelGen + side] = min(args.sel[kSelGen + side] + 1u, 256u);
         args.sel[kSelBump + side] = 1u;
       }
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x < 2) {
+    float most = -1.f;
+#pragma unroll
+    for (int w = 0; w < kBiasWaves; ++w) most = fmaxf(most, sh_change[threadIdx.x][w]);
+    if (most > 0.f) {  // (a later workgroup may find a larger value there; a stale read only costs an atomic)
+      const unsigned dbits = __builtin_bit_cast(unsigned, most);
+      unsigned* dslot = &args.sel[kSelDmax + threadIdx.x * kDmaxSlots + (blockIdx.x & (kDmaxSlots - 1))];
+      if (dbits > *dslot) atomicMax(dslot, dbits);
     }
   }
 }
