@@ -89,9 +89,15 @@ _KEPT_MAX = 1 << 26  # entries of the plan
 _state = threading.local()
 
 
-def _kept_ok(n: int, m: int, d: int, allow_tf32: bool) -> bool:
-    """Whether the product is taken on kept matrices (``fs_hvp``): they stay below 1 GiB together."""
-    return (0 < n <= 65536 and 0 < m <= _KEPT_MAX_COLUMNS and d > 0 and n * m <= _KEPT_MAX
+def _kept_ok(x, y, f_hat, g_hat, A, allow_tf32: bool) -> bool:
+    """Whether the product is taken on kept matrices (``fs_hvp``): they stay below 1 GiB together.
+    The library is handed bare pointers, so devices and lengths are settled here; a call with
+    others goes on to the general path, which complains."""
+    (n, d), m = x.shape, y.shape[0]
+    return (all(t.device == x.device for t in (y, f_hat, g_hat, A))
+            and f_hat.shape == (n,) and g_hat.shape == (m,) and A.shape == (n, d)
+            and y.shape[1] == d
+            and 0 < n <= 65536 and 0 < m <= _KEPT_MAX_COLUMNS and d > 0 and n * m <= _KEPT_MAX
             and (allow_tf32 or _lib.STRICT_OPERANDS == "fp16x2")
             and not torch.cuda.is_current_stream_capturing())
 
@@ -160,7 +166,7 @@ def hvp_x_sqeuclid_from_potentials(
     e = float(eps)
     cs = float(cost_scale)
     if (mode == "none" and cg_x0 is None and not cg_stabilise_every and not return_components
-            and _kept_ok(n, m, d, allow_tf32) and e > 0.0 and cs > 0.0):
+            and _kept_ok(x, y, f_hat, g_hat, A, allow_tf32) and e > 0.0 and cs > 0.0):
         return _kept(x, y, f_hat, g_hat, A, eps=e, cost_scale=cs, rho_x=rho_x, rho_y=rho_y,
                      tau2=float(tau2), lambda_indef=float(lambda_indef), rtol=float(cg_rtol),
                      atol=float(cg_atol), max_iter=int(max_cg_iter))

@@ -266,6 +266,17 @@ def test_kept_hvp(n, m, d, rho):
             assert info.cg_iters == iters
 
 
+def test_hvp_refuses_operands_elsewhere_and_of_other_lengths():
+    from flash_sinkhorn_amd.hvp import (hvp_x_sqeuclid_from_potentials as hvp,
+                                        inverse_hvp_x_sqeuclid_from_potentials as inverse)
+    x, y, _, _ = inputs(3, 40, 30, 4)
+    X, Y, F, G, A = dev(x, y, *(np.zeros(k, np.float32) for k in (40, 30)), x)
+    for args in ((X, Y, F, G, A.cpu()), (X, Y, G, F, A), (X, Y, F[:7], G, A), (X, Y, F, G[:7], A)):
+        for fn in (hvp, inverse):
+            with pytest.raises((RuntimeError, ValueError, AssertionError)):
+                fn(*args, eps=0.3)
+
+
 # ---- the merge of the key splits: four wavefronts share them, two, four or eight at a time ----
 @pytest.mark.parametrize("n,m", [(1, 40000), (63, 9000), (257, 20000), (1000, 3000), (5000, 5100), (20000, 700)])
 def test_merge_of_key_splits(n, m):

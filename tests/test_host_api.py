@@ -142,6 +142,20 @@ def test_launchers_reject_cpu_tensors_and_bad_shapes():
         mat5_sqeuclid(x, y, torch.zeros(6), v, x, eps=0.1)
 
 
+def test_kept_hvp_takes_only_operands_of_one_device_and_the_right_lengths(monkeypatch):
+    # (its library call reads them through bare pointers)
+    from flash_sinkhorn_amd import hvp
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    x, y, f, g, A = (torch.zeros(*s) for s in ((6, 4), (5, 4), (6,), (5,), (6, 4)))
+    good = dict(x=x, y=y, f_hat=f, g_hat=g, A=A)
+    assert hvp._kept_ok(**good, allow_tf32=True)
+    for name, t in good.items():
+        assert not hvp._kept_ok(**{**good, name: t.to("meta")}, allow_tf32=True)
+    for bad in (dict(f_hat=g, g_hat=f), dict(f_hat=f[:1]), dict(g_hat=g[:, None]), dict(A=A[:5]),
+                dict(A=A.T), dict(y=y[:, :3])):
+        assert not hvp._kept_ok(**{**good, **bad}, allow_tf32=True)
+
+
 def test_deprecated_names_are_bridged_with_a_warning():
     import flash_sinkhorn_amd.kernels as K
     with warnings.catch_warnings(record=True) as rec:
