@@ -116,6 +116,8 @@ def conjugate_gradient_device(
     while enqueued < int(max_iter):
         for _ in range(min(every, int(max_iter) - enqueued)):
             a_dir = matvec(direction).float().contiguous()
+            if a_dir.numel() != m or a_dir.device != rhs.device:
+                raise ValueError("matvec must return a vector like b.")
             _lib.check(L.fs_cg_update(a_dir.data_ptr(), sol.data_ptr(), res.data_ptr(),
                                       direction.data_ptr(), state.data_ptr(), m, stream),
                        "fs_cg_update")

@@ -58,6 +58,20 @@ def _validate_device(x: torch.Tensor, others: Sequence[Tuple[str, Optional[torch
             raise ValueError(f"{name} must be on the same device as x ({x.device}), got {t.device}.")
 
 
+def _validate_problem(x: torch.Tensor, y: torch.Tensor, of_x, of_y) -> None:
+    """Clouds of one width on one (GPU) device with the vectors that go with them, (name, tensor)
+    pairs with one entry per row: the library is handed bare pointers and cannot tell."""
+    if x.ndim != 2 or y.ndim != 2:
+        raise ValueError("x and y must be 2D tensors")
+    if x.shape[1] != y.shape[1]:
+        raise ValueError("x and y must have same feature dimension")
+    for rows, named in ((x.shape[0], of_x), (y.shape[0], of_y)):
+        for name, t in named:
+            if t.numel() != rows:
+                raise ValueError(f"{name} must have length {rows}, got {t.numel()}")
+    _validate_device(x, [("y", y), *of_x, *of_y])
+
+
 def _f32c(t: torch.Tensor) -> torch.Tensor:
     """Contiguous fp32 view/copy of t (what every launcher hands to the C ABI)."""
     return t.contiguous().float()

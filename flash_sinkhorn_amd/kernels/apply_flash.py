@@ -79,7 +79,7 @@ def apply_plan_vec_flashstyle(
 ) -> torch.Tensor:
     """axis=1: P @ vec (vec [m] -> [n]); axis=0: P^T @ vec (vec [n] -> [m])."""
     n, d = x.shape
-    m = y.shape[0]
+    m, d2 = y.shape
     assert f_hat.shape == (n,), f"f_hat shape {f_hat.shape} != ({n},)"
     assert g_hat.shape == (m,), f"g_hat shape {g_hat.shape} != ({m},)"
     assert log_a.shape == (n,), f"log_a shape {log_a.shape} != ({n},)"
@@ -90,6 +90,10 @@ def apply_plan_vec_flashstyle(
     assert vec.shape == (want,), f"vec shape {vec.shape} != ({want},) for axis={axis}"
     if not x.is_cuda:
         raise ValueError("CUDA required.")
+    if d != d2:
+        raise ValueError("x and y must have the same feature dimension.")
+    _validate_device(x, [("y", y), ("f_hat", f_hat), ("g_hat", g_hat), ("log_a", log_a),
+                         ("log_b", log_b), ("vec", vec)])
     xf, yf, vf = _f32c(x), _f32c(y), _f32c(vec)
     fh, gh, la, lb = _f32c(f_hat), _f32c(g_hat), _f32c(log_a), _f32c(log_b)
     out = torch.empty((n if axis == 1 else m,), device=x.device, dtype=torch.float32)

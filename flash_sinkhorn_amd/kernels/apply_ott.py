@@ -12,7 +12,7 @@ from typing import Optional
 import torch
 
 from flash_sinkhorn_amd import _lib
-from flash_sinkhorn_amd.kernels._common import _f32c, _validate_device
+from flash_sinkhorn_amd.kernels._common import _f32c, _validate_device, _validate_problem
 
 __all__ = ["mat5_sqeuclid"]
 
@@ -33,6 +33,8 @@ def mat5_sqeuclid(
     m, d2 = y.shape
     if d != d2 or A.shape != (n, d):
         raise ValueError("Shapes must satisfy x:(n,d), y:(m,d), A:(n,d).")
+    _validate_problem(x, y, [("f", f)] + ([] if x2 is None else [("x2", x2)]),
+                      [("g", g)] + ([] if y2 is None else [("y2", y2)]))
     xf, yf, Af = _f32c(x), _f32c(y), _f32c(A)
     x2 = (xf * xf).sum(dim=1).contiguous() if x2 is None else _f32c(x2)
     y2 = (yf * yf).sum(dim=1).contiguous() if y2 is None else _f32c(y2)

@@ -21,8 +21,8 @@ from typing import Optional, Tuple
 import torch
 
 from flash_sinkhorn_amd import _lib
-from flash_sinkhorn_amd.kernels._common import (_f32c, augment_label_cost, label_cost_active,
-                                                log_weights)
+from flash_sinkhorn_amd.kernels._common import (_f32c, _validate_device, _validate_problem,
+                                                augment_label_cost, label_cost_active, log_weights)
 
 __all__ = [
     "precompute_flashsinkhorn_inputs", "compute_bias_f", "compute_bias_g",
@@ -79,6 +79,7 @@ def flashsinkhorn_lse(
         raise ValueError("x and y must have same feature dimension")
     if bias.shape[0] != m:
         raise ValueError(f"bias must have length {m}, got {bias.shape[0]}")
+    _validate_device(x, [("y", y), ("bias", bias)])
     x, y, bias = _f32c(x), _f32c(y), _f32c(bias)
     out = torch.empty((n,), device=x.device, dtype=torch.float32)
     wp, wn, fl, _keep = _lib.lse_workspace(_lib.OP_LSE, x, y, _lib.flags(use_exp2, allow_tf32),
@@ -107,6 +108,7 @@ def flashsinkhorn_lse_fused(
         raise ValueError("x and y must have same feature dimension")
     if g_hat.shape[0] != m or log_w.shape[0] != m:
         raise ValueError(f"g_hat and log_w must have length {m}")
+    _validate_device(x, [("y", y), ("g_hat", g_hat), ("log_w", log_w)])
     x, y, g_hat, log_w = _f32c(x), _f32c(y), _f32c(g_hat), _f32c(log_w)
     out = torch.empty((n,), device=x.device, dtype=torch.float32)
     wp, wn, fl, _keep = _lib.lse_workspace(_lib.OP_LSE, x, y, _lib.flags(use_exp2, allow_tf32),
@@ -244,6 +246,8 @@ def flashsinkhorn_symmetric_step(
     realised as extra feature columns (``augment_label_cost``)."""
     if not x.is_cuda or not y.is_cuda:
         raise ValueError("x and y must be CUDA tensors")
+    _validate_problem(x, y, [("f_hat", f_hat), ("log_a", log_a)],
+                      [("g_hat", g_hat), ("log_b", log_b)])
     if label_cost_active(label_x, label_y, label_cost_matrix, lambda_y):
         x, y = augment_label_cost(x, y, label_x, label_y, label_cost_matrix, lambda_x, lambda_y)
     return _symmetric_step_raw(

@@ -15,8 +15,8 @@ from typing import Optional, Tuple
 import torch
 
 from flash_sinkhorn_amd import _lib
-from flash_sinkhorn_amd.kernels._common import (_f32c, augment_label_cost, label_cost_active,
-                                                log_weights)
+from flash_sinkhorn_amd.kernels._common import (_f32c, _validate_device, augment_label_cost,
+                                                label_cost_active, log_weights)
 
 __all__ = ["sinkhorn_geomloss_online_grad_sqeuclid"]
 
@@ -51,6 +51,7 @@ def sinkhorn_geomloss_online_grad_sqeuclid(
         raise ValueError("a and f shapes must match x.")
     if b.shape[0] != m or g.shape[0] != m:
         raise ValueError("b and g shapes must match y.")
+    _validate_device(x, [("y", y), ("a", a), ("b", b), ("f", f), ("g", g)])
     if x.dtype not in (torch.float16, torch.bfloat16, torch.float32):
         raise ValueError(f"Unsupported dtype for x/y: {x.dtype}")
     use_labels = label_cost_active(label_x, label_y, label_cost_matrix, lambda_y)

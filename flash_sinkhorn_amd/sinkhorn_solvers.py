@@ -15,8 +15,8 @@ import torch
 
 from flash_sinkhorn_amd import _graphs, _lib, _small
 from flash_sinkhorn_amd.kernels._common import (
-    _f32c, augment_label_cost, dampening, epsilon_schedule, label_cost_active, log_weights,
-    max_diameter,
+    _f32c, _validate_problem, augment_label_cost, dampening, epsilon_schedule, label_cost_active,
+    log_weights, max_diameter,
 )
 
 __all__ = ["sinkhorn_flashstyle_alternating", "sinkhorn_flashstyle_symmetric"]
@@ -118,6 +118,7 @@ def sinkhorn_flashstyle_alternating(
     rho_x, rho_y = _resolve_rho(rho, reach, rho_x, rho_y, reach_x, reach_y)
     damp_f, damp_g = dampening(eps, rho_x), dampening(eps, rho_y)
     _require_cuda(x, y)
+    _validate_problem(x, y, [("a", a)], [("b", b)])
     stops = threshold is not None and threshold > 0.0
     if (not ott_convention and eps > 0.0 and int(n_iters) > 0
             and not (stops and (check_every <= 0 or torch.cuda.is_current_stream_capturing()))
@@ -236,6 +237,7 @@ def sinkhorn_flashstyle_symmetric(
         eps_list = list(eps_list)[: int(n_iters)]
 
     _require_cuda(x, y)
+    _validate_problem(x, y, [("a", a)], [("b", b)])
     xf, yf = x.float().contiguous(), y.float().contiguous()
     alpha = (cost_scale * (xf * xf).sum(dim=1)).contiguous()
     beta = (cost_scale * (yf * yf).sum(dim=1)).contiguous()
@@ -495,6 +497,8 @@ def sinkhorn_flashstyle_symmetric_self_pair(
         if out is not None:
             return out
 
+    _require_cuda(x, y)
+    _validate_problem(x, y, [("a", a)], [("b", b)])
     xf, yf = x.detach().float().contiguous(), y.detach().float().contiguous()
     ex, ey = schedule(xf), schedule(yf)
     alpha_x = (cost_scale * (xf * xf).sum(dim=1)).contiguous()

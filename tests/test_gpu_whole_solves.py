@@ -173,6 +173,17 @@ def test_loss_and_gradients(n, m, d, debias):
         assert np.abs(g.cpu().numpy() - w).max() < GRAD * np.abs(p).max()
 
 
+def test_weights_elsewhere_are_refused():
+    from flash_sinkhorn_amd import SamplesLoss
+    x, y, a, b = inputs(8, 61, 50, 4)
+    X, Y, A, B = dev(x, y, a, b)
+    for kw in (dict(), dict(potentials=True), dict(debias=True),
+               dict(backend="alternating", use_epsilon_scaling=False, eps=0.1, n_iters=3)):
+        for w in ((A.cpu(), B), (A, B.cpu())):
+            with pytest.raises(ValueError, match="same device"):
+                SamplesLoss("sinkhorn", **kw)(w[0], X, w[1], Y)
+
+
 def test_batch_equals_its_items():
     from flash_sinkhorn_amd import SamplesLoss
     rng = np.random.default_rng(4)

@@ -142,6 +142,48 @@ def test_launchers_reject_cpu_tensors_and_bad_shapes():
         mat5_sqeuclid(x, y, torch.zeros(6), v, x, eps=0.1)
 
 
+class OnCard(torch.Tensor):
+    """A host tensor that says it is on the GPU."""
+    is_cuda = True
+    device = torch.device("cuda", 0)
+
+
+def on_card(t):
+    return t.as_subclass(OnCard)
+
+
+def test_vectors_elsewhere_or_of_other_lengths_never_reach_the_library(monkeypatch):
+    # (it takes bare pointers: a host tensor, or one that is too short, would be read all the same)
+    from flash_sinkhorn_amd import SamplesLoss, sinkhorn_solvers as S
+    from flash_sinkhorn_amd.kernels import apply_flash, apply_ott
+    from flash_sinkhorn_amd.kernels import sinkhorn_flashstyle_sqeuclid as L
+    from flash_sinkhorn_amd.kernels.sinkhorn_triton_grad_sqeuclid import (
+        sinkhorn_geomloss_online_grad_sqeuclid as grad)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    x, y, a, b = (on_card(torch.ones(*s)) for s in ((6, 4), (5, 4), (6,), (5,)))
+    fixed = dict(use_epsilon_scaling=False, eps=0.1, n_iters=2)
+    calls = [
+        (lambda x, y, a, b: S.sinkhorn_flashstyle_symmetric(x, y, a, b, fused=False, **fixed)),
+        (lambda x, y, a, b: S.sinkhorn_flashstyle_symmetric(x, y, a, b, **fixed)),
+        (lambda x, y, a, b: S.sinkhorn_flashstyle_alternating(x, y, a, b, eps=0.1, n_iters=2)),
+        (lambda x, y, a, b: S.sinkhorn_flashstyle_symmetric_self_pair(x, a, y, b, **fixed)),
+        (lambda x, y, a, b: L.flashsinkhorn_symmetric_step(x, y, a, b, a, b, 0.1)),
+        (lambda x, y, a, b: L.flashsinkhorn_lse(x, y, b, 0.1)),
+        (lambda x, y, a, b: L.flashsinkhorn_lse_fused(x, y, b, b, 0.1)),
+        (lambda x, y, a, b: apply_flash.apply_plan_vec_flashstyle(x, y, a, b, a, b, b, eps=0.1, axis=1)),
+        (lambda x, y, a, b: apply_ott.mat5_sqeuclid(x, y, a, b, x, eps=0.1)),
+        (lambda x, y, a, b: grad(x, y, a, b, a, b, eps=0.1)),
+    ]
+    for call in calls:
+        for bad in ((x, y, a, b.as_subclass(torch.Tensor)), (x, y, a, b[:3])):
+            with pytest.raises((ValueError, AssertionError), match="same device|length|shape"):
+                call(*bad)
+        with pytest.raises(ValueError, match="feature dimension|Shapes"):
+            call(x, y[:, :3], a, b)
+    with pytest.raises(ValueError, match="same device"):
+        SamplesLoss(**fixed)(a, x, b.as_subclass(torch.Tensor), y)
+
+
 def test_kept_hvp_takes_only_operands_of_one_device_and_the_right_lengths(monkeypatch):
     # (its library call reads them through bare pointers)
     from flash_sinkhorn_amd import hvp
