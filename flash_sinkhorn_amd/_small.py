@@ -122,6 +122,14 @@ def _operands_ok(allow_tf32: bool) -> bool:
     return allow_tf32 or _lib.STRICT_OPERANDS == "fp16x2"
 
 
+def held(*values: Optional[float]) -> bool:
+    """Whether fp32 holds every one of these (None: not given) as a positive normal number.  The
+    library reads zero and less as "none" (a strict marginal, no early stopping), so a relaxation of
+    zero, a negative one or one that rounds to zero would be another problem: the general path
+    takes such values, or refuses them."""
+    return all(v is None or 1.1754944e-38 <= v <= 3.4028234e38 for v in values)
+
+
 def _rho(rho: Optional[float]) -> float:
     return 0.0 if rho is None else float(rho)
 
@@ -279,12 +287,15 @@ def loss_problem(loss, args, label_x, label_y):
         return None
     if loss.threshold is not None and not loss.threshold > 0.0:
         return None
+    if not held(loss.rho_x, loss.rho_y, loss.threshold, loss.cost_scale):
+        return None
     if loss.debias and loss.rho_x != loss.rho_y and not loss.potentials:
         return None
     if loss.use_epsilon_scaling:
-        if not (loss.blur > 0.0 and 0.0 < loss.scaling < 1.0) or (loss.n_iters or 1) <= 0:
+        if not (loss.blur > 0.0 and held(loss.blur ** 2) and 0.0 < loss.scaling < 1.0) \
+                or (loss.n_iters or 1) <= 0:
             return None
-    elif loss.eps is None or loss.n_iters is None or not loss.eps > 0.0 or loss.n_iters <= 0:
+    elif loss.eps is None or loss.n_iters is None or not held(loss.eps) or loss.n_iters <= 0:
         return None
     if len(args) == 2:
         (x, y), a, b = args, None, None

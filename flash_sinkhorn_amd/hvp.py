@@ -23,7 +23,7 @@ from typing import Optional, Sequence, Tuple
 
 import torch
 
-from flash_sinkhorn_amd import _lib
+from flash_sinkhorn_amd import _lib, _small
 from flash_sinkhorn_amd.cg import conjugate_gradient, conjugate_gradient_device
 from flash_sinkhorn_amd.kernels._common import log_weights
 from flash_sinkhorn_amd.kernels.sinkhorn_triton_apply_sqeuclid import (
@@ -166,7 +166,7 @@ def hvp_x_sqeuclid_from_potentials(
     e = float(eps)
     cs = float(cost_scale)
     if (mode == "none" and cg_x0 is None and not cg_stabilise_every and not return_components
-            and _kept_ok(x, y, f_hat, g_hat, A, allow_tf32) and e > 0.0 and cs > 0.0):
+            and _kept_ok(x, y, f_hat, g_hat, A, allow_tf32) and _small.held(e, cs, rho_x, rho_y)):
         return _kept(x, y, f_hat, g_hat, A, eps=e, cost_scale=cs, rho_x=rho_x, rho_y=rho_y,
                      tau2=float(tau2), lambda_indef=float(lambda_indef), rtol=float(cg_rtol),
                      atol=float(cg_atol), max_iter=int(max_cg_iter))

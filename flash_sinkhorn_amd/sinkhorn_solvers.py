@@ -120,9 +120,9 @@ def sinkhorn_flashstyle_alternating(
     _require_cuda(x, y)
     _validate_problem(x, y, [("a", a)], [("b", b)])
     stops = threshold is not None and threshold > 0.0
-    if (not ott_convention and eps > 0.0 and int(n_iters) > 0
+    if (not ott_convention and int(n_iters) > 0
             and not (stops and (check_every <= 0 or torch.cuda.is_current_stream_capturing()))
-            and (rho_x is None or rho_x > 0.0) and (rho_y is None or rho_y > 0.0)
+            and _small.held(eps, cost_scale, rho_x, rho_y, threshold if stops else None)
             and _small.alternating_problem(x, y, a, b, allow_tf32)):
         s = _small.solve(*_small.points(x, y), _f32c(a.detach()), _f32c(b.detach()), items=1,
                          eps=float(eps), entries=int(n_iters), cost_scale=float(cost_scale),
@@ -212,7 +212,7 @@ def sinkhorn_flashstyle_symmetric(
     # small clouds: the whole solve in one library call (diagnostics of the planes and warm starts
     # are the general path's)
     if (fused is not False and not use_labels and solve_info is None
-            and f_init is None and g_init is None
+            and f_init is None and g_init is None and _small.held(cost_scale, rho_x, rho_y)
             and _small.solver_problem(x, y, a, b, allow_tf32,
                                       eps_list is None and not use_epsilon_scaling,
                                       threshold is not None and threshold > 0.0)):
@@ -392,17 +392,20 @@ def _small_symmetric(x, y, a, b, blur, scaling, use_epsilon_scaling, last_extrap
         return None
     if threshold is not None and not threshold > 0.0:
         threshold = None  # never met
+    if not _small.held(threshold):
+        return None
     if threshold is not None and return_n_iters and eps_list is None and use_epsilon_scaling \
             and diameter is None:
         diameter = max_diameter(x, y)  # (the length of the schedule is asked for)
     if x.shape[1] > _small.WIDE_D and eps_list is None and use_epsilon_scaling and diameter is None:
         diameter = max_diameter(x, y)
     if eps_list is None and not use_epsilon_scaling:
-        if eps is None or n_iters is None or not eps > 0 or int(n_iters) <= 0:
+        if eps is None or n_iters is None or not _small.held(eps) or int(n_iters) <= 0:
             return None
         sched = dict(eps=float(eps), entries=int(n_iters))
     elif eps_list is None and diameter is None:
-        if not (blur > 0 and 0.0 < scaling < 1.0) or (n_iters is not None and int(n_iters) <= 0):
+        if not (blur > 0 and _small.held(blur ** 2) and 0.0 < scaling < 1.0) \
+                or (n_iters is not None and int(n_iters) <= 0):
             return None
         sched = dict(blur=float(blur), scaling=float(scaling), cut=int(n_iters or 0))
     else:
@@ -411,7 +414,7 @@ def _small_symmetric(x, y, a, b, blur, scaling, use_epsilon_scaling, last_extrap
         eps_list = [float(e) for e in eps_list]
         if n_iters is not None:
             eps_list = eps_list[: int(n_iters)]
-        if len(eps_list) == 0 or not all(e > 0 for e in eps_list):
+        if len(eps_list) == 0 or not _small.held(*eps_list):
             return None
         sched = dict(eps_list=eps_list)
     try:
@@ -434,11 +437,12 @@ def _small_self_pair(x, a, y, b, blur, scaling, use_epsilon_scaling, last_extrap
                      eps, n_iters, rho, return_prelast):
     """``sinkhorn_flashstyle_symmetric_self_pair`` on small clouds; None as ``_small_symmetric``."""
     if use_epsilon_scaling:
-        if not (blur > 0 and 0.0 < scaling < 1.0) or (n_iters is not None and int(n_iters) <= 0):
+        if not (blur > 0 and _small.held(blur ** 2) and 0.0 < scaling < 1.0) \
+                or (n_iters is not None and int(n_iters) <= 0):
             return None
         sched = dict(blur=float(blur), scaling=float(scaling), cut=int(n_iters or 0))
     else:
-        if eps is None or n_iters is None or not eps > 0 or int(n_iters) <= 0:
+        if eps is None or n_iters is None or not _small.held(eps) or int(n_iters) <= 0:
             return None
         sched = dict(eps=float(eps), entries=int(n_iters))
     try:
@@ -491,7 +495,8 @@ def sinkhorn_flashstyle_symmetric_self_pair(
             raise ValueError("eps_list must be non-empty")
         return lst
 
-    if _small.pair_problem(x, y, a, b, allow_tf32, not use_epsilon_scaling, self_terms=2):
+    if _small.held(cost_scale, rho) and _small.pair_problem(
+            x, y, a, b, allow_tf32, not use_epsilon_scaling, self_terms=2):
         out = _small_self_pair(x, a, y, b, blur, scaling, use_epsilon_scaling, last_extrapolation,
                                cost_scale, eps, n_iters, rho, return_prelast)
         if out is not None:

@@ -84,6 +84,37 @@ def test_one_sweep_self_problems(n, m, d, eps):
             assert np.abs(p.cpu().numpy() - q).max() < 2.0 ** -20 * 4.0 * (u * u).sum(axis=1).max()
 
 
+# ---- numbers that fp32 does not hold, or that the library would take for "none" ----
+@pytest.mark.parametrize("d", [4, 200])
+def test_relaxations_of_zero_and_less_are_not_strict_marginals(d):
+    from flash_sinkhorn_amd import SamplesLoss, sinkhorn_solvers as S
+    from flash_sinkhorn_amd.hvp import hvp_x_sqeuclid_from_potentials as hvp
+    x, y, a, b = inputs(2, 60, 50, d, scale=1.0 / np.sqrt(d))
+    X, Y, A, B = dev(x, y, a, b)
+    fixed = dict(use_epsilon_scaling=False, eps=0.2, n_iters=3)
+    for rho in (dict(rho=0.0), dict(rho_x=0.0), dict(rho_y=0.0)):
+        with pytest.raises(ZeroDivisionError):
+            S.sinkhorn_flashstyle_symmetric(X, Y, A, B, **rho, **fixed)
+        with pytest.raises(ZeroDivisionError):
+            S.sinkhorn_flashstyle_alternating(X, Y, A, B, eps=0.2, n_iters=3, **rho)
+    with pytest.raises(ZeroDivisionError):
+        S.sinkhorn_flashstyle_symmetric_self_pair(X, A, Y, B, rho=0.0, **fixed)
+    for rho in (dict(rho_x=0.0), dict(rho_y=0.0)):
+        with pytest.raises(ZeroDivisionError):
+            hvp(X, Y, A.log(), B.log(), X, eps=0.2, **rho)
+    # (two launches a step and damping on the host: always the general path)
+    for rho in (-0.7, 1e-50):
+        f, g = S.sinkhorn_flashstyle_symmetric(X, Y, A, B, rho=rho, **fixed)
+        u, v = S.sinkhorn_flashstyle_symmetric(X, Y, A, B, rho=rho, fused=False, **fixed)
+        assert torch.allclose(f, u, atol=1e-5, rtol=1e-5) and torch.allclose(g, v, atol=1e-5, rtol=1e-5)
+    assert SamplesLoss(reach=1e-25, **fixed)(X, Y).isnan()  # 0 * inf: rho is zero on the device
+    for fn in (lambda: SamplesLoss(blur=1e-30)(X, Y), lambda: SamplesLoss(blur=1e-30, potentials=True)(X, Y),
+               lambda: S.sinkhorn_flashstyle_symmetric(X, Y, A, B, blur=1e-30),
+               lambda: S.sinkhorn_flashstyle_symmetric_self_pair(X, A, Y, B, blur=1e-30)):
+        with pytest.raises(RuntimeError, match="bad argument"):
+            fn()
+
+
 # ---- kept products: 256-column strips, tiles of 64, 128 and 256, both shapes of the sweep ----
 @pytest.mark.parametrize("n,m,d", [(1, 1, 129), (63, 257, 130), (256, 255, 144), (1000, 1000, 784),
                                    (2100, 4099, 200), (513, 2049, 1536)])
