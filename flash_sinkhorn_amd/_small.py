@@ -58,10 +58,15 @@ def _host_words(items: int) -> torch.Tensor:
     return buf
 
 
+_SIDES = ("f", "g", "xx", "yy")
+
+
 class Solved:
     """A solve that has been enqueued: what it read, its workspace (planes, log weights, potentials in
-    the form the gradient kernel reads), the loss per item, and the standard potentials."""
-    __slots__ = ("form", "x", "y", "a", "b", "ws", "loss", "pots", "entries")
+    the form the gradient kernel reads) where a gradient may be asked for, the loss per item, and the
+    standard potentials: of a loss in one buffer, for its own backward pass, of a solver every
+    one a tensor of its own, for the caller."""
+    __slots__ = ("form", "x", "y", "a", "b", "ws", "loss", "pots", "own", "entries")
 
     def problem(self) -> Problem:
         p = Problem.from_buffer_copy(self.form)
@@ -75,14 +80,17 @@ class Solved:
     @classmethod
     def restored(cls, form: Problem, tensors) -> "Solved":
         s = cls()
-        s.form, s.loss, s.entries = form, None, None
+        s.form, s.loss, s.own, s.entries = form, None, None, None
         s.x, s.y, s.a, s.b, s.ws, s.pots = tensors
         return s
 
     def potentials(self, which: str):
-        """("f" | "g" | "xx" | "yy") -> (of the cost, of the gradient), each [items, rows]."""
+        """("f" | "g" | "xx" | "yy") -> (of the cost, of the gradient): of a loss [items, rows] each,
+        of a solver as the caller gets them (None: not asked for)."""
+        if self.own is not None:
+            return self.own[which]
         p = self.form
-        n, m, k = p.n * p.items, p.m * p.items, ("f", "g", "xx", "yy").index(which)
+        n, m, k = p.n * p.items, p.m * p.items, _SIDES.index(which)
         at = [0, 2 * n, 2 * (n + m), 2 * (2 * n + m)][k]
         size = n if k % 2 == 0 else m
         rows = p.n if k % 2 == 0 else p.m
@@ -138,10 +146,11 @@ def solve(x, y, a, b, *, items: int, blur: float = 0.0, scaling: float = 0.0, ep
           entries: int = 0, cut: int = 0, eps_list=None, cost_scale: float, rho_x, rho_y,
           normalize: bool, self_terms: int, want_values: bool, extrapolate: bool,
           want_loss: bool, threshold: Optional[float] = None, check_every: int = 1,
-          alternating: bool = False) -> Solved:
+          alternating: bool = False, prelast: bool = False) -> Solved:
     """Enqueue one run of small problems: contiguous x [items, n, d] and y [items, m, d] of one dtype,
     weights as contiguous fp32 or None.  ``eps_list`` (host floats), ``eps`` with ``entries``, or
-    a schedule by diameter, in that order."""
+    a schedule by diameter, in that order.  Without ``want_loss``: the potentials, with ``prelast``
+    also those before the extrapolation."""
     n, d = x.shape[-2:]
     m = y.shape[-2]
     sched = 2 if eps_list is not None else (0 if eps > 0.0 else 1)
@@ -159,6 +168,10 @@ def solve(x, y, a, b, *, items: int, blur: float = 0.0, scaling: float = 0.0, ep
         int(alternating))
 
     rows = (n + m) * items * (4 if self_terms else 2)
+    # potentials for the caller: (side, kind) of every tensor
+    own = () if want_loss else tuple(
+        (side, kind) for side in ((2, 3) if self_terms == 2 else (0, 1, 2, 3) if self_terms else (0, 1))
+        for kind in range(1 + bool(prelast)))
 
     def enqueue(x, y, a, b):
         p = Problem.from_buffer_copy(form)
@@ -168,13 +181,17 @@ def solve(x, y, a, b, *, items: int, blur: float = 0.0, scaling: float = 0.0, ep
         L = _lib.lib()
         ws = torch.empty(L.fs_small_workspace_bytes(ctypes.byref(p)), dtype=torch.uint8,
                          device=x.device)
-        pots = torch.empty(rows, dtype=torch.float32, device=x.device)
-        # (a tensor of its own: a caller may change the loss in place)
-        loss = (torch.empty(x.shape[:-2], dtype=torch.float32, device=x.device) if want_loss
-                else None)
+        # (tensors of their own: a caller may change or keep the loss and every potential)
+        if want_loss:
+            pots = (torch.empty(rows, dtype=torch.float32, device=x.device),)
+            loss = torch.empty(x.shape[:-2], dtype=torch.float32, device=x.device)
+        else:
+            pots = tuple(torch.empty(x.shape[:-2] + (m if side & 1 else n,), dtype=torch.float32,
+                                     device=x.device) for side, _ in own)
+            loss = None
         words = _host_words(items).data_ptr() if sched == 1 or threshold else None
         rc = L.fs_small_solve(ctypes.byref(p), ws.data_ptr(), ws.numel(), words, _lib.ptr(loss),
-                              pots.data_ptr(), _lib.stream_of(x))
+                              pots[0].data_ptr() if want_loss else None, _lib.stream_of(x))
         if rc > 0:
             if rc == 1:
                 raise ValueError("diameter must be > 0.")
@@ -182,7 +199,13 @@ def solve(x, y, a, b, *, items: int, blur: float = 0.0, scaling: float = 0.0, ep
                 raise ValueError("the diameter of the clouds is not a number.")
             raise LongSchedule
         _lib.check(rc, "fs_small_solve")
-        return (ws, pots, loss) if want_loss else (ws, pots)
+        if own:
+            where = (_P * 8)()
+            for (side, kind), t in zip(own, pots):
+                where[2 * side + kind] = t.data_ptr()
+            _lib.check(L.fs_small_potentials(ctypes.byref(p), ws.data_ptr(), ws.numel(), where,
+                                             _lib.stream_of(x)), "fs_small_potentials")
+        return pots + ((loss,) if want_loss else ()) + ((ws,) if want_values else ())
 
     if (sched == 0 and not threshold and _graphs.eligible(n, m, entries, x.device)
             and (d <= WIDE_D or items * n * m <= 1 << 22)):  # (a graph keeps its products)
@@ -190,13 +213,18 @@ def solve(x, y, a, b, *, items: int, blur: float = 0.0, scaling: float = 0.0, ep
         key = ("self pair" if self_terms else "alternating" if alternating else "symmetric",
                int(self_terms), x.device.index, x.dtype, x.shape, y.shape,
                eps, entries, cost_scale, _rho(rho_x), _rho(rho_y), a is None, b is None, normalize,
-               want_values, extrapolate, want_loss)
+               want_values, extrapolate, want_loss, own)
         out = _graphs.run(key, enqueue, [x, y, a, b])
     else:
         out = enqueue(x, y, a, b)
     s = Solved()
     s.form, s.x, s.y, s.a, s.b = form, x, y, a, b
-    s.ws, s.pots, s.loss = out if want_loss else out + (None,)
+    s.ws = out[-1] if want_values else None
+    s.pots, s.loss = out[:2] if want_loss else (None, None)
+    s.own = None
+    if own:
+        got = dict(zip(own, out))
+        s.own = {_SIDES[side]: (got[side, 0], got.get((side, 1))) for side, kind in own if kind == 0}
     s.entries = entries
     if threshold:  # averaged steps of the first problem
         word = int(_host_words(items)[0])

@@ -525,6 +525,20 @@ int fs_small_solve(const fs_small_problem* p, void* workspace, size_t workspace_
   return hipGetLastError() == hipSuccess ? FS_OK : FS_ERR_LAUNCH_FAILED;
 }
 
+int fs_small_potentials(const fs_small_problem* p, void* workspace, size_t workspace_bytes, float* const* pots,
+                        void* stream) {
+  const int rc = checked(p);
+  if (rc != FS_OK) return rc;
+  if (!pots) return FS_ERR_NULL_POINTER;
+  SmallArgs a;
+  if (layout(p, workspace, a) > workspace_bytes || !workspace) return FS_ERR_WORKSPACE_TOO_SMALL;
+  SmallPotArgs t;
+  std::memcpy(t.pots, pots, sizeof(t.pots));
+  const dim3 grid((std::max(a.rows[0], a.rows[1]) + 1023) / 1024, a.self == 1 ? 4 : 2, a.items);
+  hipLaunchKernelGGL((small_potentials_kernel<0>), grid, dim3(1024), 0, (hipStream_t)stream, a, t);
+  return hipGetLastError() == hipSuccess ? FS_OK : FS_ERR_LAUNCH_FAILED;
+}
+
 int fs_small_grad(const fs_small_problem* p, void* workspace, size_t workspace_bytes, const float* grad_out,
                   float* grad_x, float* grad_y, void* stream) {
   const int rc = checked(p);

@@ -662,6 +662,25 @@ __global__ __launch_bounds__(1024) void small_loss_kernel(const SmallArgs a, con
   }
 }
 
+// The standard potentials alone, every side and kind into memory of its own (a program that keeps or
+// changes one of them does not hold or touch the others).  Grid (1024-row pieces, sides, items).
+struct SmallPotArgs {
+  float* pots[4][2];  // [side][of the cost, of the gradient]: [items][rows] or null
+};
+
+template <int T>
+__global__ __launch_bounds__(1024) void small_potentials_kernel(const SmallArgs a, const SmallPotArgs p) {
+  const int side = blockIdx.y + (a.self == 2 ? 2 : 0), item = blockIdx.z, mat = side & 1, rows = a.rows[mat];
+  const int i = blockIdx.x * 1024 + threadIdx.x;
+  if (i >= rows) return;
+  const int last = a.lens[item * 3 + (side < 2 ? 0 : side - 1)] + 1 + a.extrapolate;
+  const size_t half = (size_t)a.items * rows, at = (size_t)item * rows + i;
+  const float al = a.norm[mat][at];
+  if (p.pots[side][0] != nullptr) p.pots[side][0][at] = a.pot[side][(last & 1) * half + at] + al;
+  if (p.pots[side][1] != nullptr)
+    p.pots[side][1][at] = a.pot[side][(a.extrapolate ? (last & 1) ^ 1 : last & 1) * half + at] + al;
+}
+
 template <int T>
 __global__ __launch_bounds__(64) void small_loss_sum_kernel(const SmallLossArgs l, int parts) {
   float t = 0.f;

@@ -130,7 +130,7 @@ def sinkhorn_flashstyle_alternating(
                          want_values=False, extrapolate=False, want_loss=False,
                          threshold=threshold if stops else None, check_every=check_every,
                          alternating=True)
-        f, g = s.potentials("f")[0][0], s.potentials("g")[0][0]
+        f, g = s.potentials("f")[0], s.potentials("g")[0]
         return (f, g, s.entries) if return_n_iters else (f, g)
     xf, yf = x.float().contiguous(), y.float().contiguous()
     alpha = cost_scale * (xf * xf).sum(dim=1)
@@ -421,13 +421,14 @@ def _small_symmetric(x, y, a, b, blur, scaling, use_epsilon_scaling, last_extrap
         s = _small.solve(*_small.points(x, y), _f32c(a.detach()), _f32c(b.detach()), items=1,
                          cost_scale=float(cost_scale), rho_x=rho_x, rho_y=rho_y, normalize=False, self_terms=False, want_values=False,
                          extrapolate=last_extrapolation, want_loss=False, threshold=threshold,
-                         check_every=check_every, **sched)
+                         check_every=check_every, prelast=return_prelast and last_extrapolation,
+                         **sched)
     except _small.LongSchedule:
         return None
     (f, f_pre), (g, g_pre) = s.potentials("f"), s.potentials("g")
-    out = (f[0], g[0])
+    out = (f, g)
     if return_prelast and last_extrapolation:
-        out = out + (f_pre[0], g_pre[0])
+        out = out + (f_pre, g_pre)
     if return_n_iters:
         out = out + (s.entries + 1 + int(bool(last_extrapolation)),)
     return out
@@ -449,14 +450,12 @@ def _small_self_pair(x, a, y, b, blur, scaling, use_epsilon_scaling, last_extrap
         s = _small.solve(*_small.points(x, y), _f32c(a.detach()), _f32c(b.detach()), items=1,
                          cost_scale=float(cost_scale), rho_x=rho, rho_y=rho, normalize=False,
                          self_terms=2, want_values=False, extrapolate=last_extrapolation,
-                         want_loss=False, **sched)
+                         want_loss=False, prelast=return_prelast and last_extrapolation, **sched)
     except _small.LongSchedule:
         return None
-    outs = []
-    for which in ("xx", "yy"):
-        f, f_pre = (t[0] for t in s.potentials(which))
-        outs.append((f, f, f_pre, f_pre) if return_prelast and last_extrapolation else (f, f))
-    return tuple(outs)
+    # (in a self problem both potentials are one)
+    return tuple(tuple(t for t in s.potentials(which) if t is not None for _ in (0, 1))
+                 for which in ("xx", "yy"))
 
 
 def sinkhorn_flashstyle_symmetric_self_pair(

@@ -441,6 +441,15 @@ int fs_small_solve(const fs_small_problem* problem, void* workspace, size_t work
                    int* host_words, float* loss, float* pots, void* stream);
 
 /*
+ * The standard potentials of the solve that left `workspace` behind, each into memory of its own.
+ * pots: a HOST array of 8 device pointers, NULL where not wanted: f, f before the extrapolation
+ * ([items, n]), g, g before it ([items, m]), and with self_terms likewise those of (x, x) and of (y, y)
+ * (what is not part of the problem is not written).
+ */
+int fs_small_potentials(const fs_small_problem* problem, void* workspace, size_t workspace_bytes,
+                        float* const* pots, void* stream);
+
+/*
  * Gradients of `loss` in x and y (NULL: not wanted) times grad_out [items] (device), fp32
  * [items, n, d] and [items, m, d], from the workspace fs_small_solve left behind.
  * Replaces sinkhorn_geomloss_online_grad_sqeuclid

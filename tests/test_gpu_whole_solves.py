@@ -259,6 +259,29 @@ def test_the_loss_may_be_changed_in_place(batched, fixed):
         assert torch.equal(got, 2.0 * want)
 
 
+@pytest.mark.parametrize("d", [4, 200])
+def test_potentials_are_tensors_of_their_own(d):
+    from flash_sinkhorn_amd import SamplesLoss, sinkhorn_solvers as S
+    x, y, a, b = inputs(8, 64, 50, d, scale=1.0 / np.sqrt(d))
+    X, Y, A, B = dev(x, y, a, b)
+    fixed = dict(use_epsilon_scaling=False, eps=0.1, n_iters=10)
+    runs = [lambda: S.sinkhorn_flashstyle_symmetric(X, Y, A, B, return_prelast=True, **fixed),
+            lambda: S.sinkhorn_flashstyle_symmetric(X, Y, A, B, threshold=1e-3, **fixed),
+            lambda: S.sinkhorn_flashstyle_alternating(X, Y, A, B, eps=0.1, n_iters=10),
+            lambda: [p[0] for p in S.sinkhorn_flashstyle_symmetric_self_pair(X, A, Y, B, **fixed)],
+            lambda: SamplesLoss(potentials=True)(X, Y) if d < 129 else SamplesLoss(potentials=True, **fixed)(X, Y),
+            lambda: SamplesLoss(potentials=True, **fixed)(X[None].expand(3, -1, -1), Y[None].expand(3, -1, -1))]
+    for run in runs:
+        for _ in range(3):  # (eager, captured, replayed)
+            out = run()
+            assert len({t.untyped_storage().data_ptr() for t in out}) == len(out)
+            assert all(t.untyped_storage().nbytes() == 4 * t.numel() for t in out)
+            w = torch.ones_like(out[1], requires_grad=True)
+            total = (out[1] * w).sum()
+            out[0].add_(1.0)
+            total.backward()  # (out[1] has not been modified)
+
+
 def test_saved_tensors_pass_through_hooks_and_version_checks():
     from flash_sinkhorn_amd import SamplesLoss
     x, y, a, b = inputs(8, 90, 50, 4)
