@@ -29,6 +29,7 @@ MAX_ROWS = 65536
 WIDE_D = 128  # from here on the products of the clouds are kept (fs_dense.hpp), at most this many:
 MAX_KEPT = 1 << 28
 _TABLE = 511  # entries of a schedule the device keeps
+MAX_GRAPH_BYTES = 32 << 20  # of a batch's workspace, where its run is kept as a graph
 
 
 class Problem(ctypes.Structure):
@@ -173,14 +174,19 @@ def solve(x, y, a, b, *, items: int, blur: float = 0.0, scaling: float = 0.0, ep
         (side, kind) for side in ((2, 3) if self_terms == 2 else (0, 1, 2, 3) if self_terms else (0, 1))
         for kind in range(1 + bool(prelast)))
 
-    def enqueue(x, y, a, b):
+    def problem(x, y, a, b):
         p = Problem.from_buffer_copy(form)
         p.x, p.y, p.a, p.b = x.data_ptr(), y.data_ptr(), _lib.ptr(a), _lib.ptr(b)
         if table is not None:
             p.eps_list = ctypes.addressof(table)
-        L = _lib.lib()
-        ws = torch.empty(L.fs_small_workspace_bytes(ctypes.byref(p)), dtype=torch.uint8,
-                         device=x.device)
+        return p
+
+    L = _lib.lib()
+    nbytes = L.fs_small_workspace_bytes(ctypes.byref(problem(x, y, a, b)))
+
+    def enqueue(x, y, a, b):
+        p = problem(x, y, a, b)
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
         # (tensors of their own: a caller may change or keep the loss and every potential)
         if want_loss:
             pots = (torch.empty(rows, dtype=torch.float32, device=x.device),)
@@ -207,8 +213,11 @@ def solve(x, y, a, b, *, items: int, blur: float = 0.0, scaling: float = 0.0, ep
                                              _lib.stream_of(x)), "fs_small_potentials")
         return pots + ((loss,) if want_loss else ()) + ((ws,) if want_values else ())
 
-    if (sched == 0 and not threshold and _graphs.eligible(n, m, entries, x.device)
-            and (d <= WIDE_D or items * n * m <= 1 << 22)):  # (a graph keeps its products)
+    # (a graph keeps its products; of a batch it counts all items, and the workspace that a replay
+    # may copy)
+    if (sched == 0 and not threshold and _graphs.eligible(items * n, m, entries, x.device)
+            and (d <= WIDE_D or items * n * m <= 1 << 22)
+            and (items == 1 or nbytes <= MAX_GRAPH_BYTES)):
         # a fixed sequence of kernels on fixed shapes: replayed (1.9 instead of 3 us per launch)
         key = ("self pair" if self_terms else "alternating" if alternating else "symmetric",
                int(self_terms), x.device.index, x.dtype, x.shape, y.shape,

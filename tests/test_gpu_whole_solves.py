@@ -242,6 +242,24 @@ def test_a_batch_of_one_and_a_single_problem_keep_graphs_of_their_own():
         assert one.shape == () and batch.shape == (1,) and one.item() == batch.item()
 
 
+def test_graphs_of_batches_are_bounded_by_all_their_items(monkeypatch):
+    from collections import OrderedDict
+    from flash_sinkhorn_amd import SamplesLoss, _graphs
+    monkeypatch.setattr(_graphs, "_cache", OrderedDict())
+    fn = SamplesLoss("sinkhorn", use_epsilon_scaling=False, eps=0.1, n_iters=8)
+    # one item has few logits; the batch has as many as a large problem, or as large a workspace
+    for items, n, kept in ((3, 300, 1), (400, 300, 0), (8192, 16, 0)):
+        _graphs.clear()
+        x = torch.randn(items, n, 3, device="cuda").requires_grad_()
+        want = None
+        for _ in range(3):
+            loss = fn(x, x.detach().flip(0))
+            grad, = torch.autograd.grad(loss.sum(), x)
+            assert want is None or torch.equal(grad, want)
+            want = grad
+        assert len(_graphs._cache) == kept
+
+
 @pytest.mark.parametrize("batched", [False, True])
 @pytest.mark.parametrize("fixed", [False, True])
 def test_the_loss_may_be_changed_in_place(batched, fixed):
