@@ -29,6 +29,9 @@ MAX_ROWS = 65536
 WIDE_D = 128  # from here on the products of the clouds are kept (fs_dense.hpp), at most this many:
 MAX_KEPT = 1 << 28
 _TABLE = 511  # entries of a schedule the device keeps
+# Most workspace of a batch: planes, value operands and vectors of every item, until the backward pass
+# (0.9 MB for a debiased item of 2,048 x 3).  Item by item there is next to nothing to hold.
+MAX_BATCH_BYTES = 16 << 30
 MAX_GRAPH_BYTES = 32 << 20  # of a batch's workspace, where its run is kept as a graph
 
 
@@ -43,8 +46,9 @@ class Problem(ctypes.Structure):
                 ("check_every", _I), ("alternating", _I)]
 
 
-class LongSchedule(Exception):
-    """The schedule has more entries than the device keeps: the general path takes it."""
+class Declined(Exception):
+    """The schedule has more entries than the device keeps, or the workspace of a batch more bytes
+    than are right to hold: the general path takes the call, item by item."""
 
 
 _words = threading.local()
@@ -136,7 +140,10 @@ def held(*values: Optional[float]) -> bool:
     library reads zero and less as "none" (a strict marginal, no early stopping), so a relaxation of
     zero, a negative one or one that rounds to zero would be another problem: the general path
     takes such values, or refuses them."""
-    return all(v is None or 1.1754944e-38 <= v <= 3.4028234e38 for v in values)
+    for v in values:
+        if v is not None and not 1.1754944e-38 <= v <= 3.4028234e38:
+            return False
+    return True
 
 
 def _rho(rho: Optional[float]) -> float:
@@ -159,7 +166,7 @@ def solve(x, y, a, b, *, items: int, blur: float = 0.0, scaling: float = 0.0, ep
     if sched == 2:
         entries = len(eps_list)
         if entries > _TABLE:
-            raise LongSchedule
+            raise Declined
         table = (ctypes.c_float * entries)(*eps_list)
 
     form = Problem(
@@ -174,18 +181,17 @@ def solve(x, y, a, b, *, items: int, blur: float = 0.0, scaling: float = 0.0, ep
         (side, kind) for side in ((2, 3) if self_terms == 2 else (0, 1, 2, 3) if self_terms else (0, 1))
         for kind in range(1 + bool(prelast)))
 
-    def problem(x, y, a, b):
-        p = Problem.from_buffer_copy(form)
-        p.x, p.y, p.a, p.b = x.data_ptr(), y.data_ptr(), _lib.ptr(a), _lib.ptr(b)
-        if table is not None:
-            p.eps_list = ctypes.addressof(table)
-        return p
-
+    p = Problem.from_buffer_copy(form)
+    p.x, p.y = x.data_ptr(), y.data_ptr()
+    if table is not None:
+        p.eps_list = ctypes.addressof(table)
     L = _lib.lib()
-    nbytes = L.fs_small_workspace_bytes(ctypes.byref(problem(x, y, a, b)))
+    nbytes = L.fs_small_workspace_bytes(ctypes.byref(p))
+    if items > 1 and nbytes > MAX_BATCH_BYTES:
+        raise Declined
 
-    def enqueue(x, y, a, b):
-        p = problem(x, y, a, b)
+    def enqueue(x, y, a, b):  # (of these clouds, or of a graph's copies)
+        p.x, p.y, p.a, p.b = x.data_ptr(), y.data_ptr(), _lib.ptr(a), _lib.ptr(b)
         ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
         # (tensors of their own: a caller may change or keep the loss and every potential)
         if want_loss:
@@ -203,7 +209,7 @@ def solve(x, y, a, b, *, items: int, blur: float = 0.0, scaling: float = 0.0, ep
                 raise ValueError("diameter must be > 0.")
             if rc == 2:
                 raise ValueError("the diameter of the clouds is not a number.")
-            raise LongSchedule
+            raise Declined
         _lib.check(rc, "fs_small_solve")
         if own:
             where = (_P * 8)()

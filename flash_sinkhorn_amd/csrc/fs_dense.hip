@@ -80,7 +80,7 @@ void dense_plan(const SmallArgs& a, DenseArgs& t) {
 }
 
 int dense_prepare(const SmallArgs& a, const DenseArgs& t, hipStream_t st) {
-  hipLaunchKernelGGL((dense_stats_kernel<0>), dim3(kSmallStatBlocks, 2, a.items), dim3(1024), 0, st, a);
+  hipLaunchKernelGGL((dense_stats_kernel<0>), dim3(a.stat_blocks, 2, a.items), dim3(1024), 0, st, a);
   hipLaunchKernelGGL((dense_prep_kernel<0>), dim3(std::max(t.blocks[0], t.blocks[1]) + 1, 2, a.items), dim3(512), 0, st,
                      a, t);
   if (hipGetLastError() != hipSuccess) return FS_ERR_LAUNCH_FAILED;

@@ -31,9 +31,10 @@ struct DenseArgs {
   float* out[2];
   const float* l2w[2];
   const float* norm[2];
-  const float4* table;
+  const float4* table;      // [items][3][table_len]
   const int* lens;
   float rho[2];
+  int table_len;
   int step, sched, extrapolate;
   int large;               // the shape of dense_sweep_kernel
 };
@@ -96,7 +97,7 @@ __global__ __launch_bounds__(1024) void dense_stats_kernel(const SmallArgs a) {
   __syncthreads();
   if (tid == 0) {
     for (int w = 1; w < 16; ++w) am = fmaxf(am, sh[0][w]), ws += sh[1][w];
-    float* out = a.stats + (((size_t)item * 2 + mat) * kSmallStatBlocks + blockIdx.x) * kSmallStatWords;
+    float* out = a.stats + (((size_t)item * 2 + mat) * a.stat_blocks + blockIdx.x) * a.stat_words;
     out[0] = am;
     out[1] = ws;
   }
@@ -114,13 +115,8 @@ __global__ __launch_bounds__(512) void dense_prep_kernel(const SmallArgs a, cons
   const int rb = blockIdx.x, rows = a.rows[mat], d = a.d;
   if (rb >= t.blocks[mat]) return;
   const int wave = tid >> 6, lane = tid & 63, li = lane & 31, h = lane >> 5;
-  const float* st = a.stats + ((size_t)item * 2 + mat) * kSmallStatBlocks * kSmallStatWords;
-  float am = st[lane * kSmallStatWords], ws = st[lane * kSmallStatWords + 1];
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    am = fmaxf(am, __shfl_xor(am, o, 64));
-    ws += __shfl_xor(ws, o, 64);
-  }
+  float am, ws;
+  small_merge_stats(a, item, mat, am, ws);
   const float sc = f16_plane_scale(am);
   if (rb == 0 && tid == 0) a.scale[item * 2 + mat] = make_float2(sc, 1.0f / sc);
   const int row = rb * 32 + li;
@@ -292,7 +288,7 @@ __global__ __launch_bounds__(64 * WV, 4) void dense_sweep_kernel(const DenseArgs
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int entries = a.lens[item * 3];
   if (a.step > entries + a.extrapolate) return;
-  const float4 coef = a.table[(size_t)item * 3 * kSmallTable + (a.sched == 0 ? 0 : min(max(a.step - 1, 0), kSmallTable - 1))];
+  const float4 coef = a.table[(size_t)item * 3 * a.table_len + (a.sched == 0 ? 0 : min(max(a.step - 1, 0), a.table_len - 1))];
   const float qs = coef.y, kc = coef.w;
   const int r0 = (group * WV + wave) * RW;
   const float* dots = a.dots + (size_t)item * a.n * a.ld;
@@ -394,7 +390,7 @@ __global__ __launch_bounds__(256) void dense_merge_kernel(const DenseArgs a) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int entries = a.lens[item * 3];
   if (a.step > entries + a.extrapolate) return;
-  const float eps = a.table[(size_t)item * 3 * kSmallTable + (a.sched == 0 ? 0 : min(max(a.step - 1, 0), kSmallTable - 1))].x;
+  const float eps = a.table[(size_t)item * 3 * a.table_len + (a.sched == 0 ? 0 : min(max(a.step - 1, 0), a.table_len - 1))].x;
   const int row = blockIdx.x * 64 + lane, rc = min(row, rows - 1), parts = side ? a.groups : a.chunks;
   const size_t at = (size_t)item * rows + rc;
   const float old = a.pot[side][at], norm = a.norm[side][at];

@@ -44,12 +44,15 @@ size_t layout(const fs_hvp_problem* p, void* ws, HvpPlan& q) {
     s.items = 1;
     s.cost_scale = p->cost_scale;
     s.eps0 = p->eps;
+    s.stat_blocks = kSmallStatBlocks;
+    s.stat_words = 2;
+    s.table_len = 1;
     dense_plan(s, t);
     take(s.lens, 3 * 4);
     take(s.full, 3 * 4);
-    take(s.table, 3 * kSmallTable * sizeof(float4));
+    take(s.table, 3 * (size_t)s.table_len * sizeof(float4));
     take(s.scale, 2 * sizeof(float2));
-    take(s.stats, 2 * kSmallStatBlocks * kSmallStatWords * 4);
+    take(s.stats, 2 * (size_t)s.stat_blocks * s.stat_words * 4);
     for (int i = 0; i < (second ? 2 : 1); ++i) {
       take(t.planes[i], (size_t)t.blocks[i] * t.steps * 2048);
       const size_t rows = s.rows[i];
@@ -134,7 +137,7 @@ size_t layout(const fs_hvp_problem* p, void* ws, HvpPlan& q) {
 
 // (the directions' planes: one matrix, the second operand of its product is y's)
 int prepare(const SmallArgs& s, const DenseArgs& t, int mats, hipStream_t st) {
-  hipLaunchKernelGGL((dense_stats_kernel<0>), dim3(kSmallStatBlocks, mats), dim3(1024), 0, st, s);
+  hipLaunchKernelGGL((dense_stats_kernel<0>), dim3(s.stat_blocks, mats), dim3(1024), 0, st, s);
   const int blocks = mats == 2 ? std::max(t.blocks[0], t.blocks[1]) : t.blocks[0];
   hipLaunchKernelGGL((dense_prep_kernel<0>), dim3(blocks + 1, mats), dim3(512), 0, st, s, t);
   return hipGetLastError() == hipSuccess ? FS_OK : FS_ERR_LAUNCH_FAILED;

@@ -81,12 +81,12 @@ struct PairSide {
 struct PairArgs {
   PairProblem prob[3];
   PairSide side[4];         // 2 problem + (0 stationary, 1 streamed) for xy, then xx, yy
-  const float4* table;      // [items][3][kSmallTable]
+  const float4* table;      // [items][3][table_len]
   const int* lens;          // [items][3]
   float* state;             // [items][3][kPairStateWords]
   const float4* limits;     // [items] smallest and largest base-2 weight of x, of y
   const float4* reach;      // [items] largest |value|, bound of the costs, bound of a potential
-  int step, extrapolate, sched, items, nprob, first_prob, total_items;
+  int step, extrapolate, sched, items, nprob, first_prob, total_items, table_len;
   int merge_groups;         // 256-row groups of the larger cloud: workgroups beyond them write planes
 };
 
@@ -101,8 +101,8 @@ __device__ __forceinline__ float pair_scale(float most, float qs) {
 
 // Which entry of its schedule a step takes.
 __device__ __forceinline__ float4 pair_coef(const PairArgs& a, int item, int prob, int step) {
-  const float4* t = a.table + ((size_t)item * 3 + prob) * kSmallTable;
-  return t[a.sched == 0 ? 0 : min(max(step - 1, 0), kSmallTable - 1)];
+  const float4* t = a.table + ((size_t)item * 3 + prob) * a.table_len;
+  return t[a.sched == 0 ? 0 : min(max(step - 1, 0), a.table_len - 1)];
 }
 
 // Extremes a merge leaves behind, as values whose largest is kept: largest and minus smallest

@@ -24,7 +24,7 @@ struct EpsTable {
 // Schedule given by the caller: every item and problem takes the same entries.
 template <int T>
 __global__ __launch_bounds__(256) void small_table_kernel(const SmallArgs a, const EpsTable t) {
-  float4* out = a.table + (size_t)blockIdx.x * kSmallTable;
+  float4* out = a.table + (size_t)blockIdx.x * a.table_len;
   for (int i = threadIdx.x; i <= a.entries; i += 256) out[i] = small_coef(a.cost_scale, t.e[min(i, a.entries - 1)]);
   if (threadIdx.x == 0) a.lens[blockIdx.x] = a.full[blockIdx.x] = a.entries;
 }
@@ -72,6 +72,18 @@ int checked(const fs_small_problem* p) {
   if (p->threshold > 0.f && p->check_every <= 0) return FS_ERR_BAD_ARGUMENT;
   if (p->alternating && (p->sched != 0 || p->self_terms || p->want_values || p->d > kSmallMaxD)) return FS_ERR_UNSUPPORTED;
   return p->self_terms < 0 || p->self_terms > 2 ? FS_ERR_BAD_ARGUMENT : FS_OK;
+}
+
+// Entries that a schedule of this problem can have (at a fixed eps one stands for all).  By diameter: of
+// clouds whose squared diameter fp32 holds (small_schedule refuses others), one more for what the
+// logarithms round.
+int table_entries(const fs_small_problem* p) {
+  if (p->sched == 0) return 1;
+  if (p->sched == 2) return p->entries;
+  const double most = 3.0 + std::ceil(std::max(0.0, (std::log(1.845e19) - std::log(p->blur)) / -std::log(p->scaling)));
+  int k = (int)std::min<double>(most, kSmallTable - 1);
+  if (p->cut > 0) k = std::min(k, p->cut);
+  return k;
 }
 
 // Work items of a medium problem's launch: 256-row groups of the stationary rows times chunks of the
@@ -132,6 +144,7 @@ void plan_pair(const SmallArgs& a, PairArgs& t) {
 // step to step is set by pair_step_args.
 void bind_pair(const SmallArgs& a, PairArgs& t) {
   t.table = a.table;
+  t.table_len = a.table_len;
   t.lens = a.lens;
   t.limits = a.limits;
   t.reach = a.reach;
@@ -220,8 +233,13 @@ size_t layout(const fs_small_problem* p, void* ws, SmallArgs& a, PairArgs* pa = 
   take(a.lens, items * 3 * 4);
   take(a.full, items * 3 * 4);
   take(a.scale, items * 2 * sizeof(float2));
-  take(a.stats, items * 2 * kSmallStatBlocks * kSmallStatWords * 4);
-  take(a.table, items * 3 * kSmallTable * sizeof(float4));
+  // (what the device leaves per item follows the clouds: 4,096 clouds of 32 points take 70 MB with
+  // it, 700 MB with the largest of both)
+  a.stat_blocks = use_dense(p) ? kSmallStatBlocks : (int)std::min<int64_t>(kSmallStatBlocks, (std::max(p->n, p->m) + 31) / 32);
+  a.stat_words = use_dense(p) ? 2 : 4 + 2 * a.d;
+  a.table_len = table_entries(p) + 1;
+  take(a.stats, items * 2 * (size_t)a.stat_blocks * (size_t)a.stat_words * 4);
+  take(a.table, items * 3 * (size_t)a.table_len * sizeof(float4));
   for (int i = 0; i < 2; ++i) {
     const size_t rows = (size_t)a.rows[i];
     a.blocks[i] = (int)((rows + 31) / 32);
@@ -251,6 +269,7 @@ size_t layout(const fs_small_problem* p, void* ws, SmallArgs& a, PairArgs* pa = 
     take(t.part[0], items * (size_t)t.chunks * (size_t)t.n * sizeof(float2));
     take(t.part[1], items * (size_t)t.groups * (size_t)t.m * sizeof(float2));
     t.table = a.table;
+    t.table_len = a.table_len;
     t.lens = a.lens;
     t.sched = a.sched;
     t.extrapolate = a.extrapolate;
@@ -288,7 +307,7 @@ size_t layout(const fs_small_problem* p, void* ws, SmallArgs& a, PairArgs* pa = 
 template <int DP>
 int launch_prep(const SmallArgs& a, hipStream_t st) {
   const int xb = a.blocks[0] > a.blocks[1] ? a.blocks[0] : a.blocks[1];
-  hipLaunchKernelGGL((small_stats_kernel<0>), dim3(kSmallStatBlocks, 2, a.items), dim3(256), 0, st, a);
+  hipLaunchKernelGGL((small_stats_kernel<0>), dim3(a.stat_blocks, 2, a.items), dim3(256), 0, st, a);
   hipLaunchKernelGGL((small_prep_kernel<DP>), dim3(xb + 1, 2, a.items), dim3(256), 0, st, a);
   return hipGetLastError() == hipSuccess ? FS_OK : FS_ERR_LAUNCH_FAILED;
 }
@@ -299,6 +318,7 @@ SmallStepArgs step_args(const SmallArgs& a, int step) {
   t.scale = reinterpret_cast<const float4*>(a.scale);
   t.step = step;
   t.extrapolate = a.extrapolate;
+  t.coef_stride = 3 * a.table_len;
   const int first = a.self == 2 ? 2 : 0, sides = a.self == 1 ? 4 : 2;
   for (int i = 0; i < sides; ++i) {
     const int side = first + i, qm = side & 1, km = side < 2 ? qm ^ 1 : qm, prob = side < 2 ? 0 : side - 1;
@@ -309,7 +329,7 @@ SmallStepArgs step_args(const SmallArgs& a, int step) {
     s.kpot = a.pot[side < 2 ? side ^ 1 : side] + (step & 1) * nk;
     s.kl2w = a.l2w[km];
     // (the entry past the last repeats it, for the extrapolation)
-    s.coef = a.table + prob * kSmallTable + (a.sched == 0 ? 0 : std::min(std::max(step - 1, 0), kSmallTable - 1));
+    s.coef = a.table + prob * a.table_len + (a.sched == 0 ? 0 : std::min(std::max(step - 1, 0), a.table_len - 1));
     s.lens = a.lens + prob;
     s.old = a.pot[side] + (step & 1) * nq;
     s.out = a.pot[side] + ((step & 1) ^ 1) * nq;

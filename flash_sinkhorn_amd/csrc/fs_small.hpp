@@ -22,10 +22,9 @@
 
 namespace fs {
 
-constexpr int kSmallStatBlocks = 64;            // workgroups per matrix and item of small_stats_kernel
+constexpr int kSmallStatBlocks = 64;            // most workgroups per matrix and item of small_stats_kernel
 constexpr int kSmallMaxD = 128;
-constexpr int kSmallStatWords = 4 + 2 * kSmallMaxD;  // absmax; weights: sum, smallest, largest; column minima, maxima
-constexpr int kSmallTable = 512;                // entries of an eps schedule kept on the device
+constexpr int kSmallTable = 512;                // most entries of an eps schedule kept on the device
 
 // A run of small problems.  Sides: 0 f of the xy problem (rows of x against keys y), 1 g of it
 // (rows of y against keys x), 2 the self problem of x, 3 that of y.  Problems: 0 xy, 1 xx, 2 yy.
@@ -45,7 +44,10 @@ struct SmallArgs {
   double blur, scaling;
   float rho[2];           // <= 0: strict marginal
   // workspace
-  float* stats;           // [items][2][kSmallStatBlocks][kSmallStatWords]
+  // statistics of every matrix by stat_blocks workgroups, stat_words each: absmax; weights: sum, smallest,
+  // largest; column minima, maxima (the first four, or the first two, where no more is needed)
+  int stat_blocks, stat_words;
+  float* stats;           // [items][2][stat_blocks][stat_words]
   float2* scale;          // [items][2] power-of-two scales of the planes, and their inverses
   u32x4* planes[2];       // [items][blocks][2 planes][DP / 16][64]
   u32x4* values[2];       // [items][blocks][DP / 32][2 steps][2 planes][64]
@@ -53,7 +55,8 @@ struct SmallArgs {
   float* wt[2];           // [items][rows] weights as the solve takes them
   float* l2w[2];          // [items][rows] their base-2 logarithms
   float* pot[4];          // [2 parities][items][rows of the side]: shifted potentials
-  float4* table;          // [items][3][kSmallTable] per entry: eps and what the kernels derive from
+  int table_len;          // entries a schedule can have and one more
+  float4* table;          // [items][3][table_len] per entry: eps and what the kernels derive from
                           // it (small_coef); one entry past the last repeats it
   int* full;              // [items][3] entries of the schedules
   int* lens;              // [items][3] those the problem runs: fewer once it has converged
@@ -85,7 +88,7 @@ __device__ __forceinline__ float4 small_coef(float cost_scale, float eps) {
   return make_float4(eps, qs, 1.0f / qs, kLog2e / eps);
 }
 __device__ __forceinline__ const float4* small_table(const SmallArgs& a, int item, int prob) {
-  return a.table + ((size_t)item * 3 + prob) * kSmallTable;
+  return a.table + ((size_t)item * 3 + prob) * a.table_len;
 }
 // The coefficients behind the cost and the gradient: those of the schedule's last entry (which a
 // problem that stopped early keeps).
@@ -101,7 +104,7 @@ template <int T>
 __global__ __launch_bounds__(256) void small_stats_kernel(const SmallArgs a) {
   const int mat = blockIdx.y, item = blockIdx.z, tid = threadIdx.x;
   const int rows = a.rows[mat], d = a.d;
-  const int per = (rows + kSmallStatBlocks - 1) / kSmallStatBlocks;
+  const int per = (rows + a.stat_blocks - 1) / a.stat_blocks;
   const int r0 = min(rows, (int)blockIdx.x * per), r1 = min(rows, r0 + per);
   const int reps = 256 / d, act = reps * d;
   __shared__ float mn[256], mx[256];
@@ -139,10 +142,10 @@ __global__ __launch_bounds__(256) void small_stats_kernel(const SmallArgs a) {
     k = half;
   }
   __syncthreads();
-  float* out = a.stats + (((size_t)item * 2 + mat) * kSmallStatBlocks + blockIdx.x) * kSmallStatWords;
+  float* out = a.stats + (((size_t)item * 2 + mat) * a.stat_blocks + blockIdx.x) * a.stat_words;
   if (tid < d) {
     out[4 + tid] = mn[tid];
-    out[4 + kSmallMaxD + tid] = mx[tid];
+    out[4 + d + tid] = mx[tid];
   }
   __syncthreads();
   // (a NaN does not reach the plane scale: fmaxf drops it, as absmax_kernel does)
@@ -189,7 +192,7 @@ __device__ void small_schedule(const SmallArgs& a, int item) {
   __shared__ int len[3];
   if (a.sched == 0 && tid < 3) {  // one entry stands for all
     a.lens[item * 3 + tid] = a.full[item * 3 + tid] = a.entries;
-    a.table[((size_t)item * 3 + tid) * kSmallTable] = small_coef(a.cost_scale, a.eps0);
+    a.table[((size_t)item * 3 + tid) * a.table_len] = small_coef(a.cost_scale, a.eps0);
   }
   if (a.sched != 1 && !a.pair) return;
   if (tid < 3) sq[tid] = 0.f;
@@ -199,9 +202,9 @@ __device__ void small_schedule(const SmallArgs& a, int item) {
     float lo[2] = {3.0e38f, 3.0e38f}, hi[2] = {-3.0e38f, -3.0e38f};
     for (int mat = 0; mat < 2; ++mat)
 #pragma unroll 16
-      for (int b = 0; b < kSmallStatBlocks; ++b) {
-        const float* st = a.stats + (((size_t)item * 2 + mat) * kSmallStatBlocks + b) * kSmallStatWords;
-        const float l = st[4 + tid], u = st[4 + kSmallMaxD + tid];
+      for (int b = 0; b < 16 * ((a.stat_blocks + 15) / 16); ++b) {  // (sixteen at a time, the last one again)
+        const float* st = a.stats + (((size_t)item * 2 + mat) * a.stat_blocks + min(b, a.stat_blocks - 1)) * a.stat_words;
+        const float l = st[4 + tid], u = st[4 + a.d + tid];
         lo[mat] = (l < lo[mat] || !(l == l)) ? l : lo[mat];
         hi[mat] = (u > hi[mat] || !(u == u)) ? u : hi[mat];
       }
@@ -222,14 +225,14 @@ __device__ void small_schedule(const SmallArgs& a, int item) {
   if (a.pair && tid == 0) {
     float am = 0.f, lim[4];
     for (int mat = 0; mat < 2; ++mat) {
-      const float* st = a.stats + ((size_t)item * 2 + mat) * kSmallStatBlocks * kSmallStatWords;
+      const float* st = a.stats + ((size_t)item * 2 + mat) * a.stat_blocks * a.stat_words;
       float ws = 0.f, wl = 3.0e38f, wh = 0.f;
 #pragma unroll 16
-      for (int b = 0; b < kSmallStatBlocks; ++b) {
-        am = fmaxf(am, st[b * kSmallStatWords]);
-        ws += st[b * kSmallStatWords + 1];
-        wl = fminf(wl, st[b * kSmallStatWords + 2]);
-        wh = fmaxf(wh, st[b * kSmallStatWords + 3]);
+      for (int b = 0; b < a.stat_blocks; ++b) {  // (of a medium problem: all 64)
+        am = fmaxf(am, st[b * a.stat_words]);
+        ws += st[b * a.stat_words + 1];
+        wl = fminf(wl, st[b * a.stat_words + 2]);
+        wh = fmaxf(wh, st[b * a.stat_words + 3]);
       }
       if (a.w[mat] == nullptr) wl = wh = 1.0f / (float)a.rows[mat];
       else if (a.normalize) wl /= fmaxf(ws, 1e-40f), wh /= fmaxf(ws, 1e-40f);
@@ -252,6 +255,7 @@ __device__ void small_schedule(const SmallArgs& a, int item) {
       const double total = 2.0 + (cnt > 0.0 ? cnt : 0.0);
       k = total > (double)(kSmallTable - 1) ? -3 : (int)total;  // -3: longer than the table
       if (k > 0 && a.cut > 0) k = min(k, a.cut);
+      if (k >= a.table_len) k = -3;
     }
     len[tid] = k;
     a.lens[item * 3 + tid] = k;
@@ -272,8 +276,23 @@ __device__ void small_schedule(const SmallArgs& a, int item) {
     for (int i = tid; i <= len[p]; i += 256) {
       const int c = min(i, len[p] - 1);
       const double e = c == 0 ? D * D : (c == full - 1 ? a.blur * a.blur : exp(start + (c - 1) * step));
-      a.table[((size_t)item * 3 + p) * kSmallTable + i] = small_coef(a.cost_scale, (float)e);
+      a.table[((size_t)item * 3 + p) * a.table_len + i] = small_coef(a.cost_scale, (float)e);
     }
+  }
+}
+
+// Largest magnitude of a matrix and the sum of its weights, by every lane of a wavefront.
+__device__ __forceinline__ void small_merge_stats(const SmallArgs& a, int item, int mat, float& am, float& ws) {
+  static_assert(kSmallStatBlocks == 64, "one partial result per lane");
+  const int lane = threadIdx.x & 63;
+  const bool live = lane < a.stat_blocks;
+  const float* st = a.stats + (((size_t)item * 2 + mat) * a.stat_blocks + (live ? lane : 0)) * a.stat_words;
+  am = st[0];
+  ws = live ? st[1] : 0.f;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    am = fmaxf(am, __shfl_xor(am, o, 64));
+    ws += __shfl_xor(ws, o, 64);
   }
 }
 
@@ -291,14 +310,8 @@ __global__ __launch_bounds__(256) void small_prep_kernel(const SmallArgs a) {
   const int rb = blockIdx.x, rows = a.rows[mat], d = a.d;
   if (rb >= a.blocks[mat]) return;
   __shared__ float s[32 * LDW];
-  const float* st = a.stats + ((size_t)item * 2 + mat) * kSmallStatBlocks * kSmallStatWords;
-  static_assert(kSmallStatBlocks == 64, "one partial result per lane");
-  float am = st[(tid & 63) * kSmallStatWords], ws = st[(tid & 63) * kSmallStatWords + 1];
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    am = fmaxf(am, __shfl_xor(am, o, 64));
-    ws += __shfl_xor(ws, o, 64);
-  }
+  float am, ws;
+  small_merge_stats(a, item, mat, am, ws);
   const float sc = f16_plane_scale(am);
   if (rb == 0 && tid == 0) a.scale[item * 2 + mat] = make_float2(sc, 1.0f / sc);
   const int r0 = rb * 32;
@@ -440,7 +453,7 @@ struct SmallStepSide {
   const u32x4* qplanes;
   const float* kpot;   // potentials of the keys
   const float* kl2w;
-  const float4* coef;  // of this step's entry; the items' are 3 * kSmallTable apart
+  const float4* coef;  // of this step's entry; the items' are coef_stride apart
   const int* lens;     // the items' are 3 apart
   const float* old;    // this side's potentials, before ...
   float* out;          // ... and behind the step
@@ -452,7 +465,7 @@ struct SmallStepSide {
 struct SmallStepArgs {
   SmallStepSide side[4];
   const float4* scale;  // [items] scale of x, its inverse, scale of y, its inverse
-  int step, extrapolate;
+  int step, extrapolate, coef_stride;
   int full;             // alternating: full steps, the whole shifted potential is damped
 };
 
@@ -488,7 +501,7 @@ __global__ __launch_bounds__(64 * W) void small_step_kernel(const SmallStepArgs 
       for (int kk = 0; kk < KK; ++kk) q[p][kk] = b[(p * KK + kk) * 64];
   }
   const int entries = sd.lens[item * 3];
-  const float4 coef = sd.coef[(size_t)item * 3 * kSmallTable];
+  const float4 coef = sd.coef[(size_t)item * a.coef_stride];
   const float4 sc = a.scale[item];
   const float lscale = coef.y * (qm ? sc.w : sc.y) * (km ? sc.w : sc.y);
   ks.kc = coef.w;
@@ -599,7 +612,7 @@ __global__ __launch_bounds__(1024) void small_check_kernel(const SmallArgs a, in
       a.lens[item * 3 + prob] = step;
       // (the extrapolation, next, takes the schedule's last eps)
       if (a.sched != 0)
-        a.table[((size_t)item * 3 + prob) * kSmallTable + step] = small_last_coef(a, item, prob);
+        a.table[((size_t)item * 3 + prob) * a.table_len + step] = small_last_coef(a, item, prob);
     }
     __hip_atomic_store(a.host_words + item * 4 + prob, 2 * check + (stop ? 1 : 0), __ATOMIC_RELAXED,
                        __HIP_MEMORY_SCOPE_SYSTEM);

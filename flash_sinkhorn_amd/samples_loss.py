@@ -255,7 +255,7 @@ class SamplesLoss(torch.nn.Module):
                     f, g = _small.potentials(self, *small)
                     return f.view(_view_shape(args, 0)), g.view(_view_shape(args, 1))
                 return _small.loss(self, *small)
-            except _small.LongSchedule:
+            except _small.Declined:
                 pass
         parsed = _process_args(*args, normalize=self.normalize)
         if not parsed.x.is_cuda or not parsed.y.is_cuda:

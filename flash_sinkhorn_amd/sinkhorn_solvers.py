@@ -423,7 +423,7 @@ def _small_symmetric(x, y, a, b, blur, scaling, use_epsilon_scaling, last_extrap
                          extrapolate=last_extrapolation, want_loss=False, threshold=threshold,
                          check_every=check_every, prelast=return_prelast and last_extrapolation,
                          **sched)
-    except _small.LongSchedule:
+    except _small.Declined:
         return None
     (f, f_pre), (g, g_pre) = s.potentials("f"), s.potentials("g")
     out = (f, g)
@@ -451,7 +451,7 @@ def _small_self_pair(x, a, y, b, blur, scaling, use_epsilon_scaling, last_extrap
                          cost_scale=float(cost_scale), rho_x=rho, rho_y=rho, normalize=False,
                          self_terms=2, want_values=False, extrapolate=last_extrapolation,
                          want_loss=False, prelast=return_prelast and last_extrapolation, **sched)
-    except _small.LongSchedule:
+    except _small.Declined:
         return None
     # (in a self problem both potentials are one)
     return tuple(tuple(t for t in s.potentials(which) if t is not None for _ in (0, 1))

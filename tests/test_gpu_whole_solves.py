@@ -242,6 +242,38 @@ def test_a_batch_of_one_and_a_single_problem_keep_graphs_of_their_own():
         assert one.shape == () and batch.shape == (1,) and one.item() == batch.item()
 
 
+def test_batches_beyond_the_workspace_bound_go_item_by_item(monkeypatch):
+    from flash_sinkhorn_amd import SamplesLoss, _small
+    X = torch.randn(4, 70, 3, device="cuda").requires_grad_()
+    Y = torch.rand(4, 60, 3, device="cuda")
+    for kw in (dict(debias=True), dict(use_epsilon_scaling=False, eps=0.1, n_iters=9)):
+        fn, pots = SamplesLoss(**kw), SamplesLoss(potentials=True, **kw)
+        monkeypatch.setattr(_small, "MAX_BATCH_BYTES", 16 << 30)
+        want, (wf, wg) = fn(X, Y), pots(X, Y)
+        wx, = torch.autograd.grad(want.sum(), X)
+        monkeypatch.setattr(_small, "MAX_BATCH_BYTES", 1000)
+        got, (f, g) = fn(X, Y), pots(X, Y)
+        gx, = torch.autograd.grad(got.sum(), X)
+        # (two paths: 1e-5 of the costs, as above)
+        assert (got - want).abs().max() < 1e-4 and rel_err(gx, wx.cpu().numpy()) < 10 * GRAD
+        assert rel_err(f, wf.cpu().numpy()) < 2 * POT and rel_err(g, wg.cpu().numpy()) < 2 * POT
+
+
+# (a schedule's table has the entries the schedule can have, and one more)
+@pytest.mark.parametrize("blur,scaling,cut", [(0.05, 0.9, None), (0.05, 0.9, 1), (0.05, 0.9, 40), (3.0, 0.5, None),
+                                              (10.0, 0.5, None), (1e-4, 0.97, None)])
+@pytest.mark.parametrize("threshold", [None, 1e-2])
+def test_tables_of_long_and_short_schedules(blur, scaling, cut, threshold):
+    from flash_sinkhorn_amd.kernels import sinkhorn_flashstyle_symmetric as solve
+    x, y, a, b = inputs(6, 70, 90, 5, scale=0.5)
+    kw = dict(blur=blur, scaling=scaling, n_iters=cut, threshold=threshold, check_every=3,
+              return_n_iters=True)
+    f, g, used = solve(*dev(x, y, a, b), **kw)
+    wf, wg, wused = oracle.sinkhorn_symmetric(x, y, a, b, **kw)
+    assert used == wused
+    assert rel_err(f, wf) < 2 * POT and rel_err(g, wg) < 2 * POT
+
+
 def test_graphs_of_batches_are_bounded_by_all_their_items(monkeypatch):
     from collections import OrderedDict
     from flash_sinkhorn_amd import SamplesLoss, _graphs

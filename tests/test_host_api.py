@@ -86,6 +86,22 @@ def test_workspace_is_deterministic_and_zero_for_small_problems():
     assert a == L.fs_workspace_bytes(_lib.OP_GRAD, 50000, 50000, 64) and a > 0
 
 
+def test_workspace_of_a_batch_follows_the_size_of_its_items():
+    from flash_sinkhorn_amd import _small
+
+    def per_item(n, m, d, *, items=4096, debias=True, blur=0.05, scaling=0.5, eps=0.0, entries=0):
+        p = _small.Problem(1, 1, None, None, None, n, m, d, items, blur, scaling, 1.0, eps, 0.0, 0.0,
+                           0.0, 0, 0, int(debias), 1, 0 if eps else 1, entries, 0, 1, 10, 0)
+        return _lib.lib().fs_small_workspace_bytes(ctypes.byref(p)) / items
+
+    # operand planes (2 KiB per 32 rows at 16 columns), value operands (4 KiB), a dozen vectors; the
+    # schedules of the three problems: 72 entries of 16 bytes where the blur is 0.05
+    assert per_item(32, 32, 3) < 2 * (2048 + 4096 + 32 * 4 * 12) + 3 * 73 * 16 + 1024
+    assert per_item(32, 32, 3, eps=0.1, entries=100) < 2 * (2048 + 4096 + 32 * 4 * 12) + 1024
+    assert per_item(2048, 2048, 3) < 2 * 64 * (2048 + 4096 + 32 * 4 * 12) + 16384
+    assert per_item(32, 32, 3, blur=1e-3, scaling=0.999) < 48 << 10  # the longest table
+
+
 def test_helpers_match_oracle_closed_forms():
     from flash_sinkhorn_amd.kernels._common import (dampening, epsilon_schedule, log_weights,
                                                      max_diameter)
