@@ -28,6 +28,7 @@ _DTYPES = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}
 MAX_ROWS = 65536
 WIDE_D = 128  # from here on the products of the clouds are kept (fs_dense.hpp), at most this many:
 MAX_KEPT = 1 << 28
+MAX_D = 16384  # rows that the kernels take at all
 _TABLE = 511  # entries of a schedule the device keeps
 # Most workspace of a batch: planes, value operands and vectors of every item, until the backward pass
 # (0.9 MB for a debiased item of 2,048 x 3).  Item by item there is next to nothing to hold.
@@ -119,7 +120,7 @@ def _size_ok(n: int, m: int, d: int, fixed: bool, self_terms: int, stops: bool,
     side: up to 2e7 logits at fixed eps (3,000 x 128: 1.05 against 1.54 ms; 4,500: 2.8 against 2.4),
     6e7 on a schedule (6,500 x 128: 1.54 against 1.94 ms; 9,000: 3.1 against 2.8).
     """
-    if not (0 < n <= MAX_ROWS and 0 < m <= MAX_ROWS and 0 < d):
+    if not (0 < n <= MAX_ROWS and 0 < m <= MAX_ROWS and 0 < d <= MAX_D):
         return False
     if d > WIDE_D:
         return not self_terms and items * n * m <= MAX_KEPT

@@ -12,7 +12,8 @@ namespace {
 int checked(const fs_hvp_problem* p) {
   if (!p || !p->x || !p->y || !p->A || !p->f || !p->g) return FS_ERR_NULL_POINTER;
   if (p->n <= 0 || p->m <= 0 || p->d <= 0) return FS_ERR_BAD_SIZE;
-  if (p->m > FS_HVP_MAX_COLUMNS || p->n > FS_SMALL_MAX_ROWS || p->d > (1 << 20)) return FS_ERR_UNSUPPORTED;
+  if (p->m > FS_HVP_MAX_COLUMNS || p->n > FS_SMALL_MAX_ROWS || p->d > FS_SMALL_MAX_D || p->n * p->m > FS_HVP_MAX_PLAN)
+    return FS_ERR_UNSUPPORTED;
   if (p->dtype < 0 || p->dtype > 2 || !(p->eps > 0.f) || !(p->cost_scale > 0.f) || p->max_iter < 0) return FS_ERR_BAD_ARGUMENT;
   return FS_OK;
 }

@@ -57,7 +57,8 @@ int padded(int64_t d) { return d <= 16 ? 16 : (d <= 32 ? 32 : (d <= 64 ? 64 : 12
 int checked(const fs_small_problem* p) {
   if (!p || !p->x || !p->y) return FS_ERR_NULL_POINTER;
   if (p->n <= 0 || p->m <= 0 || p->d <= 0 || p->items <= 0 || p->items > 65535) return FS_ERR_BAD_SIZE;
-  if (p->n > FS_SMALL_MAX_ROWS || p->m > FS_SMALL_MAX_ROWS) return FS_ERR_UNSUPPORTED;
+  if (p->n > FS_SMALL_MAX_ROWS || p->m > FS_SMALL_MAX_ROWS || p->d > FS_SMALL_MAX_D) return FS_ERR_UNSUPPORTED;
+  if (p->d > kSmallMaxD && p->items * p->n * p->m > FS_SMALL_MAX_PRODUCTS) return FS_ERR_UNSUPPORTED;
   if (p->d > kSmallMaxD && (p->self_terms || p->want_values || p->sched == 1)) return FS_ERR_UNSUPPORTED;
   if (p->dtype < 0 || p->dtype > 2 || p->sched < 0 || p->sched > 2) return FS_ERR_BAD_ARGUMENT;
   if (p->sched != 1 && p->entries <= 0) return FS_ERR_BAD_ARGUMENT;

@@ -97,7 +97,8 @@ def _kept_ok(x, y, f_hat, g_hat, A, allow_tf32: bool) -> bool:
     return (all(t.device == x.device for t in (y, f_hat, g_hat, A))
             and f_hat.shape == (n,) and g_hat.shape == (m,) and A.shape == (n, d)
             and y.shape[1] == d
-            and 0 < n <= 65536 and 0 < m <= _KEPT_MAX_COLUMNS and d > 0 and n * m <= _KEPT_MAX
+            and 0 < n <= 65536 and 0 < m <= _KEPT_MAX_COLUMNS and n * m <= _KEPT_MAX
+            and 0 < d <= _small.MAX_D
             and (allow_tf32 or _lib.STRICT_OPERANDS == "fp16x2")
             and not torch.cuda.is_current_stream_capturing())
 

@@ -384,8 +384,10 @@ int fs_c_transform(const float* x, const float* y, const float* bias, float* min
                    uint32_t flags, void* workspace, size_t workspace_bytes, void* stream);
 
 /*
- * Whole solves of small problems (d <= 128, at most FS_SMALL_MAX_ROWS rows per cloud), the default
- * operand mode: `items` independent problems of one shape (a batch; 1 otherwise), each the balanced
+ * Whole solves of small and medium problems (at most FS_SMALL_MAX_ROWS rows per cloud), the default
+ * operand mode.  d <= 128: every form below.  Wider rows, up to FS_SMALL_MAX_D: the inner products are
+ * formed once and kept in the workspace (items * n * m fp32, at most FS_SMALL_MAX_PRODUCTS of them); no
+ * self problems, no want_values, no schedule by diameter, no alternating form.  `items` independent problems of one shape (a batch; 1 otherwise), each the balanced
  * or unbalanced symmetric problem of x [items, n, d] and y [items, m, d] and, with self_terms,
  * its two self problems (x, x) and (y, y) (self_terms 2: these alone), all advanced by one launch per step.  What a
  * solver needs before the first step (norms, log weights, operand planes, the eps schedule) is
@@ -420,6 +422,8 @@ int fs_c_transform(const float* x, const float* y, const float* bias, float* min
  * three solves of a debiased SamplesLoss (samples_loss.py:494-512) for these sizes.
  */
 #define FS_SMALL_MAX_ROWS 65536
+#define FS_SMALL_MAX_D 16384
+#define FS_SMALL_MAX_PRODUCTS (1 << 28)
 #define FS_SMALL_NO_DIAMETER 1    /* a cloud is a single point */
 #define FS_SMALL_NOT_A_NUMBER 2   /* a coordinate is not finite */
 #define FS_SMALL_LONG_SCHEDULE 3  /* more entries than the device table holds */
@@ -464,11 +468,13 @@ int fs_small_grad(const fs_small_problem* problem, void* workspace, size_t works
  * rho_x, rho_y <= 0: strict marginals; tau2 then regularises the Schur complement (eps * tau2).
  * lambda_indef weighs the indefinite part.  Conjugate gradients without preconditioner, stopped
  * at max(atol, rtol * |r0|).  Keeps two n x m matrices and a pair of planes of one (12 n m bytes of workspace);
- * at most FS_HVP_MAX_COLUMNS rows of y.  host_state: 8 words of PINNED host memory; the call waits
+ * at most FS_SMALL_MAX_ROWS rows of x, FS_HVP_MAX_COLUMNS of y, FS_HVP_MAX_PLAN pairs and
+ * FS_SMALL_MAX_D columns.  host_state: 8 words of PINNED host memory; the call waits
  * for the device.  Afterwards [1] |r0|, [3] |r|, [5] converged, [6] iterations.
  * Replaces hvp_x_sqeuclid_from_potentials (hvp.py:164-623) for these sizes.
  */
 #define FS_HVP_MAX_COLUMNS 8192
+#define FS_HVP_MAX_PLAN (1 << 26)
 typedef struct fs_hvp_problem {
   const void* x;
   const void* y;

@@ -102,6 +102,35 @@ def test_workspace_of_a_batch_follows_the_size_of_its_items():
     assert per_item(32, 32, 3, blur=1e-3, scaling=0.999) < 48 << 10  # the longest table
 
 
+def test_rows_and_products_beyond_the_limits_are_refused_by_whole_solves_too(monkeypatch):
+    from flash_sinkhorn_amd import _small, hvp
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    L, ok = _lib.lib(), lambda n, m, d, items=1: _small._size_ok(n, m, d, True, 0, False, items)
+
+    def solve_bytes(n, m, d, items=1):
+        p = _small.Problem(1, 1, None, None, None, n, m, d, items, 0, 0, 1.0, 0.1, 0.0, 0.0, 0.0, 0, 0, 0,
+                           0, 0, 10, 0, 1, 10, 0)
+        return L.fs_small_workspace_bytes(ctypes.byref(p))
+
+    def hvp_bytes(n, m, d):
+        p = hvp._Problem(1, 1, 1, 1, 1, n, m, d, 0.1, 1.0, 0.0, 0.0, 1e-5, 1.0, 1e-6, 1e-6, 0, 10)
+        return L.fs_hvp_workspace_bytes(ctypes.byref(p))
+
+    def kept(n, m, d):
+        x, y, f, g = (torch.empty(s, device="meta") for s in ((n, d), (m, d), (n,), (m,)))
+        return hvp._kept_ok(x, y, f, g, x, True)
+
+    # the general path takes rows of up to 16,384 columns (fs_workspace_bytes is 0 beyond)
+    assert L.fs_workspace_bytes(_lib.OP_LSE, 64, 64, 16384) > 0 == L.fs_workspace_bytes(_lib.OP_LSE, 64, 64, 16385)
+    for n, m, d, items, fits in ((8, 8, 16384, 1, True), (8, 8, 16385, 1, False), (16384, 16384, 130, 1, True),
+                                 (16384, 16385, 130, 1, False), (4096, 4096, 130, 16, True),
+                                 (4096, 4096, 130, 17, False), (65537, 8, 4, 1, False)):
+        assert ok(n, m, d, items) == fits and (solve_bytes(n, m, d, items) > 0) == fits
+    for n, m, d, fits in ((8, 8, 16384, True), (8, 8, 16385, False), (8192, 8192, 4, True),
+                          (8193, 8192, 4, False), (8, 8193, 4, False)):
+        assert kept(n, m, d) == fits and (hvp_bytes(n, m, d) > 0) == fits
+
+
 def test_helpers_match_oracle_closed_forms():
     from flash_sinkhorn_amd.kernels._common import (dampening, epsilon_schedule, log_weights,
                                                      max_diameter)
