@@ -5,8 +5,9 @@
 #include <atomic>
 #include <cmath>
 #include <cstring>
+#include <memory>
+#include <new>
 #include <type_traits>
-#include <vector>
 
 #include "flash_sinkhorn_hip.h"
 #include "fs_dense.hpp"
@@ -500,11 +501,14 @@ int fs_small_solve(const fs_small_problem* p, void* workspace, size_t workspace_
   }
   const int n_steps = a.alternating ? entries : entries + 1 + a.extrapolate;
   const bool early = a.threshold > 0.f;
-  std::vector<int> length;  // early stopping: entries of every problem's schedule
+  // early stopping: entries of every problem's schedule (no memory for them: an error, not an exception
+  // that would leave a C entry point)
+  const std::unique_ptr<int[]> length(early ? new (std::nothrow) int[3 * (size_t)a.items] : nullptr);
+  if (early && !length) return FS_ERR_LAUNCH_FAILED;
   if (early)
     for (int i = 0; i < a.items; ++i)
       for (int q = 0; q < 4; ++q) {
-        if (q < 3) length.push_back(a.sched == 1 ? host_words[4 * i + q] : entries);
+        if (q < 3) length[3 * (size_t)i + q] = a.sched == 1 ? host_words[4 * i + q] : entries;
         __atomic_store_n(host_words + 4 * i + q, -1, __ATOMIC_RELAXED);
       }
   int checks = 0;
