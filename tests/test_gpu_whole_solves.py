@@ -49,7 +49,7 @@ def test_small_steps(n, m, d):
 @pytest.mark.parametrize("cut", [1, 2, 3, 4, 5, 6, None])
 def test_schedules_of_every_length(n, m, d, cut):
     if n > 1000 and cut not in (1, 5):
-        pytest.skip("the long ones cost the oracle seconds each")
+        pytest.skip("the oracle takes long; test_one_sweep_steps_of_a_full_schedule runs the full length")
     x, y, a, b = inputs(3, n, m, d, scale=0.5)
     for extrapolate in (True, False):
         from flash_sinkhorn_amd.kernels import sinkhorn_flashstyle_symmetric as solve
@@ -67,6 +67,18 @@ def test_one_sweep_steps(n, m, d, eps):
     x, y, a, b = inputs(n + d, n, m, d, scale=0.5)
     a[::7] = 0.0 if eps == 0.01 else a[::7]  # (rows without weight)
     check_symmetric(x, y, a, b, use_epsilon_scaling=False, eps=eps, n_iters=3)
+
+
+# a whole schedule on these kernels (planes written behind every step), as long as it is
+def test_one_sweep_steps_of_a_full_schedule():
+    from flash_sinkhorn_amd.kernels import sinkhorn_flashstyle_symmetric as solve
+    x, y, a, b = inputs(3, 4600, 4400, 36, scale=0.5)
+    kw = dict(blur=0.5, scaling=0.5)
+    want = oracle.sinkhorn_symmetric(x, y, a, b, return_prelast=True, **kw)
+    X = dev(x, y, a, b)
+    got = solve(*X, return_prelast=True, **kw) + solve(*X, last_extrapolation=False, **kw)
+    for g, w in zip(got, want + want[2:]):
+        assert rel_err(g, w) < POT
 
 
 @pytest.mark.parametrize("n,m,d,eps", [(4700, 4650, 7, 0.05), (5100, 4209, 40, 0.01)])
@@ -127,6 +139,21 @@ def test_kept_products(n, m, d, dtype):
     f, g = solve(*dev(x, y, a, b), **kw)
     wf, wg = oracle.sinkhorn_symmetric(x.astype(np.float64), y.astype(np.float64), a, b, **kw)
     assert rel_err(f, wf) < POT and rel_err(g, wg) < POT
+
+
+@pytest.mark.parametrize("threshold", [None, 1e-3])
+def test_kept_products_of_a_batch(threshold):
+    from flash_sinkhorn_amd import SamplesLoss
+    rng = np.random.default_rng(5)
+    # (the second item is spread out further and stops later)
+    x, y = (rng.standard_normal((3, k, 200)).astype(np.float32) * np.float32([[[0.05]], [[0.1]], [[0.07]]])
+            for k in (300, 530))
+    kw = dict(use_epsilon_scaling=False, eps=0.1, n_iters=30)
+    f, g = SamplesLoss(potentials=True, threshold=threshold, inner_iterations=3, **kw)(*dev(x, y))
+    for i in range(3):
+        a, b = (np.full(k, 1.0 / k, np.float32) for k in (300, 530))
+        wf, wg = oracle.sinkhorn_symmetric(x[i], y[i], a, b, threshold=threshold, check_every=3, **kw)
+        assert rel_err(f[i], wf) < POT and rel_err(g[i], wg) < POT
 
 
 # rows that do not start at multiples of 16 bytes take the narrow loads
@@ -202,6 +229,75 @@ def test_loss_and_gradients(n, m, d, debias):
     assert abs(loss.item() - c) < 1e-4 * (abs(c) + (0.5 * d if debias else 0.0))
     for g, w, p in ((gx, wx, px), (gy, wy, py)):
         assert np.abs(g.cpu().numpy() - w).max() < GRAD * np.abs(p).max()
+
+
+# ---- medium problems: both directions of the one-sweep kernels at small eps ----
+def gradient_bound(x, y, eps):
+    """Largest error of a barycentre whose logits are off by delta: every weight by a factor e^(+-delta),
+    so at most 2 delta times the cloud's extent.  delta: inner products of two planes a side (2^-21 of
+    |x| |y|, twice over eps), potentials and norms that fp32 holds (2^-23 of the largest cost, over eps)."""
+    nx, ny = (np.sqrt((t.astype(np.float64) ** 2).sum(1)).max() for t in (x, y))
+    delta = (2.0 ** -21 * 2.0 * nx * ny + 2.0 ** -23 * 2.0 * (nx + ny) ** 2) / eps
+    return 2.0 * delta * (nx + ny)
+
+
+@pytest.mark.parametrize("n,m,d,eps", [(4500, 4470, 64, 0.01), (5003, 4201, 9, 0.003)])
+def test_one_sweep_gradients_at_small_eps(n, m, d, eps):
+    from flash_sinkhorn_amd import SamplesLoss
+    from flash_sinkhorn_amd.kernels import sinkhorn_flashstyle_symmetric as solve
+    x, y, a, b = inputs(n, n, m, d, scale=0.5, y_shift=0.2)
+    X, Y, A, B = dev(x, y, a, b)
+    X.requires_grad_(), Y.requires_grad_()
+    kw = dict(use_epsilon_scaling=False, eps=eps, n_iters=6)
+    gx, gy = torch.autograd.grad(SamplesLoss("sinkhorn", normalize=False, **kw)(A, X, B, Y), [X, Y])
+    # at the potentials of the same solve: what is left is the gradient's own error
+    _, _, fp, gp = solve(X.detach(), Y.detach(), A, B, return_prelast=True, **kw)
+    wx, wy = oracle.grad_barycentric(x, y, a, b, fp.cpu().numpy(), gp.cpu().numpy(), eps)
+    bound = gradient_bound(x, y, eps)
+    for got, want, w in ((gx, wx, a), (gy, wy, b)):
+        off = np.abs(got.cpu().numpy() - want).max(axis=1)
+        assert (off <= 2.0 * w * bound).all()
+
+
+def test_one_sweep_debiased_schedule():
+    from flash_sinkhorn_amd import SamplesLoss
+    x, y, a, b = inputs(7, 3230, 3190, 36, scale=0.5, y_shift=0.5)
+    X, Y, A, B = dev(x, y, a, b)
+    X.requires_grad_(), Y.requires_grad_()
+    kw = dict(blur=0.5, scaling=0.5)
+    loss = SamplesLoss("sinkhorn", debias=True, normalize=False, **kw)(A, X, B, Y)
+    gx, gy = torch.autograd.grad(loss, [X, Y])
+
+    def one(u, v, wu, wv):
+        f, g, fp, gp = oracle.sinkhorn_symmetric(u, v, wu, wv, return_prelast=True, **kw)
+        return (oracle.sinkhorn_cost(wu, wv, f, g, 0.25),) + oracle.grad_barycentric(u, v, wu, wv, fp, gp, 0.25)
+    c, px, py = one(x, y, a, b)
+    cx, g1, g2 = one(x, x, a, a)
+    cy, h1, h2 = one(y, y, b, b)
+    assert abs(loss.item() - (c - 0.5 * (cx + cy))) < 1e-4 * abs(c)
+    for got, w, p in ((gx, px - 0.5 * (g1 + g2), px), (gy, py - 0.5 * (h1 + h2), py)):
+        assert np.abs(got.cpu().numpy() - w).max() < GRAD * np.abs(p).max()
+
+
+@pytest.mark.parametrize("n,m,d,kw", [(4600, 4400, 10, dict(use_epsilon_scaling=False, eps=0.05, n_iters=5)),
+                                      (3230, 3190, 36, dict(blur=0.5, debias=True))])
+def test_one_sweep_batch_equals_its_items(n, m, d, kw):
+    from flash_sinkhorn_amd import SamplesLoss
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    X = 0.5 * torch.randn(2, n, d, device="cuda", generator=gen)
+    X[1] *= 3.0  # (a longer schedule)
+    Y = 0.5 * torch.randn(2, m, d, device="cuda", generator=gen)
+    X.requires_grad_(), Y.requires_grad_()
+    fn = SamplesLoss("sinkhorn", **kw)
+    loss = fn(X, Y)
+    grads = torch.autograd.grad(loss.sum(), [X, Y])
+    for i in range(2):
+        Xi, Yi = (t[i].detach().clone().requires_grad_() for t in (X, Y))
+        li = fn(Xi, Yi)
+        # (items of a batch are cut into other chunks: sums in another order)
+        assert abs(loss[i].item() - li.item()) < 1e-5 * (1.0 + d * 3.0)
+        for g, w in zip(grads, torch.autograd.grad(li, [Xi, Yi])):
+            assert rel_err(g[i], w.cpu().numpy()) < GRAD
 
 
 def test_weights_elsewhere_are_refused():
@@ -379,6 +475,22 @@ def test_kept_hvp(n, m, d, rho):
             assert info.cg_residual <= max(1e-5 * info.cg_initial_residual, 1e-12)
         elif not info.cg_converged and info.cg_initial_residual > 0.0:
             assert info.cg_iters == iters
+
+
+@pytest.mark.parametrize("n,m,d", [(37, 300, 64), (65, 130, 5), (100, 257, 136)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_kept_hvp_of_half_precision_points(n, m, d, dtype):
+    from flash_sinkhorn_amd.hvp import hvp_x_sqeuclid_from_potentials as hvp
+    x, y, a, b = inputs(n + d, n, m, d, scale=1.0 / np.sqrt(d))
+    X, Y = (t.to(dtype) for t in dev(x, y))
+    x, y = (t.float().cpu().numpy() for t in (X, Y))
+    f, g = oracle.sinkhorn_symmetric(x, y, a, b, use_epsilon_scaling=False, eps=0.25, n_iters=20)
+    f, g = (t.astype(np.float32) for t in oracle.geomloss_to_ott_potentials(f, g, a, b, 0.25))
+    A = np.random.default_rng(1).standard_normal((n, d)).astype(np.float32)
+    kw = dict(eps=0.25, cg_rtol=1e-5, cg_atol=1e-12, preconditioner="none")
+    got, _ = hvp(X, Y, *dev(f, g, A), **kw)
+    want, _ = oracle.hvp_x_from_potentials(x, y, f, g, A, **kw)
+    assert rel_err(got, want) < 2e-4  # (as above: the points are exact in two fp16 planes)
 
 
 def test_hvp_refuses_operands_elsewhere_and_of_other_lengths():
