@@ -200,13 +200,22 @@ __device__ void small_schedule(const SmallArgs& a, int item) {
   float r[3] = {0.f, 0.f, 0.f};
   if (tid < a.d) {
     float lo[2] = {3.0e38f, 3.0e38f}, hi[2] = {-3.0e38f, -3.0e38f};
+#pragma unroll
     for (int mat = 0; mat < 2; ++mat)
-#pragma unroll 16
-      for (int b = 0; b < 16 * ((a.stat_blocks + 15) / 16); ++b) {  // (sixteen at a time, the last one again)
-        const float* st = a.stats + (((size_t)item * 2 + mat) * a.stat_blocks + min(b, a.stat_blocks - 1)) * a.stat_words;
-        const float l = st[4 + tid], u = st[4 + a.d + tid];
-        lo[mat] = (l < lo[mat] || !(l == l)) ? l : lo[mat];
-        hi[mat] = (u > hi[mat] || !(u == u)) ? u : hi[mat];
+      for (int b0 = 0; b0 < a.stat_blocks; b0 += 16) {  // (sixteen loads on their way, the last one again)
+        float l[16], u[16];
+#pragma unroll
+        for (int k = 0; k < 16; ++k) {
+          const int b = min(b0 + k, a.stat_blocks - 1);
+          const float* st = a.stats + (((size_t)item * 2 + mat) * a.stat_blocks + b) * a.stat_words + 4 + tid;
+          l[k] = st[0];
+          u[k] = st[a.d];
+        }
+#pragma unroll
+        for (int k = 0; k < 16; ++k) {
+          lo[mat] = (l[k] < lo[mat] || !(l[k] == l[k])) ? l[k] : lo[mat];
+          hi[mat] = (u[k] > hi[mat] || !(u[k] == u[k])) ? u[k] : hi[mat];
+        }
       }
     const float e0 = (lo[0] < lo[1] || !(lo[0] == lo[0]) ? lo[0] : lo[1]);
     const float e1 = (hi[0] > hi[1] || !(hi[0] == hi[0]) ? hi[0] : hi[1]);
@@ -222,27 +231,32 @@ __device__ void small_schedule(const SmallArgs& a, int item) {
     if ((tid & 63) == 0 && tid < 128) atomicAdd(&sq[p], s);
   }
   __syncthreads();
-  if (a.pair && tid == 0) {
+  if (a.pair && tid < 64) {
     float am = 0.f, lim[4];
+#pragma unroll
     for (int mat = 0; mat < 2; ++mat) {
-      const float* st = a.stats + ((size_t)item * 2 + mat) * a.stat_blocks * a.stat_words;
-      float ws = 0.f, wl = 3.0e38f, wh = 0.f;
-#pragma unroll 16
-      for (int b = 0; b < a.stat_blocks; ++b) {  // (of a medium problem: all 64)
-        am = fmaxf(am, st[b * a.stat_words]);
-        ws += st[b * a.stat_words + 1];
-        wl = fminf(wl, st[b * a.stat_words + 2]);
-        wh = fmaxf(wh, st[b * a.stat_words + 3]);
+      const bool live = tid < a.stat_blocks;
+      const float* st = a.stats + (((size_t)item * 2 + mat) * a.stat_blocks + (live ? tid : 0)) * a.stat_words;
+      float m = st[0], ws = live ? st[1] : 0.f, wl = st[2], wh = st[3];
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) {
+        m = fmaxf(m, __shfl_xor(m, o, 64));
+        ws += __shfl_xor(ws, o, 64);
+        wl = fminf(wl, __shfl_xor(wl, o, 64));
+        wh = fmaxf(wh, __shfl_xor(wh, o, 64));
       }
+      am = fmaxf(am, m);
       if (a.w[mat] == nullptr) wl = wh = 1.0f / (float)a.rows[mat];
       else if (a.normalize) wl /= fmaxf(ws, 1e-40f), wh /= fmaxf(ws, 1e-40f);
       lim[2 * mat] = wl > 0.f ? small_log2(wl, 0.f) : -100000.0f * kLog2e;
       lim[2 * mat + 1] = wh > 0.f ? small_log2(wh, 0.f) : -100000.0f * kLog2e;
     }
-    a.limits[item] = make_float4(lim[0], lim[1], lim[2], lim[3]);
-    // (the diagonal of the joint bounding box bounds every distance)
-    const float far = a.cost_scale * sq[0];
-    a.reach[item] = make_float4(am, far, 2.0f * (far + a.cost_scale * (float)a.d * am * am), 0.f);
+    if (tid == 0) {
+      a.limits[item] = make_float4(lim[0], lim[1], lim[2], lim[3]);
+      // (the diagonal of the joint bounding box bounds every distance)
+      const float far = a.cost_scale * sq[0];
+      a.reach[item] = make_float4(am, far, 2.0f * (far + a.cost_scale * (float)a.d * am * am), 0.f);
+    }
   }
   if (a.sched != 1) return;
   if (tid < 3) {
