@@ -14,6 +14,7 @@ from __future__ import annotations
 
 import ctypes
 import threading
+from types import SimpleNamespace
 from typing import Optional
 
 import torch
@@ -465,17 +466,19 @@ class _SmallLoss(torch.autograd.Function):
         s = _solve_for(loss, x, y, a, b, normalize, self_terms=int(loss.debias),
                        want_values=need[0] or need[1], want_loss=True)
         ctx.save_for_backward(x, y, *s.tensors())
-        ctx.form, ctx.config = s.form, loss._make_config()
+        # (the settings as they are now, for a second backward pass)
+        ctx.form, ctx.config = s.form, dict(vars(loss))
         return s.loss
 
     @staticmethod
     def backward(ctx, grad_out):
         x, y, *solved = ctx.saved_tensors
-        s, cfg, need = Solved.restored(ctx.form, solved), ctx.config, ctx.needs_input_grad
+        s, need = Solved.restored(ctx.form, solved), ctx.needs_input_grad
         gx = gy = ga = gb = None
         if need[0] or need[1]:
             if torch.is_grad_enabled():  # create_graph
-                gx, gy = _SmallGrad.apply(x, y, grad_out, s, cfg, need[0], need[1])
+                gx, gy = _SmallGrad.apply(x, y, grad_out, s, SimpleNamespace(**ctx.config),
+                                          need[0], need[1])
             else:
                 gx, gy = _gradients(s, grad_out, need[0], need[1])
         scale = grad_out if x.ndim == 2 else grad_out[:, None]
