@@ -11,9 +11,11 @@
  *    stated otherwise; sizes are element counts
  *  - nothing here allocates or frees device memory; the caller owns inputs,
  *    outputs and the workspace (size from fs_workspace_bytes)
- *  - all work is enqueued on `stream` (a hipStream_t passed as void*) and
- *    returns without synchronising; the library keeps no mutable global state
- *    (fs_symmetric_step_noalloc remembers, per device, the address of its built-in buffer)
+ *  - all work is enqueued on `stream` (a hipStream_t passed as void*) and returns without
+ *    synchronising, but for fs_small_solve with a schedule by diameter or a threshold and for
+ *    fs_hvp, which read pinned words while the device runs; the library keeps no mutable global
+ *    state but the address of fs_symmetric_step_noalloc's built-in buffer per device and a
+ *    counter that tells one fs_small_solve call's words from another's
  *  - return value: FS_OK or a negative FS_ERR_* code (fs_error_string names it)
  *  - flags: FS_FLAG_EXP2 is accepted for interface parity (the kernels always
  *    work in base 2, which is the same function).  Operand precision (everything
@@ -398,7 +400,8 @@ int fs_c_transform(const float* x, const float* y, const float* bias, float* min
  *              and `scaling` (each problem its own, cut to `cut` entries if that is > 0);
  *              2: eps_list, a HOST array of `entries` values
  *   extrapolate  one full step at the last eps behind them; the gradient is taken before it
- *   rho_x, rho_y  <= 0: strict marginals
+ *   rho_x, rho_y  <= 0: strict marginals (a caller for whom zero is an error checks that itself);
+ *              (x, x) takes rho_x on both sides, (y, y) rho_y
  * Steps: one full step at the first entry, one averaged step (weight 1/2) per entry, the
  * extrapolation.  The workspace keeps what fs_small_grad reads (want_values != 0), so it has to
  * live until then.
@@ -409,16 +412,17 @@ int fs_c_transform(const float* x, const float* y, const float* bias, float* min
  *              compares with the initial potentials (sinkhorn_flashstyle_alternating,
  *              sinkhorn_solvers.py:94-287)
  * host_words: sched 1 or a threshold, 4 * items ints of PINNED host memory that the device can
- * write: the number of steps then depends on the clouds, and fs_small_solve waits for it (the one
- * entry point that waits for the device).  It must not be in use by another call.  Afterwards
- * word 4 * i + q holds the entries of problem q's schedule, or, with a threshold, 2 * c + 1 when
- * the problem stopped at check c (behind (c + 1) * check_every averaged steps).
+ * write: the number of steps then depends on the clouds, and fs_small_solve waits for it.  They must
+ * not be in use by another call.  Afterwards word 4 * i + q (q: 0 the xy problem, 1 (x, x), 2 (y, y))
+ * holds the entries of problem q's schedule, or, with a threshold, 2 * c + 1 when the problem
+ * stopped at check c (behind (c + 1) * check_every averaged steps).
  * loss  [items] or NULL: <a, f> + <b, g>, or (rho_x + eps/2) <a, 1 - exp(-f/rho_x)> + ... with both
  * marginals relaxed, minus half of each self problem's cost.
- * pots  or NULL: the standard potentials: f, f before the extrapolation ([items, n] each), g, g
+ * pots  or NULL: the standard potentials, in one buffer (each in memory of its own:
+ * fs_small_potentials): f, f before the extrapolation ([items, n] each), g, g
  * before it ([items, m] each), and with self_terms likewise those of (x, x) and of (y, y).
- * Returns FS_OK, an error, or one of FS_SMALL_* (sched 1: what the diameters did not allow; no
- * step was run).  Replaces sinkhorn_flashstyle_symmetric (sinkhorn_solvers.py:290-707) and the
+ * Returns FS_OK, an error, or one of FS_SMALL_* (sched 1: what the diameters did not allow; there
+ * is no result).  Replaces sinkhorn_flashstyle_symmetric (sinkhorn_solvers.py:290-707) and the
  * three solves of a debiased SamplesLoss (samples_loss.py:494-512) for these sizes.
  */
 #define FS_SMALL_MAX_ROWS 65536
