@@ -269,7 +269,7 @@ def pair_problem(x, y, a, b, allow_tf32: bool, fixed: bool, self_terms: int = 0,
     """Whether clouds and weights (any of which may need a gradient) are ones ``solve`` takes."""
     return (x.is_cuda and y.is_cuda and x.ndim == 2 and y.ndim == 2 and a.ndim == 1 and b.ndim == 1
             and x.shape[1] == y.shape[1]
-            and (0 < x.shape[1] <= WIDE_D if any_size else
+            and (0 < x.shape[1] <= WIDE_D and max(x.shape[0], y.shape[0]) <= MAX_ROWS if any_size else
                  _size_ok(x.shape[0], y.shape[0], x.shape[1], fixed, self_terms, stops)
                  # (a solver called by itself keeps to the tile-skipping kernels where it has them)
                  and (x.shape[1] <= 8 or min(x.shape[0], y.shape[0]) < 24000))

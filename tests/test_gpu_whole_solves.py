@@ -194,6 +194,16 @@ def test_alternating(n, m, d, threshold):
     assert all(rel_err(p, q) < POT for p, q in zip(got, want))
 
 
+# more rows than a whole solve takes, few enough logits for one: the general path
+@pytest.mark.parametrize("n,m", [(65537, 200), (150, 70000)])
+def test_alternating_of_long_and_thin_problems(n, m):
+    from flash_sinkhorn_amd.kernels import sinkhorn_flashstyle_alternating as solve
+    x, y, a, b = inputs(1, n, m, 3, scale=0.5)
+    f, g = solve(*dev(x, y, a, b), eps=0.3, n_iters=3)
+    wf, wg = oracle.sinkhorn_alternating(x, y, a, b, eps=0.3, n_iters=3)
+    assert rel_err(f, wf) < POT and rel_err(g, wg) < POT
+
+
 # ---- the loss, its gradients, and what a training program does with them ----
 def expected(x, y, a, b, debias, eps, n_iters):
     def one(u, v, wu, wv):

@@ -131,6 +131,15 @@ def test_rows_and_products_beyond_the_limits_are_refused_by_whole_solves_too(mon
         assert kept(n, m, d) == fits and (hvp_bytes(n, m, d) > 0) == fits
 
 
+def test_clouds_beyond_the_row_limit_of_whole_solves_stay_on_the_general_path(monkeypatch):
+    from flash_sinkhorn_amd import _small
+    for n, m, fits in ((65536, 500, True), (65537, 500, False), (300, 65537, False), (100_000, 3, False)):
+        x, y, a, b = (on_card(torch.zeros(s)) for s in ((n, 3), (m, 3), (n,), (m,)))
+        assert _small.alternating_problem(x, y, a, b, True) == fits
+        assert _small.solver_problem(x, y, a, b, True, True, False) == fits
+        assert _small.pair_problem(x, y, a, b, True, True, self_terms=2) == fits
+
+
 def test_helpers_match_oracle_closed_forms():
     from flash_sinkhorn_amd.kernels._common import (dampening, epsilon_schedule, log_weights,
                                                      max_diameter)
