@@ -479,6 +479,8 @@ class _SmallLoss(torch.autograd.Function):
         s, need = Solved.restored(ctx.form, solved), ctx.needs_input_grad
         gx = gy = ga = gb = None
         if need[0] or need[1]:
+            if x.dtype not in _DTYPES:  # (as the gradient of the general path)
+                raise ValueError(f"Unsupported dtype for x/y: {x.dtype}")
             if torch.is_grad_enabled():  # create_graph
                 gx, gy = _SmallGrad.apply(x, y, grad_out, s, SimpleNamespace(**ctx.config),
                                           need[0], need[1])

@@ -310,6 +310,17 @@ def test_one_sweep_batch_equals_its_items(n, m, d, kw):
             assert rel_err(g[i], w.cpu().numpy()) < GRAD
 
 
+def test_gradients_of_double_precision_points_are_refused_at_every_size():
+    from flash_sinkhorn_amd import SamplesLoss
+    for n in (60, 30000):
+        X = torch.rand(n, 24, device="cuda", dtype=torch.float64, requires_grad=True)
+        W = torch.full((n,), 1.0 / n, device="cuda", requires_grad=True)
+        fn = SamplesLoss("sinkhorn", blur=0.5, n_iters=1)
+        with pytest.raises(ValueError, match="Unsupported dtype"):
+            torch.autograd.grad(fn(X, X.detach() + 0.1), X)
+        torch.autograd.grad(fn(W, X.detach(), W.detach(), X.detach() + 0.1), W)
+
+
 def test_weights_elsewhere_are_refused():
     from flash_sinkhorn_amd import SamplesLoss
     x, y, a, b = inputs(8, 61, 50, 4)
