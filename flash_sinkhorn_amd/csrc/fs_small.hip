@@ -516,14 +516,17 @@ int fs_small_solve(const fs_small_problem* p, void* workspace, size_t workspace_
         __atomic_store_n(host_words + 4 * i + q, -1, __ATOMIC_RELAXED);
       }
   int checks = 0;
-  bool all_done = false;
-  // waits for what check number c has to say; all_done: no problem has entries left to run
+  bool all_done = false, ahead_of_us = false;
+  // waits for what check number c has to say; all_done: no problem has entries left to run;
+  // ahead_of_us: one of them stopped at a later check, which the device has run as well by now
   auto check_result = [&](int c) {
     return wait_for_words(st, [&]() {
       all_done = true;
+      ahead_of_us = false;
       for (int i = 0; i < a.items; ++i)
         for (int q = p0; q < p1; ++q) {
           const int v = __atomic_load_n(host_words + 4 * i + q, __ATOMIC_ACQUIRE);
+          ahead_of_us = ahead_of_us || (v >= 0 && v > 2 * c + 1);
           if ((v >= 0 && (v & 1)) || length[3 * i + q] < (c + 1) * p->check_every) continue;
           all_done = false;
           if (v < 2 * c) return false;
@@ -531,7 +534,8 @@ int fs_small_solve(const fs_small_problem* p, void* workspace, size_t workspace_
       return true;
     });
   };
-  for (int s = ahead; s < n_steps && rc == FS_OK && !all_done; ++s) {
+  int s = ahead;
+  for (; s < n_steps && rc == FS_OK && !all_done; ++s) {
     rc = run_step(s);
     const int done = a.alternating ? s + 1 : s;  // averaged steps or iterations
     if (rc != FS_OK || !early || done == 0 || done > entries || done % p->check_every != 0) continue;
@@ -541,6 +545,9 @@ int fs_small_solve(const fs_small_problem* p, void* workspace, size_t workspace_
     if (checks > 0) rc = check_result(checks - 1);
     ++checks;
   }
+  // (the extrapolation of a problem that stopped at the newest check is the next step; for the others
+  // it does nothing)
+  if (rc == FS_OK && all_done && ahead_of_us && s < n_steps && !a.alternating) rc = run_step(s);
   if (rc == FS_OK && early && checks > 0 && !all_done) rc = check_result(checks - 1);
   if (rc != FS_OK || (!loss && !pots)) return rc;
   SmallLossArgs l;

@@ -181,6 +181,27 @@ def test_early_stopping(n, m, d):
     assert all(rel_err(p, q) < POT for p, q in zip(got, want))
 
 
+# the host may look at a check only after the device has run the next one as well (here: always, every
+# launch is waited for), and find there that everything has stopped
+def test_early_stopping_seen_early():
+    import os
+    import subprocess
+    import sys
+    code = """
+import sys
+import torch
+from tests import test_gpu_whole_solves as t
+for n, m, d in ((300, 200, 20), (400, 300, 200), (4700, 4500, 8)):
+    t.test_early_stopping(n, m, d)
+for threshold in (None, 1e-3):
+    t.test_alternating(333, 65, 16, threshold)
+t.test_kept_products_of_a_batch(1e-3)
+"""
+    env = dict(os.environ, AMD_SERIALIZE_KERNEL="3", PYTHONPATH=os.getcwd())
+    res = subprocess.run([sys.executable, "-c", code], env=env, capture_output=True, text=True, timeout=100)
+    assert res.returncode == 0, res.stderr[-3000:]
+
+
 @pytest.mark.parametrize("n,m,d", [(1, 5, 2), (333, 65, 16), (200, 1600, 40), (2100, 2000, 128)])
 @pytest.mark.parametrize("threshold", [None, 1e-3])
 def test_alternating(n, m, d, threshold):
