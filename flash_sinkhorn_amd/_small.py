@@ -366,6 +366,9 @@ def loss_problem(loss, args, label_x, label_y):
     lead = x.shape[:-2]
     if lead and not 0 < lead[0] <= 65535:
         return None
+    if not (loss.normalize or loss.potentials) and any(
+            torch.is_tensor(w) and w.dtype is torch.float64 for w in (a, b)):
+        return None  # (such a loss is summed and returned in their type)
     a, norm_a = _weights(a, lead, x.shape[-2], x.device, loss.normalize)
     b, norm_b = _weights(b, lead, y.shape[-2], x.device, loss.normalize)
     if a is False or b is False:

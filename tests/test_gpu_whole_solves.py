@@ -342,6 +342,19 @@ def test_gradients_of_double_precision_points_are_refused_at_every_size():
         torch.autograd.grad(fn(W, X.detach(), W.detach(), X.detach() + 0.1), W)
 
 
+@pytest.mark.parametrize("normalize", [False, True])
+@pytest.mark.parametrize("types", [(torch.float64, torch.float64), (torch.float32, torch.float64),
+                                   (torch.float16, torch.float32)])
+def test_the_loss_keeps_the_type_that_its_weights_give_it(normalize, types):
+    from flash_sinkhorn_amd import SamplesLoss
+    x, y, a, b = inputs(8, 61, 50, 4)
+    X, Y, A, B = dev(x, y, a, b)
+    A, B = A.to(types[0]), B.to(types[1])
+    loss = SamplesLoss("sinkhorn", normalize=normalize)(A, X, B, Y)
+    assert loss.dtype == (torch.float32 if normalize else torch.promote_types(torch.float32,
+                                                                             torch.promote_types(*types)))
+
+
 def test_weights_elsewhere_are_refused():
     from flash_sinkhorn_amd import SamplesLoss
     x, y, a, b = inputs(8, 61, 50, 4)
