@@ -14,7 +14,10 @@ an LRU bound keeps the memory of forgotten shapes from piling up.  Nothing is ca
 caller is itself capturing.  An entry's static tensors are written, replayed into and cloned on
 the caller's stream, so an entry belongs to one (thread, stream) pair: both are part of the key,
 and two threads or streams solving the same shape each capture a graph of their own; the cache
-itself is guarded by a lock.  No counterpart in the reference, whose solver loop launches one
+itself is guarded by a lock.  A capture is in the "thread_local" mode: in the default one any other
+thread's allocation or synchronisation while it lasts breaks it (and the process with it, in the
+destructor of the graph), and threads capture one after the other, since PyTorch captures on one
+stream per process and waits for the device before it begins.  No counterpart in the reference, whose solver loop launches one
 Triton kernel per step (sinkhorn_solvers.py:497-531).
 """
 from __future__ import annotations
@@ -46,6 +49,7 @@ class _Entry:
 
 _cache: "OrderedDict[tuple, _Entry]" = OrderedDict()
 _lock = threading.Lock()
+_capture = threading.Lock()
 
 
 def eligible(n: int, m: int, n_steps: int, device: torch.device) -> bool:
@@ -77,7 +81,7 @@ def run(key: tuple, fn: Callable[..., Tuple[torch.Tensor, ...]],
     if entry.graph is None:
         entry.inputs = [None if t is None else t.clone() for t in inputs]
         graph = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(graph):
+        with _capture, torch.cuda.graph(graph, capture_error_mode="thread_local"):
             entry.outputs = fn(*entry.inputs)
         entry.graph = graph
     else:

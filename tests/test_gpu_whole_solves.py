@@ -443,6 +443,47 @@ def test_graphs_of_batches_are_bounded_by_all_their_items(monkeypatch):
         assert len(_graphs._cache) == kept
 
 
+# every thread has a stream, clouds and graphs of its own; captures meet other threads' allocations and waits
+def test_threads_on_streams_of_their_own():
+    import threading
+    from flash_sinkhorn_amd import SamplesLoss, _graphs
+
+    def passes(x, y):
+        out = []
+        for kw in (dict(debias=True), dict(use_epsilon_scaling=False, eps=0.1, n_iters=20),
+                   dict(use_epsilon_scaling=False, eps=0.3, n_iters=50, threshold=1e-3)):
+            u = x.clone().requires_grad_()
+            loss = SamplesLoss(**kw)(u, y)
+            out += [loss.detach(), torch.autograd.grad(loss, u)[0]]
+        return out
+
+    clouds = [dev(*(a[0] for a in (inputs(k, 100 + 37 * k, 120, 5)[:1], inputs(k + 9, 90 + k, 120, 5)[:1])))
+              for k in range(4)]
+    want = [passes(x, y) for x, y in clouds]  # (eager: the first call with a shape)
+    torch.cuda.synchronize()
+    found, start = [], threading.Barrier(4)
+
+    def run(k):
+        try:
+            stream = torch.cuda.Stream()
+            with torch.cuda.stream(stream):
+                start.wait(30)
+                for _ in range(6):  # (eager, captured, replayed)
+                    got = passes(*clouds[k])
+                    stream.synchronize()
+                    found.extend((k, i) for i, (u, v) in enumerate(zip(got, want[k])) if not torch.equal(u, v))
+        except Exception as e:
+            found.append((k, repr(e)))
+
+    threads = [threading.Thread(target=run, args=(k,)) for k in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(60)
+    assert not found
+    _graphs.clear()
+
+
 @pytest.mark.parametrize("batched", [False, True])
 @pytest.mark.parametrize("fixed", [False, True])
 def test_the_loss_may_be_changed_in_place(batched, fixed):
