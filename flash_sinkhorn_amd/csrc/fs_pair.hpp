@@ -24,6 +24,14 @@
 // they do not guarantee that every sum is exact in fp32, the launch runs the step two-sided with
 // running maxima (pair_item_two_sided): the first steps of a solve at a small fixed eps, empty
 // weights, plans that move fast.  So nothing is ever redone, and a step is these two launches.
+//
+// At small eps a plan is peaked: of the 32 x 32 units of logits all but a few have none within 44 base-2
+// units of any sum (10,000 x 10,000 x 64, N(0, I), eps = 0.01: 84 %, of a self problem 99.4).  Such units
+// end at their coarse products (pair_run_coarse), and where the potentials settle at one eps the units
+// that do not are kept as lists, which the next steps go along without a look at the others
+// (pair_run_list).  Which form a step takes follows from the same words as above (pair_mode).  Launch
+// of the 10,000 x 64 debiased step: 85 us every logit, 43 the coarse form, 27 the lists (of which
+// some 8 are the chain of loads in front of the first unit).
 #pragma once
 
 #include <type_traits>
@@ -35,7 +43,19 @@
 namespace fs {
 
 constexpr int kPairSlots = 8;        // copies of a step's extremes, over which the workgroups spread
-constexpr int kPairStateWords = 3 * kPairSlots * 8;  // three steps' worth, eight extremes each
+// three steps' worth: eight extremes in each slot, then the units that went on, a cache line per slot, then
+// what is known of the lists (pair_mode), a cache line per step
+constexpr int kPairCounts = 3 * kPairSlots * 8;
+constexpr int kPairLists = kPairCounts + 3 * kPairSlots * 32;
+constexpr int kPairTaken = kPairLists + 3 * 32;  // per step and XCD, of the first problem: work items taken
+constexpr int kPairStateWords = kPairTaken + 3 * 8 * 32;
+constexpr int kPairListWords = 4;    // 64-bit words per wavefront of a work item: [row block][half of the sub-tiles]
+constexpr int kPairMostTiles = 64;   // of a chunk
+constexpr float kPairGap = 44.f;     // base-2 distance below every sum at which a logit is left out
+// Share of units that go on up to which the coarse test pays.  The line is flat: 30 steps at a fixed eps with 0.25 /
+// 0.4 / 0.5 / 0.7 here, 12,000 x 9 (share 0.35) 1,512 / 1,250 / 1,260 / 1,351 us, 12 columns 1,240 / 1,380 / 1,385 /
+// 1,531 at eps 0.05, 18 columns there 1,600 / 1,656 / 1,655 / 1,540, 32 at 0.1 - / 1,627 / 1,715 / 1,606.
+constexpr float kPairOn = 0.4f;
 constexpr float kPairFar = -2.4e8f;  // bias of rows past the last one, in base 2 (2^12 times -58594)
 
 // One problem: stationary rows against streamed rows.  Pointers of item 0.
@@ -52,12 +72,27 @@ struct PairProblem {
   int st_blocks, str_blocks;  // 32-row blocks, padding included
   int groups, chunks, chunk;  // 256-row groups of the stationary rows; chunks (of rows) of the others
   int self;                 // a matrix with itself: a group streams only rows at or behind its first
-  int first_item, n_items;  // work items of this problem in the launch
+  float units;              // 32 x 32 units of all its work items
+  unsigned long long* list; // [items][n_items][wavefront][kPairListWords] units to visit
+  int n_items;              // work items of this problem
   // two-sided steps: (maximum, sum) per row and chunk of keys, and their work items (those of the
   // streamed rows' own half-update from two_first on; a self problem has none)
   float2* st_ms;            // [items][chunks][n_st]
   float2* str_ms;           // [items][chunks of n_st][n_str]
   int two_first, two_items;
+};
+
+// How a step is taken (pair_mode): both sides from one sweep, and with which units.
+struct PairMode {
+  int sweep;     // else two-sided with running maxima
+  int list;      // only the units on the lists
+  int coarse;    // units are ended by their coarse products where these allow it
+  int live;
+  float low;     // log2 of every sum is above that
+  float ratio;   // the next step's logits over this one's, where its eps is smaller
+  float drift;   // with a list: what a logit may have risen by since it was made
+  float base;    // ... and what no logit off it reached then
+  float reserve; // how far below this step's line a list made now begins
 };
 
 // One side of a problem in the merge: the rows whose potentials it updates.
@@ -66,8 +101,7 @@ struct PairSide {
   const float* col;         // self problems: the column sums that the groups before took
   const float2* ms;         // two-sided steps: (maximum, sum) per chunk of keys, and row
   int ms_parts;
-  const float* old;
-  float* out;
+  float* pot;               // [2 parities][items][rows] potentials
   const float* norm;
   const float* l2w;
   u32x4* bias;              // written for the next step
@@ -78,6 +112,11 @@ struct PairSide {
   float rho;
 };
 
+// What the two kernels of a step read besides the step's number.  It lies in the workspace: a kernel's
+// arguments are read past the L2 caches, a line at a time where what is needed of them depends on what was
+// read (touching all of their lines first made a launch 3 us longer).  So the only argument beside the
+// step is this address, which the command processor preloads into registers: a settled step of
+// 4,500 x 64 takes 19.9 us in two launches, 21.8 with everything in the arguments.
 struct PairArgs {
   PairProblem prob[3];
   PairSide side[4];         // 2 problem + (0 stationary, 1 streamed) for xy, then xx, yy
@@ -86,9 +125,13 @@ struct PairArgs {
   float* state;             // [items][3][kPairStateWords]
   const float4* limits;     // [items] smallest and largest base-2 weight of x, of y
   const float4* reach;      // [items] largest |value|, bound of the costs, bound of a potential
-  int step, extrapolate, sched, items, nprob, first_prob, total_items, table_len;
+  int extrapolate, sched, items, nprob, first_prob, table_len;
   int merge_groups;         // 256-row groups of the larger cloud: workgroups beyond them write planes
+  int per_xcd;              // work items of an XCD: an eighth of every problem's
+  int4* work;               // [8][per_xcd]: problem + 4 * item of it, or -1; chunk + 65536 * group; first and last streamed row
 };
+
+typedef const __attribute__((address_space(4))) PairArgs* PairArgsPtr;  // (read by scalar loads)
 
 // Largest bias that its three pieces hold, with room to spare.
 constexpr float kPairMostBias = 6.0e7f;
@@ -125,25 +168,54 @@ __device__ __forceinline__ float pair_value(unsigned k) {
 // than 2^-26 of a sum with a million terms.  Before the first step the potentials are minus the norms,
 // so e_ij = -C_ij / eps >= -bound / eps.
 // By every lane of a wavefront with the same result; `set`: which of the three sets to read.
-__device__ __forceinline__ bool pair_mode(const PairArgs& a, int item, int prob, int step) {
-  // (every load is issued before anything is decided)
-  const float4 now = pair_coef(a, item, prob, step), before = pair_coef(a, item, prob, step - 1);
-  const float4 w = a.limits[item], reach = a.reach[item];
-  const unsigned* st = reinterpret_cast<const unsigned*>(a.state) +
-                       ((size_t)item * 3 + prob) * kPairStateWords + ((step + 2) % 3) * kPairSlots * 8;
-  const int lane = threadIdx.x & 63;
-  unsigned v = st[lane];  // [slot][8]
+struct PairKnown {  // what pair_mode decides from: all loaded before anything is waited for
+  float4 now, before, next, w, reach, list;
+  unsigned ext, on;  // lane: [slot][which extreme]; units that went on, of slot lane % 8
+};
+__device__ __forceinline__ PairKnown pair_known(const PairArgs& a, int item, int prob, int step) {
+  PairKnown k;
+  k.now = pair_coef(a, item, prob, step);
+  k.before = pair_coef(a, item, prob, step - 1);
+  k.next = pair_coef(a, item, prob, step + 1);
+  k.w = a.limits[item];
+  k.reach = a.reach[item];
+  const float* st = a.state + ((size_t)item * 3 + prob) * kPairStateWords;
+  k.list = *reinterpret_cast<const float4*>(st + kPairLists + (step % 3) * 32);
+  const unsigned* at = reinterpret_cast<const unsigned*>(st);
+  const int set = (step + 2) % 3;
+  k.ext = at[set * kPairSlots * 8 + (threadIdx.x & 63)];
+  k.on = at[kPairCounts + (set * kPairSlots + (threadIdx.x & 7)) * 32];
+  __builtin_amdgcn_sched_barrier(0);
+  return k;
+}
+__device__ __forceinline__ PairMode pair_mode(const PairKnown& k, float units, int prob, int step) {
+  const float4 now = k.now, before = k.before, next = k.next, w = k.w, reach = k.reach;
   const float4 lim = prob == 0 ? w : (prob == 1 ? make_float4(w.x, w.y, w.x, w.y) : make_float4(w.z, w.w, w.z, w.w));
   bool ok = (pair_scale(reach.x, now.y) == 0.f) & (lim.x > -1000.f) & (lim.z > -1000.f) &
             (now.w * reach.z < kPairMostBias);
-  if (step == 0) return ok & (fminf(lim.x - lim.y, lim.z - lim.w) - reach.y * now.w > -80.f);
+  PairMode mode;
+  mode.ratio = fmaxf(now.x / next.x, 1.f);
+  mode.coarse = mode.list = 0;
+  mode.drift = mode.base = mode.reserve = 0.f;
+  if (step == 0) {
+    mode.low = fminf(lim.x - lim.y, lim.z - lim.w) - reach.y * now.w;
+    mode.sweep = ok & (mode.low > -80.f);
+    return mode;
+  }
   const float rho = before.x / now.x, kappa = now.w;
+  static_assert(kPairSlots == 8, "a wavefront holds them");
+  unsigned v = k.ext, on = k.on;
 #pragma unroll
-  for (int o = 8; o < 64; o <<= 1) v = max(v, (unsigned)__shfl_xor((int)v, o, 64));
-  const float mine = pair_value(v);  // lane % 8: which extreme
+  for (int o = 1; o < 8; o <<= 1) {
+    v = max(v, (unsigned)__shfl_xor((int)v, 8 * o, 64));
+    on += (unsigned)__shfl_xor((int)on, o, 64);
+  }
   float e[8];
 #pragma unroll
-  for (int k = 0; k < 8; ++k) e[k] = __shfl(mine, k, 64);
+  for (int i = 0; i < 8; ++i) e[i] = pair_value((unsigned)__builtin_amdgcn_readlane((int)v, i));
+  // (behind a two-sided step nothing is known: tried)
+  mode.coarse = (float)on < kPairOn * units;
+  mode.low = 3.0e38f;
 #pragma unroll
   for (int s = 0; s < 2; ++s) {
     // this side's sums: weights of its own rows (w) and of the others' (k)
@@ -155,11 +227,22 @@ __device__ __forceinline__ bool pair_mode(const PairArgs& a, int item, int prob,
     const float dn = rho >= 1.f ? rho * lo - (rho - 1.f) * mass : rho * lo + (1.f - rho) * kmin;
     const float U = up + kappa * (dfh + dgh) - kmax, L = dn + kappa * (dfl + dgl) + (wmin - wmax) - kmax;
     ok = ok & (U < 100.f) & (L > -80.f);
+    mode.low = fminf(mode.low, L);
   }
-  return ok;  // (false where anything is not a number)
+  mode.sweep = ok;  // (false where anything is not a number)
+  // Between two steps at one eps a logit rises by no more than the potentials of its two rows do.
+  const float rise = kappa * (e[2] + e[6]);
+  mode.drift = k.list.x + rise;
+  mode.base = k.list.y;
+  mode.list = ok && mode.coarse && k.list.z != 0.f && mode.base + mode.drift <= mode.low - kPairGap;
+  // (changes of the potentials shrink from step to step, to about a half where a plan is peaked)
+  mode.reserve = next.x == now.x ? fminf(16.f + 3.f * fmaxf(rise, 0.f), 256.f) : 0.f;
+  return mode;
 }
 
-__device__ __forceinline__ u32x4 pair_bias(float b) {
+// A row's bias as three pieces, and what its part in the cross products of the planes can add to a
+// logit (pair_cross), in a column that the matrix product multiplies by zero.
+__device__ __forceinline__ u32x4 pair_bias(float b, float cross) {
   const _Float16 s1 = (_Float16)4096.f, s2 = (_Float16)1.f, s3 = (_Float16)0.000244140625f;
   const _Float16 p1 = (_Float16)(b * 0.000244140625f);
   const float r1 = __builtin_fmaf(-4096.f, (float)p1, b);
@@ -169,8 +252,17 @@ __device__ __forceinline__ u32x4 pair_bias(float b) {
   v[0] = pack_f16((float)s1, (float)s2);
   v[1] = pack_f16((float)s3, (float)p1);
   v[2] = pack_f16((float)p2, (float)p3);
-  v[3] = 0u;
+  v[3] = pack_f16(cross, 0.f);
   return v;
+}
+// The two cross products of a logit come to at most 2^-10 |x~_i| |y~_j| (|lo| <= 2^-11 |hi|, x~ the rows as
+// the planes hold them), so to no more than the sum of 2^-11 |x~_i|^2 and 2^-11 |y~_j|^2.  On top of a row's
+// share: what fp32 sums of that size round off, values below fp16's normal range, the rounding to fp16 here.
+__device__ __forceinline__ float pair_cross(float kappa, float norm, float reach) {
+  return 1.004f * (kappa * norm * 0.0009765625f) + kappa * reach * 9.5367431640625e-07f + 0.25f;
+}
+__device__ __forceinline__ float pair_cross_of(const u32x4& bias) {
+  return (float)__builtin_bit_cast(_Float16, (unsigned short)(bias[3] & 0xffffu));
 }
 // The same row as an A operand: (b1 b2)(b3 s1)(s2 s3), nothing in the upper half-wave.
 __device__ __forceinline__ u32x4 pair_bias_a(const u32x4& v, int h) {
@@ -181,6 +273,13 @@ __device__ __forceinline__ u32x4 pair_bias_a(const u32x4& v, int h) {
   r[3] = 0u;
   if (h) r = u32x4{0u, 0u, 0u, 0u};
   return r;
+}
+
+// (Not to be computed with ahead of the path of the kernel that asks: each fills the registers.)
+__device__ __forceinline__ int pair_lane() {
+  int lane = threadIdx.x & 63;
+  asm volatile("" : "+v"(lane));
+  return lane;
 }
 
 // The streamed operand of a work item: tiles of 64 rows (both planes and the biases) in a ring of three
@@ -207,18 +306,18 @@ struct PairStream {
                                         int j_begin) {
     lds = buffers;
     wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    lane = threadIdx.x & 63;
-    gsrc = planes + ((size_t)batch * blocks + j_begin / 32) * (2 * KK * 64) + lane;
-    bsrc = bias + (size_t)batch * blocks * 32 + j_begin + lane;
+    lane = pair_lane();
+    gsrc = planes + ((size_t)batch * blocks + j_begin / 32) * (2 * KK * 64);
+    bsrc = bias + (size_t)batch * blocks * 32 + j_begin;
   }
   __device__ __forceinline__ void stage(int tile, int buf) const {
 #pragma unroll
     for (int c = 0; c < PIECES / 4; ++c)
       __builtin_amdgcn_global_load_lds(
-          (const __attribute__((address_space(1))) void*)(gsrc + (size_t)tile * (PIECES * 64) + (c * 4 + wave) * 64),
+          (const __attribute__((address_space(1))) void*)(gsrc + (size_t)tile * (PIECES * 64) + (c * 4 + wave) * 64 + lane),
           (__attribute__((address_space(3))) void*)(&lds[buf * BUF + (c * 4 + wave) * 64]), 16, 0, 0);
     // (every wavefront moves the bias piece, so that all count the same loads)
-    const auto* src = (const __attribute__((address_space(1))) void*)(bsrc + (size_t)tile * 64);
+    const auto* src = (const __attribute__((address_space(1))) void*)(bsrc + (size_t)tile * 64 + lane);
     auto* dst = (__attribute__((address_space(3))) void*)(&lds[buf * BUF + PIECES * 64]);
     if constexpr (TWO) __builtin_amdgcn_global_load_lds(src, dst, 4, 0, 0);
     else __builtin_amdgcn_global_load_lds(src, dst, 16, 0, 0);
@@ -305,7 +404,7 @@ __device__ __forceinline__ void pair_load_rows(u32x4 (&x)[2][2][KK], const u32x4
 // A work item with running maxima: 256 query rows (B operand: a lane holds one row and 16 keys)
 // against a chunk of keys, as lse2_kernel does it on the same tiles.
 template <int DP>
-__device__ __forceinline__ void pair_item_two_sided(const PairArgs& a, int batch, const PairProblem& pr, int prob, int it,
+__device__ __forceinline__ void pair_item_two_sided(const PairArgs& a, int batch, const PairProblem& pr, int prob, int step, int it,
                                                     u32x4* lds) {
   using S = PairStream<DP, true>;
   constexpr int KK = DP / 16, NM = S::NM;
@@ -314,10 +413,10 @@ __device__ __forceinline__ void pair_item_two_sided(const PairArgs& a, int batch
   const int n_k = side ? pr.n_st : pr.n_str, n_q = side ? pr.n_str : pr.n_st;
   const int groups = (n_q + 255) / 256, chunk = it / groups, group = it % groups;
   const int kblocks = side ? pr.st_blocks : pr.str_blocks, qblocks = side ? pr.str_blocks : pr.st_blocks;
-  const int lane = threadIdx.x & 63, li = lane & 31, h = lane >> 5;
+  const int lane = pair_lane(), li = lane & 31, h = lane >> 5;
   const int j_begin = chunk * pr.chunk, j_end = min(n_k, j_begin + pr.chunk);
   const int ntiles = (j_end - j_begin + 63) / 64;
-  const float4 coef = pair_coef(a, batch, prob, a.step);
+  const float4 coef = pair_coef(a, batch, prob, step);
   // (planes that cannot carry sqrt(qs) carry a power of two instead)
   const float ps = pair_scale(a.reach[batch].x, coef.y);
   const float lscale = ps == 0.f ? 1.0f : coef.y / (ps * ps);
@@ -434,58 +533,480 @@ __device__ __forceinline__ void pair_item_two_sided(const PairArgs& a, int batch
   }
 }
 
-// One step.  Grid (work items of all problems, rounded up to a multiple of 8; items of the batch).
-// A workgroup of four wavefronts owns 256 stationary rows (two blocks of 32 per wavefront, operands
-// in registers) and streams a chunk of the other matrix.  The exponentials of one 32 x 32 unit sit
-// between the MFMAs of the next in program order.
+// What a work item of the one-sweep forms is: 256 stationary rows against a chunk of streamed ones.
+struct PairItem {
+  int prob, index, chunk, group, j_begin, j_end;
+};
+typedef int PairWord __attribute__((ext_vector_type(4)));
+typedef const __attribute__((address_space(4))) PairWord* PairWork;  // (read by scalar loads)
+__device__ __forceinline__ PairItem pair_item(PairWord w) {
+  PairItem t;
+  t.prob = w[0] < 0 ? -1 : w[0] & 3;
+  t.index = w[0] >> 2;
+  t.chunk = w[1] & 65535;
+  t.group = w[1] >> 16;
+  t.j_begin = w[2];
+  t.j_end = w[3];
+  return t;
+}
+
+// The work items, once per solve.  XCD-aware: workgroups are dealt round-robin to the 8 XCDs; XCD x takes
+// the x-th eighth of every problem's items, whose order is chunk by chunk: what runs on an XCD at one
+// time shares a chunk in its L2.
+__device__ void pair_write_work(const PairArgs& a, int at) {
+  if (at >= 8 * a.per_xcd) return;
+  const int xcd = at / a.per_xcd;
+  int i = at - xcd * a.per_xcd, p = a.first_prob;
+  int4 w = make_int4(-1, 0, 0, 0);
+  for (; p < a.nprob; ++p) {
+    const int per = (a.prob[p].n_items + 7) / 8;
+    if (i < per) break;
+    i -= per;
+  }
+  const PairProblem& pr = a.prob[p];
+  const int index = xcd * ((pr.n_items + 7) / 8) + i;
+  if (index < pr.n_items) {
+    int chunk = index / pr.groups, group = index % pr.groups;
+    if (pr.self) {
+      chunk = 0;
+      group = index;
+      for (;;) {
+        const int g = self_groups_of_chunk(chunk, pr.chunk, pr.n_str, pr.groups);
+        if (group < g) break;
+        group -= g;
+        ++chunk;
+      }
+    }
+    w.x = p + 4 * index;
+    w.y = chunk + 65536 * group;
+    w.z = pr.self ? max(chunk * pr.chunk, group * 256) : chunk * pr.chunk;
+    w.w = min(pr.n_str, (chunk + 1) * pr.chunk);
+  }
+  a.work[at] = w;
+}
+
+// The streamed rows' sums on their way from the four wavefronts to memory.
+struct PairCols {
+  unsigned at;  // LDS address of [tile parity][wavefront][half-wave][row]
+  int wave, lane;
+  __device__ __forceinline__ void put(int tile, int js, float v) const {
+    asm volatile("ds_write_b32 %0, %1"
+                 :
+                 : "v"(at + 4 * ((((tile & 1) * 4 + wave) * 2 + (lane >> 5)) * 64 + js * 32 + (lane & 31))), "v"(v)
+                 : "memory");
+  }
+  // a tile's sums over the wavefronts, in a fixed order; `left`: streamed rows from its first to the chunk's end
+  __device__ __forceinline__ void flush(int tile, float* out, int left) const {
+    float c[8];
+#pragma unroll
+    for (int w = 0; w < 8; ++w)
+      asm volatile("ds_read_b32 %0, %1 offset:%2" : "=v"(c[w]) : "v"(at + 4 * ((tile & 1) * 512 + lane)), "n"(w * 256)
+                   : "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(0xC07F);
+    __builtin_amdgcn_sched_barrier(0);
+    float v = c[0] + c[1];
+#pragma unroll
+    for (int w = 1; w < 4; ++w) v += c[2 * w] + c[2 * w + 1];
+    if (lane < left) out[lane] = v;
+  }
+};
+
+// The stationary rows' sums over the lanes of a wavefront.
+__device__ __forceinline__ void pair_put_rows(const PairProblem& pr, int batch, int chunk, int blk0, float (&st)[2][16],
+                                              int lane) {
+  const int li = lane & 31, h = lane >> 5;
+  float* rowp = pr.st_part + ((size_t)batch * pr.chunks + chunk) * pr.n_st;
+#pragma unroll
+  for (int rb = 0; rb < 2; ++rb) {
+    float v = colsum_all(st[rb], li);
+    v += __shfl_xor(v, 16, 64);
+    const int row = (blk0 + rb) * 32 + colsum_key(li & 15, h);
+    if (li < 16 && row < pr.n_st) rowp[row] = v;
+  }
+}
+
+// Work items of steps in which most units (32 x 32 logits) are empty, from index `at` of the workgroup's
+// on, as long as they are such; returns the index of the first that was not taken.
+//
+// A unit's hi * hi products and biases alone (KK + 1 of 3 KK + 1 MFMAs, no exponential) say that every
+// logit of it lies kPairGap base-2 units below every sum of the step (pair_mode's lower bound on them):
+// it ends there unless hi * hi + biases + the bound on the cross products reaches that line.  What
+// is left out is below 2^-28 of any sum even with 65,536 terms.  The products of a sub-tile's two
+// units go to the matrix pipe while the units of the sub-tile before are tested between them in program order;
+// those that go on then add their cross products and take their exponentials, with the streamed
+// operands read again from LDS.  No accumulator and no LDS read on its way crosses the branch.
+//
+// The tiles of all items run through one ring of four buffers, three ahead, across the ends of items:
+// an item of nine tiles spent 5 us on its way to the first product and 10 in its tiles (10,000 x 64).
 template <int DP>
-__global__ __launch_bounds__(256, 2) void pair_sweep_kernel(const PairArgs a) {
+__device__ __forceinline__ int pair_run_coarse(const PairArgs& a, int batch, PairWork work, int at, int stride,
+                                               int count, unsigned which, const PairMode* modes, unsigned* went,
+                                               u32x4* lds, float* lds_col) {
+  using S = PairStream<DP, false>;
+  constexpr int KK = DP / 16;
+  const int lane = pair_lane(), li = lane & 31, h = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  PairCols cols{(unsigned)(size_t)(const __attribute__((address_space(3))) float*)lds_col, wave, lane};
+  S ks;
+  // ---- the tiles to come ----
+  int s_at = at - stride, s_tile = 0, s_left = 0;
+  PairWord ahead = work[at];
+  bool dry = false;
+  auto stage = [&](int buf) {
+    if (s_left == 0 && !dry) {
+      s_at += stride;
+      const PairItem n = pair_item(ahead);
+      dry = s_at >= count || n.prob < 0 || !((which >> n.prob) & 1);
+      s_tile = 0;
+      if (!dry) {
+        const PairProblem& pr = a.prob[n.prob];
+        ks.begin(lds, pr.str_planes, pr.str_bias, pr.str_blocks, batch, n.j_begin);
+        s_left = (n.j_end - n.j_begin + 63) / 64;
+        ahead = work[min(s_at + stride, count - 1)];
+      }
+    }
+    ks.stage(s_tile, buf);  // (behind the last item: a tile again, for nobody)
+    if (!dry) {
+      ++s_tile;
+      --s_left;
+    }
+  };
+  PairItem t = pair_item(ahead);
+  stage(0);
+  stage(1);
+
+  u32x4 xa[2][2][KK], xb[2];
+  float on_at[2];  // a unit goes on (onto the list) where a logit and the streamed row's share of the bound exceed that
+  auto load_rows = [&]() {
+    const PairProblem& pr = a.prob[t.prob];
+    const int blk0 = t.group * 8 + wave * 2;
+#pragma unroll
+    for (int rb = 0; rb < 2; ++rb) xb[rb] = pr.st_bias[((size_t)batch * pr.st_blocks + blk0 + rb) * 32 + li];
+    pair_load_rows(xa, pr.st_planes + ((size_t)batch * pr.st_blocks + blk0) * (2 * KK * 64), lane);
+  };
+  auto derive_rows = [&]() {
+    const float far = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(
+                          __builtin_bit_cast(int, modes[t.prob].low - modes[t.prob].reserve))) - kPairGap;
+#pragma unroll
+    for (int rb = 0; rb < 2; ++rb) {
+      float c = pair_cross_of(xb[rb]);
+#pragma unroll
+      for (int o = 16; o > 0; o >>= 1) c = fmaxf(c, __shfl_xor(c, o, 64));
+      on_at[rb] = far - c;
+      xb[rb] = pair_bias_a(xb[rb], h);
+    }
+  };
+  load_rows();
+
+  u32x4 y[KK], yb;       // high plane and bias of the sub-tile to be multiplied
+  f32x16 acc[2][2];      // [parity of the sub-tile][row block]
+  float bound[2];        // the streamed rows' share of the bound
+  float st[2][16];       // sums of the stationary rows, over the streamed rows this lane sees
+  auto read_key = [&](int k, int buf, int js) {
+    if (k < KK) y[k] = S::read(&lds[buf * S::BUF + (js * (2 * KK) + k) * 64 + lane]);
+    else yb = S::read(&lds[buf * S::BUF + S::PIECES * 64 + js * 32 + li]);
+  };
+  auto wait_reads = [&]() {
+    S::fence();
+    ks.template wait_lds<0>();
+    S::fence();
+  };
+  // products of the sub-tile in y, parity `to`; the maxima of the units of the other parity between
+  // them; y is read anew from (buf, js) behind the last MFMA that uses a piece of it
+  auto step = [&](int to, int buf, int js, bool test, float (&mx)[2]) {
+#pragma unroll
+    for (int k = 0; k <= KK; ++k) {
+#pragma unroll
+      for (int rb = 0; rb < 2; ++rb) {
+        f32x16& c = acc[to][rb];
+        if (k == 0) {
+#pragma unroll
+          for (int r = 0; r < 16; ++r) c[r] = 0.f;
+        }
+        c = k < KK ? small_mfma(xa[rb][0][k < KK ? k : 0], y[k < KK ? k : 0], c) : small_mfma(xb[rb], yb, c);
+        if (k == KK && rb == 1) bound[to] = pair_cross_of(yb);
+        if (rb == 1) read_key(k, buf, js);
+        if (test) {
+          constexpr int N = 2 * (KK + 1);
+          const int i = 2 * k + rb, v0 = i * 32 / N, v1 = (i + 1) * 32 / N;
+#pragma unroll
+          for (int v = v0; v < v1; ++v) {
+            const float l = acc[to ^ 1][v >> 4][v & 15];
+            mx[v >> 4] = (v & 15) == 0 ? l : fmaxf(mx[v >> 4], l);
+          }
+        }
+        S::fence();
+      }
+    }
+  };
+  // the units of parity `of` that go on, of sub-tile js in buffer buf; returns the streamed rows' sums
+  unsigned long long list[2][2];  // [row block][half of the sub-tiles]
+  auto finish = [&](int of, int sub, int buf, const float (&mx)[2]) {
+    float ps0 = 0.f, ps1 = 0.f;
+    const int js = sub & 1;
+    const bool on0 = wave_any(mx[0] + bound[of] > on_at[0]), on1 = wave_any(mx[1] + bound[of] > on_at[1]);
+    if (on0 || on1) {
+      const unsigned long long bit = 1ull << (sub & 63);
+      list[0][0] |= on0 && sub < 64 ? bit : 0ull;
+      list[0][1] |= on0 && sub >= 64 ? bit : 0ull;
+      list[1][0] |= on1 && sub < 64 ? bit : 0ull;
+      list[1][1] |= on1 && sub >= 64 ? bit : 0ull;
+      u32x4 z[2][KK];
+#pragma unroll
+      for (int q = 1; q >= 0; --q)
+#pragma unroll
+        for (int kk = 0; kk < KK; ++kk) z[q][kk] = S::read(&lds[buf * S::BUF + (js * (2 * KK) + q * KK + kk) * 64 + lane]);
+      wait_reads();
+#pragma unroll
+      for (int rb = 0; rb < 2; ++rb) {
+        if (rb ? !on1 : !on0) continue;
+        f32x16 c = acc[of][rb];
+#pragma unroll
+        for (int kk = 0; kk < KK; ++kk) c = small_mfma(xa[rb][0][kk], z[1][kk], c);
+#pragma unroll
+        for (int kk = 0; kk < KK; ++kk) c = small_mfma(xa[rb][1][kk], z[0][kk], c);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const float e = fast_exp2(c[r]);
+          st[rb][r] += e;
+          if (r & 1) ps1 += e; else ps0 += e;
+        }
+      }
+    }
+    return ps0 + ps1;
+  };
+
+  S::fence();
+  S::wait_tile();  // (the first tile; the second may be on its way)
+  S::fence();
+  S::barrier();
+  stage(2);
+  float* out = nullptr;  // where the sums of the tile before go
+  int left = 0;
+  for (int g = 0;;) {
+    const PairProblem& pr = a.prob[t.prob];
+    const int blk0 = t.group * 8 + wave * 2;
+    derive_rows();
+#pragma unroll
+    for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) st[rb][r] = 0.f;
+    list[0][0] = list[0][1] = list[1][0] = list[1][1] = 0ull;
+    float mx[2];
+#pragma unroll
+    for (int k = 0; k <= KK; ++k) read_key(k, g & 3, 0);
+    wait_reads();
+    step(0, g & 3, 1, false, mx);
+    wait_reads();
+    const PairWord following = work[min(at + stride, count - 1)];
+    float* colp = pr.str_part + ((size_t)batch * pr.groups + t.group) * pr.n_str + t.j_begin;
+    int sub = 0;
+    for (int n = t.j_end - t.j_begin; n > 0; n -= 64, ++g, sub += 2) {
+      const int cur = g & 3, nxt = (g + 1) & 3;
+      // tile g + 1 has landed, and every wavefront is through with tile g - 1 and its sums
+      S::fence();
+      S::wait_tile();
+      S::fence();
+      S::barrier();
+      stage((g + 3) & 3);
+      if (left > 0 && wave == (g & 3)) cols.flush(g - 1, out, left);
+      out = colp;
+      left = n;
+      colp += 64;
+      S::fence();
+      step(1, nxt, 0, true, mx);
+      wait_reads();
+      cols.put(g, 0, finish(0, sub, cur, mx));
+      S::fence();
+      step(0, nxt, 1, true, mx);
+      wait_reads();
+      cols.put(g, 1, finish(1, sub + 1, cur, mx));
+    }
+    {
+      const unsigned went_on = __popcll(list[0][0]) + __popcll(list[0][1]) + __popcll(list[1][0]) + __popcll(list[1][1]);
+      if (lane == 0 && went_on) atomicAdd(&went[t.prob], went_on);
+      unsigned long long* put = pr.list + (((size_t)batch * pr.n_items + t.index) * 4 + wave) * kPairListWords;
+      if (lane < kPairListWords) put[lane] = lane < 2 ? (lane ? list[0][1] : list[0][0]) : (lane == 3 ? list[1][1] : list[1][0]);
+    }
+    // (the next item's rows are on their way while the sums of these cross the lanes)
+    const PairItem done = t;
+    at += stride;
+    t = pair_item(following);
+    const bool more = at < count && t.prob >= 0 && ((which >> t.prob) & 1);
+    if (more) load_rows();
+    S::fence();
+    pair_put_rows(pr, batch, done.chunk, blk0, st, lane);
+    if (!more) {
+      S::wait_all();
+      __syncthreads();
+      if (wave == 0) cols.flush(g - 1, out, left);
+      return at;
+    }
+  }
+}
+
+// Work items of steps whose lists hold, from index `at` of the workgroup's on, as long as they are such:
+// only the units on the lists are visited, without a test.  A wavefront goes along its own list with the
+// streamed operands straight from global memory, one sub-tile ahead, and with no barrier but those
+// around the streamed rows' sums, which lie in LDS per wavefront until the item is done.
+template <int DP>
+__device__ __forceinline__ int pair_run_list(const PairArgs& a, int batch, PairWork work, int at, int stride,
+                                             int count, unsigned which, float* cols) {
+  constexpr int KK = DP / 16;
+  typedef unsigned long long u64;
+  struct Keys {
+    u32x4 p[2][KK], b;
+  };
+  const int lane = pair_lane(), li = lane & 31, h = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  auto words_of = [&](const PairItem& t) {
+    const PairProblem& pr = a.prob[t.prob];
+    return pr.list + (((size_t)batch * pr.n_items + t.index) * 4 + wave) * kPairListWords;
+  };
+  auto uniform = [](u64 v) {
+    return (u64)(unsigned)__builtin_amdgcn_readfirstlane((unsigned)v) |
+           (u64)(unsigned)__builtin_amdgcn_readfirstlane((unsigned)(v >> 32)) << 32;
+  };
+  PairItem t = pair_item(work[at]);
+  PairWord ahead = work[min(at + stride, count - 1)];
+  u64 w[kPairListWords];
+#pragma unroll
+  for (int k = 0; k < kPairListWords; ++k) w[k] = words_of(t)[k];
+  // (what lies there may be the other forms' tiles; each item leaves zeros again)
+  for (int i = threadIdx.x; i < 4 * a.prob[t.prob].chunk; i += 256) cols[i] = 0.f;
+  __syncthreads();
+  for (;;) {
+    const PairProblem& pr = a.prob[t.prob];
+    const PairItem now = t;
+    const int chunk = pr.chunk, blk0 = now.group * 8 + wave * 2, rows = now.j_end - now.j_begin;
+    const u64 on00 = uniform(w[0]), on01 = uniform(w[1]), on10 = uniform(w[2]), on11 = uniform(w[3]);
+    u64 left0 = on00 | on10, left1 = on01 | on11;
+    at += stride;
+    t = pair_item(ahead);
+    const bool more = at < count && t.prob >= 0 && ((which >> t.prob) & 1);
+    if (more) {
+      ahead = work[min(at + stride, count - 1)];
+#pragma unroll
+      for (int k = 0; k < kPairListWords; ++k) w[k] = words_of(t)[k];
+    }
+    float st[2][16];
+#pragma unroll
+    for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) st[rb][r] = 0.f;
+    if (left0 | left1) {
+      u32x4 xa[2][2][KK], xb[2];
+#pragma unroll
+      for (int rb = 0; rb < 2; ++rb)
+        xb[rb] = pair_bias_a(pr.st_bias[((size_t)batch * pr.st_blocks + blk0 + rb) * 32 + li], h);
+      pair_load_rows(xa, pr.st_planes + ((size_t)batch * pr.st_blocks + blk0) * (2 * KK * 64), lane);
+      const u32x4* planes = pr.str_planes + ((size_t)batch * pr.str_blocks + now.j_begin / 32) * (2 * KK * 64);
+      const u32x4* bias = pr.str_bias + (size_t)batch * pr.str_blocks * 32 + now.j_begin;
+      auto take = [&]() {  // the next sub-tile of the list, -1 behind the last
+        int sub = -1;
+        if (left0) {
+          sub = __builtin_ctzll(left0);
+          left0 &= left0 - 1;
+        } else if (left1) {
+          sub = 64 + __builtin_ctzll(left1);
+          left1 &= left1 - 1;
+        }
+        return sub;
+      };
+      auto load = [&](Keys& k, int sub) {
+        const u32x4* src = planes + (size_t)max(sub, 0) * (2 * KK * 64) + lane;
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+#pragma unroll
+          for (int kk = 0; kk < KK; ++kk) k.p[q][kk] = src[(q * KK + kk) * 64];
+        k.b = bias[max(sub, 0) * 32 + li];
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      auto run = [&](const Keys& k, int sub) {
+        const u64 bit = 1ull << (sub & 63);
+        float ps0 = 0.f, ps1 = 0.f;
+#pragma unroll
+        for (int rb = 0; rb < 2; ++rb) {
+          if (!((sub < 64 ? (rb ? on10 : on00) : (rb ? on11 : on01)) & bit)) continue;
+          f32x16 c;
+#pragma unroll
+          for (int r = 0; r < 16; ++r) c[r] = 0.f;
+#pragma unroll
+          for (int kk = 0; kk < KK; ++kk) c = small_mfma(xa[rb][0][kk], k.p[0][kk], c);
+          c = small_mfma(xb[rb], k.b, c);
+#pragma unroll
+          for (int kk = 0; kk < KK; ++kk) c = small_mfma(xa[rb][0][kk], k.p[1][kk], c);
+#pragma unroll
+          for (int kk = 0; kk < KK; ++kk) c = small_mfma(xa[rb][1][kk], k.p[0][kk], c);
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            const float e = fast_exp2(c[r]);
+            st[rb][r] += e;
+            if (r & 1) ps1 += e; else ps0 += e;
+          }
+        }
+        float ps = ps0 + ps1;
+        ps += xor32(ps);
+        if (h == 0) cols[wave * chunk + sub * 32 + li] = ps;
+      };
+      Keys k0, k1;
+      int s0 = take();
+      load(k0, s0);
+      for (;;) {
+        const int s1 = take();
+        load(k1, s1);
+        run(k0, s0);
+        if (s1 < 0) break;
+        s0 = take();
+        load(k0, s0);
+        run(k1, s1);
+        if (s0 < 0) break;
+      }
+    }
+    __syncthreads();
+    float* out = pr.str_part + ((size_t)batch * pr.groups + now.group) * pr.n_str + now.j_begin;
+    for (int j = threadIdx.x; j < rows; j += 256) {
+      float v = cols[j];
+      cols[j] = 0.f;
+#pragma unroll
+      for (int k = 1; k < 4; ++k) {
+        v += cols[k * chunk + j];
+        cols[k * chunk + j] = 0.f;
+      }
+      out[j] = v;
+    }
+    pair_put_rows(pr, batch, now.chunk, blk0, st, lane);
+    __syncthreads();
+    if (!more) return at;
+  }
+}
+
+// A work item of a step that takes both sides from one sweep, every logit of it: the exponentials
+// of one 32 x 32 unit sit between the MFMAs of the next in program order.
+template <int DP>
+__device__ __forceinline__ void pair_item_plain(const PairProblem& pr, int batch, const PairItem& it, const PairMode& mode,
+                                                unsigned* went, u32x4* lds, float* lds_col) {
   using S = PairStream<DP, false>;
   constexpr int KK = DP / 16, NM = S::NM;
-  __shared__ __attribute__((aligned(16))) u32x4 lds[3 * S::BUF];
-  __shared__ float lds_col[2][4][2][64];        // [tile parity][wavefront][half-wave][row]
-
-  const int batch = blockIdx.y;
-  // XCD-aware: workgroups are dealt round-robin to the 8 XCDs; XCD x takes the x-th eighth of the
-  // items, whose order is chunk by chunk: what runs on an XCD at one time shares a chunk in its L2
-  const int per = (a.total_items + 7) / 8;
-  int item = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
-  if ((int)(blockIdx.x >> 3) >= per || item >= a.total_items) return;
-  int p = a.first_prob;
-  while (p + 1 < a.nprob && item >= a.prob[p + 1].first_item) ++p;
-  const PairProblem& pr = a.prob[p];
-  if (a.step > a.lens[batch * 3 + p] + a.extrapolate) return;  // its schedule is shorter
-  item -= pr.first_item;
-  if (!pair_mode(a, batch, p, a.step)) {
-    for (int it = item; it < pr.two_items; it += pr.n_items) pair_item_two_sided<DP>(a, batch, pr, p, it, lds);
-    return;
-  }
-  int chunk = 0, group = item;
-  if (pr.self) {
-    for (;;) {
-      const int g = self_groups_of_chunk(chunk, pr.chunk, pr.n_str, pr.groups);
-      if (group < g) break;
-      group -= g;
-      ++chunk;
-    }
-  } else {
-    chunk = item / pr.groups;
-    group = item % pr.groups;
-  }
-  const int lane = threadIdx.x & 63, li = lane & 31, h = lane >> 5;
-  const int j_begin = pr.self ? max(chunk * pr.chunk, group * 256) : chunk * pr.chunk;
-  const int j_end = min(pr.n_str, (chunk + 1) * pr.chunk);
-  const int ntiles = (j_end - j_begin + 63) / 64;
+  const int lane = pair_lane(), li = lane & 31, h = lane >> 5;
+  const int j_begin = it.j_begin, j_end = it.j_end, ntiles = (j_end - j_begin + 63) / 64;
   S ks;
   ks.begin(lds, pr.str_planes, pr.str_bias, pr.str_blocks, batch, j_begin);
   const int wave = ks.wave;
+  const PairCols cols{(unsigned)(size_t)(const __attribute__((address_space(3))) float*)lds_col, wave, lane};
 
   // ---- stationary operands ----
-  const int blk0 = group * 8 + wave * 2;
+  const int blk0 = it.group * 8 + wave * 2;
   u32x4 xa[2][2][KK], xb[2];
   pair_load_rows(xa, pr.st_planes + ((size_t)batch * pr.st_blocks + blk0) * (2 * KK * 64), lane);
+  float cross = 0.f;
 #pragma unroll
-  for (int rb = 0; rb < 2; ++rb) xb[rb] = pair_bias_a(pr.st_bias[((size_t)batch * pr.st_blocks + blk0 + rb) * 32 + li], h);
+  for (int rb = 0; rb < 2; ++rb) {
+    const u32x4 v = pr.st_bias[((size_t)batch * pr.st_blocks + blk0 + rb) * 32 + li];
+    xb[rb] = pair_bias_a(v, h);
+    cross = pair_cross_of(v);
+  }
   // MFMA k of a unit: the cross products, hi * hi, the biases
   auto mfma_k = [&](int k, const f32x16& acc, const typename S::Keys& y, int rb) {
     if (k == 3 * KK) return small_mfma(xb[rb], y.b, acc);
@@ -498,27 +1019,8 @@ __global__ __launch_bounds__(256, 2) void pair_sweep_kernel(const PairArgs a) {
   for (int rb = 0; rb < 2; ++rb)
 #pragma unroll
     for (int r = 0; r < 16; ++r) st[rb][r] = 0.f;
-  const unsigned col_at = (unsigned)(size_t)(const __attribute__((address_space(3))) float*)&lds_col[0][0][0][0];
-  auto put_sum = [&](int tile, int js, float v) {
-    asm volatile("ds_write_b32 %0, %1" : : "v"(col_at + 4 * ((((tile & 1) * 4 + wave) * 2 + h) * 64 + js * 32 + li)), "v"(v)
-                 : "memory");
-  };
-  float* colp = pr.str_part + ((size_t)batch * pr.groups + group) * pr.n_str;
-  auto flush = [&](int tile) {  // a tile's sums over the four wavefronts, in a fixed order
-    float c[8];
-#pragma unroll
-    for (int w = 0; w < 8; ++w)
-      asm volatile("ds_read_b32 %0, %1 offset:%2" : "=v"(c[w]) : "v"(col_at + 4 * ((tile & 1) * 512 + lane)), "n"(w * 256)
-                   : "memory");
-    S::fence();
-    ks.template wait_lds<0>();
-    S::fence();
-    float v = c[0] + c[1];
-#pragma unroll
-    for (int w = 1; w < 4; ++w) v += c[2 * w] + c[2 * w + 1];
-    const int j = j_begin + tile * 64 + lane;
-    if (j < j_end) colp[j] = v;
-  };
+  float* colp = pr.str_part + ((size_t)batch * pr.groups + it.group) * pr.n_str + j_begin;
+  auto flush = [&](int tile) { cols.flush(tile, colp + tile * 64, j_end - j_begin - tile * 64); };
 
   typename S::Keys y;
   int cur = 0, nxt = 1, nx2 = 2;
@@ -556,7 +1058,7 @@ __global__ __launch_bounds__(256, 2) void pair_sweep_kernel(const PairArgs a) {
             ks.wait_tile();
             S::barrier();
             // (written behind the barrier: the reader of the tile before last is done)
-            put_sum(t, 0, pend);
+            cols.put(t, 0, pend);
             if (t >= 1 && wave == (t & 3)) flush(t - 1);
           }
           if (rb == 1) ks.read_next(y, k, js == 0 ? cur : nxt, js ^ 1);
@@ -587,7 +1089,7 @@ __global__ __launch_bounds__(256, 2) void pair_sweep_kernel(const PairArgs a) {
           if (js == 1) {
             pend = v;
           } else {
-            if (t >= 1) put_sum(t - 1, 1, v);
+            if (t >= 1) cols.put(t - 1, 1, v);
           }
         }
         S::fence();
@@ -599,25 +1101,112 @@ __global__ __launch_bounds__(256, 2) void pair_sweep_kernel(const PairArgs a) {
     nx2 = c;
   }
   // ---- the last unit, the last tile's sums ----
+  float mx = R1[0];
 #pragma unroll
   for (int r = 0; r < 16; ++r) {
+    mx = fmaxf(mx, R1[r]);
     const float e = fast_exp2(R1[r]);
     st[1][r] += e;
     if (r & 1) ps1 += e; else ps0 += e;
   }
-  put_sum(ntiles - 1, 1, ps0 + ps1);
+  cols.put(ntiles - 1, 1, ps0 + ps1);
+  {
+    // this unit says for all of the wavefront's whether the coarse test of the next step would end them
+    // (its logits and cross products are about `ratio` times these, the streamed rows' share of the
+    // latter about that of the others)
+    if (wave_any((mx + 2.0f * cross) * mode.ratio > mode.low - kPairGap) && lane == 0) atomicAdd(went, 4u * (unsigned)ntiles);
+  }
   S::wait_all();  // (also what was fetched past the chunk)
   __syncthreads();
   if (wave == 0) flush(ntiles - 1);
-  // ---- the stationary rows' sums over the lanes ----
-  float* rowp = pr.st_part + ((size_t)batch * pr.chunks + chunk) * pr.n_st;
-#pragma unroll
-  for (int rb = 0; rb < 2; ++rb) {
-    float v = colsum_all(st[rb], li);
-    v += __shfl_xor(v, 16, 64);
-    const int row = (blk0 + rb) * 32 + colsum_key(li & 15, h);
-    if (li < 16 && row < pr.n_st) rowp[row] = v;
+  pair_put_rows(pr, batch, it.chunk, blk0, st, lane);
+}
+
+// One step.  Grid (workgroups of an item of the batch, items of the batch).  A workgroup of four
+// wavefronts owns 256 stationary rows (two blocks of 32 per wavefront, operands in registers) and
+// streams a chunk of the other matrix; it takes every (workgroups)-th of its XCD's work items.
+constexpr int kPairGrid = 512;  // two workgroups per CU
+template <int DP, bool SKIP>
+__global__ __launch_bounds__(256, 2) void pair_sweep_kernel(PairArgsPtr args, int step) {
+  const PairArgs& a = *(const PairArgs*)args;
+  using S = PairStream<DP, false>;
+  // (four tiles, or the sums of a chunk's streamed rows per wavefront)
+  constexpr int kWords = !SKIP ? 3 * S::BUF : (4 * S::BUF > kPairMostTiles * 64 ? 4 * S::BUF : kPairMostTiles * 64);
+  __shared__ __attribute__((aligned(16))) u32x4 lds[kWords];
+  __shared__ float lds_col[2][4][2][64];        // [tile parity][wavefront][half-wave][row]
+  __shared__ PairMode modes[3];
+  __shared__ unsigned went[3];                  // units that went on
+  __shared__ int next_item[2];
+
+  const int batch = blockIdx.y, lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int xcd = blockIdx.x & 7, mine = blockIdx.x >> 3, stride = gridDim.x >> 3, count = a.per_xcd;
+  const PairWork work = (PairWork)(a.work + xcd * count);
+  PairWord word = work[mine];
+  if (wave >= a.first_prob && wave < a.nprob) {
+    PairMode m = pair_mode(pair_known(a, batch, wave, step), a.prob[wave].units, wave, step);
+    // (where its schedule is shorter nothing is done)
+    m.live = step <= a.lens[batch * 3 + wave] + a.extrapolate;
+    if (lane == 0) {
+      modes[wave] = m;
+      went[wave] = 0u;
+    }
   }
+  __syncthreads();
+  unsigned live = 0, sweep = 0, coarse = 0, list = 0;  // bit p: problem p
+  for (int p = a.first_prob; p < a.nprob; ++p) {
+    live |= modes[p].live ? 1u << p : 0u;
+    sweep |= modes[p].sweep ? 1u << p : 0u;
+    coarse |= SKIP && modes[p].live && modes[p].sweep && modes[p].coarse ? 1u << p : 0u;
+    list |= SKIP && modes[p].live && modes[p].list ? 1u << p : 0u;
+  }
+  live = __builtin_amdgcn_readfirstlane(live);
+  sweep = __builtin_amdgcn_readfirstlane(sweep);
+  coarse = __builtin_amdgcn_readfirstlane(coarse);
+  list = __builtin_amdgcn_readfirstlane(list);
+  coarse &= ~list;
+  // (items of these forms take long and are all alike: whoever is free takes the next)
+  int* taken = reinterpret_cast<int*>(a.state) + (size_t)batch * 3 * kPairStateWords + kPairTaken + ((step % 3) * 8 + xcd) * 32;
+  int turn = 0;
+  for (unsigned two = live & ~sweep; two; two &= two - 1) {
+    const int p = __builtin_ctz(two);
+    const PairProblem& pr = a.prob[p];
+    const int per = (pr.two_items + 7) / 8, end = min(pr.two_items, (xcd + 1) * per);
+    for (int k = xcd * per + mine; k < end; ++turn) {
+      if (threadIdx.x == 0) next_item[turn & 1] = xcd * per + stride + atomicAdd(taken + p * kPairStateWords, 1);
+      pair_item_two_sided<DP>(a, batch, pr, p, step, k, lds);  // (with a barrier in it)
+      k = __builtin_amdgcn_readfirstlane(next_item[turn & 1]);
+    }
+  }
+  const bool fetch = (live & sweep & (coarse | list)) == 0;
+  for (int i = mine; i < count;) {
+    const PairItem t = pair_item(word);
+    if (t.prob < 0 || !((live & sweep) >> t.prob & 1)) {
+      i += stride;
+    } else if (SKIP && ((list >> t.prob) & 1)) {
+      i = pair_run_list<DP>(a, batch, work, i, stride, count, list, reinterpret_cast<float*>(lds));
+    } else if (SKIP && ((coarse >> t.prob) & 1)) {
+      i = pair_run_coarse<DP>(a, batch, work, i, stride, count, coarse, modes, went, lds, &lds_col[0][0][0][0]);
+    } else {
+      if (fetch && threadIdx.x == 0) next_item[turn & 1] = stride + atomicAdd(taken + a.first_prob * kPairStateWords + 1, 1);
+      pair_item_plain<DP>(a.prob[t.prob], batch, t, modes[t.prob], &went[t.prob], lds, &lds_col[0][0][0][0]);
+      i = fetch ? __builtin_amdgcn_readfirstlane(next_item[turn & 1]) : i + stride;
+      ++turn;
+    }
+    word = work[min(i, count - 1)];
+  }
+  __syncthreads();
+  if (threadIdx.x >= a.first_prob && threadIdx.x < a.nprob && went[threadIdx.x])
+    atomicAdd(reinterpret_cast<unsigned*>(a.state) + ((size_t)batch * 3 + threadIdx.x) * kPairStateWords + kPairCounts +
+                  ((step % 3) * kPairSlots + blockIdx.x % kPairSlots) * 32,
+              went[threadIdx.x]);
+}
+
+template <int T>
+__global__ __launch_bounds__(1024) void pair_args_kernel(const PairArgs a, PairArgs* out) {
+  static_assert(sizeof(PairArgs) % 4 == 0 && sizeof(PairArgs) <= 4096, "one word a thread");
+  if (threadIdx.x < sizeof(PairArgs) / 4)
+    reinterpret_cast<int*>(out)[threadIdx.x] = reinterpret_cast<const int*>(&a)[threadIdx.x];
 }
 
 // Operand planes of one block of 32 rows at an eps: sqrt(qs) times the rows (as a sum of two floats,
@@ -660,15 +1249,19 @@ __device__ __forceinline__ void pair_write_planes(u32x4* out, const void* pts, s
 // extremes are combined in the workgroup first: with an atomic maximum per 64 rows a merge took
 // 13.6 us at 10,000 points, debiased, half of it for them.
 template <int DP>
-__global__ __launch_bounds__(1024) void pair_merge_kernel(const PairArgs a) {
+__global__ __launch_bounds__(1024) void pair_merge_kernel(PairArgsPtr args, int step, int plane_groups) {
+  const PairArgs& a = *(const PairArgs*)args;
   const int side = blockIdx.y + (a.first_prob ? 2 : 0), item = blockIdx.z, tid = threadIdx.x;
   const PairSide& sd = a.side[side];
-  const int prob = side < 2 ? 0 : side - 1, step = a.step;
-  const int entries = a.lens[item * 3 + prob];
-  const float4 next = pair_coef(a, item, prob, min(step + 1, entries + a.extrapolate));
-  if (step > entries + a.extrapolate) return;
+  const int prob = side < 2 ? 0 : side - 1;
   if ((int)blockIdx.x >= a.merge_groups) {
     // ---- planes for a step with another eps: a quarter of a workgroup per 32 rows ----
+    if ((int)blockIdx.x >= a.merge_groups + plane_groups) {
+      if (step < 0 && item == 0 && blockIdx.y == 0) pair_write_work(a, (blockIdx.x - a.merge_groups - plane_groups) * 1024 + tid);
+      return;
+    }
+    const int entries = a.lens[item * 3 + prob];
+    const float4 next = pair_coef(a, item, prob, min(step + 1, entries + a.extrapolate));
     const int blk = (blockIdx.x - a.merge_groups) * 4 + (tid >> 8);
     if (sd.planes == nullptr || blk >= sd.blocks || step >= entries + a.extrapolate) return;
     if (step >= 0 && pair_coef(a, item, prob, step).x == next.x) return;
@@ -683,12 +1276,18 @@ __global__ __launch_bounds__(1024) void pair_merge_kernel(const PairArgs a) {
   const int part = wave & 3, quarter = wave >> 2, row = blockIdx.x * 256 + quarter * 64 + lane;
   const bool live = row < sd.rows;
   const size_t at = (size_t)item * sd.rows + min(row, sd.rows - 1);
-  const float old = sd.old[at], norm = sd.norm[at];
+  // (everything is on its way before anything is waited for)
+  const int from = step < 0 ? 0 : step & 1;
+  const float old = sd.pot[from * (size_t)a.items * sd.rows + at], norm = sd.norm[at], weight = sd.l2w[at];
+  const int entries = a.lens[item * 3 + prob];
+  const PairKnown known = pair_known(a, item, prob, max(step, 0));
+  if (step > entries + a.extrapolate) return;
+  const float4 next = step < 0 ? known.now : known.next;
   // the row's log weight from the largest of its side, and the other side's largest
-  const float4 lim = a.limits[item];
+  const float4 lim = known.w;
   const bool of_x = side == 0 || side == 2;
   const float own = of_x ? lim.y : lim.w, others = side >= 2 ? own : (of_x ? lim.w : lim.y);
-  const float l2w = sd.l2w[at] - own;
+  const float l2w = weight - own;
   float f = old;
   if (step < 0) {
     if (part > 0) return;
@@ -698,9 +1297,10 @@ __global__ __launch_bounds__(1024) void pair_merge_kernel(const PairArgs a) {
   } else {
     __shared__ float2 sh[4][4][64];
     __shared__ float sh_ex[4][4];
-    const float4 coef = pair_coef(a, item, prob, step);
+    const float4 coef = known.now;
     const float r = __builtin_fmaf(coef.w, old, l2w);  // the row's bias in this step
-    const bool sweep = pair_mode(a, item, prob, step);
+    const PairMode mode = pair_mode(known, a.prob[prob].units, prob, step);
+    const bool sweep = mode.sweep;
     float2 mine = make_float2(kNegBig, 0.f);
     const int rc = min(row, sd.rows - 1);
     if (sweep) {
@@ -728,6 +1328,14 @@ __global__ __launch_bounds__(1024) void pair_merge_kernel(const PairArgs a) {
         mine.x = M;
       }
     }
+    if (blockIdx.x == 0 && (side == 0 || side >= 2) && tid == 0) {
+      // (what the next step knows of the lists)
+      float* out = a.state + ((size_t)item * 3 + prob) * kPairStateWords + kPairLists + ((step + 1) % 3) * 32;
+      const bool made = sweep && mode.coarse && !mode.list;
+      out[0] = mode.list ? mode.drift : 0.f;
+      out[1] = mode.list ? mode.base : mode.low - kPairGap - mode.reserve;
+      out[2] = next.x == coef.x && (made || mode.list) ? 1.f : 0.f;
+    }
     sh[quarter][part][lane] = mine;
     __syncthreads();
     const float2(&all)[4][64] = sh[quarter];
@@ -750,14 +1358,17 @@ __global__ __launch_bounds__(1024) void pair_merge_kernel(const PairArgs a) {
     if (damp < 1.0f) f -= alpha * (1.0f - damp) * norm;
     float ex[4] = {-3.0e38f, -3.0e38f, -3.0e38f, -3.0e38f};
     if (live && part == 0) {
-      sd.out[at] = f;
+      sd.pot[(from ^ 1) * (size_t)a.items * sd.rows + at] = f;
       const float x = __builtin_fmaf(coef.w, old, lse), df = f - old;
       ex[0] = x; ex[1] = -x; ex[2] = df; ex[3] = -df;
       if (!(x == x) || !(df == df) || !(fabsf(next.w * f) < kPairMostBias)) ex[0] = ex[1] = ex[2] = ex[3] = 3.0e38f;
     }
     // (the set that the next merge writes into)
-    if (blockIdx.x == 0 && (side == 0 || side >= 2) && tid < kPairSlots * 8)
-      state[((step + 1) % 3) * kPairSlots * 8 + tid] = 0u;
+    if (blockIdx.x == 0 && (side == 0 || side >= 2) && tid < kPairSlots * 9 + 16) {
+      const int set = (step + 1) % 3, k = tid - kPairSlots * 8, x = k - kPairSlots;
+      state[k < 0 ? set * kPairSlots * 8 + tid
+                  : x < 0 ? kPairCounts + (set * kPairSlots + k) * 32 : kPairTaken + (set * 8 + x / 2) * 32 + x % 2] = 0u;
+    }
     if (part == 0) {
       // halves of the four change places, then what is left of each
 #pragma unroll
@@ -780,7 +1391,8 @@ __global__ __launch_bounds__(1024) void pair_merge_kernel(const PairArgs a) {
   // ---- for the next step ----
   if (part > 0 || step >= entries + a.extrapolate || row >= sd.blocks * 32) return;
   const float b = live ? fmaxf(__builtin_fmaf(next.w, f, l2w), kNegBig) : kNegBig;
-  sd.bias[(size_t)item * sd.blocks * 32 + row] = pair_bias(fmaxf(b, kPairFar));
+  const float cross = live ? pair_cross(next.w, norm, known.reach.z) : 0.f;
+  sd.bias[(size_t)item * sd.blocks * 32 + row] = pair_bias(fmaxf(b, kPairFar), fminf(cross, 60000.f));
   sd.bias32[(size_t)item * sd.blocks * 32 + row] = b;
 }
 

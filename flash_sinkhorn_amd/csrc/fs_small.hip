@@ -107,6 +107,8 @@ void plan_pair(const SmallArgs& a, PairArgs& t) {
     pr.st_blocks = a.pblocks[s];
     pr.str_blocks = a.pblocks[k];
     pr.groups = (pr.n_st + 255) / 256;
+    pr.units = 0.f;
+    for (int g = 0; g < pr.groups; ++g) pr.units += 16.f * (float)((pr.n_str - (pr.self ? 256 * g : 0) + 63) / 64);
   }
   auto items_at = [&](int tiles, PairArgs& u) {
     int n = 0;
@@ -114,7 +116,6 @@ void plan_pair(const SmallArgs& a, PairArgs& t) {
       PairProblem& pr = u.prob[q];
       pr.chunk = tiles * 64;
       pr.chunks = (pr.n_str + pr.chunk - 1) / pr.chunk;
-      pr.first_item = n;
       pr.n_items = 0;
       for (int c = 0; c < pr.chunks; ++c)
         pr.n_items += pr.self ? self_groups_of_chunk(c, pr.chunk, pr.n_str, pr.groups) : pr.groups;
@@ -128,12 +129,15 @@ void plan_pair(const SmallArgs& a, PairArgs& t) {
   };
   int best = 4;
   double cost = 0.0;
-  for (int tiles = 4; tiles <= 64; ++tiles) {
+  for (int tiles = 4; tiles <= kPairMostTiles; ++tiles) {
     const double n = (double)items_at(tiles, t) * a.items;
     const double c = std::ceil(n / 512.0) * (tiles + 2);
     if (cost == 0.0 || c < cost - 1e-9) cost = c, best = tiles;
   }
-  t.total_items = items_at(best, t);
+  items_at(best, t);
+  t.per_xcd = 0;
+  for (int q = t.first_prob; q < t.nprob; ++q) t.per_xcd += (t.prob[q].n_items + 7) / 8;
+  t.merge_groups = (std::max(a.pblocks[0], a.pblocks[1]) + 7) / 8;
   for (int i = 0; i < 4; ++i) {
     PairSide& sd = t.side[i];
     const int mat = i & 1;
@@ -142,8 +146,7 @@ void plan_pair(const SmallArgs& a, PairArgs& t) {
   }
 }
 
-// Pointers of a medium problem's kernels once the workspace is laid out; what alternates from
-// step to step is set by pair_step_args.
+// Pointers of a medium problem's kernels once the workspace is laid out.
 void bind_pair(const SmallArgs& a, PairArgs& t) {
   t.table = a.table;
   t.table_len = a.table_len;
@@ -171,6 +174,7 @@ void bind_pair(const SmallArgs& a, PairArgs& t) {
       sd.ms_parts = i == ss ? pr.chunks : (pr.n_st + pr.chunk - 1) / pr.chunk;
       sd.self = pr.self;
       sd.chunk = pr.chunk;
+      sd.pot = a.pot[i];
       sd.norm = a.norm[mat];
       sd.l2w = a.l2w[mat];
       sd.pts = a.pts[mat];
@@ -184,20 +188,10 @@ void bind_pair(const SmallArgs& a, PairArgs& t) {
   }
 }
 
-void pair_step_args(const SmallArgs& a, PairArgs& t, int step) {
-  t.step = step;
-  for (int i = a.self == 2 ? 2 : 0; i < (a.self ? 4 : 2); ++i) {
-    PairSide& sd = t.side[i];
-    const size_t n = (size_t)a.items * sd.rows;
-    const int from = step < 0 ? 0 : step & 1;
-    sd.old = a.pot[i] + from * n;
-    sd.out = a.pot[i] + (from ^ 1) * n;
-  }
-}
-
 // The kernels' arguments with the workspace laid out from `ws` (null: sizes only); returns the
 // bytes the workspace takes.
-size_t layout(const fs_small_problem* p, void* ws, SmallArgs& a, PairArgs* pa = nullptr, DenseArgs* da = nullptr) {
+size_t layout(const fs_small_problem* p, void* ws, SmallArgs& a, PairArgs* pa = nullptr, DenseArgs* da = nullptr,
+              PairArgs** pair_at = nullptr) {
   std::memset(&a, 0, sizeof(a));
   a.pair = use_pair(p) ? 1 : 0;
   a.pts[0] = p->x;
@@ -293,10 +287,12 @@ size_t layout(const fs_small_problem* p, void* ws, SmallArgs& a, PairArgs* pa = 
     std::memset(&t, 0, sizeof(t));
     plan_pair(a, t);
     take(t.state, items * 3 * kPairStateWords * 4);
+    take(t.work, 8 * (size_t)t.per_xcd * sizeof(int4));
     for (int q = t.first_prob; q < t.nprob; ++q) {
       PairProblem& pr = t.prob[q];
       take(pr.st_part, items * (size_t)pr.chunks * (size_t)pr.n_st * 4);
       take(pr.str_part, items * (size_t)pr.groups * (size_t)pr.n_str * 4);
+      take(pr.list, items * (size_t)pr.n_items * (4 * kPairListWords * 8));
       take(pr.st_ms, items * (size_t)pr.chunks * (size_t)pr.n_st * sizeof(float2));
       if (!pr.self) take(pr.str_ms, items * (size_t)((pr.n_st + pr.chunk - 1) / pr.chunk) * (size_t)pr.n_str * sizeof(float2));
     }
@@ -305,16 +301,20 @@ size_t layout(const fs_small_problem* p, void* ws, SmallArgs& a, PairArgs* pa = 
       take(sd.bias, items * (size_t)sd.blocks * 32 * sizeof(u32x4));
       take(sd.bias32, items * (size_t)sd.blocks * 32 * 4);
     }
+    PairArgs* args;
+    take(args, sizeof(PairArgs));
+    if (pair_at) *pair_at = args;
     if (pa) bind_pair(a, t);
   }
   return at;
 }
 
 template <int DP>
-int launch_prep(const SmallArgs& a, hipStream_t st) {
+int launch_prep(const SmallArgs& a, const PairArgs& pa, PairArgs* pair_at, hipStream_t st) {
   const int xb = a.blocks[0] > a.blocks[1] ? a.blocks[0] : a.blocks[1];
   hipLaunchKernelGGL((small_stats_kernel<0>), dim3(a.stat_blocks, 2, a.items), dim3(256), 0, st, a);
   hipLaunchKernelGGL((small_prep_kernel<DP>), dim3(xb + 1, 2, a.items), dim3(256), 0, st, a);
+  if (a.pair) hipLaunchKernelGGL((pair_args_kernel<0>), dim3(1), dim3(1024), 0, st, pa, pair_at);
   return hipGetLastError() == hipSuccess ? FS_OK : FS_ERR_LAUNCH_FAILED;
 }
 
@@ -389,22 +389,23 @@ int launch_alternating(const SmallArgs& a, int it, hipStream_t st) {
 }
 
 template <int DP>
-int launch_pair_merge(const SmallArgs& a, PairArgs& t, int step, hipStream_t st) {
-  pair_step_args(a, t, step);
+int launch_pair_merge(const SmallArgs& a, const PairArgs& t, PairArgs* at, int step, hipStream_t st) {
   const int blocks = std::max(a.pblocks[0], a.pblocks[1]);
-  t.merge_groups = (blocks + 7) / 8;
   // (at one eps the planes are written once, before the first step)
-  const int grid = t.merge_groups + (step < 0 || a.sched != 0 ? (blocks + 3) / 4 : 0);
-  hipLaunchKernelGGL((pair_merge_kernel<DP>), dim3(grid, a.self == 1 ? 4 : 2, a.items), dim3(1024), 0, st, t);
+  const int planes = step < 0 || a.sched != 0 ? (blocks + 3) / 4 : 0;
+  const int grid = t.merge_groups + planes + (step < 0 ? (8 * t.per_xcd + 1023) / 1024 : 0);
+  hipLaunchKernelGGL((pair_merge_kernel<DP>), dim3(grid, a.self == 1 ? 4 : 2, a.items), dim3(1024), 0, st,
+                     (PairArgsPtr)at, step, planes);
   return hipGetLastError() == hipSuccess ? FS_OK : FS_ERR_LAUNCH_FAILED;
 }
 
 template <int DP>
-int launch_pair_step(const SmallArgs& a, PairArgs& t, int step, hipStream_t st) {
-  pair_step_args(a, t, step);
-  const int blocks = (t.total_items + 7) / 8 * 8;
-  hipLaunchKernelGGL((pair_sweep_kernel<DP>), dim3(blocks, a.items), dim3(256), 0, st, t);
-  return launch_pair_merge<DP>(a, t, step, st);
+int launch_pair_step(const SmallArgs& a, const PairArgs& t, PairArgs* at, int step, hipStream_t st) {
+  const int blocks = std::min(8 * t.per_xcd, kPairGrid);
+  // (clouds of few columns are not peaked at the eps they are solved at: nothing to skip)
+  const auto kernel = DP > 16 || a.d > 8 ? pair_sweep_kernel<DP, true> : pair_sweep_kernel<DP, DP != 16>;
+  hipLaunchKernelGGL(kernel, dim3(blocks, a.items), dim3(256), 0, st, (PairArgsPtr)at, step);
+  return launch_pair_merge<DP>(a, t, at, step, st);
 }
 
 template <int DP>
@@ -444,9 +445,9 @@ int fs_small_solve(const fs_small_problem* p, void* workspace, size_t workspace_
   if (rc != FS_OK) return rc;
   if ((p->sched == 1 || p->threshold > 0.f) && !host_words) return FS_ERR_NULL_POINTER;
   SmallArgs a;
-  PairArgs pa;
+  PairArgs pa, *pair_at = nullptr;
   DenseArgs da;
-  if (!workspace || layout(p, workspace, a, &pa, &da) > workspace_bytes) return FS_ERR_WORKSPACE_TOO_SMALL;
+  if (!workspace || layout(p, workspace, a, &pa, &da, &pair_at) > workspace_bytes) return FS_ERR_WORKSPACE_TOO_SMALL;
   hipStream_t st = (hipStream_t)stream;
   int entries = a.entries;
   a.host_words = host_words;
@@ -465,9 +466,9 @@ int fs_small_solve(const fs_small_problem* p, void* workspace, size_t workspace_
   const bool dense = use_dense(p);
   rc = dense ? dense_prepare(a, da, st) : by_width(p->d, [&](auto dp) {
     constexpr int DP = decltype(dp)::value;
-    const int r = launch_prep<DP>(a, st);
+    const int r = launch_prep<DP>(a, pa, pair_at, st);
     if constexpr (DP <= 64)
-      if (r == FS_OK && a.pair) return launch_pair_merge<DP>(a, pa, -1, st);
+      if (r == FS_OK && a.pair) return launch_pair_merge<DP>(a, pa, pair_at, -1, st);
     return r;
   });
   if (rc != FS_OK) return rc;
@@ -478,7 +479,7 @@ int fs_small_solve(const fs_small_problem* p, void* workspace, size_t workspace_
       constexpr int DP = decltype(dp)::value;
       if (a.alternating) return launch_alternating<DP>(a, s, st);
       if constexpr (DP <= 64)
-        if (a.pair) return launch_pair_step<DP>(a, pa, s, st);
+        if (a.pair) return launch_pair_step<DP>(a, pa, pair_at, s, st);
       return launch_step<DP>(a, s, st);
     });
   };

@@ -96,6 +96,48 @@ def test_one_sweep_self_problems(n, m, d, eps):
             assert np.abs(p.cpu().numpy() - q).max() < 2.0 ** -20 * 4.0 * (u * u).sum(axis=1).max()
 
 
+def symmetric_steps(x, y, a, b, eps, n_iters, rho=(None, None)):
+    """The same updates in double precision on the GPU (more logits than numpy takes in good time)."""
+    X, Y, A, B = (t.double() for t in dev(x, y, a, b))
+    nx, ny = (X * X).sum(1), (Y * Y).sum(1)
+    la, lb = A.clamp(min=1e-300).log(), B.clamp(min=1e-300).log()
+
+    def half(u, v, pot, lw, norm, r):  # potentials of u's rows, without the norms
+        damp = 1.0 if r is None else 1.0 / (1.0 + eps / r)
+        out = torch.cat([torch.logsumexp((2.0 * p @ v.T + pot) / eps + lw, 1) for p in u.split(1024)])
+        return -eps * damp * out - (1.0 - damp) * norm
+    f, g = -nx, -ny
+    f, g = half(X, Y, g, lb, nx, rho[0]), half(Y, X, f, la, ny, rho[1])
+    for _ in range(n_iters):
+        f, g = 0.5 * (f + half(X, Y, g, lb, nx, rho[0])), 0.5 * (g + half(Y, X, f, la, ny, rho[1]))
+    last = half(X, Y, g, lb, nx, rho[0]), half(Y, X, f, la, ny, rho[1])
+    return [t.cpu().numpy() for t in (last[0] + nx, last[1] + ny, f + nx, g + ny)]
+
+
+# ---- peaked plans: units that end at their coarse products, then lists of those that do not.  Odd
+# numbers of rows, one row group and one chunk, light rows, relaxed marginals, several clusters.  A
+# step's error, 2^-21 of the largest cost for the logits and as much for what fp32 holds of norms and
+# potentials, is halved by every averaged step: four of them at most ----
+@pytest.mark.parametrize("n,m,d,eps,mixed,rho", [(4513, 4481, 64, 0.01, False, (None, None)),
+                                                 (5003, 4201, 9, 0.002, False, (None, None)),
+                                                 (4700, 4400, 33, 0.01, True, (2.0, 0.5)),
+                                                 (250, 65000, 16, 0.003, True, (None, None)),
+                                                 (65000, 310, 40, 0.02, False, (None, 1.0))])
+def test_peaked_plans(n, m, d, eps, mixed, rho):
+    from flash_sinkhorn_amd.kernels import sinkhorn_flashstyle_symmetric as solve
+    x, y, a, b = inputs(n + d, n, m, d, scale=0.5, y_shift=0.2)
+    if mixed:
+        r = np.random.default_rng(d)
+        means = r.standard_normal((6, d)).astype(np.float32)
+        x, y = x + means[r.integers(6, size=n)], y + means[r.integers(6, size=m)]
+        a[::7] *= 1e-3
+    kw = dict(use_epsilon_scaling=False, eps=eps, n_iters=30, rho_x=rho[0], rho_y=rho[1])
+    got = solve(*dev(x, y, a, b), return_prelast=True, **kw)
+    largest = sum(np.sqrt((t.astype(np.float64) ** 2).sum(1)).max() for t in (x, y)) ** 2
+    for g, w in zip(got, symmetric_steps(x, y, a, b, eps, 30, rho)):
+        assert np.abs(g.cpu().numpy() - w).max() < 4 * 2.0 ** -21 * largest
+
+
 # ---- numbers that fp32 does not hold, or that the library would take for "none" ----
 @pytest.mark.parametrize("d", [4, 200])
 def test_relaxations_of_zero_and_less_are_not_strict_marginals(d):
