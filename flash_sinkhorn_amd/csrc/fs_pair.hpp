@@ -56,6 +56,7 @@ constexpr float kPairGap = 44.f;     // base-2 distance below every sum at which
 // 0.4 / 0.5 / 0.7 here, 12,000 x 9 (share 0.35) 1,512 / 1,250 / 1,260 / 1,351 us, 12 columns 1,240 / 1,380 / 1,385 /
 // 1,531 at eps 0.05, 18 columns there 1,600 / 1,656 / 1,655 / 1,540, 32 at 0.1 - / 1,627 / 1,715 / 1,606.
 constexpr float kPairOn = 0.4f;
+constexpr float kPairTwoOn = 0.7f;   // the same of two-sided steps
 constexpr float kPairFar = -2.4e8f;  // bias of rows past the last one, in base 2 (2^12 times -58594)
 
 // One problem: stationary rows against streamed rows.  Pointers of item 0.
@@ -72,13 +73,15 @@ struct PairProblem {
   int st_blocks, str_blocks;  // 32-row blocks, padding included
   int groups, chunks, chunk;  // 256-row groups of the stationary rows; chunks (of rows) of the others
   int self;                 // a matrix with itself: a group streams only rows at or behind its first
-  float units;              // 32 x 32 units of all its work items
+  float units;              // 32 x 32 units of all its work items; 0: every logit is computed
   unsigned long long* list; // [items][n_items][wavefront][kPairListWords] units to visit
   int n_items;              // work items of this problem
   // two-sided steps: (maximum, sum) per row and chunk of keys, and their work items (those of the
   // streamed rows' own half-update from two_first on; a self problem has none)
   float2* st_ms;            // [items][chunks][n_st]
   float2* str_ms;           // [items][chunks of n_st][n_str]
+  int* st_best;             // ... and the key of that maximum, where a coarse step has seen one (else -1)
+  int* str_best;
   int two_first, two_items;
 };
 
@@ -93,6 +96,9 @@ struct PairMode {
   float drift;   // with a list: what a logit may have risen by since it was made
   float base;    // ... and what no logit off it reached then
   float reserve; // how far below this step's line a list made now begins
+  int two;       // a two-sided step whose units are ended by their coarse products
+  float rho;     // its logits over those of the step before
+  float least[2];  // what the least change of the other rows' potentials adds to a logit of the rows of a side
 };
 
 // One side of a problem in the merge: the rows whose potentials it updates.
@@ -100,7 +106,15 @@ struct PairSide {
   const float* part;        // sums: [parts][rows]
   const float* col;         // self problems: the column sums that the groups before took
   const float2* ms;         // two-sided steps: (maximum, sum) per chunk of keys, and row
+  const int* best;
   int ms_parts;
+  // of every row: log2 of its last sum in the kernels' units, the key of its largest logit when a two-sided
+  // step last saw one (-1: none has), the two points' inner product
+  float* sum2;
+  int* key;
+  float* dot;
+  const void* other;        // points and number of the rows that its keys are
+  int others;
   float* pot;               // [2 parities][items][rows] potentials
   const float* norm;
   const float* l2w;
@@ -191,11 +205,13 @@ __device__ __forceinline__ PairKnown pair_known(const PairArgs& a, int item, int
 __device__ __forceinline__ PairMode pair_mode(const PairKnown& k, float units, int prob, int step) {
   const float4 now = k.now, before = k.before, next = k.next, w = k.w, reach = k.reach;
   const float4 lim = prob == 0 ? w : (prob == 1 ? make_float4(w.x, w.y, w.x, w.y) : make_float4(w.z, w.w, w.z, w.w));
-  bool ok = (pair_scale(reach.x, now.y) == 0.f) & (lim.x > -1000.f) & (lim.z > -1000.f) &
-            (now.w * reach.z < kPairMostBias);
+  const bool ok0 = (pair_scale(reach.x, now.y) == 0.f) & (now.w * reach.z < kPairMostBias);
+  bool ok = ok0 & (lim.x > -1000.f) & (lim.z > -1000.f);
   PairMode mode;
   mode.ratio = fmaxf(now.x / next.x, 1.f);
-  mode.coarse = mode.list = 0;
+  mode.coarse = mode.list = mode.two = 0;
+  mode.rho = 1.f;
+  mode.least[0] = mode.least[1] = 0.f;
   mode.drift = mode.base = mode.reserve = 0.f;
   if (step == 0) {
     mode.low = fminf(lim.x - lim.y, lim.z - lim.w) - reach.y * now.w;
@@ -215,6 +231,10 @@ __device__ __forceinline__ PairMode pair_mode(const PairKnown& k, float units, i
   for (int i = 0; i < 8; ++i) e[i] = pair_value((unsigned)__builtin_amdgcn_readlane((int)v, i));
   // (behind a two-sided step nothing is known: tried)
   mode.coarse = (float)on < kPairOn * units;
+  mode.two = ok0 && rho >= 1.f && (float)on < kPairTwoOn * units;
+  mode.rho = rho;
+  mode.least[0] = -kappa * e[7];
+  mode.least[1] = -kappa * e[3];
   mode.low = 3.0e38f;
 #pragma unroll
   for (int s = 0; s < 2; ++s) {
@@ -531,6 +551,182 @@ __device__ __forceinline__ void pair_item_two_sided(const PairArgs& a, int batch
     const int row = (blk0 + rb) * 32 + li;
     if (h == 0 && row < n_q) out[row] = make_float2(M, sum);
   }
+}
+
+// A work item with running maxima in a step in which most units are empty: as pair_item_two_sided, but
+// a unit ends at its hi * hi products where these, the key bias and the bound on the cross products stay
+// kPairGap base-2 units below a lower bound on the logarithm of every row's sum.  That bound is the
+// larger of two: the last step's sum, less what the potentials of the keys may have fallen by (with eps' <
+// eps and rho = eps / eps', power means give rho times the old logarithm less (rho - 1) log2 of the
+// weights' sum, which counts them from the largest), and the row's logit at the key that held its
+// largest when a step last saw it (pair_merge_kernel keeps the two points' inner product).  A lane holds
+// one query row and 16 keys, the key's bias and its share of the bound ride in the matrix product.
+template <int DP>
+__device__ __forceinline__ unsigned pair_item_two_coarse(const PairArgs& a, int batch, const PairProblem& pr, int prob,
+                                                         int step, const PairMode& mode, int it, u32x4* lds) {
+  using S = PairStream<DP, false>;
+  constexpr int KK = DP / 16;
+  const int side = it >= pr.two_first ? 1 : 0;  // the streamed rows' own half-update
+  if (side) it -= pr.two_first;
+  const PairSide& sd = a.side[prob == 0 ? side : 1 + prob];
+  const int n_k = side ? pr.n_st : pr.n_str, n_q = side ? pr.n_str : pr.n_st;
+  const int groups = (n_q + 255) / 256, chunk = it / groups, group = it % groups;
+  const int kblocks = side ? pr.st_blocks : pr.str_blocks, qblocks = side ? pr.str_blocks : pr.st_blocks;
+  const int lane = pair_lane(), li = lane & 31, h = lane >> 5;
+  const int j_begin = chunk * pr.chunk, j_end = min(n_k, j_begin + pr.chunk);
+  const int ntiles = (j_end - j_begin + 63) / 64;
+  const float4 coef = pair_coef(a, batch, prob, step);
+  const float* kbias = (side ? pr.st_bias32 : pr.str_bias32) + (size_t)batch * kblocks * 32;
+  S ks;
+  ks.begin(lds, side ? pr.st_planes : pr.str_planes, side ? pr.st_bias : pr.str_bias, kblocks, batch, j_begin);
+  const int blk0 = group * 8 + ks.wave * 2;
+  ks.stage(0, 0);
+  ks.stage(1, 1);
+  ks.stage(2, 2);
+  u32x4 x[2][2][KK];
+  pair_load_rows(x, (side ? pr.str_planes : pr.st_planes) + ((size_t)batch * qblocks + blk0) * (2 * KK * 64), lane);
+  float m[2], s[2], on_at[2];
+  int best[2];
+#pragma unroll
+  for (int rb = 0; rb < 2; ++rb) {
+    const int row = (blk0 + rb) * 32 + li;
+    const size_t at = (size_t)batch * n_q + min(row, n_q - 1);
+    const int key = sd.key[at];
+    const float sum2 = sd.sum2[at], dot = sd.dot[at];
+    const float cross = pair_cross_of((side ? pr.str_bias : pr.st_bias)[((size_t)batch * qblocks + blk0 + rb) * 32 + li]);
+    const float there = __builtin_fmaf(coef.y, dot, kbias[max(key, 0)]) - 0.5f - 9.5367431640625e-07f * coef.w * a.reach[batch].z;
+    float low = mode.rho * sum2 - (mode.rho - 1.f) * __log2f((float)n_k) + fminf(mode.least[side], 0.f) - 0.5f;
+    low = fmaxf(fmaxf(low, key >= 0 ? there : -3.0e38f), 0.5f * kNegBig);  // (also where it is not a number)
+    m[rb] = low;
+    s[rb] = 0.f;
+    best[rb] = -1;
+    on_at[rb] = row < n_q ? low - kPairGap - cross : 3.0e38f;
+  }
+  const unsigned one = 0x3c00u, s1 = 0x6c00u, s2 = 0x3c00u, s3 = 0x0c00u;  // fp16 1, 2^12, 1, 2^-12
+  // the key's bias alone, with its share of the bound, and that share taken off again
+  u32x4 qb = {0u, s1 << 16, s2 | s3 << 16, one}, qoff = {0u, 0u, 0u, one | 0x8000u};
+  if (h) qb = qoff = u32x4{0u, 0u, 0u, 0u};
+  u32x4 y[KK], yb;
+  f32x16 acc[2][2];  // [parity of the sub-tile][row block]
+  unsigned went_on = 0;
+  auto read_key = [&](int k, int buf, int js) {
+    if (k < KK) y[k] = S::read(&lds[buf * S::BUF + (js * (2 * KK) + k) * 64 + lane]);
+    else yb = S::read(&lds[buf * S::BUF + S::PIECES * 64 + js * 32 + li]);
+  };
+  auto wait_reads = [&]() {
+    S::fence();
+    ks.template wait_lds<0>();
+    S::fence();
+  };
+  auto run = [&](int to, int buf, int js, bool test, float (&mx)[2]) {
+#pragma unroll
+    for (int k = 0; k <= KK; ++k) {
+#pragma unroll
+      for (int rb = 0; rb < 2; ++rb) {
+        f32x16& c = acc[to][rb];
+        if (k == 0) {
+#pragma unroll
+          for (int r = 0; r < 16; ++r) c[r] = 0.f;
+        }
+        c = k < KK ? small_mfma(y[k < KK ? k : 0], x[rb][0][k < KK ? k : 0], c) : small_mfma(yb, qb, c);
+        if (rb == 1) read_key(k, buf, js);
+        if (test) {
+          constexpr int N = 2 * (KK + 1);
+          const int i = 2 * k + rb, v0 = i * 32 / N, v1 = (i + 1) * 32 / N;
+#pragma unroll
+          for (int v = v0; v < v1; ++v) {
+            const float l = acc[to ^ 1][v >> 4][v & 15];
+            mx[v >> 4] = (v & 15) == 0 ? l : fmaxf(mx[v >> 4], l);
+          }
+        }
+        S::fence();
+      }
+    }
+  };
+  auto finish = [&](int of, int sub, int buf, const float (&mx)[2]) {
+    const int js = sub & 1;
+    const bool on0 = wave_any(mx[0] > on_at[0]), on1 = wave_any(mx[1] > on_at[1]);
+    if (!(on0 || on1)) return;
+    u32x4 z[2][KK], zb;
+#pragma unroll
+    for (int q = 1; q >= 0; --q)
+#pragma unroll
+      for (int kk = 0; kk < KK; ++kk) z[q][kk] = S::read(&lds[buf * S::BUF + (js * (2 * KK) + q * KK + kk) * 64 + lane]);
+    zb = S::read(&lds[buf * S::BUF + S::PIECES * 64 + js * 32 + li]);
+    wait_reads();
+#pragma unroll
+    for (int rb = 0; rb < 2; ++rb) {
+      if (rb ? !on1 : !on0) continue;
+      ++went_on;
+      f32x16 c = small_mfma(zb, qoff, acc[of][rb]);
+#pragma unroll
+      for (int kk = 0; kk < KK; ++kk) c = small_mfma(z[1][kk], x[rb][0][kk], c);
+#pragma unroll
+      for (int kk = 0; kk < KK; ++kk) c = small_mfma(z[0][kk], x[rb][1][kk], c);
+      const float top = small_max16(c[0], c);
+      if (wave_any(top > m[rb])) {
+        if (top > m[rb]) {
+          s[rb] *= fast_exp2(m[rb] - top);
+          m[rb] = top;
+          int at = 0;
+#pragma unroll
+          for (int r = 1; r < 16; ++r) at = c[r] == top ? r : at;
+          best[rb] = j_begin + sub * 32 + 8 * (at >> 2) + 4 * h + (at & 3);
+        }
+      }
+      float p0 = 0.f, p1 = 0.f;
+#pragma unroll
+      for (int r = 0; r < 16; r += 2) {
+        p0 += fast_exp2(c[r] - m[rb]);
+        p1 += fast_exp2(c[r + 1] - m[rb]);
+      }
+      s[rb] += p0 + p1;
+    }
+  };
+  S::fence();
+  S::wait_all();
+  S::barrier();
+  float mx[2];
+#pragma unroll
+  for (int k = 0; k <= KK; ++k) read_key(k, 0, 0);
+  wait_reads();
+  run(0, 0, 1, false, mx);
+  wait_reads();
+  for (int t = 0; t < ntiles; ++t) {
+    const int cur = t & 3, nxt = (t + 1) & 3;
+    // tile t + 1 has landed, and every wavefront is through with tile t - 1
+    S::fence();
+    S::wait_tile();
+    S::fence();
+    S::barrier();
+    ks.stage(t + 3, (t + 3) & 3);
+    S::fence();
+    run(1, nxt, 0, true, mx);
+    wait_reads();
+    finish(0, 2 * t, cur, mx);
+    S::fence();
+    run(0, nxt, 1, true, mx);
+    wait_reads();
+    finish(1, 2 * t + 1, cur, mx);
+  }
+  S::wait_all();
+  __syncthreads();  // (the next item fills the same buffers)
+  const size_t to = ((size_t)batch * ((n_k + pr.chunk - 1) / pr.chunk) + chunk) * n_q;
+  float2* out = (side ? pr.str_ms : pr.st_ms) + to;
+  int* keys = (side ? pr.str_best : pr.st_best) + to;
+#pragma unroll
+  for (int rb = 0; rb < 2; ++rb) {
+    const float mo = xor32(m[rb]), so = xor32(s[rb]);
+    const int bo = __shfl_xor(best[rb], 32, 64);
+    const float M = fmaxf(m[rb], mo);
+    const float sum = s[rb] * fast_exp2(m[rb] - M) + so * fast_exp2(mo - M);
+    const int row = (blk0 + rb) * 32 + li;
+    if (h == 0 && row < n_q) {
+      out[row] = make_float2(M, sum);
+      keys[row] = bo >= 0 && (mo > m[rb] || best[rb] < 0) ? bo : best[rb];
+    }
+  }
+  return went_on;
 }
 
 // What a work item of the one-sweep forms is: 256 stationary rows against a chunk of streamed ones.
@@ -1153,13 +1349,15 @@ __global__ __launch_bounds__(256, 2) void pair_sweep_kernel(PairArgsPtr args, in
     }
   }
   __syncthreads();
-  unsigned live = 0, sweep = 0, coarse = 0, list = 0;  // bit p: problem p
+  unsigned live = 0, sweep = 0, coarse = 0, list = 0, ends = 0;  // bit p: problem p
   for (int p = a.first_prob; p < a.nprob; ++p) {
     live |= modes[p].live ? 1u << p : 0u;
     sweep |= modes[p].sweep ? 1u << p : 0u;
     coarse |= SKIP && modes[p].live && modes[p].sweep && modes[p].coarse ? 1u << p : 0u;
     list |= SKIP && modes[p].live && modes[p].list ? 1u << p : 0u;
   }
+  for (int p = a.first_prob; p < a.nprob; ++p) ends |= SKIP && modes[p].two ? 1u << p : 0u;
+  ends = __builtin_amdgcn_readfirstlane(ends);
   live = __builtin_amdgcn_readfirstlane(live);
   sweep = __builtin_amdgcn_readfirstlane(sweep);
   coarse = __builtin_amdgcn_readfirstlane(coarse);
@@ -1174,7 +1372,14 @@ __global__ __launch_bounds__(256, 2) void pair_sweep_kernel(PairArgsPtr args, in
     const int per = (pr.two_items + 7) / 8, end = min(pr.two_items, (xcd + 1) * per);
     for (int k = xcd * per + mine; k < end; ++turn) {
       if (threadIdx.x == 0) next_item[turn & 1] = xcd * per + stride + atomicAdd(taken + p * kPairStateWords, 1);
-      pair_item_two_sided<DP>(a, batch, pr, p, step, k, lds);  // (with a barrier in it)
+      // (with a barrier in them)
+      if (SKIP && ((ends >> p) & 1)) {
+        const unsigned on = pair_item_two_coarse<DP>(a, batch, pr, p, step, modes[p], k, lds);
+        // (both sides of the xy problem count)
+        if (lane == 0 && on) atomicAdd(&went[p], pr.self ? on : (on + 1) / 2);
+      } else {
+        pair_item_two_sided<DP>(a, batch, pr, p, step, k, lds);
+      }
       k = __builtin_amdgcn_readfirstlane(next_item[turn & 1]);
     }
   }
@@ -1292,16 +1497,20 @@ __global__ __launch_bounds__(1024) void pair_merge_kernel(PairArgsPtr args, int 
   if (step < 0) {
     if (part > 0) return;
     // (nothing is known of the sums yet)
+    if (live) sd.key[at] = -1;
     if (blockIdx.x == 0 && quarter == 0 && (side == 0 || side >= 2))
       for (int i = lane; i < kPairStateWords; i += 64) state[i] = 0u;
   } else {
     __shared__ float2 sh[4][4][64];
+    __shared__ int sh_best[4][4][64];
+    __shared__ float sh_dot[4][4][64];
     __shared__ float sh_ex[4][4];
     const float4 coef = known.now;
     const float r = __builtin_fmaf(coef.w, old, l2w);  // the row's bias in this step
     const PairMode mode = pair_mode(known, a.prob[prob].units, prob, step);
     const bool sweep = mode.sweep;
     float2 mine = make_float2(kNegBig, 0.f);
+    int best = -1;
     const int rc = min(row, sd.rows - 1);
     if (sweep) {
       float s = 0.f;
@@ -1320,13 +1529,19 @@ __global__ __launch_bounds__(1024) void pair_merge_kernel(PairArgsPtr args, int 
       mine.y = s;
     } else {
       const float2* p = sd.ms + (size_t)item * sd.ms_parts * sd.rows + rc;
+      const int* q = sd.best + (size_t)item * sd.ms_parts * sd.rows + rc;
+      float most = kNegBig;
 #pragma unroll 8
       for (int c = part; c < sd.ms_parts; c += 4) {
         const float2 v = p[(size_t)c * sd.rows];
+        const int k = mode.two ? q[(size_t)c * sd.rows] : -1;
         const float M = fmaxf(mine.x, v.x);
         mine.y = mine.y * fast_exp2(mine.x - M) + v.y * fast_exp2(v.x - M);
         mine.x = M;
+        best = k >= 0 && v.x > most ? k : best;
+        most = k >= 0 ? fmaxf(most, v.x) : most;
       }
+      sh_best[quarter][part][lane] = best;
     }
     if (blockIdx.x == 0 && (side == 0 || side >= 2) && tid == 0) {
       // (what the next step knows of the lists)
@@ -1350,6 +1565,31 @@ __global__ __launch_bounds__(1024) void pair_merge_kernel(PairArgsPtr args, int 
       for (int w = 0; w < 4; ++w) s += all[w][lane].y * fast_exp2(all[w][lane].x - M);
       lse = small_log2(fmaxf(s, 1e-40f), M + others);
     }
+    if (!sweep && mode.two) {
+      // the key of the largest logit that any chunk has seen beyond where it began, the pair's inner product
+      const float2(&ms)[4][64] = sh[quarter];
+      float most = kNegBig;
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        const int k = sh_best[quarter][w][lane];
+        best = k >= 0 && ms[w][lane].x > most ? k : (w == 0 ? -1 : best);
+        most = k >= 0 ? fmaxf(most, ms[w][lane].x) : most;
+      }
+      const bool fresh = live && best >= 0 && best != sd.key[at];
+      float dot = 0.f;
+      if (fresh) {
+        const size_t u = at * sd.d, v = ((size_t)item * sd.others + best) * sd.d;
+#pragma unroll 4
+        for (int k = part; k < sd.d; k += 4)
+          dot = __builtin_fmaf(small_load(sd.pts, u + k, sd.dtype), small_load(sd.other, v + k, sd.dtype), dot);
+      }
+      sh_dot[quarter][part][lane] = dot;
+      __syncthreads();
+      if (fresh && part == 0) {
+        sd.key[at] = best;
+        sd.dot[at] = (sh_dot[quarter][0][lane] + sh_dot[quarter][1][lane]) + (sh_dot[quarter][2][lane] + sh_dot[quarter][3][lane]);
+      }
+    }
     const float rho = sd.rho, eps = coef.x;
     const float damp = rho > 0.f ? 1.0f / (1.0f + eps / rho) : 1.0f;
     const float alpha = (step == 0 || step > entries) ? 1.0f : 0.5f;
@@ -1359,6 +1599,7 @@ __global__ __launch_bounds__(1024) void pair_merge_kernel(PairArgsPtr args, int 
     float ex[4] = {-3.0e38f, -3.0e38f, -3.0e38f, -3.0e38f};
     if (live && part == 0) {
       sd.pot[(from ^ 1) * (size_t)a.items * sd.rows + at] = f;
+      sd.sum2[at] = lse - others;
       const float x = __builtin_fmaf(coef.w, old, lse), df = f - old;
       ex[0] = x; ex[1] = -x; ex[2] = df; ex[3] = -df;
       if (!(x == x) || !(df == df) || !(fabsf(next.w * f) < kPairMostBias)) ex[0] = ex[1] = ex[2] = ex[3] = 3.0e38f;
