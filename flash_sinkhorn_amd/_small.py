@@ -107,19 +107,14 @@ class Solved:
 def _size_ok(n: int, m: int, d: int, fixed: bool, self_terms: int, stops: bool,
              items: int = 1) -> bool:
     """Whether a problem of this size is faster here than on the general path, launch by launch.
-    Whole passes are compared: the gradient alone is slower here from about 3e8 logits on at 33 .. 64
-    columns (13,000 x 13,000, both sides: 445 against 364 us; 20,000: 820 against 654), 8e8 at
-    17 .. 32, 1.3e9 at 9 .. 16 and 2.5e9 below; it is the more exact one (3 to 35 % smaller errors).
 
     d > 128: while the kept products stay below 1 GiB; reading them beats forming them at every such
     width (8,192 x 1,536: 0.07 against 0.5 ms a step).
 
-    d <= 64 (``pair_sweep_kernel`` from 2e7 logits per step on): everywhere but where two large
-    clouds let the general path skip tiles by its coarse product, from 24,000 rows on.  At fixed
-    eps that pays from its first size on (30,000 x 64, 40 steps: 9.6 against 18 ms; 22,000 x 64, no
-    skipping: 11.3 against 10.2), on a schedule only in its last steps (30,000 x 64, both gradients:
-    8.9 against 9.6 ms; 40,000 x 16: 6.9 against 6.7), and with d <= 8 not at all (50,000 x 3: 28
-    against 19 ms).
+    d <= 64 (``pair_sweep_kernel`` from 2e7 logits per step on): everywhere but at fixed eps beyond
+    2.6e9 logits a step with more than 8 columns, where the first steps, which the general path runs
+    faster, weigh more than the others (60,000 x 40, 20 steps: 16.4 against 15.8 ms; 45,000 x 64: 11.2
+    against 11.2; 50,000 x 64, 100 steps: 24.5 against 32.2; 60,000 x 64, a schedule: 20.6 against 26.3).
     d <= 128, or early stopping on a schedule: the small kernels, which go over the logits once per
     side: up to 2e7 logits at fixed eps (3,000 x 128: 1.05 against 1.54 ms; 4,500: 2.8 against 2.4),
     6e7 on a schedule (6,500 x 128: 1.54 against 1.94 ms; 9,000: 3.1 against 2.8).
@@ -131,9 +126,7 @@ def _size_ok(n: int, m: int, d: int, fixed: bool, self_terms: int, stops: bool,
     if d > 64 or (stops and not fixed):
         logits = (n * m if self_terms < 2 else 0) + ((n * n + m * m) // 2 if self_terms else 0)
         return logits <= (20_000_000 if fixed else 60_000_000)
-    if d <= 8 or min(n, m) < 24000:
-        return True
-    return not fixed and d <= 32 and n * m <= 1_600_000_000
+    return d <= 8 or not fixed or n * m <= 2_600_000_000
 
 
 def _operands_ok(allow_tf32: bool) -> bool:
@@ -271,7 +264,8 @@ def pair_problem(x, y, a, b, allow_tf32: bool, fixed: bool, self_terms: int = 0,
             and x.shape[1] == y.shape[1]
             and (0 < x.shape[1] <= WIDE_D and max(x.shape[0], y.shape[0]) <= MAX_ROWS if any_size else
                  _size_ok(x.shape[0], y.shape[0], x.shape[1], fixed, self_terms, stops)
-                 # (a solver called by itself keeps to the tile-skipping kernels where it has them)
+                 # (a solver called by itself on two large clouds takes the same kernels, to the last bit,
+                 # whether it is asked for ``solve_info`` or not)
                  and (x.shape[1] <= 8 or min(x.shape[0], y.shape[0]) < 24000))
             and x.shape[0] > 0 and y.shape[0] > 0
             and a.shape[0] == x.shape[0] and b.shape[0] == y.shape[0]

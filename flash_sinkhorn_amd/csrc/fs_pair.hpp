@@ -74,7 +74,9 @@ struct PairProblem {
   int groups, chunks, chunk;  // 256-row groups of the stationary rows; chunks (of rows) of the others
   int self;                 // a matrix with itself: a group streams only rows at or behind its first
   float units;              // 32 x 32 units of all its work items; 0: every logit is computed
+  int ends;                 // two-sided steps may end units as well
   unsigned long long* list; // [items][n_items][wavefront][kPairListWords] units to visit
+  unsigned long long* two_list;  // [items][two_items][wavefront][kPairListWords] those that a two-sided step ran
   int n_items;              // work items of this problem
   // two-sided steps: (maximum, sum) per row and chunk of keys, and their work items (those of the
   // streamed rows' own half-update from two_first on; a self problem has none)
@@ -90,7 +92,6 @@ struct PairMode {
   int sweep;     // else two-sided with running maxima
   int list;      // only the units on the lists
   int coarse;    // units are ended by their coarse products where these allow it
-  int live;
   float low;     // log2 of every sum is above that
   float ratio;   // the next step's logits over this one's, where its eps is smaller
   float drift;   // with a list: what a logit may have risen by since it was made
@@ -184,6 +185,7 @@ __device__ __forceinline__ float pair_value(unsigned k) {
 // By every lane of a wavefront with the same result; `set`: which of the three sets to read.
 struct PairKnown {  // what pair_mode decides from: all loaded before anything is waited for
   float4 now, before, next, w, reach, list;
+  float twos;        // two-sided steps with coarse products so far
   unsigned ext, on;  // lane: [slot][which extreme]; units that went on, of slot lane % 8
 };
 __device__ __forceinline__ PairKnown pair_known(const PairArgs& a, int item, int prob, int step) {
@@ -195,6 +197,7 @@ __device__ __forceinline__ PairKnown pair_known(const PairArgs& a, int item, int
   k.reach = a.reach[item];
   const float* st = a.state + ((size_t)item * 3 + prob) * kPairStateWords;
   k.list = *reinterpret_cast<const float4*>(st + kPairLists + (step % 3) * 32);
+  k.twos = st[kPairLists + (step % 3) * 32 + 4];
   const unsigned* at = reinterpret_cast<const unsigned*>(st);
   const int set = (step + 2) % 3;
   k.ext = at[set * kPairSlots * 8 + (threadIdx.x & 63)];
@@ -202,13 +205,13 @@ __device__ __forceinline__ PairKnown pair_known(const PairArgs& a, int item, int
   __builtin_amdgcn_sched_barrier(0);
   return k;
 }
-__device__ __forceinline__ PairMode pair_mode(const PairKnown& k, float units, int prob, int step) {
+__device__ __forceinline__ PairMode pair_mode(const PairKnown& k, float units, bool ends, int prob, int step) {
   const float4 now = k.now, before = k.before, next = k.next, w = k.w, reach = k.reach;
   const float4 lim = prob == 0 ? w : (prob == 1 ? make_float4(w.x, w.y, w.x, w.y) : make_float4(w.z, w.w, w.z, w.w));
   const bool ok0 = (pair_scale(reach.x, now.y) == 0.f) & (now.w * reach.z < kPairMostBias);
   bool ok = ok0 & (lim.x > -1000.f) & (lim.z > -1000.f);
   PairMode mode;
-  mode.ratio = fmaxf(now.x / next.x, 1.f);
+  mode.ratio = next.x < now.x ? now.x * __builtin_amdgcn_rcpf(next.x) : 1.f;
   mode.coarse = mode.list = mode.two = 0;
   mode.rho = 1.f;
   mode.least[0] = mode.least[1] = 0.f;
@@ -218,7 +221,7 @@ __device__ __forceinline__ PairMode pair_mode(const PairKnown& k, float units, i
     mode.sweep = ok & (mode.low > -80.f);
     return mode;
   }
-  const float rho = before.x / now.x, kappa = now.w;
+  const float rho = before.x == now.x ? 1.f : before.x * __builtin_amdgcn_rcpf(now.x), kappa = now.w;
   static_assert(kPairSlots == 8, "a wavefront holds them");
   unsigned v = k.ext, on = k.on;
 #pragma unroll
@@ -231,7 +234,9 @@ __device__ __forceinline__ PairMode pair_mode(const PairKnown& k, float units, i
   for (int i = 0; i < 8; ++i) e[i] = pair_value((unsigned)__builtin_amdgcn_readlane((int)v, i));
   // (behind a two-sided step nothing is known: tried)
   mode.coarse = (float)on < kPairOn * units;
-  mode.two = ok0 && rho >= 1.f && (float)on < kPairTwoOn * units;
+  // (the first one finds the keys from which the next can tell what is far)
+  // (before the second step the potentials jump: nothing of the last one says what is far)
+  mode.two = ends && step >= 2 && ok0 && rho >= 1.f && (k.twos == 1.f || (float)on < kPairTwoOn * units);
   mode.rho = rho;
   mode.least[0] = -kappa * e[7];
   mode.least[1] = -kappa * e[3];
@@ -255,8 +260,9 @@ __device__ __forceinline__ PairMode pair_mode(const PairKnown& k, float units, i
   mode.drift = k.list.x + rise;
   mode.base = k.list.y;
   mode.list = ok && mode.coarse && k.list.z != 0.f && mode.base + mode.drift <= mode.low - kPairGap;
-  // (changes of the potentials shrink from step to step, to about a half where a plan is peaked)
-  mode.reserve = next.x == now.x ? fminf(16.f + 3.f * fmaxf(rise, 0.f), 256.f) : 0.f;
+  // (changes of the potentials shrink from step to step, at first to about a half where a plan is peaked, slowly
+  // later: a list that reaches further costs its steps 0.28 us a unit, a new one 320 us, at 50,000 x 64)
+  mode.reserve = next.x == now.x ? fminf(16.f + 24.f * __builtin_amdgcn_sqrtf(fmaxf(rise, 0.f)), 256.f) : 0.f;
   return mode;
 }
 
@@ -567,6 +573,7 @@ __device__ __forceinline__ unsigned pair_item_two_coarse(const PairArgs& a, int 
   using S = PairStream<DP, false>;
   constexpr int KK = DP / 16;
   const int side = it >= pr.two_first ? 1 : 0;  // the streamed rows' own half-update
+  unsigned long long* put = pr.two_list + ((size_t)batch * pr.two_items + it) * (4 * kPairListWords);
   if (side) it -= pr.two_first;
   const PairSide& sd = a.side[prob == 0 ? side : 1 + prob];
   const int n_k = side ? pr.n_st : pr.n_str, n_q = side ? pr.n_str : pr.n_st;
@@ -603,12 +610,12 @@ __device__ __forceinline__ unsigned pair_item_two_coarse(const PairArgs& a, int 
     on_at[rb] = row < n_q ? low - kPairGap - cross : 3.0e38f;
   }
   const unsigned one = 0x3c00u, s1 = 0x6c00u, s2 = 0x3c00u, s3 = 0x0c00u;  // fp16 1, 2^12, 1, 2^-12
-  // the key's bias alone, with its share of the bound, and that share taken off again
-  u32x4 qb = {0u, s1 << 16, s2 | s3 << 16, one}, qoff = {0u, 0u, 0u, one | 0x8000u};
-  if (h) qb = qoff = u32x4{0u, 0u, 0u, 0u};
+  // the key's bias with its share of the bound, and without
+  u32x4 qb = {0u, s1 << 16, s2 | s3 << 16, one}, qexact = {0u, s1 << 16, s2 | s3 << 16, 0u};
+  if (h) qb = qexact = u32x4{0u, 0u, 0u, 0u};
   u32x4 y[KK], yb;
   f32x16 acc[2][2];  // [parity of the sub-tile][row block]
-  unsigned went_on = 0;
+  unsigned long long list[2][2] = {{0ull, 0ull}, {0ull, 0ull}};  // [row block][half of the sub-tiles]
   auto read_key = [&](int k, int buf, int js) {
     if (k < KK) y[k] = S::read(&lds[buf * S::BUF + (js * (2 * KK) + k) * 64 + lane]);
     else yb = S::read(&lds[buf * S::BUF + S::PIECES * 64 + js * 32 + li]);
@@ -647,6 +654,11 @@ __device__ __forceinline__ unsigned pair_item_two_coarse(const PairArgs& a, int 
     const int js = sub & 1;
     const bool on0 = wave_any(mx[0] > on_at[0]), on1 = wave_any(mx[1] > on_at[1]);
     if (!(on0 || on1)) return;
+    const unsigned long long bit = 1ull << (sub & 63);
+    list[0][0] |= on0 && sub < 64 ? bit : 0ull;
+    list[0][1] |= on0 && sub >= 64 ? bit : 0ull;
+    list[1][0] |= on1 && sub < 64 ? bit : 0ull;
+    list[1][1] |= on1 && sub >= 64 ? bit : 0ull;
     u32x4 z[2][KK], zb;
 #pragma unroll
     for (int q = 1; q >= 0; --q)
@@ -657,12 +669,17 @@ __device__ __forceinline__ unsigned pair_item_two_coarse(const PairArgs& a, int 
 #pragma unroll
     for (int rb = 0; rb < 2; ++rb) {
       if (rb ? !on1 : !on0) continue;
-      ++went_on;
-      f32x16 c = small_mfma(zb, qoff, acc[of][rb]);
+      // (anew, from the lowest weight to the bias: fewest roundings at the size of the whole)
+      f32x16 c;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) c[r] = 0.f;
 #pragma unroll
       for (int kk = 0; kk < KK; ++kk) c = small_mfma(z[1][kk], x[rb][0][kk], c);
 #pragma unroll
       for (int kk = 0; kk < KK; ++kk) c = small_mfma(z[0][kk], x[rb][1][kk], c);
+#pragma unroll
+      for (int kk = 0; kk < KK; ++kk) c = small_mfma(z[0][kk], x[rb][0][kk], c);
+      c = small_mfma(zb, qexact, c);
       const float top = small_max16(c[0], c);
       if (wave_any(top > m[rb])) {
         if (top > m[rb]) {
@@ -726,7 +743,9 @@ __device__ __forceinline__ unsigned pair_item_two_coarse(const PairArgs& a, int 
       keys[row] = bo >= 0 && (mo > m[rb] || best[rb] < 0) ? bo : best[rb];
     }
   }
-  return went_on;
+  if (lane < kPairListWords)
+    put[ks.wave * kPairListWords + lane] = lane < 2 ? (lane ? list[0][1] : list[0][0]) : (lane == 3 ? list[1][1] : list[1][0]);
+  return __popcll(list[0][0]) + __popcll(list[0][1]) + __popcll(list[1][0]) + __popcll(list[1][1]);
 }
 
 // What a work item of the one-sweep forms is: 256 stationary rows against a chunk of streamed ones.
@@ -830,7 +849,7 @@ __device__ __forceinline__ void pair_put_rows(const PairProblem& pr, int batch, 
 // it ends there unless hi * hi + biases + the bound on the cross products reaches that line.  What
 // is left out is below 2^-28 of any sum even with 65,536 terms.  The products of a sub-tile's two
 // units go to the matrix pipe while the units of the sub-tile before are tested between them in program order;
-// those that go on then add their cross products and take their exponentials, with the streamed
+// those that go on then take all of their products and their exponentials, with the streamed
 // operands read again from LDS.  No accumulator and no LDS read on its way crosses the branch.
 //
 // The tiles of all items run through one ring of four buffers, three ahead, across the ends of items:
@@ -948,20 +967,27 @@ __device__ __forceinline__ int pair_run_coarse(const PairArgs& a, int batch, Pai
       list[0][1] |= on0 && sub >= 64 ? bit : 0ull;
       list[1][0] |= on1 && sub < 64 ? bit : 0ull;
       list[1][1] |= on1 && sub >= 64 ? bit : 0ull;
-      u32x4 z[2][KK];
+      u32x4 z[2][KK], zb;
 #pragma unroll
       for (int q = 1; q >= 0; --q)
 #pragma unroll
         for (int kk = 0; kk < KK; ++kk) z[q][kk] = S::read(&lds[buf * S::BUF + (js * (2 * KK) + q * KK + kk) * 64 + lane]);
+      zb = S::read(&lds[buf * S::BUF + S::PIECES * 64 + js * 32 + li]);
       wait_reads();
 #pragma unroll
       for (int rb = 0; rb < 2; ++rb) {
         if (rb ? !on1 : !on0) continue;
-        f32x16 c = acc[of][rb];
+        // (anew, from the lowest weight on, to the same bits as the plain form and the gradient)
+        f32x16 c;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) c[r] = 0.f;
 #pragma unroll
         for (int kk = 0; kk < KK; ++kk) c = small_mfma(xa[rb][0][kk], z[1][kk], c);
 #pragma unroll
         for (int kk = 0; kk < KK; ++kk) c = small_mfma(xa[rb][1][kk], z[0][kk], c);
+#pragma unroll
+        for (int kk = 0; kk < KK; ++kk) c = small_mfma(xa[rb][0][kk], z[0][kk], c);
+        c = small_mfma(xb[rb], zb, c);
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const float e = fast_exp2(c[r]);
@@ -1129,12 +1155,12 @@ __device__ __forceinline__ int pair_run_list(const PairArgs& a, int batch, PairW
 #pragma unroll
           for (int r = 0; r < 16; ++r) c[r] = 0.f;
 #pragma unroll
-          for (int kk = 0; kk < KK; ++kk) c = small_mfma(xa[rb][0][kk], k.p[0][kk], c);
-          c = small_mfma(xb[rb], k.b, c);
-#pragma unroll
           for (int kk = 0; kk < KK; ++kk) c = small_mfma(xa[rb][0][kk], k.p[1][kk], c);
 #pragma unroll
           for (int kk = 0; kk < KK; ++kk) c = small_mfma(xa[rb][1][kk], k.p[0][kk], c);
+#pragma unroll
+          for (int kk = 0; kk < KK; ++kk) c = small_mfma(xa[rb][0][kk], k.p[0][kk], c);
+          c = small_mfma(xb[rb], k.b, c);
 #pragma unroll
           for (int r = 0; r < 16; ++r) {
             const float e = fast_exp2(c[r]);
@@ -1310,7 +1336,7 @@ __device__ __forceinline__ void pair_item_plain(const PairProblem& pr, int batch
     // this unit says for all of the wavefront's whether the coarse test of the next step would end them
     // (its logits and cross products are about `ratio` times these, the streamed rows' share of the
     // latter about that of the others)
-    if (wave_any((mx + 2.0f * cross) * mode.ratio > mode.low - kPairGap) && lane == 0) atomicAdd(went, 4u * (unsigned)ntiles);
+    if (went != nullptr && wave_any((mx + 2.0f * cross) * mode.ratio > mode.low - mode.reserve - kPairGap) && lane == 0) atomicAdd(went, 4u * (unsigned)ntiles);
   }
   S::wait_all();  // (also what was fetched past the chunk)
   __syncthreads();
@@ -1333,36 +1359,40 @@ __global__ __launch_bounds__(256, 2) void pair_sweep_kernel(PairArgsPtr args, in
   __shared__ PairMode modes[3];
   __shared__ unsigned went[3];                  // units that went on
   __shared__ int next_item[2];
+  __shared__ __attribute__((aligned(16))) unsigned mode_bits[4];
 
   const int batch = blockIdx.y, lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int xcd = blockIdx.x & 7, mine = blockIdx.x >> 3, stride = gridDim.x >> 3, count = a.per_xcd;
   const PairWork work = (PairWork)(a.work + xcd * count);
   PairWord word = work[mine];
-  if (wave >= a.first_prob && wave < a.nprob) {
-    PairMode m = pair_mode(pair_known(a, batch, wave, step), a.prob[wave].units, wave, step);
+  // The modes: of a single problem by every wavefront for itself, without a barrier (what they write to LDS for
+  // later is the same), of three by one wavefront each.
+  const bool single = a.nprob - a.first_prob == 1;
+  const int own = single ? a.first_prob : max(min(wave, a.nprob - 1), a.first_prob);
+  unsigned bits;
+  {
+    const PairKnown known = pair_known(a, batch, own, step);
+    const int entries = a.lens[batch * 3 + own];
+    const PairMode m = pair_mode(known, SKIP ? a.prob[own].units : 0.f, SKIP && a.prob[own].ends, own, step);
     // (where its schedule is shorter nothing is done)
-    m.live = step <= a.lens[batch * 3 + wave] + a.extrapolate;
-    if (lane == 0) {
-      modes[wave] = m;
-      went[wave] = 0u;
-    }
+    const bool live = step <= entries + a.extrapolate;
+    bits = (live ? 1u : 0u) | (live && m.sweep ? 8u : 0u);
+    if (SKIP)
+      bits |= (live && m.sweep && m.coarse && !m.list ? 64u : 0u) | (live && m.list ? 512u : 0u) | (m.two ? 4096u : 0u);
+    bits <<= own;
+    if (lane == 0 && (single || own == wave)) modes[own] = m;
+    if (threadIdx.x < 3) went[threadIdx.x] = 0u;
   }
-  __syncthreads();
-  unsigned live = 0, sweep = 0, coarse = 0, list = 0, ends = 0;  // bit p: problem p
-  for (int p = a.first_prob; p < a.nprob; ++p) {
-    live |= modes[p].live ? 1u << p : 0u;
-    sweep |= modes[p].sweep ? 1u << p : 0u;
-    coarse |= SKIP && modes[p].live && modes[p].sweep && modes[p].coarse ? 1u << p : 0u;
-    list |= SKIP && modes[p].live && modes[p].list ? 1u << p : 0u;
+  if (!single) {
+    if (lane == 0) mode_bits[wave] = own == wave ? bits : 0u;
+    __syncthreads();
+    const uint4 all = *reinterpret_cast<const uint4*>(mode_bits);
+    bits = all.x | all.y | all.z | all.w;
   }
-  for (int p = a.first_prob; p < a.nprob; ++p) ends |= SKIP && modes[p].two ? 1u << p : 0u;
-  ends = __builtin_amdgcn_readfirstlane(ends);
-  live = __builtin_amdgcn_readfirstlane(live);
-  sweep = __builtin_amdgcn_readfirstlane(sweep);
-  coarse = __builtin_amdgcn_readfirstlane(coarse);
-  list = __builtin_amdgcn_readfirstlane(list);
-  coarse &= ~list;
+  bits = __builtin_amdgcn_readfirstlane(bits);
+  // (bit p: problem p)
+  const unsigned live = bits & 7u, sweep = bits >> 3 & 7u, coarse = bits >> 6 & 7u, list = bits >> 9 & 7u, ends = bits >> 12 & 7u;
   // (items of these forms take long and are all alike: whoever is free takes the next)
   int* taken = reinterpret_cast<int*>(a.state) + (size_t)batch * 3 * kPairStateWords + kPairTaken + ((step % 3) * 8 + xcd) * 32;
   int turn = 0;
@@ -1383,7 +1413,7 @@ __global__ __launch_bounds__(256, 2) void pair_sweep_kernel(PairArgsPtr args, in
       k = __builtin_amdgcn_readfirstlane(next_item[turn & 1]);
     }
   }
-  const bool fetch = (live & sweep & (coarse | list)) == 0;
+  const bool fetch = (coarse | list) == 0 && count > stride;
   for (int i = mine; i < count;) {
     const PairItem t = pair_item(word);
     if (t.prob < 0 || !((live & sweep) >> t.prob & 1)) {
@@ -1394,12 +1424,13 @@ __global__ __launch_bounds__(256, 2) void pair_sweep_kernel(PairArgsPtr args, in
       i = pair_run_coarse<DP>(a, batch, work, i, stride, count, coarse, modes, went, lds, &lds_col[0][0][0][0]);
     } else {
       if (fetch && threadIdx.x == 0) next_item[turn & 1] = stride + atomicAdd(taken + a.first_prob * kPairStateWords + 1, 1);
-      pair_item_plain<DP>(a.prob[t.prob], batch, t, modes[t.prob], &went[t.prob], lds, &lds_col[0][0][0][0]);
+      pair_item_plain<DP>(a.prob[t.prob], batch, t, modes[t.prob], SKIP ? &went[t.prob] : nullptr, lds, &lds_col[0][0][0][0]);
       i = fetch ? __builtin_amdgcn_readfirstlane(next_item[turn & 1]) : i + stride;
       ++turn;
     }
-    word = work[min(i, count - 1)];
+    if (i < count) word = work[i];
   }
+  if (!SKIP) return;
   __syncthreads();
   if (threadIdx.x >= a.first_prob && threadIdx.x < a.nprob && went[threadIdx.x])
     atomicAdd(reinterpret_cast<unsigned*>(a.state) + ((size_t)batch * 3 + threadIdx.x) * kPairStateWords + kPairCounts +
@@ -1453,7 +1484,7 @@ __device__ __forceinline__ void pair_write_planes(u32x4* out, const void* pts, s
 // cloud; sides; items).  Bound by memory latency: four wavefronts share the partial sums of 64 rows.  The
 // extremes are combined in the workgroup first: with an atomic maximum per 64 rows a merge took
 // 13.6 us at 10,000 points, debiased, half of it for them.
-template <int DP>
+template <int DP, bool SKIP>
 __global__ __launch_bounds__(1024) void pair_merge_kernel(PairArgsPtr args, int step, int plane_groups) {
   const PairArgs& a = *(const PairArgs*)args;
   const int side = blockIdx.y + (a.first_prob ? 2 : 0), item = blockIdx.z, tid = threadIdx.x;
@@ -1497,18 +1528,25 @@ __global__ __launch_bounds__(1024) void pair_merge_kernel(PairArgsPtr args, int 
   if (step < 0) {
     if (part > 0) return;
     // (nothing is known of the sums yet)
-    if (live) sd.key[at] = -1;
+    if (SKIP && live) sd.key[at] = -1;
     if (blockIdx.x == 0 && quarter == 0 && (side == 0 || side >= 2))
       for (int i = lane; i < kPairStateWords; i += 64) state[i] = 0u;
   } else {
     __shared__ float2 sh[4][4][64];
-    __shared__ int sh_best[4][4][64];
-    __shared__ float sh_dot[4][4][64];
+    __shared__ int sh_best[4][4][SKIP ? 64 : 1];
+    __shared__ float sh_dot[4][4][SKIP ? 64 : 1];
     __shared__ float sh_ex[4][4];
     const float4 coef = known.now;
     const float r = __builtin_fmaf(coef.w, old, l2w);  // the row's bias in this step
-    const PairMode mode = pair_mode(known, a.prob[prob].units, prob, step);
-    const bool sweep = mode.sweep;
+    // (one wavefront decides for all: sixteen would take a SIMD's turns from each other)
+    __shared__ PairMode sh_mode;
+    if (wave == 0) {
+      const PairMode m = pair_mode(known, SKIP ? a.prob[prob].units : 0.f, SKIP && a.prob[prob].ends, prob, step);
+      if (lane == 0) sh_mode = m;
+    }
+    __syncthreads();
+    const PairMode mode = sh_mode;
+    const bool sweep = __builtin_amdgcn_readfirstlane(mode.sweep), ended = __builtin_amdgcn_readfirstlane(mode.two);
     float2 mine = make_float2(kNegBig, 0.f);
     int best = -1;
     const int rc = min(row, sd.rows - 1);
@@ -1534,22 +1572,25 @@ __global__ __launch_bounds__(1024) void pair_merge_kernel(PairArgsPtr args, int 
 #pragma unroll 8
       for (int c = part; c < sd.ms_parts; c += 4) {
         const float2 v = p[(size_t)c * sd.rows];
-        const int k = mode.two ? q[(size_t)c * sd.rows] : -1;
+        const int k = SKIP && ended ? q[(size_t)c * sd.rows] : -1;
         const float M = fmaxf(mine.x, v.x);
         mine.y = mine.y * fast_exp2(mine.x - M) + v.y * fast_exp2(v.x - M);
         mine.x = M;
         best = k >= 0 && v.x > most ? k : best;
         most = k >= 0 ? fmaxf(most, v.x) : most;
       }
-      sh_best[quarter][part][lane] = best;
+      if (SKIP) sh_best[quarter][part][lane] = best;
     }
-    if (blockIdx.x == 0 && (side == 0 || side >= 2) && tid == 0) {
+    if (SKIP && blockIdx.x == 0 && (side == 0 || side >= 2) && tid == 0) {
       // (what the next step knows of the lists)
       float* out = a.state + ((size_t)item * 3 + prob) * kPairStateWords + kPairLists + ((step + 1) % 3) * 32;
       const bool made = sweep && mode.coarse && !mode.list;
       out[0] = mode.list ? mode.drift : 0.f;
       out[1] = mode.list ? mode.base : mode.low - kPairGap - mode.reserve;
       out[2] = next.x == coef.x && (made || mode.list) ? 1.f : 0.f;
+      // (for the gradient: whose lists hold the units of this step, the one-sweep or the two-sided form's)
+      out[4] = known.twos + (!sweep && mode.two ? 1.f : 0.f);
+      out[3] = made || mode.list ? 1.f : (!sweep && mode.two ? 2.f : 0.f);
     }
     sh[quarter][part][lane] = mine;
     __syncthreads();
@@ -1565,7 +1606,7 @@ __global__ __launch_bounds__(1024) void pair_merge_kernel(PairArgsPtr args, int 
       for (int w = 0; w < 4; ++w) s += all[w][lane].y * fast_exp2(all[w][lane].x - M);
       lse = small_log2(fmaxf(s, 1e-40f), M + others);
     }
-    if (!sweep && mode.two) {
+    if (SKIP && !sweep && ended) {
       // the key of the largest logit that any chunk has seen beyond where it began, the pair's inner product
       const float2(&ms)[4][64] = sh[quarter];
       float most = kNegBig;
@@ -1599,7 +1640,7 @@ __global__ __launch_bounds__(1024) void pair_merge_kernel(PairArgsPtr args, int 
     float ex[4] = {-3.0e38f, -3.0e38f, -3.0e38f, -3.0e38f};
     if (live && part == 0) {
       sd.pot[(from ^ 1) * (size_t)a.items * sd.rows + at] = f;
-      sd.sum2[at] = lse - others;
+      if (SKIP) sd.sum2[at] = lse - others;
       const float x = __builtin_fmaf(coef.w, old, lse), df = f - old;
       ex[0] = x; ex[1] = -x; ex[2] = df; ex[3] = -df;
       if (!(x == x) || !(df == df) || !(fabsf(next.w * f) < kPairMostBias)) ex[0] = ex[1] = ex[2] = ex[3] = 3.0e38f;
@@ -1636,5 +1677,62 @@ __global__ __launch_bounds__(1024) void pair_merge_kernel(PairArgsPtr args, int 
   sd.bias[(size_t)item * sd.blocks * 32 + row] = pair_bias(fmaxf(b, kPairFar), fminf(cross, 60000.f));
   sd.bias32[(size_t)item * sd.blocks * 32 + row] = b;
 }
+
+// The key blocks (32 keys) that matter to a block of 32 query rows of the gradient: those whose unit the
+// extrapolation, which read the same potentials, did not end.  By a workgroup of 512 threads; as many blocks
+// as it returns are in `ids`, in their order (-1: that step computed every logit).
+struct PairBlocks {
+  static constexpr int kMost = 2048;
+  PairArgsPtr args;
+  int extrapolate;
+  __device__ __forceinline__ int find(int item, int prob, int qm, int qb, int nkb, unsigned short* ids) const {
+    const PairArgs& a = *(const PairArgs*)args;
+    const PairProblem& pr = a.prob[prob];
+    const int step = a.lens[item * 3 + prob] + 1;
+    const float kind = a.state[((size_t)item * 3 + prob) * kPairStateWords + kPairLists + ((step + 1) % 3) * 32 + 3];
+    if (!extrapolate || kind == 0.f || pr.units == 0.f) return -1;
+    const bool two = kind == 2.f;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int per = pr.chunk / 32;  // blocks of a chunk
+    const int side = prob == 0 && qm == 1 ? 1 : 0;
+    __shared__ unsigned long long mask[kMost / 64];
+    __syncthreads();
+    for (int seg = wave; seg * 64 < nkb; seg += 8) {
+      const int kb = seg * 64 + lane;
+      bool on = false;
+      if (kb < nkb) {
+        // stationary and streamed block of the unit
+        const bool turned = two ? false : (pr.self ? kb / 8 < qb / 8 : side == 1);
+        const int st = turned ? kb : qb, str = turned ? qb : kb, group = st / 8;
+        const int chunk = str / per;
+        int first = chunk * per, index;
+        if (two) {
+          index = (side ? pr.two_first : 0) + chunk * (((side ? pr.n_str : pr.n_st) + 255) / 256) + group;
+        } else if (pr.self) {
+          index = group;
+          for (int c = 0; c < chunk; ++c) index += self_groups_of_chunk(c, pr.chunk, pr.n_str, pr.groups);
+          first = max(first, group * 8);
+        } else {
+          index = chunk * pr.groups + group;
+        }
+        const int sub = str - first;
+        const unsigned long long* w = two ? pr.two_list + (size_t)item * pr.two_items * (4 * kPairListWords)
+                                          : pr.list + (size_t)item * pr.n_items * (4 * kPairListWords);
+        on = (w[((size_t)index * 4 + (st & 7) / 2) * kPairListWords + (st & 1) * 2 + (sub >> 6)] >> (sub & 63)) & 1;
+      }
+      const unsigned long long m = __builtin_amdgcn_ballot_w64(on);
+      if (lane == 0) mask[seg] = m;
+    }
+    __syncthreads();
+    int count = 0;
+    for (int seg = 0; seg * 64 < nkb; ++seg) {
+      const unsigned long long m = mask[seg];
+      if (wave == (seg & 7) && ((m >> lane) & 1)) ids[count + __popcll(m & ((1ull << lane) - 1))] = (unsigned short)(seg * 64 + lane);
+      count += __popcll(m);
+    }
+    __syncthreads();
+    return __builtin_amdgcn_readfirstlane(count);
+  }
+};
 
 }  // namespace fs

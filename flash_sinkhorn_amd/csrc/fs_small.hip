@@ -111,6 +111,9 @@ void plan_pair(const SmallArgs& a, PairArgs& t) {
     pr.st_blocks = a.pblocks[s];
     pr.str_blocks = a.pblocks[k];
     pr.groups = (pr.n_st + 255) / 256;
+    // (a row's few units are a smaller share the more there are: at 4,500 x 64 such a step takes as long as
+    // one that computes everything and its merge 5 us longer, at 10,000 x 64 62 against 92 us)
+    pr.ends = skips(a.d) && (double)pr.n_st * pr.n_str >= 6.0e7;
     pr.units = 0.f;
     for (int g = 0; g < pr.groups && skips(a.d); ++g) pr.units += 16.f * (float)((pr.n_str - (pr.self ? 256 * g : 0) + 63) / 64);
   }
@@ -300,6 +303,7 @@ size_t layout(const fs_small_problem* p, void* ws, SmallArgs& a, PairArgs* pa = 
       take(pr.st_part, items * (size_t)pr.chunks * (size_t)pr.n_st * 4);
       take(pr.str_part, items * (size_t)pr.groups * (size_t)pr.n_str * 4);
       take(pr.list, items * (size_t)pr.n_items * (4 * kPairListWords * 8));
+      take(pr.two_list, items * (size_t)pr.two_items * (4 * kPairListWords * 8));
       take(pr.st_ms, items * (size_t)pr.chunks * (size_t)pr.n_st * sizeof(float2));
       take(pr.st_best, items * (size_t)pr.chunks * (size_t)pr.n_st * 4);
       if (!pr.self) {
@@ -409,7 +413,8 @@ int launch_pair_merge(const SmallArgs& a, const PairArgs& t, PairArgs* at, int s
   // (at one eps the planes are written once, before the first step)
   const int planes = step < 0 || a.sched != 0 ? (blocks + 3) / 4 : 0;
   const int grid = t.merge_groups + planes + (step < 0 ? (8 * t.per_xcd + 1023) / 1024 : 0);
-  hipLaunchKernelGGL((pair_merge_kernel<DP>), dim3(grid, a.self == 1 ? 4 : 2, a.items), dim3(1024), 0, st,
+  const auto kernel = DP > 16 || skips(a.d) ? pair_merge_kernel<DP, true> : pair_merge_kernel<DP, DP != 16>;
+  hipLaunchKernelGGL(kernel, dim3(grid, a.self == 1 ? 4 : 2, a.items), dim3(1024), 0, st,
                      (PairArgsPtr)at, step, planes);
   return hipGetLastError() == hipSuccess ? FS_OK : FS_ERR_LAUNCH_FAILED;
 }
@@ -423,10 +428,16 @@ int launch_pair_step(const SmallArgs& a, const PairArgs& t, PairArgs* at, int st
 }
 
 template <int DP>
-int launch_grad(const SmallArgs& a, const SmallGradArgs& g, hipStream_t st) {
+int launch_grad(const SmallArgs& a, const SmallGradArgs& g, PairArgs* pair_at, hipStream_t st) {
   const int xb = a.blocks[0] > a.blocks[1] ? a.blocks[0] : a.blocks[1];
   const dim3 grid(!g.out[0] ? a.blocks[1] : (!g.out[1] ? a.blocks[0] : xb), g.out[0] && g.out[1] ? 2 : 1, a.items);
-  hipLaunchKernelGGL((small_grad_kernel<DP>), grid, dim3(512), 0, st, a, g);
+  if constexpr (DP <= 64)
+    if (a.pair && skips(a.d)) {
+      hipLaunchKernelGGL((small_grad_kernel<DP, PairBlocks>), grid, dim3(512), 0, st, a, g,
+                         (PairBlocks{(PairArgsPtr)pair_at, a.extrapolate}));
+      return hipGetLastError() == hipSuccess ? FS_OK : FS_ERR_LAUNCH_FAILED;
+    }
+  hipLaunchKernelGGL((small_grad_kernel<DP, SmallAllBlocks>), grid, dim3(512), 0, st, a, g, SmallAllBlocks{});
   return hipGetLastError() == hipSuccess ? FS_OK : FS_ERR_LAUNCH_FAILED;
 }
 
@@ -597,13 +608,14 @@ int fs_small_grad(const fs_small_problem* p, void* workspace, size_t workspace_b
   if (!grad_out) return FS_ERR_NULL_POINTER;
   if (!p->want_values) return FS_ERR_BAD_ARGUMENT;
   SmallArgs a;
-  if (layout(p, workspace, a) > workspace_bytes || !workspace) return FS_ERR_WORKSPACE_TOO_SMALL;
+  PairArgs* pair_at = nullptr;
+  if (layout(p, workspace, a, nullptr, nullptr, &pair_at) > workspace_bytes || !workspace) return FS_ERR_WORKSPACE_TOO_SMALL;
   if (!grad_x && !grad_y) return FS_OK;
   SmallGradArgs g;
   g.grad_out = grad_out;
   g.out[0] = grad_x;
   g.out[1] = grad_y;
-  return by_width(p->d, [&](auto dp) { return launch_grad<decltype(dp)::value>(a, g, (hipStream_t)stream); });
+  return by_width(p->d, [&](auto dp) { return launch_grad<decltype(dp)::value>(a, g, pair_at, (hipStream_t)stream); });
 }
 
 }  // extern "C"

@@ -726,13 +726,20 @@ struct SmallGradArgs {
   float* out[2];          // [items, rows, d] or null
 };
 
-template <int DP>
-__global__ __launch_bounds__(512, 2) void small_grad_kernel(const SmallArgs a, const SmallGradArgs g) {
+// The key blocks that matter to a block of query rows, where the solve has kept that (fs_pair.hpp).
+struct SmallAllBlocks {
+  static constexpr int kMost = 1;
+  __device__ __forceinline__ int find(int, int, int, int, int, unsigned short*) const { return -1; }
+};
+
+template <int DP, typename Lists>
+__global__ __launch_bounds__(512, 2) void small_grad_kernel(const SmallArgs a, const SmallGradArgs g, const Lists lists) {
   constexpr int KK = DP / 16, NDB = (DP + 31) / 32, W = 8;
   constexpr int LDW = NDB * 32 + 4;                 // padded row of a wavefront's partial output
   constexpr int PER = NDB * 32 * 32 / 512;          // outputs per thread
   __shared__ __attribute__((aligned(16))) float sh_o[W][32 * LDW];
   __shared__ float2 sh_ms[W][32];
+  __shared__ unsigned short sh_blocks[Lists::kMost];
   const int rb = blockIdx.x, item = blockIdx.z, tid = threadIdx.x;
   const int qm = g.out[0] == nullptr ? 1 : blockIdx.y;
   if (rb >= a.blocks[qm]) return;
@@ -786,12 +793,16 @@ __global__ __launch_bounds__(512, 2) void small_grad_kernel(const SmallArgs a, c
     for (int cb = 0; cb < NDB; ++cb)
 #pragma unroll
       for (int r = 0; r < 16; ++r) o[cb][r] = 0.f;
+    const int found = lists.find(item, prob, qm, rb, nkb, sh_blocks);  // (with barriers, or -1: all of them)
+    const int count = found < 0 ? nkb : found;
+    auto block_at = [&](int i) { return found < 0 ? i : (int)sh_blocks[min(i, count - 1)]; };
     SmallKeys<KK> kr;
-    ks.load(kr, wave);
-    for (int blk = wave; blk < nkb; blk += W) {
+    if (wave < count) ks.load(kr, block_at(wave));
+    for (int i = wave; i < count; i += W) {
+      const int blk = __builtin_amdgcn_readfirstlane(block_at(i));
       const u32x4* v = vp + (size_t)blk * (NDB * 4 * 64);
       const f32x16 acc = ks.logits(kr, q, blk);
-      if (blk + W < nkb) ks.load(kr, blk + W);
+      if (i + W < count) ks.load(kr, block_at(i + W));
       // the two half-waves of a column feed one sum: they share its maximum
       float mx = small_max16(ks.masked, acc) * lscale;
       mx = fmaxf(mx, xor32(mx));

@@ -314,14 +314,17 @@ def gradient_bound(x, y, eps):
     return 2.0 * delta * (nx + ny)
 
 
-@pytest.mark.parametrize("n,m,d,eps", [(4500, 4470, 64, 0.01), (5003, 4201, 9, 0.003)])
-def test_one_sweep_gradients_at_small_eps(n, m, d, eps):
+# (6 steps end in a two-sided one, 25 in one that goes along its lists)
+@pytest.mark.parametrize("n,m,d,eps,n_iters", [(4500, 4470, 64, 0.01, 6), (5003, 4201, 9, 0.003, 6),
+                                               (4513, 4490, 64, 0.01, 25), (310, 65000, 33, 0.01, 25),
+                                               (65000, 290, 16, 0.003, 25)])
+def test_one_sweep_gradients_at_small_eps(n, m, d, eps, n_iters):
     from flash_sinkhorn_amd import SamplesLoss
     from flash_sinkhorn_amd.kernels import sinkhorn_flashstyle_symmetric as solve
     x, y, a, b = inputs(n, n, m, d, scale=0.5, y_shift=0.2)
     X, Y, A, B = dev(x, y, a, b)
     X.requires_grad_(), Y.requires_grad_()
-    kw = dict(use_epsilon_scaling=False, eps=eps, n_iters=6)
+    kw = dict(use_epsilon_scaling=False, eps=eps, n_iters=n_iters)
     gx, gy = torch.autograd.grad(SamplesLoss("sinkhorn", normalize=False, **kw)(A, X, B, Y), [X, Y])
     # at the potentials of the same solve: what is left is the gradient's own error
     _, _, fp, gp = solve(X.detach(), Y.detach(), A, B, return_prelast=True, **kw)
@@ -330,6 +333,30 @@ def test_one_sweep_gradients_at_small_eps(n, m, d, eps):
     for got, want, w in ((gx, wx, a), (gy, wy, b)):
         off = np.abs(got.cpu().numpy() - want).max(axis=1)
         assert (off <= 2.0 * w * bound).all()
+
+
+def test_one_sweep_gradients_of_peaked_self_problems():
+    from flash_sinkhorn_amd import SamplesLoss
+    from flash_sinkhorn_amd.kernels import sinkhorn_flashstyle_symmetric as solve
+    from flash_sinkhorn_amd.sinkhorn_solvers import sinkhorn_flashstyle_symmetric_self_pair as pair
+    n, m, d, eps = 3313, 3190, 20, 0.02
+    x, y, a, b = inputs(n, n, m, d, scale=0.5, y_shift=0.2)
+    x[1::2] = x[:-1:2] + 0.02 * x[1::2]  # (a point's own weight is not all of its row)
+    X, Y, A, B = dev(x, y, a, b)
+    X.requires_grad_(), Y.requires_grad_()
+    kw = dict(use_epsilon_scaling=False, eps=eps, n_iters=25)
+    gx, gy = torch.autograd.grad(SamplesLoss("sinkhorn", normalize=False, debias=True, **kw)(A, X, B, Y), [X, Y])
+    X, Y = X.detach(), Y.detach()
+    _, _, fp, gp = (t.cpu().numpy() for t in solve(X, Y, A, B, return_prelast=True, **kw))
+    (_, _, fx, _), (_, _, fy, _) = pair(X, A, Y, B, return_prelast=True, **kw)
+    fx, fy = fx.cpu().numpy(), fy.cpu().numpy()
+    wx, wy = oracle.grad_barycentric(x, y, a, b, fp, gp, eps)
+    # (a self problem has its gradient once for either role of the points, and is taken off by half)
+    wx = wx - oracle.grad_barycentric(x, x, a, a, fx, fx, eps)[0]
+    wy = wy - oracle.grad_barycentric(y, y, b, b, fy, fy, eps)[0]
+    for got, want, w, (u, v) in ((gx, wx, a, (x, x)), (gy, wy, b, (y, y))):
+        off = np.abs(got.cpu().numpy() - want).max(axis=1)
+        assert (off <= 2.0 * w * (gradient_bound(x, y, eps) + gradient_bound(u, v, eps))).all()
 
 
 def test_one_sweep_debiased_schedule():
