@@ -565,7 +565,8 @@ __device__ __forceinline__ void pair_item_two_sided(const PairArgs& a, int batch
 // larger of two: the last step's sum, less what the potentials of the keys may have fallen by (with eps' <
 // eps and rho = eps / eps', power means give rho times the old logarithm less (rho - 1) log2 of the
 // weights' sum, which counts them from the largest), and the row's logit at the key that held its
-// largest when a step last saw it (pair_merge_kernel keeps the two points' inner product).  A lane holds
+// largest when a step last saw it (pair_merge_kernel keeps the two points' inner product).  The running
+// maximum starts there, so that every larger logit that is found raises the line.  A lane holds
 // one query row and 16 keys, the key's bias and its share of the bound ride in the matrix product.
 template <int DP>
 __device__ __forceinline__ unsigned pair_item_two_coarse(const PairArgs& a, int batch, const PairProblem& pr, int prob,
@@ -592,7 +593,7 @@ __device__ __forceinline__ unsigned pair_item_two_coarse(const PairArgs& a, int 
   ks.stage(2, 2);
   u32x4 x[2][2][KK];
   pair_load_rows(x, (side ? pr.str_planes : pr.st_planes) + ((size_t)batch * qblocks + blk0) * (2 * KK * 64), lane);
-  float m[2], s[2], on_at[2];
+  float m[2], s[2], off[2];  // a unit goes on where a logit exceeds m - off
   int best[2];
 #pragma unroll
   for (int rb = 0; rb < 2; ++rb) {
@@ -607,7 +608,7 @@ __device__ __forceinline__ unsigned pair_item_two_coarse(const PairArgs& a, int 
     m[rb] = low;
     s[rb] = 0.f;
     best[rb] = -1;
-    on_at[rb] = row < n_q ? low - kPairGap - cross : 3.0e38f;
+    off[rb] = row < n_q ? kPairGap + cross : -3.0e38f;
   }
   const unsigned one = 0x3c00u, s1 = 0x6c00u, s2 = 0x3c00u, s3 = 0x0c00u;  // fp16 1, 2^12, 1, 2^-12
   // the key's bias with its share of the bound, and without
@@ -652,7 +653,7 @@ __device__ __forceinline__ unsigned pair_item_two_coarse(const PairArgs& a, int 
   };
   auto finish = [&](int of, int sub, int buf, const float (&mx)[2]) {
     const int js = sub & 1;
-    const bool on0 = wave_any(mx[0] > on_at[0]), on1 = wave_any(mx[1] > on_at[1]);
+    const bool on0 = wave_any(mx[0] > m[0] - off[0]), on1 = wave_any(mx[1] > m[1] - off[1]);
     if (!(on0 || on1)) return;
     const unsigned long long bit = 1ull << (sub & 63);
     list[0][0] |= on0 && sub < 64 ? bit : 0ull;
@@ -892,7 +893,8 @@ __device__ __forceinline__ int pair_run_coarse(const PairArgs& a, int batch, Pai
   stage(1);
 
   u32x4 xa[2][2][KK], xb[2];
-  float on_at[2];  // a unit goes on (onto the list) where a logit and the streamed row's share of the bound exceed that
+  float on_at[2];  // a unit goes on where a logit and the streamed row's share of the bound exceed that
+  float far = 0.f;
   auto load_rows = [&]() {
     const PairProblem& pr = a.prob[t.prob];
     const int blk0 = t.group * 8 + wave * 2;
@@ -901,8 +903,8 @@ __device__ __forceinline__ int pair_run_coarse(const PairArgs& a, int batch, Pai
     pair_load_rows(xa, pr.st_planes + ((size_t)batch * pr.st_blocks + blk0) * (2 * KK * 64), lane);
   };
   auto derive_rows = [&]() {
-    const float far = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(
-                          __builtin_bit_cast(int, modes[t.prob].low - modes[t.prob].reserve))) - kPairGap;
+    far = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(
+              __builtin_bit_cast(int, modes[t.prob].low - modes[t.prob].reserve))) - kPairGap;
 #pragma unroll
     for (int rb = 0; rb < 2; ++rb) {
       float c = pair_cross_of(xb[rb]);
@@ -962,11 +964,6 @@ __device__ __forceinline__ int pair_run_coarse(const PairArgs& a, int batch, Pai
     const int js = sub & 1;
     const bool on0 = wave_any(mx[0] + bound[of] > on_at[0]), on1 = wave_any(mx[1] + bound[of] > on_at[1]);
     if (on0 || on1) {
-      const unsigned long long bit = 1ull << (sub & 63);
-      list[0][0] |= on0 && sub < 64 ? bit : 0ull;
-      list[0][1] |= on0 && sub >= 64 ? bit : 0ull;
-      list[1][0] |= on1 && sub < 64 ? bit : 0ull;
-      list[1][1] |= on1 && sub >= 64 ? bit : 0ull;
       u32x4 z[2][KK], zb;
 #pragma unroll
       for (int q = 1; q >= 0; --q)
@@ -988,6 +985,12 @@ __device__ __forceinline__ int pair_run_coarse(const PairArgs& a, int batch, Pai
 #pragma unroll
         for (int kk = 0; kk < KK; ++kk) c = small_mfma(xa[rb][0][kk], z[0][kk], c);
         c = small_mfma(xb[rb], zb, c);
+        // (its logits themselves, which the bound is far above, say whether it is kept)
+        if (wave_any(small_max16(c[0], c) > far - 0.5f)) {
+          const unsigned long long bit = 1ull << (sub & 63);
+          list[rb][0] |= sub < 64 ? bit : 0ull;
+          list[rb][1] |= sub >= 64 ? bit : 0ull;
+        }
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const float e = fast_exp2(c[r]);
@@ -1069,12 +1072,15 @@ __device__ __forceinline__ int pair_run_coarse(const PairArgs& a, int batch, Pai
 }
 
 // Work items of steps whose lists hold, from index `at` of the workgroup's on, as long as they are such:
-// only the units on the lists are visited, without a test.  A wavefront goes along its own list with the
-// streamed operands straight from global memory, one sub-tile ahead, and with no barrier but those
-// around the streamed rows' sums, which lie in LDS per wavefront until the item is done.
+// only the units on the lists are visited, without a test, with the streamed operands straight from global
+// memory, one sub-tile ahead.  The sub-tiles on the lists of an item's four blocks of 64 rows are shared
+// out evenly between the wavefronts (some rows have near keys everywhere: with a block to each a settled
+// launch at 50,000 x 64 took 103 us, with even shares 80), so a wavefront may finish one block's list and
+// begin the next one's.  Both kinds of sums lie in LDS until the item is done: of streamed rows per block, of stationary
+// rows per block and wavefront, each added in a fixed order.
 template <int DP>
 __device__ __forceinline__ int pair_run_list(const PairArgs& a, int batch, PairWork work, int at, int stride,
-                                             int count, unsigned which, float* cols) {
+                                             int count, unsigned which, float* cols, float* rows) {
   constexpr int KK = DP / 16;
   typedef unsigned long long u64;
   struct Keys {
@@ -1082,42 +1088,57 @@ __device__ __forceinline__ int pair_run_list(const PairArgs& a, int batch, PairW
   };
   const int lane = pair_lane(), li = lane & 31, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // lane (4 block + word) % 16: one of the item's words
   auto words_of = [&](const PairItem& t) {
     const PairProblem& pr = a.prob[t.prob];
-    return pr.list + (((size_t)batch * pr.n_items + t.index) * 4 + wave) * kPairListWords;
-  };
-  auto uniform = [](u64 v) {
-    return (u64)(unsigned)__builtin_amdgcn_readfirstlane((unsigned)v) |
-           (u64)(unsigned)__builtin_amdgcn_readfirstlane((unsigned)(v >> 32)) << 32;
+    return pr.list[((size_t)batch * pr.n_items + t.index) * (4 * kPairListWords) + (lane & 15)];
   };
   PairItem t = pair_item(work[at]);
   PairWord ahead = work[min(at + stride, count - 1)];
-  u64 w[kPairListWords];
-#pragma unroll
-  for (int k = 0; k < kPairListWords; ++k) w[k] = words_of(t)[k];
+  u64 w = words_of(t);
   // (what lies there may be the other forms' tiles; each item leaves zeros again)
   for (int i = threadIdx.x; i < 4 * a.prob[t.prob].chunk; i += 256) cols[i] = 0.f;
   __syncthreads();
   for (;;) {
     const PairProblem& pr = a.prob[t.prob];
     const PairItem now = t;
-    const int chunk = pr.chunk, blk0 = now.group * 8 + wave * 2, rows = now.j_end - now.j_begin;
-    const u64 on00 = uniform(w[0]), on01 = uniform(w[1]), on10 = uniform(w[2]), on11 = uniform(w[3]);
-    u64 left0 = on00 | on10, left1 = on01 | on11;
+    const int chunk = pr.chunk, len = now.j_end - now.j_begin;
+    auto word = [&](u64 v, int i) {
+      return (u64)(unsigned)__builtin_amdgcn_readlane((int)(unsigned)v, i) |
+             (u64)(unsigned)__builtin_amdgcn_readlane((int)(unsigned)(v >> 32), i) << 32;
+    };
+    const u64 mine = w;
     at += stride;
     t = pair_item(ahead);
     const bool more = at < count && t.prob >= 0 && ((which >> t.prob) & 1);
     if (more) {
       ahead = work[min(at + stride, count - 1)];
-#pragma unroll
-      for (int k = 0; k < kPairListWords; ++k) w[k] = words_of(t)[k];
+      w = words_of(t);
     }
-    float st[2][16];
+    int total = 0;
 #pragma unroll
-    for (int rb = 0; rb < 2; ++rb)
+    for (int o = 0; o < 4; ++o)
+      total += __popcll(word(mine, 4 * o) | word(mine, 4 * o + 2)) + __popcll(word(mine, 4 * o + 1) | word(mine, 4 * o + 3));
+    const int from = wave * total / 4, to = (wave + 1) * total / 4;
+    int before = 0;
+#pragma unroll 1
+    for (int o = 0; o < 4; ++o) {
+      const u64 on00 = word(mine, 4 * o), on01 = word(mine, 4 * o + 1), on10 = word(mine, 4 * o + 2), on11 = word(mine, 4 * o + 3);
+      u64 left0 = on00 | on10, left1 = on01 | on11;
+      const int here = __popcll(left0) + __popcll(left1);
+      int skip = max(from - before, 0), left = min(to - before, here) - skip;
+      before += here;
+      float* sum = rows + (o * 4 + wave) * 64;
+      if (left <= 0) {
+        sum[lane] = 0.f;
+        continue;
+      }
+      float st[2][16];
 #pragma unroll
-      for (int r = 0; r < 16; ++r) st[rb][r] = 0.f;
-    if (left0 | left1) {
+      for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) st[rb][r] = 0.f;
+      const int blk0 = now.group * 8 + o * 2;
       u32x4 xa[2][2][KK], xb[2];
 #pragma unroll
       for (int rb = 0; rb < 2; ++rb)
@@ -1125,14 +1146,20 @@ __device__ __forceinline__ int pair_run_list(const PairArgs& a, int batch, PairW
       pair_load_rows(xa, pr.st_planes + ((size_t)batch * pr.st_blocks + blk0) * (2 * KK * 64), lane);
       const u32x4* planes = pr.str_planes + ((size_t)batch * pr.str_blocks + now.j_begin / 32) * (2 * KK * 64);
       const u32x4* bias = pr.str_bias + (size_t)batch * pr.str_blocks * 32 + now.j_begin;
-      auto take = [&]() {  // the next sub-tile of the list, -1 behind the last
+      const int low = __popcll(left0);
+      for (int k = min(skip, low); k > 0; --k) left0 &= left0 - 1;
+      for (int k = skip - low; k > 0; --k) left1 &= left1 - 1;
+      auto take = [&]() {  // the next sub-tile, -1 behind the last
         int sub = -1;
-        if (left0) {
-          sub = __builtin_ctzll(left0);
-          left0 &= left0 - 1;
-        } else if (left1) {
-          sub = 64 + __builtin_ctzll(left1);
-          left1 &= left1 - 1;
+        if (left > 0) {
+          if (left0) {
+            sub = __builtin_ctzll(left0);
+            left0 &= left0 - 1;
+          } else {
+            sub = 64 + __builtin_ctzll(left1);
+            left1 &= left1 - 1;
+          }
+          --left;
         }
         return sub;
       };
@@ -1170,7 +1197,7 @@ __device__ __forceinline__ int pair_run_list(const PairArgs& a, int batch, PairW
         }
         float ps = ps0 + ps1;
         ps += xor32(ps);
-        if (h == 0) cols[wave * chunk + sub * 32 + li] = ps;
+        if (h == 0) cols[o * chunk + sub * 32 + li] = ps;
       };
       Keys k0, k1;
       int s0 = take();
@@ -1185,10 +1212,22 @@ __device__ __forceinline__ int pair_run_list(const PairArgs& a, int batch, PairW
         run(k1, s1);
         if (s0 < 0) break;
       }
+#pragma unroll
+      for (int rb = 0; rb < 2; ++rb) {
+        float v = colsum_all(st[rb], li);
+        v += __shfl_xor(v, 16, 64);
+        if (li < 16) sum[rb * 32 + colsum_key(li, h)] = v;
+      }
     }
     __syncthreads();
+    {
+      const float* sum = rows + (threadIdx.x >> 6) * 256 + lane;
+      const int row = now.group * 256 + threadIdx.x;
+      if (row < pr.n_st)
+        pr.st_part[((size_t)batch * pr.chunks + now.chunk) * pr.n_st + row] = (sum[0] + sum[64]) + (sum[128] + sum[192]);
+    }
     float* out = pr.str_part + ((size_t)batch * pr.groups + now.group) * pr.n_str + now.j_begin;
-    for (int j = threadIdx.x; j < rows; j += 256) {
+    for (int j = threadIdx.x; j < len; j += 256) {
       float v = cols[j];
       cols[j] = 0.f;
 #pragma unroll
@@ -1198,7 +1237,6 @@ __device__ __forceinline__ int pair_run_list(const PairArgs& a, int batch, PairW
       }
       out[j] = v;
     }
-    pair_put_rows(pr, batch, now.chunk, blk0, st, lane);
     __syncthreads();
     if (!more) return at;
   }
@@ -1419,7 +1457,8 @@ __global__ __launch_bounds__(256, 2) void pair_sweep_kernel(PairArgsPtr args, in
     if (t.prob < 0 || !((live & sweep) >> t.prob & 1)) {
       i += stride;
     } else if (SKIP && ((list >> t.prob) & 1)) {
-      i = pair_run_list<DP>(a, batch, work, i, stride, count, list, reinterpret_cast<float*>(lds));
+      i = pair_run_list<DP>(a, batch, work, i, stride, count, list, reinterpret_cast<float*>(lds),
+                            &lds_col[0][0][0][0]);
     } else if (SKIP && ((coarse >> t.prob) & 1)) {
       i = pair_run_coarse<DP>(a, batch, work, i, stride, count, coarse, modes, went, lds, &lds_col[0][0][0][0]);
     } else {
