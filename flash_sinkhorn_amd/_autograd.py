@@ -13,6 +13,7 @@ from typing import Optional, Tuple
 
 import torch
 
+from flash_sinkhorn_amd import _small
 from flash_sinkhorn_amd.hvp import geomloss_to_ott_potentials, hvp_x_sqeuclid_from_potentials
 from flash_sinkhorn_amd.kernels.sinkhorn_triton_grad_sqeuclid import (
     sinkhorn_geomloss_online_grad_sqeuclid,
@@ -63,15 +64,20 @@ class _SinkhornGradFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, y, a, b, f_grad, g_grad, grad_scale, eps: float,
                 config: _SinkhornConfig, compute_grad_x: bool, compute_grad_y: bool,
-                label_x=None, label_y=None, label_cost_matrix=None, seed_keys=None):
+                label_x=None, label_y=None, label_cost_matrix=None, seed_keys=None, products=None):
+        kept = products is not None and bool(compute_grad_x)
         gx, gy = sinkhorn_geomloss_online_grad_sqeuclid(
             x, y, a, b, f_grad, g_grad, eps=float(eps), allow_tf32=config.allow_tf32,
             use_exp2=config.use_exp2, grad_scale=grad_scale,
-            compute_grad_x=bool(compute_grad_x), compute_grad_y=bool(compute_grad_y),
+            compute_grad_x=bool(compute_grad_x) and not kept, compute_grad_y=bool(compute_grad_y),
             cost_scale=config.cost_scale, label_x=label_x, label_y=label_y,
             label_cost_matrix=label_cost_matrix, lambda_x=config.lambda_x,
             lambda_y=config.lambda_y, _seed_keys=seed_keys)
-        ctx.save_for_backward(x, y, a, b, f_grad, g_grad, grad_scale)
+        if kept:
+            gx = products.gradient(grad_scale)
+        ctx.save_for_backward(x, y, a, b, f_grad, g_grad, grad_scale,
+                              *(() if products is None else products.tensors()))
+        ctx.products = None if products is None else products.form
         ctx.eps = float(eps)
         ctx.config = config
         ctx.use_label_cost = (label_x is not None and label_y is not None
@@ -80,7 +86,7 @@ class _SinkhornGradFn(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_grad_x, grad_grad_y):
-        x, y, a, b, f_grad, g_grad, grad_scale = ctx.saved_tensors
+        x, y, a, b, f_grad, g_grad, grad_scale, *kept = ctx.saved_tensors
         cfg = ctx.config
         if grad_grad_y is not None:
             raise NotImplementedError("Double backward w.r.t y is not implemented yet.")
@@ -103,9 +109,10 @@ class _SinkhornGradFn(torch.autograd.Function):
                     preconditioner=cfg.hvp_preconditioner, precond_terms=cfg.hvp_precond_terms,
                     use_preconditioner=cfg.hvp_use_preconditioner,
                     allow_tf32=False,  # second order needs full fp32 operands
-                    use_exp2=cfg.use_exp2)
+                    use_exp2=cfg.use_exp2,
+                    _products=_small.Products(ctx.products, *kept) if kept else None)
                 out_x = hvp * grad_scale
-        return (out_x,) + (None,) * 14
+        return (out_x,) + (None,) * 15
 
 
 class _SinkhornCostFn(torch.autograd.Function):
@@ -121,6 +128,7 @@ class _SinkhornCostFn(torch.autograd.Function):
         solver need not find out again (two passes over the clouds and a wait for the device)."""
         eps_last = float(eps_list[-1])
         seed_keys = None
+        products = None
         if presolved is not None:
             if config.last_extrapolation:
                 f_cost, g_cost, f_grad, g_grad = presolved
@@ -137,6 +145,8 @@ class _SinkhornCostFn(torch.autograd.Function):
             balanced_formula = True
         else:
             info = {} if x.shape[1] <= 128 else None  # (wide rows: no tile tests, nothing to ask for)
+            products = ([] if ctx.needs_input_grad[0] and config.last_extrapolation
+                        and _small.keeps_products(x, y) else None)
             out = sinkhorn_flashstyle_symmetric(
                 x, y, a, b, solve_info=info, eps_list=eps_list if schedule_of_points else None,
                 blur=config.blur, scaling=config.scaling,
@@ -147,7 +157,7 @@ class _SinkhornCostFn(torch.autograd.Function):
                 return_prelast=config.last_extrapolation, threshold=config.threshold,
                 check_every=config.inner_iterations, label_x=label_x, label_y=label_y,
                 label_cost_matrix=label_cost_matrix, lambda_x=config.lambda_x,
-                lambda_y=config.lambda_y)
+                lambda_y=config.lambda_y, _products=products)
             if config.last_extrapolation:
                 f_cost, g_cost, f_grad, g_grad = out
             else:
@@ -163,7 +173,10 @@ class _SinkhornCostFn(torch.autograd.Function):
                 if kx is not None and ky is not None:
                     seed_keys = (kx.clone(), ky.clone())
 
-        ctx.save_for_backward(x, y, a, b, f_cost, g_cost, f_grad, g_grad)
+        products = products[0] if products else None
+        ctx.save_for_backward(x, y, a, b, f_cost, g_cost, f_grad, g_grad,
+                              *(() if products is None else products.tensors()))
+        ctx.products = None if products is None else products.form
         ctx.eps = eps_last
         ctx.config = config
         ctx.seed_keys = seed_keys
@@ -178,12 +191,13 @@ class _SinkhornCostFn(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_out):
-        x, y, a, b, f_cost, g_cost, f_grad, g_grad = ctx.saved_tensors
+        x, y, a, b, f_cost, g_cost, f_grad, g_grad, *kept = ctx.saved_tensors
         grad_x = grad_y = grad_a = grad_b = None
         if x.requires_grad or y.requires_grad:
             gx, gy = _SinkhornGradFn.apply(x, y, a, b, f_grad, g_grad, grad_out, ctx.eps,
                                            ctx.config, x.requires_grad, y.requires_grad,
-                                           *ctx.labels, ctx.seed_keys)
+                                           *ctx.labels, ctx.seed_keys,
+                                           _small.Products(ctx.products, *kept) if kept else None)
             grad_x = gx if x.requires_grad else None
             grad_y = gy if y.requires_grad else None
         if a.requires_grad:

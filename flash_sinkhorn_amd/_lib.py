@@ -74,6 +74,10 @@ _SIGNATURES = {
     "fs_small_potentials": (ctypes.c_int, [_P, _P, _Z, _P, _P]),
     "fs_hvp_workspace_bytes": (_Z, [_P]),
     "fs_hvp": (ctypes.c_int, [_P, _P, _Z, _P, _P, _P]),
+    "fs_dense_grad_workspace_bytes": (_Z, [_P]),
+    "fs_dense_grad": (ctypes.c_int, [_P, _P, _Z, _P, _P, _P, _Z, _P]),
+    "fs_hvp_solved_workspace_bytes": (_Z, [_P]),
+    "fs_hvp_solved": (ctypes.c_int, [_P, _P, _P, _Z, _P, _Z, _P, _P, _P]),
     "fs_small_grad": (ctypes.c_int, [_P, _P, _Z, _P, _P, _P, _P]),
 }
 EXPORTED_SYMBOLS = tuple(_SIGNATURES)

@@ -152,11 +152,12 @@ def solve(x, y, a, b, *, items: int, blur: float = 0.0, scaling: float = 0.0, ep
           entries: int = 0, cut: int = 0, eps_list=None, cost_scale: float, rho_x, rho_y,
           normalize: bool, self_terms: int, want_values: bool, extrapolate: bool,
           want_loss: bool, threshold: Optional[float] = None, check_every: int = 1,
-          alternating: bool = False, prelast: bool = False) -> Solved:
+          alternating: bool = False, prelast: bool = False, keep: bool = False) -> Solved:
     """Enqueue one run of small problems: contiguous x [items, n, d] and y [items, m, d] of one dtype,
     weights as contiguous fp32 or None.  ``eps_list`` (host floats), ``eps`` with ``entries``, or
     a schedule by diameter, in that order.  Without ``want_loss``: the potentials, with ``prelast``
-    also those before the extrapolation."""
+    also those before the extrapolation.  ``keep``: the workspace stays with the result also without
+    ``want_values``."""
     n, d = x.shape[-2:]
     m = y.shape[-2]
     sched = 2 if eps_list is not None else (0 if eps > 0.0 else 1)
@@ -215,11 +216,11 @@ def solve(x, y, a, b, *, items: int, blur: float = 0.0, scaling: float = 0.0, ep
                 where[2 * side + kind] = t.data_ptr()
             _lib.check(L.fs_small_potentials(ctypes.byref(p), ws.data_ptr(), ws.numel(), where,
                                              _lib.stream_of(x)), "fs_small_potentials")
-        return pots + ((loss,) if want_loss else ()) + ((ws,) if want_values else ())
+        return pots + ((loss,) if want_loss else ()) + ((ws,) if want_values or keep else ())
 
     # (a graph keeps its products; of a batch it counts all items, and the workspace that a replay
     # may copy)
-    if (sched == 0 and not threshold and _graphs.eligible(items * n, m, entries, x.device)
+    if (sched == 0 and not threshold and not keep and _graphs.eligible(items * n, m, entries, x.device)
             and (d <= WIDE_D or items * n * m <= 1 << 22)
             and (items == 1 or nbytes <= MAX_GRAPH_BYTES)):
         # a fixed sequence of kernels on fixed shapes: replayed (1.9 instead of 3 us per launch)
@@ -232,7 +233,7 @@ def solve(x, y, a, b, *, items: int, blur: float = 0.0, scaling: float = 0.0, ep
         out = enqueue(x, y, a, b)
     s = Solved()
     s.form, s.x, s.y, s.a, s.b = form, x, y, a, b
-    s.ws = out[-1] if want_values else None
+    s.ws = out[-1] if want_values or keep else None
     s.pots, s.loss = out[:2] if want_loss else (None, None)
     s.own = None
     if own:
@@ -294,6 +295,44 @@ def alternating_problem(x, y, a, b, allow_tf32: bool) -> bool:
     n, m, d = x.shape[0], y.shape[0], x.shape[-1]
     return (solver_problem(x, y, a, b, allow_tf32, True, False, any_size=True)
             and n * m <= (140_000_000 if d <= 32 else 65_000_000 if d <= 64 else 36_000_000))
+
+
+class Products:
+    """The inner products that a solve of wide rows has kept, for the gradient in x and the Hessian-vector
+    product behind it.  ``tensors`` are what an autograd node saves (the points as the solve read them and
+    its workspace), ``restored`` makes it of them again."""
+    __slots__ = ("form", "x", "y", "ws")
+
+    def __init__(self, form: Problem, x, y, ws):
+        self.form, self.x, self.y, self.ws = form, x, y, ws
+
+    def tensors(self):
+        return self.x, self.y, self.ws
+
+    def problem(self) -> Problem:
+        p = Problem.from_buffer_copy(self.form)
+        p.x, p.y = self.x.data_ptr(), self.y.data_ptr()
+        return p
+
+    def gradient(self, grad_out):
+        """The gradient in x times the scalar ``grad_out``, fp32 [n, d]."""
+        p, L = self.problem(), _lib.lib()
+        scratch = torch.empty(L.fs_dense_grad_workspace_bytes(ctypes.byref(p)), dtype=torch.uint8,
+                              device=self.x.device)
+        gx = torch.empty(self.x.shape, dtype=torch.float32, device=self.x.device)
+        gs = grad_out.detach().to(dtype=torch.float32).reshape(1).contiguous()
+        _lib.check(L.fs_dense_grad(ctypes.byref(p), self.ws.data_ptr(), self.ws.numel(), gs.data_ptr(),
+                                   gx.data_ptr(), scratch.data_ptr(), scratch.numel(),
+                                   _lib.stream_of(self.x)), "fs_dense_grad")
+        return gx
+
+
+def keeps_products(x, y) -> bool:
+    """Whether a loss keeps the products of its solve for what follows it: of wide rows, where forming them
+    again takes longer than a step (up to 2^22 of them a solve is a replayed graph, whose
+    workspace is the next call's).  They stay below 1 GiB."""
+    return (x.ndim == 2 and WIDE_D < x.shape[1] <= MAX_D and x.dtype in _DTYPES and y.dtype is x.dtype
+            and 1 << 22 < x.shape[0] * y.shape[0] <= MAX_KEPT)
 
 
 def _weights(w, lead, count, device, normalize):

@@ -32,4 +32,10 @@ int cg_init(const float* b, float* sol, float* res, float* dir, float* state, lo
 int cg_update(const float* a_dir, float* sol, float* res, float* dir, float* state, long long m, float* host, int iter,
               hipStream_t st);
 
+// The arguments of the kernels of a solve of wide rows that left `workspace` behind (fs_small.hip), with one
+// item and an extrapolation.
+struct SmallArgs;
+struct DenseArgs;
+int dense_solved(const fs_small_problem* p, void* workspace, size_t workspace_bytes, SmallArgs& a, DenseArgs& t);
+
 }  // namespace fs

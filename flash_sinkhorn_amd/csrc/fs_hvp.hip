@@ -25,7 +25,14 @@ struct HvpPlan {
   HvpArgs a;
 };
 
-size_t layout(const fs_hvp_problem* p, void* ws, HvpPlan& q) {
+// What a solve of the same points has left: nothing of it is formed again.
+struct Kept {
+  SmallArgs a;
+  DenseArgs t;
+};
+
+// `shared`: the products come from a solve, `kept` where more than the sizes is asked for.
+size_t layout(const fs_hvp_problem* p, void* ws, HvpPlan& q, bool shared, const Kept* kept = nullptr) {
   std::memset(&q, 0, sizeof(q));
   const int n = (int)p->n, m = (int)p->m, d = (int)p->d;
   size_t at = 0;
@@ -35,7 +42,8 @@ size_t layout(const fs_hvp_problem* p, void* ws, HvpPlan& q) {
     at += (bytes + 255) & ~(size_t)255;
   };
   // ---- the three matrices' planes ----
-  auto prepare = [&](SmallArgs& s, DenseArgs& t, const void* first, const void* second, int rows0, int rows1, int dtype) {
+  auto prepare = [&](SmallArgs& s, DenseArgs& t, const void* first, const void* second, int rows0, int rows1, int dtype,
+                     bool mine) {
     s.pts[0] = first;
     s.pts[1] = second;
     s.rows[0] = rows0;
@@ -49,6 +57,7 @@ size_t layout(const fs_hvp_problem* p, void* ws, HvpPlan& q) {
     s.stat_words = 2;
     s.table_len = 1;
     dense_plan(s, t);
+    if (!mine) return;
     take(s.lens, 3 * 4);
     take(s.full, 3 * 4);
     take(s.table, 3 * (size_t)s.table_len * sizeof(float4));
@@ -63,8 +72,15 @@ size_t layout(const fs_hvp_problem* p, void* ws, HvpPlan& q) {
       take(s.pot[i], rows * 4);
     }
   };
-  prepare(q.pts, q.td, p->x, p->y, n, m, p->dtype);
-  prepare(q.dir, q.ta, p->A, nullptr, n, m, 0);
+  prepare(q.pts, q.td, p->x, p->y, n, m, p->dtype, !shared);
+  prepare(q.dir, q.ta, p->A, nullptr, n, m, 0, true);
+  if (kept) {
+    for (int i = 0; i < 2; ++i) {
+      q.td.planes[i] = kept->t.planes[i];
+      q.pts.norm[i] = kept->a.norm[i];
+    }
+    q.pts.scale = kept->a.scale;
+  }
   HvpArgs& a = q.a;
   a.x = p->x;
   a.y = p->y;
@@ -92,7 +108,8 @@ size_t layout(const fs_hvp_problem* p, void* ws, HvpPlan& q) {
   a.norm_a = q.dir.norm[0];
   a.scale = q.pts.scale;
   const size_t N = n, M = m, L = a.ld;
-  take(a.dots, N * L * 4);
+  if (!shared) take(a.dots, N * L * 4);
+  if (kept) a.dots = kept->t.dots;
   take(a.prod, N * L * 4);
   for (float** r : {&a.xa, &a.ra, &a.mass, &a.r1, &a.inv_diag, &a.w, &a.alpha, &a.s, &a.v_scale}) take(*r, N * 4);
   for (float** r : {&a.cb, &a.denom, &a.r2, &a.vec, &a.sol, &a.res, &a.a_dir}) take(*r, L * 4);
@@ -153,6 +170,50 @@ int strips(const HvpArgs& a, hipStream_t st) {
   return hipGetLastError() == hipSuccess ? FS_OK : FS_ERR_LAUNCH_FAILED;
 }
 
+// The planes, sums and products behind a gradient on kept products.
+struct GradPlan {
+  DenseGradArgs g;
+  TransposedArgs yt;
+  DenseGemmArgs product;
+};
+
+size_t grad_layout(const SmallArgs& s, const DenseArgs& t, void* ws, GradPlan& q) {
+  std::memset(&q, 0, sizeof(q));
+  size_t at = 0;
+  auto take = [&](auto& ptr, size_t bytes) {
+    ptr = reinterpret_cast<std::remove_cv_t<std::remove_reference_t<decltype(ptr)>>>(static_cast<char*>(ws) + at);
+    at += (bytes + 255) & ~(size_t)255;
+  };
+  DenseGradArgs& g = q.g;
+  g.ldo = (s.d + 255) / 256 * 256;
+  const size_t steps = t.ld / 16;
+  take(g.planes, (size_t)t.blocks[0] * steps * 2048);
+  take(q.yt.yt, (size_t)(g.ldo / 32) * steps * 2048);
+  take(g.sums, (size_t)(t.ld / 256) * t.n * 4);
+  q.yt.y = s.pts[1];
+  q.yt.scale = s.scale;
+  q.yt.m = t.m;
+  q.yt.d = s.d;
+  q.yt.ld = t.ld;
+  q.yt.dtype = s.dtype;
+  DenseGemmArgs& m = q.product;
+  m.a = g.planes;
+  m.b = q.yt.yt;
+  m.a_blocks = t.blocks[0];
+  m.b_blocks = g.ldo / 32;
+  m.steps = (int)steps;
+  m.rows = t.n;
+  m.ld = g.ldo;
+  dense_gemm_plan(m, true);
+  g.splits = m.splits;
+  take(m.out, (size_t)m.splits * t.n * g.ldo * 4);
+  g.prod = m.out;
+  return at;
+}
+
+int run_hvp(const fs_hvp_problem* p, const Kept* kept, void* workspace, size_t workspace_bytes, float* out,
+            float* host_state, hipStream_t st);
+
 }  // namespace
 }  // namespace fs
 
@@ -163,21 +224,72 @@ extern "C" {
 size_t fs_hvp_workspace_bytes(const fs_hvp_problem* p) {
   if (checked(p) != FS_OK) return 0;
   HvpPlan q;
-  return layout(p, nullptr, q);
+  return layout(p, nullptr, q, false);
+}
+
+size_t fs_hvp_solved_workspace_bytes(const fs_hvp_problem* p) {
+  if (checked(p) != FS_OK) return 0;
+  HvpPlan q;
+  return layout(p, nullptr, q, true);
 }
 
 int fs_hvp(const fs_hvp_problem* p, void* workspace, size_t workspace_bytes, float* out, float* host_state, void* stream) {
+  return run_hvp(p, nullptr, workspace, workspace_bytes, out, host_state, (hipStream_t)stream);
+}
+
+int fs_hvp_solved(const fs_hvp_problem* p, const fs_small_problem* solved, void* solved_workspace, size_t solved_bytes,
+                  void* workspace, size_t workspace_bytes, float* out, float* host_state, void* stream) {
+  if (!p || !solved || !solved_workspace) return FS_ERR_NULL_POINTER;
+  Kept kept;
+  const int rc = dense_solved(solved, solved_workspace, solved_bytes, kept.a, kept.t);
+  if (rc != FS_OK) return rc;
+  if (solved->n != p->n || solved->m != p->m || solved->d != p->d || solved->cost_scale != p->cost_scale) return FS_ERR_BAD_SIZE;
+  return run_hvp(p, &kept, workspace, workspace_bytes, out, host_state, (hipStream_t)stream);
+}
+
+size_t fs_dense_grad_workspace_bytes(const fs_small_problem* p) {
+  SmallArgs a;
+  DenseArgs t;
+  GradPlan q;
+  return dense_solved(p, nullptr, ~(size_t)0, a, t) == FS_OK ? grad_layout(a, t, nullptr, q) : 0;
+}
+
+int fs_dense_grad(const fs_small_problem* p, void* solved_workspace, size_t solved_bytes, const float* grad_out,
+                  float* grad_x, void* workspace, size_t workspace_bytes, void* stream) {
+  if (!p || !solved_workspace || !workspace || !grad_out || !grad_x) return FS_ERR_NULL_POINTER;
+  SmallArgs a;
+  DenseArgs t;
+  GradPlan q;
+  int rc = dense_solved(p, solved_workspace, solved_bytes, a, t);
+  if (rc != FS_OK) return rc;
+  if (grad_layout(a, t, workspace, q) > workspace_bytes) return FS_ERR_WORKSPACE_TOO_SMALL;
+  hipStream_t st = (hipStream_t)stream;
+  q.g.grad_out = grad_out;
+  q.g.out = grad_x;
+  hipLaunchKernelGGL((dense_plan_kernel<0>), dim3((t.n + 255) / 256 * 8, t.ld / 256), dim3(256), 0, st, a, t, q.g);
+  hipLaunchKernelGGL((hvp_yt_kernel<0>), dim3((t.ld / 16 + 3) / 4, q.g.ldo / 32), dim3(256), 0, st, q.yt);
+  if ((rc = dense_gemm(q.product, 1, st)) != FS_OK) return rc;
+  hipLaunchKernelGGL((dense_grad_kernel<0>), dim3(t.n), dim3(256), 0, st, a, t, q.g);
+  return hipGetLastError() == hipSuccess ? FS_OK : FS_ERR_LAUNCH_FAILED;
+}
+
+}  // extern "C"
+
+namespace fs {
+namespace {
+
+int run_hvp(const fs_hvp_problem* p, const Kept* kept, void* workspace, size_t workspace_bytes, float* out,
+            float* host_state, hipStream_t st) {
   int rc = checked(p);
   if (rc != FS_OK) return rc;
   if (!out || !host_state) return FS_ERR_NULL_POINTER;
   HvpPlan q;
-  if (!workspace || layout(p, workspace, q) > workspace_bytes) return FS_ERR_WORKSPACE_TOO_SMALL;
-  hipStream_t st = (hipStream_t)stream;
+  if (!workspace || layout(p, workspace, q, kept != nullptr, kept) > workspace_bytes) return FS_ERR_WORKSPACE_TOO_SMALL;
   HvpArgs& a = q.a;
   a.out = out;
-  if ((rc = prepare(q.pts, q.td, 2, st)) != FS_OK || (rc = prepare(q.dir, q.ta, 1, st)) != FS_OK) return rc;
+  if ((!kept && (rc = prepare(q.pts, q.td, 2, st)) != FS_OK) || (rc = prepare(q.dir, q.ta, 1, st)) != FS_OK) return rc;
   hipLaunchKernelGGL((hvp_rows_kernel<0>), dim3((a.n + a.ld + 3) / 4), dim3(256), 0, st, a);
-  if ((rc = dense_gemm(q.dots, 1, st)) != FS_OK || (rc = dense_gemm(q.prod, 1, st)) != FS_OK) return rc;
+  if ((!kept && (rc = dense_gemm(q.dots, 1, st)) != FS_OK) || (rc = dense_gemm(q.prod, 1, st)) != FS_OK) return rc;
   if (q.td.large) hipLaunchKernelGGL((hvp_mass_kernel<8>), dim3(a.groups, a.chunks), dim3(512), 0, st, a);
   else hipLaunchKernelGGL((hvp_mass_kernel<4>), dim3(a.groups, a.chunks), dim3(256), 0, st, a);
   hipLaunchKernelGGL((hvp_merge_kernel<0>), dim3((std::max(a.n, a.m) + 63) / 64, 2), dim3(256), 0, st, a);
@@ -202,7 +314,8 @@ int fs_hvp(const fs_hvp_problem* p, void* workspace, size_t workspace_bytes, flo
   if ((rc = strips<2>(a, st)) != FS_OK) return rc;
   hipLaunchKernelGGL((hvp_limits_kernel<0>), dim3(1), dim3(1024), 0, st, a);
   hipLaunchKernelGGL((hvp_v_kernel<0>), dim3((a.n + 255) / 256 * 8, a.ld / 256), dim3(256), 0, st, a);
-  hipLaunchKernelGGL((hvp_yt_kernel<0>), dim3((a.ld / 16 + 3) / 4, a.yt_blocks), dim3(256), 0, st, a);
+  hipLaunchKernelGGL((hvp_yt_kernel<0>), dim3((a.ld / 16 + 3) / 4, a.yt_blocks), dim3(256), 0, st,
+                     (TransposedArgs{a.y, a.scale, a.yt, a.m, a.d, a.ld, a.dtype}));
   if ((rc = dense_gemm(q.last, 1, st)) != FS_OK) return rc;
   const int blocks = (int)std::min<size_t>(4096, ((size_t)a.n * a.d + 255) / 256);
   hipLaunchKernelGGL((hvp_result_kernel<0>), dim3(blocks), dim3(256), 0, st, a);
@@ -211,4 +324,5 @@ int fs_hvp(const fs_hvp_problem* p, void* workspace, size_t workspace_bytes, flo
   return done ? FS_OK : wait_for_words(st, [&]() { return seen(p->max_iter); });
 }
 
-}  // extern "C"
+}  // namespace
+}  // namespace fs

@@ -387,8 +387,14 @@ __global__ __launch_bounds__(256) void hvp_v_kernel(const HvpArgs a) {
 }
 
 // Planes of y^T: the rows are y's columns.  A wavefront per 32 columns and 16 points.
+struct TransposedArgs {
+  const void* y;
+  const float2* scale;  // of x, y
+  u32x4* yt;            // [column blocks][ld / 16][2][64]
+  int m, d, ld, dtype;
+};
 template <int T>
-__global__ __launch_bounds__(256) void hvp_yt_kernel(const HvpArgs a) {
+__global__ __launch_bounds__(256) void hvp_yt_kernel(const TransposedArgs a) {
   const int blk = blockIdx.y, kk = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (kk >= a.ld / 16) return;
   const int col = blk * 32 + (lane & 31), j0 = 16 * kk + 8 * (lane >> 5);
@@ -407,6 +413,97 @@ __global__ __launch_bounds__(256) void hvp_yt_kernel(const HvpArgs a) {
   u32x4* out = a.yt + ((size_t)blk * (a.ld / 16) + kk) * kDenseStep + lane;
   out[0] = hi;
   out[64] = lo;
+}
+
+// The gradient in x of a solve whose products are kept:
+//   2 cs gs w_i (x_i - sum_j P_ij y_j / sum_j P_ij),  P_ij = 2^(qs x_i.y_j + c_j - L_i),
+// c_j the biases of y before the extrapolation and L_i the logarithm of the row's sum over them, which is what
+// the extrapolation made the potential of x of.
+struct DenseGradArgs {
+  const float* grad_out;
+  float* out;
+  u32x4* planes;             // of P, [n blocks][ld / 16][2][64]
+  float* sums;               // [ld / 256][n] sums of a row's P over 256 columns
+  const float* prod;         // [splits][n][ldo] P y
+  int ldo, splits;
+};
+constexpr float kDenseGradScale = 4096.f;  // P is at most one, but for the rounding of L
+
+// Planes of P, in the shape of hvp_v_kernel, and the sums of its rows.  Bound by memory: 8,192 x 8,192 in 116 us (4.6
+// TB/s); the product behind it 520, the result 113, where forming the plan's products again took 1.65 ms.
+template <int T>
+__global__ __launch_bounds__(256) void dense_plan_kernel(const SmallArgs a, const DenseArgs t, const DenseGradArgs g) {
+  constexpr int UNIT = 528;
+  __shared__ __attribute__((aligned(16))) unsigned char lds[2 * 32 * UNIT];
+  const int blk = blockIdx.x, c0 = blockIdx.y * 256;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int last = a.lens[0] + 2;
+  const float4 coef = small_last_coef(a, 0, 0);
+  const float* f = a.pot[0] + (size_t)(last & 1) * t.n;            // behind the extrapolation
+  const float* y = a.pot[1] + (size_t)((last & 1) ^ 1) * t.m;      // before it
+  const float damp = a.rho[0] > 0.f ? 1.0f / (1.0f + coef.x / a.rho[0]) : 1.0f;
+  float kb[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int col = c0 + 4 * lane + k, cc = min(col, t.m - 1);
+    kb[k] = col < t.m ? fmaxf(__builtin_fmaf(coef.w, y[cc], a.l2w[1][cc]), kNegBig) : kNegBig;
+  }
+  float sum[8];
+#pragma unroll
+  for (int r = 0; r < 8; ++r) {
+    const int i = wave * 8 + r, row = blk * 32 + i, rc = min(row, t.n - 1);
+    float v[4];
+    *reinterpret_cast<float4*>(v) = *reinterpret_cast<const float4*>(t.dots + (size_t)rc * t.ld + c0 + 4 * lane);
+    const float fr = f[rc], shift = damp < 1.0f ? (1.0f - damp) * a.norm[0][rc] : 0.f;
+    const float lse = -(fr + shift) / (coef.x * damp * kLn2);
+    _Float16 hi[4], lo[4];
+    sum[r] = 0.f;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const float p = row < t.n ? kDenseGradScale * fast_exp2(__builtin_fmaf(v[k], coef.y, kb[k] - lse)) : 0.f;
+      sum[r] += p;
+      hi[k] = (_Float16)p;
+      lo[k] = (_Float16)(p - (float)hi[k]);
+    }
+    unsigned char* o = lds + (lane >> 1) * UNIT + i * 16 + (lane & 1) * 8;  // (as in hvp_v_kernel)
+    *reinterpret_cast<uint2*>(o) = make_uint2(pack_f16((float)hi[0], (float)hi[1]), pack_f16((float)hi[2], (float)hi[3]));
+    *reinterpret_cast<uint2*>(o + 32 * UNIT) =
+        make_uint2(pack_f16((float)lo[0], (float)lo[1]), pack_f16((float)lo[2], (float)lo[3]));
+  }
+  // the rows' sums over the lanes: halves of the rows change places, then what is left of each
+#pragma unroll
+  for (int o = 32, n = 4; n > 0; o >>= 1, n >>= 1) {
+    const bool up = lane & o;
+#pragma unroll
+    for (int r = 0; r < n; ++r) sum[r] = (up ? sum[r + n] : sum[r]) + __shfl_xor(up ? sum[r] : sum[r + n], o, 64);
+  }
+#pragma unroll
+  for (int o = 4; o > 0; o >>= 1) sum[0] += __shfl_xor(sum[0], o, 64);
+  const int mine = blk * 32 + wave * 8 + (lane >> 3);
+  if ((lane & 7) == 0 && mine < t.n) g.sums[(size_t)blockIdx.y * t.n + mine] = sum[0];
+  __syncthreads();
+  u32x4* out = g.planes + ((size_t)blk * (t.ld / 16) + c0 / 16) * kDenseStep;
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    const int w = threadIdx.x + 256 * q;
+    const int kk = w >> 7, plane = (w >> 6) & 1, half = (w >> 5) & 1, i = w & 31;
+    out[w] = *reinterpret_cast<const u32x4*>(lds + (plane * 32 + kk * 2 + half) * UNIT + i * 16);
+  }
+}
+
+// A workgroup per row.
+template <int T>
+__global__ __launch_bounds__(256) void dense_grad_kernel(const SmallArgs a, const DenseArgs t, const DenseGradArgs g) {
+  const int row = blockIdx.x;
+  float s = 0.f;
+  for (int c = 0; c < t.ld / 256; ++c) s += g.sums[(size_t)c * t.n + row];
+  const float inv = a.scale[1].y / fmaxf(s, 1e-40f), coef = 2.0f * a.cost_scale * g.grad_out[0] * a.wt[0][row];
+  for (int col = threadIdx.x; col < a.d; col += 256) {
+    float v = 0.f;
+    for (int k = 0; k < g.splits; ++k) v += g.prod[((size_t)k * t.n + row) * g.ldo + col];
+    const size_t e = (size_t)row * a.d + col;
+    g.out[e] = coef * (small_load(a.pts[0], e, a.dtype) - v * inv);
+  }
 }
 
 // The result.

@@ -452,6 +452,14 @@ int by_width(int64_t d, F&& f) {
 }
 
 }  // namespace
+
+int dense_solved(const fs_small_problem* p, void* workspace, size_t workspace_bytes, SmallArgs& a, DenseArgs& t) {
+  const int rc = checked(p);
+  if (rc != FS_OK) return rc;
+  if (!use_dense(p) || p->items != 1 || !p->extrapolate) return FS_ERR_UNSUPPORTED;
+  return layout(p, workspace, a, nullptr, &t) > workspace_bytes ? FS_ERR_WORKSPACE_TOO_SMALL : FS_OK;
+}
+
 }  // namespace fs
 
 using namespace fs;

@@ -104,8 +104,11 @@ def _kept_ok(x, y, f_hat, g_hat, A, allow_tf32: bool) -> bool:
 
 
 def _kept(x, y, f_hat, g_hat, A, *, eps, cost_scale, rho_x, rho_y, tau2, lambda_indef, rtol, atol,
-          max_iter):
-    """One library call: three contractions, the rest passes over kept matrices."""
+          max_iter, products=None):
+    """One library call: three contractions, the rest passes over kept matrices.  ``products``: those that
+    the solve of the same points has kept, so that two contractions are left."""
+    if products is not None:
+        x, y = products.x, products.y
     if x.dtype not in _DTYPES or y.dtype is not x.dtype:
         x, y = x.float(), y.float()
     x, y, A, f, g = x.detach().contiguous(), y.detach().contiguous(), *(
@@ -119,10 +122,17 @@ def _kept(x, y, f_hat, g_hat, A, *, eps, cost_scale, rho_x, rho_y, tau2, lambda_
                  0.0 if rho_y is None else float(rho_y), tau2, lambda_indef, rtol, atol,
                  _DTYPES[x.dtype], max(0, max_iter))
     L = _lib.lib()
-    ws = torch.empty(L.fs_hvp_workspace_bytes(ctypes.byref(p)), dtype=torch.uint8, device=x.device)
+    size = L.fs_hvp_workspace_bytes if products is None else L.fs_hvp_solved_workspace_bytes
+    ws = torch.empty(size(ctypes.byref(p)), dtype=torch.uint8, device=x.device)
     out = torch.empty((n, d), dtype=torch.float32, device=x.device)
-    _lib.check(L.fs_hvp(ctypes.byref(p), ws.data_ptr(), ws.numel(), out.data_ptr(),
-                        host.data_ptr(), _lib.stream_of(x)), "fs_hvp")
+    if products is None:
+        _lib.check(L.fs_hvp(ctypes.byref(p), ws.data_ptr(), ws.numel(), out.data_ptr(),
+                            host.data_ptr(), _lib.stream_of(x)), "fs_hvp")
+    else:
+        solved = products.problem()
+        _lib.check(L.fs_hvp_solved(ctypes.byref(p), ctypes.byref(solved), products.ws.data_ptr(),
+                                   products.ws.numel(), ws.data_ptr(), ws.numel(), out.data_ptr(),
+                                   host.data_ptr(), _lib.stream_of(x)), "fs_hvp_solved")
     r0, r, converged, iters = (float(host[i]) for i in (1, 3, 5, 6))
     return out, HvpInfo(converged != 0.0, int(iters) if converged else max_iter, r, r0)
 
@@ -137,6 +147,7 @@ def hvp_x_sqeuclid_from_potentials(
     block_m=None, block_n=None, block_k=None, num_warps: int = 4, num_stages: int = 2,
     use_fused_matvec: bool = False, use_batched_cg: bool = False, use_compiled_cg: bool = False,
     use_dense_cg: bool = False, autotune: bool = True, cg_x0: Optional[torch.Tensor] = None,
+    _products=None,
 ):
     """H @ A for OTT-convention potentials (f_hat, g_hat); returns (hvp [n,d], HvpInfo).
 
@@ -170,7 +181,7 @@ def hvp_x_sqeuclid_from_potentials(
             and _kept_ok(x, y, f_hat, g_hat, A, allow_tf32) and _small.held(e, cs, rho_x, rho_y)):
         return _kept(x, y, f_hat, g_hat, A, eps=e, cost_scale=cs, rho_x=rho_x, rho_y=rho_y,
                      tau2=float(tau2), lambda_indef=float(lambda_indef), rtol=float(cg_rtol),
-                     atol=float(cg_atol), max_iter=int(max_cg_iter))
+                     atol=float(cg_atol), max_iter=int(max_cg_iter), products=_products)
     xf, yf, Af = x.float().contiguous(), y.float().contiguous(), A.float().contiguous()
     x_sq = (xf * xf).sum(dim=1).contiguous()
     y_sq = (yf * yf).sum(dim=1).contiguous()

@@ -182,7 +182,7 @@ def sinkhorn_flashstyle_symmetric(
     f_init: Optional[torch.Tensor] = None, g_init: Optional[torch.Tensor] = None,
     label_x: Optional[torch.Tensor] = None, label_y: Optional[torch.Tensor] = None,
     label_cost_matrix: Optional[torch.Tensor] = None, lambda_x: float = 1.0,
-    lambda_y: float = 0.0, solve_info: Optional[dict] = None,
+    lambda_y: float = 0.0, solve_info: Optional[dict] = None, _products: Optional[list] = None,
 ):
     """GeomLoss-style symmetric (Jacobi, averaged) Sinkhorn with an eps schedule.
 
@@ -218,7 +218,7 @@ def sinkhorn_flashstyle_symmetric(
                                       threshold is not None and threshold > 0.0)):
         out = _small_symmetric(x, y, a, b, blur, scaling, use_epsilon_scaling, last_extrapolation,
                                cost_scale, eps, n_iters, diameter, eps_list, rho_x, rho_y,
-                               threshold, check_every, return_n_iters, return_prelast)
+                               threshold, check_every, return_n_iters, return_prelast, _products)
         if out is not None:
             return out
 
@@ -384,9 +384,10 @@ def sinkhorn_flashstyle_symmetric(
 
 def _small_symmetric(x, y, a, b, blur, scaling, use_epsilon_scaling, last_extrapolation, cost_scale,
                      eps, n_iters, diameter, eps_list, rho_x, rho_y, threshold, check_every,
-                     return_n_iters, return_prelast):
+                     return_n_iters, return_prelast, products=None):
     """``sinkhorn_flashstyle_symmetric`` on small clouds (``_small``); None when the schedule is not
-    one that path takes (the general one then builds it, and complains where it has to)."""
+    one that path takes (the general one then builds it, and complains where it has to).  ``products``: a
+    list that receives the ``_small.Products`` of wide rows."""
     sched = {}
     if threshold is not None and (check_every <= 0 or torch.cuda.is_current_stream_capturing()):
         return None
@@ -422,9 +423,11 @@ def _small_symmetric(x, y, a, b, blur, scaling, use_epsilon_scaling, last_extrap
                          cost_scale=float(cost_scale), rho_x=rho_x, rho_y=rho_y, normalize=False, self_terms=False, want_values=False,
                          extrapolate=last_extrapolation, want_loss=False, threshold=threshold,
                          check_every=check_every, prelast=return_prelast and last_extrapolation,
-                         **sched)
+                         keep=products is not None and x.shape[1] > _small.WIDE_D, **sched)
     except _small.Declined:
         return None
+    if products is not None and s.ws is not None:
+        products.append(_small.Products(s.form, s.x, s.y, s.ws))
     (f, f_pre), (g, g_pre) = s.potentials("f"), s.potentials("g")
     out = (f, g)
     if return_prelast and last_extrapolation:

@@ -613,6 +613,42 @@ def test_saved_tensors_pass_through_hooks_and_version_checks():
             loss.backward()
 
 
+# ---- gradients and Hessian-vector products on the products that a solve of wide rows keeps (from 2^22
+# of them on): odd sizes, columns that fill no step, one cloud far larger, half precision, relaxed ----
+@pytest.mark.parametrize("n,m,d,dtype,rho,stop", [(2051, 2100, 129, torch.float32, None, None),
+                                                  (600, 8001, 200, torch.float32, 1.5, None),
+                                                  (8200, 515, 300, torch.float16, None, 0.02),
+                                                  (2305, 1830, 1000, torch.bfloat16, None, None)])
+def test_gradients_on_kept_products(n, m, d, dtype, rho, stop):
+    from flash_sinkhorn_amd import SamplesLoss
+    from flash_sinkhorn_amd.hvp import geomloss_to_ott_potentials, hvp_x_sqeuclid_from_potentials
+    from flash_sinkhorn_amd.kernels import sinkhorn_flashstyle_symmetric as solve
+    x, y, a, b = inputs(n, n, m, d, scale=1.0 / np.sqrt(d), y_shift=0.3 / np.sqrt(d))
+    X, Y, A, B = dev(x, y, a, b)
+    X, Y = X.to(dtype).requires_grad_(), Y.to(dtype).requires_grad_()
+    x, y = (t.detach().float().cpu().numpy() for t in (X, Y))
+    eps = 0.1
+    kw = dict(use_epsilon_scaling=False, eps=eps, n_iters=4)
+    kw.update(n_iters=60, threshold=stop) if stop else None
+    fn = SamplesLoss("sinkhorn", normalize=False, reach_x=rho, reach_y=rho, **kw)
+    gx, gy = torch.autograd.grad(2.0 * fn(A, X, B, Y), [X, Y])
+    relaxed = dict(reach_x=rho, reach_y=rho)
+    _, _, fp, gp = solve(X.detach(), Y.detach(), A, B, return_prelast=True, **relaxed, **kw)
+    wx, wy = oracle.grad_barycentric(x, y, a, b, fp.cpu().numpy(), gp.cpu().numpy(), eps)
+    # (a gradient comes back in the type of the points)
+    tol = GRAD + (0.0 if dtype is torch.float32 else 2.0 ** -8 if dtype is torch.bfloat16 else 2.0 ** -11)
+    assert rel_err(gx.float(), 2.0 * wx) < tol and rel_err(gy.float(), 2.0 * wy) < tol
+    if dtype is torch.float32:
+        (gx,) = torch.autograd.grad(2.0 * fn(A, X, B, Y.detach()), X, create_graph=True)
+        v = torch.randn(n, d, device="cuda", generator=torch.Generator(device="cuda").manual_seed(1))
+        (got,) = torch.autograd.grad((gx * v).sum(), X)
+        ott = geomloss_to_ott_potentials(fp, gp, A, B, eps=eps)
+        want, _ = hvp_x_sqeuclid_from_potentials(X.detach(), Y.detach(), *ott, v, eps=eps,
+                                                 rho_x=rho and rho ** 2, rho_y=rho and rho ** 2)
+        # (the same sums of the same products, formed once instead of twice)
+        assert torch.equal(got, 2.0 * want)
+
+
 # ---- Hessian-vector products: whole rows in registers (2,048, 4,096, 8,192 columns) ----
 @pytest.mark.parametrize("n,m,d", [(1, 1, 1), (37, 2048, 64), (300, 2049, 5), (65, 4097, 130), (257, 200, 129),
                                    (40, 8192, 20)])
