@@ -77,6 +77,7 @@ void dense_plan(const SmallArgs& a, DenseArgs& t) {
   }
   t.chunk = run * 256;
   t.chunks = (iters + run - 1) / run;
+  t.turns = (size_t)a.items * t.n * t.ld * 4 > ((size_t)32 << 20);
 }
 
 int dense_prepare(const SmallArgs& a, const DenseArgs& t, hipStream_t st) {
