@@ -55,7 +55,8 @@ int loss_parts(const SmallArgs& a) {
 
 int padded(int64_t d) { return d <= 16 ? 16 : (d <= 32 ? 32 : (d <= 64 ? 64 : 128)); }
 
-int checked(const fs_small_problem* p) {
+// `solved`: the problem has been, and its list of eps is not looked at again (the workspace has the table).
+int checked(const fs_small_problem* p, bool solved = false) {
   if (!p || !p->x || !p->y) return FS_ERR_NULL_POINTER;
   if (p->n <= 0 || p->m <= 0 || p->d <= 0 || p->items <= 0 || p->items > 65535) return FS_ERR_BAD_SIZE;
   if (p->n > FS_SMALL_MAX_ROWS || p->m > FS_SMALL_MAX_ROWS || p->d > FS_SMALL_MAX_D) return FS_ERR_UNSUPPORTED;
@@ -65,9 +66,9 @@ int checked(const fs_small_problem* p) {
   if (p->sched != 1 && p->entries <= 0) return FS_ERR_BAD_ARGUMENT;
   if (p->sched == 0 && !(p->eps > 0.f)) return FS_ERR_BAD_ARGUMENT;
   if (p->sched == 1 && !(p->blur > 0.0 && p->scaling > 0.0 && p->scaling < 1.0)) return FS_ERR_BAD_ARGUMENT;
-  if (p->sched == 2) {
+  if (p->sched == 2 && p->entries >= kSmallTable) return FS_ERR_UNSUPPORTED;
+  if (p->sched == 2 && !solved) {
     if (!p->eps_list) return FS_ERR_NULL_POINTER;
-    if (p->entries >= kSmallTable) return FS_ERR_UNSUPPORTED;
     for (int i = 0; i < p->entries; ++i)
       if (!(p->eps_list[i] > 0.f)) return FS_ERR_BAD_ARGUMENT;
   }
@@ -454,7 +455,7 @@ int by_width(int64_t d, F&& f) {
 }  // namespace
 
 int dense_solved(const fs_small_problem* p, void* workspace, size_t workspace_bytes, SmallArgs& a, DenseArgs& t) {
-  const int rc = checked(p);
+  const int rc = checked(p, true);
   if (rc != FS_OK) return rc;
   if (!use_dense(p) || p->items != 1 || !p->extrapolate) return FS_ERR_UNSUPPORTED;
   return layout(p, workspace, a, nullptr, &t) > workspace_bytes ? FS_ERR_WORKSPACE_TOO_SMALL : FS_OK;

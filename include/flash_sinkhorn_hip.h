@@ -498,7 +498,7 @@ int fs_hvp(const fs_hvp_problem* problem, void* workspace, size_t workspace_byte
  * What follows a solve of wide rows (`solved`: d > 128, one item, with an extrapolation), from the inner
  * products that its workspace keeps.  fs_dense_grad: the gradient of the cost in x times grad_out [1]
  * (device), fp32 [n, d], at the potentials before the extrapolation; the extrapolated ones normalise
- * the plan's rows.  fs_hvp_solved: fs_hvp of the same points.
+ * the plan's rows.  fs_hvp_solved: fs_hvp of the same points.  A list of eps is not read again.
  */
 size_t fs_dense_grad_workspace_bytes(const fs_small_problem* solved);
 int fs_dense_grad(const fs_small_problem* solved, void* solved_workspace, size_t solved_bytes,

@@ -618,7 +618,8 @@ def test_saved_tensors_pass_through_hooks_and_version_checks():
 @pytest.mark.parametrize("n,m,d,dtype,rho,stop", [(2051, 2100, 129, torch.float32, None, None),
                                                   (600, 8001, 200, torch.float32, 1.5, None),
                                                   (8200, 515, 300, torch.float16, None, 0.02),
-                                                  (2305, 1830, 1000, torch.bfloat16, None, None)])
+                                                  (2305, 1830, 1000, torch.bfloat16, None, None),
+                                                  (2049, 2048, 130, torch.float32, 2.0, "scaling")])
 def test_gradients_on_kept_products(n, m, d, dtype, rho, stop):
     from flash_sinkhorn_amd import SamplesLoss
     from flash_sinkhorn_amd.hvp import geomloss_to_ott_potentials, hvp_x_sqeuclid_from_potentials
@@ -629,7 +630,10 @@ def test_gradients_on_kept_products(n, m, d, dtype, rho, stop):
     x, y = (t.detach().float().cpu().numpy() for t in (X, Y))
     eps = 0.1
     kw = dict(use_epsilon_scaling=False, eps=eps, n_iters=4)
-    kw.update(n_iters=60, threshold=stop) if stop else None
+    if stop == "scaling":  # (a list of eps)
+        kw = dict(blur=eps ** 0.5, scaling=0.5)
+    elif stop:
+        kw.update(n_iters=60, threshold=stop)
     fn = SamplesLoss("sinkhorn", normalize=False, reach_x=rho, reach_y=rho, **kw)
     gx, gy = torch.autograd.grad(2.0 * fn(A, X, B, Y), [X, Y])
     relaxed = dict(reach_x=rho, reach_y=rho)
