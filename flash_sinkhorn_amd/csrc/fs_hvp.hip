@@ -317,7 +317,7 @@ int run_hvp(const fs_hvp_problem* p, const Kept* kept, void* workspace, size_t w
   hipLaunchKernelGGL((hvp_yt_kernel<0>), dim3((a.ld / 16 + 3) / 4, a.yt_blocks), dim3(256), 0, st,
                      (TransposedArgs{a.y, a.scale, a.yt, a.m, a.d, a.ld, a.dtype}));
   if ((rc = dense_gemm(q.last, 1, st)) != FS_OK) return rc;
-  const int blocks = (int)std::min<size_t>(4096, ((size_t)a.n * a.d + 255) / 256);
+  const int blocks = (int)std::min<size_t>(4096, ((size_t)a.n * ((a.d + 3) / 4) + 255) / 256);
   hipLaunchKernelGGL((hvp_result_kernel<0>), dim3(blocks), dim3(256), 0, st, a);
   if (hipGetLastError() != hipSuccess) return FS_ERR_LAUNCH_FAILED;
   // (the last iteration's state, for the caller's report)

@@ -423,14 +423,14 @@ struct DenseGradArgs {
   const float* grad_out;
   float* out;
   u32x4* planes;             // of P, [n blocks][ld / 16][2][64]
-  float* sums;               // [ld / 256][n] sums of a row's P over 256 columns
+  float* sums;               // [n][ld / 256] sums of a row's P over 256 columns
   const float* prod;         // [splits][n][ldo] P y
   int ldo, splits;
 };
 constexpr float kDenseGradScale = 4096.f;  // P is at most one, but for the rounding of L
 
 // Planes of P, in the shape of hvp_v_kernel, and the sums of its rows.  Bound by memory: 8,192 x 8,192 in 116 us (4.6
-// TB/s); the product behind it 520, the result 113, where forming the plan's products again took 1.65 ms.
+// TB/s); the product behind it 520, the result 48, where forming the plan's products again took 1.65 ms.
 template <int T>
 __global__ __launch_bounds__(256) void dense_plan_kernel(const SmallArgs a, const DenseArgs t, const DenseGradArgs g) {
   constexpr int UNIT = 528;
@@ -480,7 +480,7 @@ __global__ __launch_bounds__(256) void dense_plan_kernel(const SmallArgs a, cons
 #pragma unroll
   for (int o = 4; o > 0; o >>= 1) sum[0] += __shfl_xor(sum[0], o, 64);
   const int mine = blk * 32 + wave * 8 + (lane >> 3);
-  if ((lane & 7) == 0 && mine < t.n) g.sums[(size_t)blockIdx.y * t.n + mine] = sum[0];
+  if ((lane & 7) == 0 && mine < t.n) g.sums[(size_t)mine * (t.ld / 256) + blockIdx.y] = sum[0];
   __syncthreads();
   u32x4* out = g.planes + ((size_t)blk * (t.ld / 16) + c0 / 16) * kDenseStep;
 #pragma unroll
@@ -491,31 +491,76 @@ __global__ __launch_bounds__(256) void dense_plan_kernel(const SmallArgs a, cons
   }
 }
 
-// A workgroup per row.
+// Four columns of a row: by a 16-byte word where every row of floats starts at one, else element by element up to
+// the d-th.
+__device__ __forceinline__ bool hvp_wide(const void* p, int d, int dtype) { return dtype == 0 && dense_wide(p, d, 0); }
+__device__ __forceinline__ float4 hvp_load4(const void* p, size_t at, int dtype, bool wide, int left) {
+  if (wide) return *reinterpret_cast<const float4*>(static_cast<const float*>(p) + at);
+  float4 v = make_float4(small_load(p, at, dtype), 0.f, 0.f, 0.f);
+  if (left > 1) v.y = small_load(p, at + 1, dtype);
+  if (left > 2) v.z = small_load(p, at + 2, dtype);
+  if (left > 3) v.w = small_load(p, at + 3, dtype);
+  return v;
+}
+__device__ __forceinline__ void hvp_store4(float* p, size_t at, float4 v, bool wide, int left) {
+  if (wide) {
+    *reinterpret_cast<float4*>(p + at) = v;
+    return;
+  }
+  p[at] = v.x;
+  if (left > 1) p[at + 1] = v.y;
+  if (left > 2) p[at + 2] = v.z;
+  if (left > 3) p[at + 3] = v.w;
+}
+// The parts of a split contraction (their rows are padded to whole words).
+__device__ __forceinline__ float4 hvp_parts(const float* p, size_t stride, int splits) {
+  float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll 4
+  for (int k = 0; k < splits; ++k) {
+    const float4 u = *reinterpret_cast<const float4*>(p + k * stride);
+    v.x += u.x, v.y += u.y, v.z += u.z, v.w += u.w;
+  }
+  return v;
+}
+
+// A workgroup per row, a thread four columns.  Bound by memory: 8,192 x 1,536 in four parts (302 MB) 48 us, 6.2
+// TB/s (by single columns, each thread adding up the row's sums by itself, 113).
 template <int T>
 __global__ __launch_bounds__(256) void dense_grad_kernel(const SmallArgs a, const DenseArgs t, const DenseGradArgs g) {
-  const int row = blockIdx.x;
+  const int row = blockIdx.x, lane = threadIdx.x & 63, parts = t.ld / 256;
+  const bool wx = hvp_wide(a.pts[0], a.d, a.dtype), wo = hvp_wide(g.out, a.d, 0);
   float s = 0.f;
-  for (int c = 0; c < t.ld / 256; ++c) s += g.sums[(size_t)c * t.n + row];
+  for (int c = lane; c < parts; c += 64) s += g.sums[(size_t)row * parts + c];
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
   const float inv = a.scale[1].y / fmaxf(s, 1e-40f), coef = 2.0f * a.cost_scale * g.grad_out[0] * a.wt[0][row];
-  for (int col = threadIdx.x; col < a.d; col += 256) {
-    float v = 0.f;
-    for (int k = 0; k < g.splits; ++k) v += g.prod[((size_t)k * t.n + row) * g.ldo + col];
+  for (int col = 4 * threadIdx.x; col < a.d; col += 1024) {
     const size_t e = (size_t)row * a.d + col;
-    g.out[e] = coef * (small_load(a.pts[0], e, a.dtype) - v * inv);
+    const float4 x = hvp_load4(a.pts[0], e, a.dtype, wx, a.d - col);
+    const float4 v = hvp_parts(g.prod + (size_t)row * g.ldo + col, (size_t)t.n * g.ldo, g.splits);
+    hvp_store4(g.out, e,
+               make_float4(coef * (x.x - v.x * inv), coef * (x.y - v.y * inv), coef * (x.z - v.z * inv), coef * (x.w - v.w * inv)),
+               wo, a.d - col);
   }
 }
 
-// The result.
+// The result, four columns at a time.  Bound by memory: 8,192 x 1,536 in four parts (352 MB) 62 us, 5.7
+// TB/s (by single columns, with a 64-bit division each, 91).
 template <int T>
 __global__ __launch_bounds__(256) void hvp_result_kernel(const HvpArgs a) {
-  const size_t count = (size_t)a.n * a.d;
-  for (size_t e = (size_t)blockIdx.x * 256 + threadIdx.x; e < count; e += (size_t)gridDim.x * 256) {
-    const int row = (int)(e / a.d), col = (int)(e - (size_t)row * a.d);
-    float v = 0.f;
-    for (int s = 0; s < a.splits; ++s) v += a.prod_out[((size_t)s * a.n + row) * a.ldo + col];
-    v *= a.scale[1].y / a.v_scale[row];
-    a.out[e] = a.s[row] * small_load(a.x, e, a.dtype) + 2.0f * a.cs * a.mass[row] * a.A[e] + v;
+  const unsigned quads = (unsigned)(a.d + 3) / 4, count = (unsigned)a.n * quads;  // (at most 65,536 x 4,096)
+  const bool wx = hvp_wide(a.x, a.d, a.dtype), wa = hvp_wide(a.A, a.d, 0), wo = hvp_wide(a.out, a.d, 0);
+  for (unsigned i = blockIdx.x * 256 + threadIdx.x; i < count; i += gridDim.x * 256) {
+    const unsigned row = i / quads;
+    const int col = 4 * (int)(i - row * quads), left = a.d - col;
+    const size_t e = (size_t)row * a.d + col;
+    const float4 x = hvp_load4(a.x, e, a.dtype, wx, left), A = hvp_load4(a.A, e, 0, wa, left);
+    const float4 v = hvp_parts(a.prod_out + (size_t)row * a.ldo + col, (size_t)a.n * a.ldo, a.splits);
+    const float k = a.scale[1].y / a.v_scale[row], s = a.s[row], w = 2.0f * a.cs * a.mass[row];
+    hvp_store4(a.out, e,
+               make_float4(s * x.x + w * A.x + v.x * k, s * x.y + w * A.y + v.y * k, s * x.z + w * A.z + v.z * k,
+                           s * x.w + w * A.w + v.w * k),
+               wo, left);
   }
 }
 
