@@ -32,11 +32,11 @@ __global__ __launch_bounds__(256) void small_table_kernel(const SmallArgs a, con
 
 // Which kernels a problem takes.  d <= 64: both sides of a step from one sweep (fs_pair.hpp) where
 // that saves more than its second launch per step costs.  Fixed eps: from 2e7 logits per step on
-// (one problem of 4,500 points, d = 64, 40 steps: 1.19 against 1.50 ms; 3,000 points: 0.85 against
-// 0.65 ms).  A schedule rewrites the planes behind every step and has few steps: 5e7 (d = 3, 6,500 points:
-// 0.48 against 0.42 ms; 9,000: 0.67 against 0.75), 2e7 where the planes are wide (d = 64, 4,500:
-// 0.58 against 0.62 ms).  Items of a batch fill the chip without it: 12 x 2,048 x 8, debiased, 0.81
-// against 0.66 ms.  Early stopping on a schedule is only built for the small kernels.
+// (one problem of 4,500 points, d = 64, 40 steps: 1.08 against 1.47 ms, d = 3 0.74 against 0.82; 3,600 points, d = 64:
+// 0.88 against 0.78 ms).  A schedule rewrites the planes behind every step and has few steps: 5e7 (d = 3, 6,500 points:
+// 0.40 against 0.40 ms; 9,000: 0.56 against 0.71), 2e7 where the planes are wide (d = 64, 4,500: 0.54 against
+// 0.58 ms; 3,600: 0.44 against 0.33).  Items of a batch fill the chip without it: 12 x 2,048 x 8, debiased, 0.96
+// against 0.74 ms.  Early stopping on a schedule is only built for the small kernels.
 bool use_pair(const fs_small_problem* p) {
   if (p->alternating || p->d > 64 || (p->threshold > 0.f && p->sched != 0)) return false;
   const double n = (double)p->n, m = (double)p->m;
