@@ -1477,13 +1477,6 @@ __global__ __launch_bounds__(256, 2) void pair_sweep_kernel(PairArgsPtr args, in
               went[threadIdx.x]);
 }
 
-template <int T>
-__global__ __launch_bounds__(1024) void pair_args_kernel(const PairArgs a, PairArgs* out) {
-  static_assert(sizeof(PairArgs) % 4 == 0 && sizeof(PairArgs) <= 4096, "one word a thread");
-  if (threadIdx.x < sizeof(PairArgs) / 4)
-    reinterpret_cast<int*>(out)[threadIdx.x] = reinterpret_cast<const int*>(&a)[threadIdx.x];
-}
-
 // Operand planes of one block of 32 rows at an eps: sqrt(qs) times the rows (as a sum of two floats,
 // so that the product of two of them is qs to 2^-46), two fp16 planes.  By 256 threads.
 template <int DP>

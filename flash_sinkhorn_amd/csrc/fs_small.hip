@@ -333,8 +333,12 @@ template <int DP>
 int launch_prep(const SmallArgs& a, const PairArgs& pa, PairArgs* pair_at, hipStream_t st) {
   const int xb = a.blocks[0] > a.blocks[1] ? a.blocks[0] : a.blocks[1];
   hipLaunchKernelGGL((small_stats_kernel<0>), dim3(a.stat_blocks, 2, a.items), dim3(256), 0, st, a);
-  hipLaunchKernelGGL((small_prep_kernel<DP>), dim3(xb + 1, 2, a.items), dim3(256), 0, st, a);
-  if (a.pair) hipLaunchKernelGGL((pair_args_kernel<0>), dim3(1), dim3(1024), 0, st, pa, pair_at);
+  const dim3 grid(xb + 1, 2, a.items);
+  if constexpr (DP <= 64)
+    if (a.pair) hipLaunchKernelGGL((small_prep_kernel<DP, PairArgs>), grid, dim3(256), 0, st, a, pa, pair_at);
+  if (!a.pair)
+    hipLaunchKernelGGL((small_prep_kernel<DP, SmallNothing>), grid, dim3(256), 0, st, a, SmallNothing(),
+                       static_cast<SmallNothing*>(nullptr));
   return hipGetLastError() == hipSuccess ? FS_OK : FS_ERR_LAUNCH_FAILED;
 }
 
