@@ -1713,16 +1713,27 @@ __global__ __launch_bounds__(1024) void pair_merge_kernel(PairArgsPtr args, int 
 // The key blocks (32 keys) that matter to a block of 32 query rows of the gradient: those whose unit the
 // extrapolation, which read the same potentials, did not end.  By a workgroup of 512 threads; as many blocks
 // as it returns are in `ids`, in their order (-1: that step computed every logit).
+//
+// Everything comes by value from the workspace that the gradient is given (pair_blocks), nothing from PairArgs: an
+// autograd node's workspace need not be the memory that the solve ran in (a replayed graph's is the next
+// call's, and hooks of saved tensors bring it back elsewhere), so the addresses inside say nothing.
 struct PairBlocks {
   static constexpr int kMost = 2048;
-  PairArgsPtr args;
+  struct Lists {
+    const unsigned long long* list;
+    const unsigned long long* two_list;
+    int n_items, two_items, two_first, n_st, n_str, chunk, groups, self;
+  };
+  Lists prob[3];
+  const int* lens;
+  const float* state;
   int extrapolate;
-  __device__ __forceinline__ int find(int item, int prob, int qm, int qb, int nkb, unsigned short* ids) const {
-    const PairArgs& a = *(const PairArgs*)args;
-    const PairProblem& pr = a.prob[prob];
-    const int step = a.lens[item * 3 + prob] + 1;
-    const float kind = a.state[((size_t)item * 3 + prob) * kPairStateWords + kPairLists + ((step + 1) % 3) * 32 + 3];
-    if (!extrapolate || kind == 0.f || pr.units == 0.f) return -1;
+  __device__ __forceinline__ int find(int item, int prob_at, int qm, int qb, int nkb, unsigned short* ids) const {
+    const int prob = __builtin_amdgcn_readfirstlane(prob_at);
+    const Lists& pr = this->prob[prob];
+    const int step = lens[item * 3 + prob] + 1;
+    const float kind = state[((size_t)item * 3 + prob) * kPairStateWords + kPairLists + ((step + 1) % 3) * 32 + 3];
+    if (!extrapolate || kind == 0.f) return -1;
     const bool two = kind == 2.f;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int per = pr.chunk / 32;  // blocks of a chunk
@@ -1766,5 +1777,18 @@ struct PairBlocks {
     return __builtin_amdgcn_readfirstlane(count);
   }
 };
+
+// The lists of a solve whose workspace is laid out in `t` (host side).
+inline PairBlocks pair_blocks(const PairArgs& t, int extrapolate) {
+  PairBlocks b = {};
+  b.lens = t.lens;
+  b.state = t.state;
+  b.extrapolate = extrapolate;
+  for (int q = t.first_prob; q < t.nprob; ++q) {
+    const PairProblem& pr = t.prob[q];
+    b.prob[q] = {pr.list, pr.two_list, pr.n_items, pr.two_items, pr.two_first, pr.n_st, pr.n_str, pr.chunk, pr.groups, pr.self};
+  }
+  return b;
+}
 
 }  // namespace fs

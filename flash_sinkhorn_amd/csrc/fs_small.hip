@@ -433,13 +433,12 @@ int launch_pair_step(const SmallArgs& a, const PairArgs& t, PairArgs* at, int st
 }
 
 template <int DP>
-int launch_grad(const SmallArgs& a, const SmallGradArgs& g, PairArgs* pair_at, hipStream_t st) {
+int launch_grad(const SmallArgs& a, const PairArgs& pa, const SmallGradArgs& g, hipStream_t st) {
   const int xb = a.blocks[0] > a.blocks[1] ? a.blocks[0] : a.blocks[1];
   const dim3 grid(!g.out[0] ? a.blocks[1] : (!g.out[1] ? a.blocks[0] : xb), g.out[0] && g.out[1] ? 2 : 1, a.items);
   if constexpr (DP <= 64)
     if (a.pair && skips(a.d)) {
-      hipLaunchKernelGGL((small_grad_kernel<DP, PairBlocks>), grid, dim3(512), 0, st, a, g,
-                         (PairBlocks{(PairArgsPtr)pair_at, a.extrapolate}));
+      hipLaunchKernelGGL((small_grad_kernel<DP, PairBlocks>), grid, dim3(512), 0, st, a, g, pair_blocks(pa, a.extrapolate));
       return hipGetLastError() == hipSuccess ? FS_OK : FS_ERR_LAUNCH_FAILED;
     }
   hipLaunchKernelGGL((small_grad_kernel<DP, SmallAllBlocks>), grid, dim3(512), 0, st, a, g, SmallAllBlocks{});
@@ -621,14 +620,14 @@ int fs_small_grad(const fs_small_problem* p, void* workspace, size_t workspace_b
   if (!grad_out) return FS_ERR_NULL_POINTER;
   if (!p->want_values) return FS_ERR_BAD_ARGUMENT;
   SmallArgs a;
-  PairArgs* pair_at = nullptr;
-  if (layout(p, workspace, a, nullptr, nullptr, &pair_at) > workspace_bytes || !workspace) return FS_ERR_WORKSPACE_TOO_SMALL;
+  PairArgs pa;
+  if (layout(p, workspace, a, &pa) > workspace_bytes || !workspace) return FS_ERR_WORKSPACE_TOO_SMALL;
   if (!grad_x && !grad_y) return FS_OK;
   SmallGradArgs g;
   g.grad_out = grad_out;
   g.out[0] = grad_x;
   g.out[1] = grad_y;
-  return by_width(p->d, [&](auto dp) { return launch_grad<decltype(dp)::value>(a, g, pair_at, (hipStream_t)stream); });
+  return by_width(p->d, [&](auto dp) { return launch_grad<decltype(dp)::value>(a, pa, g, (hipStream_t)stream); });
 }
 
 }  // extern "C"

@@ -459,7 +459,8 @@ int fs_small_potentials(const fs_small_problem* problem, void* workspace, size_t
 
 /*
  * Gradients of `loss` in x and y (NULL: not wanted) times grad_out [items] (device), fp32
- * [items, n, d] and [items, m, d], from the workspace fs_small_solve left behind.
+ * [items, n, d] and [items, m, d], from the workspace fs_small_solve left behind, or from a copy of
+ * it at another address (256-byte aligned): nothing in it is followed as an address.
  * Replaces sinkhorn_geomloss_online_grad_sqeuclid
  * (kernels/sinkhorn_triton_grad_sqeuclid.py:891-1207) for these sizes.
  */

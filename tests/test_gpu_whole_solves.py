@@ -613,6 +613,37 @@ def test_saved_tensors_pass_through_hooks_and_version_checks():
             loss.backward()
 
 
+# ---- gradients along lists read nothing but the workspace that the autograd node holds: behind other
+# losses of the same replayed graph, behind a graph that is forgotten, at another address ----
+@pytest.mark.parametrize("n,m,d,eps,debias", [(4513, 4490, 64, 0.01, False), (3300, 3290, 20, 0.02, True)])
+@pytest.mark.parametrize("between", ["nothing", "graphs forgotten", "saved on the host"])
+def test_gradients_along_lists_after_their_workspace_was_copied(monkeypatch, n, m, d, eps, debias, between):
+    from flash_sinkhorn_amd import SamplesLoss, _graphs
+    fn = SamplesLoss("sinkhorn", normalize=False, use_epsilon_scaling=False, eps=eps, n_iters=25, debias=debias)
+    sets = [dev(*inputs(seed, n, m, d, scale=0.5, y_shift=0.2)) for seed in range(4)]
+    for k, (x, y, _, _) in enumerate(sets):
+        if debias:  # (partners at another distance in every set: other lists of a cloud with itself)
+            x[n // 2:] = x[:n // 2].roll(300 * k, 0) + 0.02 * x[n // 2:]
+        else:
+            x[1::2] = x[:-1:2] + 0.02 * x[1::2]
+        x.requires_grad_(), y.requires_grad_()
+    with monkeypatch.context() as off:
+        off.setattr(_graphs, "ENABLED", False)
+        want = [torch.autograd.grad(fn(a, x, b, y), [x, y]) for x, y, a, b in sets]
+    _graphs.clear()
+    if between == "saved on the host":
+        with torch.autograd.graph.save_on_cpu():
+            losses = [fn(a, x, b, y) for x, y, a, b in sets]
+    else:
+        losses = [fn(a, x, b, y) for x, y, a, b in sets]  # (launch by launch, captured, replayed twice)
+    if between != "nothing":
+        _graphs.clear()
+        torch.cuda.empty_cache()
+    for i in (3, 2, 1, 0):
+        got = torch.autograd.grad(losses[i], sets[i][:2])
+        assert all(torch.equal(g, w) for g, w in zip(got, want[i]))
+
+
 # ---- gradients and Hessian-vector products on the products that a solve of wide rows keeps (from 2^22
 # of them on): odd sizes, columns that fill no step, one cloud far larger, half precision, relaxed ----
 @pytest.mark.parametrize("n,m,d,dtype,rho,stop", [(2051, 2100, 129, torch.float32, None, None),
