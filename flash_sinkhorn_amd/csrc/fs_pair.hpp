@@ -559,6 +559,30 @@ __device__ __forceinline__ void pair_item_two_sided(const PairArgs& a, int batch
   }
 }
 
+// The key that accumulator register r of half-wave h belongs to, in the sub-tile whose first key is `first`; -1
+// behind the last one.  There the bias is kPairFar, and so is that of real keys whose potential or weight is not a
+// number or off every scale (one weight of infinity makes all of its side's such), so the padding
+// may hold a row's largest logit: pair_merge_kernel reads the point of the key that is kept.
+constexpr int pair_key_of(int first, int r, int h, int keys) {
+  const int key = first + 8 * (r >> 2) + 4 * h + (r & 3);
+  return key < keys ? key : -1;
+}
+constexpr bool pair_keys_end_at_the_last_row() {
+  for (int keys = 1; keys <= 130; ++keys)
+    for (int first = 0; first < (keys + 63) / 64 * 64; first += 32) {
+      int seen = 0;
+      for (int e = 0; e < 32; ++e) {
+        const int key = pair_key_of(first, e >> 1, e & 1, keys);
+        if (key >= keys || key < -1 || (key >= 0 && key < first)) return false;
+        seen += key >= 0;
+      }
+      const int left = keys - first;
+      if (seen != (left < 0 ? 0 : left > 32 ? 32 : left)) return false;
+    }
+  return true;
+}
+static_assert(pair_keys_end_at_the_last_row(), "no key behind the last row, and every other one");
+
 // A work item with running maxima in a step in which most units are empty: as pair_item_two_sided, but
 // a unit ends at its hi * hi products where these, the key bias and the bound on the cross products stay
 // kPairGap base-2 units below a lower bound on the logarithm of every row's sum.  That bound is the
@@ -689,7 +713,7 @@ __device__ __forceinline__ unsigned pair_item_two_coarse(const PairArgs& a, int 
           int at = 0;
 #pragma unroll
           for (int r = 1; r < 16; ++r) at = c[r] == top ? r : at;
-          best[rb] = j_begin + sub * 32 + 8 * (at >> 2) + 4 * h + (at & 3);
+          best[rb] = pair_key_of(j_begin + sub * 32, at, h, n_k);
         }
       }
       float p0 = 0.f, p1 = 0.f;

@@ -139,6 +139,23 @@ def test_peaked_plans(n, m, d, eps, mixed, rho):
 
 
 # ---- numbers that fp32 does not hold, or that the library would take for "none" ----
+# One infinite weight leaves every key of its side as far away as the padding behind the last one, which then
+# holds the largest logits of rows whose products are all negative: no such key may be kept (that every index
+# stays inside is asserted where the kernel is compiled), and the next solve finds nothing of it.
+def test_infinite_weights_on_opposite_clouds():
+    from flash_sinkhorn_amd.kernels import sinkhorn_flashstyle_symmetric as solve
+    x, y, a, b = inputs(2, 8013, 7950, 20, scale=0.2)
+    X, Y, A, B = dev(x + 1.0, y - 1.0, a, b)
+    kw = dict(use_epsilon_scaling=False, eps=0.1, n_iters=12)
+    want = solve(X, Y, A, B, **kw)
+    W = A.clone()
+    W[17] = float("inf")
+    for weights in ((W, B), (A, W[:7950])):
+        for t in solve(X, Y, *weights, **kw):
+            assert not t.isfinite().all() or t.abs().max() > 1e3 * want[0].abs().max()
+    assert all(torch.equal(g, w) for g, w in zip(solve(X, Y, A, B, **kw), want))
+
+
 @pytest.mark.parametrize("d", [4, 200])
 def test_relaxations_of_zero_and_less_are_not_strict_marginals(d):
     from flash_sinkhorn_amd import SamplesLoss, sinkhorn_solvers as S
