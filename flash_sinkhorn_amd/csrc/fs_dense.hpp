@@ -27,6 +27,7 @@ struct DenseArgs {
   int steps;               // 16-column steps
   int n, m, ld, items, chunk, chunks, groups;
   float2* part[2];         // (maximum, sum): [items][chunks][n] of the rows, [items][groups][m] of the columns
+  float* top;              // [items][n] the largest logit of a row of x in the extrapolation, for dense_plan_kernel
   const float* pot[2];     // this step's potentials, log weights, norms
   float* out[2];
   const float* l2w[2];
@@ -426,6 +427,7 @@ __global__ __launch_bounds__(256) void dense_merge_kernel(const DenseArgs a) {
   if (alpha != 1.0f) f += (1.0f - alpha) * old;
   if (damp < 1.0f) f -= alpha * (1.0f - damp) * norm;
   a.out[side][at] = f;
+  if (side == 0 && a.step > entries) a.top[at] = M;
 }
 
 // Host side (fs_dense.hip).

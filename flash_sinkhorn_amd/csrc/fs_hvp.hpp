@@ -416,9 +416,11 @@ __global__ __launch_bounds__(256) void hvp_yt_kernel(const TransposedArgs a) {
 }
 
 // The gradient in x of a solve whose products are kept:
-//   2 cs gs w_i (x_i - sum_j P_ij y_j / sum_j P_ij),  P_ij = 2^(qs x_i.y_j + c_j - L_i),
-// c_j the biases of y before the extrapolation and L_i the logarithm of the row's sum over them, which is what
-// the extrapolation made the potential of x of.
+//   2 cs gs w_i (x_i - sum_j P_ij y_j / sum_j P_ij),  P_ij = 2^(qs x_i.y_j + c_j - M_i),
+// c_j the biases of y before the extrapolation and M_i the largest logit of the row, which the extrapolation has
+// formed of the same numbers by the same instruction: a row's largest P is one, whatever the sizes of its
+// logits.  (Not from the potential that it left: with weak relaxations, damp << 1, that is the norm and next
+// to nothing of the row's sum, and what is got back by dividing by damp is off by many powers of two.)
 struct DenseGradArgs {
   const float* grad_out;
   float* out;
@@ -427,7 +429,7 @@ struct DenseGradArgs {
   const float* prod;         // [splits][n][ldo] P y
   int ldo, splits;
 };
-constexpr float kDenseGradScale = 4096.f;  // P is at most one, but for the rounding of L
+constexpr float kDenseGradScale = 4096.f;
 
 // Planes of P, in the shape of hvp_v_kernel, and the sums of its rows.  Bound by memory: 8,192 x 8,192 in 116 us (4.6
 // TB/s); the product behind it 520, the result 48, where forming the plan's products again took 1.65 ms.
@@ -439,9 +441,7 @@ __global__ __launch_bounds__(256) void dense_plan_kernel(const SmallArgs a, cons
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int last = a.lens[0] + 2;
   const float4 coef = small_last_coef(a, 0, 0);
-  const float* f = a.pot[0] + (size_t)(last & 1) * t.n;            // behind the extrapolation
-  const float* y = a.pot[1] + (size_t)((last & 1) ^ 1) * t.m;      // before it
-  const float damp = a.rho[0] > 0.f ? 1.0f / (1.0f + coef.x / a.rho[0]) : 1.0f;
+  const float* y = a.pot[1] + (size_t)((last & 1) ^ 1) * t.m;      // before the extrapolation
   float kb[4];
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
@@ -454,13 +454,12 @@ __global__ __launch_bounds__(256) void dense_plan_kernel(const SmallArgs a, cons
     const int i = wave * 8 + r, row = blk * 32 + i, rc = min(row, t.n - 1);
     float v[4];
     *reinterpret_cast<float4*>(v) = *reinterpret_cast<const float4*>(t.dots + (size_t)rc * t.ld + c0 + 4 * lane);
-    const float fr = f[rc], shift = damp < 1.0f ? (1.0f - damp) * a.norm[0][rc] : 0.f;
-    const float lse = -(fr + shift) / (coef.x * damp * kLn2);
+    const float top = t.top[rc];
     _Float16 hi[4], lo[4];
     sum[r] = 0.f;
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-      const float p = row < t.n ? kDenseGradScale * fast_exp2(__builtin_fmaf(v[k], coef.y, kb[k] - lse)) : 0.f;
+      const float p = row < t.n ? kDenseGradScale * fast_exp2(__builtin_fmaf(v[k], coef.y, kb[k]) - top) : 0.f;
       sum[r] += p;
       hi[k] = (_Float16)p;
       lo[k] = (_Float16)(p - (float)hi[k]);

@@ -279,6 +279,7 @@ size_t layout(const fs_small_problem* p, void* ws, SmallArgs& a, PairArgs* pa = 
     for (int i = 0; i < 2; ++i) take(t.planes[i], items * (size_t)t.blocks[i] * (size_t)t.steps * 2048);
     take(t.part[0], items * (size_t)t.chunks * (size_t)t.n * sizeof(float2));
     take(t.part[1], items * (size_t)t.groups * (size_t)t.m * sizeof(float2));
+    take(t.top, items * (size_t)t.n * 4);
     t.table = a.table;
     t.table_len = a.table_len;
     t.lens = a.lens;

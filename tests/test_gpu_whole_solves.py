@@ -701,6 +701,23 @@ def test_gradients_on_kept_products(n, m, d, dtype, rho, stop):
         assert torch.equal(got, 2.0 * want)
 
 
+# Features as they come (|x|^2 of 3.2e7) with a small reach: potentials are the norms and a little more, and
+# say next to nothing of a row's sum.  The bound is that of logits, gradient_bound.
+def test_gradients_on_kept_products_at_a_small_reach():
+    from flash_sinkhorn_amd import SamplesLoss
+    from flash_sinkhorn_amd.kernels import sinkhorn_flashstyle_symmetric as solve
+    x, y, a, b = inputs(5, 2051, 2100, 200, scale=400.0, y_shift=100.0)
+    X, Y, A, B = dev(x, y, a, b)
+    X.requires_grad_()
+    eps = 4e4
+    kw = dict(use_epsilon_scaling=False, eps=eps, n_iters=4)
+    gx, = torch.autograd.grad(SamplesLoss("sinkhorn", normalize=False, reach=0.4, **kw)(A, X, B, Y), X)
+    _, _, fp, gp = solve(X.detach(), Y, A, B, return_prelast=True, rho_x=0.16, rho_y=0.16, **kw)
+    want, _ = oracle.grad_barycentric(x, y, a, b, fp.cpu().numpy(), gp.cpu().numpy(), eps)
+    off = np.abs(gx.cpu().numpy() - want).max(axis=1)
+    assert (off <= 2.0 * a * gradient_bound(x, y, eps)).all()
+
+
 # ---- Hessian-vector products: whole rows in registers (2,048, 4,096, 8,192 columns) ----
 @pytest.mark.parametrize("n,m,d", [(1, 1, 1), (37, 2048, 64), (300, 2049, 5), (65, 4097, 130), (257, 200, 129),
                                    (40, 8192, 20)])
