@@ -13,6 +13,7 @@ run it (``solve``) and differentiate it (``_SmallLoss``, same conventions as ``_
 from __future__ import annotations
 
 import ctypes
+import os
 import threading
 from types import SimpleNamespace
 from typing import Optional
@@ -30,6 +31,7 @@ MAX_ROWS = 65536
 WIDE_D = 128  # from here on the products of the clouds are kept (fs_dense.hpp), at most this many:
 MAX_KEPT = 1 << 28
 MAX_D = 16384  # rows that the kernels take at all
+KEEP_PRODUCTS = os.environ.get("FLASH_SINKHORN_KEEP_PRODUCTS", "1") != "0"  # (keeps_products)
 _TABLE = 511  # entries of a schedule the device keeps
 # Most workspace of a batch: planes, value operands and vectors of every item, until the backward pass
 # (0.9 MB for a debiased item of 2,048 x 3).  Item by item there is next to nothing to hold.
@@ -327,12 +329,28 @@ class Products:
         return gx
 
 
+def _room(device, nbytes: int) -> bool:
+    """Whether half of the card stays free with ``nbytes`` more of it held (what PyTorch's allocator
+    has idle counts as free).  While a graph is captured its pool is the caller's: not asked."""
+    if torch.cuda.is_current_stream_capturing():
+        return True
+    free, total = torch.cuda.mem_get_info(device)
+    if free - nbytes < total // 2:
+        free += torch.cuda.memory_reserved(device) - torch.cuda.memory_allocated(device)
+    return free - nbytes >= total // 2
+
+
 def keeps_products(x, y) -> bool:
     """Whether a loss keeps the products of its solve for what follows it: of wide rows, where forming them
     again takes longer than a step (up to 2^22 of them a solve is a replayed graph, whose
-    workspace is the next call's).  They stay below 1 GiB."""
-    return (x.ndim == 2 and WIDE_D < x.shape[1] <= MAX_D and x.dtype in _DTYPES and y.dtype is x.dtype
-            and 1 << 22 < x.shape[0] * y.shape[0] <= MAX_KEPT)
+    workspace is the next call's).
+
+    They stay below 1 GiB, but until the loss's graph is freed, and a program may hold hundreds of losses:
+    where less than half of the card would be left, or with FLASH_SINKHORN_KEEP_PRODUCTS=0, the
+    gradient forms them again (8,192 x 1,536: 1.65 ms for 0.70) and nothing is held."""
+    return (KEEP_PRODUCTS and x.ndim == 2 and WIDE_D < x.shape[1] <= MAX_D and x.dtype in _DTYPES
+            and y.dtype is x.dtype and 1 << 22 < x.shape[0] * y.shape[0] <= MAX_KEPT
+            and _room(x.device, 4 * (x.shape[0] * y.shape[0] + (x.shape[0] + y.shape[0]) * x.shape[1])))
 
 
 def _weights(w, lead, count, device, normalize):

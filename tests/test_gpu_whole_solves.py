@@ -718,6 +718,31 @@ def test_gradients_on_kept_products_at_a_small_reach():
     assert (off <= 2.0 * a * gradient_bound(x, y, eps)).all()
 
 
+# Products are held only while half of the card stays free, and not at all where that is asked for: the
+# gradient then forms them again.
+@pytest.mark.parametrize("kept", ["as a rule", "declined", "card half full", "allocator idle"])
+def test_products_are_kept_where_there_is_room(monkeypatch, kept):
+    from flash_sinkhorn_amd import SamplesLoss, _small
+    x, y, a, b = inputs(6, 2600, 2500, 140, scale=0.1)
+    X, Y, A, B = dev(x, y, a, b)
+    X.requires_grad_()
+    fn = SamplesLoss("sinkhorn", normalize=False, use_epsilon_scaling=False, eps=0.1, n_iters=4)
+    want, = torch.autograd.grad(fn(A, X, B, Y), X)
+    if kept == "declined":
+        monkeypatch.setattr(_small, "KEEP_PRODUCTS", False)
+    elif kept != "as a rule":
+        total = 100 << 30
+        monkeypatch.setattr(torch.cuda, "mem_get_info", lambda device: ((50 << 30) + (1 << 20), total))
+        idle = (1 << 30) if kept == "allocator idle" else 0
+        monkeypatch.setattr(torch.cuda, "memory_reserved", lambda device: torch.cuda.memory_allocated(device) + idle)
+    before = torch.cuda.memory_allocated()
+    loss = fn(A, X, B, Y)
+    held = torch.cuda.memory_allocated() - before
+    assert (held >= 4 * 2600 * 2500) == (kept in ("as a rule", "allocator idle"))
+    got, = torch.autograd.grad(loss, X)
+    assert rel_err(got, want.cpu().numpy()) < GRAD
+
+
 # ---- Hessian-vector products: whole rows in registers (2,048, 4,096, 8,192 columns) ----
 @pytest.mark.parametrize("n,m,d", [(1, 1, 1), (37, 2048, 64), (300, 2049, 5), (65, 4097, 130), (257, 200, 129),
                                    (40, 8192, 20)])
