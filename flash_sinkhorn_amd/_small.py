@@ -107,16 +107,27 @@ class Solved:
 
 
 def _size_ok(n: int, m: int, d: int, fixed: bool, self_terms: int, stops: bool,
-             items: int = 1) -> bool:
+             items: int = 1, steps: int = 0) -> bool:
     """Whether a problem of this size is faster here than on the general path, launch by launch.
+    ``steps``: averaged steps at a fixed eps (0: of no matter, the problem is not large).
 
     d > 128: while the kept products stay below 1 GiB; reading them beats forming them at every such
     width (8,192 x 1,536: 0.07 against 0.5 ms a step).
 
-    d <= 64 (``pair_sweep_kernel`` from 2e7 logits per step on): everywhere but at fixed eps beyond
-    2.6e9 logits a step with more than 8 columns, where the first steps, which the general path runs
-    faster, weigh more than the others (60,000 x 40, 20 steps: 16.4 against 15.8 ms; 45,000 x 64: 11.2
-    against 11.2; 50,000 x 64, 100 steps: 24.5 against 32.2; 60,000 x 64, a schedule: 20.6 against 26.3).
+    d <= 64 (``pair_sweep_kernel`` from 2e7 logits per step on): everywhere but for few steps at a fixed eps
+    on two clouds of 24,000 rows and more.  The general path runs the first steps faster, these
+    kernels the others, so the line is a number of steps that grows with the logits of one: 12 per 1e9 of
+    them less 4 on 33 .. 64 columns, 5 less 5 on fewer.  Loss and gradient here / there, ms, N(0, I) at eps
+    0.01 and 0.1, eight clusters at 0.01, 64 columns, after 8 | 20 | 100 steps:
+      40,000: 6.9 / 6.3, 9.2 / 7.6, 8.1 / 7.6 | 8.0 / 8.3, 12.1 / 11.0, 9.6 / 10.1 | 15.6 / 21.3, 30.8 / 34.4, 17.2 / 26.4
+      50,000: 10.3 / 8.9, 13.3 / 10.7, 12.0 / 10.9 | 11.7 / 11.1, 17.8 / 15.1, 13.7 / 13.6 | 21.0 / 26.3, 42.5 / 44.1, 23.8 / 33.4
+      65,000: 16.3 / 12.9, 21.3 / 15.8, 19.1 / 16.0 | 18.0 / 15.5, 27.9 / 21.3, 21.7 / 19.6 | 30.9 / 33.7, 63.4 / 59.6, 35.6 / 42.7
+    and 12 columns:
+      50,000: 6.1 / 5.6, 7.3 / 10.3, 5.9 / 5.7 | 8.9 / 8.1, 12.0 / 16.8, 7.4 / 8.4 | 24.0 / 25.1, 42.6 / 60.1, 16.2 / 26.4
+      65,000: 9.6 / 7.9, 11.7 / 15.7, 9.1 / 7.9 | 13.9 / 11.0, 19.5 / 26.1, 11.1 / 11.4 | 36.5 / 32.4, 71.9 / 95.6, 23.2 / 32.8
+    With self problems these kernels are faster at all of them (60,000 x 64, 10 steps: 18.5 / 20.0, 45,000: 10.7 / 12.7),
+    and so they are on schedules (60,000 x 64: 20.6 / 26.3).
+
     d <= 128, or early stopping on a schedule: the small kernels, which go over the logits once per
     side: up to 2e7 logits at fixed eps (3,000 x 128: 1.05 against 1.54 ms; 4,500: 2.8 against 2.4),
     6e7 on a schedule (6,500 x 128: 1.54 against 1.94 ms; 9,000: 3.1 against 2.8).
@@ -128,7 +139,10 @@ def _size_ok(n: int, m: int, d: int, fixed: bool, self_terms: int, stops: bool,
     if d > 64 or (stops and not fixed):
         logits = (n * m if self_terms < 2 else 0) + ((n * n + m * m) // 2 if self_terms else 0)
         return logits <= (20_000_000 if fixed else 60_000_000)
-    return d <= 8 or not fixed or n * m <= 2_600_000_000
+    if d <= 8 or not fixed or self_terms or not steps or min(n, m) < 24000:
+        return True
+    logits = n * m / 1e9
+    return steps >= (12 * logits - 4 if d > 32 else 5 * logits - 5)
 
 
 def _operands_ok(allow_tf32: bool) -> bool:
@@ -410,7 +424,7 @@ def loss_problem(loss, args, label_x, label_y):
         return None
     if not _size_ok(x.shape[-2], y.shape[-2], x.shape[-1], not loss.use_epsilon_scaling,
                     int(loss.debias and not loss.potentials), loss.threshold is not None,
-                    x.shape[0] if x.ndim == 3 else 1):
+                    x.shape[0] if x.ndim == 3 else 1, 0 if loss.use_epsilon_scaling else loss.n_iters):
         return None
     if x.shape[-1] > WIDE_D and (loss.use_epsilon_scaling or not loss.potentials):
         return None  # (by the solver alone: neither cost, gradients nor diameters are built for it)

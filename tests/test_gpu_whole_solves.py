@@ -352,6 +352,38 @@ def test_one_sweep_gradients_at_small_eps(n, m, d, eps, n_iters):
         assert (off <= 2.0 * w * bound).all()
 
 
+# Large clouds at a fixed eps: on either side of the line between these kernels and the general path both give
+# the same.  (What two solves may lie apart: a potential by four steps' worth of 2^-21 of the largest cost
+# each, a gradient by its own bound and by what such potentials do to the logits.)
+@pytest.mark.parametrize("n,m,d,n_iters,small", [(25013, 26000, 40, 3, False), (25013, 26000, 40, 4, True),
+                                                 (53000, 50007, 33, 30, True), (53000, 50007, 33, 20, False),
+                                                 (53000, 50007, 32, 9, True), (53000, 50007, 16, 8, False)])
+def test_both_routes_of_large_losses_agree(monkeypatch, n, m, d, n_iters, small):
+    from flash_sinkhorn_amd import SamplesLoss, _small
+    assert _small._size_ok(n, m, d, True, 0, False, 1, n_iters) == small
+    assert _small._size_ok(n, m, d, True, 1, False, 1, n_iters) and _small._size_ok(n, m, d, False, 0, False)
+    x, y, a, b = inputs(n, n, m, d, scale=0.5, y_shift=0.2)
+    X, Y, A, B = dev(x, y, a, b)
+    X.requires_grad_(), Y.requires_grad_()
+    eps, out = 0.05, {}
+    kw = dict(use_epsilon_scaling=False, eps=eps, n_iters=n_iters, normalize=False)
+    for route in (True, False):
+        with monkeypatch.context() as forced:
+            forced.setattr(_small, "_size_ok", lambda *_: route)
+            loss = SamplesLoss("sinkhorn", **kw)(A, X, B, Y)
+            out[route] = [loss.detach(), *torch.autograd.grad(loss, [X, Y]),
+                          *SamplesLoss("sinkhorn", potentials=True, **kw)(A, X.detach(), B, Y.detach())]
+    loss = SamplesLoss("sinkhorn", **kw)(A, X, B, Y)
+    assert torch.equal(loss, out[small][0])
+    largest = sum(np.sqrt((t.astype(np.float64) ** 2).sum(1)).max() for t in (x, y)) ** 2
+    off = 4 * 2.0 ** -21 * largest
+    (l0, gx0, gy0, f0, g0), (l1, gx1, gy1, f1, g1) = out[False], out[True]
+    assert (f0 - f1).abs().max() < 2 * off and (g0 - g1).abs().max() < 2 * off and abs(l0 - l1) < 4 * off
+    bound = 2 * gradient_bound(x, y, eps) + 2 * (4 * off / eps) * largest ** 0.5
+    for u, v, w in ((gx0, gx1, A), (gy0, gy1, B)):
+        assert ((u - v).abs().amax(1) <= 2.0 * w * bound).all()
+
+
 def test_one_sweep_gradients_of_peaked_self_problems():
     from flash_sinkhorn_amd import SamplesLoss
     from flash_sinkhorn_amd.kernels import sinkhorn_flashstyle_symmetric as solve
