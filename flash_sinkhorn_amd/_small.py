@@ -362,7 +362,7 @@ def keeps_products(x, y) -> bool:
     They stay below 1 GiB, but until the loss's graph is freed, and a program may hold hundreds of losses:
     where less than half of the card would be left, or with FLASH_SINKHORN_KEEP_PRODUCTS=0, the
     gradient forms them again (8,192 x 1,536: 1.65 ms for 0.70) and nothing is held."""
-    return (KEEP_PRODUCTS and x.ndim == 2 and WIDE_D < x.shape[1] <= MAX_D and x.dtype in _DTYPES
+    return (KEEP_PRODUCTS and x.is_cuda and x.ndim == 2 and WIDE_D < x.shape[1] <= MAX_D and x.dtype in _DTYPES
             and y.dtype is x.dtype and 1 << 22 < x.shape[0] * y.shape[0] <= MAX_KEPT
             and _room(x.device, 4 * (x.shape[0] * y.shape[0] + (x.shape[0] + y.shape[0]) * x.shape[1])))
 

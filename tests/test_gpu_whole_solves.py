@@ -750,6 +750,23 @@ def test_gradients_on_kept_products_at_a_small_reach():
     assert (off <= 2.0 * a * gradient_bound(x, y, eps)).all()
 
 
+# (the workspace comes back at another address; gradient and Hessian-vector product read nothing else)
+def test_kept_products_pass_through_hooks():
+    from flash_sinkhorn_amd import SamplesLoss
+    x, y, a, b = inputs(9, 2051, 2100, 140, scale=0.1)
+    X, Y, A, B = dev(x, y, a, b)
+    X.requires_grad_()
+    fn = SamplesLoss("sinkhorn", normalize=False, use_epsilon_scaling=False, eps=0.1, n_iters=4)
+
+    def pass_through(loss):
+        g, = torch.autograd.grad(loss, X, create_graph=True)
+        return g, torch.autograd.grad((g * Y[:1]).sum(), X)[0]
+    want = pass_through(fn(A, X, B, Y))
+    with torch.autograd.graph.save_on_cpu():
+        loss = fn(A, X, B, Y)
+        assert all(torch.equal(g, w) for g, w in zip(pass_through(loss), want))
+
+
 # Products are held only while half of the card stays free, and not at all where that is asked for: the
 # gradient then forms them again.
 @pytest.mark.parametrize("kept", ["as a rule", "declined", "card half full", "allocator idle"])

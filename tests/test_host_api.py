@@ -140,6 +140,12 @@ def test_clouds_beyond_the_row_limit_of_whole_solves_stay_on_the_general_path(mo
         assert _small.pair_problem(x, y, a, b, True, True, self_terms=2) == fits
 
 
+def test_products_of_points_on_the_host_are_not_asked_about(monkeypatch):
+    from flash_sinkhorn_amd import _small
+    monkeypatch.setattr(_small, "_room", lambda *_: pytest.fail("a card was looked for"))
+    assert not _small.keeps_products(torch.empty(2500, 130), torch.empty(2500, 130))
+
+
 def test_helpers_match_oracle_closed_forms():
     from flash_sinkhorn_amd.kernels._common import (dampening, epsilon_schedule, log_weights,
                                                      max_diameter)
