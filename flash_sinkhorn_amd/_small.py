@@ -125,8 +125,8 @@ def _size_ok(n: int, m: int, d: int, fixed: bool, self_terms: int, stops: bool,
     and 12 columns:
       50,000: 6.1 / 5.6, 7.3 / 10.3, 5.9 / 5.7 | 8.9 / 8.1, 12.0 / 16.8, 7.4 / 8.4 | 24.0 / 25.1, 42.6 / 60.1, 16.2 / 26.4
       65,000: 9.6 / 7.9, 11.7 / 15.7, 9.1 / 7.9 | 13.9 / 11.0, 19.5 / 26.1, 11.1 / 11.4 | 36.5 / 32.4, 71.9 / 95.6, 23.2 / 32.8
-    With self problems these kernels are faster at all of them (60,000 x 64, 10 steps: 18.5 / 20.0, 45,000: 10.7 / 12.7),
-    and so they are on schedules (60,000 x 64: 20.6 / 26.3).
+    With self problems these kernels were faster in all of 160 settings from 26,000 to 60,000 rows (60,000 x 64, 10
+    steps: 18.5 / 20.0, 45,000: 10.7 / 12.7), and so they are on schedules (60,000 x 64: 20.6 / 26.3).
 
     d <= 128, or early stopping on a schedule: the small kernels, which go over the logits once per
     side: up to 2e7 logits at fixed eps (3,000 x 128: 1.05 against 1.54 ms; 4,500: 2.8 against 2.4),
