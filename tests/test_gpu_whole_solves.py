@@ -384,6 +384,56 @@ def test_both_routes_of_large_losses_agree(monkeypatch, n, m, d, n_iters, small)
         assert ((u - v).abs().amax(1) <= 2.0 * w * bound).all()
 
 
+# ... in every form that the line sends to these kernels above 2.6e9 logits
+@pytest.mark.parametrize("form", ["debiased", "batch", "float16", "bfloat16", "relaxed", "no weights", "strided",
+                                  "no extrapolation", "early stopping", "half cost"])
+def test_both_routes_of_the_largest_losses_agree_in_every_form(monkeypatch, form):
+    from flash_sinkhorn_amd import SamplesLoss, _small
+    n, m, d, eps = 52001, 50400, 14, 0.05
+    x, y, a, b = inputs(11, n, m, d, scale=0.5, y_shift=0.2)
+    X, Y, A, B = dev(x, y, a, b)
+    kw = dict(use_epsilon_scaling=False, eps=eps, n_iters=16, normalize=False)
+    if form == "debiased":
+        kw.update(debias=True)
+    if form in ("float16", "bfloat16"):
+        X, Y = X.to(getattr(torch, form)), Y.to(getattr(torch, form))
+    if form == "relaxed":
+        kw.update(reach_x=1.5, reach_y=2.0)
+    if form == "no extrapolation":
+        kw.update(last_extrapolation=False)
+    if form == "early stopping":
+        kw.update(threshold=1e-2, inner_iterations=3)
+    if form == "half cost":
+        kw.update(half_cost=True)
+    if form == "batch":
+        X, Y, A, B = (torch.stack([t, t.roll(5, 0)]) for t in (X, Y, A, B))
+    if form == "strided":
+        X = X.t().contiguous().t()
+    X.requires_grad_(), Y.requires_grad_()
+    args = (X, Y) if form == "no weights" else (A, X, B, Y)
+    runs, solve = [], _small.solve
+    monkeypatch.setattr(_small, "solve", lambda *p, **q: runs.append(1) or solve(*p, **q))
+    fn, out = SamplesLoss("sinkhorn", **kw), []
+    for route in ("these", "general"):
+        if route == "general":
+            monkeypatch.setattr(_small, "_size_ok", lambda *_: False)
+        loss = fn(*args)
+        out.append([loss.detach(), *torch.autograd.grad(loss.sum(), [X, Y])])
+        assert len(runs) == 1
+    x, y = (t.detach().float().reshape(-1, d).cpu().numpy() for t in (X, Y))
+    largest = sum(np.sqrt((t.astype(np.float64) ** 2).sum(1)).max() for t in (x, y)) ** 2
+    off = 4 * 2.0 ** -21 * largest + (1e-2 if form == "early stopping" else 0.0)
+    (l0, gx0, gy0), (l1, gx1, gy1) = out
+    assert l0.shape == l1.shape and (l0 - l1).abs().max() < 12 * off
+    bound = 3 * (2 * gradient_bound(x, y, eps) + 2 * (4 * off / eps) * largest ** 0.5)
+    grain = {"float16": 2.0 ** -10, "bfloat16": 2.0 ** -7}.get(form, 0.0)
+    for u, v, w in ((gx0, gx1, A), (gy0, gy1, B)):
+        w = torch.full_like(w, 1.0 / w.shape[-1]) if form == "no weights" else w
+        assert u.dtype == v.dtype
+        u, v = u.float(), v.float()
+        assert ((u - v).abs().amax(-1) <= 2.0 * w * bound + grain * u.abs().amax(-1) + (grain and 2.0 ** -24)).all()
+
+
 def test_one_sweep_gradients_of_peaked_self_problems():
     from flash_sinkhorn_amd import SamplesLoss
     from flash_sinkhorn_amd.kernels import sinkhorn_flashstyle_symmetric as solve
