@@ -5,10 +5,11 @@
 // 8192 x 8192 x 1536 by six (495 us for a one-sweep step that forms them, about 70 for one that reads
 // 268 MB).  So the products x_i.y_j are formed once per solve, in the same two-plane arithmetic, and
 // kept as fp32 [n][ld]; 288 GB of HBM hold them many times over, and up to 256 MB of them stay
-// in the last-level cache between steps.  Three kernels:
+// in the last-level cache between steps.  Kernels:
 //   dense_gemm_kernel   C = A B^T on two-plane operands in MFMA order
 //   dense_sweep_kernel  both half-updates' soft-max statistics from one reading of the products
 //   dense_merge_kernel  the new potentials from them
+//   dense_rows_kernel   both in one launch, on the products and their transpose (up to 1e7 of them)
 #pragma once
 
 #include "fs_common.hpp"
@@ -22,6 +23,8 @@ constexpr int kDenseStep = 2 * 64;
 
 struct DenseArgs {
   float* dots;             // [items][n][ld], ld a multiple of 256, zero beyond the m-th column
+  float* dots_t;           // [items][m][ld_t]: the same transposed, where a step is one launch (`rows`)
+  int ld_t, rows;          // rows: rows of a wavefront in dense_rows_kernel, 0: dense_sweep_kernel
   u32x4* planes[2];        // [items][blocks][steps][2][64]
   int blocks[2];           // 32-row blocks, a multiple of 8 (zero rows behind the last one)
   int steps;               // 16-column steps
@@ -178,6 +181,8 @@ struct DenseGemmArgs {
   const float2* scale;      // [items][2]: the planes' scales and inverses; null: the result as it is
   const float2* scale_a;    // of the rows where they are not those of the same array
   float* out;               // [splits or items][rows][ld]
+  float* out_t;             // [items][cols][ld_t], the result transposed, or null
+  int cols, ld_t;
   int row_tiles, col_tiles;
 };
 
@@ -267,6 +272,21 @@ __global__ __launch_bounds__(64 * WR * WC, 2) void dense_gemm_kernel(const Dense
 #pragma unroll
         for (int j = 0; j < CB; ++j) out[(size_t)row * g.ld + (ct * TC + wc * CB + j) * 32 + li] = acc[i][j][r] * inv;
     }
+  if (g.out_t == nullptr) return;
+  // (a lane holds four consecutive rows of one column, four times)
+  float* out_t = g.out_t + (size_t)z * g.cols * g.ld_t;
+#pragma unroll
+  for (int j = 0; j < CB; ++j) {
+    const int col = (ct * TC + wc * CB + j) * 32 + li;
+    if (col < g.cols)
+#pragma unroll
+      for (int i = 0; i < RB; ++i)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          *reinterpret_cast<float4*>(out_t + (size_t)col * g.ld_t + (rt * TR + wr * RB + i) * 32 + 8 * q + 4 * h) =
+              make_float4(acc[i][j][4 * q] * inv, acc[i][j][4 * q + 1] * inv, acc[i][j][4 * q + 2] * inv,
+                          acc[i][j][4 * q + 3] * inv);
+  }
 }
 
 __device__ __forceinline__ void dense_join(float& m, float& s, float m2, float s2) {
@@ -421,6 +441,96 @@ __global__ __launch_bounds__(256) void dense_merge_kernel(const DenseArgs a) {
   if (wave > 0 || row >= rows) return;
 #pragma unroll
   for (int w = 1; w < 4; ++w) dense_join(M, S, sh[w][lane].x, sh[w][lane].y);
+  const float rho = a.rho[side], damp = rho > 0.f ? 1.0f / (1.0f + eps / rho) : 1.0f;
+  const float alpha = (a.step == 0 || a.step > entries) ? 1.0f : 0.5f;
+  float f = alpha * (-eps * damp * kLn2 * small_log2(fmaxf(S, 1e-40f), M));
+  if (alpha != 1.0f) f += (1.0f - alpha) * old;
+  if (damp < 1.0f) f -= alpha * (1.0f - damp) * norm;
+  a.out[side][at] = f;
+  if (side == 0 && a.step > entries) a.top[at] = M;
+}
+
+// A whole step in one launch, where the products and their transpose stay in the L2s: a wavefront owns R
+// rows of one side and reads all of their products, so nothing is left to a merge; the columns are rows of
+// the transposed copy, which the product's epilogue writes beside the other.  Bound by the launch and the
+// chain of loads in front of the first logit (1,000 points: 4.0 us a step, 7.5 by sweep and merge), so the
+// products' first piece is on its way before the biases of the keys, which the workgroup's eight
+// wavefronts share in LDS; from 2,000 points on by reading 2 x 4 bytes a product (7.3 us, 4.4 TB/s).  Grid (rows of x, then
+// of y; items).
+constexpr int kDenseRowKeys = 4096;  // most keys (their biases in LDS)
+template <int R>
+__global__ __launch_bounds__(512) void dense_rows_kernel(const DenseArgs a) {
+  constexpr int P = 4;  // 16-byte words of a row per lane and piece: 1024 keys
+  __shared__ __attribute__((aligned(16))) float bias[kDenseRowKeys];
+  const int first = (a.n + 8 * R - 1) / (8 * R), item = blockIdx.y, tid = threadIdx.x;
+  const int side = (int)blockIdx.x >= first, nq = side ? a.m : a.n, nk = side ? a.n : a.m, ld = side ? a.ld_t : a.ld;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int row0 = (((int)blockIdx.x - (side ? first : 0)) * 8 + wave) * R;
+  const float* dots = (side ? a.dots_t : a.dots) + (size_t)item * nq * ld + 4 * lane;
+  const float* row[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) row[r] = dots + (size_t)min(row0 + r, nq - 1) * ld;
+  // (a piece may end behind a row's last word: that word again, for nobody)
+  auto load = [&](float4 (&v)[R][P], int c0) {
+#pragma unroll
+    for (int k = 0; k < P; ++k)
+#pragma unroll
+      for (int r = 0; r < R; ++r) v[r][k] = *reinterpret_cast<const float4*>(row[r] + min(c0 + 256 * k, ld - 256));
+  };
+  float4 v[R][P];
+  load(v, 0);
+  const int entries = a.lens[item * 3];
+  const float4 coef = a.table[(size_t)item * 3 * a.table_len + (a.sched == 0 ? 0 : min(max(a.step - 1, 0), a.table_len - 1))];
+  const size_t at = (size_t)item * nq + min(row0 + min(lane, R - 1), nq - 1);
+  const float old = a.pot[side][at], norm = a.norm[side][at];
+  const float* kpot = a.pot[side ^ 1] + (size_t)item * nk;
+  const float* kl2w = a.l2w[side ^ 1] + (size_t)item * nk;
+  const float eps = coef.x, qs = coef.y, kc = coef.w;
+  for (int j = tid; j < ld; j += 512) {
+    const float b = __builtin_fmaf(kc, kpot[min(j, nk - 1)], kl2w[min(j, nk - 1)]);
+    bias[j] = j < nk ? fmaxf(b, kNegBig) : kNegBig;
+  }
+  __syncthreads();
+  if (a.step > entries + a.extrapolate) return;
+
+  float m[R], s[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) m[r] = kNegBig, s[r] = 0.f;
+  for (int c0 = 0; c0 < ld; c0 += 256 * P) {
+    float4 next[R][P];
+    if (c0 + 256 * P < ld) load(next, c0 + 256 * P);
+#pragma unroll
+    for (int k = 0; k < P; ++k) {
+      if (c0 + 256 * k >= ld) break;
+      const float4 kb = *reinterpret_cast<const float4*>(&bias[c0 + 256 * k + 4 * lane]);
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const float l0 = __builtin_fmaf(v[r][k].x, qs, kb.x), l1 = __builtin_fmaf(v[r][k].y, qs, kb.y);
+        const float l2 = __builtin_fmaf(v[r][k].z, qs, kb.z), l3 = __builtin_fmaf(v[r][k].w, qs, kb.w);
+        const float M = fmaxf(fmaxf(fmaxf(l0, l1), fmaxf(l2, l3)), m[r]);
+        s[r] = s[r] * fast_exp2(m[r] - M) +
+               ((fast_exp2(l0 - M) + fast_exp2(l1 - M)) + (fast_exp2(l2 - M) + fast_exp2(l3 - M)));
+        m[r] = M;
+      }
+    }
+    if (c0 + 256 * P < ld)
+#pragma unroll
+      for (int k = 0; k < P; ++k)
+#pragma unroll
+        for (int r = 0; r < R; ++r) v[r][k] = next[r][k];
+  }
+  float M = kNegBig, S = 0.f;  // lane r: row r
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    float t = m[r];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) t = fmaxf(t, __shfl_xor(t, o, 64));
+    float u = s[r] * fast_exp2(m[r] - t);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) u += __shfl_xor(u, o, 64);
+    if (lane == r) M = t, S = u;
+  }
+  if (lane >= R || row0 + lane >= nq) return;
   const float rho = a.rho[side], damp = rho > 0.f ? 1.0f / (1.0f + eps / rho) : 1.0f;
   const float alpha = (a.step == 0 || a.step > entries) ? 1.0f : 0.5f;
   float f = alpha * (-eps * damp * kLn2 * small_log2(fmaxf(S, 1e-40f), M));

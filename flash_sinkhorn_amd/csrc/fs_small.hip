@@ -276,6 +276,7 @@ size_t layout(const fs_small_problem* p, void* ws, SmallArgs& a, PairArgs* pa = 
     // and 14.53, at it 3.61 and 14.57, 2.75 KiB 3.58 and 15.7; other sizes lie within 1 %.
     at = ((at + 4095) & ~(size_t)4095) + 1024;
     take(t.dots, items * (size_t)t.n * (size_t)t.ld * 4);
+    if (t.rows) take(t.dots_t, items * (size_t)t.m * (size_t)t.ld_t * 4);
     for (int i = 0; i < 2; ++i) take(t.planes[i], items * (size_t)t.blocks[i] * (size_t)t.steps * 2048);
     take(t.part[0], items * (size_t)t.chunks * (size_t)t.n * sizeof(float2));
     take(t.part[1], items * (size_t)t.groups * (size_t)t.m * sizeof(float2));

@@ -59,6 +59,16 @@ def test_schedules_of_every_length(n, m, d, cut):
         assert rel_err(f, wf) < POT and rel_err(g, wg) < POT
 
 
+# ---- wide rows, one launch per step (up to 1e7 products and 4,096 keys): one and two rows a wavefront, pieces
+# of 1,024 keys, and the sizes just past the line ----
+@pytest.mark.parametrize("n,m,d", [(1, 1, 129), (5, 300, 130), (1023, 1025, 200), (1024, 1025, 140),
+                                   (2400, 4096, 129), (30, 4097, 129), (2441, 4096, 131)])
+def test_wide_steps_of_one_launch(n, m, d):
+    x, y, a, b = inputs(n + d, n, m, d, scale=0.3)
+    check_symmetric(x, y, a, b, use_epsilon_scaling=False, eps=0.5, n_iters=4)
+    check_symmetric(x, y, a, b, use_epsilon_scaling=False, eps=0.2, n_iters=3, rho_x=0.7, rho_y=2.0)
+
+
 # ---- both half-updates from one sweep (from 2e7 logits per step on): 256-row groups, chunks of
 # 64-row tiles; eps at which steps go without running maxima, and at which the first ones may not ----
 @pytest.mark.parametrize("n,m,d,eps", [(4481, 4703, 3, 0.5), (4608, 4352, 16, 0.01),
