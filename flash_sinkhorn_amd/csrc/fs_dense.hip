@@ -9,7 +9,8 @@ namespace {
 
 template <int WR, int WC, int RB, int CB>
 int launch_gemm(DenseGemmArgs& g, int items, hipStream_t st) {
-  g.row_tiles = (g.rows + 32 * WR * RB - 1) / (32 * WR * RB);
+  // (the transposed copy is read up to the end of its rows, so every column of it is written)
+  g.row_tiles = ((g.out_t ? g.ld_t : g.rows) + 32 * WR * RB - 1) / (32 * WR * RB);
   g.col_tiles = g.ld / (32 * WC * CB);
   const int tiles = g.row_tiles * g.col_tiles;
   hipLaunchKernelGGL((dense_gemm_kernel<WR, WC, RB, CB>), dim3((tiles + 7) / 8 * 8, items, g.splits), dim3(64 * WR * WC), 0, st, g);
