@@ -71,6 +71,8 @@ _SIGNATURES = {
     "fs_c_transform": (ctypes.c_int, [_P] * 5 + [_I] * 3 + [_F] + _TAIL),
     "fs_small_workspace_bytes": (_Z, [_P]),
     "fs_small_solve": (ctypes.c_int, [_P, _P, _Z, _P, _P, _P, _P]),
+    "fs_small_products_bytes": (_Z, [_P]),
+    "fs_small_solve_products": (ctypes.c_int, [_P, _P, _Z, _P, _Z, _P, _P, _P, _P]),
     "fs_small_potentials": (ctypes.c_int, [_P, _P, _Z, _P, _P]),
     "fs_hvp_workspace_bytes": (_Z, [_P]),
     "fs_hvp": (ctypes.c_int, [_P, _P, _Z, _P, _P, _P]),

@@ -204,6 +204,7 @@ def solve(x, y, a, b, *, items: int, blur: float = 0.0, scaling: float = 0.0, ep
     nbytes = L.fs_small_workspace_bytes(ctypes.byref(p))
     if items > 1 and nbytes > MAX_BATCH_BYTES:
         raise Declined
+    kept = L.fs_small_products_bytes(ctypes.byref(p)) if d > 16 else 0  # (none at narrower rows)
 
     def enqueue(x, y, a, b):  # (of these clouds, or of a graph's copies)
         p.x, p.y, p.a, p.b = x.data_ptr(), y.data_ptr(), _lib.ptr(a), _lib.ptr(b)
@@ -217,8 +218,11 @@ def solve(x, y, a, b, *, items: int, blur: float = 0.0, scaling: float = 0.0, ep
                                      device=x.device) for side, _ in own)
             loss = None
         words = _host_words(items).data_ptr() if sched == 1 or threshold else None
-        rc = L.fs_small_solve(ctypes.byref(p), ws.data_ptr(), ws.numel(), words, _lib.ptr(loss),
-                              pots[0].data_ptr() if want_loss else None, _lib.stream_of(x))
+        # (of the solve alone: what follows it reads the workspace)
+        products = torch.empty(kept, dtype=torch.uint8, device=x.device) if kept else None
+        rc = L.fs_small_solve_products(
+            ctypes.byref(p), ws.data_ptr(), ws.numel(), _lib.ptr(products), kept, words, _lib.ptr(loss),
+            pots[0].data_ptr() if want_loss else None, _lib.stream_of(x))
         if rc > 0:
             if rc == 1:
                 raise ValueError("diameter must be > 0.")
@@ -237,7 +241,7 @@ def solve(x, y, a, b, *, items: int, blur: float = 0.0, scaling: float = 0.0, ep
     # (a graph keeps its products; of a batch it counts all items, and the workspace that a replay
     # may copy)
     if (sched == 0 and not threshold and not keep and _graphs.eligible(items * n, m, entries, x.device)
-            and (d <= WIDE_D or items * n * m <= 1 << 22)
+            and (d <= WIDE_D or items * n * m <= 1 << 22) and kept <= MAX_GRAPH_BYTES
             and (items == 1 or nbytes <= MAX_GRAPH_BYTES)):
         # a fixed sequence of kernels on fixed shapes: replayed (1.9 instead of 3 us per launch)
         key = ("self pair" if self_terms else "alternating" if alternating else "symmetric",

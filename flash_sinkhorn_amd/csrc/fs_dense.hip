@@ -105,8 +105,10 @@ int dense_prepare(const SmallArgs& a, const DenseArgs& t, hipStream_t st) {
   g.steps = t.steps;
   g.rows = t.n;
   g.ld = t.ld;
-  g.scale = a.scale;
-  g.scale_a = nullptr;
+  g.scale[0] = a.scale;
+  g.scale[1] = a.scale + 1;
+  g.step_words = kDenseStep;
+  g.plane_words = 64;
   g.out = t.dots;
   g.out_t = t.rows ? t.dots_t : nullptr;
   g.cols = t.m;
@@ -115,18 +117,21 @@ int dense_prepare(const SmallArgs& a, const DenseArgs& t, hipStream_t st) {
   return dense_gemm(g, a.items, st);
 }
 
+int dense_rows_step(const DenseRowArgs& t, int rows, int sides, int items, hipStream_t st) {
+  int most = 0;
+  for (int i = 0; i < sides; ++i) most = std::max(most, t.s.side[i].nq);
+  const dim3 grid((most + 8 * rows - 1) / (8 * rows), sides, items);
+  if (rows == 1) hipLaunchKernelGGL((dense_rows_kernel<1>), grid, dim3(512), 0, st, t);
+  else hipLaunchKernelGGL((dense_rows_kernel<2>), grid, dim3(512), 0, st, t);
+  return hipGetLastError() == hipSuccess ? FS_OK : FS_ERR_LAUNCH_FAILED;
+}
+
 int dense_step(const SmallArgs& a, DenseArgs& t, int step, hipStream_t st) {
   t.step = step;
   for (int i = 0; i < 2; ++i) {
     const size_t half = (size_t)a.items * a.rows[i];
     t.pot[i] = a.pot[i] + (step & 1) * half;
     t.out[i] = a.pot[i] + ((step & 1) ^ 1) * half;
-  }
-  if (t.rows) {
-    const dim3 grid((t.n + 8 * t.rows - 1) / (8 * t.rows) + (t.m + 8 * t.rows - 1) / (8 * t.rows), a.items);
-    if (t.rows == 1) hipLaunchKernelGGL((dense_rows_kernel<1>), grid, dim3(512), 0, st, t);
-    else hipLaunchKernelGGL((dense_rows_kernel<2>), grid, dim3(512), 0, st, t);
-    return hipGetLastError() == hipSuccess ? FS_OK : FS_ERR_LAUNCH_FAILED;
   }
   const dim3 grid(t.groups, t.chunks, a.items);
   if (t.large) hipLaunchKernelGGL((dense_sweep_kernel<8, 8>), grid, dim3(512), 0, st, t);

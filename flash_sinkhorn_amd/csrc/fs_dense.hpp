@@ -178,12 +178,14 @@ struct DenseGemmArgs {
   int a_blocks, b_blocks;   // blocks per item
   int steps, rows, ld;      // rows: of the result, per item
   int splits, run;          // parts of the contraction (each a result of its own) and their steps
-  const float2* scale;      // [items][2]: the planes' scales and inverses; null: the result as it is
-  const float2* scale_a;    // of the rows where they are not those of the same array
+  const float2* scale[2];   // of the rows' and of the columns' planes, with inverses, two words an item; null: none
   float* out;               // [splits or items][rows][ld]
   float* out_t;             // [items][cols][ld_t], the result transposed, or null
   int cols, ld_t;
   int row_tiles, col_tiles;
+  // words from one 16-column step to the next and from the hi to the lo plane (of both operands): kDenseStep and 64,
+  // or those of planes in the order of small_prep_kernel, whose blocks are not padded to whole tiles
+  int step_words, plane_words;
 };
 
 template <int WR, int WC, int RB, int CB>
@@ -210,16 +212,17 @@ __global__ __launch_bounds__(64 * WR * WC, 2) void dense_gemm_kernel(const Dense
   for (int i = 0; i < LOADS; ++i) {
     const int p = wave * LOADS + i, blk = p / 2;
     const bool of_a = blk < TR;
-    const int gb = of_a ? rt * TR + blk : ct * TC + blk - TR;  // (blocks are padded to whole tiles of 8)
+    // (past the last block: that one again, for results that nobody takes)
+    const int gb = of_a ? min(rt * TR + blk, g.a_blocks - 1) : min(ct * TC + blk - TR, g.b_blocks - 1);
     src[i] = (of_a ? g.a + ((size_t)z * g.a_blocks + gb) * (size_t)g.steps * kDenseStep
                    : g.b + ((size_t)z * g.b_blocks + gb) * (size_t)g.steps * kDenseStep) +
-             ((size_t)k_begin * kDenseStep + (p & 1) * 64 + lane);
+             ((size_t)k_begin * g.step_words + (p & 1) * g.plane_words + lane);
   }
   auto stage = [&](int k, int buf) {
 #pragma unroll
     for (int i = 0; i < LOADS; ++i)
       __builtin_amdgcn_global_load_lds(
-          (const __attribute__((address_space(1))) void*)(src[i] + (size_t)min(k, steps - 1) * kDenseStep),
+          (const __attribute__((address_space(1))) void*)(src[i] + (size_t)min(k, steps - 1) * g.step_words),
           (__attribute__((address_space(3))) void*)(&lds[(buf * PIECES + wave * LOADS + i) * 64]), 16, 0, 0);
   };
   const unsigned base = (unsigned)(size_t)(const __attribute__((address_space(3))) u32x4*)&lds[0] + lane * 16;
@@ -261,7 +264,7 @@ __global__ __launch_bounds__(64 * WR * WC, 2) void dense_gemm_kernel(const Dense
     });
   }
   __builtin_amdgcn_s_waitcnt(0);
-  const float inv = g.scale == nullptr ? 1.0f : (g.scale_a ? g.scale_a[0].y : g.scale[z * 2].y) * g.scale[z * 2 + 1].y;
+  const float inv = g.scale[0] == nullptr ? 1.0f : g.scale[0][z * 2].y * g.scale[1][z * 2].y;
   float* out = g.out + (size_t)(z + split) * g.rows * g.ld;  // (one item where the contraction is split)
 #pragma unroll
   for (int i = 0; i < RB; ++i)
@@ -450,23 +453,31 @@ __global__ __launch_bounds__(256) void dense_merge_kernel(const DenseArgs a) {
   if (side == 0 && a.step > entries) a.top[at] = M;
 }
 
-// A whole step in one launch, where the products and their transpose stay in the L2s: a wavefront owns R
-// rows of one side and reads all of their products, so nothing is left to a merge; the columns are rows of
-// the transposed copy, which the product's epilogue writes beside the other.  Bound by the launch and the
-// chain of loads in front of the first logit (1,000 points: 4.0 us a step, 7.5 by sweep and merge), so the
-// products' first piece is on its way before the biases of the keys, which the workgroup's eight
-// wavefronts share in LDS; from 2,000 points on by reading 2 x 4 bytes a product (7.3 us, 4.4 TB/s).  Grid (rows of x, then
-// of y; items).
+// A step of every problem in one launch, where the products and their transposes stay in the L2s and the last-level
+// cache: a wavefront owns R rows of one side and reads all of their products, so nothing is left to a merge; the
+// columns of the xy products are rows of a transposed copy, which the product's epilogue writes beside the
+// other.  Bound by the launch and the chain of loads in front of the first logit (1,000 points: 4.0 us a
+// step, 7.5 by sweep and merge), so the products' first piece is on its way before the biases of the keys, which
+// the workgroup's eight wavefronts share in LDS; from 2,000 points on by reading 2 x 4 bytes a product (7.3 us,
+// 4.4 TB/s).  Grid (rows of the largest side, sides, items).
 constexpr int kDenseRowKeys = 4096;  // most keys (their biases in LDS)
+struct DenseRowArgs {
+  SmallStepArgs s;        // (the planes are not read)
+  const float* dots[4];   // [items][rows][ld] of every side
+  int ld[4];
+  float* top;             // [items][nq] the largest logit of a row of side 0 in the extrapolation, or null
+};
 template <int R>
-__global__ __launch_bounds__(512) void dense_rows_kernel(const DenseArgs a) {
+__global__ __launch_bounds__(512) void dense_rows_kernel(const DenseRowArgs a) {
   constexpr int P = 4;  // 16-byte words of a row per lane and piece: 1024 keys
   __shared__ __attribute__((aligned(16))) float bias[kDenseRowKeys];
-  const int first = (a.n + 8 * R - 1) / (8 * R), item = blockIdx.y, tid = threadIdx.x;
-  const int side = (int)blockIdx.x >= first, nq = side ? a.m : a.n, nk = side ? a.n : a.m, ld = side ? a.ld_t : a.ld;
+  const int side = blockIdx.y, item = blockIdx.z, tid = threadIdx.x;
+  const SmallStepSide& sd = a.s.side[side];
+  const int nq = sd.nq, nk = sd.nk, ld = a.ld[side];
+  if ((int)blockIdx.x * 8 * R >= nq) return;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-  const int row0 = (((int)blockIdx.x - (side ? first : 0)) * 8 + wave) * R;
-  const float* dots = (side ? a.dots_t : a.dots) + (size_t)item * nq * ld + 4 * lane;
+  const int row0 = ((int)blockIdx.x * 8 + wave) * R;
+  const float* dots = a.dots[side] + (size_t)item * nq * ld + 4 * lane;
   const float* row[R];
 #pragma unroll
   for (int r = 0; r < R; ++r) row[r] = dots + (size_t)min(row0 + r, nq - 1) * ld;
@@ -479,19 +490,19 @@ __global__ __launch_bounds__(512) void dense_rows_kernel(const DenseArgs a) {
   };
   float4 v[R][P];
   load(v, 0);
-  const int entries = a.lens[item * 3];
-  const float4 coef = a.table[(size_t)item * 3 * a.table_len + (a.sched == 0 ? 0 : min(max(a.step - 1, 0), a.table_len - 1))];
+  const int entries = sd.lens[item * 3], step = a.s.step;
+  const float4 coef = sd.coef[(size_t)item * a.s.coef_stride];
   const size_t at = (size_t)item * nq + min(row0 + min(lane, R - 1), nq - 1);
-  const float old = a.pot[side][at], norm = a.norm[side][at];
-  const float* kpot = a.pot[side ^ 1] + (size_t)item * nk;
-  const float* kl2w = a.l2w[side ^ 1] + (size_t)item * nk;
+  const float old = sd.old[at], norm = sd.norm[at];
+  const float* kpot = sd.kpot + (size_t)item * nk;
+  const float* kl2w = sd.kl2w + (size_t)item * nk;
   const float eps = coef.x, qs = coef.y, kc = coef.w;
   for (int j = tid; j < ld; j += 512) {
     const float b = __builtin_fmaf(kc, kpot[min(j, nk - 1)], kl2w[min(j, nk - 1)]);
     bias[j] = j < nk ? fmaxf(b, kNegBig) : kNegBig;
   }
   __syncthreads();
-  if (a.step > entries + a.extrapolate) return;
+  if (step > entries + a.s.extrapolate) return;  // (its schedule is shorter)
 
   float m[R], s[R];
 #pragma unroll
@@ -531,13 +542,13 @@ __global__ __launch_bounds__(512) void dense_rows_kernel(const DenseArgs a) {
     if (lane == r) M = t, S = u;
   }
   if (lane >= R || row0 + lane >= nq) return;
-  const float rho = a.rho[side], damp = rho > 0.f ? 1.0f / (1.0f + eps / rho) : 1.0f;
-  const float alpha = (a.step == 0 || a.step > entries) ? 1.0f : 0.5f;
+  const float rho = sd.rho, damp = rho > 0.f ? 1.0f / (1.0f + eps / rho) : 1.0f;
+  const float alpha = (step == 0 || step > entries) ? 1.0f : 0.5f;
   float f = alpha * (-eps * damp * kLn2 * small_log2(fmaxf(S, 1e-40f), M));
   if (alpha != 1.0f) f += (1.0f - alpha) * old;
   if (damp < 1.0f) f -= alpha * (1.0f - damp) * norm;
-  a.out[side][at] = f;
-  if (side == 0 && a.step > entries) a.top[at] = M;
+  sd.out[at] = f;
+  if (side == 0 && a.top != nullptr && step > entries) a.top[at] = M;
 }
 
 // Host side (fs_dense.hip).
@@ -546,5 +557,6 @@ void dense_gemm_plan(DenseGemmArgs& g, bool may_split);
 int dense_gemm(DenseGemmArgs& g, int items, hipStream_t st);
 int dense_prepare(const SmallArgs& a, const DenseArgs& t, hipStream_t st);
 int dense_step(const SmallArgs& a, DenseArgs& t, int step, hipStream_t st);
+int dense_rows_step(const DenseRowArgs& t, int rows, int sides, int items, hipStream_t st);
 
 }  // namespace fs

@@ -129,7 +129,7 @@ size_t layout(const fs_hvp_problem* p, void* ws, HvpPlan& q, bool shared, const 
   take(a.vplanes, (size_t)v_blocks * (L / 16) * 2048);
   take(a.yt, (size_t)a.yt_blocks * (L / 16) * 2048);
   auto product = [&](DenseGemmArgs& g, const u32x4* rows, int row_blocks, const u32x4* cols, int col_blocks, int steps, int ld,
-                     const float2* scale, const float2* scale_a, const float* out, bool split) {
+                     const float2* scale_a, const float2* scale_b, const float* out, bool split) {
     g.a = rows;
     g.b = cols;
     g.a_blocks = row_blocks;
@@ -137,15 +137,17 @@ size_t layout(const fs_hvp_problem* p, void* ws, HvpPlan& q, bool shared, const 
     g.steps = steps;
     g.rows = n;
     g.ld = ld;
-    g.scale = scale;
-    g.scale_a = scale_a;
+    g.scale[0] = scale_a;
+    g.scale[1] = scale_b;
+    g.step_words = kDenseStep;
+    g.plane_words = 64;
     g.out = const_cast<float*>(out);
     dense_gemm_plan(g, split);
   };
-  product(q.dots, q.td.planes[0], q.td.blocks[0], q.td.planes[1], q.td.blocks[1], q.td.steps, a.ld, q.pts.scale, nullptr,
-          a.dots, false);
-  product(q.prod, q.ta.planes[0], q.ta.blocks[0], q.td.planes[1], q.td.blocks[1], q.td.steps, a.ld, q.pts.scale,
-          q.dir.scale, a.prod, false);
+  product(q.dots, q.td.planes[0], q.td.blocks[0], q.td.planes[1], q.td.blocks[1], q.td.steps, a.ld, q.pts.scale,
+          q.pts.scale + 1, a.dots, false);
+  product(q.prod, q.ta.planes[0], q.ta.blocks[0], q.td.planes[1], q.td.blocks[1], q.td.steps, a.ld, q.dir.scale,
+          q.pts.scale + 1, a.prod, false);
   product(q.last, a.vplanes, v_blocks, a.yt, a.yt_blocks, (int)(L / 16), a.ldo, nullptr, nullptr, nullptr, true);
   a.splits = q.last.splits;
   take(a.prod_out, (size_t)a.splits * N * a.ldo * 4);
@@ -204,6 +206,8 @@ size_t grad_layout(const SmallArgs& s, const DenseArgs& t, void* ws, GradPlan& q
   m.steps = (int)steps;
   m.rows = t.n;
   m.ld = g.ldo;
+  m.step_words = kDenseStep;
+  m.plane_words = 64;
   dense_gemm_plan(m, true);
   g.splits = m.splits;
   take(m.out, (size_t)m.splits * t.n * g.ldo * 4);

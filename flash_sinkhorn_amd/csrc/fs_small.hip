@@ -47,6 +47,77 @@ bool use_pair(const fs_small_problem* p) {
 // Wide rows: the products are formed once and kept (fs_dense.hpp).
 bool use_dense(const fs_small_problem* p) { return p->d > kSmallMaxD; }
 
+// Narrower rows whose products are formed once and kept for the steps of a solve (dense_rows_kernel).  A workgroup
+// of small_step_kernel reads the planes of all keys for 32 rows, 2, 4, 8 or 16 bytes a logit by the padded width, from the
+// caches; a kept product is 4.  `read`: the bytes of a step, which have to stay in the L2s (4 MiB each) against the narrower
+// planes.  Potentials after 50 steps at a fixed eps, and after a schedule of 14, planes -> products, us:
+//   d = 64:  256 points 244 -> 193, 74 -> 74; 1,000: 383 -> 236, 106 -> 83; 2,048 (32 MiB): 572 -> 397, 156 -> 126;
+//            2,500 (49 MiB): 657 -> 712, 177 -> 201; with self problems 1,000 (16 MiB): 388 -> 306, 110 -> 101;
+//            1,500 (35 MiB): 477 -> 507, 137 -> 159
+//   d = 128: 256: 327 -> 202, 93 -> 73; 1,000: 585 -> 244, 154 -> 85; 3,000 (70 MiB): 1,192 -> 845, 305 -> 243; 4,000
+//            (125 MiB): 1,639 -> 1,447, 413 -> 391 (d = 100: 401 -> 417); with self problems 2,500 (98 MiB): 1,957 -> 1,083
+//   d = 32, fixed eps: 512: 238 -> 200; 1,000 (8 MiB): 302 -> 233; 1,500 (18 MiB): 359 -> 345; its schedules 89 -> 80 to
+//            73 -> 79; d <= 16: 270 -> 230 at 1,000, 0.93 to 1.0 at 256 and 1,500
+bool use_products(const fs_small_problem* p) {
+  if (p->alternating || p->d <= 16 || use_dense(p) || use_pair(p)) return false;
+  const double n = (double)p->n, m = (double)p->m;
+  const double ldx = std::ceil(n / 256) * 256, ldy = std::ceil(m / 256) * 256;
+  if (std::max(ldx, ldy) > kDenseRowKeys) return false;
+  if (p->sched != 1 && p->entries < 8) return false;  // (forming them takes what some six steps gain)
+  const double read = 4.0 * (double)p->items *
+                      ((p->self_terms < 2 ? n * ldy + m * ldx : 0.) + (p->self_terms ? n * ldx + m * ldy : 0.));
+  if (p->d <= 32) return p->sched == 0 && read <= 9.0e6;
+  return read <= (p->d <= 64 ? 3.4e7 : 1.1e8);
+}
+
+// The products of every side [items][rows][ld] and bytes they take.
+struct Products {
+  float* dots[4];
+  int ld[4];
+  size_t bytes;
+};
+Products products_at(const SmallArgs& a, void* at) {
+  Products t;
+  char* p = static_cast<char*>(at);
+  for (int side = 0; side < 4; ++side) {
+    const int mat = side & 1, keys = side < 2 ? mat ^ 1 : mat;
+    t.dots[side] = nullptr;
+    t.ld[side] = (a.rows[keys] + 255) / 256 * 256;
+    if (side < 2 ? a.self == 2 : a.self == 0) continue;
+    t.dots[side] = reinterpret_cast<float*>(p);
+    p += (size_t)a.items * a.rows[mat] * t.ld[side] * 4;  // (a multiple of 1 KiB)
+  }
+  t.bytes = (size_t)(p - static_cast<char*>(at));
+  return t;
+}
+
+// Forms them, from the planes of small_prep_kernel.
+int form_products(const SmallArgs& a, const Products& t, int steps, hipStream_t st) {
+  for (int prob = a.self == 2 ? 1 : 0; prob < (a.self ? 3 : 1); ++prob) {
+    const int r = prob == 2 ? 1 : 0, c = prob == 0 ? 1 : r;
+    DenseGemmArgs g;
+    std::memset(&g, 0, sizeof(g));
+    g.a = a.planes[r];
+    g.b = a.planes[c];
+    g.a_blocks = a.blocks[r];
+    g.b_blocks = a.blocks[c];
+    g.steps = steps;
+    g.step_words = 64;
+    g.plane_words = steps * 64;
+    g.rows = a.rows[r];
+    g.cols = a.rows[c];
+    g.scale[0] = a.scale + r;
+    g.scale[1] = a.scale + c;
+    g.out = t.dots[prob == 0 ? 0 : prob + 1];
+    g.ld = t.ld[prob == 0 ? 0 : prob + 1];
+    if (prob == 0) g.out_t = t.dots[1], g.ld_t = t.ld[1];
+    dense_gemm_plan(g, false);
+    const int rc = dense_gemm(g, a.items, st);
+    if (rc != FS_OK) return rc;
+  }
+  return FS_OK;
+}
+
 // Workgroups over which the loss of an item is spread: one for what a workgroup does in three rounds.
 int loss_parts(const SmallArgs& a) {
   const int rows = std::max(a.rows[0], a.rows[1]);
@@ -377,6 +448,18 @@ SmallStepArgs step_args(const SmallArgs& a, int step) {
   return t;
 }
 
+int launch_rows(const SmallArgs& a, int step, const float* const* dots, const int* ld, float* top, int rows, hipStream_t st) {
+  DenseRowArgs t;
+  t.s = step_args(a, step);
+  const int first = a.self == 2 ? 2 : 0, sides = a.self == 1 ? 4 : 2;
+  for (int i = 0; i < 4; ++i) {
+    t.dots[i] = i < sides ? dots[first + i] : nullptr;
+    t.ld[i] = i < sides ? ld[first + i] : 0;
+  }
+  t.top = top;
+  return dense_rows_step(t, rows, sides, a.items, st);
+}
+
 // Wavefronts that share the keys of 32 rows: sixteen where eight would leave the chip half empty and
 // there are keys for them (3,001 x 4,567 x 33: 326 against 424 us a solve; from 257 workgroups on, and
 // at 128 columns, where they cost registers, eight are faster).
@@ -478,8 +561,20 @@ size_t fs_small_workspace_bytes(const fs_small_problem* p) {
   return layout(p, nullptr, a);
 }
 
+size_t fs_small_products_bytes(const fs_small_problem* p) {
+  if (checked(p) != FS_OK || !use_products(p)) return 0;
+  SmallArgs a;
+  layout(p, nullptr, a);
+  return products_at(a, nullptr).bytes;
+}
+
 int fs_small_solve(const fs_small_problem* p, void* workspace, size_t workspace_bytes, int* host_words,
                    float* loss, float* pots, void* stream) {
+  return fs_small_solve_products(p, workspace, workspace_bytes, nullptr, 0, host_words, loss, pots, stream);
+}
+
+int fs_small_solve_products(const fs_small_problem* p, void* workspace, size_t workspace_bytes, void* products,
+                            size_t products_bytes, int* host_words, float* loss, float* pots, void* stream) {
   int rc = checked(p);
   if (rc != FS_OK) return rc;
   if ((p->sched == 1 || p->threshold > 0.f) && !host_words) return FS_ERR_NULL_POINTER;
@@ -488,6 +583,13 @@ int fs_small_solve(const fs_small_problem* p, void* workspace, size_t workspace_
   DenseArgs da;
   if (!workspace || layout(p, workspace, a, &pa, &da, &pair_at) > workspace_bytes) return FS_ERR_WORKSPACE_TOO_SMALL;
   hipStream_t st = (hipStream_t)stream;
+  const bool dense = use_dense(p);
+  const bool kept = products && use_products(p);
+  Products by_rows = products_at(a, products);
+  if (kept && by_rows.bytes > products_bytes) return FS_ERR_WORKSPACE_TOO_SMALL;
+  if (dense) by_rows = Products{{da.dots, da.dots_t}, {da.ld, da.ld_t}, 0};
+  const double rows = (double)a.items * (a.rows[0] + a.rows[1]) * (a.self == 1 ? 2 : 1);
+  const int wave_rows = dense ? da.rows : (kept ? (rows <= 2048 ? 1 : 2) : 0);
   int entries = a.entries;
   a.host_words = host_words;
   if (a.sched == 1) {
@@ -502,17 +604,18 @@ int fs_small_solve(const fs_small_problem* p, void* workspace, size_t workspace_
     hipLaunchKernelGGL((small_table_kernel<0>), dim3(a.items * 3), dim3(256), 0, st, a, t);
     if (hipGetLastError() != hipSuccess) return FS_ERR_LAUNCH_FAILED;
   }
-  const bool dense = use_dense(p);
   rc = dense ? dense_prepare(a, da, st) : by_width(p->d, [&](auto dp) {
     constexpr int DP = decltype(dp)::value;
     const int r = launch_prep<DP>(a, pa, pair_at, st);
     if constexpr (DP <= 64)
       if (r == FS_OK && a.pair) return launch_pair_merge<DP>(a, pa, pair_at, -1, st);
+    if (r == FS_OK && kept) return form_products(a, by_rows, DP / 16, st);
     return r;
   });
   if (rc != FS_OK) return rc;
   const int p0 = a.self == 2 ? 1 : 0, p1 = a.self == 0 ? 1 : 3;  // the problems that are solved
   auto run_step = [&](int s) {
+    if (wave_rows) return launch_rows(a, s, by_rows.dots, by_rows.ld, dense ? da.top : nullptr, wave_rows, st);
     if (dense) return dense_step(a, da, s, st);
     return by_width(p->d, [&](auto dp) {
       constexpr int DP = decltype(dp)::value;

@@ -447,6 +447,13 @@ typedef struct fs_small_problem {
 size_t fs_small_workspace_bytes(const fs_small_problem* problem);
 int fs_small_solve(const fs_small_problem* problem, void* workspace, size_t workspace_bytes,
                    int* host_words, float* loss, float* pots, void* stream);
+/*
+ * The same on inner products that are formed once: fs_small_products_bytes says how much memory they take (0: the
+ * steps of this problem are faster without).  Nothing behind the call reads them.
+ */
+size_t fs_small_products_bytes(const fs_small_problem* problem);
+int fs_small_solve_products(const fs_small_problem* problem, void* workspace, size_t workspace_bytes, void* products,
+                            size_t products_bytes, int* host_words, float* loss, float* pots, void* stream);
 
 /*
  * The standard potentials of the solve that left `workspace` behind, each into memory of its own.

@@ -69,6 +69,55 @@ def test_wide_steps_of_one_launch(n, m, d):
     check_symmetric(x, y, a, b, use_epsilon_scaling=False, eps=0.2, n_iters=3, rho_x=0.7, rho_y=2.0)
 
 
+# ---- narrower rows on kept products (8 steps and more; up to 3.4e7 bytes of them at d <= 64): planes of one to
+# eight 16-column steps, blocks that are no multiple of the product's tiles, rows of 4,096 keys ----
+@pytest.mark.parametrize("n,m,d", [(1, 1, 17), (31, 33, 33), (255, 257, 32), (1025, 769, 48), (2048, 2048, 64),
+                                   (5, 4096, 65), (2050, 1023, 128)])
+def test_steps_on_products_of_narrow_rows(n, m, d):
+    x, y, a, b = inputs(n + d, n, m, d, scale=0.3)
+    check_symmetric(x, y, a, b, use_epsilon_scaling=False, eps=0.5, n_iters=8, rho_x=0.7, rho_y=2.0)
+    check_symmetric(x, y, a, b, use_epsilon_scaling=False, eps=0.5, n_iters=8)
+
+
+@pytest.mark.parametrize("self_terms", [0, 1, 2])
+@pytest.mark.parametrize("n,m,d,items", [(300, 257, 40, 3), (513, 200, 100, 1), (90, 300, 64, 2)])
+def test_steps_on_products_equal_those_on_planes(n, m, d, items, self_terms):
+    """The same call of the library with and without memory for the products: potentials of every problem, of every
+    item of a batch, on a schedule by diameter."""
+    import ctypes
+    from flash_sinkhorn_amd import _lib, _small
+    L, gen = _lib.lib(), torch.Generator(device="cuda").manual_seed(n + d)
+    x, y = (0.4 * torch.randn(items, k, d, device="cuda", generator=gen) for k in (n, m))
+    p = _small.Problem(x.data_ptr(), y.data_ptr(), None, None, None, n, m, d, items, 0.1, 0.5, 1.0, 0.0, 0.0, 1.5, 0.0,
+                       0, 0, self_terms, 0, 1, 0, 0, 1, 1, 0)
+    ref = ctypes.byref(p)
+    size = L.fs_small_products_bytes(ref)
+    assert size > 0
+    results = []
+    for kept in (0, size):
+        ws = torch.empty(L.fs_small_workspace_bytes(ref), dtype=torch.uint8, device="cuda")
+        # (what the memory held before shows in what is read past the end of a row)
+        products = torch.full((max(kept, 4) // 4,), float("nan"), device="cuda")
+        words = torch.empty(4 * items, dtype=torch.int32, pin_memory=True)
+        rows = {0: n, 2: m, 4: n, 6: m}
+        pots = {k: torch.zeros(items, r, device="cuda") for k, r in rows.items()
+                if (self_terms < 2 if k < 4 else self_terms)}
+        where = (ctypes.c_void_p * 8)(*[pots[k].data_ptr() if k in pots else None for k in range(8)])
+        stream = torch.cuda.current_stream().cuda_stream
+        assert L.fs_small_solve_products(ref, ws.data_ptr(), ws.numel(), products.data_ptr() if kept else None, kept,
+                                         words.data_ptr(), None, None, stream) == 0
+        assert L.fs_small_potentials(ref, ws.data_ptr(), ws.numel(), where, stream) == 0
+        results.append(pots)
+    # (a self problem's potentials are small differences of a shifted one and a norm, which is off by 2^-21 of
+    # itself: the bound counts from the largest squared norm)
+    norm = max(float((t * t).sum(-1).max()) for t in (x, y))
+    for k, want in results[0].items():
+        assert (results[1][k] - want).abs().max() <= 2.0 ** -21 * norm + POT * want.abs().max()
+    if size > 4:  # memory too short for them is an error, not a write past its end
+        assert L.fs_small_solve_products(ref, ws.data_ptr(), ws.numel(), products.data_ptr(), size - 1,
+                                         words.data_ptr(), None, None, stream) != 0
+
+
 # ---- both half-updates from one sweep (from 2e7 logits per step on): 256-row groups, chunks of
 # 64-row tiles; eps at which steps go without running maxima, and at which the first ones may not ----
 @pytest.mark.parametrize("n,m,d,eps", [(4481, 4703, 3, 0.5), (4608, 4352, 16, 0.01),
