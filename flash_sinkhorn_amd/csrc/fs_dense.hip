@@ -7,13 +7,28 @@
 namespace fs {
 namespace {
 
+// Tiles of a result in tiles of the kernel.
 template <int WR, int WC, int RB, int CB>
-int launch_gemm(DenseGemmArgs& g, int items, hipStream_t st) {
+int tile_up(DenseGemmArgs& g) {
   // (the transposed copy is read up to the end of its rows, so every column of it is written)
   g.row_tiles = ((g.out_t ? g.ld_t : g.rows) + 32 * WR * RB - 1) / (32 * WR * RB);
   g.col_tiles = g.ld / (32 * WC * CB);
-  const int tiles = g.row_tiles * g.col_tiles;
+  return g.row_tiles * g.col_tiles;
+}
+
+template <int WR, int WC, int RB, int CB>
+int launch_gemm(DenseGemmArgs& g, int items, hipStream_t st) {
+  const int tiles = tile_up<WR, WC, RB, CB>(g);
   hipLaunchKernelGGL((dense_gemm_kernel<WR, WC, RB, CB>), dim3((tiles + 7) / 8 * 8, items, g.splits), dim3(64 * WR * WC), 0, st, g);
+  return hipGetLastError() == hipSuccess ? FS_OK : FS_ERR_LAUNCH_FAILED;
+}
+
+template <int WR, int WC, int RB, int CB>
+int launch_jobs(DenseGemmJobs& g, int jobs, int items, hipStream_t st) {
+  int tiles = 0;
+  for (int i = 0; i < jobs; ++i) tiles = std::max(tiles, tile_up<WR, WC, RB, CB>(g.job[i]));
+  hipLaunchKernelGGL((dense_gemm_jobs_kernel<WR, WC, RB, CB>), dim3((tiles + 7) / 8 * 8, items, jobs), dim3(64 * WR * WC), 0,
+                     st, g);
   return hipGetLastError() == hipSuccess ? FS_OK : FS_ERR_LAUNCH_FAILED;
 }
 
@@ -61,6 +76,17 @@ int dense_gemm(DenseGemmArgs& g, int items, hipStream_t st) {
   if (side == 256) return launch_gemm<2, 4, 4, 2>(g, items, st);
   if (side == 128) return launch_gemm<2, 2, 2, 2>(g, items, st);
   return launch_gemm<2, 2, 1, 1>(g, items, st);
+}
+
+// (rows of every result padded to 256 columns, so that each takes any of the tiles)
+int dense_gemm_jobs(DenseGemmJobs& g, int jobs, int items, hipStream_t st) {
+  int most = 0;
+  for (int i = 1; i < jobs; ++i)
+    if ((double)g.job[i].rows * g.job[i].ld > (double)g.job[most].rows * g.job[most].ld) most = i;
+  const int side = best_side(g.job[most], 1, items * jobs);
+  if (side == 256) return launch_jobs<2, 4, 4, 2>(g, jobs, items, st);
+  if (side == 128) return launch_jobs<2, 2, 2, 2>(g, jobs, items, st);
+  return launch_jobs<2, 2, 1, 1>(g, jobs, items, st);
 }
 
 void dense_plan(const SmallArgs& a, DenseArgs& t) {

@@ -189,7 +189,7 @@ struct DenseGemmArgs {
 };
 
 template <int WR, int WC, int RB, int CB>
-__global__ __launch_bounds__(64 * WR * WC, 2) void dense_gemm_kernel(const DenseGemmArgs g) {
+__device__ __forceinline__ void dense_gemm_tile(const DenseGemmArgs& g, int split) {
   constexpr int W = WR * WC, TR = WR * RB, TC = WC * CB, PIECES = 2 * (TR + TC), LOADS = PIECES / W, ST = 4;
   static_assert(PIECES % W == 0, "every wavefront moves the same number of pieces");
   static_assert(2 * RB * 1024 <= 65535 && 2 * CB * 1024 <= 65535, "offsets of the LDS reads");
@@ -201,7 +201,7 @@ __global__ __launch_bounds__(64 * WR * WC, 2) void dense_gemm_kernel(const Dense
   if (((int)blockIdx.x >> 3) >= per_xcd || item >= tiles) return;
   const int band = item / (4 * g.col_tiles), within = item % (4 * g.col_tiles);
   const int nb = min(4, g.row_tiles - 4 * band);
-  const int rt = 4 * band + within % nb, ct = within / nb, z = blockIdx.y, split = blockIdx.z;
+  const int rt = 4 * band + within % nb, ct = within / nb, z = blockIdx.y;
   const int k_begin = split * g.run, steps = min(g.steps - k_begin, g.run);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int li = lane & 31, h = lane >> 5, wr = wave / WC, wc = wave % WC;
@@ -290,6 +290,20 @@ __global__ __launch_bounds__(64 * WR * WC, 2) void dense_gemm_kernel(const Dense
               make_float4(acc[i][j][4 * q] * inv, acc[i][j][4 * q + 1] * inv, acc[i][j][4 * q + 2] * inv,
                           acc[i][j][4 * q + 3] * inv);
   }
+}
+
+template <int WR, int WC, int RB, int CB>
+__global__ __launch_bounds__(64 * WR * WC, 2) void dense_gemm_kernel(const DenseGemmArgs g) {
+  dense_gemm_tile<WR, WC, RB, CB>(g, blockIdx.z);
+}
+
+// Up to four products of the same depth in one launch.
+struct DenseGemmJobs {
+  DenseGemmArgs job[4];
+};
+template <int WR, int WC, int RB, int CB>
+__global__ __launch_bounds__(64 * WR * WC, 2) void dense_gemm_jobs_kernel(const DenseGemmJobs g) {
+  dense_gemm_tile<WR, WC, RB, CB>(g.job[blockIdx.z], 0);
 }
 
 __device__ __forceinline__ void dense_join(float& m, float& s, float m2, float s2) {
@@ -555,6 +569,7 @@ __global__ __launch_bounds__(512) void dense_rows_kernel(const DenseRowArgs a) {
 void dense_plan(const SmallArgs& a, DenseArgs& t);
 void dense_gemm_plan(DenseGemmArgs& g, bool may_split);
 int dense_gemm(DenseGemmArgs& g, int items, hipStream_t st);
+int dense_gemm_jobs(DenseGemmJobs& g, int jobs, int items, hipStream_t st);
 int dense_prepare(const SmallArgs& a, const DenseArgs& t, hipStream_t st);
 int dense_step(const SmallArgs& a, DenseArgs& t, int step, hipStream_t st);
 int dense_rows_step(const DenseRowArgs& t, int rows, int sides, int items, hipStream_t st);

@@ -91,12 +91,17 @@ Products products_at(const SmallArgs& a, void* at) {
   return t;
 }
 
-// Forms them, from the planes of small_prep_kernel.
+// Forms them, from the planes of small_prep_kernel.  Both sides of a problem get a product of their own: a
+// transposed copy would add a logit's cross products in the other order (those of its key first), and a cloud solved
+// against itself would have f and g that differ by a rounding.
 int form_products(const SmallArgs& a, const Products& t, int steps, hipStream_t st) {
-  for (int prob = a.self == 2 ? 1 : 0; prob < (a.self ? 3 : 1); ++prob) {
-    const int r = prob == 2 ? 1 : 0, c = prob == 0 ? 1 : r;
-    DenseGemmArgs g;
-    std::memset(&g, 0, sizeof(g));
+  DenseGemmJobs jobs;
+  std::memset(&jobs, 0, sizeof(jobs));
+  int n = 0;
+  for (int side = 0; side < 4; ++side) {
+    if (t.dots[side] == nullptr) continue;
+    const int r = side & 1, c = side < 2 ? r ^ 1 : r;
+    DenseGemmArgs& g = jobs.job[n++];
     g.a = a.planes[r];
     g.b = a.planes[c];
     g.a_blocks = a.blocks[r];
@@ -108,14 +113,11 @@ int form_products(const SmallArgs& a, const Products& t, int steps, hipStream_t 
     g.cols = a.rows[c];
     g.scale[0] = a.scale + r;
     g.scale[1] = a.scale + c;
-    g.out = t.dots[prob == 0 ? 0 : prob + 1];
-    g.ld = t.ld[prob == 0 ? 0 : prob + 1];
-    if (prob == 0) g.out_t = t.dots[1], g.ld_t = t.ld[1];
+    g.out = t.dots[side];
+    g.ld = t.ld[side];
     dense_gemm_plan(g, false);
-    const int rc = dense_gemm(g, a.items, st);
-    if (rc != FS_OK) return rc;
   }
-  return FS_OK;
+  return dense_gemm_jobs(jobs, n, a.items, st);
 }
 
 // Workgroups over which the loss of an item is spread: one for what a workgroup does in three rounds.
