@@ -122,6 +122,18 @@ SidePlan plan_side(int mode, int64_t nq, int64_t nk, const Family& fam, int rb_f
   return p;
 }
 
+// What carried margins depend on: the pairing of matrices, the scale of the dot products and the coefficients
+// of the bias terms.  Never 0, the cleared state.
+unsigned tag_of(const Side& sd, const SidePlan& p) {
+  auto bits = [](float v) { unsigned u; std::memcpy(&u, &v, 4); return u; };
+  unsigned t = 0x9e3779b9u * (unsigned)(1 + sd.ps_q + 2 * sd.ps_k);
+  for (unsigned w : {bits(sd.qscale), bits(sd.kc0), bits(sd.kc1), bits(sd.kc2),
+                     (unsigned)(sd.kb1 != nullptr) + 2u * (unsigned)(sd.kb2 != nullptr),
+                     (unsigned)sd.nq, (unsigned)sd.nk, (unsigned)p.chunk})
+    t = (t ^ w) * 0x85ebca6bu + 0xc2b2ae35u;
+  return t | 1u;
+}
+
 // Per-tile records of the key bias for lse_coarse_kernel (see coarse_bias_kernel).
 size_t coarse_aux_bytes(int64_t nk) {
   return (size_t)(ceil_div(nk, 64) + kAuxPadTiles) * kAuxWords * sizeof(unsigned);
@@ -227,14 +239,26 @@ size_t tiled_bytes(int64_t rows, const LseConfig& c) {
   return (size_t)ceil_div(rows + kPlanePadRowsApi, 32) * 32 * (size_t)c.dp * 4;
 }
 
+// Two more of these arrays for rows of 65 .. 128 columns: the 2-norms of their planes (Side::qnorms).
+bool plane_norms(const LseConfig& c) { return !c.gemm && c.prec == 3 && c.dp == 128; }
+
 size_t plane_bytes(int64_t rows, const LseConfig& c) {
-  return planes_only_bytes(rows, c) + 4 * row_array_bytes(rows) + tiled_bytes(rows, c);
+  return planes_only_bytes(rows, c) + (plane_norms(c) ? 6 : 4) * row_array_bytes(rows) + tiled_bytes(rows, c);
 }
 
 // Carried margins of lse_coarse_kernel: per wavefront (64 rows) and 32-key sub-tile two entries.
 // A slot serves any pairing of the set's matrices as (stationary, streamed).
+// (rows of 65 .. 128 columns: one fp16 number per 32 x 32 unit)
+int slack_stride_for(int64_t max_rows) { return ceil_div(max_rows, 128) * 4; }
+size_t slack_bytes(int64_t max_rows) {
+  return ((size_t)ceil_div(max_rows, 32) * (size_t)slack_stride_for(max_rows) * 2 + 15) & ~(size_t)15;
+}
 int margin_stride_for(int64_t max_rows) { return (ceil_div(max_rows, 128) + 1) * 4; }
 size_t margin_slot_bytes(int64_t max_rows, const LseConfig& c) {
+  if (plane_norms(c)) {  // Side::slack, marks, slack_bias, slack_floor and slack_rest
+    const size_t b = 3 * slack_bytes(max_rows) + 2 * row_array_bytes(max_rows) + 2 * row_array_bytes(ceil_div(max_rows, 32) + 4);
+    return b <= ((size_t)512 << 20) ? b : 0;
+  }
   if (c.gemm || c.prec != 3 || c.dp > 64) return 0;
   // wavefront rows in whole workgroups of four: the last workgroup's spare wavefronts keep entries too
   const size_t b = (size_t)ceil_div(max_rows, 256) * 4 * (size_t)margin_stride_for(max_rows) * 8;
@@ -260,6 +284,7 @@ size_t npieces_bytes(int64_t max_rows) { return ((size_t)ceil_div(max_rows, 256)
 // counts for either side.
 size_t margin_region_bytes(int64_t max_rows, const LseConfig& c) {
   const size_t slot = margin_slot_bytes(max_rows, c);
+  if (plane_norms(c)) return 2 * slot;
   return slot > 0 ? 2 * slot + kQueueBytes + 2 * npieces_bytes(max_rows) : 0;
 }
 
@@ -331,7 +356,7 @@ int* best_keys_of(const PlaneSet& ps, const LseConfig& c, void* ws, const float*
 }
 
 float* row_array_of(const PlaneSet& ps, const LseConfig& c, void* ws, const float* src, int rows,
-                    int which) {  // 1: last maxima, 2: last biases, 3: this launch's starting values
+                    int which) {  // 1: last maxima, 2: last biases, 3: this launch's starting values, 4: norms
   int* keys = best_keys_of(ps, c, ws, src, rows);
   if (keys == nullptr) return nullptr;
   return reinterpret_cast<float*>(reinterpret_cast<char*>(keys) + which * row_array_bytes(rows));
@@ -959,8 +984,11 @@ int run_stream(int mode, bool sepv, Side* sides, int nsides, int64_t d, void* ws
   // choice lives in state that belongs to prepared planes (a call that writes its own planes
   // would start it afresh), so without them FS_FLAG_COARSE_AUTO means the plain kernel.
   // (rows of 65 .. 128 columns: lse_coarse128_kernel, without carried margins)
-  const bool can_coarse = lse2 && mode == kLse && prec == 3 && dp2 <= 128 && !(flags & FS_FLAG_NO_TILE_SKIP);
   const bool wide = dp2 == 128;
+  int64_t most_rows = 0;
+  for (int s = 0; s < nsides; ++s) most_rows = std::max<int64_t>(most_rows, std::max(sides[s].nq, sides[s].nk));
+  const bool can_coarse = lse2 && mode == kLse && prec == 3 && dp2 <= 128 && !(flags & FS_FLAG_NO_TILE_SKIP) &&
+                          (!wide || margin_slot_bytes(most_rows, cfg) > 0);
   const bool coarse = (flags & FS_FLAG_COARSE_TEST) && can_coarse;
   const bool auto_sel = (flags & FS_FLAG_COARSE_AUTO) && can_coarse && !coarse && prepared;
   Family fam_plan = fam;
@@ -1058,6 +1086,12 @@ int run_stream(int mode, bool sepv, Side* sides, int nsides, int64_t d, void* ws
     sd.margins = nullptr;
     sd.npieces = nullptr;
     sd.seed = nullptr;
+    sd.qnorms = sd.knorms = nullptr;
+    sd.slack = nullptr;
+    sd.marks = nullptr;
+    sd.slack_bias = sd.slack_floor = nullptr;
+    sd.slack_rest = nullptr;
+    sd.slack_stride = 0;
     sd.sparse_group = 1;
     sd.ktiled = sd.qtiled = nullptr;
     sd.m_prev = nullptr;
@@ -1086,6 +1120,21 @@ int run_stream(int mode, bool sepv, Side* sides, int nsides, int64_t d, void* ws
         sd.best_key = best_keys_of(ps, cfg, ws, sd.q, sd.nq);
         sd.seed = row_array_of(ps, cfg, ws, sd.q, sd.nq, 3);
         sd.key_aux = reinterpret_cast<unsigned*>(static_cast<char*>(ws) + aux_off + (s == 1 ? aux_bytes[0] : 0));
+        if (wide) {
+          // (a slot per matrix that holds query rows; both sides of one matrix: no slack outlives the launch)
+          const bool shared = nsides == 2 && plane_index(ps, sides[0].q, sides[0].nq) == plane_index(ps, sides[1].q, sides[1].nq);
+          const int rows = std::max(ps.rows[0], ps.n > 1 ? ps.rows[1] : 0);
+          char* slot = static_cast<char*>(ws) + ps.margin_off + (size_t)(shared ? s : sd.ps_q) * ps.margin_slot;
+          sd.slack = reinterpret_cast<unsigned short*>(slot);
+          sd.marks = reinterpret_cast<unsigned*>(slot + slack_bytes(rows));
+          sd.slack_bias = reinterpret_cast<float*>(slot + 3 * slack_bytes(rows));
+          sd.slack_floor = reinterpret_cast<float*>(slot + 3 * slack_bytes(rows) + row_array_bytes(rows));
+          sd.slack_rest = reinterpret_cast<int*>(slot + 3 * slack_bytes(rows) + 2 * row_array_bytes(rows));
+          sd.slack_stride = slack_stride_for(rows);
+          a.tag[s] = shared ? 0u : tag_of(sd, p);
+        }
+        sd.qnorms = wide ? row_array_of(ps, cfg, ws, sd.q, sd.nq, 4) : nullptr;
+        sd.knorms = wide ? row_array_of(ps, cfg, ws, sd.k, sd.nk, 4) : nullptr;
       }
       if (margins) {
         // (slot and state words go with the matrix that holds the query rows)
@@ -1098,15 +1147,7 @@ int run_stream(int mode, bool sepv, Side* sides, int nsides, int64_t d, void* ws
                      (size_t)s * npieces_bytes(std::max(ps.rows[0], ps.n > 1 ? ps.rows[1] : 0));
         sd.m_prev = row_array_of(ps, cfg, ws, sd.q, sd.nq, 1);
         sd.bias_prev = row_array_of(ps, cfg, ws, sd.k, sd.nk, 2);
-        // what the margins depend on: the pairing of matrices, the scale of the dot products
-        // and the coefficients of the bias terms
-        auto bits = [](float v) { unsigned u; std::memcpy(&u, &v, 4); return u; };
-        unsigned t = 0x9e3779b9u * (unsigned)(1 + sd.ps_q + 2 * sd.ps_k);
-        for (unsigned w : {bits(sd.qscale), bits(sd.kc0), bits(sd.kc1), bits(sd.kc2),
-                           (unsigned)(sd.kb1 != nullptr) + 2u * (unsigned)(sd.kb2 != nullptr),
-                           (unsigned)sd.nq, (unsigned)sd.nk, (unsigned)p.chunk})
-          t = (t ^ w) * 0x85ebca6bu + 0xc2b2ae35u;
-        a.tag[s] = t | 1u;  // never 0, the cleared state
+        a.tag[s] = tag_of(sd, p);
       }
     }
     a.side[s] = sd;

@@ -127,6 +127,18 @@ struct Side {
   float* m_prev;
   float* bias_prev;
   float* seed;          // per query row: where this launch's running maximum starts (raw units)
+  // rows of 65 .. 128 columns: 2-norm of every row's hi plane, and, from [(rows + 3) & ~3] on, of its lo plane
+  const float* qnorms;
+  const float* knorms;
+  // ... and, per 32 rows a line of slack_stride units of 32 keys, which keys are taken (a bit each) and by how much the
+  // others are left out (fp16 in base-2 units, rounded down; not above zero: they are taken too), with the keys'
+  // biases and the rows' lines that they were left out by, in raw units (lse_test128_kernel)
+  unsigned* marks;
+  unsigned short* slack;
+  float* slack_bias;
+  float* slack_floor;
+  int* slack_rest;     // what lse_listed128_kernel leaves to a second launch of it
+  int slack_stride;
   // lse_sparse_kernel: per (64-row group, key range) how many of the range's partial results it
   // wrote (the merge kernel reads only those); index row group * ranges + range
   unsigned char* npieces;
@@ -190,6 +202,9 @@ __host__ __device__ inline int self_groups_of_chunk(int s, int chunk, int n, int
 // 64 on, kQueueSlots 64-bit slots for the remainders (0: empty, all ones: taken).
 constexpr int kQueueBase = 0, kQueueTail = 16, kQueueHead = 32, kQueueSlot0 = 64, kQueueSlots = 224;
 constexpr int kQueueWords = kQueueSlot0 + 2 * kQueueSlots;
+constexpr int kCoarse128Rows = 384;  // query rows of a workgroup of lse_coarse128_kernel
+constexpr int kCoarse128Grid = 512;  // two of its workgroups per CU
+constexpr int kCoarse128Lds = 4 * 64 * 64 + 4 * 64, kTest128Lds = 2 * (64 * 64 + 4 * 128);  // LDS in words
 constexpr size_t kQueueBytes = (size_t)2 * 8 * kQueueWords * 4;
 constexpr int kSparseBlocks = 512;
 
@@ -197,6 +212,9 @@ constexpr int kSparseBlocks = 512;
 // b_j - 2^18 a_j per key, then the largest bias of each 32-key sub-tile in the first two of 64
 // words: three parts that one wavefront moves with one full instruction each (16, 4 and 4
 // bytes per lane).
+// For rows of 65 .. 128 columns, words 2 and 3 of that part: the tile's largest 2-norm of a hi plane, and of
+// a lo plane with 2^-19 of the former on top; words 4 and 5: by how much the biases of each sub-tile have risen
+// since Side::slack was written, at most, 8 and 9 by which of its keys, 6 and 7 by how much all others have.
 constexpr int kAuxA = 0, kAuxB = 256, kAuxMax = 320, kAuxWords = 384, kAuxPadTiles = 8;
 
 // Device state of the variant choice (unsigned words), zeroed when the operand planes are
@@ -223,7 +241,12 @@ constexpr int kDmaxSlots = 16;
 constexpr int kSelDmax = kSelForm + 2;
 // likewise per role: margin entries of the current generation exist (lse_coarse_kernel left them
 // behind, or lse_sparse_kernel ran); without them the sparse form would visit every unit
+constexpr unsigned kListsFrom = 26214u, kListsMost = 6554u, kListsGrow = 1311u, kListsWait = 16u;  // (40, 10 and 2 %)
 constexpr int kSelHave = kSelDmax + 2 * kDmaxSlots;
+// Rows of 65 .. 128 columns use five of these words per role their own way: kSelMode (launches go by lists), kSelHave
+// and kSelTag (Side::slack is that of a launch under this tag), kSelBump (the launch under way had rows without a
+// start), kSelGen (the share of keys taken when they were all tested, in 65536ths), kSelCum (launches until lists are
+// tried again) and the kSelDmax slots (keys taken in the launch under way, by 32).
 // the share of units the plain kernel left out in the first launch of its current stretch, in
 // 65536ths plus one (0: not taken yet)
 constexpr int kSelBase = kSelHave + 2;
@@ -396,6 +419,64 @@ __device__ __forceinline__ void state_after_launch(unsigned* st, int lane, int c
         st[kSelBump + role[i]] = 0u;
       }
   }
+}
+
+// Rows of 65 .. 128 columns: does a side's launch go by lists (lse_coarse128_kernel, lse_listed128_kernel)?
+__device__ __forceinline__ bool coarse128_lists(const unsigned* st, int role) { return st != nullptr && st[kSelMode + role] != 0u; }
+// ... and are all units of it tested (or is the slack of an earlier launch good)?
+__device__ __forceinline__ bool slack_renewed(const unsigned* st, unsigned tag, int role) {
+  return st == nullptr || tag == 0u || st[kSelHave + role] == 0u || st[kSelTag + role] != tag;
+}
+// One wavefront, in front of state_after_launch.  At 20,000 x 30,000 a launch in place takes 210 us and 0.5 for every
+// thousand units of 586 that go on; one by lists 25 us and 1.4 for every thousand times 32 keys of a row block's
+// list, and 150 to 200 more with the test.  Lists are tried where 40 % of the units go on at most, all rows
+// having a start, and kept while they hold 10 % of the keys (else not for sixteen launches); a test is good
+// until the lists have grown by a further 2 % of the keys.  (1 % 3.97 ms, 2 % 4.0 for ten iterations there, at
+// eps 0.05 4.44 and 4.35.)
+__device__ __forceinline__ void slack_after_launch(unsigned* st, int lane, const unsigned (&tag)[2], int sides, const int (&role)[2]) {
+  const unsigned e = st[kSelEnded + lane], u = st[kSelUnits + lane], word = st[kSelWord];
+  unsigned taken = lane < 2 * kDmaxSlots ? st[kSelDmax + lane] : 0u;
+  unsigned have[2] = {0u, 0u}, known[2] = {0u, 0u}, bump[2] = {0u, 0u}, base[2] = {0u, 0u}, lists[2] = {0u, 0u}, wait[2] = {0u, 0u};
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+    if (i < sides) {
+      lists[i] = st[kSelMode + role[i]];
+      have[i] = st[kSelHave + role[i]];
+      known[i] = st[kSelTag + role[i]];
+      bump[i] = st[kSelBump + role[i]];
+      base[i] = st[kSelGen + role[i]];
+      wait[i] = st[kSelCum + role[i]];
+    }
+  unsigned long long es = e, us = u;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) es += __shfl_xor(es, o, 64), us += __shfl_xor(us, o, 64);
+#pragma unroll
+  for (int o = kDmaxSlots / 2; o > 0; o >>= 1) taken += (unsigned)__shfl_xor((int)taken, o, 64);
+  const unsigned of_role[2] = {(unsigned)__shfl((int)taken, 0, 64), (unsigned)__shfl((int)taken, kDmaxSlots, 64)};
+  if (word != 0u || us == 0) return;  // (word: the plain kernel ran)
+  if (lane < 2 * kDmaxSlots) st[kSelDmax + lane] = 0u;
+  if (lane != 0) return;
+  const unsigned share = (unsigned)(((us - min(es, us)) << 16) / us);
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+    if (i < sides) {
+      const int r = role[i];
+      const bool renewed = tag[i] == 0u || have[i] == 0u || known[i] != tag[i];
+      const unsigned keys = (unsigned)(((unsigned long long)of_role[r] << 16) * sides / us);
+      if (lists[i] == 0u) {
+        st[kSelMode + r] = wait[i] == 0u && bump[i] == 0u && share < kListsFrom ? 1u : 0u;
+        st[kSelCum + r] = wait[i] - (wait[i] != 0u ? 1u : 0u);
+        st[kSelHave + r] = 0u;
+      } else if (renewed) {
+        st[kSelHave + r] = tag[i] != 0u && bump[i] == 0u ? 1u : 0u;
+        st[kSelTag + r] = tag[i];
+        st[kSelGen + r] = keys;
+        if (keys > kListsMost) st[kSelMode + r] = 0u, st[kSelCum + r] = kListsWait;
+      } else if (keys > base[i] + kListsGrow) {
+        st[kSelHave + r] = 0u;
+      }
+      st[kSelBump + r] = 0u;
+    }
 }
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }

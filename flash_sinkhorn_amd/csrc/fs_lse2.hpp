@@ -95,7 +95,8 @@ __global__ __launch_bounds__(256) void absmax_kernel(const float* __restrict__ a
 // absmax_kernel; block 0 also publishes it in *scale_out for the consuming kernel and clears
 // the kSelWords words at `clear_state` (the variant-choice state that belongs to the planes);
 // `best_keys` (may be null) starts three arrays of one value per row, (rows + 3) & ~3 values apart:
-// the keys (reset to -1), the rows' last maxima (3e38) and the rows' last biases as keys (0).
+// the keys (reset to -1), the rows' last maxima (3e38) and the rows' last biases as keys (0); two more
+// behind a fourth hold the norms of the planes of 128-column rows (Side::qnorms).
 // With `chunked` the two planes are interleaved per 32 columns (layout of lse_gemm_kernel).
 // `tiled` (may be null; not with `chunked`): a second copy in MFMA operand order, see Side::ktiled.
 __global__ __launch_bounds__(256) void fill_zero_kernel(unsigned* __restrict__ p, long long n) {
@@ -157,6 +158,18 @@ __global__ __launch_bounds__(256) void split_planes_f16_kernel(const SplitArgs a
   const unsigned l01 = pack_f16(v[0] - (float)a[0], v[1] - (float)a[1]);
   const unsigned l23 = pack_f16(v[2] - (float)b[0], v[3] - (float)b[1]);
   unsigned* o = dst + (size_t)r * (size_t)dp;  // two planes of dp/2 words
+  if (best_keys != nullptr && dp == 128 && !chunked) {  // (half a wavefront holds a row: its planes' 2-norms)
+    const f16x2 c = __builtin_bit_cast(f16x2, l01), e = __builtin_bit_cast(f16x2, l23);
+    float nh = (float)a[0] * (float)a[0] + (float)a[1] * (float)a[1] + (float)b[0] * (float)b[0] + (float)b[1] * (float)b[1];
+    float nl = (float)c[0] * (float)c[0] + (float)c[1] * (float)c[1] + (float)e[0] * (float)e[0] + (float)e[1] * (float)e[1];
+#pragma unroll
+    for (int k = 16; k > 0; k >>= 1) nh += __shfl_xor(nh, k, 64), nl += __shfl_xor(nl, k, 64);
+    if ((idx & 31) == 0 && r < rows) {
+      float* norms = reinterpret_cast<float*>(best_keys) + 4 * ((rows + 3) & ~3);
+      norms[r] = sqrtf(nh);
+      norms[((rows + 3) & ~3) + r] = sqrtf(nl);
+    }
+  }
   if (chunked) {
     // per 32 columns: 16 words of the hi plane, then 16 words of the lo plane (dp % 32 == 0)
     unsigned* oc = o + (c4 / 32) * 32 + (c4 % 32) / 2;

@@ -58,8 +58,8 @@ namespace fs {
 
 // What lse_coarse_kernel needs of the key bias, once per launch instead of once per workgroup:
 // one wavefront per 64-key tile writes the tile's record (layout: kAux* in fs_common.hpp) in raw
-// units: a_j as eight fp16 copies, b_j - 2^18 a_j, and the largest bias of each 32-key
-// sub-tile.  Keys past the end of the key set get a bias that masks them.  T only makes this a
+// units: a_j as eight fp16 copies, b_j - 2^18 a_j (for rows of more than 64 columns b_j itself,
+// which is all that lse_coarse128_kernel reads), and the largest bias of each 32-key sub-tile.  Keys past the end of the key set get a bias that masks them.  T only makes this a
 // template (header-defined kernel).
 //
 // The wavefronts behind the tiles (kSeedRows query rows each, side 0 first: seed_blocks0 of them) compute
@@ -190,11 +190,48 @@ __global__ __launch_bounds__(64 * kBiasWaves) void coarse_bias_kernel(const Laun
     ah = __builtin_bit_cast(_Float16, (unsigned short)(__builtin_bit_cast(unsigned short, ah) - 1));
   const unsigned aw = (unsigned)__builtin_bit_cast(unsigned short, ah) * 0x00010001u;
   unsigned* rec = sd.key_aux + (size_t)tile * kAuxWords;
+  float most_hi = 0.f, most_lo = 0.f;
+  if (sd.knorms != nullptr) {
+    if (j < sd.nk) most_hi = sd.knorms[j], most_lo = sd.knorms[((sd.nk + 3) & ~3) + j];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      most_hi = fmaxf(most_hi, __shfl_xor(most_hi, o, 64));
+      most_lo = fmaxf(most_lo, __shfl_xor(most_lo, o, 64));
+    }
+    most_hi *= 1.0001f;
+    most_lo = 1.0001f * most_lo + 0x1p-19f * most_hi;
+  }
+  if (sd.slack != nullptr && in && tile == 0 && lane == 0) sd.slack_rest[0] = 0;
+  // by how much a sub-tile's biases have risen since its units were tested, the largest and (of a single key that has
+  // risen by far) the second largest
+  float rise = 0.f, rise2 = 0.f;
+  int top = 0;
+  if (sd.slack != nullptr && in && j < sd.nk) {
+    if (slack_renewed(args.sel, args.tag[second ? 1 : 0], sd.ps_q)) sd.slack_bias[j] = b;
+    else rise = b - sd.slack_bias[j];
+  }
+  if (sd.slack != nullptr) {
+    if (j >= sd.nk) rise = -3.0e38f;
+    const float own = rise;
+#pragma unroll
+    for (int o = 16; o > 0; o >>= 1) rise = fmaxf(rise, __shfl_xor(rise, o, 64));
+    const unsigned long long tops = __builtin_amdgcn_ballot_w64(!(own < rise));
+    top = __builtin_ctzll((h ? tops >> 32 : tops & 0xffffffffull) | 0x100000000ull) & 31;
+    rise2 = li == top ? -3.0e38f : own;
+#pragma unroll
+    for (int o = 16; o > 0; o >>= 1) rise2 = fmaxf(rise2, __shfl_xor(rise2, o, 64));
+    rise = __shfl(rise, (lane & 1) * 32, 64);
+    rise2 = __shfl(rise2, (lane & 1) * 32, 64);
+    top = __shfl(top, (lane & 1) * 32, 64);
+  }
   const float mx_sub = __shfl(mx, (lane & 1) * 32, 64);  // lanes 0 and 1: the two sub-tiles' maxima
   if (in) {
     *reinterpret_cast<u32x4*>(rec + kAuxA + lane * 4) = u32x4{aw, aw, aw, aw};
-    rec[kAuxB + lane] = __builtin_bit_cast(unsigned, b - (float)ah * 0x1p18f);
-    rec[kAuxMax + lane] = lane < 2 ? __builtin_bit_cast(unsigned, mx_sub) : 0u;
+    rec[kAuxB + lane] = __builtin_bit_cast(unsigned, dp > 64 ? b : b - (float)ah * 0x1p18f);
+    rec[kAuxMax + lane] = lane < 2 ? __builtin_bit_cast(unsigned, mx_sub)
+                                   : lane < 4 ? __builtin_bit_cast(unsigned, lane == 2 ? most_hi : most_lo)
+                                   : lane < 6 ? __builtin_bit_cast(unsigned, rise)
+                                   : lane < 8 ? __builtin_bit_cast(unsigned, rise2) : lane < 10 ? (unsigned)top : 0u;
   }
 
   // Carried margins: the largest change of a key's bias since the last launch with this side

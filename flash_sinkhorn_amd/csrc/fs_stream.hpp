@@ -489,6 +489,10 @@ __global__ __launch_bounds__(finish_threads(HAS_O)) void finish_kernel(const Lau
           role[i] = ms.ps_q;
           ls[i] = ms.qscale / (ms.plane_scale[ms.ps_q] * ms.plane_scale[ms.ps_k]);
         }
+      if (args.side[0].slack != nullptr) {
+        const int sides = args.side[1].slack != args.side[0].slack ? 2 : 1, r[2] = {args.side[0].ps_q, args.side[1].ps_q};
+        slack_after_launch(args.sel, threadIdx.x, args.tag, sides, r);
+      }
       state_after_launch(args.sel, threadIdx.x, commit_sides, role, ls);
     }
   }

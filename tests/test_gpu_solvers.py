@@ -1085,3 +1085,50 @@ def test_graph_replays_equal_eager_solves(monkeypatch):
     wf, wg, wfp, wgp = oracle.sinkhorn_symmetric(x, y, a, b, use_epsilon_scaling=False, eps=0.05,
                                                  n_iters=12, return_prelast=True)
     assert rel_err(f, wf) < RTOL and rel_err(g, wg) < RTOL and rel_err(fp, wfp) < RTOL
+
+
+@pytest.mark.parametrize("n,m,d", [(33, 700, 65), (33, 6100, 65), (384, 8192, 128), (385, 6401, 100), (2300, 9000, 96),
+                                   (100, 40000, 70)])
+def test_half_updates_by_lists_on_rows_of_65_to_128_columns(n, m, d):
+    """``lse_test128_kernel`` / ``lse_listed128_kernel``: potentials that stay, drift, or change for single keys, for all
+    keys but one and for everything, behind one test of all units; keys without mass; against fp64.  Sizes
+    around the row groups of 32 and 384 rows, the pieces of 128 keys and the 64 pieces a wavefront takes at a time."""
+    from flash_sinkhorn_amd import _lib
+    from flash_sinkhorn_amd.kernels.sinkhorn_flashstyle_sqeuclid import flashsinkhorn_lse_fused
+    gen = torch.Generator(device="cuda").manual_seed(n + d)
+    x = torch.randn(n, d, device="cuda", generator=gen)
+    y = 1.5 * torch.randn(m, d, device="cuda", generator=gen)
+    eps, g = 0.004, -(y * y).sum(1)
+    lw = torch.log(torch.rand(m, device="cuda", generator=gen) + 0.1)
+    prep = _lib.PreparedOperands(x, y, _lib.flags(True, False))
+    xy = 2.0 * x.double() @ y.double().T
+    # the planes hold 22 bits of x.y, whose sum and the bias are rounded to fp32 a few times
+    tol = 2e-6 * float((x * x).sum(1).max() + (y * y).sum(1).max())
+
+    def check():
+        out = flashsinkhorn_lse_fused(x, y, g, lw, eps, allow_tf32=False, _prepared=prep, _coarse=True)
+        want = -eps * torch.logsumexp((xy + g.double()) / eps + lw.double(), 1)
+        assert float((out - want).abs().max()) <= tol
+
+    for _ in range(4):
+        check()
+    assert prep.variant_state()["by_lists"] or m < 1000  # (of few keys most units hold a row's best)
+    best = (xy + g.double()).argmax(1)
+    g += 0.01 * torch.randn(m, device="cuda", generator=gen)
+    check()
+    g[m // 2] += 40.0  # one key rises over most others
+    check()
+    g[best[0]] -= 60.0  # and the keys of some rows fall: their lines do
+    g[best[n // 2]] -= 200.0
+    check()
+    g += 25.0  # all alike: nothing is used up
+    check()
+    g[: m // 3] -= 300.0
+    check()
+    lw[: m // 2] = -100000.0  # no mass
+    check()
+    lw[: m // 2] = 0.0
+    check()
+    g += 30.0 * torch.randn(m, device="cuda", generator=gen)
+    check()
+    check()
