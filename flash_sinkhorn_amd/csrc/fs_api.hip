@@ -94,6 +94,31 @@ Family family_for(int64_t d) {
   return f;
 }
 
+// The key split of plan-vector products and c-transforms: all workgroups do the same work, two at a time on a CU, so
+// a split is priced by full rounds of 512 of them, each as long as a workgroup's 64-key tiles and one and a half
+// more (its prologue), and by the merge, which writes and reads three words a row and range (3.5 us a tile, 4.5
+// TB/s).  Doubling the split until 2,048 workgroups were there left part of the last round empty, and made more of them
+// than pays: P v of 9,000 x 7,000 x 64 57 us, now 49; c-transforms of 12,000 x 12,001 x 100 159 and 152, of 5,000 x
+// 40,000 x 128 230 and 211, of 20,000 x 15,013 x 32 117 and 112, of 25,000 x 30,000 x 100 579 and 578.  Kernels of
+// narrow rows have three and four workgroups a CU, but rounds of 768 or 1,024 predict their times worse: over
+// products of 1,200 to 48,000 rows this rule is 1.2 % above the best of 20 splits, doubling 7.5 %.
+// (Products with a matrix stay with doubling: a range is summed in one fp32 accumulator, and where ranges got longer
+// by this rule results were 6 % further from fp64; with shorter ones only, gradients of peaked plans 2 % slower.)
+SidePlan plan_rounds(SidePlan p, int64_t nq, int64_t nk, int cap) {
+  double best = 0.0;
+  const int most = (int)std::max<int64_t>(1, std::min<int64_t>(cap, nk / 128));
+  for (int s = 1; s <= most; ++s) {
+    const int tiles = ceil_div(ceil_div(nk, s), 64), splits = ceil_div(nk, (int64_t)tiles * 64);
+    const double cost = (double)ceil_div((int64_t)p.igroups * splits, 512) * (tiles + 1.5) + 0.06 * tiles +
+                        (splits > 1 ? 1.5e-6 * (double)nq * splits : 0.0);
+    if (s > 1 && cost >= best) continue;
+    best = cost;
+    p.chunk = tiles * 64;
+    p.splits = splits;
+  }
+  return p;
+}
+
 // Rows per wavefront (RB blocks of 32) and the key split for one side.
 SidePlan plan_side(int mode, int64_t nq, int64_t nk, const Family& fam, int rb_force = 0,
                    int min_splits = 1) {
@@ -112,8 +137,9 @@ SidePlan plan_side(int mode, int64_t nq, int64_t nk, const Family& fam, int rb_f
     if (rb_force > 0) p.rb = rb_force;
     p.igroups = ceil_div(nq, 128 * p.rb);
   }
-  const int max_splits = (int)std::max<int64_t>(1, nk / (4 * jt));
   const int cap = has_o ? 16 : 64;
+  if ((mode == kVec || mode == kArgmax) && !fam.sliced) return plan_rounds(p, nq, nk, cap);
+  const int max_splits = (int)std::max<int64_t>(1, nk / (4 * jt));
   int s = 1;
   while (p.igroups * s < target && s * 2 <= max_splits && s * 2 <= cap) s *= 2;
   s = std::max(s, min_splits);

@@ -264,8 +264,8 @@ __global__ __launch_bounds__(256, 2) void lse2_kernel(const LaunchArgs args) {
   if (sd.margins != nullptr && bid == 0 && threadIdx.x == 0) args.sel[kSelForm + sd.ps_q] = 0u;
   const int d = args.d;
 
-  const int split = bid % sd.splits;
-  const int ig = bid / sd.splits;
+  int split = bid % sd.splits, ig = bid / sd.splits;
+  if constexpr (VEC) product_item(bid, sd, split, ig);
   const int tid = threadIdx.x;
   const int wave = tid >> 6;
   const int lane = tid & 63;

@@ -67,8 +67,8 @@ __global__ __launch_bounds__(256, (MODE == kMat5 && DP == 128) ? 1 : 2) void pla
   const int d = args.d;
   const bool vec_ok = args.vec_ok != 0;
 
-  const int split = bid % sd.splits;
-  const int ig = bid / sd.splits;
+  int split = bid % sd.splits, ig = bid / sd.splits;
+  if constexpr (MODE == kVec || MODE == kArgmax) product_item(bid, sd, split, ig);
   const int tid = threadIdx.x;
   const int wave = tid >> 6;
   const int lane = tid & 63;

@@ -27,6 +27,18 @@
 
 namespace fs {
 
+// Which key range and row group a workgroup of a plan-vector product or a c-transform takes.  Workgroups are dealt
+// to the eight XCDs in turn, and each XCD has an L2 of its own: an XCD takes one run of the ranges, all row groups of
+// a range before the next, so that the 64 workgroups it holds read the same key tiles whatever the number of ranges.
+// (Dealt range by range every L2 sees all keys unless that number is a multiple of eight: the c-transform of 25,000 x
+// 30,000 x 100 in 13 ranges 594 us, this way 564.)
+__device__ __forceinline__ void product_item(int bid, const Side& sd, int& split, int& ig) {
+  const int total = sd.splits * sd.igroups, x = bid & 7;
+  const int at = x * (total >> 3) + min(x, total & 7) + (bid >> 3);
+  split = at / sd.igroups;
+  ig = at - split * sd.igroups;
+}
+
 template <int DP>
 struct Geo {
   static constexpr int JT = (DP >= 128) ? 32 : 64;  // key rows per LDS tile

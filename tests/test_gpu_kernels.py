@@ -317,6 +317,37 @@ def test_products_with_two_row_blocks_per_wave(n, m, d):
     assert np.abs(c.cpu().numpy()[rows] - wc).max() <= 1e-5 * max(np.abs(wc).max(), 1.0)
 
 
+@pytest.mark.parametrize("n,m,d", [
+    (513, 127, 40), (513, 128, 40),      # one range of keys, where the merge is left out
+    (3900, 255, 128), (3900, 257, 70),   # two ranges, the second of nearly all, and of one key
+    (2049, 4225, 64),                    # a last range of a single tile
+    (130, 8193, 16),                     # as many ranges as there may be, a key behind the last tile
+    (16385, 1411, 20)])                  # 65 row groups: five ranges, not a power of two
+def test_products_over_uneven_key_ranges(n, m, d):
+    """Key ranges of any number and length: sampled rows of plan*matrix, plan*vector and the
+    c-transform against the oracle, at the bars of the tests above."""
+    from flash_sinkhorn_amd.kernels.apply_flash import (
+        apply_plan_mat_flashstyle, apply_plan_vec_flashstyle)
+    from flash_sinkhorn_amd import c_transform_fwd
+    x, y, a, b, fh, gh = problem(n, m, d, seed=21)
+    la, lb = np.log(a), np.log(b)
+    rng = np.random.default_rng(22)
+    V = rng.standard_normal((m, d)).astype(np.float32)
+    v, psi = rng.standard_normal((2, m)).astype(np.float32)
+    rows = np.concatenate([rng.choice(n, 100, replace=False), [0, 31, 32, 127, 128, n - 1]])
+    at = torch.from_numpy(rows).cuda()
+    X, Y, F, G, LA, LB = dev(x, y, fh, gh, la, lb)
+    kw = dict(eps=0.4, cost_scale=0.5)
+    args = (x[rows], y, fh[rows], gh, la[rows], lb)
+    got = apply_plan_mat_flashstyle(X, Y, F, G, LA, LB, dev(V)[0], axis=1, **kw)
+    assert rel_err(got[at], oracle.apply_plan_mat(*args, V, axis=1, **kw)) < RTOL
+    got = apply_plan_vec_flashstyle(X, Y, F, G, LA, LB, dev(v)[0], axis=1, **kw)
+    assert rel_err(got[at], oracle.apply_plan_vec(*args, v, axis=1, **kw)) < RTOL
+    c, _ = c_transform_fwd(X, Y, dev(psi)[0], cost_scale=0.5)
+    wc, _ = oracle.c_transform(x[rows], y, psi, 0.5)
+    assert np.abs(c.cpu().numpy()[rows] - wc).max() <= 1e-5 * max(np.abs(wc).max(), 1.0)
+
+
 @pytest.mark.parametrize("n,m,d,eps", [(40000, 200000, 4, 0.5), (30000, 120000, 16, 0.05)])
 def test_long_key_chunks_keep_fp32_accuracy(n, m, d, eps):
     """Hundreds of key tiles per workgroup: whatever is applied once per tile (the rescale of
