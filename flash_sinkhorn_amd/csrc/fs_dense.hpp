@@ -23,8 +23,6 @@ constexpr int kDenseStep = 2 * 64;
 
 struct DenseArgs {
   float* dots;             // [items][n][ld], ld a multiple of 256, zero beyond the m-th column
-  float* dots_t;           // [items][m][ld_t]: the same transposed, where a step is one launch (`rows`)
-  int ld_t, rows;          // rows: rows of a wavefront in dense_rows_kernel, 0: dense_sweep_kernel
   u32x4* planes[2];        // [items][blocks][steps][2][64]
   int blocks[2];           // 32-row blocks, a multiple of 8 (zero rows behind the last one)
   int steps;               // 16-column steps
@@ -42,6 +40,9 @@ struct DenseArgs {
   int step, sched, extrapolate;
   int large;               // the shape of dense_sweep_kernel
   int turns;               // every other step reads the products backwards
+  // (not read by the kernels that take this, and behind what they read)
+  float* dots_t;           // [items][m][ld_t]: the products transposed, where a step is one launch (`rows`)
+  int ld_t, rows;          // rows: rows of a wavefront in dense_rows_kernel, 0: dense_sweep_kernel
 };
 
 // Eight consecutive elements as floats; `wide`: by whole 16-byte words.
