@@ -537,6 +537,15 @@ __device__ __forceinline__ unsigned pack_f16(float a, float b) {
   return __builtin_bit_cast(unsigned, __builtin_convertvector(v, f16x2));
 }
 
+// What fp16 leaves of x, as x - (float)h in one instruction (v_fma_mix_f32, the same bits) in place of a conversion and a
+// subtraction; `one` is 1.0f that the compiler cannot see (opaque_one), else it makes a subtraction of it again.
+__device__ __forceinline__ float opaque_one() {
+  float one = 1.0f;
+  asm("" : "+s"(one));
+  return one;
+}
+__device__ __forceinline__ float f16_rest(float x, _Float16 h, float one) { return __builtin_fmaf(-(float)h, one, x); }
+
 // f(integral_constant<int, 0>{}), ..., f(integral_constant<int, N - 1>{}) in order
 template <int... I, class F>
 __device__ __forceinline__ void static_for_impl(std::integer_sequence<int, I...>, F&& f) {

@@ -260,6 +260,11 @@ __global__ __launch_bounds__(256, (MODE == kMat5 && DP == 128) ? 1 : 2) void pla
     asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(a), "+v"(b));
   };
 
+  // Up to 32 columns: what fp16 leaves of a probability in one instruction, and no sums of the plan where nobody
+  // divides by them (the gradient does): the map of 20,000 x 15,013 x 32 with its vector products 385 -> 376 us.  (At 64 and 128 columns both cost a matrix product
+  // registers that it does not have: 25,000 x 30,000 x 64 with its vector products 1,295 -> 1,317.)
+  const float one = opaque_one();
+  const bool sums = MODE == kMat && (DP >= 64 || sd.ep.kind == kEpiGrad);
   int buf = 0;
   for (int t = 0; t < ntiles; ++t) {
     const int j0 = j_begin + t * kPtKeys;
@@ -429,13 +434,14 @@ __global__ __launch_bounds__(256, (MODE == kMat5 && DP == 128) ? 1 : 2) void pla
           }
         }
         float p[16];
-        float ps = 0.f;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          p[r] = fast_exp2(__builtin_fmaf(acc[r], lscale, run_c[rb]));
-          ps += p[r];
+        for (int r = 0; r < 16; ++r) p[r] = fast_exp2(__builtin_fmaf(acc[r], lscale, run_c[rb]));
+        if (sums) {
+          float ps = 0.f;
+#pragma unroll
+          for (int r = 0; r < 16; ++r) ps += p[r];
+          run_s[rb] += ps;
         }
-        run_s[rb] += ps;
         if constexpr (MODE == kVec) {
           float po = 0.f;
 #pragma unroll
@@ -456,7 +462,8 @@ __global__ __launch_bounds__(256, (MODE == kMat5 && DP == 128) ? 1 : 2) void pla
               const float x0 = p[8 * s + 2 * e], x1 = p[8 * s + 2 * e + 1];
               hi[e] = pack_f16(x0, x1);
               const f16x2 hh = __builtin_bit_cast(f16x2, hi[e]);
-              lo[e] = pack_f16(x0 - (float)hh[0], x1 - (float)hh[1]);
+              lo[e] = DP >= 64 ? pack_f16(x0 - (float)hh[0], x1 - (float)hh[1])
+                               : pack_f16(f16_rest(x0, hh[0], one), f16_rest(x1, hh[1], one));
             }
             const f16x8 bh = __builtin_bit_cast(f16x8, u32x4{hi[0], hi[1], hi[2], hi[3]});
             const f16x8 bl = __builtin_bit_cast(f16x8, u32x4{lo[0], lo[1], lo[2], lo[3]});

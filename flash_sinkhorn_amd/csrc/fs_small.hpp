@@ -827,6 +827,7 @@ __global__ __launch_bounds__(512, 2) void small_grad_kernel(const SmallArgs a, c
           for (int r = 0; r < 16; ++r) o[cb][r] *= f;
       }
       // probabilities times 2^11, as two fp16 planes in the order of the value operands' keys
+      const float one = opaque_one();
       u32x4 ph[2], pl[2];
       float ps = 0.f;
 #pragma unroll
@@ -837,9 +838,10 @@ __global__ __launch_bounds__(512, 2) void small_grad_kernel(const SmallArgs a, c
           const float e0 = fast_exp2(__builtin_fmaf(acc[r], lscale, 11.0f - m));
           const float e1 = fast_exp2(__builtin_fmaf(acc[r + 1], lscale, 11.0f - m));
           ps += e0 + e1;
-          const _Float16 h0 = (_Float16)e0, h1 = (_Float16)e1;
-          ph[t][c] = pack_f16((float)h0, (float)h1);
-          pl[t][c] = pack_f16(e0 - (float)h0, e1 - (float)h1);
+          const unsigned both = pack_f16(e0, e1);
+          const f16x2 hi = __builtin_bit_cast(f16x2, both);
+          ph[t][c] = both;
+          pl[t][c] = pack_f16(f16_rest(e0, hi[0], one), f16_rest(e1, hi[1], one));
         }
       s += ps;
 #pragma unroll
