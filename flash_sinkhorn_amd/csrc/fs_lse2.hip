@@ -102,9 +102,10 @@ static int launch_coarse(const LaunchArgs& a, int dp, int rb, int blocks, hipStr
       const bool both = blocks > a.blocks0;
       const double l0 = (double)a.side[0].nq * a.side[0].nk, l1 = both ? (double)a.side[1].nq * a.side[1].nk : 0.0;
       const int t0 = both ? std::min(kCoarse128Grid - 8, std::max(8, (int)(kCoarse128Grid * (l0 / (l0 + l1)) + 0.5))) : kCoarse128Grid;
-      hipLaunchKernelGGL((lse_coarse128_kernel<0>), dim3(blocks), dim3(256), 0, st, c);
-      c.blocks0 = t0;
-      hipLaunchKernelGGL((lse_test128_kernel<0>), dim3(kCoarse128Grid), dim3(256), 0, st, c);
+      c.blocks_sparse = t0;
+      c.blocks0 = std::max(a.blocks0, t0);
+      hipLaunchKernelGGL((lse_coarse128_kernel<0>), dim3(c.blocks0 + (both ? std::max(blocks - a.blocks0, kCoarse128Grid - t0) : 0)),
+                         dim3(256), 0, st, c);
       if (hipGetLastError() != hipSuccess) return FS_ERR_LAUNCH_FAILED;
       c.blocks0 = (a.side[0].nq + 31) / 32;
       hipLaunchKernelGGL((lse_listed128_kernel<false>), dim3(c.blocks0 + (both ? (a.side[1].nq + 31) / 32 : 0)), dim3(256), 0, st, c);

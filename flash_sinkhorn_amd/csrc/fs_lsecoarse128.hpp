@@ -607,8 +607,12 @@ __device__ __forceinline__ void coarse128_in_place(const LaunchArgs& args, const
   }
 }
 
+// Either form of both sides in one launch (as two, one of them found nothing to do: 4 us of a step).  Side 0 has
+// the first blocks0 workgroups, as many as the larger of its forms; the test's are blocks_sparse of them (and what is
+// left of kCoarse128Grid on side 1).
 template <int T>
 __global__ __launch_bounds__(256, 2) void lse_coarse128_kernel(const LaunchArgs args) {
+  static_assert(kTest128Lds <= kCoarse128Lds, "");
   __shared__ __attribute__((aligned(16))) unsigned lds[kCoarse128Lds];
   // variant chosen on the device: the launch of the variant that was not chosen ends here
   if (args.sel_pred && args.sel[kSelWord] != args.sel_want) return;
@@ -616,19 +620,12 @@ __global__ __launch_bounds__(256, 2) void lse_coarse128_kernel(const LaunchArgs 
   const bool second = bid >= args.blocks0;
   if (second) bid -= args.blocks0;
   const Side& sd = second ? args.side[1] : args.side[0];
-  if (!coarse128_lists(args.sel, sd.ps_q)) coarse128_in_place(args, sd, bid, lds);
-}
-
-template <int T>
-__global__ __launch_bounds__(256, 2) void lse_test128_kernel(const LaunchArgs args) {
-  __shared__ __attribute__((aligned(16))) unsigned lds[kTest128Lds];
-  if (args.sel_pred && args.sel[kSelWord] != args.sel_want) return;
-  int bid = blockIdx.x;
-  const bool second = bid >= args.blocks0;
-  if (second) bid -= args.blocks0;
-  const Side& sd = second ? args.side[1] : args.side[0];
-  if (coarse128_lists(args.sel, sd.ps_q))
-    coarse128_test(args, sd, args.tag[second ? 1 : 0], bid, second ? gridDim.x - args.blocks0 : args.blocks0, lds);
+  if (coarse128_lists(args.sel, sd.ps_q)) {
+    const int grid = second ? kCoarse128Grid - args.blocks_sparse : args.blocks_sparse;
+    if (bid < grid) coarse128_test(args, sd, args.tag[second ? 1 : 0], bid, grid, lds);
+  } else if (bid < sd.igroups * sd.splits) {
+    coarse128_in_place(args, sd, bid, lds);
+  }
 }
 
 // A workgroup takes 32 query rows, each of its wavefronts a quarter of the keys.  First the keys on the list; what
