@@ -132,7 +132,7 @@ struct Side {
   const float* knorms;
   // ... and, per 32 rows a line of slack_stride units of 32 keys, which keys are taken (a bit each) and by how much the
   // others are left out (fp16 in base-2 units, rounded down; not above zero: they are taken too), with the keys'
-  // biases and the rows' lines that they were left out by, in raw units (lse_test128_kernel)
+  // biases and the rows' lines that they were left out by, in raw units (coarse128_test)
   unsigned* marks;
   unsigned short* slack;
   float* slack_bias;

@@ -107,6 +107,7 @@ static int launch_coarse(const LaunchArgs& a, int dp, int rb, int blocks, hipStr
       hipLaunchKernelGGL((lse_coarse128_kernel<0>), dim3(c.blocks0 + (both ? std::max(blocks - a.blocks0, kCoarse128Grid - t0) : 0)),
                          dim3(256), 0, st, c);
       if (hipGetLastError() != hipSuccess) return FS_ERR_LAUNCH_FAILED;
+      if (a.side[0].slack == nullptr) return FS_OK;  // (lists would not pay in this launch)
       c.blocks0 = (a.side[0].nq + 31) / 32;
       hipLaunchKernelGGL((lse_listed128_kernel<false>), dim3(c.blocks0 + (both ? (a.side[1].nq + 31) / 32 : 0)), dim3(256), 0, st, c);
       c.blocks0 = both ? kCoarse128Grid / 2 : kCoarse128Grid;

@@ -11,7 +11,7 @@
 //
 // By lists, in two or three launches.  On a peaked plan nearly every unit that goes on does so for one logit
 // (20,000 x 30,000 x 128, eps 0.0025: 1.04 a unit, 37,000 units of 586,000), and which ones these are
-// hardly changes from one half-update to the next.  lse_test128_kernel is nothing but the hi*hi products
+// hardly changes from one half-update to the next.  coarse128_test is nothing but the hi*hi products
 // and their test, and leaves per unit which keys any of its 32 rows needs (Side::marks) and by how much all other logits
 // stay below (Side::slack).  lse_listed128_kernel gathers the keys of 32 rows, 32 at a time, forms their
 // logits from the start and runs the online soft-max.  Where the slack of an earlier launch covers what
@@ -620,7 +620,7 @@ __global__ __launch_bounds__(256, 2) void lse_coarse128_kernel(const LaunchArgs 
   const bool second = bid >= args.blocks0;
   if (second) bid -= args.blocks0;
   const Side& sd = second ? args.side[1] : args.side[0];
-  if (coarse128_lists(args.sel, sd.ps_q)) {
+  if (sd.slack != nullptr && coarse128_lists(args.sel, sd.ps_q)) {
     const int grid = second ? kCoarse128Grid - args.blocks_sparse : args.blocks_sparse;
     if (bid < grid) coarse128_test(args, sd, args.tag[second ? 1 : 0], bid, grid, lds);
   } else if (bid < sd.igroups * sd.splits) {

@@ -261,8 +261,9 @@ __global__ __launch_bounds__(256, (MODE == kMat5 && DP == 128) ? 1 : 2) void pla
   };
 
   // Up to 32 columns: what fp16 leaves of a probability in one instruction, and no sums of the plan where nobody
-  // divides by them (the gradient does): the map of 20,000 x 15,013 x 32 with its vector products 385 -> 376 us.  (At 64 and 128 columns both cost a matrix product
-  // registers that it does not have: 25,000 x 30,000 x 64 with its vector products 1,295 -> 1,317.)
+  // divides by them (the gradient does): the map of 20,000 x 15,013 x 32 with its vector products 385 -> 376 us.
+  // (At 64 and 128 columns both cost a matrix product registers that it does not have: 25,000 x 30,000 x 64 with
+  // its vector products 1,295 -> 1,317.)
   const float one = opaque_one();
   const bool sums = MODE == kMat && (DP >= 64 || sd.ep.kind == kEpiGrad);
   int buf = 0;
