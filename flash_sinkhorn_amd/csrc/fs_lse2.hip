@@ -93,7 +93,7 @@ static int launch_coarse(const LaunchArgs& a, int dp, int rb, int blocks, hipStr
     case 16: return launch_coarse_dp<16>(a, blocks, st);
     case 32: return launch_coarse_dp<32>(a, blocks, st);
     case 64: return launch_coarse_dp<64>(a, blocks, st);
-    case 128:  // no carried margins, no sparse form
+    case 128:  // lists of keys in place of margins
       if (a.side[0].margins != nullptr) return FS_ERR_BAD_ARGUMENT;
     {
       // in place a workgroup per row group and chunk; by lists the workgroups that test are shared out between the

@@ -1090,7 +1090,7 @@ def test_graph_replays_equal_eager_solves(monkeypatch):
 @pytest.mark.parametrize("n,m,d", [(33, 700, 65), (33, 6100, 65), (384, 8192, 128), (385, 6401, 100), (2300, 9000, 96),
                                    (100, 40000, 70)])
 def test_half_updates_by_lists_on_rows_of_65_to_128_columns(n, m, d):
-    """``lse_test128_kernel`` / ``lse_listed128_kernel``: potentials that stay, drift, or change for single keys, for all
+    """``coarse128_test`` / ``lse_listed128_kernel``: potentials that stay, drift, or change for single keys, for all
     keys but one and for everything, behind one test of all units; keys without mass; against fp64.  Sizes
     around the row groups of 32 and 384 rows, the pieces of 128 keys and the 64 pieces a wavefront takes at a time."""
     from flash_sinkhorn_amd import _lib
