@@ -433,7 +433,9 @@ __device__ __forceinline__ bool slack_renewed(const unsigned* st, unsigned tag, 
 // having a start, and kept while they hold 10 % of the keys (else not for sixteen launches); a test is good
 // until the lists have grown by a further 2 % of the keys.  (1 % 3.97 ms, 2 % 4.0 for ten iterations there, at
 // eps 0.05 4.44 and 4.35.)
-__device__ __forceinline__ void slack_after_launch(unsigned* st, int lane, const unsigned (&tag)[2], int sides, const int (&role)[2]) {
+// `chosen`: the device chose the variant, and the plain one ran where the word is set.  (A launch that asks for the test
+// runs it whatever the word says, and has written slack under its own tag.)
+__device__ __forceinline__ void slack_after_launch(unsigned* st, int lane, bool chosen, const unsigned (&tag)[2], int sides, const int (&role)[2]) {
   const unsigned e = st[kSelEnded + lane], u = st[kSelUnits + lane], word = st[kSelWord];
   unsigned taken = lane < 2 * kDmaxSlots ? st[kSelDmax + lane] : 0u;
   unsigned have[2] = {0u, 0u}, known[2] = {0u, 0u}, bump[2] = {0u, 0u}, base[2] = {0u, 0u}, lists[2] = {0u, 0u}, wait[2] = {0u, 0u};
@@ -453,7 +455,7 @@ __device__ __forceinline__ void slack_after_launch(unsigned* st, int lane, const
 #pragma unroll
   for (int o = kDmaxSlots / 2; o > 0; o >>= 1) taken += (unsigned)__shfl_xor((int)taken, o, 64);
   const unsigned of_role[2] = {(unsigned)__shfl((int)taken, 0, 64), (unsigned)__shfl((int)taken, kDmaxSlots, 64)};
-  if (word != 0u || us == 0) return;  // (word: the plain kernel ran)
+  if ((chosen && word != 0u) || us == 0) return;
   if (lane < 2 * kDmaxSlots) st[kSelDmax + lane] = 0u;
   if (lane != 0) return;
   const unsigned share = (unsigned)(((us - min(es, us)) << 16) / us);

@@ -503,7 +503,7 @@ __global__ __launch_bounds__(finish_threads(HAS_O)) void finish_kernel(const Lau
         }
       if (args.side[0].slack != nullptr) {
         const int sides = args.side[1].slack != args.side[0].slack ? 2 : 1, r[2] = {args.side[0].ps_q, args.side[1].ps_q};
-        slack_after_launch(args.sel, threadIdx.x, args.tag, sides, r);
+        slack_after_launch(args.sel, threadIdx.x, args.sel_pred != 0, args.tag, sides, r);
       }
       state_after_launch(args.sel, threadIdx.x, commit_sides, role, ls);
     }

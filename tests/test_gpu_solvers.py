@@ -1132,3 +1132,30 @@ def test_half_updates_by_lists_on_rows_of_65_to_128_columns(n, m, d):
     g += 30.0 * torch.randn(m, device="cuda", generator=gen)
     check()
     check()
+
+
+@pytest.mark.parametrize("n,m,d,eps,other", [(5000, 8000, 128, 0.2, 0.001), (5000, 8000, 128, 0.1, 0.001),
+                                             (2300, 9000, 96, 0.05, 0.0005)])
+def test_lists_of_one_eps_do_not_serve_another(n, m, d, eps, other):
+    """Half-updates by lists at one eps, one or two at a much smaller one, and back: there fewer keys count, and what
+    is left out lies further off in its units.  Every launch against fp64."""
+    from flash_sinkhorn_amd import _lib
+    from flash_sinkhorn_amd.kernels.sinkhorn_flashstyle_sqeuclid import flashsinkhorn_lse_fused
+    gen = torch.Generator(device="cuda").manual_seed(n + d)
+    x = torch.randn(n, d, device="cuda", generator=gen)
+    y = 1.5 * torch.randn(m, d, device="cuda", generator=gen)
+    g = -(y * y).sum(1)
+    lw = torch.log(torch.rand(m, device="cuda", generator=gen) + 0.1)
+    prep = _lib.PreparedOperands(x, y, _lib.flags(True, False))
+    logits = 2.0 * x.double() @ y.double().T + g.double()
+    tol = 2e-6 * float((x * x).sum(1).max() + (y * y).sum(1).max())  # (as in the test above)
+
+    def check(e):
+        out = flashsinkhorn_lse_fused(x, y, g, lw, e, allow_tf32=False, _prepared=prep, _coarse=True)
+        assert float((out + e * torch.logsumexp(logits / e + lw.double(), 1)).abs().max()) <= tol
+
+    for _ in range(6):
+        check(eps)
+    assert prep.variant_state()["by_lists"]
+    for e in (other, eps, eps, other, other, eps):
+        check(e)
