@@ -1170,6 +1170,11 @@ int run_stream(int mode, bool sepv, Side* sides, int nsides, int64_t d, void* ws
           sd.slack_rest = reinterpret_cast<int*>(slot + 3 * slack_bytes(rows) + 2 * row_array_bytes(rows));
           sd.slack_stride = slack_stride_for(rows);
           a.tag[s] = shared ? 0u : tag_of(sd, p);
+          if (sd.slack != nullptr) {
+            a.lists.sides = nsides;
+            a.lists.role[s] = sd.ps_q;
+            a.lists.tag[s] = a.tag[s];
+          }
         }
         sd.qnorms = wide ? row_array_of(ps, cfg, ws, sd.q, sd.nq, 4) : nullptr;
         sd.knorms = wide ? row_array_of(ps, cfg, ws, sd.k, sd.nk, 4) : nullptr;
@@ -1298,7 +1303,7 @@ int run_stream(int mode, bool sepv, Side* sides, int nsides, int64_t d, void* ws
     return hipGetLastError() == hipSuccess ? FS_OK : FS_ERR_LAUNCH_FAILED;
   }
   if (a.sel != nullptr && !any_split) {  // no merge launch to carry the decision
-    hipLaunchKernelGGL((coarse_decide_kernel<0>), dim3(1), dim3(64), 0, st, a.sel);
+    hipLaunchKernelGGL((coarse_decide_kernel<0>), dim3(1), dim3(64), 0, st, a);
     if (hipGetLastError() != hipSuccess) return FS_ERR_LAUNCH_FAILED;
   }
   if (any_split) {

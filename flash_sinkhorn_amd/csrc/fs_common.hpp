@@ -187,6 +187,13 @@ struct LaunchArgs {
   float* col_part_b;
   int sw_items0, sw_items;
   int sw_part_mult;  // partial rows per key chunk (2 for lse_gemm_kernel, else 1; 0 reads as 1)
+  // Rows of 65 .. 128 columns, launches that may go by lists: what becomes of their state (slack_after_launch), for all
+  // sides of the launch, merged or not.
+  struct Lists {
+    int sides;
+    int role[2];      // Side::ps_q
+    unsigned tag[2];
+  } lists;
 };
 
 // Row groups (of 256 rows) that have keys at or beyond their first row in key chunk s of a
@@ -435,7 +442,10 @@ __device__ __forceinline__ bool slack_renewed(const unsigned* st, unsigned tag, 
 // eps 0.05 4.44 and 4.35.)
 // `chosen`: the device chose the variant, and the plain one ran where the word is set.  (A launch that asks for the test
 // runs it whatever the word says, and has written slack under its own tag.)
-__device__ __forceinline__ void slack_after_launch(unsigned* st, int lane, bool chosen, const unsigned (&tag)[2], int sides, const int (&role)[2]) {
+__device__ __forceinline__ void slack_after_launch(unsigned* st, int lane, bool chosen, const LaunchArgs::Lists& of) {
+  const int sides = of.sides;
+  const int (&role)[2] = of.role;
+  const unsigned (&tag)[2] = of.tag;
   const unsigned e = st[kSelEnded + lane], u = st[kSelUnits + lane], word = st[kSelWord];
   unsigned taken = lane < 2 * kDmaxSlots ? st[kSelDmax + lane] : 0u;
   unsigned have[2] = {0u, 0u}, known[2] = {0u, 0u}, bump[2] = {0u, 0u}, base[2] = {0u, 0u}, lists[2] = {0u, 0u}, wait[2] = {0u, 0u};

@@ -501,10 +501,7 @@ __global__ __launch_bounds__(finish_threads(HAS_O)) void finish_kernel(const Lau
           role[i] = ms.ps_q;
           ls[i] = ms.qscale / (ms.plane_scale[ms.ps_q] * ms.plane_scale[ms.ps_k]);
         }
-      if (args.side[0].slack != nullptr) {
-        const int sides = args.side[1].slack != args.side[0].slack ? 2 : 1, r[2] = {args.side[0].ps_q, args.side[1].ps_q};
-        slack_after_launch(args.sel, threadIdx.x, args.sel_pred != 0, args.tag, sides, r);
-      }
+      if (args.lists.sides > 0) slack_after_launch(args.sel, threadIdx.x, args.sel_pred != 0, args.lists);
       state_after_launch(args.sel, threadIdx.x, commit_sides, role, ls);
     }
   }
@@ -748,10 +745,11 @@ __device__ __forceinline__ void sweep_step_merge(const LaunchArgs& args, int ite
 
 // The decision alone, for a step whose launch split no keys (no merge follows).
 template <int T>
-__global__ __launch_bounds__(64) void coarse_decide_kernel(unsigned* state) {
+__global__ __launch_bounds__(64) void coarse_decide_kernel(const LaunchArgs args) {
   const int role[2] = {0, 0};
   const float ls[2] = {0.f, 0.f};
-  state_after_launch(state, threadIdx.x, 0, role, ls);
+  if (args.lists.sides > 0) slack_after_launch(args.sel, threadIdx.x, args.sel_pred != 0, args.lists);
+  state_after_launch(args.sel, threadIdx.x, 0, role, ls);
 }
 
 // kArgmax: merge the partial (largest value, key) pairs of the key splits; equal values keep

@@ -1,4 +1,6 @@
 """Solvers, SamplesLoss, gradients and HVP on the GPU vs the oracle and golden vectors."""
+import math
+
 import numpy as np
 import pytest
 import torch
@@ -1159,3 +1161,48 @@ def test_lists_of_one_eps_do_not_serve_another(n, m, d, eps, other):
     assert prep.variant_state()["by_lists"]
     for e in (other, eps, eps, other, other, eps):
         check(e)
+
+
+def test_lists_of_a_pair_survive_a_step_of_the_self_problems():
+    """One cloud's own 400 keys are not split over workgroups, the other's are: a launch of both self problems writes
+    lists of either and merges one side only.  Half-updates between the clouds before and behind it, against fp64."""
+    from flash_sinkhorn_amd import _lib
+    from flash_sinkhorn_amd.kernels.sinkhorn_flashstyle_sqeuclid import _self_pair_steps_raw, flashsinkhorn_lse_fused
+    n, m, d, eps = 400, 9000, 96, 0.1
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    x = torch.randn(n, d, device="cuda", generator=gen)
+    y = 1.5 * torch.randn(m, d, device="cuda", generator=gen)
+    f, g = -(x * x).sum(1), -(y * y).sum(1)
+    la, lb = torch.full((n,), -math.log(n), device="cuda"), torch.log(torch.rand(m, device="cuda", generator=gen) + 0.1)
+    prep = _lib.PreparedOperands(x, y, _lib.flags(True, False), self_pair=True)
+    want = -eps * torch.logsumexp((2.0 * x.double() @ y.double().T + g.double()) / eps + lb.double(), 1)
+    tol = 2e-6 * float((x * x).sum(1).max() + (y * y).sum(1).max())
+    small = [(0.0005, 0.0005, 1.0, 1.0, 1.0)] * 4  # (another eps, at which fewer keys count)
+    for turn in range(3):
+        for _ in range(5):
+            out = flashsinkhorn_lse_fused(x, y, g, lb, eps, allow_tf32=False, _prepared=prep, _coarse=True)
+            assert float((out - want).abs().max()) <= tol
+        assert turn or prep.variant_state()["by_lists"]
+        _self_pair_steps_raw(x, y, f, g, la, lb, small, cost_scale=1.0, prepared=prep, allow_tf32=False, coarse=True)
+
+
+def test_lists_go_by_the_tag_of_their_own_side():
+    """9,000 rows against 400 keys and the other way round in one launch: only one side's keys are split, and
+    what its state says does not depend on which of the two is first."""
+    from flash_sinkhorn_amd import _lib
+    from flash_sinkhorn_amd.kernels.sinkhorn_flashstyle_sqeuclid import _symmetric_steps_raw
+    n, m, d, eps = 9000, 400, 96, 0.01
+    gen = torch.Generator(device="cuda").manual_seed(6)
+    x, y = (torch.randn(k, d, device="cuda", generator=gen) for k in (n, m))
+    x[:10 * m] = 0.1 * x[:10 * m] + y.repeat_interleave(10, 0)  # (ten neighbours each)
+    la, lb = torch.full((n,), -math.log(n), device="cuda"), torch.full((m,), -math.log(m), device="cuda")
+    f, g = -(x * x).sum(1), -(y * y).sum(1)
+    of_y = 0 if y.data_ptr() < x.data_ptr() else 1
+    tags = []
+    for args in ((x, y, f, g, la, lb), (y, x, g, f, lb, la)):
+        prep = _lib.PreparedOperands(args[0], args[1], _lib.flags(True, False))
+        _symmetric_steps_raw(*args, [(eps, 0.5, 1.0, 1.0)] * 8, cost_scale=1.0, prepared=prep, allow_tf32=False, coarse=True)
+        assert prep.variant_state()["by_lists"]
+        words = prep.ws[prep.state_offset:prep.state_offset + 4 * 146].view(torch.int32).tolist()
+        tags.append(words[138 + of_y])  # (kSelTag)
+    assert tags[0] == tags[1] != 0
