@@ -1174,6 +1174,7 @@ int run_stream(int mode, bool sepv, Side* sides, int nsides, int64_t d, void* ws
             a.lists.sides = nsides;
             a.lists.role[s] = sd.ps_q;
             a.lists.tag[s] = a.tag[s];
+            a.lists.units[s] = (unsigned)ceil_div(sd.nq, 32) * (unsigned)ceil_div(sd.nk, 128) * 4u;
           }
         }
         sd.qnorms = wide ? row_array_of(ps, cfg, ws, sd.q, sd.nq, 4) : nullptr;

@@ -193,6 +193,7 @@ struct LaunchArgs {
     int sides;
     int role[2];      // Side::ps_q
     unsigned tag[2];
+    unsigned units[2];  // 32 x 32 units of the side, in whole pieces of 128 keys
   } lists;
 };
 
@@ -474,7 +475,9 @@ __device__ __forceinline__ void slack_after_launch(unsigned* st, int lane, bool 
     if (i < sides) {
       const int r = role[i];
       const bool renewed = tag[i] == 0u || have[i] == 0u || known[i] != tag[i];
-      const unsigned keys = (unsigned)(((unsigned long long)of_role[r] << 16) * sides / us);
+      // (both sides of one matrix count into the same words)
+      const unsigned long long units = of.units[i] + (sides == 2 && role[i ^ 1] == r ? of.units[i ^ 1] : 0u);
+      const unsigned keys = (unsigned)(((unsigned long long)of_role[r] << 16) / units);
       if (lists[i] == 0u) {
         st[kSelMode + r] = wait[i] == 0u && bump[i] == 0u && share < kListsFrom ? 1u : 0u;
         st[kSelCum + r] = wait[i] - (wait[i] != 0u ? 1u : 0u);

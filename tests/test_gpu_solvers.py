@@ -1206,3 +1206,31 @@ def test_lists_go_by_the_tag_of_their_own_side():
         words = prep.ws[prep.state_offset:prep.state_offset + 4 * 146].view(torch.int32).tolist()
         tags.append(words[138 + of_y])  # (kSelTag)
     assert tags[0] == tags[1] != 0
+
+
+@pytest.mark.parametrize("n,m", [(8192, 0), (8192, 2048), (2048, 8192)])
+def test_lists_are_kept_up_to_a_tenth_of_the_keys(n, m):
+    """Fourteen clusters of points in order: a block of rows needs the 7 % of the keys that are in its own.  A cloud
+    against itself (m = 0), and two clouds of their own in one launch, whose sizes differ."""
+    from flash_sinkhorn_amd import _lib
+    from flash_sinkhorn_amd.kernels.sinkhorn_flashstyle_sqeuclid import _self_pair_steps_raw, _symmetric_steps_raw
+    gen = torch.Generator(device="cuda").manual_seed(7)
+    centres = 10.0 * torch.randn(14, 96, device="cuda", generator=gen)
+
+    def cloud(k):
+        c = centres[torch.arange(k, device="cuda") * 14 // k]
+        return c + 0.1 * torch.randn(k, 96, device="cuda", generator=gen)
+
+    x = cloud(n)
+    la = torch.full((n,), -math.log(n), device="cuda")
+    f, kw = -(x * x).sum(1), dict(cost_scale=1.0, allow_tf32=False, coarse=True)
+    if m == 0:
+        prep = _lib.PreparedOperands(x, x, _lib.flags(True, False))
+        _symmetric_steps_raw(x, x, f, f.clone(), la, la.clone(), [(1.0, 0.5, 1.0, 1.0)] * 8, prepared=prep, **kw)
+    else:
+        y = cloud(m)
+        lb = torch.full((m,), -math.log(m), device="cuda")
+        prep = _lib.PreparedOperands(x, y, _lib.flags(True, False), self_pair=True)
+        _self_pair_steps_raw(x, y, f, -(y * y).sum(1), la, lb, [(1.0, 1.0, 0.5, 1.0, 1.0)] * 8, prepared=prep, **kw)
+    words = prep.ws[prep.state_offset:prep.state_offset + 4 * 146].view(torch.int32).tolist()
+    assert words[144:146] == ([1, 1] if m else [1, 0])  # (kSelMode)
