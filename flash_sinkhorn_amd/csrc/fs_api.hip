@@ -1174,7 +1174,9 @@ int run_stream(int mode, bool sepv, Side* sides, int nsides, int64_t d, void* ws
             a.lists.sides = nsides;
             a.lists.role[s] = sd.ps_q;
             a.lists.tag[s] = a.tag[s];
-            a.lists.units[s] = (unsigned)ceil_div(sd.nq, 32) * (unsigned)ceil_div(sd.nk, 128) * 4u;
+            // (both sides of one matrix count into the same words)
+            for (int t = 0; t < nsides; ++t)
+              if (t == s || shared) a.lists.units[s] += (unsigned)ceil_div(sides[t].nq, 32) * (unsigned)ceil_div(sides[t].nk, 128) * 4u;
           }
         }
         sd.qnorms = wide ? row_array_of(ps, cfg, ws, sd.q, sd.nq, 4) : nullptr;

@@ -193,7 +193,7 @@ struct LaunchArgs {
     int sides;
     int role[2];      // Side::ps_q
     unsigned tag[2];
-    unsigned units[2];  // 32 x 32 units of the side, in whole pieces of 128 keys
+    unsigned units[2];  // 32 x 32 units of the sides of that role, in whole pieces of 128 keys
   } lists;
 };
 
@@ -249,12 +249,13 @@ constexpr int kDmaxSlots = 16;
 constexpr int kSelDmax = kSelForm + 2;
 // likewise per role: margin entries of the current generation exist (lse_coarse_kernel left them
 // behind, or lse_sparse_kernel ran); without them the sparse form would visit every unit
-constexpr unsigned kListsFrom = 26214u, kListsMost = 6554u, kListsGrow = 1311u, kListsWait = 16u;  // (40, 10 and 2 %)
+constexpr unsigned kListsFrom = 26214u, kListsClear = 2949u, kListsMost = 6554u, kListsGrow = 1311u, kListsWait = 16u;  // (40, 4.5, 10 and 2 %)
 constexpr int kSelHave = kSelDmax + 2 * kDmaxSlots;
-// Rows of 65 .. 128 columns use five of these words per role their own way: kSelMode (launches go by lists), kSelHave
-// and kSelTag (Side::slack is that of a launch under this tag), kSelBump (the launch under way had rows without a
-// start), kSelGen (the share of keys taken when they were all tested, in 65536ths), kSelCum (launches until lists are
-// tried again) and the kSelDmax slots (keys taken in the launch under way, by 32).
+// Rows of 65 .. 128 columns use these words per role their own way: kSelMode (launches go by lists), kSelTag (that of
+// the last launch), kSelHave (Side::slack is that of a launch under this tag), kSelBump (the launch under way had rows
+// without a start), kSelGen (the share of keys taken when they were all tested, in 65536ths), kSelCum (launches until
+// lists are tried again) and the kSelDmax slots (of the launch under way, by lists: keys taken, by 32; in place: units
+// without a key that lists would take).  The kSelSkip slots count the units of launches by lists, which are in none of the others.
 // the share of units the plain kernel left out in the first launch of its current stretch, in
 // 65536ths plus one (0: not taken yet)
 constexpr int kSelBase = kSelHave + 2;
@@ -335,12 +336,13 @@ __device__ __forceinline__ bool margins_settled(const unsigned* st, int side, fl
 //   * the launch's unit counters join the totals and are cleared; the kSelDecideSteps-th launch
 //     of the coarse variant with counts decides, and leaves it when too few of its units ended;
 //     the plain kernel counts the units whose exponentials it left out, and a launch that left
-//     out clearly more than the first of its stretch hands the next one back to the coarse variant;
+//     out clearly more than the first of its stretch hands the next one back to the coarse variant
+//     (a launch by lists, which take keys long before they matter, says nothing to that: `lists`);
 //   * per side with carried margins (`commit_sides` of them, their matrices' roles in
 //     `role`, base-2 units per raw unit in `lscale`): the launch's largest bias change joins the
 //     running sum (or starts it, after a launch that began a generation), and the form that ran
 //     is remembered for the hysteresis of margins_settled.
-__device__ __forceinline__ void state_after_launch(unsigned* st, int lane, int commit_sides,
+__device__ __forceinline__ void state_after_launch(unsigned* st, int lane, bool lists, int commit_sides,
                                                    const int (&role)[2], const float (&lscale)[2]) {
   // ---- loads ----
   const unsigned e = st[kSelEnded + lane], u = st[kSelUnits + lane], k = st[kSelSkip + lane];
@@ -382,11 +384,14 @@ __device__ __forceinline__ void state_after_launch(unsigned* st, int lane, int c
   for (int i = 0; i < 2; ++i)
     if (i < commit_sides && lane >= role[i] * kDmaxSlots && lane < (role[i] + 1) * kDmaxSlots)
       st[kSelDmax + lane] = 0u;
-  if (lane == 0 && us > 0) {
+  const unsigned long long listed = lists ? ks : 0ull;
+  if (lane == 0 && us + listed > 0) {
     unsigned long long* out = reinterpret_cast<unsigned long long*>(st + kSelCumEnded);
-    out[0] = c0 + es;
-    out[1] = c1 + us;
+    out[0] = c0 + es + listed;
+    out[1] = c1 + us + listed;
     out[2] = c2 + ks;
+  }
+  if (lane == 0 && us > 0 && listed == 0) {
     if (word == 0u) {
       if (seen < kSelDecideSteps) {  // the share of the last of these launches decides
         st[kSelDecisions] = seen + 1u;
@@ -429,67 +434,69 @@ __device__ __forceinline__ void state_after_launch(unsigned* st, int lane, int c
   }
 }
 
-// Rows of 65 .. 128 columns: does a side's launch go by lists (lse_coarse128_kernel, lse_listed128_kernel)?
-__device__ __forceinline__ bool coarse128_lists(const unsigned* st, int role) { return st != nullptr && st[kSelMode + role] != 0u; }
+// Rows of 65 .. 128 columns: does a side's launch go by lists (lse_coarse128_kernel, lse_listed128_kernel)?  Under another
+// tag than the launch before it goes on in place.
+__device__ __forceinline__ bool coarse128_lists(const unsigned* st, unsigned tag, int role) {
+  return st != nullptr && st[kSelMode + role] != 0u && st[kSelTag + role] == tag;
+}
 // ... and are all units of it tested (or is the slack of an earlier launch good)?
 __device__ __forceinline__ bool slack_renewed(const unsigned* st, unsigned tag, int role) {
   return st == nullptr || tag == 0u || st[kSelHave + role] == 0u || st[kSelTag + role] != tag;
 }
 // One wavefront, in front of state_after_launch.  At 20,000 x 30,000 a launch in place takes 210 us and 0.5 for every
 // thousand units of 586 that go on; one by lists 25 us and 1.4 for every thousand times 32 keys of a row block's
-// list, and 150 to 200 more with the test.  Lists are tried where 40 % of the units go on at most, all rows
-// having a start, and kept while they hold 10 % of the keys (else not for sixteen launches); a test is good
-// until the lists have grown by a further 2 % of the keys.  (1 % 3.97 ms, 2 % 4.0 for ten iterations there, at
+// list, and 150 to 200 more with the test.  Lists are kept while they hold 10 % of the keys; a test is good
+// until they have grown by a further 2 % of the keys.  (1 % 3.97 ms, 2 % 4.0 for ten iterations there, at
 // eps 0.05 4.44 and 4.35.)
+// They are tried where a launch in place, under the same tag as the one before it and all rows having a start, finished
+// 40 % of the units at most and left 4.5 % or more without a key that lists would take, which a tenth of the keys do: 0.9^32 =
+// 3.4 % where they are spread evenly, 5 and 7 % were measured at 9.5 and 8.8 % of N(0, I)'s.  (A launch by lists of most
+// keys takes several in place: 30,000 x 28,000 x 96 at eps 0.2 2,800 us for 780.)  Where they hold more after all the
+// next try is 16 launches away, 64 with more than twice that.
 // `chosen`: the device chose the variant, and the plain one ran where the word is set.  (A launch that asks for the test
 // runs it whatever the word says, and has written slack under its own tag.)
 __device__ __forceinline__ void slack_after_launch(unsigned* st, int lane, bool chosen, const LaunchArgs::Lists& of) {
-  const int sides = of.sides;
-  const int (&role)[2] = of.role;
-  const unsigned (&tag)[2] = of.tag;
-  const unsigned e = st[kSelEnded + lane], u = st[kSelUnits + lane], word = st[kSelWord];
+  const unsigned e = st[kSelEnded + lane], u = st[kSelUnits + lane], k = st[kSelSkip + lane], word = st[kSelWord];
   unsigned taken = lane < 2 * kDmaxSlots ? st[kSelDmax + lane] : 0u;
-  unsigned have[2] = {0u, 0u}, known[2] = {0u, 0u}, bump[2] = {0u, 0u}, base[2] = {0u, 0u}, lists[2] = {0u, 0u}, wait[2] = {0u, 0u};
+  unsigned known[2] = {0u, 0u}, bump[2] = {0u, 0u}, base[2] = {0u, 0u}, wait[2] = {0u, 0u};
+  bool lists[2] = {false, false}, renewed[2] = {false, false};
 #pragma unroll
   for (int i = 0; i < 2; ++i)
-    if (i < sides) {
-      lists[i] = st[kSelMode + role[i]];
-      have[i] = st[kSelHave + role[i]];
-      known[i] = st[kSelTag + role[i]];
-      bump[i] = st[kSelBump + role[i]];
-      base[i] = st[kSelGen + role[i]];
-      wait[i] = st[kSelCum + role[i]];
+    if (i < of.sides) {
+      lists[i] = coarse128_lists(st, of.tag[i], of.role[i]);
+      renewed[i] = slack_renewed(st, of.tag[i], of.role[i]);
+      known[i] = st[kSelTag + of.role[i]];
+      bump[i] = st[kSelBump + of.role[i]];
+      base[i] = st[kSelGen + of.role[i]];
+      wait[i] = st[kSelCum + of.role[i]];
     }
-  unsigned long long es = e, us = u;
+  unsigned long long es = e, us = u, ks = k;
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) es += __shfl_xor(es, o, 64), us += __shfl_xor(us, o, 64);
+  for (int o = 32; o > 0; o >>= 1) es += __shfl_xor(es, o, 64), us += __shfl_xor(us, o, 64), ks += __shfl_xor(ks, o, 64);
 #pragma unroll
   for (int o = kDmaxSlots / 2; o > 0; o >>= 1) taken += (unsigned)__shfl_xor((int)taken, o, 64);
   const unsigned of_role[2] = {(unsigned)__shfl((int)taken, 0, 64), (unsigned)__shfl((int)taken, kDmaxSlots, 64)};
-  if ((chosen && word != 0u) || us == 0) return;
+  if ((chosen && word != 0u) || us + ks == 0) return;
   if (lane < 2 * kDmaxSlots) st[kSelDmax + lane] = 0u;
   if (lane != 0) return;
-  const unsigned share = (unsigned)(((us - min(es, us)) << 16) / us);
+  const bool few = (us - min(es, us)) << 16 < us * kListsFrom;  // (of the sides in place)
 #pragma unroll
   for (int i = 0; i < 2; ++i)
-    if (i < sides) {
-      const int r = role[i];
-      const bool renewed = tag[i] == 0u || have[i] == 0u || known[i] != tag[i];
-      // (both sides of one matrix count into the same words)
-      const unsigned long long units = of.units[i] + (sides == 2 && role[i ^ 1] == r ? of.units[i ^ 1] : 0u);
-      const unsigned keys = (unsigned)(((unsigned long long)of_role[r] << 16) / units);
-      if (lists[i] == 0u) {
-        st[kSelMode + r] = wait[i] == 0u && bump[i] == 0u && share < kListsFrom ? 1u : 0u;
+    if (i < of.sides) {
+      const int r = of.role[i];
+      const unsigned share = (unsigned)(((unsigned long long)of_role[r] << 16) / of.units[i]);
+      if (!lists[i]) {
+        st[kSelMode + r] = wait[i] == 0u && bump[i] == 0u && known[i] == of.tag[i] && few && share >= kListsClear ? 1u : 0u;
         st[kSelCum + r] = wait[i] - (wait[i] != 0u ? 1u : 0u);
         st[kSelHave + r] = 0u;
-      } else if (renewed) {
-        st[kSelHave + r] = tag[i] != 0u && bump[i] == 0u ? 1u : 0u;
-        st[kSelTag + r] = tag[i];
-        st[kSelGen + r] = keys;
-        if (keys > kListsMost) st[kSelMode + r] = 0u, st[kSelCum + r] = kListsWait;
-      } else if (keys > base[i] + kListsGrow) {
+      } else if (renewed[i]) {
+        st[kSelHave + r] = of.tag[i] != 0u && bump[i] == 0u ? 1u : 0u;
+        st[kSelGen + r] = share;
+        if (share > kListsMost) st[kSelMode + r] = 0u, st[kSelCum + r] = share > 2u * kListsMost ? 4u * kListsWait : kListsWait;
+      } else if (share > base[i] + kListsGrow) {
         st[kSelHave + r] = 0u;
       }
+      st[kSelTag + r] = of.tag[i];
       st[kSelBump + r] = 0u;
     }
 }

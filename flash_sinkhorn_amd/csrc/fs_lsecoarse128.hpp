@@ -413,6 +413,8 @@ __device__ __forceinline__ void coarse128_in_place(const LaunchArgs& args, const
     return m;
   };
 
+  const float clear = args.skip_log2 - kTakeReserve;
+
   // ---- running statistics.  The logits stay in absolute raw units (of the full logit with
   // its key bias); the running maximum M is kept as run_c = -M * lscale, rounded once: the
   // constant of the exponentials and what the test compares with (subtracted inside the
@@ -442,7 +444,7 @@ __device__ __forceinline__ void coarse128_in_place(const LaunchArgs& args, const
     started[rb] = seeded;
     if (!seeded) run_c[rb] = 0.f;
   }
-  unsigned n_ended = 0;
+  unsigned n_ended = 0, n_clear = 0;  // n_clear: units of which lists would take nothing
 
   // ---- prologue: tile 0 and its bias terms ----
   if (ntiles > 0) {
@@ -494,7 +496,9 @@ __device__ __forceinline__ void coarse128_in_place(const LaunchArgs& args, const
         const float corr = __builtin_fmaf(norm_lo[rb], most_hi, __builtin_fmaf(norm_hi[rb], most_lo, inv_lscale));
         // every logit of the unit at least 2^40 below its row's running maximum, whatever the
         // cross products add: nothing of it could change the fp32 sums
-        if (started[rb] && !wave_any(__builtin_fmaf(tmax + corr, lscale, run_c[rb]) > args.skip_log2)) {
+        const float above = __builtin_fmaf(tmax + corr, lscale, run_c[rb]);
+        n_clear += wave_any(above > clear) ? 0u : 1u;
+        if (started[rb] && !wave_any(above > args.skip_log2)) {
           ++n_ended;
           continue;
         }
@@ -582,6 +586,7 @@ __device__ __forceinline__ void coarse128_in_place(const LaunchArgs& args, const
     const int slot = blockIdx.x % kSelSlots;
     atomicAdd(&args.sel[kSelEnded + slot], n_ended);
     atomicAdd(&args.sel[kSelUnits + slot], (unsigned)(ntiles * NSUB * RB));
+    if (n_clear > 0) atomicAdd(&args.sel[kSelDmax + sd.ps_q * kDmaxSlots + (blockIdx.x & (kDmaxSlots - 1))], n_clear);
   }
 
 #pragma unroll
@@ -620,7 +625,7 @@ __global__ __launch_bounds__(256, 2) void lse_coarse128_kernel(const LaunchArgs 
   const bool second = bid >= args.blocks0;
   if (second) bid -= args.blocks0;
   const Side& sd = second ? args.side[1] : args.side[0];
-  int lists = __builtin_amdgcn_readfirstlane(sd.slack != nullptr && coarse128_lists(args.sel, sd.ps_q) ? 1 : 0);
+  int lists = __builtin_amdgcn_readfirstlane(sd.slack != nullptr && coarse128_lists(args.sel, args.tag[second ? 1 : 0], sd.ps_q) ? 1 : 0);
   if (lists == 0 && bid < sd.igroups * sd.splits) coarse128_in_place(args, sd, bid, lds);
   // (one behind the other for the compiler: as two branches of one condition they shared what the form in place had no
   // registers for, and it spilled: 20,000 x 30,000 x 128 at eps 0.2 256 and 284 us a half-update for 244 and 262)
@@ -650,7 +655,7 @@ __global__ __launch_bounds__(256, 2) void lse_listed128_kernel(const LaunchArgs 
   constexpr int kListKeys = 256;
   __shared__ unsigned short lds_keys[4][kListKeys];  // of the batch's first key
   __shared__ float sh_max[4][32], sh_sum[4][32], sh_top[4][32];
-  __shared__ int sh_key[4][32], sh_count[2][4];
+  __shared__ int sh_key[4][32], sh_count[4];
 
   if (args.sel_pred && args.sel[kSelWord] != args.sel_want) return;
   int bid = blockIdx.x;
@@ -659,7 +664,7 @@ __global__ __launch_bounds__(256, 2) void lse_listed128_kernel(const LaunchArgs 
   const Side& sd = second ? args.side[1] : args.side[0];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int li = lane & 31, h = lane >> 5;
-  if (!coarse128_lists(args.sel, sd.ps_q)) return;
+  if (!coarse128_lists(args.sel, args.tag[second ? 1 : 0], sd.ps_q)) return;
   // (left to the second launch: their number, the row blocks, and by how much their lines have fallen)
   int* put_off = sd.slack_rest;
   float* put_off_fall = reinterpret_cast<float*>(sd.slack_rest) + (sd.nq + 31) / 32 + 4;
@@ -696,7 +701,7 @@ __global__ __launch_bounds__(256, 2) void lse_listed128_kernel(const LaunchArgs 
 
   // ---- the keys that are taken, in order, of 64 pieces of 128 at a time (one a lane) ----
   unsigned taken[4] = {0u, 0u, 0u, 0u};
-  int n_on = 0, n_taken = 0;
+  int n_taken = 0;
   auto load_marks = [&](int from, bool rest) {
     const int piece = min(from + lane, piece1 - 1);
     const size_t at = (size_t)block * sd.slack_stride + piece * 4;
@@ -716,7 +721,6 @@ __global__ __launch_bounds__(256, 2) void lse_listed128_kernel(const LaunchArgs 
       if (from + lane >= piece1 || keys <= 0) t = 0u;
       else if (keys < 32) t &= (1u << keys) - 1u;
       taken[k] = t;
-      if (!rest) n_on += __builtin_popcountll(__builtin_amdgcn_ballot_w64(t != 0u));
     }
   };
   // (a list of what fits of them from key number `first` of the batch on)
@@ -812,9 +816,9 @@ __global__ __launch_bounds__(256, 2) void lse_listed128_kernel(const LaunchArgs 
     }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) keys += __shfl_xor(keys, o, 64);
-    if (lane == 0) sh_count[0][wave] = keys;
+    if (lane == 0) sh_count[wave] = keys;
     __syncthreads();
-    keys = sh_count[0][0] + sh_count[0][1] + sh_count[0][2] + sh_count[0][3];
+    keys = sh_count[0] + sh_count[1] + sh_count[2] + sh_count[3];
     __syncthreads();
     if (keys == 0) break;
     if (keys > kRestKeys && sd.splits > 1) {
@@ -994,21 +998,16 @@ __global__ __launch_bounds__(256, 2) void lse_listed128_kernel(const LaunchArgs 
       sh_top[wave][li] = best_v;
       sh_key[wave][li] = best_j;
     }
-    if (lane == 0) sh_count[0][wave] = n_on, sh_count[1][wave] = n_taken;
+    if (lane == 0) sh_count[wave] = n_taken;
   }
   __syncthreads();
   // unit counts for the variant choice on the device (one set of atomics per workgroup: one per wavefront took 17 us
   // of a launch's 51)
   if (args.sel != nullptr && threadIdx.x == 0) {
-    const int at = blockIdx.x % kSelSlots;
-    const unsigned units = (unsigned)(4 * pieces), on = (unsigned)(sh_count[0][0] + sh_count[0][1] + sh_count[0][2] + sh_count[0][3]);
     unsigned gathered = 0u;
 #pragma unroll
-    for (int w = 0; w < 4; ++w) gathered += (unsigned)((sh_count[1][w] + 31) / 32);
-    if (!REST) {
-      atomicAdd(&args.sel[kSelEnded + at], units - min(on, units));
-      atomicAdd(&args.sel[kSelUnits + at], units);
-    }
+    for (int w = 0; w < 4; ++w) gathered += (unsigned)((sh_count[w] + 31) / 32);
+    if (!REST) atomicAdd(&args.sel[kSelSkip + blockIdx.x % kSelSlots], (unsigned)(4 * pieces));
     atomicAdd(&args.sel[kSelDmax + sd.ps_q * kDmaxSlots + (blockIdx.x & (kDmaxSlots - 1))], gathered);
   }
   if (row < sd.nq && h == 0) {

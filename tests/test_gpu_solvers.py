@@ -1234,3 +1234,38 @@ def test_lists_are_kept_up_to_a_tenth_of_the_keys(n, m):
         _self_pair_steps_raw(x, y, f, -(y * y).sum(1), la, lb, [(1.0, 1.0, 0.5, 1.0, 1.0)] * 8, prepared=prep, **kw)
     words = prep.ws[prep.state_offset:prep.state_offset + 4 * 146].view(torch.int32).tolist()
     assert words[144:146] == ([1, 1] if m else [1, 0])  # (kSelMode)
+
+
+def _steps_by_launch(x, y, eps, steps):
+    """Two-sided steps with the variant left to the device, one launch a call: what the state says behind each."""
+    from flash_sinkhorn_amd import _lib
+    from flash_sinkhorn_amd.kernels.sinkhorn_flashstyle_sqeuclid import _symmetric_step_raw
+    n, m = x.shape[0], y.shape[0]
+    la, lb = torch.full((n,), -math.log(n), device="cuda"), torch.full((m,), -math.log(m), device="cuda")
+    f, g = -(x * x).sum(1), -(y * y).sum(1)
+    prep, states = _lib.PreparedOperands(x, y, _lib.flags(True, False)), []
+    for _ in range(steps):
+        f, g = _symmetric_step_raw(x, y, f, g, la, lb, eps, cost_scale=1.0, alpha=0.5, damping_f=1.0, damping_g=1.0,
+                                   allow_tf32=False, coarse="auto", prepared=prep)
+        states.append(prep.variant_state())
+    return states
+
+
+def test_lists_are_not_tried_where_they_would_hold_most_keys():
+    """At eps 0.2 most units end at the test, but nearly all hold a key that lists would take: a launch by lists
+    of them takes several in place."""
+    gen = torch.Generator(device="cuda").manual_seed(8)
+    x, y = (torch.randn(k, 128, device="cuda", generator=gen) for k in (8000, 9000))
+    states = _steps_by_launch(x, y, 0.2, 12)
+    assert not any(s["by_lists"] for s in states)
+    assert not states[-1]["plain_selected"] and states[-1]["tiles_ended"] > 0.5 * states[-1]["tiles_tested"]
+
+
+def test_launches_by_lists_do_not_choose_the_variant():
+    """At eps 0.05 the second launch, in place, ends most units at the test, and the lists of the third hold a key of
+    most of them, which says nothing about the test."""
+    gen = torch.Generator(device="cuda").manual_seed(8)
+    x, y = (torch.randn(k, 128, device="cuda", generator=gen) for k in (8000, 9000))
+    states = _steps_by_launch(x, y, 0.05, 6)
+    assert [s["by_lists"] for s in states] == [False] + [True] * 5
+    assert [s["decisions"] for s in states] == [1] + [2] * 5 and not states[-1]["plain_selected"]
