@@ -437,7 +437,7 @@ __device__ __forceinline__ void coarse128_in_place(const LaunchArgs& args, const
   }
   // (wavefront-uniform: without a starting value for every row the first unit sets the maxima)
   seeded = __builtin_amdgcn_ballot_w64(seeded) == ~0ull;
-  if (!seeded && args.sel != nullptr && lane == 0) args.sel[kSelBump + sd.ps_q] = 1u;
+  if (!seeded && args.sel != nullptr && sd.slack != nullptr && lane == 0) args.sel[kSelBump + sd.ps_q] = 1u;
   bool started[RB];
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb) {
@@ -586,7 +586,7 @@ __device__ __forceinline__ void coarse128_in_place(const LaunchArgs& args, const
     const int slot = blockIdx.x % kSelSlots;
     atomicAdd(&args.sel[kSelEnded + slot], n_ended);
     atomicAdd(&args.sel[kSelUnits + slot], (unsigned)(ntiles * NSUB * RB));
-    if (n_clear > 0) atomicAdd(&args.sel[kSelDmax + sd.ps_q * kDmaxSlots + (blockIdx.x & (kDmaxSlots - 1))], n_clear);
+    if (n_clear > 0 && sd.slack != nullptr) atomicAdd(&args.sel[kSelDmax + sd.ps_q * kDmaxSlots + (blockIdx.x & (kDmaxSlots - 1))], n_clear);
   }
 
 #pragma unroll

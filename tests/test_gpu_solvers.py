@@ -1269,3 +1269,20 @@ def test_launches_by_lists_do_not_choose_the_variant():
     states = _steps_by_launch(x, y, 0.05, 6)
     assert [s["by_lists"] for s in states] == [False] + [True] * 5
     assert [s["decisions"] for s in states] == [1] + [2] * 5 and not states[-1]["plain_selected"]
+
+
+def test_steps_without_lists_leave_no_counts():
+    """Steps whose eps changes from one to the next go without lists: what their launches in place would count for them
+    would stand until the next launch that has lists."""
+    from flash_sinkhorn_amd import _lib
+    from flash_sinkhorn_amd.kernels.sinkhorn_flashstyle_sqeuclid import _symmetric_steps_raw
+    gen = torch.Generator(device="cuda").manual_seed(9)
+    x, y = (torch.randn(k, 96, device="cuda", generator=gen) for k in (3000, 4000))
+    la, lb = (torch.full((k,), -math.log(k), device="cuda") for k in (3000, 4000))
+    prep = _lib.PreparedOperands(x, y, _lib.flags(True, False))
+    steps = [(0.02, 0.5, 1.0, 1.0), (0.03, 0.5, 1.0, 1.0)] * 5
+    _symmetric_steps_raw(x, y, -(x * x).sum(1), -(y * y).sum(1), la, lb, steps, cost_scale=1.0, prepared=prep,
+                         allow_tf32=False, coarse=True)
+    words = prep.ws[prep.state_offset:prep.state_offset + 4 * 244].view(torch.int32).tolist()
+    assert prep.variant_state()["tiles_tested"] > 0
+    assert not any(words[212:244]) and not any(words[142:144])  # (kSelDmax, kSelBump)
