@@ -1021,12 +1021,9 @@ int run_stream(int mode, bool sepv, Side* sides, int nsides, int64_t d, void* ws
   // the kernel variant with the coarse tile test: asked for, or left to the device.  The device's
   // choice lives in state that belongs to prepared planes (a call that writes its own planes
   // would start it afresh), so without them FS_FLAG_COARSE_AUTO means the plain kernel.
-  // (rows of 65 .. 128 columns: lse_coarse128_kernel, without carried margins)
+  // (rows of 65 .. 128 columns: lse_coarse128_kernel, by lists in place of carried margins, at any size without them)
   const bool wide = dp2 == 128;
-  int64_t most_rows = 0;
-  for (int s = 0; s < nsides; ++s) most_rows = std::max<int64_t>(most_rows, std::max(sides[s].nq, sides[s].nk));
-  const bool can_coarse = lse2 && mode == kLse && prec == 3 && dp2 <= 128 && !(flags & FS_FLAG_NO_TILE_SKIP) &&
-                          (!wide || margin_slot_bytes(most_rows, cfg) > 0);
+  const bool can_coarse = lse2 && mode == kLse && prec == 3 && dp2 <= 128 && !(flags & FS_FLAG_NO_TILE_SKIP);
   const bool coarse = (flags & FS_FLAG_COARSE_TEST) && can_coarse;
   const bool auto_sel = (flags & FS_FLAG_COARSE_AUTO) && can_coarse && !coarse && prepared;
   Family fam_plan = fam;
@@ -1163,7 +1160,7 @@ int run_stream(int mode, bool sepv, Side* sides, int nsides, int64_t d, void* ws
           const bool shared = nsides == 2 && plane_index(ps, sides[0].q, sides[0].nq) == plane_index(ps, sides[1].q, sides[1].nq);
           const int rows = std::max(ps.rows[0], ps.n > 1 ? ps.rows[1] : 0);
           char* slot = static_cast<char*>(ws) + ps.margin_off + (size_t)(shared ? s : sd.ps_q) * ps.margin_slot;
-          sd.slack = (flags & kFlagNoLists) ? nullptr : reinterpret_cast<unsigned short*>(slot);
+          sd.slack = (flags & kFlagNoLists) || ps.margin_slot == 0 ? nullptr : reinterpret_cast<unsigned short*>(slot);
           sd.marks = reinterpret_cast<unsigned*>(slot + slack_bytes(rows));
           sd.slack_bias = reinterpret_cast<float*>(slot + 3 * slack_bytes(rows));
           sd.slack_floor = reinterpret_cast<float*>(slot + 3 * slack_bytes(rows) + row_array_bytes(rows));

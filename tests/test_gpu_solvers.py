@@ -1286,3 +1286,25 @@ def test_steps_without_lists_leave_no_counts():
     words = prep.ws[prep.state_offset:prep.state_offset + 4 * 244].view(torch.int32).tolist()
     assert prep.variant_state()["tiles_tested"] > 0
     assert not any(words[212:244]) and not any(words[142:144])  # (kSelDmax, kSelBump)
+
+
+@pytest.mark.parametrize("n,lists", [(301000, True), (303000, False)])
+def test_the_tile_test_runs_on_clouds_too_large_for_lists(n, lists):
+    """Rows of 65 to 128 columns: the state of lists is kept up to 512 MiB a cloud; the form in place needs none of it."""
+    from flash_sinkhorn_amd import _lib
+    from flash_sinkhorn_amd.kernels.sinkhorn_flashstyle_sqeuclid import flashsinkhorn_lse_fused
+    m, d, eps = 2500, 66, 0.002
+    gen = torch.Generator(device="cuda").manual_seed(10)
+    x, y = (torch.randn(k, d, device="cuda", generator=gen) for k in (n, m))
+    g, lw = -(y * y).sum(1), torch.full((m,), -math.log(m), device="cuda")
+    rows = torch.arange(0, n, 997, device="cuda")
+    want = -eps * torch.logsumexp((2.0 * x[rows].double() @ y.double().T + g.double()) / eps + lw.double(), 1)
+    tol = 2e-6 * float((x * x).sum(1).max() + (y * y).sum(1).max())
+    prep, by_lists = _lib.PreparedOperands(x, y, _lib.flags(True, False)), []
+    for _ in range(4):
+        out = flashsinkhorn_lse_fused(x, y, g, lw, eps, allow_tf32=False, _prepared=prep, _coarse=True)
+        assert float((out[rows] - want).abs().max()) <= tol
+        by_lists.append(prep.variant_state()["by_lists"])
+    state = prep.variant_state()
+    assert state["tiles_ended"] > 0.5 * state["tiles_tested"] > 0
+    assert any(by_lists) == lists
