@@ -415,7 +415,7 @@ int launch_plane_set(const PlaneSet& ps, const LseConfig& c, int64_t d, void* ws
   if (ps.n == 0) return FS_OK;
   char* base = static_cast<char*>(ws);
   int rc = FS_OK;
-  if (keep && ps.margin_slot > 0)
+  if (keep && ps.margin_slot > 0 && !plane_norms(c))  // (lists are written before they are read)
     rc = launch_fill_zero(reinterpret_cast<unsigned*>(base + ps.margin_off),
                           (long long)(2 * ps.margin_slot / 4), st);
   if (rc != FS_OK) return rc;
@@ -837,7 +837,10 @@ int run_plan_tile(int mode, Side* sides, int nsides, int64_t d, const LseConfig&
   const bool has_o = (mode == kMat || mat5);
   // one row block where two would spill: 128-column rows and mat5
   if (dpk == 128 || mat5) rb = 1;
-  size_t need = ps.end;
+  // (the state of the lists of 65 .. 128 columns is no part of a product's workspace: on prepared planes the product
+  // takes its place, and the next launch that has lists starts them afresh)
+  const bool lists = plane_norms(cfg) && ps.margin_slot > 0;
+  size_t need = lists ? ps.margin_off : ps.end;
   SidePlan plans[2];
   size_t vt_off[2] = {0, 0}, part_off[2], q2_off = 0, bounds_off = 0;
   for (int s = 0; s < nsides; ++s) {
@@ -914,6 +917,7 @@ int run_plan_tile(int mode, Side* sides, int nsides, int64_t d, const LseConfig&
   if (total <= 0) return FS_OK;
 
   if (!prepared) rc = launch_plane_set(ps, cfg, d, ws, st);
+  else if (lists) rc = launch_fill_zero(select_state(ps, ws) + kSelHave, 2, st);
   if (any_seed && rc == FS_OK) rc = launch_row_seeds(a, dpk, nsides, st);
   if (mat5 && rc == FS_OK) {
     const Side& sd = sides[0];
@@ -968,7 +972,7 @@ size_t pt_ws_bytes(int mode, int64_t n, int64_t m, int64_t d, bool both, bool ei
   LseConfig c;
   c.gemm = false; c.prec = 3; c.dp = dpk; c.np = 2;
   const size_t planes = plane_bytes(n, c) + plane_bytes(m, c) + 64 + kPlaneAuxBytes +
-                        margin_region_bytes(std::max(n, m), c);  // the whole plane set
+                        (plane_norms(c) ? 0 : margin_region_bytes(std::max(n, m), c));  // the whole plane set
   auto side = [&](int64_t nq, int64_t nk) {
     size_t b = 0;
     for (int rb = 1; rb <= 2; ++rb)

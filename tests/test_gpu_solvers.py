@@ -1308,3 +1308,31 @@ def test_the_tile_test_runs_on_clouds_too_large_for_lists(n, lists):
     state = prep.variant_state()
     assert state["tiles_ended"] > 0.5 * state["tiles_tested"] > 0
     assert any(by_lists) == lists
+
+
+def test_a_product_on_prepared_planes_and_lists_share_a_workspace():
+    """A plan-vector product in the workspace of half-updates by lists, no larger than either needs: both against fp64,
+    in turn."""
+    from flash_sinkhorn_amd import _lib
+    from flash_sinkhorn_amd.kernels.sinkhorn_flashstyle_sqeuclid import flashsinkhorn_lse_fused
+    n, m, d, eps = 9000, 8000, 96, 0.02
+    L, gen = _lib.lib(), torch.Generator(device="cuda").manual_seed(11)
+    x, y = (torch.randn(k, d, device="cuda", generator=gen) for k in (n, m))
+    g, lb, la = -(y * y).sum(1), torch.full((m,), -math.log(m), device="cuda"), torch.full((n,), -math.log(n), device="cuda")
+    v, out = torch.rand(m, device="cuda", generator=gen), torch.empty(n, device="cuda")
+    prep = _lib.PreparedOperands(x, y, _lib.flags(True, False))
+    assert prep.nbytes >= L.fs_workspace_bytes(_lib.OP_APPLY_VEC, n, m, d)
+    logits = (2.0 * x.double() @ y.double().T + g.double()) / eps + lb.double()
+    want_f = -eps * torch.logsumexp(logits, 1)
+    want_v = (torch.softmax(logits, 1) @ v.double()) / n
+    tol = 2e-6 * float((x * x).sum(1).max() + (y * y).sum(1).max())
+    for _ in range(3):
+        for _ in range(4):
+            f = flashsinkhorn_lse_fused(x, y, g, lb, eps, allow_tf32=False, _prepared=prep, _coarse=True)
+            assert float((f - want_f).abs().max()) <= tol
+        assert prep.variant_state()["by_lists"]
+        flags = _lib.flags(True, False) | _lib.FS_FLAG_OPERANDS_PREPARED
+        assert L.fs_apply_vec(x.data_ptr(), y.data_ptr(), f.data_ptr(), g.data_ptr(), la.data_ptr(), lb.data_ptr(),
+                              v.data_ptr(), out.data_ptr(), n, m, d, eps, 2.0, 1, flags, prep.ws.data_ptr(), prep.nbytes,
+                              _lib.stream_of(x)) == 0
+        assert float((out - want_v).abs().max()) <= tol / eps * float(want_v.max())  # (an error of tol in a potential)

@@ -86,6 +86,13 @@ def test_workspace_is_deterministic_and_zero_for_small_problems():
     assert a == L.fs_workspace_bytes(_lib.OP_GRAD, 50000, 50000, 64) and a > 0
 
 
+@pytest.mark.parametrize("op", ["GRAD", "APPLY_VEC", "APPLY_MAT", "MAT5", "C_TRANSFORM"])
+def test_products_of_rows_of_65_to_128_columns_need_no_room_for_lists(op):
+    """The state of lists grows with the square of the rows; only log-sum-exp launches read it."""
+    need = [_lib.lib().fs_workspace_bytes(getattr(_lib, "OP_" + op), n, n, 100) for n in (100_000, 200_000)]
+    assert 0 < need[1] <= 2.01 * need[0]
+
+
 def test_workspace_of_a_batch_follows_the_size_of_its_items():
     from flash_sinkhorn_amd import _small
 
