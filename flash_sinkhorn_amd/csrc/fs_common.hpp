@@ -187,7 +187,7 @@ struct LaunchArgs {
   float* col_part_b;
   int sw_items0, sw_items;
   int sw_part_mult;  // partial rows per key chunk (2 for lse_gemm_kernel, else 1; 0 reads as 1)
-  // Rows of 65 .. 128 columns, launches that may go by lists: what becomes of their state (slack_after_launch), for all
+  // Rows of 65 .. 128 columns, launches that may go by lists: what becomes of their state (lists_after_launch), for all
   // sides of the launch, merged or not.
   struct Lists {
     int sides;
@@ -330,6 +330,75 @@ __device__ __forceinline__ bool margins_settled(const unsigned* st, int side, fl
   return d < (st[kSelMode + side] != 0u ? kUnsettleAbove : kSettleBelow);  // false when d is not a number
 }
 
+// Rows of 65 .. 128 columns: does a side's launch go by lists (lse_coarse128_kernel, lse_listed128_kernel)?  Under another
+// tag than the launch before it goes on in place.
+__device__ __forceinline__ bool coarse128_lists(const unsigned* st, unsigned tag, int role) {
+  return st != nullptr && st[kSelMode + role] != 0u && st[kSelTag + role] == tag;
+}
+// ... and are all units of it tested (or is the slack of an earlier launch good)?
+__device__ __forceinline__ bool slack_renewed(const unsigned* st, unsigned tag, int role) {
+  return st == nullptr || tag == 0u || st[kSelHave + role] == 0u || st[kSelTag + role] != tag;
+}
+// The state of lists, read and brought up to date by state_after_launch.  At 20,000 x 30,000 a launch in place takes 210 us and 0.5 for every
+// thousand units of 586 that go on; one by lists 25 us and 1.4 for every thousand times 32 keys of a row block's
+// list, and 150 to 200 more with the test.  Lists are kept while they hold 10 % of the keys; a test is good
+// until they have grown by a further 2 % of the keys.  (1 % 3.97 ms, 2 % 4.0 for ten iterations there, at
+// eps 0.05 4.44 and 4.35.)
+// They are tried where a launch in place, under the same tag as the one before it and all rows having a start, finished
+// 40 % of the units at most and left 4.5 % or more without a key that lists would take, which a tenth of the keys do: 0.9^32 =
+// 3.4 % where they are spread evenly, 5 and 7 % were measured at 9.5 and 8.8 % of N(0, I)'s.  (A launch by lists of most
+// keys takes several in place: 30,000 x 28,000 x 96 at eps 0.2 2,800 us for 780.)  Where they hold more after all the
+// next try is 16 launches away, 64 with more than twice that.
+struct ListsState {
+  unsigned known[2], bump[2], base[2], wait[2], taken;  // (taken: a slot a lane)
+  bool lists[2], renewed[2];
+};
+__device__ __forceinline__ ListsState lists_state(const unsigned* st, int lane, const LaunchArgs::Lists& of) {
+  ListsState s;
+  s.taken = lane < 2 * kDmaxSlots ? st[kSelDmax + lane] : 0u;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int r = of.role[i];  // (of one side: its words twice)
+    s.lists[i] = coarse128_lists(st, of.tag[i], r);
+    s.renewed[i] = slack_renewed(st, of.tag[i], r);
+    s.known[i] = st[kSelTag + r];
+    s.bump[i] = st[kSelBump + r];
+    s.base[i] = st[kSelGen + r];
+    s.wait[i] = st[kSelCum + r];
+  }
+  return s;
+}
+// es of us units in place ended at the test.
+__device__ __forceinline__ void lists_after_launch(unsigned* st, int lane, const LaunchArgs::Lists& of, const ListsState& s,
+                                                   unsigned long long es, unsigned long long us) {
+  unsigned taken = s.taken;
+#pragma unroll
+  for (int o = kDmaxSlots / 2; o > 0; o >>= 1) taken += (unsigned)__shfl_xor((int)taken, o, 64);
+  const unsigned of_role[2] = {(unsigned)__shfl((int)taken, 0, 64), (unsigned)__shfl((int)taken, kDmaxSlots, 64)};
+  if (lane < 2 * kDmaxSlots) st[kSelDmax + lane] = 0u;
+  if (lane != 0) return;
+  const bool few = (us - min(es, us)) << 16 < us * kListsFrom;
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+    if (i < of.sides) {
+      const int r = of.role[i];
+      const unsigned share = (unsigned)(((unsigned long long)of_role[r] << 16) / of.units[i]);
+      if (!s.lists[i]) {
+        st[kSelMode + r] = s.wait[i] == 0u && s.bump[i] == 0u && s.known[i] == of.tag[i] && few && share >= kListsClear ? 1u : 0u;
+        st[kSelCum + r] = s.wait[i] - (s.wait[i] != 0u ? 1u : 0u);
+        st[kSelHave + r] = 0u;
+      } else if (s.renewed[i]) {
+        st[kSelHave + r] = of.tag[i] != 0u && s.bump[i] == 0u ? 1u : 0u;
+        st[kSelGen + r] = share;
+        if (share > kListsMost) st[kSelMode + r] = 0u, st[kSelCum + r] = share > 2u * kListsMost ? 4u * kListsWait : kListsWait;
+      } else if (share > s.base[i] + kListsGrow) {
+        st[kSelHave + r] = 0u;
+      }
+      st[kSelTag + r] = of.tag[i];
+      st[kSelBump + r] = 0u;
+    }
+}
+
 // What the merge kernel does to the state words after a launch, by one wavefront.  Every word is
 // read before any is written (they live in one buffer, and loads placed behind stores to it would
 // each wait for their own round trip: the chain used to be the longest thing in the kernel).
@@ -337,12 +406,14 @@ __device__ __forceinline__ bool margins_settled(const unsigned* st, int side, fl
 //     of the coarse variant with counts decides, and leaves it when too few of its units ended;
 //     the plain kernel counts the units whose exponentials it left out, and a launch that left
 //     out clearly more than the first of its stretch hands the next one back to the coarse variant
-//     (a launch by lists, which take keys long before they matter, says nothing to that: `lists`);
+//     (a launch by lists, which take keys long before they matter, says nothing to that);
+//   * rows of 65 .. 128 columns: the state of lists, unless the device chose the plain kernel (`chosen`: it chooses.  A
+//     launch that asks for the test runs it whatever the word says, and has written slack under its own tag);
 //   * per side with carried margins (`commit_sides` of them, their matrices' roles in
 //     `role`, base-2 units per raw unit in `lscale`): the launch's largest bias change joins the
 //     running sum (or starts it, after a launch that began a generation), and the form that ran
 //     is remembered for the hysteresis of margins_settled.
-__device__ __forceinline__ void state_after_launch(unsigned* st, int lane, bool lists, int commit_sides,
+__device__ __forceinline__ void state_after_launch(unsigned* st, int lane, bool chosen, const LaunchArgs::Lists& of, int commit_sides,
                                                    const int (&role)[2], const float (&lscale)[2]) {
   // ---- loads ----
   const unsigned e = st[kSelEnded + lane], u = st[kSelUnits + lane], k = st[kSelSkip + lane];
@@ -360,6 +431,8 @@ __device__ __forceinline__ void state_after_launch(unsigned* st, int lane, bool 
       cum[i] = st[kSelCum + role[i]];
       have[i] = st[kSelHave + role[i]];
     }
+  ListsState ls;
+  if (of.sides > 0) ls = lists_state(st, lane, of);
   // (lanes 0..31: the slots of both roles)
   unsigned dslot = lane < 2 * kDmaxSlots ? st[kSelDmax + lane] : 0u;
   // ---- the decision ----
@@ -384,7 +457,8 @@ __device__ __forceinline__ void state_after_launch(unsigned* st, int lane, bool 
   for (int i = 0; i < 2; ++i)
     if (i < commit_sides && lane >= role[i] * kDmaxSlots && lane < (role[i] + 1) * kDmaxSlots)
       st[kSelDmax + lane] = 0u;
-  const unsigned long long listed = lists ? ks : 0ull;
+  const unsigned long long listed = of.sides > 0 ? ks : 0ull;
+  if (of.sides > 0 && us + ks > 0 && !(chosen && word != 0u)) lists_after_launch(st, lane, of, ls, es, us);
   if (lane == 0 && us + listed > 0) {
     unsigned long long* out = reinterpret_cast<unsigned long long*>(st + kSelCumEnded);
     out[0] = c0 + es + listed;
@@ -432,73 +506,6 @@ __device__ __forceinline__ void state_after_launch(unsigned* st, int lane, bool 
         st[kSelBump + role[i]] = 0u;
       }
   }
-}
-
-// Rows of 65 .. 128 columns: does a side's launch go by lists (lse_coarse128_kernel, lse_listed128_kernel)?  Under another
-// tag than the launch before it goes on in place.
-__device__ __forceinline__ bool coarse128_lists(const unsigned* st, unsigned tag, int role) {
-  return st != nullptr && st[kSelMode + role] != 0u && st[kSelTag + role] == tag;
-}
-// ... and are all units of it tested (or is the slack of an earlier launch good)?
-__device__ __forceinline__ bool slack_renewed(const unsigned* st, unsigned tag, int role) {
-  return st == nullptr || tag == 0u || st[kSelHave + role] == 0u || st[kSelTag + role] != tag;
-}
-// One wavefront, in front of state_after_launch.  At 20,000 x 30,000 a launch in place takes 210 us and 0.5 for every
-// thousand units of 586 that go on; one by lists 25 us and 1.4 for every thousand times 32 keys of a row block's
-// list, and 150 to 200 more with the test.  Lists are kept while they hold 10 % of the keys; a test is good
-// until they have grown by a further 2 % of the keys.  (1 % 3.97 ms, 2 % 4.0 for ten iterations there, at
-// eps 0.05 4.44 and 4.35.)
-// They are tried where a launch in place, under the same tag as the one before it and all rows having a start, finished
-// 40 % of the units at most and left 4.5 % or more without a key that lists would take, which a tenth of the keys do: 0.9^32 =
-// 3.4 % where they are spread evenly, 5 and 7 % were measured at 9.5 and 8.8 % of N(0, I)'s.  (A launch by lists of most
-// keys takes several in place: 30,000 x 28,000 x 96 at eps 0.2 2,800 us for 780.)  Where they hold more after all the
-// next try is 16 launches away, 64 with more than twice that.
-// `chosen`: the device chose the variant, and the plain one ran where the word is set.  (A launch that asks for the test
-// runs it whatever the word says, and has written slack under its own tag.)
-__device__ __forceinline__ void slack_after_launch(unsigned* st, int lane, bool chosen, const LaunchArgs::Lists& of) {
-  const unsigned e = st[kSelEnded + lane], u = st[kSelUnits + lane], k = st[kSelSkip + lane], word = st[kSelWord];
-  unsigned taken = lane < 2 * kDmaxSlots ? st[kSelDmax + lane] : 0u;
-  unsigned known[2] = {0u, 0u}, bump[2] = {0u, 0u}, base[2] = {0u, 0u}, wait[2] = {0u, 0u};
-  bool lists[2] = {false, false}, renewed[2] = {false, false};
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-    if (i < of.sides) {
-      lists[i] = coarse128_lists(st, of.tag[i], of.role[i]);
-      renewed[i] = slack_renewed(st, of.tag[i], of.role[i]);
-      known[i] = st[kSelTag + of.role[i]];
-      bump[i] = st[kSelBump + of.role[i]];
-      base[i] = st[kSelGen + of.role[i]];
-      wait[i] = st[kSelCum + of.role[i]];
-    }
-  unsigned long long es = e, us = u, ks = k;
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) es += __shfl_xor(es, o, 64), us += __shfl_xor(us, o, 64), ks += __shfl_xor(ks, o, 64);
-#pragma unroll
-  for (int o = kDmaxSlots / 2; o > 0; o >>= 1) taken += (unsigned)__shfl_xor((int)taken, o, 64);
-  const unsigned of_role[2] = {(unsigned)__shfl((int)taken, 0, 64), (unsigned)__shfl((int)taken, kDmaxSlots, 64)};
-  if ((chosen && word != 0u) || us + ks == 0) return;
-  if (lane < 2 * kDmaxSlots) st[kSelDmax + lane] = 0u;
-  if (lane != 0) return;
-  const bool few = (us - min(es, us)) << 16 < us * kListsFrom;  // (of the sides in place)
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-    if (i < of.sides) {
-      const int r = of.role[i];
-      const unsigned share = (unsigned)(((unsigned long long)of_role[r] << 16) / of.units[i]);
-      if (!lists[i]) {
-        st[kSelMode + r] = wait[i] == 0u && bump[i] == 0u && known[i] == of.tag[i] && few && share >= kListsClear ? 1u : 0u;
-        st[kSelCum + r] = wait[i] - (wait[i] != 0u ? 1u : 0u);
-        st[kSelHave + r] = 0u;
-      } else if (renewed[i]) {
-        st[kSelHave + r] = of.tag[i] != 0u && bump[i] == 0u ? 1u : 0u;
-        st[kSelGen + r] = share;
-        if (share > kListsMost) st[kSelMode + r] = 0u, st[kSelCum + r] = share > 2u * kListsMost ? 4u * kListsWait : kListsWait;
-      } else if (share > base[i] + kListsGrow) {
-        st[kSelHave + r] = 0u;
-      }
-      st[kSelTag + r] = of.tag[i];
-      st[kSelBump + r] = 0u;
-    }
 }
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }

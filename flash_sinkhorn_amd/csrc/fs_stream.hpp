@@ -501,8 +501,7 @@ __global__ __launch_bounds__(finish_threads(HAS_O)) void finish_kernel(const Lau
           role[i] = ms.ps_q;
           ls[i] = ms.qscale / (ms.plane_scale[ms.ps_q] * ms.plane_scale[ms.ps_k]);
         }
-      if (args.lists.sides > 0) slack_after_launch(args.sel, threadIdx.x, args.sel_pred != 0, args.lists);
-      state_after_launch(args.sel, threadIdx.x, args.lists.sides > 0, commit_sides, role, ls);
+      state_after_launch(args.sel, threadIdx.x, args.sel_pred != 0, args.lists, commit_sides, role, ls);
     }
   }
   if constexpr (!HAS_O) {
@@ -748,8 +747,7 @@ template <int T>
 __global__ __launch_bounds__(64) void coarse_decide_kernel(const LaunchArgs args) {
   const int role[2] = {0, 0};
   const float ls[2] = {0.f, 0.f};
-  if (args.lists.sides > 0) slack_after_launch(args.sel, threadIdx.x, args.sel_pred != 0, args.lists);
-  state_after_launch(args.sel, threadIdx.x, args.lists.sides > 0, 0, role, ls);
+  state_after_launch(args.sel, threadIdx.x, args.sel_pred != 0, args.lists, 0, role, ls);
 }
 
 // kArgmax: merge the partial (largest value, key) pairs of the key splits; equal values keep
