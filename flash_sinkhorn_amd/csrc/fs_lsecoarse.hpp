@@ -58,9 +58,9 @@ namespace fs {
 
 // What lse_coarse_kernel needs of the key bias, once per launch instead of once per workgroup:
 // one wavefront per 64-key tile writes the tile's record (layout: kAux* in fs_common.hpp) in raw
-// units: a_j as eight fp16 copies, b_j - 2^18 a_j (for rows of more than 64 columns b_j itself,
-// which is all that lse_coarse128_kernel reads), and the largest bias of each 32-key sub-tile.  Keys past the end of the key set get a bias that masks them.  T only makes this a
-// template (header-defined kernel).
+// units: a_j as eight fp16 copies, b_j - 2^18 a_j (for rows of more than 64 columns only b_j itself), and the
+// largest bias of each 32-key sub-tile.  Keys past the end of the key set get a bias that masks them.  T only makes
+// this a template (header-defined kernel).
 //
 // The wavefronts behind the tiles (kSeedRows query rows each, side 0 first: seed_blocks0 of them) compute
 // where the rows' running maxima start.  A row whose largest logit of the last launch sat at key
@@ -226,7 +226,7 @@ __global__ __launch_bounds__(64 * kBiasWaves) void coarse_bias_kernel(const Laun
   }
   const float mx_sub = __shfl(mx, (lane & 1) * 32, 64);  // lanes 0 and 1: the two sub-tiles' maxima
   if (in) {
-    *reinterpret_cast<u32x4*>(rec + kAuxA + lane * 4) = u32x4{aw, aw, aw, aw};
+    if (dp <= 64) *reinterpret_cast<u32x4*>(rec + kAuxA + lane * 4) = u32x4{aw, aw, aw, aw};
     rec[kAuxB + lane] = __builtin_bit_cast(unsigned, dp > 64 ? b : b - (float)ah * 0x1p18f);
     rec[kAuxMax + lane] = lane < 2 ? __builtin_bit_cast(unsigned, mx_sub)
                                    : lane < 4 ? __builtin_bit_cast(unsigned, lane == 2 ? most_hi : most_lo)

@@ -356,9 +356,6 @@ __device__ __forceinline__ void coarse128_in_place(const LaunchArgs& args, const
     asm volatile("ds_read_b32 %0, %1" : "=v"(v) : "v"(lds_addr(p)) : "memory");
     return v;
   };
-  auto ds_write4 = [&](float* p, float v) {
-    asm volatile("ds_write_b32 %0, %1" : : "v"(lds_addr(p)), "v"(v) : "memory");
-  };
   auto fence = [&]() { __builtin_amdgcn_sched_barrier(0); };
   auto wait_lds = [&]() {  // lgkmcnt(0), and nothing moves across
     fence();
@@ -639,8 +636,8 @@ __global__ __launch_bounds__(256, 2) void lse_coarse128_kernel(const LaunchArgs 
 // A workgroup takes 32 query rows, each of its wavefronts a quarter of the keys.  First the keys on the list; what
 // they make of the rows' maxima tells by how much the rows' lines have fallen at most (the key that a
 // row's maximum was held by may have lost its lead to another on the list), and which units' slack that uses up:
-// their other keys follow.  Bound by the chain of loads in front of the first logits and behind it, so three
-// wavefronts per SIMD and three quarters of a unit each in flight.
+// their other keys follow.  Bound by the chain of loads in front of the first logits and behind it, so each wavefront has three
+// quarters of a unit in flight.
 //
 // A row block whose lines have fallen by more than most of its units' slack (one row of the 32 will do) is left to a
 // second launch, REST, which shares its units out over up to 16 workgroups: alone, it took 250 us.
