@@ -252,6 +252,7 @@ struct PlaneSet {
   const float* src[2];
   int rows[2];
   size_t off[2];
+  size_t rows_at[2];  // the arrays of one value per row, by role
   size_t aux_off, end;
   size_t margin_off, margin_slot;  // two slots of carried margins behind the aux block (0: none)
   size_t queue_off;                // behind them: the work queues of lse_sparse_kernel
@@ -355,6 +356,13 @@ int make_plane_set(const float* const* ptrs, const int* rows, int count, const L
   }
   ps.aux_off = need;
   ps.end = need + kPlaneAuxBytes;
+  // What launches carry goes with the role of a matrix as the stationary one.  A matrix on its own has both roles in a
+  // two-sided launch, whose sides differ in all but the matrix, and a second set of the arrays behind the aux block.
+  for (int i = 0; i < ps.n; ++i) ps.rows_at[i] = ps.off[i] + planes_only_bytes(ps.rows[i], c);
+  if (ps.n == 1 && !c.gemm) {
+    ps.rows_at[1] = ps.end;
+    ps.end += 4 * row_array_bytes(ps.rows[0]);
+  }
   int64_t max_rows = 0;
   for (int i = 0; i < ps.n; ++i) max_rows = std::max<int64_t>(max_rows, ps.rows[i]);
   ps.margin_off = ps.end;
@@ -384,6 +392,11 @@ const unsigned* plane_of(const PlaneSet& ps, void* ws, const float* src, int row
     if (ps.src[i] == src && ps.rows[i] == rows)
       return reinterpret_cast<const unsigned*>(static_cast<char*>(ws) + ps.off[i]);
   return nullptr;
+}
+
+// Of a role: 0: best keys, 1: last maxima, 2: last biases, 3: this launch's starting values.
+float* carried_row_array(const PlaneSet& ps, void* ws, int role, int which) {
+  return reinterpret_cast<float*>(static_cast<char*>(ws) + ps.rows_at[role] + which * row_array_bytes(ps.rows[ps.n == 1 ? 0 : role]));
 }
 
 int* best_keys_of(const PlaneSet& ps, const LseConfig& c, void* ws, const float* src, int rows) {
@@ -430,7 +443,8 @@ int launch_plane_set(const PlaneSet& ps, const LseConfig& c, int64_t d, void* ws
       s.m[i] = {ps.src[i], reinterpret_cast<unsigned*>(base + ps.off[i]), ps.rows[i], partial + 256 * i,
                 scales + i, two ? nullptr : scales + 1, i == 0 ? select_state(ps, ws) : nullptr,
                 best_keys_of(ps, c, ws, ps.src[i], ps.rows[i]),
-                keep ? tiled_of(ps, c, ws, ps.src[i], ps.rows[i]) : nullptr};
+                keep ? tiled_of(ps, c, ws, ps.src[i], ps.rows[i]) : nullptr,
+                two || c.gemm ? nullptr : reinterpret_cast<int*>(carried_row_array(ps, ws, 1, 0))};
     if (rc == FS_OK) rc = launch_split_planes_f16(s, st);
   }
   return rc;
@@ -1153,31 +1167,29 @@ int run_stream(int mode, bool sepv, Side* sides, int nsides, int64_t d, void* ws
       sd.qplanes = plane_of(ps, ws, sd.q, sd.nq);
       sd.kplanes = plane_of(ps, ws, sd.k, sd.nk);
       sd.plane_scale = plane_scales(ps, ws);
-      sd.ps_q = plane_index(ps, sd.q, sd.nq);
-      sd.ps_k = plane_index(ps, sd.k, sd.nk);
+      // (of one matrix alone the sides of a two-sided launch have a role each)
+      const bool alone = ps.n == 1 && nsides == 2;
+      sd.ps_q = alone ? s : plane_index(ps, sd.q, sd.nq);
+      sd.ps_k = alone ? s ^ 1 : plane_index(ps, sd.k, sd.nk);
       if (coarse || auto_sel) {
-        sd.best_key = best_keys_of(ps, cfg, ws, sd.q, sd.nq);
-        sd.seed = row_array_of(ps, cfg, ws, sd.q, sd.nq, 3);
+        sd.best_key = reinterpret_cast<int*>(carried_row_array(ps, ws, sd.ps_q, 0));
+        sd.seed = carried_row_array(ps, ws, sd.ps_q, 3);
         sd.key_aux = reinterpret_cast<unsigned*>(static_cast<char*>(ws) + aux_off + (s == 1 ? aux_bytes[0] : 0));
-        if (wide) {
-          // (a slot per matrix that holds query rows; both sides of one matrix: no slack outlives the launch)
-          const bool shared = nsides == 2 && plane_index(ps, sides[0].q, sides[0].nq) == plane_index(ps, sides[1].q, sides[1].nq);
+        if (wide) {  // (a slot per role)
           const int rows = std::max(ps.rows[0], ps.n > 1 ? ps.rows[1] : 0);
-          char* slot = static_cast<char*>(ws) + ps.margin_off + (size_t)(shared ? s : sd.ps_q) * ps.margin_slot;
+          char* slot = static_cast<char*>(ws) + ps.margin_off + (size_t)sd.ps_q * ps.margin_slot;
           sd.slack = (flags & kFlagNoLists) || ps.margin_slot == 0 ? nullptr : reinterpret_cast<unsigned short*>(slot);
           sd.marks = reinterpret_cast<unsigned*>(slot + slack_bytes(rows));
           sd.slack_bias = reinterpret_cast<float*>(slot + 3 * slack_bytes(rows));
           sd.slack_floor = reinterpret_cast<float*>(slot + 3 * slack_bytes(rows) + row_array_bytes(rows));
           sd.slack_rest = reinterpret_cast<int*>(slot + 3 * slack_bytes(rows) + 2 * row_array_bytes(rows));
           sd.slack_stride = slack_stride_for(rows);
-          a.tag[s] = shared ? 0u : tag_of(sd, p);
+          a.tag[s] = tag_of(sd, p);
           if (sd.slack != nullptr) {
             a.lists.sides = nsides;
             a.lists.role[s] = sd.ps_q;
             a.lists.tag[s] = a.tag[s];
-            // (both sides of one matrix count into the same words)
-            for (int t = 0; t < nsides; ++t)
-              if (t == s || shared) a.lists.units[s] += (unsigned)ceil_div(sides[t].nq, 32) * (unsigned)ceil_div(sides[t].nk, 128) * 4u;
+            a.lists.units[s] = (unsigned)ceil_div(sd.nq, 32) * (unsigned)ceil_div(sd.nk, 128) * 4u;
           }
         }
         sd.qnorms = wide ? row_array_of(ps, cfg, ws, sd.q, sd.nq, 4) : nullptr;
@@ -1192,8 +1204,8 @@ int run_stream(int mode, bool sepv, Side* sides, int nsides, int64_t d, void* ws
         sd.qtiled = tiled_of(ps, cfg, ws, sd.q, sd.nq);
         sd.npieces = reinterpret_cast<unsigned char*>(static_cast<char*>(ws) + ps.queue_off + kQueueBytes) +
                      (size_t)s * npieces_bytes(std::max(ps.rows[0], ps.n > 1 ? ps.rows[1] : 0));
-        sd.m_prev = row_array_of(ps, cfg, ws, sd.q, sd.nq, 1);
-        sd.bias_prev = row_array_of(ps, cfg, ws, sd.k, sd.nk, 2);
+        sd.m_prev = carried_row_array(ps, ws, sd.ps_q, 1);
+        sd.bias_prev = carried_row_array(ps, ws, sd.ps_k, 2);
         a.tag[s] = tag_of(sd, p);
       }
     }

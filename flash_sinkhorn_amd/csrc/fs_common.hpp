@@ -193,7 +193,7 @@ struct LaunchArgs {
     int sides;
     int role[2];      // Side::ps_q
     unsigned tag[2];
-    unsigned units[2];  // 32 x 32 units of the sides of that role, in whole pieces of 128 keys
+    unsigned units[2];  // 32 x 32 units of the side, in whole pieces of 128 keys
   } lists;
 };
 
@@ -337,7 +337,7 @@ __device__ __forceinline__ bool coarse128_lists(const unsigned* st, unsigned tag
 }
 // ... and are all units of it tested (or is the slack of an earlier launch good)?
 __device__ __forceinline__ bool slack_renewed(const unsigned* st, unsigned tag, int role) {
-  return st == nullptr || tag == 0u || st[kSelHave + role] == 0u || st[kSelTag + role] != tag;
+  return st == nullptr || st[kSelHave + role] == 0u || st[kSelTag + role] != tag;
 }
 // The state of lists, read and brought up to date by state_after_launch.  At 20,000 x 30,000 a launch in place takes 210 us and 0.5 for every
 // thousand units of 586 that go on; one by lists 25 us and 1.4 for every thousand times 32 keys of a row block's
@@ -388,7 +388,7 @@ __device__ __forceinline__ void lists_after_launch(unsigned* st, int lane, const
         st[kSelCum + r] = s.wait[i] - (s.wait[i] != 0u ? 1u : 0u);
         st[kSelHave + r] = 0u;
       } else if (s.renewed[i]) {
-        st[kSelHave + r] = of.tag[i] != 0u && s.bump[i] == 0u ? 1u : 0u;
+        st[kSelHave + r] = s.bump[i] == 0u ? 1u : 0u;
         st[kSelGen + r] = share;
         if (share > kListsMost) st[kSelMode + r] = 0u, st[kSelCum + r] = share > 2u * kListsMost ? 4u * kListsWait : kListsWait;
       } else if (share > s.base[i] + kListsGrow) {

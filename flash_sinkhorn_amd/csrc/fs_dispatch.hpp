@@ -13,7 +13,7 @@ int launch_sliced(int mode, const LaunchArgs& a, int nw, int nsl, int blocks, hi
 // fp16 planes: absmax over the (at most two) operand matrices -> partial[2][256]; then the split of
 // all of them (one launch: 5 us less per operation than one each), which also writes a matrix's
 // power-of-two scale to *scale_out and clears the variant-choice state at clear_state (kSelWords
-// words; may be null) and resets best_keys (one int per row; may be null) to -1.
+// words; may be null) and resets best_keys and best_keys2 (one int per row; may be null) to -1.
 // n 32-bit words at p (16-byte aligned) set to zero by a kernel (graph-capture safe).
 int launch_fill_zero(unsigned* p, long long n, hipStream_t st);
 int launch_absmax(const float* a, long long na, const float* b, long long nb, float* partial,
@@ -31,6 +31,7 @@ struct SplitMatrix {
   unsigned* clear_state;   // or null
   int* best_keys;          // or null
   unsigned* tiled;         // or null
+  int* best_keys2;         // or null: a second set of the arrays at best_keys
 };
 struct SplitArgs {
   SplitMatrix m[2];

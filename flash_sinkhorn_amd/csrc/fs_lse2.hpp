@@ -96,7 +96,8 @@ __global__ __launch_bounds__(256) void absmax_kernel(const float* __restrict__ a
 // the kSelWords words at `clear_state` (the variant-choice state that belongs to the planes);
 // `best_keys` (may be null) starts three arrays of one value per row, (rows + 3) & ~3 values apart:
 // the keys (reset to -1), the rows' last maxima (3e38) and the rows' last biases as keys (0); two more
-// behind a fourth hold the norms of the planes of 128-column rows (Side::qnorms).
+// behind a fourth hold the norms of the planes of 128-column rows (Side::qnorms).  `best_keys2` (may be null): the first
+// three a second time, for the second side of a problem of the matrix with itself.
 // With `chunked` the two planes are interleaved per 32 columns (layout of lse_gemm_kernel).
 // `tiled` (may be null; not with `chunked`): a second copy in MFMA operand order, see Side::ktiled.
 __global__ __launch_bounds__(256) void fill_zero_kernel(unsigned* __restrict__ p, long long n) {
@@ -140,11 +141,16 @@ __global__ __launch_bounds__(256) void split_planes_f16_kernel(const SplitArgs a
 
   const int per_row = dp / 4;
   const long long idx = (long long)blockIdx.x * 256 + threadIdx.x;
-  if (best_keys != nullptr && idx < rows) {  // new planes: the three per-row arrays behind them
+  if (idx < rows) {  // new planes: the three per-row arrays behind them
     const int stride = (rows + 3) & ~3;
-    best_keys[idx] = -1;                                                  // no key known yet
-    reinterpret_cast<float*>(best_keys)[stride + idx] = 3.0e38f;          // no maximum known yet
-    reinterpret_cast<float*>(best_keys)[2 * stride + idx] = 0.f;          // no bias seen yet
+#pragma unroll
+    for (int set = 0; set < 2; ++set) {
+      int* keys = set ? mat.best_keys2 : best_keys;
+      if (keys == nullptr) continue;
+      keys[idx] = -1;                                                  // no key known yet
+      reinterpret_cast<float*>(keys)[stride + idx] = 3.0e38f;          // no maximum known yet
+      reinterpret_cast<float*>(keys)[2 * stride + idx] = 0.f;          // no bias seen yet
+    }
   }
   if (idx >= (long long)(rows + kPlanePadRows) * per_row) return;
   const int r = (int)(idx / per_row);

@@ -1233,7 +1233,7 @@ def test_lists_are_kept_up_to_a_tenth_of_the_keys(n, m):
         prep = _lib.PreparedOperands(x, y, _lib.flags(True, False), self_pair=True)
         _self_pair_steps_raw(x, y, f, -(y * y).sum(1), la, lb, [(1.0, 1.0, 0.5, 1.0, 1.0)] * 8, prepared=prep, **kw)
     words = prep.ws[prep.state_offset:prep.state_offset + 4 * 146].view(torch.int32).tolist()
-    assert words[144:146] == ([1, 1] if m else [1, 0])  # (kSelMode)
+    assert words[144:146] == [1, 1]  # (kSelMode)
 
 
 def _steps_by_launch(x, y, eps, steps):
@@ -1336,3 +1336,32 @@ def test_a_product_on_prepared_planes_and_lists_share_a_workspace():
                               v.data_ptr(), out.data_ptr(), n, m, d, eps, 2.0, 1, flags, prep.ws.data_ptr(), prep.nbytes,
                               _lib.stream_of(x)) == 0
         assert float((out - want_v).abs().max()) <= tol / eps * float(want_v.max())  # (an error of tol in a potential)
+
+
+@pytest.mark.parametrize("variant", [True, None])
+@pytest.mark.parametrize("d,eps", [(24, 0.02), (96, 0.02)])
+def test_a_cloud_against_itself_under_other_weights(monkeypatch, d, eps, variant):
+    """One cloud passed twice, almost all mass of the second on half of it: two potentials that have nothing in common
+    but the matrix; with the tile test against the plain solve, and against the fp64 oracle."""
+    import flash_sinkhorn_amd.sinkhorn_solvers as solvers
+    rng = np.random.default_rng(71)
+    n = 2500
+    x, _ = _clustered(rng, n, d, spread=0.7)
+    a, b = np.full(n, 1.0 / n, np.float32), rng.random(n).astype(np.float32) + 0.1
+    b[: n // 2] *= 1e-3
+    b /= b.sum()
+    X, A, B = dev(x, a, b)
+    kw = dict(use_epsilon_scaling=False, eps=eps, n_iters=25, allow_tf32=False)
+    monkeypatch.setattr(solvers, "_COARSE_MIN_ROWS", 2048)
+    monkeypatch.setattr(solvers, "_COARSE_MIN_ROWS_WIDE", 2048)
+    monkeypatch.setattr(solvers, "COARSE_TEST", variant)
+    info = {}
+    f, g = solvers.sinkhorn_flashstyle_symmetric(X, X, A, B, solve_info=info, **kw)
+    assert info["prepared"].variant_state()["tiles_tested"] > 0
+    monkeypatch.setattr(solvers, "COARSE_TEST", False)
+    wf, wg = solvers.sinkhorn_flashstyle_symmetric(X, X, A, B, solve_info=info, **kw)
+    scale = float((X * X).sum(dim=1).max())
+    assert float((f - wf).abs().max()) < 2e-6 * scale and float((g - wg).abs().max()) < 2e-6 * scale
+    wf, wg = oracle.sinkhorn_symmetric(x, x, a, b, eps=eps, n_iters=25, use_epsilon_scaling=False)[:2]
+    assert float((f.cpu().double() - torch.from_numpy(wf)).abs().max()) < 4e-6 * scale
+    assert float((g.cpu().double() - torch.from_numpy(wg)).abs().max()) < 4e-6 * scale
