@@ -102,6 +102,9 @@ Family family_for(int64_t d) {
 // 40,000 x 128 230 and 211, of 20,000 x 15,013 x 32 117 and 112, of 25,000 x 30,000 x 100 579 and 578.  Kernels of
 // narrow rows have three and four workgroups a CU, but rounds of 768 or 1,024 predict their times worse: over
 // products of 1,200 to 48,000 rows this rule is 1.2 % above the best of 20 splits, doubling 7.5 %.
+// Ranges are up to five times as long as doubling made them (512 -> 2,560 keys at 20,000 x 15,013 x 32), and a range's
+// sum is one fp32 accumulator per lane: mean errors against fp64 over the rows of ten shapes from 1,200 x 30,000 x 128 to 48,000 x 48,000 x
+// 8, six seeds each, lie between 0.5 % below and 0.4 % above doubling's (1.27e-6 there, 4.7e-7 at 48,000).
 // (Products with a matrix stay with doubling: a range is summed in one fp32 accumulator, and where ranges got longer
 // by this rule results were 6 % further from fp64; with shorter ones only, gradients of peaked plans 2 % slower.)
 SidePlan plan_rounds(SidePlan p, int64_t nq, int64_t nk, int cap) {

@@ -348,6 +348,31 @@ def test_products_over_uneven_key_ranges(n, m, d):
     assert np.abs(c.cpu().numpy()[rows] - wc).max() <= 1e-5 * max(np.abs(wc).max(), 1.0)
 
 
+@pytest.mark.parametrize("n,m,d,eps", [(20000, 15013, 32, 2.0), (20000, 15013, 32, 0.05), (5000, 40000, 128, 0.2),
+                                       (48000, 48000, 8, 0.2)])
+def test_vector_products_keep_fp32_accuracy_over_long_key_ranges(n, m, d, eps):
+    """Key ranges of a thousand and more keys, summed in one fp32 accumulator per lane and row: the mean error over
+    sampled rows against fp64.  A probability is off by its logit's error: two planes hold 22 bits of each coordinate, so
+    2^-22 of 2 |x| |y| / eps at the most and about an eighth of it in the mean, its sum with the bias is rounded
+    to fp32 three times, and the log weights, of log n and log m, once each, which costs a quarter of a last place
+    (2^-25 of the value at the most) in the mean; a lane adds 16 probabilities a step in a tree and one to its sum, which over s
+    steps of equal size costs about sqrt(s) / 4 units in the mean, and the exponential one."""
+    from flash_sinkhorn_amd.kernels import apply_plan_vec_flashstyle
+    gen = torch.Generator(device="cuda").manual_seed(n + d)
+    x, y = (torch.randn(k, d, device="cuda", generator=gen) / d ** 0.5 for k in (n, m))
+    la, lb = (torch.full((k,), -float(np.log(k)), device="cuda") for k in (n, m))
+    f, g, v = -(x * x).sum(1), -(y * y).sum(1), torch.rand(m, device="cuda", generator=gen)
+    got = apply_plan_vec_flashstyle(x, y, f, g, la, lb, v, eps=eps, axis=1)
+    rows = torch.arange(0, n, max(1, n // 1000), device="cuda")
+    plan = (2.0 * x[rows].double() @ y.double().T + f[rows, None].double() + g.double()) / eps
+    want = torch.exp(plan + la[rows, None].double() + lb.double()) @ v.double()
+    unit, logit = 2.0 ** -24, 2.0 * float((x * x).sum(1).max() * (y * y).sum(1).max()) ** 0.5 / eps
+    bound = (logit * 2.0 ** -22 / 8 + 1.5 * unit * logit + unit / 2 * (np.log(n) + np.log(m)) +
+             unit * (2560 / 64) ** 0.5 / 4 + unit)
+    error = float(((got[rows].double() - want) / want).abs().mean())
+    assert error <= bound
+
+
 @pytest.mark.parametrize("n,m,d,eps", [(40000, 200000, 4, 0.5), (30000, 120000, 16, 0.05)])
 def test_long_key_chunks_keep_fp32_accuracy(n, m, d, eps):
     """Hundreds of key tiles per workgroup: whatever is applied once per tile (the rescale of
