@@ -93,6 +93,17 @@ def test_products_of_rows_of_65_to_128_columns_need_no_room_for_lists(op):
     assert 0 < need[1] <= 2.01 * need[0]
 
 
+@pytest.mark.parametrize("d", [10, 40, 70, 128])
+@pytest.mark.parametrize("n,m", [(1, 1), (4, 8), (100, 31), (11_000, 10_500), (12_000, 12_000), (30_011, 29_989)])
+def test_counters_of_launches_have_cache_lines_of_their_own(n, m, d):
+    """The first eight words of the choice's state are read by every workgroup, those behind are added to: the line ends between."""
+    L, x = _lib.lib(), 0x7F0000000000
+    y = x + 4 * n * d
+    at = L.fs_variant_state_offset(x, y, n, m, d, 0)
+    assert at > 0 and (at + 4 * 8) % 128 == 0
+    assert at + 4 * (_lib._SEL_REDONE + 1) <= L.fs_workspace_bytes(_lib.OP_SYMMETRIC_STEP, n, m, d)
+
+
 def test_workspace_of_a_batch_follows_the_size_of_its_items():
     from flash_sinkhorn_amd import _small
 
