@@ -9,7 +9,9 @@
 // workgroup's other wavefronts at the next barrier: with a tenth of the units going on the matrix pipe is
 // busy 38 % of the time.  This form runs where rows have no start yet, or much goes on.
 //
-// By lists, in two or three launches.  On a peaked plan nearly every unit that goes on does so for one logit
+// By lists, in three launches, which are enqueued in every call that may go by them: the test (a launch that comes back at
+// once where no unit is tested again), the keys on the lists, and what is left over of them (mostly nothing); in place
+// the latter two find nothing to do, 9 us.  On a peaked plan nearly every unit that goes on does so for one logit
 // (20,000 x 30,000 x 128, eps 0.0025: 1.04 a unit, 37,000 units of 586,000), and which ones these are
 // hardly changes from one half-update to the next.  coarse128_test is nothing but the hi*hi products
 // and their test, and leaves per unit which keys any of its 32 rows needs (Side::marks) and by how much all other logits
@@ -18,10 +20,11 @@
 // biases and maxima have moved by since, the test is not run at all (slack_renewed); units where it
 // does not are taken whole, or but for one key where that one alone has risen.
 //
-// A half-update of the 20,000 x 30,000 x 128 problem, launches around it included: 270 us in place; 240 - 285 by lists with
-// their test (180 - 205 of it, 150 without marking), 80 - 150 without, of which 30 are launches that find nothing
-// to do and the merge.  Ten iterations 6.0 -> 3.9 ms; 40 symmetric steps of 30,000 x 28,000 x 128 in eight clusters at
-// eps 0.01 32 -> 13 ms; 100 of three problems of 10,000 x 128 23.8 -> 11.4 ms.
+// A half-update of the 20,000 x 30,000 x 128 problem, launches around it included: 290 - 310 us in place; 235 - 255 by lists
+// with their test (185 - 195 of it), 60 - 140 without, of which 30 are launches that find nothing
+// to do and the merge.  Ten iterations 5.9 -> 3.9 ms; 40 symmetric steps of 30,000 x 28,000 x 128 in eight clusters at
+// eps 0.01 32 -> 13 ms; 100 of three problems of 10,000 x 128 23.8 -> 11.4 ms.  Where no lists pay the two launches
+// are lost: flat plans of 12,000 - 16,000 rows take 2 - 3 % longer than without (16,000 x 12,000 x 100, eps 0.5: 3.32 -> 3.40 ms).
 //
 // What a row's logits are tested against is a lower bound of its maximum: its logit at the key that
 // held its maximum in the launch before (Side::seed, computed by coarse_bias_kernel's seed blocks from
@@ -57,6 +60,9 @@ __device__ __forceinline__ float half_min(float v) {
   return __builtin_bit_cast(float, x);
 }
 // Keys that come this close to the line, in base-2 units, are taken as well, so that what is left out stays so for a while.
+// More of it makes fewer tests and longer lists.  64, 256, 512 and 1,024 units, ms: ten alternating iterations of 20,000 x
+// 30,000 x 128 at eps 0.0025 4.0, 4.0, 3.6, 3.4, at 0.05 3.4, 3.2, 3.5, 5.9; twenty of 12,000 x 14,000 x 80 at 0.01 2.9, 2.5, 2.5, 2.7; 40
+// symmetric steps of 30,000 x 28,000 x 96 at 0.05 11.3, 9.9, 14.4, 29.9, of x 128 in clusters at 0.01 12.4, 13.1, 12.5, 10.9.
 constexpr float kTakeReserve = 256.f;
 // fp16, rounded towards zero
 __device__ __forceinline__ unsigned pack_down(float v) {
@@ -641,6 +647,8 @@ __global__ __launch_bounds__(256, 2) void lse_coarse128_kernel(const LaunchArgs 
 //
 // A row block whose lines have fallen by more than most of its units' slack (one row of the 32 will do) is left to a
 // second launch, REST, which shares its units out over up to 16 workgroups: alone, it took 250 us.
+// (Left to it from more than this many keys on: 256, 1,024, 4,096 and never take 4.65, 4.0, 4.25 and 4.3 ms for the ten iterations
+// at 20,000 x 30,000 x 128, 11.8, 13.1, 13.5 and 14.2 for 40 steps in clusters; at larger eps and of fewer columns all are within 3 %.)
 constexpr int kRestKeys = 1024;  // (as many are a workgroup's own)
 template <bool REST>
 __global__ __launch_bounds__(256, 2) void lse_listed128_kernel(const LaunchArgs args) {

@@ -36,9 +36,9 @@ COARSE_TEST = {"1": True, "0": False}.get(os.environ.get("FLASH_SINKHORN_COARSE_
 _COARSE_MIN_ROWS = 24000
 _COARSE_MIN_STEPS = 8
 # rows of 65 .. 128 columns (twice the matrix work per tile to save): from fewer rows on (20 alternating
-# iterations at d = 128, eps = 0.01, units that go on finished in place: 8192 rows per cloud 3.5 -> 3.8 ms,
-# 12,000 rows 6.1 -> 5.1, 16,000 x 100 columns 9.3 -> 6.6, 30,000 rows 28.6 -> 16.1; on a flat plan, eps = 0.5 at
-# 16,000 rows, the device's way back to the plain kernel costs 9.7 -> 11.1)
+# iterations at d = 128, plain kernel -> left to the device: eps = 0.01 8192 rows per cloud 2.9 -> 1.95 ms,
+# 12,000 rows 5.3 -> 2.3, 16,000 x 100 columns 8.3 -> 2.7, 30,000 rows 27.4 -> 5.1; on a flat plan, eps = 0.5,
+# 8192 rows 2.8 -> 3.7, 12,000 5.3 -> 6.1, 16,000 8.8 -> 9.4, which is why not from fewer on)
 _COARSE_MIN_ROWS_WIDE = 10000
 
 

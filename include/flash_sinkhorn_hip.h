@@ -151,7 +151,8 @@ int fs_prepare_operands(const float* x, const float* y, int64_t n, int64_t m, in
  * (0: coarse tile test, 1: plain), [1] decisions taken so far, [2..3] a 64-bit count of the
  * 32 x 32 logits tiles that ended at the coarse test or were not visited at all (in launches of
  * the plain variant: whose exponentials were left out), [4..5] of all tiles of those launches,
- * [6..7] of the tiles not visited (carried margins, part of [2..3]); [247] non-zero: the next
+ * [6..7] of the tiles not visited (carried margins, part of [2..3]; at 65 to 128 columns those of launches by lists);
+ * [144..145] at 65 to 128 columns, non-zero: half-updates of a matrix's rows go by lists of keys; [247] non-zero: the next
  * two-sided step may take both sides' sums from one sweep; [269] how many such steps the
  * two-sided kernel had to redo so far.
  * Host arithmetic only.  No counterpart in the reference.
