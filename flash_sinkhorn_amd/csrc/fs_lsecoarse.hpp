@@ -174,8 +174,8 @@ __global__ __launch_bounds__(64 * kBiasWaves) void coarse_bias_kernel(const Laun
   const float inv_lscale = 1.0f / lscale;
   float b = 2.0f * kNegBig;
   if (j < sd.nk) {
-    b = sd.kc0 * sd.kb0[j];
-    if (sd.kb1) b += sd.kc1 * sd.kb1[j];
+    // (the first term, the largest, is rounded with the sum only, as in lse2_kernel)
+    b = __builtin_fmaf(sd.kc0, sd.kb0[j], sd.kb1 ? sd.kc1 * sd.kb1[j] : 0.f);
     if (sd.kb2) b += sd.kc2 * sd.kb2[j];
     b = fmaxf(b, kNegBig);
   }

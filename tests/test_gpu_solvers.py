@@ -1365,3 +1365,23 @@ def test_a_cloud_against_itself_under_other_weights(monkeypatch, d, eps, variant
     wf, wg = oracle.sinkhorn_symmetric(x, x, a, b, eps=eps, n_iters=25, use_epsilon_scaling=False)[:2]
     assert float((f.cpu().double() - torch.from_numpy(wf)).abs().max()) < 4e-6 * scale
     assert float((g.cpu().double() - torch.from_numpy(wg)).abs().max()) < 4e-6 * scale
+
+
+@pytest.mark.parametrize("d,eps", [(70, 0.05), (96, 0.05), (128, 0.004), (128, 0.5)])
+def test_the_tile_test_rounds_as_often_as_the_plain_kernel(d, eps):
+    """Errors against fp64 in place (the first two launches) and by lists, over the plain kernel's.  Both round a key's bias
+    in its sum and its scale; rounding its largest term by itself as well makes the errors 1.075 to 1.12 times as large, other
+    orders of the sums 0.995 to 1.013."""
+    from flash_sinkhorn_amd import _lib
+    from flash_sinkhorn_amd.kernels.sinkhorn_flashstyle_sqeuclid import flashsinkhorn_lse_fused
+    ratios = []
+    for seed in range(4):
+        gen = torch.Generator(device="cuda").manual_seed(seed)
+        x, y = (torch.randn(n, d, device="cuda", generator=gen) for n in (3000, 5000))
+        g, lw = -(y * y).sum(1), torch.log(torch.rand(5000, device="cuda", generator=gen) + 0.01)
+        want = -eps * torch.logsumexp((2.0 * x.double() @ y.double().T + g.double()) / eps + lw.double(), 1)
+        prep = _lib.PreparedOperands(x, y, _lib.flags(True, False))
+        plain = flashsinkhorn_lse_fused(x, y, g, lw, eps, allow_tf32=False)
+        ratios.append([float((flashsinkhorn_lse_fused(x, y, g, lw, eps, allow_tf32=False, _prepared=prep, _coarse=True)
+                              - want).norm() / (plain - want).norm()) for _ in range(4)])
+    assert all(sum(of_launch) / 4 < 1.04 for of_launch in zip(*ratios))
