@@ -143,12 +143,13 @@ int dense_prepare(const SmallArgs& a, const DenseArgs& t, hipStream_t st) {
   return dense_gemm(g, a.items, st);
 }
 
-int dense_rows_step(const DenseRowArgs& t, int rows, int sides, int items, hipStream_t st) {
+int dense_rows_step(const DenseRowArgs& t, int rows, bool raw, int sides, int items, hipStream_t st) {
   int most = 0;
   for (int i = 0; i < sides; ++i) most = std::max(most, t.s.side[i].nq);
   const dim3 grid((most + 8 * rows - 1) / (8 * rows), sides, items);
-  if (rows == 1) hipLaunchKernelGGL((dense_rows_kernel<1>), grid, dim3(512), 0, st, t);
-  else hipLaunchKernelGGL((dense_rows_kernel<2>), grid, dim3(512), 0, st, t);
+  auto* kernel = rows == 1 ? (raw ? dense_rows_kernel<1, true> : dense_rows_kernel<1, false>)
+                           : (raw ? dense_rows_kernel<2, true> : dense_rows_kernel<2, false>);
+  hipLaunchKernelGGL(kernel, grid, dim3(512), 0, st, t);
   return hipGetLastError() == hipSuccess ? FS_OK : FS_ERR_LAUNCH_FAILED;
 }
 

@@ -189,7 +189,9 @@ struct DenseGemmArgs {
   int step_words, plane_words;
 };
 
-template <int WR, int WC, int RB, int CB>
+// APART: the cross products of all steps before hi * hi of the first, in a second pass (see dense_gemm_jobs_kernel), a
+// stage of which is the hi planes of two steps (an even number of them).
+template <int WR, int WC, int RB, int CB, bool APART>
 __device__ __forceinline__ void dense_gemm_tile(const DenseGemmArgs& g, int split) {
   constexpr int W = WR * WC, TR = WR * RB, TC = WC * CB, PIECES = 2 * (TR + TC), LOADS = PIECES / W, ST = 4;
   static_assert(PIECES % W == 0, "every wavefront moves the same number of pieces");
@@ -219,11 +221,17 @@ __device__ __forceinline__ void dense_gemm_tile(const DenseGemmArgs& g, int spli
                    : g.b + ((size_t)z * g.b_blocks + gb) * (size_t)g.steps * kDenseStep) +
              ((size_t)k_begin * g.step_words + (p & 1) * g.plane_words + lane);
   }
+  const int total = APART ? steps + steps / 2 : steps;
+  static_assert(LOADS % 2 == 0, "load i of a wavefront is of plane i % 2");
   auto stage = [&](int k, int buf) {
+    k = min(k, total - 1);
+    const bool hi = APART && k >= steps;
+    if (hi) k = 2 * (k - steps);
+    const long long at[2] = {(long long)k * g.step_words, (long long)(k + (hi ? 1 : 0)) * g.step_words - (hi ? g.plane_words : 0)};
 #pragma unroll
     for (int i = 0; i < LOADS; ++i)
       __builtin_amdgcn_global_load_lds(
-          (const __attribute__((address_space(1))) void*)(src[i] + (size_t)min(k, steps - 1) * g.step_words),
+          (const __attribute__((address_space(1))) void*)(src[i] + at[i & 1]),
           (__attribute__((address_space(3))) void*)(&lds[(buf * PIECES + wave * LOADS + i) * 64]), 16, 0, 0);
   };
   const unsigned base = (unsigned)(size_t)(const __attribute__((address_space(3))) u32x4*)&lds[0] + lane * 16;
@@ -240,7 +248,7 @@ __device__ __forceinline__ void dense_gemm_tile(const DenseGemmArgs& g, int spli
   stage(0, 0);
   stage(1, 1);
   stage(2, 2);
-  for (int k = 0; k < steps; ++k) {
+  for (int k = 0; k < total; ++k) {
     __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_waitcnt(0x0F70 | ((2 * LOADS) & 15) | (((2 * LOADS) >> 4) << 14));  // step k has landed
     __builtin_amdgcn_sched_barrier(0);
@@ -257,11 +265,18 @@ __device__ __forceinline__ void dense_gemm_tile(const DenseGemmArgs& g, int spli
       __builtin_amdgcn_sched_barrier(0);
       __builtin_amdgcn_s_waitcnt(0xC07F | ((2 * (CB - 1 - j)) << 8));  // this column block has been read
       __builtin_amdgcn_sched_barrier(0);
+      if (!APART || k < steps) {
 #pragma unroll
-      for (int prod = 0; prod < 3; ++prod)
+        for (int prod = 0; prod < (APART ? 2 : 3); ++prod)
 #pragma unroll
-        for (int i = 0; i < RB; ++i)
-          acc[i][j] = small_mfma(x[i][prod == 0 ? 1 : 0], y[j][prod == 1 ? 1 : 0], acc[i][j]);
+          for (int i = 0; i < RB; ++i)
+            acc[i][j] = small_mfma(x[i][prod == 0 ? 1 : 0], y[j][prod == 1 ? 1 : 0], acc[i][j]);
+      } else {
+#pragma unroll
+        for (int step = 0; step < 2; ++step)
+#pragma unroll
+          for (int i = 0; i < RB; ++i) acc[i][j] = small_mfma(x[i][step], y[j][step], acc[i][j]);
+      }
     });
   }
   __builtin_amdgcn_s_waitcnt(0);
@@ -295,16 +310,20 @@ __device__ __forceinline__ void dense_gemm_tile(const DenseGemmArgs& g, int spli
 
 template <int WR, int WC, int RB, int CB>
 __global__ __launch_bounds__(64 * WR * WC, 2) void dense_gemm_kernel(const DenseGemmArgs g) {
-  dense_gemm_tile<WR, WC, RB, CB>(g, blockIdx.z);
+  dense_gemm_tile<WR, WC, RB, CB, false>(g, blockIdx.z);
 }
 
-// Up to four products of the same depth in one launch.
+// Up to four products of the same depth in one launch, summed in the order of steps on planes: the cross products before
+// hi * hi.  (Added to hi * hi step by step, each is rounded to the last place of a sum 2^11 times as large, and not alike
+// for both sides of a pair: potentials of 1,000 to 2,500 points after 40 steps were 1.1 to 1.6 times as far from fp64, with
+// the logits of dense_rows_kernel in base 2; now they are as far.  The second pass takes 13 us for 11 at 2,048 x 64, 37 for 28 at
+// 3,000 x 2,800 x 100.)
 struct DenseGemmJobs {
   DenseGemmArgs job[4];
 };
 template <int WR, int WC, int RB, int CB>
 __global__ __launch_bounds__(64 * WR * WC, 2) void dense_gemm_jobs_kernel(const DenseGemmJobs g) {
-  dense_gemm_tile<WR, WC, RB, CB>(g.job[blockIdx.z], 0);
+  dense_gemm_tile<WR, WC, RB, CB, true>(g.job[blockIdx.z], 0);
 }
 
 __device__ __forceinline__ void dense_join(float& m, float& s, float m2, float s2) {
@@ -474,7 +493,9 @@ __global__ __launch_bounds__(256) void dense_merge_kernel(const DenseArgs a) {
 // other.  Bound by the launch and the chain of loads in front of the first logit (1,000 points: 4.0 us a
 // step, 7.5 by sweep and merge), so the products' first piece is on its way before the biases of the keys, which
 // the workgroup's eight wavefronts share in LDS; from 2,000 points on by reading 2 x 4 bytes a product (7.3 us,
-// 4.4 TB/s).  Grid (rows of the largest side, sides, items).
+// 4.4 TB/s).  RAW: logits in units of the products, as the steps on planes of the same problems have them (there a row's
+// logit and that of its column, which each hold the other's potential, are rounded alike, and what does not cancel adds
+// up in the slow modes of a peaked plan).  Grid (rows of the largest side, sides, items).
 constexpr int kDenseRowKeys = 4096;  // most keys (their biases in LDS)
 struct DenseRowArgs {
   SmallStepArgs s;        // (the planes are not read)
@@ -482,7 +503,7 @@ struct DenseRowArgs {
   int ld[4];
   float* top;             // [items][nq] the largest logit of a row of side 0 in the extrapolation, or null
 };
-template <int R>
+template <int R, bool RAW>
 __global__ __launch_bounds__(512) void dense_rows_kernel(const DenseRowArgs a) {
   constexpr int P = 4;  // 16-byte words of a row per lane and piece: 1024 keys
   __shared__ __attribute__((aligned(16))) float bias[kDenseRowKeys];
@@ -512,16 +533,17 @@ __global__ __launch_bounds__(512) void dense_rows_kernel(const DenseRowArgs a) {
   const float* kpot = sd.kpot + (size_t)item * nk;
   const float* kl2w = sd.kl2w + (size_t)item * nk;
   const float eps = coef.x, qs = coef.y, kc = coef.w;
+  const float raw = RAW ? coef.z : 1.0f, masked = fmaxf(kNegBig * raw, -3.0e38f);
   for (int j = tid; j < ld; j += 512) {
-    const float b = __builtin_fmaf(kc, kpot[min(j, nk - 1)], kl2w[min(j, nk - 1)]);
-    bias[j] = j < nk ? fmaxf(b, kNegBig) : kNegBig;
+    const float b = __builtin_fmaf(kc, kpot[min(j, nk - 1)], kl2w[min(j, nk - 1)]) * raw;
+    bias[j] = j < nk ? fmaxf(b, masked) : masked;
   }
   __syncthreads();
   if (step > entries + a.s.extrapolate) return;  // (its schedule is shorter)
 
   float m[R], s[R];
 #pragma unroll
-  for (int r = 0; r < R; ++r) m[r] = kNegBig, s[r] = 0.f;
+  for (int r = 0; r < R; ++r) m[r] = RAW ? 0.5f * masked * qs : kNegBig, s[r] = 0.f;
   for (int c0 = 0; c0 < ld; c0 += 256 * P) {
     float4 next[R][P];
     if (c0 + 256 * P < ld) load(next, c0 + 256 * P);
@@ -531,6 +553,17 @@ __global__ __launch_bounds__(512) void dense_rows_kernel(const DenseRowArgs a) {
       const float4 kb = *reinterpret_cast<const float4*>(&bias[c0 + 256 * k + 4 * lane]);
 #pragma unroll
       for (int r = 0; r < R; ++r) {
+        if constexpr (RAW) {
+          const float l0 = v[r][k].x + kb.x, l1 = v[r][k].y + kb.y, l2 = v[r][k].z + kb.z, l3 = v[r][k].w + kb.w;
+          float M = fmaxf(fmaxf(l0, l1), fmaxf(l2, l3)) * qs;
+          asm("" : "+v"(M));  // (rounded once, whatever it is used for)
+          M = fmaxf(M, m[r]);
+          s[r] = s[r] * fast_exp2(m[r] - M) +
+                 ((fast_exp2(__builtin_fmaf(l0, qs, -M)) + fast_exp2(__builtin_fmaf(l1, qs, -M))) +
+                  (fast_exp2(__builtin_fmaf(l2, qs, -M)) + fast_exp2(__builtin_fmaf(l3, qs, -M))));
+          m[r] = M;
+          continue;
+        }
         const float l0 = __builtin_fmaf(v[r][k].x, qs, kb.x), l1 = __builtin_fmaf(v[r][k].y, qs, kb.y);
         const float l2 = __builtin_fmaf(v[r][k].z, qs, kb.z), l3 = __builtin_fmaf(v[r][k].w, qs, kb.w);
         const float M = fmaxf(fmaxf(fmaxf(l0, l1), fmaxf(l2, l3)), m[r]);
@@ -573,6 +606,6 @@ int dense_gemm(DenseGemmArgs& g, int items, hipStream_t st);
 int dense_gemm_jobs(DenseGemmJobs& g, int jobs, int items, hipStream_t st);
 int dense_prepare(const SmallArgs& a, const DenseArgs& t, hipStream_t st);
 int dense_step(const SmallArgs& a, DenseArgs& t, int step, hipStream_t st);
-int dense_rows_step(const DenseRowArgs& t, int rows, int sides, int items, hipStream_t st);
+int dense_rows_step(const DenseRowArgs& t, int rows, bool raw, int sides, int items, hipStream_t st);
 
 }  // namespace fs

@@ -51,13 +51,13 @@ bool use_dense(const fs_small_problem* p) { return p->d > kSmallMaxD; }
 // of small_step_kernel reads the planes of all keys for 32 rows, 2, 4, 8 or 16 bytes a logit by the padded width, from the
 // caches; a kept product is 4.  `read`: the bytes of a step, which have to stay in the L2s (4 MiB each) against the narrower
 // planes.  Potentials after 50 steps at a fixed eps, and after a schedule of 14, planes -> products, us:
-//   d = 64:  256 points 244 -> 193, 74 -> 74; 1,000: 383 -> 236, 106 -> 83; 2,048 (32 MiB): 572 -> 397, 156 -> 126;
+//   d = 64:  256 points 243 -> 196, 91 -> 94; 1,000: 370 -> 238, 131 -> 102; 2,048 (32 MiB): 553 -> 395, 187 -> 152;
 //            2,500 (49 MiB): 657 -> 712, 177 -> 201; with self problems 1,000 (16 MiB): 388 -> 306, 110 -> 101;
 //            1,500 (35 MiB): 477 -> 507, 137 -> 159
-//   d = 128: 256: 327 -> 202, 93 -> 73; 1,000: 585 -> 244, 154 -> 85; 3,000 (70 MiB): 1,192 -> 845, 305 -> 243; 4,000
+//   d = 128: 256: 320 -> 201, 110 -> 96; 1,000: 563 -> 246, 175 -> 104; 3,000 (70 MiB): 1,143 -> 849, 344 -> 290; 4,000
 //            (125 MiB): 1,639 -> 1,447, 413 -> 391 (d = 100: 401 -> 417); with self problems 2,500 (98 MiB): 1,957 -> 1,083
-//   d = 32, fixed eps: 512: 238 -> 200; 1,000 (8 MiB): 302 -> 233; 1,500 (18 MiB): 359 -> 345; its schedules 89 -> 80 to
-//            73 -> 79; d <= 16: 270 -> 230 at 1,000, 0.93 to 1.0 at 256 and 1,500
+//   d = 32, fixed eps: 512: 233 -> 200; 1,000 (8 MiB): 295 -> 236; 1,500 (18 MiB): 359 -> 345; its schedules 85 -> 86 and
+//            102 -> 101; d <= 16: 270 -> 230 at 1,000, 0.93 to 1.0 at 256 and 1,500
 bool use_products(const fs_small_problem* p) {
   if (p->alternating || p->d <= 16 || use_dense(p) || use_pair(p)) return false;
   const double n = (double)p->n, m = (double)p->m;
@@ -459,7 +459,7 @@ int launch_rows(const SmallArgs& a, int step, const float* const* dots, const in
     t.ld[i] = i < sides ? ld[first + i] : 0;
   }
   t.top = top;
-  return dense_rows_step(t, rows, sides, a.items, st);
+  return dense_rows_step(t, rows, top == nullptr, sides, a.items, st);  // (wide rows have `top`)
 }
 
 // Wavefronts that share the keys of 32 rows: sixteen where eight would leave the chip half empty and
