@@ -64,6 +64,10 @@ bool use_products(const fs_small_problem* p) {
   const double ldx = std::ceil(n / 256) * 256, ldy = std::ceil(m / 256) * 256;
   if (std::max(ldx, ldy) > kDenseRowKeys) return false;
   if (p->sched != 1 && p->entries < 8) return false;  // (forming them takes what some six steps gain)
+  // (a schedule by diameter is not replayed, and below this the host, with one launch and one tensor more, is what its
+  // caller waits for: 64 x 64 points at 40, 64 and 100 columns 88 -> 94, 89 -> 93, 91 -> 95 us; debiased 256 x 64 96 -> 92,
+  // 128 x 128 101 -> 95)
+  if (p->sched == 1 && (double)p->items * std::max(n, m) * (p->d <= 64 ? 64 : 128) < 16384.0) return false;
   const double read = 4.0 * (double)p->items *
                       ((p->self_terms < 2 ? n * ldy + m * ldx : 0.) + (p->self_terms ? n * ldx + m * ldy : 0.));
   if (p->d <= 32) return p->sched == 0 && read <= 9.0e6;

@@ -120,6 +120,15 @@ def test_workspace_of_a_batch_follows_the_size_of_its_items():
     assert per_item(32, 32, 3, blur=1e-3, scaling=0.999) < 48 << 10  # the longest table
 
 
+@pytest.mark.parametrize("n,d,items,kept", [(64, 64, 1, False), (255, 40, 1, False), (256, 40, 1, True), (64, 33, 4, True),
+                                            (127, 65, 1, False), (128, 100, 1, True)])
+def test_the_smallest_schedules_keep_no_products(n, d, items, kept):
+    from flash_sinkhorn_amd import _small
+    p = _small.Problem(1, 1, None, None, None, n, n, d, items, 0.1, 0.5, 1.0, 0.0, 0.0, 0.0, 0.0, 0, 0, 0, 0, 1, 0, 0,
+                       1, 1, 0)
+    assert (_lib.lib().fs_small_products_bytes(ctypes.byref(p)) > 0) == kept
+
+
 def test_rows_and_products_beyond_the_limits_are_refused_by_whole_solves_too(monkeypatch):
     from flash_sinkhorn_amd import _small, hvp
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
