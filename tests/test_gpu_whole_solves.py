@@ -151,6 +151,17 @@ def test_steps_on_products_are_as_exact_as_those_on_planes(monkeypatch, n, m, d,
     assert np.log(np.array(errors[0]) / errors[1]).mean() < 0.03
 
 
+@pytest.mark.parametrize("n,m,d,far", [(1, 300, 33, 1e4), (300, 1, 70, 1e5), (1, 1, 20, 1e5), (1, 1500, 128, 1e6)])
+def test_steps_on_products_of_clouds_far_apart(n, m, d, far):
+    """Logits of 1e10 to 1e15, whose rounding in base 2 is past what an exponential holds: the largest of a row counts as one."""
+    x, y, a, b = inputs(n + d, n, m, d, scale=0.3)
+    if n == 1:
+        x = x + np.float32(far)
+    else:
+        y = y + np.float32(far)
+    check_symmetric(x, y, a, b, use_epsilon_scaling=False, eps=0.25, n_iters=10)
+
+
 # ---- both half-updates from one sweep (from 2e7 logits per step on): 256-row groups, chunks of
 # 64-row tiles; eps at which steps go without running maxima, and at which the first ones may not ----
 @pytest.mark.parametrize("n,m,d,eps", [(4481, 4703, 3, 0.5), (4608, 4352, 16, 0.01),
