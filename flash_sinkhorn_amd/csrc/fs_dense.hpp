@@ -534,7 +534,7 @@ __global__ __launch_bounds__(512) void dense_rows_kernel(const DenseRowArgs a) {
   const float* kl2w = sd.kl2w + (size_t)item * nk;
   const float eps = coef.x, qs = coef.y, kc = coef.w;
   const float raw = RAW ? coef.z : 1.0f, masked = fmaxf(kNegBig * raw, -3.0e38f);
-  const float start = RAW ? 0.5f * masked : kNegBig, qs1 = RAW ? qs : 1.0f;  // of a row's maximum, in units of `bias`
+  const float no_max = RAW ? 0.5f * masked * qs : kNegBig;
   for (int j = tid; j < ld; j += 512) {
     const float b = __builtin_fmaf(kc, kpot[min(j, nk - 1)], kl2w[min(j, nk - 1)]) * raw;
     bias[j] = j < nk ? fmaxf(b, masked) : masked;
@@ -543,82 +543,65 @@ __global__ __launch_bounds__(512) void dense_rows_kernel(const DenseRowArgs a) {
   if (step > entries + a.s.extrapolate) return;  // (its schedule is shorter)
 
   float m[R], s[R];
-  auto sweep = [&](auto far_) {
-    constexpr bool FAR = decltype(far_)::value;
 #pragma unroll
-    for (int r = 0; r < R; ++r) m[r] = FAR ? start : start * qs1, s[r] = 0.f;
-    for (int c0 = 0; c0 < ld; c0 += 256 * P) {
-      float4 next[R][P];
-      if (c0 + 256 * P < ld) load(next, c0 + 256 * P);
-      if constexpr (RAW) {
-        float M[R];
+  for (int r = 0; r < R; ++r) m[r] = no_max, s[r] = 0.f;
+  for (int c0 = 0; c0 < ld; c0 += 256 * P) {
+    float4 next[R][P];
+    if (c0 + 256 * P < ld) load(next, c0 + 256 * P);
+    if constexpr (RAW) {  // one maximum and rescale for the piece
+      float M[R];
 #pragma unroll
-        for (int r = 0; r < R; ++r) M[r] = start;
+      for (int r = 0; r < R; ++r) M[r] = 0.5f * masked;
 #pragma unroll
-        for (int k = 0; k < P; ++k) {
-          if (c0 + 256 * k >= ld) break;
-          const float4 kb = *reinterpret_cast<const float4*>(&bias[c0 + 256 * k + 4 * lane]);
-#pragma unroll
-          for (int r = 0; r < R; ++r) {
-            float4& l = v[r][k];
-            l = make_float4(l.x + kb.x, l.y + kb.y, l.z + kb.z, l.w + kb.w);
-            M[r] = fmaxf(M[r], fmaxf(fmaxf(l.x, l.y), fmaxf(l.z, l.w)));
-          }
-        }
+      for (int k = 0; k < P; ++k) {
+        if (c0 + 256 * k >= ld) break;
+        const float4 kb = *reinterpret_cast<const float4*>(&bias[c0 + 256 * k + 4 * lane]);
 #pragma unroll
         for (int r = 0; r < R; ++r) {
-          if (!FAR) M[r] *= qs;
-          asm("" : "+v"(M[r]));  // (rounded once, whatever it is used for)
-          M[r] = fmaxf(M[r], m[r]);
-          s[r] *= fast_exp2(FAR ? (m[r] - M[r]) * qs : m[r] - M[r]);
-          m[r] = M[r];
-        }
-        auto term = [&](float l, int r) { return fast_exp2(FAR ? (l - M[r]) * qs : __builtin_fmaf(l, qs, -M[r])); };
-#pragma unroll
-        for (int k = 0; k < P; ++k) {
-          if (c0 + 256 * k >= ld) break;
-#pragma unroll
-          for (int r = 0; r < R; ++r) {
-            const float4 l = v[r][k];
-            s[r] += (term(l.x, r) + term(l.y, r)) + (term(l.z, r) + term(l.w, r));
-          }
-        }
-      } else {
-#pragma unroll
-        for (int k = 0; k < P; ++k) {
-          if (c0 + 256 * k >= ld) break;
-          const float4 kb = *reinterpret_cast<const float4*>(&bias[c0 + 256 * k + 4 * lane]);
-#pragma unroll
-          for (int r = 0; r < R; ++r) {
-            const float l0 = __builtin_fmaf(v[r][k].x, qs, kb.x), l1 = __builtin_fmaf(v[r][k].y, qs, kb.y);
-            const float l2 = __builtin_fmaf(v[r][k].z, qs, kb.z), l3 = __builtin_fmaf(v[r][k].w, qs, kb.w);
-            const float M = fmaxf(fmaxf(fmaxf(l0, l1), fmaxf(l2, l3)), m[r]);
-            s[r] = s[r] * fast_exp2(m[r] - M) +
-                   ((fast_exp2(l0 - M) + fast_exp2(l1 - M)) + (fast_exp2(l2 - M) + fast_exp2(l3 - M)));
-            m[r] = M;
-          }
+          float4& l = v[r][k];
+          l = make_float4(l.x + kb.x, l.y + kb.y, l.z + kb.z, l.w + kb.w);
+          M[r] = fmaxf(M[r], fmaxf(fmaxf(l.x, l.y), fmaxf(l.z, l.w)));
         }
       }
-      if (c0 + 256 * P < ld)
 #pragma unroll
-        for (int k = 0; k < P; ++k)
+      for (int r = 0; r < R; ++r) {
+        M[r] *= qs;
+        asm("" : "+v"(M[r]));  // (rounded once, whatever it is used for)
+        M[r] = fmaxf(M[r], m[r]);
+        s[r] *= fast_exp2(m[r] - M[r]);
+        m[r] = M[r];
+      }
 #pragma unroll
-          for (int r = 0; r < R; ++r) v[r][k] = next[r][k];
+      for (int k = 0; k < P; ++k) {
+        if (c0 + 256 * k >= ld) break;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          const float4 l = v[r][k];
+          s[r] += (fast_exp2(__builtin_fmaf(l.x, qs, -m[r])) + fast_exp2(__builtin_fmaf(l.y, qs, -m[r]))) +
+                  (fast_exp2(__builtin_fmaf(l.z, qs, -m[r])) + fast_exp2(__builtin_fmaf(l.w, qs, -m[r])));
+        }
+      }
+    } else {
+#pragma unroll
+      for (int k = 0; k < P; ++k) {
+        if (c0 + 256 * k >= ld) break;
+        const float4 kb = *reinterpret_cast<const float4*>(&bias[c0 + 256 * k + 4 * lane]);
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          const float l0 = __builtin_fmaf(v[r][k].x, qs, kb.x), l1 = __builtin_fmaf(v[r][k].y, qs, kb.y);
+          const float l2 = __builtin_fmaf(v[r][k].z, qs, kb.z), l3 = __builtin_fmaf(v[r][k].w, qs, kb.w);
+          const float M = fmaxf(fmaxf(fmaxf(l0, l1), fmaxf(l2, l3)), m[r]);
+          s[r] = s[r] * fast_exp2(m[r] - M) +
+                 ((fast_exp2(l0 - M) + fast_exp2(l1 - M)) + (fast_exp2(l2 - M) + fast_exp2(l3 - M)));
+          m[r] = M;
+        }
+      }
     }
-  };
-  sweep(std::false_type{});
-  if constexpr (RAW) {
-    // The maximum's rounding to base 2 is part of every exponential: past 2^24 it is one and more, past 2^31 it would take
-    // the sum to zero or infinity.  There (clouds 1e9 eps apart) the row is swept again, logits less the maximum first.
-    bool far = false;
+    if (c0 + 256 * P < ld)
 #pragma unroll
-    for (int r = 0; r < R; ++r) far = far || (fabsf(m[r]) > 0x1p24f && m[r] != start * qs1);
-    if (wave_any(far)) {
-      load(v, 0);
-      sweep(std::true_type{});
+      for (int k = 0; k < P; ++k)
 #pragma unroll
-      for (int r = 0; r < R; ++r) m[r] *= qs;
-    }
+        for (int r = 0; r < R; ++r) v[r][k] = next[r][k];
   }
   float M = kNegBig, S = 0.f;  // lane r: row r
 #pragma unroll
@@ -634,7 +617,7 @@ __global__ __launch_bounds__(512) void dense_rows_kernel(const DenseRowArgs a) {
   if (lane >= R || row0 + lane >= nq) return;
   const float rho = sd.rho, damp = rho > 0.f ? 1.0f / (1.0f + eps / rho) : 1.0f;
   const float alpha = (step == 0 || step > entries) ? 1.0f : 0.5f;
-  float f = alpha * (-eps * damp * kLn2 * small_log2(fmaxf(S, 1e-40f), M));
+  float f = alpha * (-eps * damp * kLn2 * small_log2(RAW ? small_sum(S, M) : fmaxf(S, 1e-40f), M));
   if (alpha != 1.0f) f += (1.0f - alpha) * old;
   if (damp < 1.0f) f -= alpha * (1.0f - damp) * norm;
   sd.out[at] = f;

@@ -470,6 +470,15 @@ __device__ __forceinline__ float small_max16(float m, const f32x16& a) {
   return m;
 }
 
+// A row's sum of exponentials, with its maximum in base 2.  In units of the products the rounding of that maximum is part of every
+// exponential, which the logarithm of the sum takes out again; past 2^31 (clouds some 1e9 eps apart) it is 128 and more, and the sum
+// zero, infinite or neither.  The largest key counts as one there: no number of keys weighs up against the rounding.
+__device__ __forceinline__ float small_sum(float s, float m) {
+  if (__builtin_amdgcn_classf(s, 0x267))  // (NaN, infinite, zero)
+    if (fabsf(m) > 0x1p30f && fabsf(m) < 3.0e38f) s = 1.0f;
+  return fmaxf(s, 1e-40f);
+}
+
 // What one step of one side needs, laid out so that a workgroup has it after one round of
 // argument loads (pointers of item 0).
 struct SmallStepSide {
@@ -585,7 +594,7 @@ __global__ __launch_bounds__(64 * W) void small_step_kernel(const SmallStepArgs 
   const float eps = coef.x, rho = sd.rho;
   const float damp = rho > 0.f ? 1.0f / (1.0f + eps / rho) : 1.0f;
   const float alpha = (a.full || step == 0 || step > entries) ? 1.0f : 0.5f;
-  float r = alpha * (-eps * damp * kLn2 * small_log2(fmaxf(S, 1e-40f), M));
+  float r = alpha * (-eps * damp * kLn2 * small_log2(small_sum(S, M), M));
   if (alpha != 1.0f) r += (1.0f - alpha) * old;
   if (damp < 1.0f && !a.full) r -= alpha * (1.0f - damp) * shift;
   sd.out[at] = r;

@@ -151,15 +151,18 @@ def test_steps_on_products_are_as_exact_as_those_on_planes(monkeypatch, n, m, d,
     assert np.log(np.array(errors[0]) / errors[1]).mean() < 0.03
 
 
-@pytest.mark.parametrize("n,m,d,far", [(1, 300, 33, 1e4), (300, 1, 70, 1e5), (1, 1, 20, 1e5), (1, 1500, 128, 1e6)])
-def test_steps_on_products_of_clouds_far_apart(n, m, d, far):
+@pytest.mark.parametrize("n,m,d,far", [(1, 300, 33, 1e4), (300, 1, 70, 1e5), (1, 1, 20, 1e5), (1, 1500, 128, 1e6),
+                                       (1, 700, 12, 1e5), (60, 1, 3, 1e6)])
+@pytest.mark.parametrize("n_iters", [3, 10])  # (from 8 on, and from 17 columns, on kept products)
+def test_small_steps_of_clouds_far_apart(n, m, d, far, n_iters):
     """Logits of 1e10 to 1e15, whose rounding in base 2 is past what an exponential holds: the largest of a row counts as one."""
     x, y, a, b = inputs(n + d, n, m, d, scale=0.3)
     if n == 1:
         x = x + np.float32(far)
     else:
         y = y + np.float32(far)
-    check_symmetric(x, y, a, b, use_epsilon_scaling=False, eps=0.25, n_iters=10)
+    check_symmetric(x, y, a, b, use_epsilon_scaling=False, eps=0.25, n_iters=n_iters)
+    check_symmetric(x, y, a, b, use_epsilon_scaling=True, blur=0.5, scaling=0.5)
 
 
 # ---- both half-updates from one sweep (from 2e7 logits per step on): 256-row groups, chunks of
