@@ -57,6 +57,7 @@ constexpr float kPairGap = 44.f;     // base-2 distance below every sum at which
 // 1,531 at eps 0.05, 18 columns there 1,600 / 1,656 / 1,655 / 1,540, 32 at 0.1 - / 1,627 / 1,715 / 1,606.
 constexpr float kPairOn = 0.4f;
 constexpr float kPairTwoOn = 0.7f;   // the same of two-sided steps
+constexpr float kPairLeast = -84.f, kPairMost = 120.f;  // log2 of the smallest and largest sum of a one-sweep step
 constexpr float kPairFar = -2.4e8f;  // bias of rows past the last one, in base 2 (2^12 times -58594)
 
 // One problem: stationary rows against streamed rows.  Pointers of item 0.
@@ -75,6 +76,7 @@ struct PairProblem {
   int self;                 // a matrix with itself: a group streams only rows at or behind its first
   float units;              // 32 x 32 units of all its work items; 0: every logit is computed
   int ends;                 // two-sided steps may end units as well
+  int strict;               // neither marginal is relaxed
   unsigned long long* list; // [items][n_items][wavefront][kPairListWords] units to visit
   unsigned long long* two_list;  // [items][two_items][wavefront][kPairListWords] those that a two-sided step ran
   int n_items;              // work items of this problem
@@ -93,6 +95,7 @@ struct PairMode {
   int list;      // only the units on the lists
   int coarse;    // units are ended by their coarse products where these allow it
   float low;     // log2 of every sum is above that
+  float shift;   // taken off every base-2 logit of a one-sweep step, so that its sums fit fp32
   float ratio;   // the next step's logits over this one's, where its eps is smaller
   float drift;   // with a list: what a logit may have risen by since it was made
   float base;    // ... and what no logit off it reached then
@@ -139,7 +142,7 @@ struct PairArgs {
   const int* lens;          // [items][3]
   float* state;             // [items][3][kPairStateWords]
   const float4* limits;     // [items] smallest and largest base-2 weight of x, of y
-  const float4* reach;      // [items] largest |value|, bound of the costs, bound of a potential
+  const float4* reach;      // [items] largest |value|, bound of the costs, bound of a potential, log2 of the larger mass
   int extrapolate, sched, items, nprob, first_prob, table_len;
   int merge_groups;         // 256-row groups of the larger cloud: workgroups beyond them write planes
   int per_xcd;              // work items of an XCD: an eighth of every problem's
@@ -164,7 +167,8 @@ __device__ __forceinline__ float4 pair_coef(const PairArgs& a, int item, int pro
 }
 
 // Extremes a merge leaves behind, as values whose largest is kept: largest and minus smallest
-// log2 of a row's sum over its weight, of a streamed row's, of the changes of both sides' potentials.
+// log2 of a row's sum over its weight with the row's new potential, of a streamed row's, of the changes of both
+// sides' potentials.
 __device__ __forceinline__ unsigned pair_key(float v) {  // order-preserving
   const unsigned u = __builtin_bit_cast(unsigned, v);
   return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
@@ -175,12 +179,19 @@ __device__ __forceinline__ float pair_value(unsigned k) {
 
 // May step `step` of a problem take both sides from one sweep?  x: log2(R_i / a_i) = log2 of
 // sum_j b_j 2^(e_ij), e = the exponent without weights.  The next step's sum is
-// sum_j b_j 2^(rho e_ij + kappa (df_i + dg_j)), rho = eps / eps', kappa = log2(e) / eps'.  With
-// B = sum b: for rho >= 1 the power means give  rho x - (rho - 1) log2 B <= log2 sum_j b_j 2^(rho e)
+// sum_j b_j 2^(rho (e_ij + kappa (df_i + dg_j))), rho = eps / eps', kappa = log2(e) / eps.  The merge leaves the
+// extremes of z_i = x_i + kappa df_i, so at the old eps the new logarithms lie between z_i + kappa min dg and
+// z_i + kappa max dg (the extremes of x_i and of df_i by themselves would count a change twice where an averaged
+// step halves x_i: 30,011 x 29,989 x 64 to blur 0.05 took two steps more two-sided, 0.70 and 0.96 ms for 0.33
+// each).  Where neither marginal is relaxed and the step was averaged, kappa df_i = -x_i / 2 and
+// kappa dg_j = -y_j / 2, so a new term is the geometric mean of b_j 2^(e_ij - x_i), of which a row's sum is one, and
+// of b_j 2^(e_ij - y_j) <= b_j / a_i: the sum is at most sqrt(B / a_i), B = sum b.  From there to the
+// new eps, for rho >= 1 the power means give  rho x - (rho - 1) log2 B <= log2 sum_j b_j 2^(rho e)
 // <= rho x - (rho - 1) log2 b_min  (and the other way round for rho < 1).  The biases count the
 // weights from the largest of their side (so that logits are small where eps is large, and what a
-// matrix product rounds off them is too).  Every sum taken so has to lie in [2^-80, 2^100]: then no exponential overflows, and what is lost below 2^-126 is less
-// than 2^-26 of a sum with a million terms.  Before the first step the potentials are minus the norms,
+// matrix product rounds off them is too).  Every sum has to lie in [2^-84, 2^120] once all logits are
+// shifted by one number: then no exponential overflows, and what is lost below 2^-126 is less
+// than 2^-26 of a sum with 65,536 terms.  Before the first step the potentials are minus the norms,
 // so e_ij = -C_ij / eps >= -bound / eps.
 // By every lane of a wavefront with the same result; `set`: which of the three sets to read.
 struct PairKnown {  // what pair_mode decides from: all loaded before anything is waited for
@@ -205,7 +216,7 @@ __device__ __forceinline__ PairKnown pair_known(const PairArgs& a, int item, int
   __builtin_amdgcn_sched_barrier(0);
   return k;
 }
-__device__ __forceinline__ PairMode pair_mode(const PairKnown& k, float units, bool ends, int prob, int step) {
+__device__ __forceinline__ PairMode pair_mode(const PairKnown& k, float units, bool ends, bool strict, int prob, int step) {
   const float4 now = k.now, before = k.before, next = k.next, w = k.w, reach = k.reach;
   const float4 lim = prob == 0 ? w : (prob == 1 ? make_float4(w.x, w.y, w.x, w.y) : make_float4(w.z, w.w, w.z, w.w));
   const bool ok0 = (pair_scale(reach.x, now.y) == 0.f) & (now.w * reach.z < kPairMostBias);
@@ -215,10 +226,18 @@ __device__ __forceinline__ PairMode pair_mode(const PairKnown& k, float units, b
   mode.coarse = mode.list = mode.two = 0;
   mode.rho = 1.f;
   mode.least[0] = mode.least[1] = 0.f;
-  mode.drift = mode.base = mode.reserve = 0.f;
+  mode.drift = mode.base = mode.reserve = mode.shift = 0.f;
+  const float mass = reach.w;  // log2 of the larger sum of weights
+  float most = -3.0e38f;       // log2 of every sum is below that
+  // (whole numbers, which fp16 holds)
+  auto fit = [&]() {
+    mode.shift = most > kPairMost ? ceilf(most - kPairMost) : (mode.low < kPairLeast ? floorf(mode.low - kPairLeast) : 0.f);
+    return (most - mode.shift <= kPairMost) & (mode.low - mode.shift >= kPairLeast) & (fabsf(mode.shift) < 2000.f);
+  };
   if (step == 0) {
     mode.low = fminf(lim.x - lim.y, lim.z - lim.w) - reach.y * now.w;
-    mode.sweep = ok & (mode.low > -80.f);
+    most = mass - fminf(lim.y, lim.w);
+    mode.sweep = ok & fit();
     return mode;
   }
   const float rho = before.x == now.x ? 1.f : before.x * __builtin_amdgcn_rcpf(now.x), kappa = now.w;
@@ -241,33 +260,36 @@ __device__ __forceinline__ PairMode pair_mode(const PairKnown& k, float units, b
   mode.least[0] = -kappa * e[7];
   mode.least[1] = -kappa * e[3];
   mode.low = 3.0e38f;
+  const bool averaged = strict && step >= 2;
 #pragma unroll
   for (int s = 0; s < 2; ++s) {
     // this side's sums: weights of its own rows (w) and of the others' (k)
-    const float hi = e[4 * s], lo = -e[4 * s + 1];
-    const float dfh = e[4 * s + 2], dfl = -e[4 * s + 3], dgh = e[4 * (s ^ 1) + 2], dgl = -e[4 * (s ^ 1) + 3];
-    const float wmin = s ? lim.z : lim.x, wmax = s ? lim.w : lim.y, kmin = s ? lim.x : lim.z;
-    const float kmax = s ? lim.y : lim.w, mass = kmax + 20.f;  // log2 B is at most that, with up to a million keys
-    const float up = rho >= 1.f ? rho * hi - (rho - 1.f) * kmin : rho * hi + (1.f - rho) * mass;
-    const float dn = rho >= 1.f ? rho * lo - (rho - 1.f) * mass : rho * lo + (1.f - rho) * kmin;
-    const float U = up + kappa * (dfh + dgh) - kmax, L = dn + kappa * (dfl + dgl) + (wmin - wmax) - kmax;
-    ok = ok & (U < 100.f) & (L > -80.f);
+    const float dgh = e[4 * (s ^ 1) + 2], dgl = -e[4 * (s ^ 1) + 3];
+    const float hi = e[4 * s] + before.w * dgh, lo = -e[4 * s + 1] + before.w * dgl;
+    const float wmin = s ? lim.z : lim.x, wmax = s ? lim.w : lim.y, kmin = s ? lim.x : lim.z, kmax = s ? lim.y : lim.w;
+    const float up = rho >= 1.f ? -(rho - 1.f) * kmin : (1.f - rho) * mass;
+    const float dn = rho >= 1.f ? -(rho - 1.f) * mass : (1.f - rho) * kmin;
+    // (linear in the row's own weight, so largest at one end of it)
+    const float mean = fmaxf(rho * 0.5f * (mass - wmin) + (wmin - wmax), rho * 0.5f * (mass - wmax)) + 1.f;
+    const float U = (averaged ? fminf(rho * hi, mean) : rho * hi) + up - kmax, L = rho * lo + dn + (wmin - wmax) - kmax;
+    ok = ok & (U < 3.0e38f) & (L > -3.0e38f);  // (false where anything is not a number)
+    most = fmaxf(most, U);
     mode.low = fminf(mode.low, L);
   }
-  mode.sweep = ok;  // (false where anything is not a number)
+  mode.sweep = ok & fit();
   // Between two steps at one eps a logit rises by no more than the potentials of its two rows do.
   const float rise = kappa * (e[2] + e[6]);
   mode.drift = k.list.x + rise;
   mode.base = k.list.y;
-  mode.list = ok && mode.coarse && k.list.z != 0.f && mode.base + mode.drift <= mode.low - kPairGap;
+  mode.list = mode.sweep && mode.coarse && k.list.z != 0.f && mode.base + mode.drift <= mode.low - kPairGap;
   // (changes of the potentials shrink from step to step, at first to about a half where a plan is peaked, slowly
   // later: a list that reaches further costs its steps 0.28 us a unit, a new one 320 us, at 50,000 x 64)
   mode.reserve = next.x == now.x ? fminf(16.f + 24.f * __builtin_amdgcn_sqrtf(fmaxf(rise, 0.f)), 256.f) : 0.f;
   return mode;
 }
 
-// A row's bias as three pieces, and what its part in the cross products of the planes can add to a
-// logit (pair_cross), in a column that the matrix product multiplies by zero.
+// A row's bias as three pieces, what its part in the cross products of the planes can add to a
+// logit (pair_cross), in a column that the matrix product multiplies by zero, and a one for the logits' shift.
 __device__ __forceinline__ u32x4 pair_bias(float b, float cross) {
   const _Float16 s1 = (_Float16)4096.f, s2 = (_Float16)1.f, s3 = (_Float16)0.000244140625f;
   const _Float16 p1 = (_Float16)(b * 0.000244140625f);
@@ -278,7 +300,7 @@ __device__ __forceinline__ u32x4 pair_bias(float b, float cross) {
   v[0] = pack_f16((float)s1, (float)s2);
   v[1] = pack_f16((float)s3, (float)p1);
   v[2] = pack_f16((float)p2, (float)p3);
-  v[3] = pack_f16(cross, 0.f);
+  v[3] = pack_f16(cross, 1.f);
   return v;
 }
 // The two cross products of a logit come to at most 2^-10 |x~_i| |y~_j| (|lo| <= 2^-11 |hi|, x~ the rows as
@@ -290,13 +312,13 @@ __device__ __forceinline__ float pair_cross(float kappa, float norm, float reach
 __device__ __forceinline__ float pair_cross_of(const u32x4& bias) {
   return (float)__builtin_bit_cast(_Float16, (unsigned short)(bias[3] & 0xffffu));
 }
-// The same row as an A operand: (b1 b2)(b3 s1)(s2 s3), nothing in the upper half-wave.
-__device__ __forceinline__ u32x4 pair_bias_a(const u32x4& v, int h) {
+// The same row as an A operand: (b1 b2)(b3 s1)(s2 s3)(0 -shift), nothing in the upper half-wave.
+__device__ __forceinline__ u32x4 pair_bias_a(const u32x4& v, int h, float shift) {
   u32x4 r;
   r[0] = __builtin_amdgcn_alignbit(v[2], v[1], 16);
   r[1] = __builtin_amdgcn_alignbit(v[0], v[2], 16);
   r[2] = __builtin_amdgcn_alignbit(v[1], v[0], 16);
-  r[3] = 0u;
+  r[3] = pack_f16(0.f, -shift);
   if (h) r = u32x4{0u, 0u, 0u, 0u};
   return r;
 }
@@ -927,15 +949,16 @@ __device__ __forceinline__ int pair_run_coarse(const PairArgs& a, int batch, Pai
     pair_load_rows(xa, pr.st_planes + ((size_t)batch * pr.st_blocks + blk0) * (2 * KK * 64), lane);
   };
   auto derive_rows = [&]() {
+    const float shift = modes[t.prob].shift;
     far = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(
-              __builtin_bit_cast(int, modes[t.prob].low - modes[t.prob].reserve))) - kPairGap;
+              __builtin_bit_cast(int, modes[t.prob].low - shift - modes[t.prob].reserve))) - kPairGap;
 #pragma unroll
     for (int rb = 0; rb < 2; ++rb) {
       float c = pair_cross_of(xb[rb]);
 #pragma unroll
       for (int o = 16; o > 0; o >>= 1) c = fmaxf(c, __shfl_xor(c, o, 64));
       on_at[rb] = far - c;
-      xb[rb] = pair_bias_a(xb[rb], h);
+      xb[rb] = pair_bias_a(xb[rb], h, shift);
     }
   };
   load_rows();
@@ -1104,7 +1127,7 @@ __device__ __forceinline__ int pair_run_coarse(const PairArgs& a, int batch, Pai
 // rows per block and wavefront, each added in a fixed order.
 template <int DP>
 __device__ __forceinline__ int pair_run_list(const PairArgs& a, int batch, PairWork work, int at, int stride,
-                                             int count, unsigned which, float* cols, float* rows) {
+                                             int count, unsigned which, const PairMode* modes, float* cols, float* rows) {
   constexpr int KK = DP / 16;
   typedef unsigned long long u64;
   struct Keys {
@@ -1166,7 +1189,7 @@ __device__ __forceinline__ int pair_run_list(const PairArgs& a, int batch, PairW
       u32x4 xa[2][2][KK], xb[2];
 #pragma unroll
       for (int rb = 0; rb < 2; ++rb)
-        xb[rb] = pair_bias_a(pr.st_bias[((size_t)batch * pr.st_blocks + blk0 + rb) * 32 + li], h);
+        xb[rb] = pair_bias_a(pr.st_bias[((size_t)batch * pr.st_blocks + blk0 + rb) * 32 + li], h, modes[now.prob].shift);
       pair_load_rows(xa, pr.st_planes + ((size_t)batch * pr.st_blocks + blk0) * (2 * KK * 64), lane);
       const u32x4* planes = pr.str_planes + ((size_t)batch * pr.str_blocks + now.j_begin / 32) * (2 * KK * 64);
       const u32x4* bias = pr.str_bias + (size_t)batch * pr.str_blocks * 32 + now.j_begin;
@@ -1288,7 +1311,7 @@ __device__ __forceinline__ void pair_item_plain(const PairProblem& pr, int batch
 #pragma unroll
   for (int rb = 0; rb < 2; ++rb) {
     const u32x4 v = pr.st_bias[((size_t)batch * pr.st_blocks + blk0 + rb) * 32 + li];
-    xb[rb] = pair_bias_a(v, h);
+    xb[rb] = pair_bias_a(v, h, mode.shift);
     cross = pair_cross_of(v);
   }
   // MFMA k of a unit: the cross products, hi * hi, the biases
@@ -1398,7 +1421,7 @@ __device__ __forceinline__ void pair_item_plain(const PairProblem& pr, int batch
     // this unit says for all of the wavefront's whether the coarse test of the next step would end them
     // (its logits and cross products are about `ratio` times these, the streamed rows' share of the
     // latter about that of the others)
-    if (went != nullptr && wave_any((mx + 2.0f * cross) * mode.ratio > mode.low - mode.reserve - kPairGap) && lane == 0) atomicAdd(went, 4u * (unsigned)ntiles);
+    if (went != nullptr && wave_any((mx + mode.shift + 2.0f * cross) * mode.ratio > mode.low - mode.reserve - kPairGap) && lane == 0) atomicAdd(went, 4u * (unsigned)ntiles);
   }
   S::wait_all();  // (also what was fetched past the chunk)
   __syncthreads();
@@ -1436,7 +1459,7 @@ __global__ __launch_bounds__(256, 2) void pair_sweep_kernel(PairArgsPtr args, in
   {
     const PairKnown known = pair_known(a, batch, own, step);
     const int entries = a.lens[batch * 3 + own];
-    const PairMode m = pair_mode(known, SKIP ? a.prob[own].units : 0.f, SKIP && a.prob[own].ends, own, step);
+    const PairMode m = pair_mode(known, SKIP ? a.prob[own].units : 0.f, SKIP && a.prob[own].ends, a.prob[own].strict, own, step);
     // (where its schedule is shorter nothing is done)
     const bool live = step <= entries + a.extrapolate;
     bits = (live ? 1u : 0u) | (live && m.sweep ? 8u : 0u);
@@ -1481,7 +1504,7 @@ __global__ __launch_bounds__(256, 2) void pair_sweep_kernel(PairArgsPtr args, in
     if (t.prob < 0 || !((live & sweep) >> t.prob & 1)) {
       i += stride;
     } else if (SKIP && ((list >> t.prob) & 1)) {
-      i = pair_run_list<DP>(a, batch, work, i, stride, count, list, reinterpret_cast<float*>(lds),
+      i = pair_run_list<DP>(a, batch, work, i, stride, count, list, modes, reinterpret_cast<float*>(lds),
                             &lds_col[0][0][0][0]);
     } else if (SKIP && ((coarse >> t.prob) & 1)) {
       i = pair_run_coarse<DP>(a, batch, work, i, stride, count, coarse, modes, went, lds, &lds_col[0][0][0][0]);
@@ -1597,7 +1620,7 @@ __global__ __launch_bounds__(1024) void pair_merge_kernel(PairArgsPtr args, int 
     // (one wavefront decides for all: sixteen would take a SIMD's turns from each other)
     __shared__ PairMode sh_mode;
     if (wave == 0) {
-      const PairMode m = pair_mode(known, SKIP ? a.prob[prob].units : 0.f, SKIP && a.prob[prob].ends, prob, step);
+      const PairMode m = pair_mode(known, SKIP ? a.prob[prob].units : 0.f, SKIP && a.prob[prob].ends, a.prob[prob].strict, prob, step);
       if (lane == 0) sh_mode = m;
     }
     __syncthreads();
@@ -1653,7 +1676,7 @@ __global__ __launch_bounds__(1024) void pair_merge_kernel(PairArgsPtr args, int 
     const float2(&all)[4][64] = sh[quarter];
     float lse;
     if (sweep) {
-      lse = small_log2((all[0][lane].y + all[1][lane].y) + (all[2][lane].y + all[3][lane].y), others) - r;
+      lse = small_log2((all[0][lane].y + all[1][lane].y) + (all[2][lane].y + all[3][lane].y), others + mode.shift) - r;
     } else {
       float M = kNegBig, s = 0.f;
 #pragma unroll
@@ -1697,9 +1720,9 @@ __global__ __launch_bounds__(1024) void pair_merge_kernel(PairArgsPtr args, int 
     if (live && part == 0) {
       sd.pot[(from ^ 1) * (size_t)a.items * sd.rows + at] = f;
       if (SKIP) sd.sum2[at] = lse - others;
-      const float x = __builtin_fmaf(coef.w, old, lse), df = f - old;
-      ex[0] = x; ex[1] = -x; ex[2] = df; ex[3] = -df;
-      if (!(x == x) || !(df == df) || !(fabsf(next.w * f) < kPairMostBias)) ex[0] = ex[1] = ex[2] = ex[3] = 3.0e38f;
+      const float z = __builtin_fmaf(coef.w, f, lse), df = f - old;
+      ex[0] = z; ex[1] = -z; ex[2] = df; ex[3] = -df;
+      if (!(z == z) || !(df == df) || !(fabsf(next.w * f) < kPairMostBias)) ex[0] = ex[1] = ex[2] = ex[3] = 3.0e38f;
     }
     // (the set that the next merge writes into)
     if (blockIdx.x == 0 && (side == 0 || side >= 2) && tid < kPairSlots * 9 + 16) {

@@ -192,6 +192,7 @@ void plan_pair(const SmallArgs& a, PairArgs& t) {
     // (a row's few units are a smaller share the more there are: at 4,500 x 64 such a step takes as long as
     // one that computes everything and its merge 5 us longer, at 10,000 x 64 62 against 92 us)
     pr.ends = skips(a.d) && (double)pr.n_st * pr.n_str >= 6.0e7;
+    pr.strict = !(a.rho[s] > 0.f) && !(a.rho[k] > 0.f);
     pr.units = 0.f;
     for (int g = 0; g < pr.groups && skips(a.d); ++g) pr.units += 16.f * (float)((pr.n_str - (pr.self ? 256 * g : 0) + 63) / 64);
   }

@@ -232,7 +232,7 @@ __device__ void small_schedule(const SmallArgs& a, int item) {
   }
   __syncthreads();
   if (a.pair && tid < 64) {
-    float am = 0.f, lim[4];
+    float am = 0.f, mass = 1.f, lim[4];
 #pragma unroll
     for (int mat = 0; mat < 2; ++mat) {
       const bool live = tid < a.stat_blocks;
@@ -248,6 +248,7 @@ __device__ void small_schedule(const SmallArgs& a, int item) {
       am = fmaxf(am, m);
       if (a.w[mat] == nullptr) wl = wh = 1.0f / (float)a.rows[mat];
       else if (a.normalize) wl /= fmaxf(ws, 1e-40f), wh /= fmaxf(ws, 1e-40f);
+      else mass = !(mass >= ws) ? ws : mass;  // (NaN too)
       lim[2 * mat] = wl > 0.f ? small_log2(wl, 0.f) : -100000.0f * kLog2e;
       lim[2 * mat + 1] = wh > 0.f ? small_log2(wh, 0.f) : -100000.0f * kLog2e;
     }
@@ -255,7 +256,7 @@ __device__ void small_schedule(const SmallArgs& a, int item) {
       a.limits[item] = make_float4(lim[0], lim[1], lim[2], lim[3]);
       // (the diagonal of the joint bounding box bounds every distance)
       const float far = a.cost_scale * sq[0];
-      a.reach[item] = make_float4(am, far, 2.0f * (far + a.cost_scale * (float)a.d * am * am), 0.f);
+      a.reach[item] = make_float4(am, far, 2.0f * (far + a.cost_scale * (float)a.d * am * am), small_log2(mass, 0.01f));
     }
   }
   if (a.sched != 1) return;

@@ -175,6 +175,18 @@ def test_one_sweep_steps(n, m, d, eps):
     check_symmetric(x, y, a, b, use_epsilon_scaling=False, eps=eps, n_iters=3)
 
 
+# At a small fixed eps an averaged step halves how far the smallest sum lies below one, some hundreds of base-2 units at
+# first, and relaxed marginals take every sum away from one: each of these ends in a step whose sums fit fp32 only
+# with their logits shifted, or just before or behind one.
+@pytest.mark.parametrize("n,m,d,eps,rho,mass", [(4513, 4481, 20, 0.01, None, 1.0), (4481, 4609, 9, 0.02, None, 1.0),
+                                                (4700, 4650, 33, 0.02, 0.7, 1.3)])
+@pytest.mark.parametrize("n_iters", [3, 4, 5, 6, 7])
+def test_one_sweep_steps_whose_sums_need_a_shift(n, m, d, eps, rho, mass, n_iters):
+    x, y, a, b = inputs(n + d, n, m, d, scale=0.5, y_shift=0.2)
+    check_symmetric(x, y, a, (mass * b).astype(b.dtype), use_epsilon_scaling=False, eps=eps, n_iters=n_iters,
+                    rho_x=rho, rho_y=rho)
+
+
 # a whole schedule on these kernels (planes written behind every step), as long as it is
 def test_one_sweep_steps_of_a_full_schedule():
     from flash_sinkhorn_amd.kernels import sinkhorn_flashstyle_symmetric as solve
