@@ -130,7 +130,16 @@ int loss_parts(const SmallArgs& a) {
   return rows <= 3072 ? 1 : std::min(64, (rows + 1023) / 1024);
 }
 
-int padded(int64_t d) { return d <= 16 ? 16 : (d <= 32 ? 32 : (d <= 64 ? 64 : 128)); }
+// Columns that planes hold: as few 16-column steps as the rows fill, in steps of 32 from 64 on (80 and 112 columns were not
+// built).  A step streams and multiplies all of them, so the last quarter counts: with 64 and 128 columns -> 48 and 96,
+// loss and gradient, us: schedules 3,001 x 4,567 x 33 315 -> 283, 5,000 x 5,100 x 40 492 -> 385 and x 80 1,210 -> 953, 30,000 x
+// 29,000 x 40 5,730 -> 4,020; 3,112 x 2,124 x 37, debiased, 73 steps 1,592 -> 1,399; 10,000 x 44, 60 steps, mostly along lists
+// 2,327 -> 2,170.  Products of narrow rows are formed two steps at a time, so a solve on these takes 64 for 48.
+int padded(const fs_small_problem* p) {
+  if (p->d <= 32) return p->d <= 16 ? 16 : 32;
+  if (p->d <= 64) return p->d <= 48 && !use_products(p) ? 48 : 64;
+  return p->d <= 96 ? 96 : 128;
+}
 
 // `solved`: the problem has been, and its list of eps is not looked at again (the workspace has the table).
 int checked(const fs_small_problem* p, bool solved = false) {
@@ -307,7 +316,7 @@ size_t layout(const fs_small_problem* p, void* ws, SmallArgs& a, PairArgs* pa = 
   a.scaling = p->scaling;
   a.rho[0] = p->rho_x;
   a.rho[1] = p->rho_y;
-  const int dp = padded(p->d), ndb = (dp + 31) / 32;
+  const int dp = use_dense(p) ? 0 : padded(p), ndb = (dp + 31) / 32;
   size_t at = 0;
   char* base = static_cast<char*>(ws);
   auto take = [&](auto& ptr, size_t bytes) {
@@ -538,11 +547,13 @@ int launch_grad(const SmallArgs& a, const PairArgs& pa, const SmallGradArgs& g, 
 }
 
 template <typename F>
-int by_width(int64_t d, F&& f) {
-  switch (padded(d)) {
+int by_width(const fs_small_problem* p, F&& f) {
+  switch (padded(p)) {
     case 16: return f(std::integral_constant<int, 16>{});
     case 32: return f(std::integral_constant<int, 32>{});
+    case 48: return f(std::integral_constant<int, 48>{});
     case 64: return f(std::integral_constant<int, 64>{});
+    case 96: return f(std::integral_constant<int, 96>{});
     default: return f(std::integral_constant<int, 128>{});
   }
 }
@@ -611,7 +622,7 @@ int fs_small_solve_products(const fs_small_problem* p, void* workspace, size_t w
     hipLaunchKernelGGL((small_table_kernel<0>), dim3(a.items * 3), dim3(256), 0, st, a, t);
     if (hipGetLastError() != hipSuccess) return FS_ERR_LAUNCH_FAILED;
   }
-  rc = dense ? dense_prepare(a, da, st) : by_width(p->d, [&](auto dp) {
+  rc = dense ? dense_prepare(a, da, st) : by_width(p, [&](auto dp) {
     constexpr int DP = decltype(dp)::value;
     const int r = launch_prep<DP>(a, pa, pair_at, st);
     if constexpr (DP <= 64)
@@ -624,7 +635,7 @@ int fs_small_solve_products(const fs_small_problem* p, void* workspace, size_t w
   auto run_step = [&](int s) {
     if (wave_rows) return launch_rows(a, s, by_rows.dots, by_rows.ld, dense ? da.top : nullptr, wave_rows, st);
     if (dense) return dense_step(a, da, s, st);
-    return by_width(p->d, [&](auto dp) {
+    return by_width(p, [&](auto dp) {
       constexpr int DP = decltype(dp)::value;
       if (a.alternating) return launch_alternating<DP>(a, s, st);
       if constexpr (DP <= 64)
@@ -739,7 +750,7 @@ int fs_small_grad(const fs_small_problem* p, void* workspace, size_t workspace_b
   g.grad_out = grad_out;
   g.out[0] = grad_x;
   g.out[1] = grad_y;
-  return by_width(p->d, [&](auto dp) { return launch_grad<decltype(dp)::value>(a, pa, g, (hipStream_t)stream); });
+  return by_width(p, [&](auto dp) { return launch_grad<decltype(dp)::value>(a, pa, g, (hipStream_t)stream); });
 }
 
 }  // extern "C"

@@ -439,6 +439,22 @@ def test_loss_and_gradients(n, m, d, debias):
         assert np.abs(g.cpu().numpy() - w).max() < GRAD * np.abs(p).max()
 
 
+# ---- planes of 48 and 96 columns: the last one they hold and the first they do not, in every form ----
+@pytest.mark.parametrize("n,m,d", [(33, 70, 33), (300, 257, 47), (65, 1600, 48), (300, 130, 49), (90, 129, 65),
+                                   (257, 200, 95), (40, 300, 96), (130, 90, 97), (4500, 4471, 48)])
+def test_columns_of_the_planes(n, m, d):
+    from flash_sinkhorn_amd.kernels import sinkhorn_flashstyle_alternating as alternating
+    x, y, a, b = inputs(n + d, n, m, d, scale=0.5, y_shift=0.2)
+    # (below eight steps on planes, from there on, where they fit, on kept products)
+    for n_iters in (3, 9)[:1 if n > 1000 else 2]:
+        check_symmetric(x, y, a, b, use_epsilon_scaling=False, eps=0.1, n_iters=n_iters)
+        got = alternating(*dev(x, y, a, b), eps=0.1, n_iters=n_iters)
+        for g, w in zip(got, oracle.sinkhorn_alternating(x, y, a, b, eps=0.1, n_iters=n_iters)):
+            assert rel_err(g, w) < POT
+    for debias in (False, True)[:1 if n > 1000 else 2]:
+        test_loss_and_gradients(n, m, d, debias)
+
+
 # ---- medium problems: both directions of the one-sweep kernels at small eps ----
 def gradient_bound(x, y, eps):
     """Largest error of a barycentre whose logits are off by delta: every weight by a factor e^(+-delta),
