@@ -126,7 +126,8 @@ def ptr(t: Optional[torch.Tensor]):
 
 
 def stream_of(t: torch.Tensor):
-    return torch.cuda.current_stream(t.device).cuda_stream
+    # (without a Stream object around it: 0.1 for 2.1 us)
+    return torch._C._cuda_getCurrentRawStream(t.device.index)
 
 
 def workspace(op: int, n: int, m: int, d: int, device) -> Optional[torch.Tensor]:

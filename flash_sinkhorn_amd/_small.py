@@ -532,8 +532,32 @@ def _item_weights(w, rows, i, normalize, device):
     return w / w.sum().clamp(min=1e-40) if normalize else w
 
 
+def _differentiate(form: Problem, config: dict, grad_out, tensors, need):
+    """Gradients of a loss in x, y and its weights from what its node has saved: x and y, then
+    ``Solved.tensors``."""
+    x, y, *solved = tensors
+    s = Solved.restored(form, solved)
+    gx = gy = ga = gb = None
+    if need[0] or need[1]:
+        if x.dtype not in _DTYPES:  # (as the gradient of the general path)
+            raise ValueError(f"Unsupported dtype for x/y: {x.dtype}")
+        if torch.is_grad_enabled():  # create_graph
+            gx, gy = _SmallGrad.apply(x, y, grad_out, s, SimpleNamespace(**config), need[0], need[1])
+        else:
+            gx, gy = _gradients(s, grad_out, need[0], need[1])
+    scale = grad_out if x.ndim == 2 else grad_out[:, None]
+    if need[2]:
+        f = s.potentials("f")[0] - s.potentials("xx")[0] if form.self_terms else s.potentials("f")[0]
+        ga = scale * (f if x.ndim == 3 else f[0])
+    if need[3]:
+        g = s.potentials("g")[0] - s.potentials("yy")[0] if form.self_terms else s.potentials("g")[0]
+        gb = scale * (g if x.ndim == 3 else g[0])
+    return gx, gy, ga, gb
+
+
 class _SmallLoss(torch.autograd.Function):
-    """Cost of every item, debiased or not, from one run; scalar for a single problem."""
+    """Cost of every item, debiased or not, from one run; scalar for a single problem.  For tensors that only a
+    Function serves or refuses (tangents, functorch, subclasses); the others have a native node (``loss``)."""
 
     @staticmethod
     def forward(ctx, x, y, a, b, loss, normalize):
@@ -547,26 +571,46 @@ class _SmallLoss(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_out):
-        x, y, *solved = ctx.saved_tensors
-        s, need = Solved.restored(ctx.form, solved), ctx.needs_input_grad
-        gx = gy = ga = gb = None
-        if need[0] or need[1]:
-            if x.dtype not in _DTYPES:  # (as the gradient of the general path)
-                raise ValueError(f"Unsupported dtype for x/y: {x.dtype}")
-            if torch.is_grad_enabled():  # create_graph
-                gx, gy = _SmallGrad.apply(x, y, grad_out, s, SimpleNamespace(**ctx.config),
-                                          need[0], need[1])
-            else:
-                gx, gy = _gradients(s, grad_out, need[0], need[1])
-        scale = grad_out if x.ndim == 2 else grad_out[:, None]
-        if need[2]:
-            f = s.potentials("f")[0] - s.potentials("xx")[0] if s.form.self_terms else s.potentials("f")[0]
-            ga = scale * (f if x.ndim == 3 else f[0])
-        if need[3]:
-            g = s.potentials("g")[0] - s.potentials("yy")[0] if s.form.self_terms else s.potentials("g")[0]
-            gb = scale * (g if x.ndim == 3 else g[0])
-        return gx, gy, ga, gb, None, None
+        return _differentiate(ctx.form, ctx.config, grad_out, ctx.saved_tensors, ctx.needs_input_grad) + (None, None)
+
+
+class _Ask:
+    """What a native node calls for a gradient that it does not form itself."""
+    __slots__ = ("form", "config")
+
+    def __init__(self, form, config):
+        self.form, self.config = form, config
+
+    def __call__(self, grad_out, tensors, need):
+        return _differentiate(self.form, self.config, grad_out, tensors, need)
+
+
+_NATIVE = None
+
+
+def _native():
+    """The module with the native node, and the address of the gradient it calls."""
+    global _NATIVE
+    if _NATIVE is None:
+        try:
+            from flash_sinkhorn_amd import _native as module
+        except ImportError as e:
+            raise RuntimeError(f"flash_sinkhorn_amd._native is missing or does not load ({e}): build it with "
+                               f"`make -C {_lib.CSRC_DIR}`.") from e
+        _NATIVE = module, ctypes.cast(_lib.lib().fs_small_grad, _P).value
+    return _NATIVE
 
 
 def loss(module, x, y, a, b, normalize):
-    return _SmallLoss.apply(x, y, a, b, module, normalize)
+    given = [x, y, a, b]
+    native, grad = _native()
+    if not native.ordinary(given):
+        return _SmallLoss.apply(x, y, a, b, module, normalize)
+    need = [torch.is_grad_enabled() and t is not None and t.requires_grad for t in given]
+    s = _solve_for(module, x, y, a, b, normalize, self_terms=int(module.debias),
+                   want_values=need[0] or need[1], want_loss=True)
+    if True not in need:
+        return s.loss
+    # (the settings as they are now, for a second backward pass)
+    return native.attach(s.loss, a, b, [x, y, *s.tensors()], ctypes.addressof(s.form), ctypes.sizeof(s.form), grad,
+                         _Ask(s.form, dict(vars(module))))

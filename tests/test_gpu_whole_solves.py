@@ -846,6 +846,56 @@ def test_saved_tensors_pass_through_hooks_and_version_checks():
             loss.backward()
 
 
+# The native autograd node against the Function that it stands for, to the bit; what only a Function serves or
+# refuses still reaches one.
+@pytest.mark.parametrize("form", ["x", "y", "both", "weights", "batch", "float16", "strided", "replayed", "scaled", "hooks"])
+@pytest.mark.parametrize("debias", [False, True])
+def test_native_node_equals_the_function(monkeypatch, form, debias):
+    from flash_sinkhorn_amd import SamplesLoss, _small
+    from types import SimpleNamespace
+    x, y, a, b = inputs(21, 130, 97, 20, scale=0.5, y_shift=0.2)
+    X, Y, A, B = dev(x, y, a, b)
+    if form == "batch":
+        X, Y, A, B = (torch.stack([t, t.flip(0)]) for t in (X, Y, A, B))
+    if form == "float16":
+        X, Y = X.half(), Y.half()
+    if form == "strided":
+        X = X.t().contiguous().t()
+    kw = dict(use_epsilon_scaling=False, eps=0.1, n_iters=12) if form == "replayed" else dict(blur=0.2)
+    fn = SamplesLoss("sinkhorn", debias=debias, **kw)
+    wanted = {"x": [X], "y": [Y], "weights": [A, X, B, Y]}.get(form, [X, Y])
+    for t in wanted:
+        t.requires_grad_()
+    native, grad = _small._native()
+    out = []
+    for ordinary in (True, False):
+        with monkeypatch.context() as m:
+            m.setattr(_small, "_NATIVE", (SimpleNamespace(ordinary=lambda _: ordinary, attach=native.attach), grad))
+            for _ in range(3):
+                if form == "hooks":
+                    with torch.autograd.graph.save_on_cpu():
+                        loss = fn(A, X, B, Y)
+                else:
+                    loss = fn(A, X, B, Y)
+                seed = torch.full_like(loss, 3.0) if form == "scaled" else torch.ones_like(loss)
+                grads = torch.autograd.grad(loss, wanted, seed, retain_graph=True)
+                again = torch.autograd.grad(loss, wanted, seed)
+            assert all(torch.equal(u, v) for u, v in zip(grads, again))
+            with pytest.raises(RuntimeError, match="second time"):
+                torch.autograd.grad(loss, wanted, seed)
+            out.append((loss.detach(), *grads))
+    assert all(u.dtype is v.dtype and torch.equal(u, v) for u, v in zip(*out))
+    if form == "x" and not debias:
+        with torch.no_grad():
+            assert not fn(A, X, B, Y).requires_grad
+        gx, = torch.autograd.grad(fn(A, X, B, Y), X, create_graph=True)
+        assert torch.equal(gx.detach(), out[0][1])
+        with torch.autograd.forward_ad.dual_level(), pytest.raises(NotImplementedError, match="jvp"):
+            fn(torch.autograd.forward_ad.make_dual(X.detach(), torch.ones_like(X)), Y)
+        with pytest.raises(RuntimeError, match="functorch"):
+            torch.func.grad(lambda t: fn(t, Y))(X.detach())
+
+
 # ---- gradients along lists read nothing but the workspace that the autograd node holds: behind other
 # losses of the same replayed graph, behind a graph that is forgotten, at another address ----
 @pytest.mark.parametrize("n,m,d,eps,debias", [(4513, 4490, 64, 0.01, False), (3300, 3290, 20, 0.02, True)])
