@@ -14,7 +14,7 @@ from typing import Optional, Tuple
 import torch
 
 from flash_sinkhorn_amd import _small
-from flash_sinkhorn_amd.hvp import geomloss_to_ott_potentials, hvp_x_sqeuclid_from_potentials
+from flash_sinkhorn_amd.hvp import hvp_x_sqeuclid_from_potentials
 from flash_sinkhorn_amd.kernels.sinkhorn_triton_grad_sqeuclid import (
     sinkhorn_geomloss_online_grad_sqeuclid,
 )
@@ -100,9 +100,8 @@ class _SinkhornGradFn(torch.autograd.Function):
             if not grad_grad_x.is_cuda:
                 raise ValueError("grad_grad_x must be a CUDA tensor.")
             with torch.no_grad():
-                f_ott, g_ott = geomloss_to_ott_potentials(f_grad, g_grad, a, b, eps=ctx.eps)
-                hvp, _ = hvp_x_sqeuclid_from_potentials(
-                    x, y, f_ott, g_ott, grad_grad_x, eps=ctx.eps, rho_x=cfg.rho_x,
+                out_x, _ = hvp_x_sqeuclid_from_potentials(
+                    x, y, f_grad, g_grad, grad_grad_x, eps=ctx.eps, rho_x=cfg.rho_x,
                     rho_y=cfg.rho_y, cost_scale=cfg.cost_scale, tau2=cfg.hvp_tau2,
                     max_cg_iter=cfg.hvp_max_cg_iter, cg_rtol=cfg.hvp_cg_rtol,
                     cg_atol=cfg.hvp_cg_atol, cg_stabilise_every=cfg.hvp_cg_stabilise_every,
@@ -110,8 +109,8 @@ class _SinkhornGradFn(torch.autograd.Function):
                     use_preconditioner=cfg.hvp_use_preconditioner,
                     allow_tf32=False,  # second order needs full fp32 operands
                     use_exp2=cfg.use_exp2,
-                    _products=_small.Products(ctx.products, *kept) if kept else None)
-                out_x = hvp * grad_scale
+                    _products=_small.Products(ctx.products, *kept) if kept else None,
+                    _weights=(a, b), _scale=grad_scale)
         return (out_x,) + (None,) * 15
 
 

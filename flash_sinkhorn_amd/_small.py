@@ -487,8 +487,7 @@ class _SmallGrad(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad_grad_x, grad_grad_y):
         x, y, grad_out = ctx.saved_tensors[:3]
-        from flash_sinkhorn_amd.hvp import (geomloss_to_ott_potentials,
-                                            hvp_x_sqeuclid_from_potentials)
+        from flash_sinkhorn_amd.hvp import hvp_x_sqeuclid_from_potentials
         cfg, s = ctx.config, Solved.restored(ctx.form, ctx.saved_tensors[3:])
         if grad_grad_y is not None or s.form.self_terms:
             raise NotImplementedError("Double backward w.r.t y is not implemented yet.")
@@ -500,20 +499,18 @@ class _SmallGrad(torch.autograd.Function):
             gs = grad_out.reshape(-1)
             for i in range(items):
                 xi, yi, v = (t if t.ndim == 2 else t[i] for t in (x, y, grad_grad_x))
-                a, b = (_item_weights(w, rows, i, s.form.normalize, x.device)
-                        for w, rows in ((s.a, s.form.n), (s.b, s.form.m)))
-                eps = _last_eps(cfg, xi, yi)
-                f_ott, g_ott = geomloss_to_ott_potentials(f[i], g[i], a, b, eps=eps)
+                weights = tuple(_item_weights(w, rows, i, s.form.normalize)
+                                for w, rows in ((s.a, s.form.n), (s.b, s.form.m)))
                 hvp, _ = hvp_x_sqeuclid_from_potentials(
-                    xi, yi, f_ott, g_ott, v, eps=eps, rho_x=cfg.rho_x, rho_y=cfg.rho_y,
+                    xi, yi, f[i], g[i], v, eps=_last_eps(cfg, xi, yi), rho_x=cfg.rho_x, rho_y=cfg.rho_y,
                     cost_scale=cfg.cost_scale, tau2=cfg.hvp_tau2, max_cg_iter=cfg.hvp_max_cg_iter,
                     cg_rtol=cfg.hvp_cg_rtol, cg_atol=cfg.hvp_cg_atol,
                     cg_stabilise_every=cfg.hvp_cg_stabilise_every,
                     preconditioner=cfg.hvp_preconditioner, precond_terms=cfg.hvp_precond_terms,
                     use_preconditioner=cfg.hvp_use_preconditioner,
                     allow_tf32=False,  # second order needs full fp32 operands
-                    use_exp2=cfg.use_exp2)
-                outs.append(hvp * gs[i])
+                    use_exp2=cfg.use_exp2, _weights=weights, _scale=gs[i])
+                outs.append(hvp)
         return (outs[0] if x.ndim == 2 else torch.stack(outs),) + (None,) * 6
 
 
@@ -525,9 +522,9 @@ def _last_eps(cfg, x, y) -> float:
     return epsilon_schedule(max_diameter(x, y), cfg.blur, cfg.scaling)[: cfg.n_iters][-1]
 
 
-def _item_weights(w, rows, i, normalize, device):
+def _item_weights(w, rows, i, normalize):
     if w is None:
-        return torch.full((rows,), 1.0 / rows, device=device, dtype=torch.float32)
+        return None
     w = w.reshape(-1, rows)[i]
     return w / w.sum().clamp(min=1e-40) if normalize else w
 

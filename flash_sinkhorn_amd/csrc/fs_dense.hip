@@ -24,11 +24,12 @@ int launch_gemm(DenseGemmArgs& g, int items, hipStream_t st) {
 }
 
 template <int WR, int WC, int RB, int CB>
-int launch_jobs(DenseGemmJobs& g, int jobs, int items, hipStream_t st) {
+int launch_jobs(DenseGemmJobs& g, int jobs, int items, hipStream_t st, bool apart) {
   int tiles = 0;
   for (int i = 0; i < jobs; ++i) tiles = std::max(tiles, tile_up<WR, WC, RB, CB>(g.job[i]));
-  hipLaunchKernelGGL((dense_gemm_jobs_kernel<WR, WC, RB, CB>), dim3((tiles + 7) / 8 * 8, items, jobs), dim3(64 * WR * WC), 0,
-                     st, g);
+  const dim3 grid((tiles + 7) / 8 * 8, items, jobs), block(64 * WR * WC);
+  if (apart) hipLaunchKernelGGL((dense_gemm_jobs_kernel<WR, WC, RB, CB, true>), grid, block, 0, st, g);
+  else hipLaunchKernelGGL((dense_gemm_jobs_kernel<WR, WC, RB, CB, false>), grid, block, 0, st, g);
   return hipGetLastError() == hipSuccess ? FS_OK : FS_ERR_LAUNCH_FAILED;
 }
 
@@ -79,14 +80,14 @@ int dense_gemm(DenseGemmArgs& g, int items, hipStream_t st) {
 }
 
 // (rows of every result padded to 256 columns, so that each takes any of the tiles)
-int dense_gemm_jobs(DenseGemmJobs& g, int jobs, int items, hipStream_t st) {
+int dense_gemm_jobs(DenseGemmJobs& g, int jobs, int items, hipStream_t st, bool apart) {
   int most = 0;
   for (int i = 1; i < jobs; ++i)
     if ((double)g.job[i].rows * g.job[i].ld > (double)g.job[most].rows * g.job[most].ld) most = i;
   const int side = best_side(g.job[most], 1, items * jobs);
-  if (side == 256) return launch_jobs<2, 4, 4, 2>(g, jobs, items, st);
-  if (side == 128) return launch_jobs<2, 2, 2, 2>(g, jobs, items, st);
-  return launch_jobs<2, 2, 1, 1>(g, jobs, items, st);
+  if (side == 256) return launch_jobs<2, 4, 4, 2>(g, jobs, items, st, apart);
+  if (side == 128) return launch_jobs<2, 2, 2, 2>(g, jobs, items, st, apart);
+  return launch_jobs<2, 2, 1, 1>(g, jobs, items, st, apart);
 }
 
 void dense_plan(const SmallArgs& a, DenseArgs& t) {

@@ -71,9 +71,8 @@ __device__ __forceinline__ bool dense_wide(const void* p, int d, int dtype) {
 
 // Largest magnitude and sum of the weights of a slice of one matrix (small_stats_kernel's first two
 // words; no bounding boxes: a schedule comes as a table here).  Bound by memory.
-template <int T>
-__global__ __launch_bounds__(1024) void dense_stats_kernel(const SmallArgs a) {
-  const int mat = blockIdx.y, item = blockIdx.z, tid = threadIdx.x;
+__device__ __forceinline__ void dense_stats_of(const SmallArgs& a, int mat, int item) {
+  const int tid = threadIdx.x;
   const size_t count = (size_t)a.rows[mat] * a.d, base = item * count;
   const bool wide = dense_wide(a.pts[mat], a.d, a.dtype);
   float am = 0.f, ws = 0.f;
@@ -108,12 +107,15 @@ __global__ __launch_bounds__(1024) void dense_stats_kernel(const SmallArgs a) {
     out[1] = ws;
   }
 }
+template <int T>
+__global__ __launch_bounds__(1024) void dense_stats_kernel(const SmallArgs a) {
+  dense_stats_of(a, blockIdx.y, blockIdx.z);
+}
 
 // Planes of 32 rows, their norms, log weights and initial potentials.  Grid (blocks of the larger
 // matrix and one more, which fills the table of a fixed eps; matrices; items).
-template <int T>
-__global__ __launch_bounds__(512) void dense_prep_kernel(const SmallArgs a, const DenseArgs t) {
-  const int mat = blockIdx.y, item = blockIdx.z, tid = threadIdx.x;
+__device__ __forceinline__ void dense_prep_of(const SmallArgs& a, const DenseArgs& t, int mat, int item) {
+  const int tid = threadIdx.x;
   if ((int)blockIdx.x == gridDim.x - 1) {
     if (mat == 0) small_schedule(a, item);
     return;
@@ -166,6 +168,10 @@ __global__ __launch_bounds__(512) void dense_prep_kernel(const SmallArgs a, cons
   a.wt[mat][at] = w;
   a.l2w[mat][at] = w > 0.f ? small_log2(w, 0.f) : -100000.0f * kLog2e;
   a.pot[mat][at] = -al;
+}
+template <int T>
+__global__ __launch_bounds__(512) void dense_prep_kernel(const SmallArgs a, const DenseArgs t) {
+  dense_prep_of(a, t, blockIdx.y, blockIdx.z);
 }
 
 // One operand's tile stream and C = A B^T: a workgroup of WR x WC wavefronts owns 32 WR RB rows and
@@ -321,9 +327,9 @@ __global__ __launch_bounds__(64 * WR * WC, 2) void dense_gemm_kernel(const Dense
 struct DenseGemmJobs {
   DenseGemmArgs job[4];
 };
-template <int WR, int WC, int RB, int CB>
+template <int WR, int WC, int RB, int CB, bool APART>
 __global__ __launch_bounds__(64 * WR * WC, 2) void dense_gemm_jobs_kernel(const DenseGemmJobs g) {
-  dense_gemm_tile<WR, WC, RB, CB, true>(g.job[blockIdx.z], 0);
+  dense_gemm_tile<WR, WC, RB, CB, APART>(g.job[blockIdx.z], 0);
 }
 
 __device__ __forceinline__ void dense_join(float& m, float& s, float m2, float s2) {
@@ -628,7 +634,7 @@ __global__ __launch_bounds__(512) void dense_rows_kernel(const DenseRowArgs a) {
 void dense_plan(const SmallArgs& a, DenseArgs& t);
 void dense_gemm_plan(DenseGemmArgs& g, bool may_split);
 int dense_gemm(DenseGemmArgs& g, int items, hipStream_t st);
-int dense_gemm_jobs(DenseGemmJobs& g, int jobs, int items, hipStream_t st);
+int dense_gemm_jobs(DenseGemmJobs& g, int jobs, int items, hipStream_t st, bool apart = true);
 int dense_prepare(const SmallArgs& a, const DenseArgs& t, hipStream_t st);
 int dense_step(const SmallArgs& a, DenseArgs& t, int step, hipStream_t st);
 int dense_rows_step(const DenseRowArgs& t, int rows, bool raw, int sides, int items, hipStream_t st);

@@ -3,6 +3,7 @@
 #include "fs_hvp.hpp"
 
 #include <algorithm>
+#include <cmath>
 #include <cstring>
 #include <type_traits>
 
@@ -87,6 +88,12 @@ size_t layout(const fs_hvp_problem* p, void* ws, HvpPlan& q, bool shared, const 
   a.A = p->A;
   a.f = p->f;
   a.g = p->g;
+  a.log_a = p->log_a;
+  a.log_b = p->log_b;
+  a.log_n = std::log((float)(1.0 / n));
+  a.log_m = std::log((float)(1.0 / m));
+  a.weighted = p->weighted;
+  a.out_scale = p->out_scale;
   a.n = n;
   a.m = m;
   a.d = d;
@@ -155,19 +162,30 @@ size_t layout(const fs_hvp_problem* p, void* ws, HvpPlan& q, bool shared, const 
   return at;
 }
 
-// (the directions' planes: one matrix, the second operand of its product is y's)
-int prepare(const SmallArgs& s, const DenseArgs& t, int mats, hipStream_t st) {
-  hipLaunchKernelGGL((dense_stats_kernel<0>), dim3(s.stat_blocks, mats), dim3(1024), 0, st, s);
-  const int blocks = mats == 2 ? std::max(t.blocks[0], t.blocks[1]) : t.blocks[0];
-  hipLaunchKernelGGL((dense_prep_kernel<0>), dim3(blocks + 1, mats), dim3(512), 0, st, s, t);
-  return hipGetLastError() == hipSuccess ? FS_OK : FS_ERR_LAUNCH_FAILED;
+// The planes of x and y, where no solve has left them, and of the direction (one matrix, the second operand of its
+// product is y's), what of the operands is taken row by row, and the products.
+int prepare(HvpPlan& q, bool kept, hipStream_t st) {
+  const HvpArgs& a = q.a;
+  const int mats = kept ? 0 : 2, blocks = kept ? q.ta.blocks[0] : std::max(q.td.blocks[0], q.td.blocks[1]);
+  hipLaunchKernelGGL((hvp_stats_kernel<0>), dim3(kSmallStatBlocks, mats + 1), dim3(1024), 0, st, q.pts, q.dir, mats);
+  hipLaunchKernelGGL((hvp_prep_kernel<0>), dim3(blocks + 1, mats + 1), dim3(512), 0, st, q.pts, q.td, q.dir, q.ta, mats);
+  const TransposedArgs yt = {a.y, a.scale, a.yt, a.m, a.d, a.ld, a.dtype};
+  hipLaunchKernelGGL((hvp_rows_kernel<0>), dim3((a.n + a.ld + 3) / 4 + (a.ld / 16 + 3) / 4 * a.yt_blocks), dim3(256), 0, st, a, yt);
+  if (hipGetLastError() != hipSuccess) return FS_ERR_LAUNCH_FAILED;
+  if (kept) return dense_gemm(q.prod, 1, st);
+  DenseGemmJobs jobs;
+  std::memset(&jobs, 0, sizeof(jobs));
+  jobs.job[0] = q.dots;
+  jobs.job[1] = q.prod;
+  return dense_gemm_jobs(jobs, 2, 1, st, false);
 }
 
 template <int MODE>
 int strips(const HvpArgs& a, hipStream_t st) {
-  if (a.ld <= 2048) hipLaunchKernelGGL((hvp_strip_kernel<1, 8, MODE>), dim3(a.strips), dim3(512), 0, st, a);
-  else if (a.ld <= 4096) hipLaunchKernelGGL((hvp_strip_kernel<2, 8, MODE>), dim3(a.strips), dim3(512), 0, st, a);
-  else hipLaunchKernelGGL((hvp_strip_kernel<4, 4, MODE>), dim3(a.strips), dim3(512), 0, st, a);
+  const int wgs = a.strips + (MODE == 2 ? 1 : 0);
+  if (a.ld <= 2048) hipLaunchKernelGGL((hvp_strip_kernel<1, 8, MODE>), dim3(wgs), dim3(512), 0, st, a);
+  else if (a.ld <= 4096) hipLaunchKernelGGL((hvp_strip_kernel<2, 8, MODE>), dim3(wgs), dim3(512), 0, st, a);
+  else hipLaunchKernelGGL((hvp_strip_kernel<4, 4, MODE>), dim3(wgs), dim3(512), 0, st, a);
   if constexpr (MODE < 2) hipLaunchKernelGGL((hvp_columns_kernel<MODE>), dim3((a.m + 63) / 64), dim3(256), 0, st, a);
   return hipGetLastError() == hipSuccess ? FS_OK : FS_ERR_LAUNCH_FAILED;
 }
@@ -282,6 +300,11 @@ int fs_dense_grad(const fs_small_problem* p, void* solved_workspace, size_t solv
 namespace fs {
 namespace {
 
+// On a few thousand points no launch but the mass' and V's takes longer than a launch does (3 to 6 us), so there are as few as the
+// data's way allows: the operands of both products prepared together, the two products in one launch, y^T with the rows,
+// the limits with the last strips, the weights and the outer factor in kernels that read the potentials and
+// write the result (26 launches and some 15 small ones around them -> 21 and none: loss, gradient and product of 2,048 x
+// 2,048 x 64 717 -> 640 us, 1,500 x 1,400 x 20 668 -> 493, 7,000 x 5,000 x 60 1,458 -> 1,400, 6,000 x 7,500 x 900 3,061 -> 3,014).
 int run_hvp(const fs_hvp_problem* p, const Kept* kept, void* workspace, size_t workspace_bytes, float* out,
             float* host_state, hipStream_t st) {
   int rc = checked(p);
@@ -291,9 +314,7 @@ int run_hvp(const fs_hvp_problem* p, const Kept* kept, void* workspace, size_t w
   if (!workspace || layout(p, workspace, q, kept != nullptr, kept) > workspace_bytes) return FS_ERR_WORKSPACE_TOO_SMALL;
   HvpArgs& a = q.a;
   a.out = out;
-  if ((!kept && (rc = prepare(q.pts, q.td, 2, st)) != FS_OK) || (rc = prepare(q.dir, q.ta, 1, st)) != FS_OK) return rc;
-  hipLaunchKernelGGL((hvp_rows_kernel<0>), dim3((a.n + a.ld + 3) / 4), dim3(256), 0, st, a);
-  if ((!kept && (rc = dense_gemm(q.dots, 1, st)) != FS_OK) || (rc = dense_gemm(q.prod, 1, st)) != FS_OK) return rc;
+  if ((rc = prepare(q, kept != nullptr, st)) != FS_OK) return rc;
   if (q.td.large) hipLaunchKernelGGL((hvp_mass_kernel<8>), dim3(a.groups, a.chunks), dim3(512), 0, st, a);
   else hipLaunchKernelGGL((hvp_mass_kernel<4>), dim3(a.groups, a.chunks), dim3(256), 0, st, a);
   hipLaunchKernelGGL((hvp_merge_kernel<0>), dim3((std::max(a.n, a.m) + 63) / 64, 2), dim3(256), 0, st, a);
@@ -316,10 +337,7 @@ int run_hvp(const fs_hvp_problem* p, const Kept* kept, void* workspace, size_t w
   }
   a.vec = a.sol;
   if ((rc = strips<2>(a, st)) != FS_OK) return rc;
-  hipLaunchKernelGGL((hvp_limits_kernel<0>), dim3(1), dim3(1024), 0, st, a);
   hipLaunchKernelGGL((hvp_v_kernel<0>), dim3((a.n + 255) / 256 * 8, a.ld / 256), dim3(256), 0, st, a);
-  hipLaunchKernelGGL((hvp_yt_kernel<0>), dim3((a.ld / 16 + 3) / 4, a.yt_blocks), dim3(256), 0, st,
-                     (TransposedArgs{a.y, a.scale, a.yt, a.m, a.d, a.ld, a.dtype}));
   if ((rc = dense_gemm(q.last, 1, st)) != FS_OK) return rc;
   const int blocks = (int)std::min<size_t>(4096, ((size_t)a.n * ((a.d + 3) / 4) + 255) / 256);
   hipLaunchKernelGGL((hvp_result_kernel<0>), dim3(blocks), dim3(256), 0, st, a);

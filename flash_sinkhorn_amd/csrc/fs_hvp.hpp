@@ -24,6 +24,11 @@ struct HvpArgs {
   const float* A;
   const float* f;            // potentials with P_ij = exp((f_i + g_j - C_ij) / eps)
   const float* g;
+  const float* log_a;        // weighted: ... of a_i b_j exp(..) instead, with the weights' logarithms (null: uniform ones)
+  const float* log_b;
+  float log_n, log_m;        // of uniform weights
+  int weighted;
+  const float* out_scale;    // the result is multiplied by it, or null
   float* out;
   int n, m, d, ld, dtype;
   float eps, cs, lambda, fac_x, fac_y, floor, ridge;
@@ -64,9 +69,71 @@ struct HvpArgs {
   float* a_dir;
 };
 
-// x_i.A_i and the base-2 biases: a wavefront per row, the rows of y behind those of x.
+// The preparation of x and y (where no solve has kept it: mats = 2, else 0) and of A, each of its two launches for all
+// of them (a launch on a few blocks takes 3.5 to 4.5 us, whatever it does).
 template <int T>
-__global__ __launch_bounds__(256) void hvp_rows_kernel(const HvpArgs a) {
+__global__ __launch_bounds__(1024) void hvp_stats_kernel(const SmallArgs pts, const SmallArgs dir, int mats) {
+  if ((int)blockIdx.y < mats) dense_stats_of(pts, blockIdx.y, 0);
+  else dense_stats_of(dir, 0, 0);
+}
+template <int T>
+__global__ __launch_bounds__(512) void hvp_prep_kernel(const SmallArgs pts, const DenseArgs td, const SmallArgs dir,
+                                                       const DenseArgs ta, int mats) {
+  if ((int)blockIdx.y < mats) dense_prep_of(pts, td, blockIdx.y, 0);
+  else dense_prep_of(dir, ta, 0, 0);
+}
+
+// Planes of y^T: the rows are y's columns.  A wavefront per 32 columns and 16 points.
+struct TransposedArgs {
+  const void* y;
+  const float2* scale;  // of x, y
+  u32x4* yt;            // [column blocks][ld / 16][2][64]
+  int m, d, ld, dtype;
+};
+__device__ __forceinline__ void hvp_yt_of(const TransposedArgs& a, int blk, int kk) {
+  const int lane = threadIdx.x & 63;
+  if (kk >= a.ld / 16) return;
+  const int col = blk * 32 + (lane & 31), j0 = 16 * kk + 8 * (lane >> 5);
+  const float sc = a.scale[1].x;
+  float v[8];
+#pragma unroll
+  for (int q = 0; q < 8; ++q)
+    v[q] = col < a.d && j0 + q < a.m ? sc * small_load(a.y, (size_t)(j0 + q) * a.d + col, a.dtype) : 0.f;
+  u32x4 hi, lo;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const _Float16 h0 = (_Float16)v[2 * q], h1 = (_Float16)v[2 * q + 1];
+    hi[q] = pack_f16((float)h0, (float)h1);
+    lo[q] = pack_f16(v[2 * q] - (float)h0, v[2 * q + 1] - (float)h1);
+  }
+  u32x4* out = a.yt + ((size_t)blk * (a.ld / 16) + kk) * kDenseStep + lane;
+  out[0] = hi;
+  out[64] = lo;
+}
+template <int T>
+__global__ __launch_bounds__(256) void hvp_yt_kernel(const TransposedArgs a) {
+  hvp_yt_of(a, blockIdx.y, blockIdx.x * 4 + (threadIdx.x >> 6));
+}
+
+// A potential in the convention of the product, from one that leaves the weight to the plan (no weight, or one below
+// zero: a logarithm of -100,000).
+__device__ __forceinline__ float hvp_potential(const HvpArgs& a, const float* pot, const float* log_w, float uniform, int i) {
+#pragma clang fp contract(off)  // (the number that a caller would hand over otherwise)
+  if (!a.weighted) return pot[i];
+  const float l = log_w == nullptr ? uniform : log_w[i], t = a.eps * (l > -__builtin_inff() ? l : -100000.0f);
+  return pot[i] + t;
+}
+
+// x_i.A_i and the base-2 biases: a wavefront per row, the rows of y behind those of x.  Behind them the planes of y^T,
+// which the last product reads (by itself that launch took 5.4 us at 2,048 x 64).
+template <int T>
+__global__ __launch_bounds__(256) void hvp_rows_kernel(const HvpArgs a, const TransposedArgs t) {
+  const int row_blocks = (a.n + a.ld + 3) / 4;
+  if ((int)blockIdx.x >= row_blocks) {
+    const int b = blockIdx.x - row_blocks, per = (t.ld / 16 + 3) / 4;
+    hvp_yt_of(t, b / per, b % per * 4 + (threadIdx.x >> 6));
+    return;
+  }
   const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   const float k = kLog2e / a.eps;
   if (row < a.n) {
@@ -77,11 +144,11 @@ __global__ __launch_bounds__(256) void hvp_rows_kernel(const HvpArgs a) {
     for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
     if (lane == 0) {
       a.xa[row] = s;
-      a.ra[row] = k * (a.f[row] - a.norm_x[row]);
+      a.ra[row] = k * (hvp_potential(a, a.f, a.log_a, a.log_n, row) - a.norm_x[row]);
     }
   } else if (row - a.n < a.ld && lane == 0) {
     const int j = row - a.n;
-    a.cb[j] = j < a.m ? k * (a.g[j] - a.norm_y[j]) : kNegBig;
+    a.cb[j] = j < a.m ? k * (hvp_potential(a, a.g, a.log_b, a.log_m, j) - a.norm_y[j]) : kNegBig;
   }
 }
 
@@ -186,13 +253,30 @@ __global__ __launch_bounds__(256) void hvp_merge_kernel(const HvpArgs a) {
   }
 }
 
+// Largest |z| and |y_j|, for the scales of V's rows, by a workgroup of 512 threads.
+__device__ __forceinline__ void hvp_limits(const HvpArgs& a) {
+  float z = 0.f, y = 0.f;
+  for (int j = threadIdx.x; j < a.m; j += 512) z = fmaxf(z, fabsf(a.sol[j])), y = fmaxf(y, a.norm_y[j]);
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) z = fmaxf(z, __shfl_xor(z, o, 64)), y = fmaxf(y, __shfl_xor(y, o, 64));
+  __shared__ float sh[2][8];
+  if ((threadIdx.x & 63) == 0) sh[0][threadIdx.x >> 6] = z, sh[1][threadIdx.x >> 6] = y;
+  __syncthreads();
+  if (threadIdx.x > 0) return;
+  for (int w = 1; w < 8; ++w) z = fmaxf(z, sh[0][w]), y = fmaxf(y, sh[1][w]);
+  a.limits[0] = z;
+  a.limits[1] = sqrtf(y / a.cs);
+}
+
 // Whole rows of the plan in registers: a workgroup owns `strip_rows` rows, R at a time, its 512
 // threads 4 CP columns each.  MODE 0: column sums of P_ij w_i; 1: the same with w = P vec / diag_x, so
 // that one reading serves both products of a Schur-complement step; 2: P vec alone, and what the
-// result needs of it.  Bound by memory; the next R rows are in flight while the sums cross the workgroup.
+// result needs of it; one workgroup more finds hvp_limits.  Bound by memory; the next R rows are in flight while the
+// sums cross the workgroup.
 template <int CP, int R, int MODE>
 __global__ __launch_bounds__(512, 2) void hvp_strip_kernel(const HvpArgs a) {
   if (MODE == 1 && a.cg[4] != 0.f) return;  // converged: what was enqueued behind it does nothing
+  if (MODE == 2 && (int)blockIdx.x == a.strips) return hvp_limits(a);
   __shared__ float sh[2][8][R];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int first = blockIdx.x * a.strip_rows, last = min(a.n, first + a.strip_rows);
@@ -311,22 +395,6 @@ __global__ __launch_bounds__(256) void hvp_columns_kernel(const HvpArgs a) {
   a.a_dir[col] = MODE == 0 ? a.r2[col] - t : __builtin_fmaf(a.denom[col], a.vec[col], -t);
 }
 
-// Largest |z| and |y_j|, for the scales of V's rows.
-template <int T>
-__global__ __launch_bounds__(1024) void hvp_limits_kernel(const HvpArgs a) {
-  float z = 0.f, y = 0.f;
-  for (int j = threadIdx.x; j < a.m; j += 1024) z = fmaxf(z, fabsf(a.sol[j])), y = fmaxf(y, a.norm_y[j]);
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) z = fmaxf(z, __shfl_xor(z, o, 64)), y = fmaxf(y, __shfl_xor(y, o, 64));
-  __shared__ float sh[2][16];
-  if ((threadIdx.x & 63) == 0) sh[0][threadIdx.x >> 6] = z, sh[1][threadIdx.x >> 6] = y;
-  __syncthreads();
-  if (threadIdx.x > 0) return;
-  for (int w = 1; w < 16; ++w) z = fmaxf(z, sh[0][w]), y = fmaxf(y, sh[1][w]);
-  a.limits[0] = z;
-  a.limits[1] = sqrtf(y / a.cs);
-}
-
 // Power of two that takes a row of V below 2^15 (f16_plane_scale without its clamp at 2^40: the
 // plan of a cloud with many points is small).
 __device__ __forceinline__ float hvp_scale(float most) {
@@ -384,35 +452,6 @@ __global__ __launch_bounds__(256) void hvp_v_kernel(const HvpArgs a) {
     const int kk = w >> 7, plane = (w >> 6) & 1, half = (w >> 5) & 1, i = w & 31;
     out[w] = *reinterpret_cast<const u32x4*>(lds + (plane * 32 + kk * 2 + half) * UNIT + i * 16);
   }
-}
-
-// Planes of y^T: the rows are y's columns.  A wavefront per 32 columns and 16 points.
-struct TransposedArgs {
-  const void* y;
-  const float2* scale;  // of x, y
-  u32x4* yt;            // [column blocks][ld / 16][2][64]
-  int m, d, ld, dtype;
-};
-template <int T>
-__global__ __launch_bounds__(256) void hvp_yt_kernel(const TransposedArgs a) {
-  const int blk = blockIdx.y, kk = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-  if (kk >= a.ld / 16) return;
-  const int col = blk * 32 + (lane & 31), j0 = 16 * kk + 8 * (lane >> 5);
-  const float sc = a.scale[1].x;
-  float v[8];
-#pragma unroll
-  for (int q = 0; q < 8; ++q)
-    v[q] = col < a.d && j0 + q < a.m ? sc * small_load(a.y, (size_t)(j0 + q) * a.d + col, a.dtype) : 0.f;
-  u32x4 hi, lo;
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const _Float16 h0 = (_Float16)v[2 * q], h1 = (_Float16)v[2 * q + 1];
-    hi[q] = pack_f16((float)h0, (float)h1);
-    lo[q] = pack_f16(v[2 * q] - (float)h0, v[2 * q + 1] - (float)h1);
-  }
-  u32x4* out = a.yt + ((size_t)blk * (a.ld / 16) + kk) * kDenseStep + lane;
-  out[0] = hi;
-  out[64] = lo;
 }
 
 // The gradient in x of a solve whose products are kept:
@@ -549,6 +588,7 @@ template <int T>
 __global__ __launch_bounds__(256) void hvp_result_kernel(const HvpArgs a) {
   const unsigned quads = (unsigned)(a.d + 3) / 4, count = (unsigned)a.n * quads;  // (at most 65,536 x 4,096)
   const bool wx = hvp_wide(a.x, a.d, a.dtype), wa = hvp_wide(a.A, a.d, 0), wo = hvp_wide(a.out, a.d, 0);
+  const float gs = a.out_scale == nullptr ? 1.0f : *a.out_scale;
   for (unsigned i = blockIdx.x * 256 + threadIdx.x; i < count; i += gridDim.x * 256) {
     const unsigned row = i / quads;
     const int col = 4 * (int)(i - row * quads), left = a.d - col;
@@ -557,8 +597,8 @@ __global__ __launch_bounds__(256) void hvp_result_kernel(const HvpArgs a) {
     const float4 v = hvp_parts(a.prod_out + (size_t)row * a.ldo + col, (size_t)a.n * a.ldo, a.splits);
     const float k = a.scale[1].y / a.v_scale[row], s = a.s[row], w = 2.0f * a.cs * a.mass[row];
     hvp_store4(a.out, e,
-               make_float4(s * x.x + w * A.x + v.x * k, s * x.y + w * A.y + v.y * k, s * x.z + w * A.z + v.z * k,
-                           s * x.w + w * A.w + v.w * k),
+               make_float4(gs * (s * x.x + w * A.x + v.x * k), gs * (s * x.y + w * A.y + v.y * k),
+                           gs * (s * x.z + w * A.z + v.z * k), gs * (s * x.w + w * A.w + v.w * k)),
                wo, left);
   }
 }

@@ -80,7 +80,7 @@ class _Problem(ctypes.Structure):
     _fields_ = [("x", _P), ("y", _P), ("A", _P), ("f", _P), ("g", _P), ("n", _I64), ("m", _I64),
                 ("d", _I64), ("eps", _F), ("cost_scale", _F), ("rho_x", _F), ("rho_y", _F),
                 ("tau2", _F), ("lambda_indef", _F), ("rtol", _F), ("atol", _F), ("dtype", _I),
-                ("max_iter", _I)]
+                ("max_iter", _I), ("log_a", _P), ("log_b", _P), ("out_scale", _P), ("weighted", _I)]
 
 
 _DTYPES = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}
@@ -103,10 +103,17 @@ def _kept_ok(x, y, f_hat, g_hat, A, allow_tf32: bool) -> bool:
             and not torch.cuda.is_current_stream_capturing())
 
 
+def _rest_ok(weights, scale, x, y) -> bool:
+    return ((weights is None or all(w is None or (w.device == x.device and w.shape == (t.shape[0],))
+                                    for w, t in zip(weights, (x, y))))
+            and (scale is None or (scale.device == x.device and scale.ndim == 0)))
+
+
 def _kept(x, y, f_hat, g_hat, A, *, eps, cost_scale, rho_x, rho_y, tau2, lambda_indef, rtol, atol,
-          max_iter, products=None):
+          max_iter, products=None, weights=None, scale=None):
     """One library call: three contractions, the rest passes over kept matrices.  ``products``: those that
-    the solve of the same points has kept, so that two contractions are left."""
+    the solve of the same points has kept, so that two contractions are left.  ``weights``, ``scale``: see
+    ``hvp_x_sqeuclid_from_potentials``."""
     if products is not None:
         x, y = products.x, products.y
     if x.dtype not in _DTYPES or y.dtype is not x.dtype:
@@ -121,6 +128,12 @@ def _kept(x, y, f_hat, g_hat, A, *, eps, cost_scale, rho_x, rho_y, tau2, lambda_
                  eps, cost_scale, 0.0 if rho_x is None else float(rho_x),
                  0.0 if rho_y is None else float(rho_y), tau2, lambda_indef, rtol, atol,
                  _DTYPES[x.dtype], max(0, max_iter))
+    if weights is not None:
+        log_a, log_b = (None if w is None else w.detach().float().log().contiguous() for w in weights)
+        p.log_a, p.log_b, p.weighted = _lib.ptr(log_a), _lib.ptr(log_b), 1
+    if scale is not None:
+        scale = scale.detach().float()
+        p.out_scale = scale.data_ptr()
     L = _lib.lib()
     size = L.fs_hvp_workspace_bytes if products is None else L.fs_hvp_solved_workspace_bytes
     ws = torch.empty(size(ctypes.byref(p)), dtype=torch.uint8, device=x.device)
@@ -147,7 +160,7 @@ def hvp_x_sqeuclid_from_potentials(
     block_m=None, block_n=None, block_k=None, num_warps: int = 4, num_stages: int = 2,
     use_fused_matvec: bool = False, use_batched_cg: bool = False, use_compiled_cg: bool = False,
     use_dense_cg: bool = False, autotune: bool = True, cg_x0: Optional[torch.Tensor] = None,
-    _products=None,
+    _products=None, _weights=None, _scale=None,
 ):
     """H @ A for OTT-convention potentials (f_hat, g_hat); returns (hvp [n,d], HvpInfo).
 
@@ -156,6 +169,9 @@ def hvp_x_sqeuclid_from_potentials(
     regularisation is added.  ``preconditioner``: "none" solves
     ``denom*z - P^T((Pz)/diag_x) = rhs``; "neumann"/"jacobi" solve ``z - Bz = rhs/denom``
     (Neumann adds ``precond_terms`` terms of the series as M^-1).
+
+    For the backward pass of a loss: with ``_weights`` (of the points, None: uniform) the potentials are those
+    of ``a b exp((f+g-C)/eps)``, and the product is multiplied by the tensor ``_scale``.
     """
     if x.ndim != 2 or y.ndim != 2 or A.ndim != 2:
         raise ValueError("x,y,A must be 2D tensors.")
@@ -178,10 +194,16 @@ def hvp_x_sqeuclid_from_potentials(
     e = float(eps)
     cs = float(cost_scale)
     if (mode == "none" and cg_x0 is None and not cg_stabilise_every and not return_components
-            and _kept_ok(x, y, f_hat, g_hat, A, allow_tf32) and _small.held(e, cs, rho_x, rho_y)):
+            and _kept_ok(x, y, f_hat, g_hat, A, allow_tf32) and _small.held(e, cs, rho_x, rho_y)
+            and _rest_ok(_weights, _scale, x, y)):
         return _kept(x, y, f_hat, g_hat, A, eps=e, cost_scale=cs, rho_x=rho_x, rho_y=rho_y,
                      tau2=float(tau2), lambda_indef=float(lambda_indef), rtol=float(cg_rtol),
-                     atol=float(cg_atol), max_iter=int(max_cg_iter), products=_products)
+                     atol=float(cg_atol), max_iter=int(max_cg_iter), products=_products,
+                     weights=_weights, scale=_scale)
+    if _weights is not None:
+        a, b = (torch.full((rows,), 1.0 / rows, device=x.device, dtype=torch.float32) if w is None else w
+                for w, rows in zip(_weights, (n, m)))
+        f_hat, g_hat = geomloss_to_ott_potentials(f_hat, g_hat, a, b, eps=e)
     xf, yf, Af = x.float().contiguous(), y.float().contiguous(), A.float().contiguous()
     x_sq = (xf * xf).sum(dim=1).contiguous()
     y_sq = (yf * yf).sum(dim=1).contiguous()
@@ -277,7 +299,8 @@ def hvp_x_sqeuclid_from_potentials(
                    float(cg.cg_initial_residual))
     if return_components:
         return psd, indef, info
-    return (psd + indef if lambda_indef == 1.0 else psd + lambda_indef * indef), info
+    hvp = psd + indef if lambda_indef == 1.0 else psd + lambda_indef * indef
+    return (hvp if _scale is None else hvp * _scale), info
 
 
 def hvp_x_sqeuclid(

@@ -497,6 +497,10 @@ typedef struct fs_hvp_problem {
   int64_t n, m, d;
   float eps, cost_scale, rho_x, rho_y, tau2, lambda_indef, rtol, atol;
   int dtype, max_iter;
+  const float* log_a;     /* where `weighted`: [n], [m] logarithms of the points' weights, null: uniform ones */
+  const float* log_b;
+  const float* out_scale; /* [1] on the device: the result times it; null: as it is */
+  int weighted;           /* P_ij = a_i b_j exp(..) instead */
 } fs_hvp_problem;
 
 size_t fs_hvp_workspace_bytes(const fs_hvp_problem* problem);

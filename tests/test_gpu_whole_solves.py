@@ -1055,6 +1055,30 @@ def test_kept_hvp(n, m, d, rho):
             assert info.cg_iters == iters
 
 
+# Potentials that leave the weights to the plan (uniform ones need no tensor; a point without mass), and a scaled result:
+# the same numbers, formed by the kernel that reads the potentials and by the last one.
+@pytest.mark.parametrize("n,m,d", [(1, 1, 1), (130, 257, 5), (65, 2049, 129), (2047, 300, 64)])
+@pytest.mark.parametrize("uniform", [(False, False), (True, False), (False, True), (True, True)])
+def test_kept_hvp_of_weighted_plans(n, m, d, uniform):
+    from flash_sinkhorn_amd.hvp import geomloss_to_ott_potentials, hvp_x_sqeuclid_from_potentials as hvp
+    x, y, a, b = inputs(n + d, n, m, d, scale=1.0 / np.sqrt(d))
+    a, b = (np.full_like(w, 1.0 / len(w)) if u else w for w, u in zip((a, b), uniform))
+    if n > 100 and not uniform[0]:
+        a[3] = 0.0
+    f, g = oracle.sinkhorn_symmetric(x, y, a, b, use_epsilon_scaling=False, eps=0.25, n_iters=5)
+    X, Y, A, B, F, G = dev(x, y, a, b, f.astype(np.float32), g.astype(np.float32))
+    V = dev(np.random.default_rng(1).standard_normal((n, d)).astype(np.float32))[0]
+    kw = dict(eps=0.25, cg_rtol=1e-5, cg_atol=1e-12, preconditioner="none")
+    scale = torch.tensor(-1.7, device="cuda")
+    want, _ = hvp(X, Y, *geomloss_to_ott_potentials(F, G, A, B, eps=0.25), V, **kw)
+    got, _ = hvp(X, Y, F, G, V, _weights=tuple(None if u else w for u, w in zip(uniform, (A, B))), _scale=scale, **kw)
+    if not any(uniform):
+        assert torch.equal(got, want * scale)
+    # (the logarithm of a uniform weight is the host's, 1e-7 of its 8 or less, and so 1e-7 of any entry of the plan: as far as
+    # conjugate gradients to 1e-5 take that)
+    assert rel_err(got, (want * scale).cpu().numpy()) < 2e-4
+
+
 @pytest.mark.parametrize("n,m,d", [(37, 300, 64), (65, 130, 5), (100, 257, 136)])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_kept_hvp_of_half_precision_points(n, m, d, dtype):
