@@ -656,6 +656,10 @@ int fs_small_solve_products(const fs_small_problem* p, void* workspace, size_t w
       return true;
     });
     if (rc != FS_OK) return rc;
+    for (int i = 0; i < a.items; ++i) {  // (see small_schedule)
+      const int lens = __atomic_load_n(host_words + 4 * i + 2, __ATOMIC_RELAXED);
+      for (int q = 0; q < 3; ++q) __atomic_store_n(host_words + 4 * i + q, (lens >> (10 * q) & 1023) - 3, __ATOMIC_RELAXED);
+    }
     entries = 0;
     for (int i = 0; i < a.items; ++i)
       for (int q = p0; q < p1; ++q) {

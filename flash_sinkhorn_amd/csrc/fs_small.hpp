@@ -189,33 +189,63 @@ __device__ __forceinline__ float small_log2(float v, float c) {
 __device__ void small_schedule(const SmallArgs& a, int item) {
   const int tid = threadIdx.x;
   __shared__ float sq[3];
-  __shared__ int len[3];
+  __shared__ int len[3], full[3];
   if (a.sched == 0 && tid < 3) {  // one entry stands for all
     a.lens[item * 3 + tid] = a.full[item * 3 + tid] = a.entries;
     a.table[((size_t)item * 3 + tid) * a.table_len] = small_coef(a.cost_scale, a.eps0);
   }
   if (a.sched != 1 && !a.pair) return;
+  // The partial results, all on their way at once: of the boxes up to sixteen threads a column, whose minima and maxima
+  // meet in LDS (a thread a column, sixteen blocks at a time, was eight round trips; with the logarithms below side by side and no
+  // fence the kernel went from 9.4 to 8.2 us at 256 points, 16.0 to 10.1 at 4,567 and 20.5 to 14.4 at 30,011; it takes
+  // 4.3 where there is no schedule).
+  const int wave_lane = tid & 63;
+  float4 part[2];
+  if (a.pair && tid < 64) {
+#pragma unroll
+    for (int mat = 0; mat < 2; ++mat) {
+      const float* st = a.stats + (((size_t)item * 2 + mat) * a.stat_blocks + (tid < a.stat_blocks ? tid : 0)) * a.stat_words;
+      part[mat] = make_float4(st[0], st[1], st[2], st[3]);
+    }
+  }
+  __shared__ float box[2][2][256];
+  const int groups = min(16, 256 / a.d), group = tid / a.d, col = tid - group * a.d;
   if (tid < 3) sq[tid] = 0.f;
+  if (group < groups) {
+#pragma unroll
+    for (int mat = 0; mat < 2; ++mat) {
+      const float* st = a.stats + ((size_t)item * 2 + mat) * a.stat_blocks * a.stat_words + 4 + col;
+      float lo = 3.0e38f, hi = -3.0e38f;
+      for (int b0 = group; b0 < a.stat_blocks; b0 += 8 * groups) {  // (eight on their way, the last one again)
+        float l[8], u[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+          const float* at = st + (size_t)min(b0 + k * groups, a.stat_blocks - 1) * a.stat_words;
+          l[k] = at[0];
+          u[k] = at[a.d];
+        }
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+          lo = (l[k] < lo || !(l[k] == l[k])) ? l[k] : lo;
+          hi = (u[k] > hi || !(u[k] == u[k])) ? u[k] : hi;
+        }
+      }
+      box[mat][0][tid] = lo;
+      box[mat][1][tid] = hi;
+    }
+  }
   __syncthreads();
   float r[3] = {0.f, 0.f, 0.f};
   if (tid < a.d) {
     float lo[2] = {3.0e38f, 3.0e38f}, hi[2] = {-3.0e38f, -3.0e38f};
 #pragma unroll
     for (int mat = 0; mat < 2; ++mat)
-      for (int b0 = 0; b0 < a.stat_blocks; b0 += 16) {  // (sixteen loads on their way, the last one again)
-        float l[16], u[16];
 #pragma unroll
-        for (int k = 0; k < 16; ++k) {
-          const int b = min(b0 + k, a.stat_blocks - 1);
-          const float* st = a.stats + (((size_t)item * 2 + mat) * a.stat_blocks + b) * a.stat_words + 4 + tid;
-          l[k] = st[0];
-          u[k] = st[a.d];
-        }
-#pragma unroll
-        for (int k = 0; k < 16; ++k) {
-          lo[mat] = (l[k] < lo[mat] || !(l[k] == l[k])) ? l[k] : lo[mat];
-          hi[mat] = (u[k] > hi[mat] || !(u[k] == u[k])) ? u[k] : hi[mat];
-        }
+      for (int g = 0; g < 16; ++g) {
+        const int at = tid + min(g, groups - 1) * a.d;
+        const float l = box[mat][0][at], u = box[mat][1][at];
+        lo[mat] = (l < lo[mat] || !(l == l)) ? l : lo[mat];
+        hi[mat] = (u > hi[mat] || !(u == u)) ? u : hi[mat];
       }
     const float e0 = (lo[0] < lo[1] || !(lo[0] == lo[0]) ? lo[0] : lo[1]);
     const float e1 = (hi[0] > hi[1] || !(hi[0] == hi[0]) ? hi[0] : hi[1]);
@@ -236,8 +266,7 @@ __device__ void small_schedule(const SmallArgs& a, int item) {
 #pragma unroll
     for (int mat = 0; mat < 2; ++mat) {
       const bool live = tid < a.stat_blocks;
-      const float* st = a.stats + (((size_t)item * 2 + mat) * a.stat_blocks + (live ? tid : 0)) * a.stat_words;
-      float m = st[0], ws = live ? st[1] : 0.f, wl = st[2], wh = st[3];
+      float m = part[mat].x, ws = live ? part[mat].y : 0.f, wl = part[mat].z, wh = part[mat].w;
 #pragma unroll
       for (int o = 32; o > 0; o >>= 1) {
         m = fmaxf(m, __shfl_xor(m, o, 64));
@@ -260,39 +289,51 @@ __device__ void small_schedule(const SmallArgs& a, int item) {
     }
   }
   if (a.sched != 1) return;
-  if (tid < 3) {
-    const double D = (double)sqrtf(sq[tid]);
-    int k = -2;                      // not a number
-    if (D <= 0.0) k = -1;            // one point
-    else if (D < 3.0e38) {
-      const double start = 2.0 * log(D), stop = 2.0 * log(a.blur), step = 2.0 * log(a.scaling);
-      const double cnt = ceil((stop - start) / step);
-      const double total = 2.0 + (cnt > 0.0 ? cnt : 0.0);
-      k = total > (double)(kSmallTable - 1) ? -3 : (int)total;  // -3: longer than the table
-      if (k > 0 && a.cut > 0) k = min(k, a.cut);
-      if (k >= a.table_len) k = -3;
+  __shared__ double from[3], per_step;
+  if (tid < 64) {  // one logarithm a lane: of the diameters, of the end and of a step
+    const double D = (double)sqrtf(sq[min(tid, 2)]);
+    const double twice = 2.0 * log(wave_lane == 3 ? a.blur : (wave_lane == 4 ? a.scaling : D));
+    const double stop = __shfl(twice, 3, 64), step = __shfl(twice, 4, 64);
+    if (tid < 3) {
+      int k = -2;                      // not a number
+      if (D <= 0.0) k = -1;            // one point
+      else if (D < 3.0e38) {
+        const double cnt = ceil((stop - twice) / step);
+        const double total = 2.0 + (cnt > 0.0 ? cnt : 0.0);
+        k = total > (double)(kSmallTable - 1) ? -3 : (int)total;  // -3: longer than the table
+        full[tid] = k;
+        if (k > 0 && a.cut > 0) k = min(k, a.cut);
+        if (k >= a.table_len) k = -3;
+      }
+      len[tid] = k;
+      from[tid] = twice;
+      if (tid == 0) per_step = step;
+      a.lens[item * 3 + tid] = k;
+      a.full[item * 3 + tid] = k;
     }
-    len[tid] = k;
-    a.lens[item * 3 + tid] = k;
-    a.full[item * 3 + tid] = k;
-    __hip_atomic_store(a.host_words + item * 4 + tid, k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   }
   __syncthreads();
-  if (tid == 0) {  // (the same wavefront wrote the three words)
-    __threadfence_system();
-    __hip_atomic_store(a.host_words + item * 4 + 3, a.host_token, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-  }
-  for (int p = 0; p < 3; ++p) {
-    const double D = (double)sqrtf(sq[p]);
-    if (len[p] <= 0) continue;
-    const double start = 2.0 * log(D), stop = 2.0 * log(a.blur), step = 2.0 * log(a.scaling);
-    const double cnt = ceil((stop - start) / step);
-    const int full = 2 + (cnt > 0.0 ? (int)cnt : 0);
-    for (int i = tid; i <= len[p]; i += 256) {
-      const int c = min(i, len[p] - 1);
-      const double e = c == 0 ? D * D : (c == full - 1 ? a.blur * a.blur : exp(start + (c - 1) * step));
-      a.table[((size_t)item * 3 + p) * a.table_len + i] = small_coef(a.cost_scale, (float)e);
+  // One store, so that nothing has to be ordered (a fence in front of the token writes back an L2): three lengths in
+  // one word, ten bits each from -3 up, and the token in the next.
+  if (tid == 0) {
+    const unsigned lens = (unsigned)(len[0] + 3) | (unsigned)(len[1] + 3) << 10 | (unsigned)(len[2] + 3) << 20;
+    int* words = a.host_words + item * 4 + 2;
+    if ((reinterpret_cast<size_t>(words) & 7) == 0) {
+      __hip_atomic_store(reinterpret_cast<unsigned long long*>(words), (unsigned long long)(unsigned)a.host_token << 32 | lens,
+                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    } else {  // (words of a caller that are only aligned as such)
+      __hip_atomic_store(words, (int)lens, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      __threadfence_system();
+      __hip_atomic_store(words + 1, a.host_token, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
+  }
+  const int n0 = max(0, len[0] + (len[0] > 0)), n1 = max(0, len[1] + (len[1] > 0)), n2 = max(0, len[2] + (len[2] > 0));
+  for (int k = tid; k < n0 + n1 + n2; k += 256) {  // (the entries of all three)
+    const int p = k < n0 ? 0 : (k < n0 + n1 ? 1 : 2), i = k - (p == 0 ? 0 : (p == 1 ? n0 : n0 + n1));
+    const double D = (double)sqrtf(sq[p]);
+    const int c = min(i, len[p] - 1);
+    const double e = c == 0 ? D * D : (c == full[p] - 1 ? a.blur * a.blur : exp(from[p] + (c - 1) * per_step));
+    a.table[((size_t)item * 3 + p) * a.table_len + i] = small_coef(a.cost_scale, (float)e);
   }
 }
 
@@ -335,18 +376,26 @@ __global__ __launch_bounds__(256) void small_prep_kernel(const SmallArgs a, cons
   const int rb = blockIdx.x, rows = a.rows[mat], d = a.d;
   if (rb >= a.blocks[mat]) return;
   __shared__ float s[32 * LDW];
+  // (the points are on their way beside the statistics)
+  const int r0 = rb * 32;
+  const size_t base = ((size_t)item * rows + r0) * d;
+  float point[DP / 8];
+#pragma unroll
+  for (int k = 0; k < DP / 8; ++k) {
+    const int e = min(tid + 256 * k, (min(32, rows - r0) * d) - 1);
+    point[k] = small_load(a.pts[mat], base + e, a.dtype);
+  }
   float am, ws;
   small_merge_stats(a, item, mat, am, ws);
   const float sc = f16_plane_scale(am);
   if (rb == 0 && tid == 0) a.scale[item * 2 + mat] = make_float2(sc, 1.0f / sc);
-  const int r0 = rb * 32;
   if (d < NDB * 32)
     for (int e = tid; e < 32 * LDW; e += 256) s[e] = 0.f;
   __syncthreads();
-  const size_t base = ((size_t)item * rows + r0) * d;
-  for (int e = tid; e < 32 * d; e += 256) {
-    const int r = e / d;
-    s[r * LDW + (e - r * d)] = r0 + r < rows ? sc * small_load(a.pts[mat], base + e, a.dtype) : 0.f;
+#pragma unroll
+  for (int k = 0; k < DP / 8; ++k) {
+    const int e = tid + 256 * k, r = e / d;
+    if (e < 32 * d) s[r * LDW + (e - r * d)] = r0 + r < rows ? sc * point[k] : 0.f;
   }
   __syncthreads();
   // planes
@@ -669,28 +718,52 @@ __global__ __launch_bounds__(1024) void small_loss_kernel(const SmallArgs a, con
   const int item = blockIdx.y, part = blockIdx.x, tid = threadIdx.x;
   float total = 0.f;
   size_t off = a.self == 2 ? 2 * (size_t)a.items * (a.rows[0] + a.rows[1]) : 0;
-  const int sides = a.self ? 4 : 2;
-  for (int side = a.self == 2 ? 2 : 0; side < sides; ++side) {
+  const int first = a.self == 2 ? 2 : 0, sides = a.self ? 4 : 2;
+  // What a thread's first row of every side needs is loaded before the first sum, both potentials for the one that the
+  // schedule's length names (each side a chain of its own: 7.5 us at 2,000 points debiased, now 4.8).
+  struct Row {
+    float norm, weight, pot[2];
+  };
+  auto load = [&](int side, int i) {
     const int mat = side & 1, rows = a.rows[mat];
-    const int prob = side < 2 ? 0 : side - 1;
-    const int last = a.lens[item * 3 + prob] + 1 + a.extrapolate;
-    const float eps_last = small_last_coef(a, item, prob).x;
+    const size_t half = (size_t)a.items * rows, at = (size_t)item * rows + min(i, rows - 1);
+    return Row{a.norm[mat][at], a.wt[mat][at], {a.pot[side][at], a.pot[side][half + at]}};
+  };
+  Row row[4];
+  int lens[4];
+  float eps_last[4];
+  const int i0 = part * 1024 + tid;
+#pragma unroll
+  for (int side = 0; side < 4; ++side)
+    if (side >= first && side < sides) {
+      const int prob = side < 2 ? 0 : side - 1;
+      row[side] = load(side, i0);
+      lens[side] = a.lens[item * 3 + prob];
+      eps_last[side] = l.relaxed ? small_last_coef(a, item, prob).x : 0.f;
+    }
+#pragma unroll
+  for (int side = 0; side < 4; ++side) {
+    if (side < first || side >= sides) continue;
+    const int mat = side & 1, rows = a.rows[mat];
+    const int last = (lens[side] + 1 + a.extrapolate) & 1;
     const size_t half = (size_t)a.items * rows;
     const float rho = a.rho[mat];
     // (a self problem has this potential twice: its cost is 2 <a, f>)
     const float sign = side < 2 ? 1.0f : -1.0f;
     float sum = 0.f;
-    for (int i = part * 1024 + tid; i < rows; i += 1024 * gridDim.x) {
+    Row v = row[side];
+    for (int i = i0; i < rows;) {
       const size_t at = (size_t)item * rows + i;
-      const float al = a.norm[mat][at];
-      const float f = a.pot[side][(last & 1) * half + at] + al;
+      const float f = (last ? v.pot[1] : v.pot[0]) + v.norm;
       if (l.pots != nullptr) {
         l.pots[off + at] = f;
-        l.pots[off + half + at] = a.extrapolate ? a.pot[side][((last & 1) ^ 1) * half + at] + al : f;
+        l.pots[off + half + at] = a.extrapolate ? (last ? v.pot[0] : v.pot[1]) + v.norm : f;
       }
-      sum += a.wt[mat][at] * (l.relaxed ? 1.0f - expf(-f / rho) : f);
+      sum += v.weight * (l.relaxed ? 1.0f - expf(-f / rho) : f);
+      i += 1024 * gridDim.x;
+      if (i < rows) v = load(side, i);
     }
-    if (l.relaxed) sum *= rho + 0.5f * eps_last;
+    if (l.relaxed) sum *= rho + 0.5f * eps_last[side];
     total += sign * sum;
     off += 2 * half;
   }
@@ -770,14 +843,18 @@ __global__ __launch_bounds__(512, 2) void small_grad_kernel(const SmallArgs a, c
 #pragma unroll
   for (int i = 0; i < PER; ++i) bary[i] = 0.f;
 
+  // (what either pass starts from is on its way before the first one)
+  const int len0 = a.lens[item * 3], len1 = a.self ? a.lens[item * 3 + 1 + qm] : 0;
+  const float4 coef0 = small_last_coef(a, item, 0), coef1 = a.self ? small_last_coef(a, item, 1 + qm) : coef0;
+  const float2 sq = a.scale[item * 2 + qm], other = a.scale[item * 2 + (qm ^ 1)];
   for (int pass = 0; pass <= a.self; ++pass) {
     const int km = pass == 0 ? qm ^ 1 : qm;
     const int kside = pass == 0 ? km : 2 + km;
     const int prob = pass == 0 ? 0 : 1 + km;
     const int nk = a.rows[km], nkb = a.blocks[km];
-    const int last = a.lens[item * 3 + prob] + 1;  // (the step before the extrapolation)
-    const float4 coef = small_last_coef(a, item, prob);
-    const float2 sq = a.scale[item * 2 + qm], sk = a.scale[item * 2 + km];
+    const int last = (pass == 0 ? len0 : len1) + 1;  // (the step before the extrapolation)
+    const float4 coef = pass == 0 ? coef0 : coef1;
+    const float2 sk = pass == 0 ? other : sq;
     const u32x4* qp = pass == 0 || a.self_planes[qm] == nullptr ? a.planes[qm] : a.self_planes[qm];
     const u32x4* kp = pass == 0 || a.self_planes[km] == nullptr ? a.planes[km] : a.self_planes[km];
     if (pass == 0 || qp != a.planes[qm]) {

@@ -61,6 +61,48 @@ def test_schedules_of_every_length(n, m, d, cut):
 
 # ---- wide rows, one launch per step (up to 1e7 products and 4,096 keys): one and two rows a wavefront, pieces
 # of 1,024 keys, and the sizes just past the line ----
+# lengths of schedules, from boxes whose farthest corner lies in one block of rows and one column of either cloud (up to
+# 64 blocks, sixteen threads a column or as many as 256 hold)
+@pytest.mark.parametrize("n,m,d", [(2, 3, 1), (40, 33, 2), (300, 65, 3), (513, 290, 15), (260, 545, 16), (1100, 2049, 17),
+                                   (2080, 700, 33), (90, 1000, 85), (333, 2100, 86), (2050, 100, 128), (4600, 4500, 5)])
+def test_lengths_of_schedules(n, m, d):
+    from flash_sinkhorn_amd import SamplesLoss, _small
+    rng = np.random.default_rng(n + d)
+    base = [rng.uniform(-1, 1, (rows, d)).astype(np.float32) for rows in (n, m)]
+    for cloud, row, col, far in [(0, 0, 0, 40.0), (0, -1, -1, -90.0), (1, 0, -1, 200.0), (1, -1, 0, -17.0), (0, n // 2, d // 2, 70.0)]:
+        pts = [p.copy() for p in base]
+        pts[cloud][row, col] = far
+        boxes = [(p.min(0), p.max(0)) for p in pts]
+        joint = (np.minimum(boxes[0][0], boxes[1][0]), np.maximum(boxes[0][1], boxes[1][1]))
+        # (rounded otherwise than on the device by 2^-20 at most: a length that this changes would be seen as another seed's)
+        diameters = [float(np.sqrt(((hi - lo).astype(np.float64) ** 2).sum())) for lo, hi in [joint] + boxes]
+        want = [2 + max(0, int(np.ceil(2 * np.log(0.05 / D) / (2 * np.log(0.5))))) for D in diameters]
+        loss = SamplesLoss(blur=0.05, scaling=0.5, debias=True)(*dev(*pts))
+        assert torch.isfinite(loss) and _small._host_words(1)[:3].tolist() == want
+
+
+# sums over one to several rows a thread and workgroup, of every combination of sides
+@pytest.mark.parametrize("n,m", [(1, 1025), (1024, 3), (1030, 2049), (3073, 3072), (4500, 1000)])
+@pytest.mark.parametrize("reach", [None, 1.3])
+@pytest.mark.parametrize("debias", [False, True])
+def test_losses_from_their_potentials(n, m, reach, debias):
+    from flash_sinkhorn_amd import SamplesLoss
+    x, y, a, b = dev(*inputs(5, n, m, 3, scale=0.5))
+    kw = dict(use_epsilon_scaling=False, eps=0.2, n_iters=3, reach_x=reach, reach_y=reach)
+    def cost(*clouds):
+        f, g = (t.double() for t in SamplesLoss(potentials=True, **kw)(*clouds))
+        if reach is None:
+            return (clouds[0].double() * f).sum() + (clouds[2].double() * g).sum()
+        rho = reach ** 2
+        return (rho + 0.1) * ((clouds[0].double() * (1 - torch.exp(-f / rho))).sum() + (clouds[2].double() * (1 - torch.exp(-g / rho))).sum())
+    want = cost(a, x, b, y)
+    if debias:
+        want = want - 0.5 * (cost(a, x, a, x) + cost(b, y, b, y))
+    got = SamplesLoss(debias=debias, **kw)(a, x, b, y)
+    # potentials are the same bits; sums of 4,500 terms in fp32 lie 1e-6 of their largest part apart
+    assert abs(float(got) - float(want)) < 3e-6 * abs(float(cost(a, x, b, y)))
+
+
 @pytest.mark.parametrize("n,m,d", [(1, 1, 129), (5, 300, 130), (1023, 1025, 200), (1024, 1025, 140),
                                    (2400, 4096, 129), (30, 4097, 129), (2441, 4096, 131)])
 def test_wide_steps_of_one_launch(n, m, d):
