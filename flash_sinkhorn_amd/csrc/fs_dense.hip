@@ -16,10 +16,20 @@ int tile_up(DenseGemmArgs& g) {
   return g.row_tiles * g.col_tiles;
 }
 
+// Tiles of 64 x 64 run with eight stages of LDS, and two steps to a barrier, where a CU gets so few workgroups that it holds that
+// many of each; with four where there are more: they cover each other's waits, four to a CU.
+constexpr double kDeepTiles = 512.0;
+
 template <int WR, int WC, int RB, int CB>
 int launch_gemm(DenseGemmArgs& g, int items, hipStream_t st) {
   const int tiles = tile_up<WR, WC, RB, CB>(g);
-  hipLaunchKernelGGL((dense_gemm_kernel<WR, WC, RB, CB>), dim3((tiles + 7) / 8 * 8, items, g.splits), dim3(64 * WR * WC), 0, st, g);
+  const dim3 grid((tiles + 7) / 8 * 8, items, g.splits), block(64 * WR * WC);
+  if constexpr (WR * RB == 2)
+    if ((double)tiles * items * g.splits <= kDeepTiles) {
+      hipLaunchKernelGGL((dense_gemm_kernel<WR, WC, RB, CB, 8>), grid, block, 0, st, g);
+      return hipGetLastError() == hipSuccess ? FS_OK : FS_ERR_LAUNCH_FAILED;
+    }
+  hipLaunchKernelGGL((dense_gemm_kernel<WR, WC, RB, CB, 4>), grid, block, 0, st, g);
   return hipGetLastError() == hipSuccess ? FS_OK : FS_ERR_LAUNCH_FAILED;
 }
 
@@ -28,8 +38,14 @@ int launch_jobs(DenseGemmJobs& g, int jobs, int items, hipStream_t st, bool apar
   int tiles = 0;
   for (int i = 0; i < jobs; ++i) tiles = std::max(tiles, tile_up<WR, WC, RB, CB>(g.job[i]));
   const dim3 grid((tiles + 7) / 8 * 8, items, jobs), block(64 * WR * WC);
-  if (apart) hipLaunchKernelGGL((dense_gemm_jobs_kernel<WR, WC, RB, CB, true>), grid, block, 0, st, g);
-  else hipLaunchKernelGGL((dense_gemm_jobs_kernel<WR, WC, RB, CB, false>), grid, block, 0, st, g);
+  if constexpr (WR * RB == 2)
+    if ((double)tiles * items * jobs <= kDeepTiles) {
+      if (apart) hipLaunchKernelGGL((dense_gemm_jobs_kernel<WR, WC, RB, CB, true, 8>), grid, block, 0, st, g);
+      else hipLaunchKernelGGL((dense_gemm_jobs_kernel<WR, WC, RB, CB, false, 8>), grid, block, 0, st, g);
+      return hipGetLastError() == hipSuccess ? FS_OK : FS_ERR_LAUNCH_FAILED;
+    }
+  if (apart) hipLaunchKernelGGL((dense_gemm_jobs_kernel<WR, WC, RB, CB, true, 4>), grid, block, 0, st, g);
+  else hipLaunchKernelGGL((dense_gemm_jobs_kernel<WR, WC, RB, CB, false, 4>), grid, block, 0, st, g);
   return hipGetLastError() == hipSuccess ? FS_OK : FS_ERR_LAUNCH_FAILED;
 }
 

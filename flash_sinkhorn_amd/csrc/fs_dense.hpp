@@ -175,8 +175,8 @@ __global__ __launch_bounds__(512) void dense_prep_kernel(const SmallArgs a, cons
 }
 
 // One operand's tile stream and C = A B^T: a workgroup of WR x WC wavefronts owns 32 WR RB rows and
-// 32 WC CB columns; per 16-column step both operands' blocks come into one of four LDS stages by
-// direct global -> LDS loads of 1 KiB per wavefront, three steps ahead, one barrier per step.
+// 32 WC CB columns; per 16-column step both operands' blocks come into one of ST LDS stages by
+// direct global -> LDS loads of 1 KiB per wavefront, ST - 1 steps ahead, one barrier per step.
 // Bound by the matrix pipe: RB CB 3 MFMAs per wavefront and step against 2 (RB + CB) LDS reads.
 // LDS reads are written out by hand (the compiler would have each wait for the loads in flight).
 struct DenseGemmArgs {
@@ -197,9 +197,16 @@ struct DenseGemmArgs {
 
 // APART: the cross products of all steps before hi * hi of the first, in a second pass (see dense_gemm_jobs_kernel), a
 // stage of which is the hi planes of two steps (an even number of them).
-template <int WR, int WC, int RB, int CB, bool APART>
+//
+// With eight stages a barrier lies between two steps and the next two: a tile of 64 x 64 has three products a step and
+// wavefront, and where a CU has one or two workgroups nothing covers the barrier and the LDS reads in front of them (with
+// eight stages and a barrier a step nothing was gained).  1,000 x 1,000 x 784 13.4 -> 12.3 us, 600 x 700 x 1,400 16.5 -> 13.9,
+// 900 x 1,300 x 163 8.4 -> 8.2, of which some 5 are the launch, the first loads and the results.
+template <int WR, int WC, int RB, int CB, bool APART, int ST>
 __device__ __forceinline__ void dense_gemm_tile(const DenseGemmArgs& g, int split) {
-  constexpr int W = WR * WC, TR = WR * RB, TC = WC * CB, PIECES = 2 * (TR + TC), LOADS = PIECES / W, ST = 4;
+  constexpr int W = WR * WC, TR = WR * RB, TC = WC * CB, PIECES = 2 * (TR + TC), LOADS = PIECES / W;
+  constexpr int PER = ST == 8 ? 2 : 1;  // steps between two barriers
+  static_assert((ST & (ST - 1)) == 0 && (ST - 2 * PER) * LOADS < 64, "stages in turn, and loads in flight that a wait can count");
   static_assert(PIECES % W == 0, "every wavefront moves the same number of pieces");
   static_assert(2 * RB * 1024 <= 65535 && 2 * CB * 1024 <= 65535, "offsets of the LDS reads");
   __shared__ __attribute__((aligned(16))) u32x4 lds[ST * PIECES * 64];
@@ -251,37 +258,44 @@ __device__ __forceinline__ void dense_gemm_tile(const DenseGemmArgs& g, int spli
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
 
-  stage(0, 0);
-  stage(1, 1);
-  stage(2, 2);
-  for (int k = 0; k < total; ++k) {
+#pragma unroll
+  for (int k = 0; k < ST - PER; ++k) stage(k, k);
+  for (int k = 0; k < total; k += PER) {
+    constexpr int newer = (ST - 2 * PER) * LOADS;
     __builtin_amdgcn_sched_barrier(0);
-    __builtin_amdgcn_s_waitcnt(0x0F70 | ((2 * LOADS) & 15) | (((2 * LOADS) >> 4) << 14));  // step k has landed
+    __builtin_amdgcn_s_waitcnt(0x0F70 | (newer & 15) | ((newer >> 4) << 14));  // the steps from k on have landed
     __builtin_amdgcn_sched_barrier(0);
     asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_barrier();  // for everyone, and step k - 1 has been read by everyone
+    __builtin_amdgcn_s_barrier();  // for everyone, and those before have been read by everyone
     asm volatile("" ::: "memory");
-    stage(k + 3, (k + 3) & 3);
-    const unsigned off = (k & 3) * (PIECES * 1024);
-    u32x4 x[RB][2], y[CB][2];
-    static_for<2 * RB>([&](auto i) { x[i / 2][i % 2] = lds_read16<decltype(i)::value * 1024>(abase + off); });
-    static_for<2 * CB>([&](auto i) { y[i / 2][i % 2] = lds_read16<decltype(i)::value * 1024>(bbase + off); });
-    static_for<CB>([&](auto j_) {
-      constexpr int j = decltype(j_)::value;
+#pragma unroll
+    for (int q = 0; q < PER; ++q) stage(k + ST - PER + q, (k + ST - PER + q) & (ST - 1));
+    u32x4 x[PER][RB][2], y[PER][CB][2];
+    static_for<PER>([&](auto q_) {
+      constexpr int q = decltype(q_)::value;
+      const unsigned off = ((k + q) & (ST - 1)) * (PIECES * 1024);
+      static_for<2 * RB>([&](auto i) { x[q][i / 2][i % 2] = lds_read16<decltype(i)::value * 1024>(abase + off); });
+      static_for<2 * CB>([&](auto i) { y[q][i / 2][i % 2] = lds_read16<decltype(i)::value * 1024>(bbase + off); });
+    });
+    static_for<PER * CB>([&](auto at) {
+      constexpr int q = decltype(at)::value / CB, j = decltype(at)::value % CB;
+      // this column block has been read; LDS returns in order
+      constexpr int later = 2 * (CB - 1 - j) + 2 * (PER - 1 - q) * (RB + CB);
       __builtin_amdgcn_sched_barrier(0);
-      __builtin_amdgcn_s_waitcnt(0xC07F | ((2 * (CB - 1 - j)) << 8));  // this column block has been read
+      __builtin_amdgcn_s_waitcnt(0xC07F | (later << 8));
       __builtin_amdgcn_sched_barrier(0);
+      if (q > 0 && k + q >= total) return;  // (an odd number of steps)
       if (!APART || k < steps) {
 #pragma unroll
         for (int prod = 0; prod < (APART ? 2 : 3); ++prod)
 #pragma unroll
           for (int i = 0; i < RB; ++i)
-            acc[i][j] = small_mfma(x[i][prod == 0 ? 1 : 0], y[j][prod == 1 ? 1 : 0], acc[i][j]);
+            acc[i][j] = small_mfma(x[q][i][prod == 0 ? 1 : 0], y[q][j][prod == 1 ? 1 : 0], acc[i][j]);
       } else {
 #pragma unroll
         for (int step = 0; step < 2; ++step)
 #pragma unroll
-          for (int i = 0; i < RB; ++i) acc[i][j] = small_mfma(x[i][step], y[j][step], acc[i][j]);
+          for (int i = 0; i < RB; ++i) acc[i][j] = small_mfma(x[q][i][step], y[q][j][step], acc[i][j]);
       }
     });
   }
@@ -314,9 +328,9 @@ __device__ __forceinline__ void dense_gemm_tile(const DenseGemmArgs& g, int spli
   }
 }
 
-template <int WR, int WC, int RB, int CB>
+template <int WR, int WC, int RB, int CB, int ST>
 __global__ __launch_bounds__(64 * WR * WC, 2) void dense_gemm_kernel(const DenseGemmArgs g) {
-  dense_gemm_tile<WR, WC, RB, CB, false>(g, blockIdx.z);
+  dense_gemm_tile<WR, WC, RB, CB, false, ST>(g, blockIdx.z);
 }
 
 // Up to four products of the same depth in one launch, summed in the order of steps on planes: the cross products before
@@ -327,9 +341,9 @@ __global__ __launch_bounds__(64 * WR * WC, 2) void dense_gemm_kernel(const Dense
 struct DenseGemmJobs {
   DenseGemmArgs job[4];
 };
-template <int WR, int WC, int RB, int CB, bool APART>
+template <int WR, int WC, int RB, int CB, bool APART, int ST>
 __global__ __launch_bounds__(64 * WR * WC, 2) void dense_gemm_jobs_kernel(const DenseGemmJobs g) {
-  dense_gemm_tile<WR, WC, RB, CB, APART>(g.job[blockIdx.z], 0);
+  dense_gemm_tile<WR, WC, RB, CB, APART, ST>(g.job[blockIdx.z], 0);
 }
 
 __device__ __forceinline__ void dense_join(float& m, float& s, float m2, float s2) {

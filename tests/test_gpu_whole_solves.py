@@ -360,6 +360,14 @@ def test_kept_products(n, m, d, dtype):
     assert rel_err(f, wf) < POT and rel_err(g, wg) < POT
 
 
+# products in tiles of 64 with eight stages: odd and even numbers of 16-column steps, up to the number of tiles where four take over
+@pytest.mark.parametrize("n,m,d", [(70, 90, 131), (65, 300, 160), (130, 64, 163), (300, 200, 192), (500, 129, 239), (90, 260, 300),
+                                   (1400, 1500, 145), (1500, 1600, 150)])
+def test_kept_products_of_small_tiles(n, m, d):
+    x, y, a, b = inputs(n + d, n, m, d, scale=1.0 / np.sqrt(d))
+    check_symmetric(x, y, a, b, use_epsilon_scaling=False, eps=0.1, n_iters=3)
+
+
 @pytest.mark.parametrize("threshold", [None, 1e-3])
 def test_kept_products_of_a_batch(threshold):
     from flash_sinkhorn_amd import SamplesLoss
