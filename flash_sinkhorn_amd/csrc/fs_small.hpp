@@ -99,15 +99,16 @@ __device__ __forceinline__ float4 small_last_coef(const SmallArgs& a, int item, 
 
 // Partial statistics of a slice of one matrix of one item: largest magnitude (the plane scale),
 // sum of the weights, and per column the smallest and largest value (the bounding box behind a
-// schedule by diameter).  A thread stays on one column.
-template <int T>
-__global__ __launch_bounds__(256) void small_stats_kernel(const SmallArgs a) {
+// schedule by diameter).  A thread stays on one column.  Bound by the loads in flight: NT
+// threads a workgroup, 256 or 1,024 (kWideStats).
+template <int NT>
+__global__ __launch_bounds__(NT) void small_stats_kernel(const SmallArgs a) {
   const int mat = blockIdx.y, item = blockIdx.z, tid = threadIdx.x;
   const int rows = a.rows[mat], d = a.d;
   const int per = (rows + a.stat_blocks - 1) / a.stat_blocks;
   const int r0 = min(rows, (int)blockIdx.x * per), r1 = min(rows, r0 + per);
-  const int reps = 256 / d, act = reps * d;
-  __shared__ float mn[256], mx[256];
+  const int reps = NT / d, act = reps * d;
+  __shared__ float mn[NT], mx[NT];
   float lo = 3.0e38f, hi = -3.0e38f, ws = 0.f;
   bool nan = false;
   if (tid < act) {
@@ -122,7 +123,7 @@ __global__ __launch_bounds__(256) void small_stats_kernel(const SmallArgs a) {
   }
   float wl = 3.0e38f, wh = 0.f;
   if (a.w[mat] != nullptr)
-    for (int r = r0 + tid; r < r1; r += 256) {
+    for (int r = r0 + tid; r < r1; r += NT) {
       const float w = a.w[mat][(size_t)item * rows + r];
       ws += w;
       wl = fminf(wl, w);
@@ -158,18 +159,25 @@ __global__ __launch_bounds__(256) void small_stats_kernel(const SmallArgs a) {
     wh = fmaxf(wh, __shfl_xor(wh, o, 64));
   }
   __syncthreads();
+  constexpr int NW = NT / 64;
   if ((tid & 63) == 0) {
     mn[tid >> 6] = am;
     mx[tid >> 6] = ws;
-    mn[4 + (tid >> 6)] = wl;
-    mx[4 + (tid >> 6)] = wh;
+    mn[NW + (tid >> 6)] = wl;
+    mx[NW + (tid >> 6)] = wh;
   }
   __syncthreads();
   if (tid == 0) {
-    out[0] = fmaxf(fmaxf(mn[0], mn[1]), fmaxf(mn[2], mn[3]));
-    out[1] = (mx[0] + mx[1]) + (mx[2] + mx[3]);
-    out[2] = fminf(fminf(mn[4], mn[5]), fminf(mn[6], mn[7]));
-    out[3] = fmaxf(fmaxf(mx[4], mx[5]), fmaxf(mx[6], mx[7]));
+    for (int w = 1; w < NW; ++w) {
+      am = fmaxf(am, mn[w]);
+      ws += mx[w];
+      wl = fminf(wl, mn[NW + w]);
+      wh = fmaxf(wh, mx[NW + w]);
+    }
+    out[0] = am;
+    out[1] = ws;
+    out[2] = wl;
+    out[3] = wh;
   }
 }
 

@@ -64,7 +64,8 @@ def test_schedules_of_every_length(n, m, d, cut):
 # lengths of schedules, from boxes whose farthest corner lies in one block of rows and one column of either cloud (up to
 # 64 blocks, sixteen threads a column or as many as 256 hold)
 @pytest.mark.parametrize("n,m,d", [(2, 3, 1), (40, 33, 2), (300, 65, 3), (513, 290, 15), (260, 545, 16), (1100, 2049, 17),
-                                   (2080, 700, 33), (90, 1000, 85), (333, 2100, 86), (2050, 100, 128), (4600, 4500, 5)])
+                                   (2080, 700, 33), (90, 1000, 85), (333, 2100, 86), (2050, 100, 128), (4600, 4500, 5),
+                                   (3073, 500, 128), (300, 5700, 69), (24600, 1000, 16)])
 def test_lengths_of_schedules(n, m, d):
     from flash_sinkhorn_amd import SamplesLoss, _small
     rng = np.random.default_rng(n + d)
