@@ -45,43 +45,19 @@ struct DenseArgs {
   int ld_t, rows;          // rows: rows of a wavefront in dense_rows_kernel, 0: dense_sweep_kernel
 };
 
-// Eight consecutive elements as floats; `wide`: by whole 16-byte words.
-__device__ __forceinline__ void dense_load8(float (&v)[8], const void* p, size_t at, int dtype, bool wide) {
-  if (wide && dtype == 0) {
-    const float4* q = reinterpret_cast<const float4*>(static_cast<const float*>(p) + at);
-    const float4 u = q[0], w = q[1];
-    v[0] = u.x, v[1] = u.y, v[2] = u.z, v[3] = u.w, v[4] = w.x, v[5] = w.y, v[6] = w.z, v[7] = w.w;
-  } else if (wide) {
-    const uint4 u = *reinterpret_cast<const uint4*>(static_cast<const unsigned short*>(p) + at);
-    const unsigned w[4] = {u.x, u.y, u.z, u.w};
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      const unsigned short b = (unsigned short)(w[k >> 1] >> (16 * (k & 1)));
-      v[k] = dtype == 1 ? (float)__builtin_bit_cast(_Float16, b) : __builtin_bit_cast(float, (unsigned)b << 16);
-    }
-  } else {
-#pragma unroll
-    for (int k = 0; k < 8; ++k) v[k] = small_load(p, at + k, dtype);
-  }
-}
-// Do rows of d elements start at multiples of 16 bytes?
-__device__ __forceinline__ bool dense_wide(const void* p, int d, int dtype) {
-  return ((size_t)p & 15) == 0 && (d & (dtype == 0 ? 3 : 7)) == 0;
-}
-
 // Largest magnitude and sum of the weights of a slice of one matrix (small_stats_kernel's first two
 // words; no bounding boxes: a schedule comes as a table here).  Bound by memory.
 __device__ __forceinline__ void dense_stats_of(const SmallArgs& a, int mat, int item) {
   const int tid = threadIdx.x;
   const size_t count = (size_t)a.rows[mat] * a.d, base = item * count;
-  const bool wide = dense_wide(a.pts[mat], a.d, a.dtype);
+  const bool wide = small_wide(a.pts[mat], a.d, a.dtype);
   float am = 0.f, ws = 0.f;
   const size_t stride = (size_t)gridDim.x * 1024 * 8;
 #pragma unroll 2
   for (size_t i = ((size_t)blockIdx.x * 1024 + tid) * 8; i < count; i += stride) {
     float v[8];
     if (i + 8 <= count) {
-      dense_load8(v, a.pts[mat], base + i, a.dtype, wide);
+      small_load8(v, a.pts[mat], base + i, a.dtype, wide);
     } else {
 #pragma unroll
       for (int k = 0; k < 8; ++k) v[k] = i + k < count ? small_load(a.pts[mat], base + i + k, a.dtype) : 0.f;
@@ -128,7 +104,7 @@ __device__ __forceinline__ void dense_prep_of(const SmallArgs& a, const DenseArg
   const float sc = f16_plane_scale(am);
   if (rb == 0 && tid == 0) a.scale[item * 2 + mat] = make_float2(sc, 1.0f / sc);
   const int row = rb * 32 + li;
-  const bool live = row < rows, wide = dense_wide(a.pts[mat], d, a.dtype);
+  const bool live = row < rows, wide = small_wide(a.pts[mat], d, a.dtype);
   const size_t base = ((size_t)item * rows + min(row, rows - 1)) * d;
   u32x4* po = t.planes[mat] + ((size_t)item * t.blocks[mat] + rb) * (size_t)t.steps * kDenseStep + lane;
   float q = 0.f;
@@ -136,7 +112,7 @@ __device__ __forceinline__ void dense_prep_of(const SmallArgs& a, const DenseArg
     float v[8];
     const int c0 = 16 * kk + 8 * h;
     if (c0 + 8 <= d) {
-      dense_load8(v, a.pts[mat], base + c0, a.dtype, wide);
+      small_load8(v, a.pts[mat], base + c0, a.dtype, wide);
     } else {
 #pragma unroll
       for (int k = 0; k < 8; ++k) v[k] = c0 + k < d ? small_load(a.pts[mat], base + c0 + k, a.dtype) : 0.f;

@@ -531,7 +531,7 @@ __global__ __launch_bounds__(256) void dense_plan_kernel(const SmallArgs a, cons
 
 // Four columns of a row: by a 16-byte word where every row of floats starts at one, else element by element up to
 // the d-th.
-__device__ __forceinline__ bool hvp_wide(const void* p, int d, int dtype) { return dtype == 0 && dense_wide(p, d, 0); }
+__device__ __forceinline__ bool hvp_wide(const void* p, int d, int dtype) { return dtype == 0 && small_wide(p, d, 0); }
 __device__ __forceinline__ float4 hvp_load4(const void* p, size_t at, int dtype, bool wide, int left) {
   if (wide) return *reinterpret_cast<const float4*>(static_cast<const float*>(p) + at);
   float4 v = make_float4(small_load(p, at, dtype), 0.f, 0.f, 0.f);

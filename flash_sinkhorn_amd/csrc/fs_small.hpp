@@ -81,6 +81,30 @@ __device__ __forceinline__ float small_load(const void* p, size_t i, int dtype) 
   return __builtin_bit_cast(float, (unsigned)static_cast<const unsigned short*>(p)[i] << 16);
 }
 
+// Eight consecutive elements as floats; `wide`: by whole 16-byte words.
+__device__ __forceinline__ void small_load8(float (&v)[8], const void* p, size_t at, int dtype, bool wide) {
+  if (wide && dtype == 0) {
+    const float4* q = reinterpret_cast<const float4*>(static_cast<const float*>(p) + at);
+    const float4 u = q[0], w = q[1];
+    v[0] = u.x, v[1] = u.y, v[2] = u.z, v[3] = u.w, v[4] = w.x, v[5] = w.y, v[6] = w.z, v[7] = w.w;
+  } else if (wide) {
+    const uint4 u = *reinterpret_cast<const uint4*>(static_cast<const unsigned short*>(p) + at);
+    const unsigned w[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const unsigned short b = (unsigned short)(w[k >> 1] >> (16 * (k & 1)));
+      v[k] = dtype == 1 ? (float)__builtin_bit_cast(_Float16, b) : __builtin_bit_cast(float, (unsigned)b << 16);
+    }
+  } else {
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = small_load(p, at + k, dtype);
+  }
+}
+// Do rows of d elements start at multiples of 16 bytes?
+__device__ __forceinline__ bool small_wide(const void* p, int d, int dtype) {
+  return ((size_t)p & 15) == 0 && (d & (dtype == 0 ? 3 : 7)) == 0;
+}
+
 // What a step derives from its eps: eps, base-2 logit per unit of x.y, its inverse, base-2 units
 // per unit of a potential.
 __device__ __forceinline__ float4 small_coef(float cost_scale, float eps) {

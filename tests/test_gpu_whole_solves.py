@@ -82,6 +82,20 @@ def test_lengths_of_schedules(n, m, d):
         assert torch.isfinite(loss) and _small._host_words(1)[:3].tolist() == want
 
 
+# planes that are written anew for every eps, from rows by whole 16-byte words and one by one: the same bits
+@pytest.mark.parametrize("n,m,d", [(4600, 4500, 36), (4600, 4500, 60), (4520, 4609, 64), (7200, 7100, 4), (7200, 7100, 20)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+def test_planes_of_unaligned_rows(n, m, d, dtype):
+    from flash_sinkhorn_amd import SamplesLoss
+    x, y = (t.to(dtype) for t in dev(*inputs(7, n, m, d, scale=0.5)[:2]))
+    def off(t):
+        u = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)[1:].view_as(t)
+        return u.copy_(t)
+    loss = SamplesLoss(blur=0.3, potentials=True)
+    for got, want in zip(loss(off(x), off(y)), loss(x, y)):
+        assert torch.equal(got, want)
+
+
 # sums over one to several rows a thread and workgroup, of every combination of sides
 @pytest.mark.parametrize("n,m", [(1, 1025), (1024, 3), (1030, 2049), (3073, 3072), (4500, 1000)])
 @pytest.mark.parametrize("reach", [None, 1.3])
