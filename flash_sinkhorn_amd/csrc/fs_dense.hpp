@@ -338,8 +338,8 @@ __device__ __forceinline__ void dense_join(float& m, float& s, float m2, float s
 // Every other step over more products than the L2s hold goes from the last to the first, and finds in the
 // 256 MB of the last-level cache what the step before has read last (in one order, what does not fit pushes
 // out all of it).  50 steps of 9,000 x 9,000 (324 MB) 5.15 -> 4.18 ms, 12,000 points 7.87 -> 7.13, 16,000 13.0 ->
-// 12.2, 4,000 x 5,000 1.59 -> 1.52; 8,192 points (268 MB) 3.07 as before.  Up to 32 MB an XCD finds in its L2 what
-// it has read itself, and only in the same order: 2,000 points would take 0.86 ms for 0.80.
+// 12.2, 4,000 x 5,000 1.59 -> 1.52; 8,192 points (268 MB) 3.07 as before.  Up to 32 MB one order
+// is faster: 2,000 points 0.80 ms for 0.86.
 template <int RW, int WV>
 __global__ __launch_bounds__(64 * WV, 4) void dense_sweep_kernel(const DenseArgs a) {
   constexpr int B = 8;  // rows in registers
@@ -483,7 +483,7 @@ __global__ __launch_bounds__(256) void dense_merge_kernel(const DenseArgs a) {
   if (side == 0 && a.step > entries) a.top[at] = M;
 }
 
-// A step of every problem in one launch, where the products and their transposes stay in the L2s and the last-level
+// A step of every problem in one launch, where the products and their transposes stay in the last-level
 // cache: a wavefront owns R rows of one side and reads all of their products, so nothing is left to a merge; the
 // columns of the xy products are rows of a transposed copy, which the product's epilogue writes beside the
 // other.  Bound by the launch and the chain of loads in front of the first logit (1,000 points: 4.0 us a
