@@ -81,6 +81,8 @@ _SIGNATURES = {
     "fs_hvp_solved_workspace_bytes": (_Z, [_P]),
     "fs_hvp_solved": (ctypes.c_int, [_P, _P, _P, _Z, _P, _Z, _P, _P, _P]),
     "fs_small_grad": (ctypes.c_int, [_P, _P, _Z, _P, _P, _P, _P]),
+    "fs_row_start": (ctypes.c_int, [_P] * 4 + [_I] * 3 + [_F, _P, _P]),
+    "fs_change": (ctypes.c_int, [_P, _P, _I, _P, _P, _I, _P, _P]),
 }
 EXPORTED_SYMBOLS = tuple(_SIGNATURES)
 

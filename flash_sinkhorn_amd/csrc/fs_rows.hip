@@ -1,0 +1,107 @@
+// What a solve of the general path starts from and looks at between its steps, a launch each.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+
+#include "flash_sinkhorn_hip.h"
+
+namespace fs {
+namespace {
+
+struct RowStart {
+  const float* pts[2];
+  const float* w[2];
+  float *norm[2], *logw[2], *pot[2];
+  int rows[2], blocks0, d, wide;
+  float cost_scale;
+};
+
+// cost_scale |row|^2, its negative (the potential that a solve starts from) and the logarithm of a row's weight, of both
+// clouds.  Sixteen lanes a row, sixteen rows a workgroup.  Bound by reading the points.  As operations of their own products, sums,
+// logarithms and selections were fourteen launches of 65 us together at 50,000 rows of 128 columns, and the host took longer
+// than they did: ten alternating iterations with this and change_kernel 3,998 -> 3,850 us, of 7,000 x 7,500 x 100 1,435 ->
+// 1,305, of 15,000 x 14,000 x 8 1,300 -> 1,163.
+constexpr int kRowsOfBlock = 16;
+__global__ __launch_bounds__(256) void row_start_kernel(const RowStart a) {
+  const int mat = (int)blockIdx.x >= a.blocks0 ? 1 : 0, tid = threadIdx.x, lane = tid & 15;
+  const int row = ((int)blockIdx.x - (mat ? a.blocks0 : 0)) * kRowsOfBlock + (tid >> 4), rows = a.rows[mat], d = a.d;
+  const float* p = a.pts[mat] + (size_t)min(row, rows - 1) * d;
+  const float w = a.w[mat][min(row, rows - 1)];
+  float s = 0.f;
+  if (a.wide) {
+#pragma unroll 4
+    for (int c = 4 * lane; c < d; c += 64) {
+      const float4 v = *reinterpret_cast<const float4*>(p + c);
+      s = __builtin_fmaf(v.x, v.x, __builtin_fmaf(v.y, v.y, __builtin_fmaf(v.z, v.z, __builtin_fmaf(v.w, v.w, s))));
+    }
+  } else {
+#pragma unroll 4
+    for (int c = lane; c < d; c += 16) s = __builtin_fmaf(p[c], p[c], s);
+  }
+#pragma unroll
+  for (int o = 8; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+  if (lane > 0 || row >= rows) return;
+  s *= a.cost_scale;
+  a.norm[mat][row] = s;
+  a.pot[mat][row] = -s;
+  a.logw[mat][row] = w > 0.f ? logf(w) : -100000.0f;
+}
+
+// out[i]: the largest |now[i] - before[i]| (not a number where one of the differences is none).  A workgroup each: mostly its launch.
+struct Change {
+  const float *now[2], *before[2];
+  int rows[2];
+  float* out;
+};
+__global__ __launch_bounds__(1024) void change_kernel(const Change a) {
+  const int i = blockIdx.x, tid = threadIdx.x, rows = a.rows[i];
+  unsigned most = 0;  // (of numbers without a sign, and of what is none behind them)
+#pragma unroll 8
+  for (int r = tid; r < rows; r += 1024) {
+    const float v = a.now[i][r] - a.before[i][r];
+    most = max(most, __builtin_bit_cast(unsigned, v) & 0x7fffffffu);
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) most = max(most, (unsigned)__shfl_xor((int)most, o, 64));
+  __shared__ unsigned sh[16];
+  if ((tid & 63) == 0) sh[tid >> 6] = most;
+  __syncthreads();
+  if (tid > 0) return;
+#pragma unroll
+  for (int w = 1; w < 16; ++w) most = max(most, sh[w]);
+  a.out[i] = __builtin_bit_cast(float, most);
+}
+
+bool bad_rows(int64_t n, int64_t m) { return n <= 0 || m <= 0 || n > (1 << 30) || m > (1 << 30); }
+
+}  // namespace
+}  // namespace fs
+
+extern "C" {
+
+int fs_row_start(const float* x, const float* y, const float* a, const float* b, int64_t n, int64_t m, int64_t d,
+                 float cost_scale, float* const* out, void* stream) {
+  using namespace fs;
+  if (!x || !y || !a || !b || !out) return FS_ERR_NULL_POINTER;
+  for (int i = 0; i < 6; ++i)
+    if (!out[i]) return FS_ERR_NULL_POINTER;
+  if (bad_rows(n, m) || d <= 0 || d > (1 << 20)) return FS_ERR_BAD_SIZE;
+  RowStart t{{x, y}, {a, b}, {out[0], out[1]}, {out[2], out[3]}, {out[4], out[5]}, {(int)n, (int)m}, 0, (int)d, 0, cost_scale};
+  t.wide = d % 4 == 0 && ((reinterpret_cast<size_t>(x) | reinterpret_cast<size_t>(y)) & 15) == 0;
+  t.blocks0 = (int)((n + kRowsOfBlock - 1) / kRowsOfBlock);
+  const int blocks = t.blocks0 + (int)((m + kRowsOfBlock - 1) / kRowsOfBlock);
+  hipLaunchKernelGGL(row_start_kernel, dim3(blocks), dim3(256), 0, (hipStream_t)stream, t);
+  return hipGetLastError() == hipSuccess ? FS_OK : FS_ERR_LAUNCH_FAILED;
+}
+
+int fs_change(const float* f, const float* f_before, int64_t n, const float* g, const float* g_before, int64_t m, float* out,
+              void* stream) {
+  using namespace fs;
+  if (!f || !f_before || !g || !g_before || !out) return FS_ERR_NULL_POINTER;
+  if (bad_rows(n, m)) return FS_ERR_BAD_SIZE;
+  const Change t{{f, g}, {f_before, g_before}, {(int)n, (int)m}, out};
+  hipLaunchKernelGGL(change_kernel, dim3(2), dim3(1024), 0, (hipStream_t)stream, t);
+  return hipGetLastError() == hipSuccess ? FS_OK : FS_ERR_LAUNCH_FAILED;
+}
+
+}  // extern "C"

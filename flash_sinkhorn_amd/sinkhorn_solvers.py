@@ -8,6 +8,7 @@ correction live in the kernel epilogue.
 """
 from __future__ import annotations
 
+import ctypes
 import os
 from typing import Optional, Sequence, Tuple
 
@@ -90,6 +91,24 @@ def _max_change(f, g, prev_f, prev_g) -> float:
     return max((f - prev_f).abs().max().item(), (g - prev_g).abs().max().item())
 
 
+def _row_start(xf, yf, a, b, cost_scale):
+    """cost_scale |row|^2 and log weights of both clouds and the potentials that a solve starts from, in one launch."""
+    n, m = xf.shape[0], yf.shape[0]
+    out = [torch.empty(k, device=xf.device, dtype=torch.float32) for k in (n, m) * 3]
+    _lib.check(_lib.lib().fs_row_start(
+        xf.data_ptr(), yf.data_ptr(), a.data_ptr(), b.data_ptr(), n, m, xf.shape[1], float(cost_scale),
+        (ctypes.c_void_p * 6)(*[t.data_ptr() for t in out]), _lib.stream_of(xf)), "fs_row_start")
+    return out
+
+
+def _largest_change(f, g, prev_f, prev_g) -> float:
+    """``_max_change`` in one launch and one wait."""
+    out = torch.empty(2, device=f.device, dtype=torch.float32)
+    _lib.check(_lib.lib().fs_change(f.data_ptr(), prev_f.data_ptr(), f.numel(), g.data_ptr(), prev_g.data_ptr(), g.numel(),
+                                    out.data_ptr(), _lib.stream_of(f)), "fs_change")
+    return max(out.tolist())
+
+
 def sinkhorn_flashstyle_alternating(
     x: torch.Tensor, y: torch.Tensor, a: torch.Tensor, b: torch.Tensor, *,
     eps: float = 0.1, n_iters: int = 100, cost_scale: float = 1.0,
@@ -132,11 +151,16 @@ def sinkhorn_flashstyle_alternating(
         f, g = s.potentials("f")[0], s.potentials("g")[0]
         return (f, g, s.entries) if return_n_iters else (f, g)
     xf, yf = x.float().contiguous(), y.float().contiguous()
-    alpha = cost_scale * (xf * xf).sum(dim=1)
-    beta = cost_scale * (yf * yf).sum(dim=1)
-    log_a, log_b = log_weights(a), log_weights(b)
-    f_hat, g_hat = -alpha, -beta
-    prev_f, prev_g = (f_hat.clone(), g_hat.clone()) if threshold is not None else (None, None)
+    plain = xf.shape[0] > 0 and yf.shape[0] > 0 and not (
+        torch.is_grad_enabled() and any(t.requires_grad for t in (x, y, a, b)))
+    if plain:
+        alpha, beta, log_a, log_b, f_hat, g_hat = _row_start(xf, yf, _f32c(a), _f32c(b), cost_scale)
+    else:  # (alpha and beta pass gradients on to the points)
+        alpha = cost_scale * (xf * xf).sum(dim=1)
+        beta = cost_scale * (yf * yf).sum(dim=1)
+        log_a, log_b = log_weights(a), log_weights(b)
+        f_hat, g_hat = -alpha, -beta
+    prev_f, prev_g = f_hat, g_hat  # (a half-update writes into memory of its own)
     # operand planes are converted once for the whole loop
     prepared = _lib.PreparedOperands(xf, yf, _lib.flags(use_exp2, allow_tf32))
     # the kernel variant with the coarse tile test (see COARSE_TEST): every half-update starts
@@ -158,9 +182,9 @@ def sinkhorn_flashstyle_alternating(
             g_hat = flashsinkhorn_lse_fused(yf, xf, f_hat, log_a, eps, damping=damp_g, **kw)
         used += 1
         if threshold is not None and (it + 1) % check_every == 0:
-            if _max_change(f_hat, g_hat, prev_f, prev_g) < threshold:
+            if (_largest_change if plain else _max_change)(f_hat, g_hat, prev_f, prev_g) < threshold:
                 break
-            prev_f, prev_g = f_hat.clone(), g_hat.clone()
+            prev_f, prev_g = f_hat, g_hat
 
     f, g = f_hat + alpha, g_hat + beta
     return (f, g, used) if return_n_iters else (f, g)

@@ -521,6 +521,16 @@ int fs_hvp_solved(const fs_hvp_problem* problem, const fs_small_problem* solved,
                   size_t solved_bytes, void* workspace, size_t workspace_bytes, float* out, float* host_state,
                   void* stream);
 
+/*
+ * What a solve starts from.  out: cost_scale |x_i|^2 [n], the same of y [m]; log a_i (weights that are not positive: -100000)
+ * [n], of b [m]; the negatives of the first two.  Replaces sinkhorn_solvers.py:200-215.
+ */
+int fs_row_start(const float* x, const float* y, const float* a, const float* b, int64_t n, int64_t m, int64_t d,
+                 float cost_scale, float* const* out, void* stream);
+/* out [2]: the largest |f - f_before| and |g - g_before| (NaN where a difference is). */
+int fs_change(const float* f, const float* f_before, int64_t n, const float* g, const float* g_before, int64_t m, float* out,
+              void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -1385,3 +1385,43 @@ def test_the_tile_test_rounds_as_often_as_the_plain_kernel(d, eps):
         ratios.append([float((flashsinkhorn_lse_fused(x, y, g, lw, eps, allow_tf32=False, _prepared=prep, _coarse=True)
                               - want).norm() / (plain - want).norm()) for _ in range(4)])
     assert all(sum(of_launch) / 4 < 1.04 for of_launch in zip(*ratios))
+
+
+# ---- what an alternating solve of the general path starts from and is stopped by ----
+@pytest.mark.parametrize("n,m,d", [(1, 1, 1), (17, 31, 3), (16, 33, 4), (100, 1, 63), (257, 130, 64), (33, 70, 100), (50, 49, 130),
+                                   (1025, 2047, 128)])
+@pytest.mark.parametrize("off", [0, 1])
+def test_row_start(n, m, d, off):
+    from flash_sinkhorn_amd.kernels._common import log_weights
+    from flash_sinkhorn_amd.sinkhorn_solvers import _row_start
+    gen = torch.Generator(device="cuda").manual_seed(n + d)
+    x, y = (torch.randn(k * d + off, device="cuda", generator=gen)[off:].view(k, d) for k in (n, m))
+    a, b = (torch.rand(k, device="cuda", generator=gen) for k in (n, m))
+    a[0], b[-1] = 0.0, -1.0
+    if n > 2:
+        a[1], a[2] = float("nan"), float("inf")
+    got = _row_start(x, y, a, b, 0.7)
+    for i, (p, w) in enumerate(((x, a), (y, b))):
+        want = 0.7 * (p.double() ** 2).sum(1)
+        # d terms of one sign in fp32, in sixteen parts
+        assert torch.allclose(got[i].double(), want, rtol=(d / 16 + 8) * 2.0 ** -24, atol=1e-30)
+        assert torch.equal(got[4 + i], -got[i])
+        assert torch.allclose(got[2 + i], log_weights(w), rtol=2.0 ** -22, atol=0)
+
+
+@pytest.mark.parametrize("n,m", [(1, 1), (63, 1025), (1024, 64), (8193, 20000)])
+def test_largest_change(n, m):
+    from flash_sinkhorn_amd.sinkhorn_solvers import _largest_change, _max_change
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    f, g, p, q = (torch.randn(k, device="cuda", generator=gen) for k in (n, m, n, m))
+    same = lambda: np.testing.assert_equal(_largest_change(f, g, p, q), _max_change(f, g, p, q))  # noqa: E731
+    same()
+    f[-1], g[-1] = 50.0, -60.0
+    same()
+    g[0] = float("inf")
+    same()
+    q[0] = float("inf")  # (not a number: of the second pair, then of both)
+    same()
+    f[0] = -float("nan")
+    same()
+    assert _largest_change(p, q[1:], p, q[1:]) == 0.0 if m > 1 else True
