@@ -262,11 +262,18 @@ def sinkhorn_flashstyle_symmetric(
     _require_cuda(x, y)
     _validate_problem(x, y, [("a", a)], [("b", b)])
     xf, yf = x.float().contiguous(), y.float().contiguous()
-    alpha = (cost_scale * (xf * xf).sum(dim=1)).contiguous()
-    beta = (cost_scale * (yf * yf).sum(dim=1)).contiguous()
-    log_a, log_b = _f32c(log_weights(a)), _f32c(log_weights(b))
-    f_hat = -alpha if f_init is None else _f32c(f_init) - alpha
-    g_hat = -beta if g_init is None else _f32c(g_init) - beta
+    if xf.shape[0] > 0 and yf.shape[0] > 0 and not (
+            torch.is_grad_enabled() and any(t.requires_grad for t in (x, y, a, b))):
+        alpha, beta, log_a, log_b, f_hat, g_hat = _row_start(xf, yf, _f32c(a), _f32c(b), cost_scale)
+    else:
+        alpha = (cost_scale * (xf * xf).sum(dim=1)).contiguous()
+        beta = (cost_scale * (yf * yf).sum(dim=1)).contiguous()
+        log_a, log_b = _f32c(log_weights(a)), _f32c(log_weights(b))
+        f_hat, g_hat = -alpha, -beta
+    if f_init is not None:
+        f_hat = _f32c(f_init) - alpha
+    if g_init is not None:
+        g_hat = _f32c(g_init) - beta
     if fused is None:
         fused = True
     if use_labels:
@@ -531,10 +538,13 @@ def sinkhorn_flashstyle_symmetric_self_pair(
     _validate_problem(x, y, [("a", a)], [("b", b)])
     xf, yf = x.detach().float().contiguous(), y.detach().float().contiguous()
     ex, ey = schedule(xf), schedule(yf)
-    alpha_x = (cost_scale * (xf * xf).sum(dim=1)).contiguous()
-    alpha_y = (cost_scale * (yf * yf).sum(dim=1)).contiguous()
-    log_a, log_b = _f32c(log_weights(a.detach())), _f32c(log_weights(b.detach()))
-    fx, fy = -alpha_x, -alpha_y
+    if xf.shape[0] > 0 and yf.shape[0] > 0:
+        alpha_x, alpha_y, log_a, log_b, fx, fy = _row_start(xf, yf, _f32c(a.detach()), _f32c(b.detach()), cost_scale)
+    else:
+        alpha_x = (cost_scale * (xf * xf).sum(dim=1)).contiguous()
+        alpha_y = (cost_scale * (yf * yf).sum(dim=1)).contiguous()
+        log_a, log_b = _f32c(log_weights(a.detach())), _f32c(log_weights(b.detach()))
+        fx, fy = -alpha_x, -alpha_y
     shift_x = alpha_x if rho is not None else None
     shift_y = alpha_y if rho is not None else None
     flag_bits = _lib.flags(use_exp2, allow_tf32)
