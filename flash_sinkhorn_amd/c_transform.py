@@ -14,7 +14,8 @@ from typing import Optional
 
 import torch
 
-from flash_sinkhorn_amd.kernels._common import _validate_device
+from flash_sinkhorn_amd import _lib
+from flash_sinkhorn_amd.kernels._common import _f32c, _validate_device
 from flash_sinkhorn_amd.kernels.c_transform_sqeuclid import c_transform_kernel
 
 __all__ = ["c_transform_fwd", "c_transform_cost"]
@@ -45,12 +46,17 @@ def c_transform_fwd(x: torch.Tensor, y: torch.Tensor, psi: torch.Tensor, *,
         raise NotImplementedError("grad_y not supported for c_transform_fwd. "
                                   "Detach y or use a solver that supports grad_y.")
     with torch.no_grad():
-        xf, yf = x.float(), y.float()
-        bias = cost_scale * (yf * yf).sum(dim=1) - psi.float()
+        xf, yf, pf = _f32c(x), _f32c(y), _f32c(psi)
+        if n == 0:
+            bias, x_sq = cost_scale * (yf * yf).sum(dim=1) - pf, cost_scale * (xf * xf).sum(dim=1)
+        else:
+            x_sq, bias = (torch.empty(k, device=x.device, dtype=torch.float32) for k in (n, m))
+            _lib.check(_lib.lib().fs_c_bias(xf.data_ptr(), yf.data_ptr(), pf.data_ptr(), n, m, d, float(cost_scale),
+                                            x_sq.data_ptr(), bias.data_ptr(), _lib.stream_of(x)), "fs_c_bias")
         inner, idx = c_transform_kernel(xf, yf, bias, cost_scale=cost_scale,
                                         allow_tf32=allow_tf32, autotune=autotune,
                                         **kernel_kwargs)
-        values = cost_scale * (xf * xf).sum(dim=1) + inner
+        values = x_sq + inner
     return values, idx
 
 

@@ -10,7 +10,8 @@ namespace {
 
 struct RowStart {
   const float* pts[2];
-  const float* w[2];
+  const float* w[2];     // weights, null: no logarithms
+  const float* less[2];  // taken off the norms, null: nothing
   float *norm[2], *logw[2], *pot[2];
   int rows[2], blocks0, d, wide;
   float cost_scale;
@@ -20,13 +21,15 @@ struct RowStart {
 // clouds.  Sixteen lanes a row, sixteen rows a workgroup.  Bound by reading the points.  As operations of their own products, sums,
 // logarithms and selections were fourteen launches of 65 us together at 50,000 rows of 128 columns, and the host took longer
 // than they did: ten alternating iterations with this and change_kernel 3,998 -> 3,850 us, of 7,000 x 7,500 x 100 1,435 ->
-// 1,305, of 15,000 x 14,000 x 8 1,300 -> 1,163.
+// 1,305, of 15,000 x 14,000 x 8 1,300 -> 1,163.  Norms and biases of a c-transform were seven: 2,716 x 2,506 x 35 77 -> 46 us,
+// 20,000 x 15,000 x 8 105 -> 87, 48,000 x 48,000 x 100 1,591 -> 1,548.
 constexpr int kRowsOfBlock = 16;
 __global__ __launch_bounds__(256) void row_start_kernel(const RowStart a) {
   const int mat = (int)blockIdx.x >= a.blocks0 ? 1 : 0, tid = threadIdx.x, lane = tid & 15;
   const int row = ((int)blockIdx.x - (mat ? a.blocks0 : 0)) * kRowsOfBlock + (tid >> 4), rows = a.rows[mat], d = a.d;
   const float* p = a.pts[mat] + (size_t)min(row, rows - 1) * d;
-  const float w = a.w[mat][min(row, rows - 1)];
+  const float w = a.w[mat] != nullptr ? a.w[mat][min(row, rows - 1)] : 0.f;
+  const float less = a.less[mat] != nullptr ? a.less[mat][min(row, rows - 1)] : 0.f;
   float s = 0.f;
   if (a.wide) {
 #pragma unroll 4
@@ -42,7 +45,8 @@ __global__ __launch_bounds__(256) void row_start_kernel(const RowStart a) {
   for (int o = 8; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
   if (lane > 0 || row >= rows) return;
   s *= a.cost_scale;
-  a.norm[mat][row] = s;
+  a.norm[mat][row] = s - less;
+  if (a.w[mat] == nullptr) return;
   a.pot[mat][row] = -s;
   a.logw[mat][row] = w > 0.f ? logf(w) : -100000.0f;
 }
@@ -72,6 +76,14 @@ __global__ __launch_bounds__(1024) void change_kernel(const Change a) {
   a.out[i] = __builtin_bit_cast(float, most);
 }
 
+int launch_rows(RowStart& t, hipStream_t st) {
+  t.wide = t.d % 4 == 0 && ((reinterpret_cast<size_t>(t.pts[0]) | reinterpret_cast<size_t>(t.pts[1])) & 15) == 0;
+  t.blocks0 = (t.rows[0] + kRowsOfBlock - 1) / kRowsOfBlock;
+  const int blocks = t.blocks0 + (t.rows[1] + kRowsOfBlock - 1) / kRowsOfBlock;
+  hipLaunchKernelGGL(row_start_kernel, dim3(blocks), dim3(256), 0, st, t);
+  return hipGetLastError() == hipSuccess ? FS_OK : FS_ERR_LAUNCH_FAILED;
+}
+
 bool bad_rows(int64_t n, int64_t m) { return n <= 0 || m <= 0 || n > (1 << 30) || m > (1 << 30); }
 
 }  // namespace
@@ -86,12 +98,17 @@ int fs_row_start(const float* x, const float* y, const float* a, const float* b,
   for (int i = 0; i < 6; ++i)
     if (!out[i]) return FS_ERR_NULL_POINTER;
   if (bad_rows(n, m) || d <= 0 || d > (1 << 20)) return FS_ERR_BAD_SIZE;
-  RowStart t{{x, y}, {a, b}, {out[0], out[1]}, {out[2], out[3]}, {out[4], out[5]}, {(int)n, (int)m}, 0, (int)d, 0, cost_scale};
-  t.wide = d % 4 == 0 && ((reinterpret_cast<size_t>(x) | reinterpret_cast<size_t>(y)) & 15) == 0;
-  t.blocks0 = (int)((n + kRowsOfBlock - 1) / kRowsOfBlock);
-  const int blocks = t.blocks0 + (int)((m + kRowsOfBlock - 1) / kRowsOfBlock);
-  hipLaunchKernelGGL(row_start_kernel, dim3(blocks), dim3(256), 0, (hipStream_t)stream, t);
-  return hipGetLastError() == hipSuccess ? FS_OK : FS_ERR_LAUNCH_FAILED;
+  RowStart t{{x, y}, {a, b}, {nullptr, nullptr}, {out[0], out[1]}, {out[2], out[3]}, {out[4], out[5]}, {(int)n, (int)m}, 0, (int)d, 0, cost_scale};
+  return launch_rows(t, (hipStream_t)stream);
+}
+
+int fs_c_bias(const float* x, const float* y, const float* psi, int64_t n, int64_t m, int64_t d, float cost_scale,
+              float* x_norm, float* bias, void* stream) {
+  using namespace fs;
+  if (!x || !y || !psi || !x_norm || !bias) return FS_ERR_NULL_POINTER;
+  if (bad_rows(n, m) || d <= 0 || d > (1 << 20)) return FS_ERR_BAD_SIZE;
+  RowStart t{{x, y}, {nullptr, nullptr}, {nullptr, psi}, {x_norm, bias}, {nullptr, nullptr}, {nullptr, nullptr}, {(int)n, (int)m}, 0, (int)d, 0, cost_scale};
+  return launch_rows(t, (hipStream_t)stream);
 }
 
 int fs_change(const float* f, const float* f_before, int64_t n, const float* g, const float* g_before, int64_t m, float* out,

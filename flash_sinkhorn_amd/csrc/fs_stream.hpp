@@ -759,6 +759,7 @@ __global__ __launch_bounds__(256) void finish_argmax_kernel(const LaunchArgs arg
   if (row >= sd.nq) return;
   float best = -3.0e38f;
   int bj = 0x7fffffff;
+#pragma unroll 8
   for (int sp = 0; sp < sd.splits; ++sp) {
     const float2 v = *reinterpret_cast<const float2*>(&sd.part_ms[2 * ((size_t)sp * sd.nq + row)]);
     const int j = __builtin_bit_cast(int, v.y);

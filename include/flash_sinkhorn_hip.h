@@ -527,6 +527,9 @@ int fs_hvp_solved(const fs_hvp_problem* problem, const fs_small_problem* solved,
  */
 int fs_row_start(const float* x, const float* y, const float* a, const float* b, int64_t n, int64_t m, int64_t d,
                  float cost_scale, float* const* out, void* stream);
+/* What a c-transform is made of besides fs_c_transform: cost_scale |x_i|^2 [n] and bias_j = cost_scale |y_j|^2 - psi_j [m]. */
+int fs_c_bias(const float* x, const float* y, const float* psi, int64_t n, int64_t m, int64_t d, float cost_scale,
+              float* x_norm, float* bias, void* stream);
 /* out [2]: the largest |f - f_before| and |g - g_before| (NaN where a difference is). */
 int fs_change(const float* f, const float* f_before, int64_t n, const float* g, const float* g_before, int64_t m, float* out,
               void* stream);

@@ -1409,6 +1409,21 @@ def test_row_start(n, m, d, off):
         assert torch.allclose(got[2 + i], log_weights(w), rtol=2.0 ** -22, atol=0)
 
 
+@pytest.mark.parametrize("n,m,d", [(1, 1, 1), (17, 31, 3), (33, 70, 64), (50, 49, 130)])
+@pytest.mark.parametrize("off", [0, 1])
+def test_c_bias(n, m, d, off):
+    from flash_sinkhorn_amd import _lib
+    gen = torch.Generator(device="cuda").manual_seed(n + d)
+    x, y = (torch.randn(k * d + off, device="cuda", generator=gen)[off:].view(k, d) for k in (n, m))
+    psi = torch.randn(m, device="cuda", generator=gen)
+    norm, bias = torch.empty(n, device="cuda"), torch.empty(m, device="cuda")
+    _lib.check(_lib.lib().fs_c_bias(x.data_ptr(), y.data_ptr(), psi.data_ptr(), n, m, d, 0.7, norm.data_ptr(), bias.data_ptr(),
+                                    _lib.stream_of(x)), "fs_c_bias")
+    for got, p, less in ((norm, x, 0.0), (bias, y, psi.double())):
+        want = 0.7 * (p.double() ** 2).sum(1)
+        assert ((got.double() - (want - less)).abs() <= (d / 16 + 8) * 2.0 ** -24 * (want + abs(less))).all()
+
+
 @pytest.mark.parametrize("n,m", [(1, 1), (63, 1025), (1024, 64), (8193, 20000)])
 def test_largest_change(n, m):
     from flash_sinkhorn_amd.sinkhorn_solvers import _largest_change, _max_change
