@@ -523,7 +523,7 @@ int fs_hvp_solved(const fs_hvp_problem* problem, const fs_small_problem* solved,
 
 /*
  * What a solve starts from.  out: cost_scale |x_i|^2 [n], the same of y [m]; log a_i (weights that are not positive: -100000)
- * [n], of b [m]; the negatives of the first two.  Replaces sinkhorn_solvers.py:200-215.
+ * [n], of b [m]; the negatives of the first two.  (The operations in front of the loops of sinkhorn_solvers.py.)
  */
 int fs_row_start(const float* x, const float* y, const float* a, const float* b, int64_t n, int64_t m, int64_t d,
                  float cost_scale, float* const* out, void* stream);
