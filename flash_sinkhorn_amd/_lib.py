@@ -83,6 +83,8 @@ _SIGNATURES = {
     "fs_small_grad": (ctypes.c_int, [_P, _P, _Z, _P, _P, _P, _P]),
     "fs_row_start": (ctypes.c_int, [_P] * 4 + [_I] * 3 + [_F, _P, _P]),
     "fs_c_bias": (ctypes.c_int, [_P] * 3 + [_I] * 3 + [_F] + [_P] * 3),
+    "fs_diameter_workspace_bytes": (_Z, [_I]),
+    "fs_diameter": (ctypes.c_int, [_P] * 2 + [_I] * 3 + [_P, _P, _Z, _P]),
     "fs_change": (ctypes.c_int, [_P, _P, _I, _P, _P, _I, _P, _P]),
 }
 EXPORTED_SYMBOLS = tuple(_SIGNATURES)

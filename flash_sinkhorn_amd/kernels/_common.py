@@ -11,6 +11,8 @@ from typing import List, Optional, Sequence, Tuple
 
 import torch
 
+from flash_sinkhorn_amd import _lib
+
 __all__ = ["dampening", "log_weights", "max_diameter", "epsilon_schedule"]
 # label_cost_active / augment_label_cost are shared by the launchers that take OTDD labels
 
@@ -28,6 +30,16 @@ def log_weights(w: torch.Tensor) -> torch.Tensor:
 
 def max_diameter(x: torch.Tensor, y: torch.Tensor) -> float:
     """Length of the diagonal of the joint bounding box of x and y (host float; syncs)."""
+    if (x.is_cuda and x.device == y.device and x.ndim == 2 and y.ndim == 2 and x.shape[1] == y.shape[1]
+            and x.numel() > 0 and y.numel() > 0 and x.is_floating_point() and y.is_floating_point()):
+        xf = _f32c(x.detach())
+        yf = xf if y is x else _f32c(y.detach())
+        d = xf.shape[1]
+        nbytes = _lib.lib().fs_diameter_workspace_bytes(d)
+        ws = torch.empty(nbytes // 4 + 1, device=x.device, dtype=torch.float32)
+        _lib.check(_lib.lib().fs_diameter(xf.data_ptr(), yf.data_ptr(), xf.shape[0], yf.shape[0], d, ws[-1:].data_ptr(),
+                                          ws.data_ptr(), nbytes, _lib.stream_of(x)), "fs_diameter")
+        return ws[-1].item()
     xf, yf = x.float(), y.float()
     lo = torch.minimum(xf.amin(dim=0), yf.amin(dim=0))
     hi = torch.maximum(xf.amax(dim=0), yf.amax(dim=0))

@@ -530,6 +530,10 @@ int fs_row_start(const float* x, const float* y, const float* a, const float* b,
 /* What a c-transform is made of besides fs_c_transform: cost_scale |x_i|^2 [n] and bias_j = cost_scale |y_j|^2 - psi_j [m]. */
 int fs_c_bias(const float* x, const float* y, const float* psi, int64_t n, int64_t m, int64_t d, float cost_scale,
               float* x_norm, float* bias, void* stream);
+/* out [1]: the length of the diagonal of the joint bounding box of x and y (NaN where a coordinate is). */
+size_t fs_diameter_workspace_bytes(int64_t d);
+int fs_diameter(const float* x, const float* y, int64_t n, int64_t m, int64_t d, float* out, void* workspace,
+                size_t workspace_bytes, void* stream);
 /* out [2]: the largest |f - f_before| and |g - g_before| (NaN where a difference is). */
 int fs_change(const float* f, const float* f_before, int64_t n, const float* g, const float* g_before, int64_t m, float* out,
               void* stream);

@@ -1424,6 +1424,25 @@ def test_c_bias(n, m, d, off):
         assert ((got.double() - (want - less)).abs() <= (d / 16 + 8) * 2.0 ** -24 * (want + abs(less))).all()
 
 
+@pytest.mark.parametrize("n,m,d", [(1, 1, 1), (2, 40, 1), (33, 31, 3), (100, 2049, 64), (5000, 70, 90), (64, 65, 171), (300, 40, 256),
+                                   (70, 90, 512), (40, 33, 513), (65, 20, 1024), (9, 70, 1030), (3, 5, 2500)])
+def test_diameter(n, m, d):
+    from flash_sinkhorn_amd.kernels._common import max_diameter
+    gen = torch.Generator(device="cuda").manual_seed(n + d)
+    x, y = (torch.randn(k, d, device="cuda", generator=gen) for k in (n, m))
+    def want(*clouds):
+        z = torch.cat(clouds).double()
+        return float((z.amax(0) - z.amin(0)).norm())
+    for cloud, row, col, far in [(x, 0, 0, 30.0), (x, -1, -1, -70.0), (y, m // 2, d // 2, 200.0), (y, -1, 0, -500.0)]:
+        cloud[row, col] = far
+        # d squares of one sign in fp32
+        for clouds in ((x, y), (x, x), (y, y)):
+            assert max_diameter(*clouds) == pytest.approx(want(*clouds), rel=(d / 16 + 16) * 2.0 ** -24, abs=1e-30)
+    assert max_diameter(x.half(), y.half()) == pytest.approx(want(x.half(), y.half()), rel=(d / 16 + 16) * 2.0 ** -24, abs=1e-30)
+    y[m // 2, -1] = float("nan")
+    assert math.isnan(max_diameter(x, y)) and not math.isnan(max_diameter(x, x))
+
+
 @pytest.mark.parametrize("n,m", [(1, 1), (63, 1025), (1024, 64), (8193, 20000)])
 def test_largest_change(n, m):
     from flash_sinkhorn_amd.sinkhorn_solvers import _largest_change, _max_change
