@@ -262,8 +262,9 @@ class SamplesLoss(torch.nn.Module):
             raise ValueError("flash_sinkhorn.SamplesLoss requires CUDA tensors.")
         config = self._make_config()
 
-        def ot(xb, yb, ab, bb, lx, ly, presolved=None):
-            sched = tuple(self._eps_list_for_inputs(xb, yb))
+        def ot(xb, yb, ab, bb, lx, ly, presolved=None, sched=None):
+            if sched is None:
+                sched = tuple(self._eps_list_for_inputs(xb, yb))
             of_points = (self.use_epsilon_scaling and self.diameter is None
                          and self.eps_list is None)
             return _SinkhornCostFn.apply(xb, yb, ab, bb, sched, config, lx, ly,
@@ -297,21 +298,23 @@ class SamplesLoss(torch.nn.Module):
             # clouds are launch bound, and the launches of medium ones leave CUs idle.  Their
             # results are handed to this stream with an event wait, and record_stream keeps the
             # allocator from reusing them early.
+            # (the schedules first: a diameter is waited for, and behind the solves that left the device without work)
+            sched_xy, sched_x, sched_y = (tuple(self._eps_list_for_inputs(p, q)) for p, q in ((xb, yb), (xb, xb), (yb, yb)))
             main = torch.cuda.current_stream(xb.device)
             if DEBIAS_SIDE_STREAM:
                 side = _side_stream(xb.device)
                 side.wait_stream(main)
                 with torch.cuda.stream(side):
                     pre_x, pre_y = solve_self_pair(xb, yb, ab, bb)
-                c = ot(xb, yb, ab, bb, label_x, label_y)
+                c = ot(xb, yb, ab, bb, label_x, label_y, sched=sched_xy)
                 main.wait_stream(side)
                 for t in pre_x + pre_y:
                     t.record_stream(main)
             else:
                 pre_x, pre_y = solve_self_pair(xb, yb, ab, bb)
-                c = ot(xb, yb, ab, bb, label_x, label_y)
-            return c - 0.5 * ot(xb, xb, ab, ab, label_x, label_x, pre_x) \
-                     - 0.5 * ot(yb, yb, bb, bb, label_y, label_y, pre_y)
+                c = ot(xb, yb, ab, bb, label_x, label_y, sched=sched_xy)
+            return c - 0.5 * ot(xb, xb, ab, ab, label_x, label_x, pre_x, sched_x) \
+                     - 0.5 * ot(yb, yb, bb, bb, label_y, label_y, pre_y, sched_y)
 
         if parsed.batched:
             items = list(zip(parsed.x, parsed.y, parsed.a, parsed.b))
