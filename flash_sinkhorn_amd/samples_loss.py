@@ -277,14 +277,15 @@ class SamplesLoss(torch.nn.Module):
         pair_ok = (self.backend == "symmetric" and self.threshold is None and not labelled
                    and self.rho_x == self.rho_y)
 
-        def solve_self_pair(xb, yb, ab, bb):
+        def solve_self_pair(xb, yb, ab, bb, scheds):
             return sinkhorn_flashstyle_symmetric_self_pair(
                 xb, ab, yb, bb, blur=self.blur, scaling=self.scaling,
                 use_epsilon_scaling=self.use_epsilon_scaling, eps=self.eps,
                 n_iters=self.n_iters, allow_tf32=self.allow_tf32,
                 use_exp2=self.use_exp2, cost_scale=self.cost_scale, rho=self.rho_x,
                 last_extrapolation=self.last_extrapolation,
-                return_prelast=self.last_extrapolation)
+                return_prelast=self.last_extrapolation,
+                _schedules=scheds if self.diameter is None and self.eps_list is None else None)
 
         def cost(xb, yb, ab, bb):
             # debias: OT(a,b) - OT(a,a)/2 - OT(b,b)/2
@@ -305,13 +306,13 @@ class SamplesLoss(torch.nn.Module):
                 side = _side_stream(xb.device)
                 side.wait_stream(main)
                 with torch.cuda.stream(side):
-                    pre_x, pre_y = solve_self_pair(xb, yb, ab, bb)
+                    pre_x, pre_y = solve_self_pair(xb, yb, ab, bb, (sched_x, sched_y))
                 c = ot(xb, yb, ab, bb, label_x, label_y, sched=sched_xy)
                 main.wait_stream(side)
                 for t in pre_x + pre_y:
                     t.record_stream(main)
             else:
-                pre_x, pre_y = solve_self_pair(xb, yb, ab, bb)
+                pre_x, pre_y = solve_self_pair(xb, yb, ab, bb, (sched_x, sched_y))
                 c = ot(xb, yb, ab, bb, label_x, label_y, sched=sched_xy)
             return c - 0.5 * ot(xb, xb, ab, ab, label_x, label_x, pre_x, sched_x) \
                      - 0.5 * ot(yb, yb, bb, bb, label_y, label_y, pre_y, sched_y)

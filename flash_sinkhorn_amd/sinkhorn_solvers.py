@@ -497,7 +497,7 @@ def sinkhorn_flashstyle_symmetric_self_pair(
     last_extrapolation: bool = True, cost_scale: float = 1.0,
     eps: Optional[float] = None, n_iters: Optional[int] = None,
     rho: Optional[float] = None, allow_tf32: bool = True, use_exp2: bool = True,
-    return_prelast: bool = False,
+    return_prelast: bool = False, _schedules=None,
 ):
     """The two self problems of a debiased divergence solved together.
 
@@ -537,7 +537,8 @@ def sinkhorn_flashstyle_symmetric_self_pair(
     _require_cuda(x, y)
     _validate_problem(x, y, [("a", a)], [("b", b)])
     xf, yf = x.detach().float().contiguous(), y.detach().float().contiguous()
-    ex, ey = schedule(xf), schedule(yf)
+    # (_schedules: those of a caller who has them; a diameter is waited for)
+    ex, ey = (list(e) for e in _schedules) if _schedules is not None else (schedule(xf), schedule(yf))
     if xf.shape[0] > 0 and yf.shape[0] > 0:
         alpha_x, alpha_y, log_a, log_b, fx, fy = _row_start(xf, yf, _f32c(a.detach()), _f32c(b.detach()), cost_scale)
     else:
