@@ -231,7 +231,8 @@ __device__ __forceinline__ PairMode pair_mode(const PairKnown& k, float units, b
   float most = -3.0e38f;       // log2 of every sum is below that
   // (whole numbers, which fp16 holds)
   auto fit = [&]() {
-    mode.shift = most > kPairMost ? ceilf(most - kPairMost) : (mode.low < kPairLeast ? floorf(mode.low - kPairLeast) : 0.f);
+    // (one of the two is zero, or no number fits; by branches, in front of every step: 0.15 us of 26 at 10,850 x 7,531 x 23)
+    mode.shift = fmaxf(ceilf(most - kPairMost), 0.f) + fminf(floorf(mode.low - kPairLeast), 0.f);
     return (most - mode.shift <= kPairMost) & (mode.low - mode.shift >= kPairLeast) & (fabsf(mode.shift) < 2000.f);
   };
   if (step == 0) {
