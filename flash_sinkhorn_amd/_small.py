@@ -581,6 +581,26 @@ class _Ask:
     def __call__(self, grad_out, tensors, need):
         return _differentiate(self.form, self.config, grad_out, tensors, need)
 
+    def node(self, tensors, shape, given):
+        """A tensor whose node is a Function's with the same gradient, of stand-ins for x, y and the weights: compiled
+        autograd records such a node as a call."""
+        with torch.enable_grad():
+            return _LateLoss.apply(self, tensors, shape, *given)
+
+
+class _LateLoss(torch.autograd.Function):
+    """See ``_Ask.node``."""
+
+    @staticmethod
+    def forward(ctx, ask, tensors, shape, x, y, a, b):
+        ctx.ask = ask
+        ctx.save_for_backward(*tensors)
+        return tensors[2].new_empty(shape, dtype=torch.float32)
+
+    @staticmethod
+    def backward(ctx, grad_out):
+        return (None, None, None) + tuple(ctx.ask(grad_out, ctx.saved_tensors, ctx.needs_input_grad[3:]))
+
 
 _NATIVE = None
 

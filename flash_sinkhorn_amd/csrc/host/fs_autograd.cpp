@@ -44,11 +44,7 @@ struct SmallLoss : public Node {
   }
 
   variable_list apply(variable_list&& grads) override {
-    std::array<Tensor, kSaved> t;
-    {
-      std::lock_guard<std::mutex> lock(mutex_);
-      for (int i = 0; i < kSaved; ++i) t[i] = saved[i].unpack();
-    }
+    const std::array<Tensor, kSaved> t = unpacked();
     const Tensor out = grads[0].defined() ? grads[0] : at::zeros(shape, t[2].options().dtype(at::kFloat));
     std::array<bool, 4> need;
     for (int i = 0; i < 4; ++i) need[i] = edge[i] >= 0 && task_should_compute_output(edge[i]);
@@ -76,6 +72,13 @@ struct SmallLoss : public Node {
     return result;
   }
 
+  std::array<Tensor, kSaved> unpacked() {
+    std::lock_guard<std::mutex> lock(mutex_);
+    std::array<Tensor, kSaved> t;
+    for (int i = 0; i < kSaved; ++i) t[i] = saved[i].unpack();
+    return t;
+  }
+
   template <typename Give>
   void ask_python(const Tensor& out, const std::array<Tensor, kSaved>& t, const std::array<bool, 4>& need, Give&& give) {
     py::gil_scoped_acquire gil;
@@ -88,9 +91,53 @@ struct SmallLoss : public Node {
   }
 
   void release_variables() override {
-    std::lock_guard<std::mutex> lock(mutex_);
-    for (SavedVariable& v : saved) v.reset_data();
+    {
+      std::lock_guard<std::mutex> lock(mutex_);
+      for (SavedVariable& v : saved) v.reset_data();
+    }
+    std::shared_ptr<Node> gone;  // (with Python in it: not under the lock)
+    std::lock_guard<std::mutex> lock(late_lock);
+    gone.swap(late);
   }
+
+  // Compiled autograd (PyTorch's, which records a backward pass as a graph): left to a node of a Python Function over the
+  // same tensors, whose call it records as one operation.  It goes through the nodes of a pass one after the other, on one thread.
+  void compiled_args(torch::dynamo::autograd::CompiledNodeArgs& args) const override {
+    std::array<Tensor, kSaved> t;
+    {
+      py::gil_scoped_release release;  // (a hook that unpacks a tensor takes it, under the node's lock)
+      t = const_cast<SmallLoss*>(this)->unpacked();
+    }
+    py::list tensors, given;
+    for (const Tensor& v : t) tensors.append(v.defined() ? py::cast(v) : py::none());
+    for (int i = 0; i < 4; ++i) {  // stand-ins: where the gradients go is this node's
+      if (edge[i] < 0) {
+        given.append(py::none());
+        continue;
+      }
+      const torch::autograd::Edge& e = next_edge(edge[i]);
+      if (!e.is_valid()) {
+        given.append(py::cast(at::empty({0}, t[2].options().dtype(at::kFloat))));
+        continue;
+      }
+      const torch::autograd::InputMetadata& m = e.function->input_metadata(e.input_nr);
+      given.append(py::cast(at::empty_symint(m.shape_as_dim_vector(), m.options()).requires_grad_()));
+    }
+    const py::object out = py::reinterpret_borrow<py::object>(ask.ptr(getPyInterpreter())).attr("node")(tensors, shape, given);
+    std::shared_ptr<Node> node = out.cast<Tensor>().grad_fn();
+    if (node) node->compiled_args(args);
+    std::lock_guard<std::mutex> lock(late_lock);
+    late.swap(node);
+  }
+  variable_list apply_with_saved(const variable_list& inputs, torch::dynamo::autograd::SwapSavedVariables& saved) override {
+    std::shared_ptr<Node> node;
+    {
+      std::lock_guard<std::mutex> lock(late_lock);
+      node = late;
+    }
+    return node ? node->apply_with_saved(inputs, saved) : variable_list(num_outputs());
+  }
+
   std::string name() const override { return "SmallLossBackward"; }
 
   fs_small_problem form;
@@ -100,6 +147,8 @@ struct SmallLoss : public Node {
   std::array<SavedVariable, kSaved> saved;
   std::array<int, 4> edge{-1, -1, -1, -1};  // of x, y and the weights that there are
   bool plain;
+  mutable std::shared_ptr<Node> late;  // see compiled_args
+  mutable std::mutex late_lock;
 };
 
 // Whether autograd sees nothing in these tensors but what a node of this kind serves: no transform of functorch, no
