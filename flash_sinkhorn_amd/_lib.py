@@ -120,6 +120,22 @@ def lib() -> ctypes.CDLL:
     return _lib
 
 
+def native():
+    """The module built against PyTorch, beside the library (csrc/host)."""
+    try:
+        from flash_sinkhorn_amd import _native as module
+    except ImportError as e:
+        raise RuntimeError(f"flash_sinkhorn_amd._native is missing or does not load ({e}): build it with "
+                           f"`make -C {CSRC_DIR}`.") from e
+    return module
+
+
+def ordinary(*tensors: torch.Tensor) -> bool:
+    """Whether these carry nothing that only tensor operations pass on: no tangents, no transform of functorch, no
+    subclass."""
+    return native().ordinary(list(tensors))
+
+
 def check(code: int, what: str) -> None:
     if code != 0:
         msg = lib().fs_error_string(code).decode()

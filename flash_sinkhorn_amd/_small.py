@@ -609,12 +609,7 @@ def _native():
     """The module with the native node, and the address of the gradient it calls."""
     global _NATIVE
     if _NATIVE is None:
-        try:
-            from flash_sinkhorn_amd import _native as module
-        except ImportError as e:
-            raise RuntimeError(f"flash_sinkhorn_amd._native is missing or does not load ({e}): build it with "
-                               f"`make -C {_lib.CSRC_DIR}`.") from e
-        _NATIVE = module, ctypes.cast(_lib.lib().fs_small_grad, _P).value
+        _NATIVE = _lib.native(), ctypes.cast(_lib.lib().fs_small_grad, _P).value
     return _NATIVE
 
 

@@ -47,7 +47,7 @@ def c_transform_fwd(x: torch.Tensor, y: torch.Tensor, psi: torch.Tensor, *,
                                   "Detach y or use a solver that supports grad_y.")
     with torch.no_grad():
         xf, yf, pf = _f32c(x), _f32c(y), _f32c(psi)
-        if n == 0:
+        if n == 0 or not _lib.ordinary(x, y, psi):  # (tangents go through tensor operations)
             bias, x_sq = cost_scale * (yf * yf).sum(dim=1) - pf, cost_scale * (xf * xf).sum(dim=1)
         else:
             x_sq, bias = (torch.empty(k, device=x.device, dtype=torch.float32) for k in (n, m))

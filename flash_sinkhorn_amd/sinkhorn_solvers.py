@@ -91,6 +91,12 @@ def _max_change(f, g, prev_f, prev_g) -> float:
     return max((f - prev_f).abs().max().item(), (g - prev_g).abs().max().item())
 
 
+def _starts_plain(x, y, a, b) -> bool:
+    """Whether a solve may start from ``_row_start``, which neither gradients nor tangents pass through."""
+    return (x.shape[0] > 0 and y.shape[0] > 0 and _lib.ordinary(x, y, a, b)
+            and not (torch.is_grad_enabled() and any(t.requires_grad for t in (x, y, a, b))))
+
+
 def _row_start(xf, yf, a, b, cost_scale):
     """cost_scale |row|^2 and log weights of both clouds and the potentials that a solve starts from, in one launch."""
     n, m = xf.shape[0], yf.shape[0]
@@ -151,11 +157,10 @@ def sinkhorn_flashstyle_alternating(
         f, g = s.potentials("f")[0], s.potentials("g")[0]
         return (f, g, s.entries) if return_n_iters else (f, g)
     xf, yf = x.float().contiguous(), y.float().contiguous()
-    plain = xf.shape[0] > 0 and yf.shape[0] > 0 and not (
-        torch.is_grad_enabled() and any(t.requires_grad for t in (x, y, a, b)))
+    plain = _starts_plain(x, y, a, b)
     if plain:
         alpha, beta, log_a, log_b, f_hat, g_hat = _row_start(xf, yf, _f32c(a), _f32c(b), cost_scale)
-    else:  # (alpha and beta pass gradients on to the points)
+    else:  # (alpha and beta pass gradients and tangents on to the points)
         alpha = cost_scale * (xf * xf).sum(dim=1)
         beta = cost_scale * (yf * yf).sum(dim=1)
         log_a, log_b = log_weights(a), log_weights(b)
@@ -262,8 +267,7 @@ def sinkhorn_flashstyle_symmetric(
     _require_cuda(x, y)
     _validate_problem(x, y, [("a", a)], [("b", b)])
     xf, yf = x.float().contiguous(), y.float().contiguous()
-    if xf.shape[0] > 0 and yf.shape[0] > 0 and not (
-            torch.is_grad_enabled() and any(t.requires_grad for t in (x, y, a, b))):
+    if _starts_plain(x, y, a, b):
         alpha, beta, log_a, log_b, f_hat, g_hat = _row_start(xf, yf, _f32c(a), _f32c(b), cost_scale)
     else:
         alpha = (cost_scale * (xf * xf).sum(dim=1)).contiguous()

@@ -1459,3 +1459,25 @@ def test_largest_change(n, m):
     f[0] = -float("nan")
     same()
     assert _largest_change(p, q[1:], p, q[1:]) == 0.0 if m > 1 else True
+
+
+# Tangents (forward-mode differentiation) go through the tensor operations around the kernels: of a potential or a c-transform
+# there is that of cost_scale |x|^2, whatever the sizes.
+def test_tangents_of_squared_norms():
+    import torch.autograd.forward_ad as fw
+
+    from flash_sinkhorn_amd import c_transform_fwd
+    from flash_sinkhorn_amd.kernels import sinkhorn_flashstyle_alternating, sinkhorn_flashstyle_symmetric
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    x, t = (torch.randn(40, 3, device="cuda", generator=gen) for _ in range(2))
+    y, psi = torch.randn(50, 3, device="cuda", generator=gen), torch.randn(50, device="cuda", generator=gen)
+    a, b = torch.full((40,), 1 / 40, device="cuda"), torch.full((50,), 1 / 50, device="cuda")
+    kw = dict(eps=0.1, n_iters=2, cost_scale=0.5)
+    with fw.dual_level():
+        X = fw.make_dual(x, t)
+        values = [sinkhorn_flashstyle_alternating(X, y, a, b, ott_convention=True, threshold=1e-9, check_every=1, **kw)[0],
+                  sinkhorn_flashstyle_symmetric(X, y, a, b, f_init=torch.zeros_like(a), use_epsilon_scaling=False, **kw)[0],
+                  c_transform_fwd(X, y, psi, cost_scale=0.5)[0]]
+        for v in values:
+            tangent = fw.unpack_dual(v).tangent
+            assert tangent is not None and rel_err(tangent, (x * t).sum(1).cpu().numpy()) < 1e-5
