@@ -553,8 +553,9 @@ def _differentiate(form: Problem, config: dict, grad_out, tensors, need):
 
 
 class _SmallLoss(torch.autograd.Function):
-    """Cost of every item, debiased or not, from one run; scalar for a single problem.  For tensors that only a
-    Function serves or refuses (tangents, functorch, subclasses); the others have a native node (``loss``)."""
+    """Cost of every item, debiased or not, from one run; scalar for a single problem.  For what only a Function
+    serves or refuses (tangents, any call inside a transform of functorch, subclasses); the others have a native
+    node (``loss``)."""
 
     @staticmethod
     def forward(ctx, x, y, a, b, loss, normalize):
@@ -616,7 +617,7 @@ def _native():
 def loss(module, x, y, a, b, normalize):
     given = [x, y, a, b]
     native, grad = _native()
-    if not native.ordinary(given):
+    if torch._C._are_functorch_transforms_active() or not native.ordinary(given):
         return _SmallLoss.apply(x, y, a, b, module, normalize)
     need = [torch.is_grad_enabled() and t is not None and t.requires_grad for t in given]
     s = _solve_for(module, x, y, a, b, normalize, self_terms=int(module.debias),

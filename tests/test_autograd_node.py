@@ -1,6 +1,7 @@
 """The native autograd node of a small loss (csrc/host/fs_autograd.cpp): what PyTorch asks of a node besides its
 backward pass."""
 import ctypes
+from types import SimpleNamespace
 
 import pytest
 import torch
@@ -51,6 +52,15 @@ def test_compiled_autograd(need):
         with compiled_autograd._enable(lambda graph: graph):
             got = gradients()
         assert all(torch.equal(g, w) for g, w in zip(got, want))
+
+
+# A loss of other tensors than those that a transform of functorch follows is refused as one of these is: a Function without rules
+# for transforms is, and the native node says nothing of them.
+def test_losses_inside_a_transform_are_refused(monkeypatch):
+    x, y = torch.randn(3, 2, requires_grad=True), torch.randn(4, 2)
+    monkeypatch.setattr(_small, "_solve_for", lambda *_, **__: pytest.fail("solved"))
+    with pytest.raises(RuntimeError, match="functorch"):
+        torch.func.grad(lambda s: s * _small.loss(SimpleNamespace(debias=False), x, y, None, None, False))(torch.tensor(2.0))
 
 
 @pytest.mark.gpu
