@@ -31,7 +31,9 @@ def log_weights(w: torch.Tensor) -> torch.Tensor:
 def max_diameter(x: torch.Tensor, y: torch.Tensor) -> float:
     """Length of the diagonal of the joint bounding box of x and y (host float; syncs)."""
     if (x.is_cuda and x.device == y.device and x.ndim == 2 and y.ndim == 2 and x.shape[1] == y.shape[1]
-            and x.numel() > 0 and y.numel() > 0 and x.is_floating_point() and y.is_floating_point()):
+            and x.numel() > 0 and y.numel() > 0 and x.is_floating_point() and y.is_floating_point()
+            and x.shape[1] <= 1 << 20 and max(x.shape[0], y.shape[0]) <= 1 << 30  # (what fs_diameter takes)
+            and _lib.ordinary(x, y)):
         xf = _f32c(x.detach())
         yf = xf if y is x else _f32c(y.detach())
         d = xf.shape[1]

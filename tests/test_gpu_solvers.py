@@ -1443,6 +1443,17 @@ def test_diameter(n, m, d):
     assert math.isnan(max_diameter(x, y)) and not math.isnan(max_diameter(x, x))
 
 
+# rows of more columns than the library takes (no solver does), and a cloud inside a transform of functorch
+def test_diameter_by_tensor_operations():
+    from flash_sinkhorn_amd.kernels._common import max_diameter
+    x = torch.zeros(2, (1 << 20) + 1, device="cuda")
+    x[1, -1] = 3.0
+    assert max_diameter(x, x) == 3.0
+    got = []
+    torch.func.grad(lambda t: (got.append(max_diameter(t, t)), t.sum())[1])(x[:, -4:].clone())
+    assert got == [3.0]
+
+
 @pytest.mark.parametrize("n,m", [(1, 1), (63, 1025), (1024, 64), (8193, 20000)])
 def test_largest_change(n, m):
     from flash_sinkhorn_amd.sinkhorn_solvers import _largest_change, _max_change
