@@ -309,7 +309,7 @@ __device__ void small_schedule(const SmallArgs& a, int item) {
       am = fmaxf(am, m);
       if (a.w[mat] == nullptr) wl = wh = 1.0f / (float)a.rows[mat];
       else if (a.normalize) wl /= fmaxf(ws, 1e-40f), wh /= fmaxf(ws, 1e-40f);
-      else mass = !(mass >= ws) ? ws : mass;  // (NaN too)
+      else mass = (ws > mass || !(ws == ws)) ? ws : mass;  // (NaN too, of either matrix)
       lim[2 * mat] = wl > 0.f ? small_log2(wl, 0.f) : -100000.0f * kLog2e;
       lim[2 * mat + 1] = wh > 0.f ? small_log2(wh, 0.f) : -100000.0f * kLog2e;
     }

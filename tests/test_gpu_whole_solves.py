@@ -331,6 +331,23 @@ def test_infinite_weights_on_opposite_clouds():
     assert all(torch.equal(g, w) for g, w in zip(solve(X, Y, A, B, **kw), want))
 
 
+# A weight that is not a number is none, as one of zero is, and nothing is known of its side's mass: the steps take both sides
+# apart then, whichever side it is on.
+@pytest.mark.parametrize("of_x", [False, True])
+def test_weights_that_are_no_numbers(of_x):
+    from flash_sinkhorn_amd.kernels import sinkhorn_flashstyle_symmetric as solve
+    x, y, a, b = inputs(5, 4620, 4513, 12, scale=0.5)
+    X, Y, A, B = dev(x, y, a, b)
+    heavy, at = (A, 17) if of_x else (B, 4400)
+    heavy *= 2.0 ** 30
+    kw = dict(use_epsilon_scaling=False, eps=0.05, n_iters=6)
+    heavy[at] = 0.0
+    want = solve(X, Y, A, B, **kw)
+    heavy[at] = float("nan")
+    for g, w in zip(solve(X, Y, A, B, **kw), want):
+        assert rel_err(g, w.cpu().numpy()) < POT
+
+
 @pytest.mark.parametrize("d", [4, 200])
 def test_relaxations_of_zero_and_less_are_not_strict_marginals(d):
     from flash_sinkhorn_amd import SamplesLoss, sinkhorn_solvers as S
