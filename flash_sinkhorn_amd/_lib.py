@@ -72,6 +72,7 @@ _SIGNATURES = {
     "fs_small_workspace_bytes": (_Z, [_P]),
     "fs_small_solve": (ctypes.c_int, [_P, _P, _Z, _P, _P, _P, _P]),
     "fs_small_products_bytes": (_Z, [_P]),
+    "fs_small_last_step_offset": (_Z, [_P, ctypes.c_int, ctypes.c_int]),
     "fs_small_solve_products": (ctypes.c_int, [_P, _P, _Z, _P, _Z, _P, _P, _P, _P]),
     "fs_small_potentials": (ctypes.c_int, [_P, _P, _Z, _P, _P]),
     "fs_hvp_workspace_bytes": (_Z, [_P]),

@@ -48,7 +48,8 @@ constexpr int kPairSlots = 8;        // copies of a step's extremes, over which 
 constexpr int kPairCounts = 3 * kPairSlots * 8;
 constexpr int kPairLists = kPairCounts + 3 * kPairSlots * 32;
 constexpr int kPairTaken = kPairLists + 3 * 32;  // per step and XCD, of the first problem: work items taken
-constexpr int kPairStateWords = kPairTaken + 3 * 8 * 32;
+constexpr int kPairModes = kPairTaken + 3 * 8 * 32;  // how the newest step was taken (PairMode)
+constexpr int kPairStateWords = kPairModes + 32;
 constexpr int kPairListWords = 4;    // 64-bit words per wavefront of a work item: [row block][half of the sub-tiles]
 constexpr int kPairMostTiles = 64;   // of a chunk
 constexpr float kPairGap = 44.f;     // base-2 distance below every sum at which a logit is left out
@@ -89,8 +90,11 @@ struct PairProblem {
   int two_first, two_items;
 };
 
-// How a step is taken (pair_mode): both sides from one sweep, and with which units.
-struct PairMode {
+// How a step is taken (pair_mode): both sides from one sweep, and with which units.  Found where the step begins, by the
+// sweep's workgroups, and left in the problem's state for the merge, which has to add the very shift that the sweep took off
+// (found a second time there, a settled step of 4,500 x 3 took 15.1 us, now 14.7, 4,500 x 8 the same, 4,800 x 4,300 x 16
+// 16.9 -> 16.3, 10,850 x 7,531 x 23 30.9 -> 30.4, 10,000 x 64 37.0 -> 36.4).
+struct PairMode {  // (the first five are an interface: fs_small_last_step_offset)
   int sweep;     // else two-sided with running maxima
   int list;      // only the units on the lists
   int coarse;    // units are ended by their coarse products where these allow it
@@ -104,6 +108,7 @@ struct PairMode {
   float rho;     // its logits over those of the step before
   float least[2];  // what the least change of the other rows' potentials adds to a logit of the rows of a side
 };
+static_assert(sizeof(PairMode) <= 32 * sizeof(float), "a cache line of the state");
 
 // One side of a problem in the merge: the rows whose potentials it updates.
 struct PairSide {
@@ -231,7 +236,7 @@ __device__ __forceinline__ PairMode pair_mode(const PairKnown& k, float units, b
   float most = -3.0e38f;       // log2 of every sum is below that
   // (whole numbers, which fp16 holds)
   auto fit = [&]() {
-    // (one of the two is zero, or no number fits; by branches, in front of every step: 0.15 us of 26 at 10,850 x 7,531 x 23)
+    // (one of the two is zero, or no number fits; by branches 0.15 us of a step at 10,850 x 7,531 x 23)
     mode.shift = fmaxf(ceilf(most - kPairMost), 0.f) + fminf(floorf(mode.low - kPairLeast), 0.f);
     return (most - mode.shift <= kPairMost) & (mode.low - mode.shift >= kPairLeast) & (fabsf(mode.shift) < 2000.f);
   };
@@ -261,7 +266,8 @@ __device__ __forceinline__ PairMode pair_mode(const PairKnown& k, float units, b
   mode.least[0] = -kappa * e[7];
   mode.least[1] = -kappa * e[3];
   mode.low = 3.0e38f;
-  const bool averaged = strict && step >= 2;
+  // (no bound by the mean, where the step before was no average; a select: this is in front of every step)
+  const float slack = strict & (step >= 2) ? 1.f : 3.0e38f;
 #pragma unroll
   for (int s = 0; s < 2; ++s) {
     // this side's sums: weights of its own rows (w) and of the others' (k)
@@ -271,8 +277,8 @@ __device__ __forceinline__ PairMode pair_mode(const PairKnown& k, float units, b
     const float up = rho >= 1.f ? -(rho - 1.f) * kmin : (1.f - rho) * mass;
     const float dn = rho >= 1.f ? -(rho - 1.f) * mass : (1.f - rho) * kmin;
     // (linear in the row's own weight, so largest at one end of it)
-    const float mean = fmaxf(rho * 0.5f * (mass - wmin) + (wmin - wmax), rho * 0.5f * (mass - wmax)) + 1.f;
-    const float U = (averaged ? fminf(rho * hi, mean) : rho * hi) + up - kmax, L = rho * lo + dn + (wmin - wmax) - kmax;
+    const float mean = fmaxf(rho * 0.5f * (mass - wmin) + (wmin - wmax), rho * 0.5f * (mass - wmax)) + slack;
+    const float U = fminf(rho * hi, mean) + up - kmax, L = rho * lo + dn + (wmin - wmax) - kmax;
     ok = ok & (U < 3.0e38f) & (L > -3.0e38f);  // (false where anything is not a number)
     most = fmaxf(most, U);
     mode.low = fminf(mode.low, L);
@@ -1467,7 +1473,10 @@ __global__ __launch_bounds__(256, 2) void pair_sweep_kernel(PairArgsPtr args, in
     if (SKIP)
       bits |= (live && m.sweep && m.coarse && !m.list ? 64u : 0u) | (live && m.list ? 512u : 0u) | (m.two ? 4096u : 0u);
     bits <<= own;
-    if (lane == 0 && (single || own == wave)) modes[own] = m;
+    if (lane == 0 && (single || own == wave)) {
+      modes[own] = m;
+      if (blockIdx.x == 0 && live) *reinterpret_cast<PairMode*>(a.state + ((size_t)batch * 3 + own) * kPairStateWords + kPairModes) = m;
+    }
     if (threadIdx.x < 3) went[threadIdx.x] = 0u;
   }
   if (!single) {
@@ -1605,6 +1614,7 @@ __global__ __launch_bounds__(1024) void pair_merge_kernel(PairArgsPtr args, int 
   const int from = step < 0 ? 0 : step & 1;
   const float old = sd.pot[from * (size_t)a.items * sd.rows + at], norm = sd.norm[at], weight = sd.l2w[at];
   const int entries = a.lens[item * 3 + prob];
+  const PairMode mode = *reinterpret_cast<const PairMode*>(state + kPairModes);
   const PairKnown known = pair_known(a, item, prob, max(step, 0));
   if (step > entries + a.extrapolate) return;
   const float4 next = step < 0 ? known.now : known.next;
@@ -1627,14 +1637,6 @@ __global__ __launch_bounds__(1024) void pair_merge_kernel(PairArgsPtr args, int 
     __shared__ float sh_ex[4][4];
     const float4 coef = known.now;
     const float r = __builtin_fmaf(coef.w, old, l2w);  // the row's bias in this step
-    // (one wavefront decides for all: sixteen would take a SIMD's turns from each other)
-    __shared__ PairMode sh_mode;
-    if (wave == 0) {
-      const PairMode m = pair_mode(known, SKIP ? a.prob[prob].units : 0.f, SKIP && a.prob[prob].ends, a.prob[prob].strict, prob, step);
-      if (lane == 0) sh_mode = m;
-    }
-    __syncthreads();
-    const PairMode mode = sh_mode;
     const bool sweep = __builtin_amdgcn_readfirstlane(mode.sweep), ended = __builtin_amdgcn_readfirstlane(mode.two);
     float2 mine = make_float2(kNegBig, 0.f);
     int best = -1;

@@ -593,6 +593,15 @@ size_t fs_small_products_bytes(const fs_small_problem* p) {
   return products_at(a, nullptr).bytes;
 }
 
+size_t fs_small_last_step_offset(const fs_small_problem* p, int item, int prob) {
+  if (checked(p) != FS_OK || !use_pair(p) || item < 0 || item >= p->items || prob < 0 || prob > 2) return 0;
+  SmallArgs a;
+  PairArgs t;
+  layout(p, nullptr, a, &t);
+  if (prob < t.first_prob || prob >= t.nprob) return 0;
+  return reinterpret_cast<size_t>(t.state) + (((size_t)item * 3 + prob) * kPairStateWords + kPairModes) * 4;
+}
+
 int fs_small_solve(const fs_small_problem* p, void* workspace, size_t workspace_bytes, int* host_words,
                    float* loss, float* pots, void* stream) {
   return fs_small_solve_products(p, workspace, workspace_bytes, nullptr, 0, host_words, loss, pots, stream);

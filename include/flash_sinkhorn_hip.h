@@ -457,6 +457,13 @@ int fs_small_solve_products(const fs_small_problem* problem, void* workspace, si
                             size_t products_bytes, int* host_words, float* loss, float* pots, void* stream);
 
 /*
+ * Where a solve's workspace says how its last step took a problem (0: xy, 1: xx, 2: yy) of an item: the byte offset of three
+ * ints (both sides from one sweep; along lists; units end at coarse products) and two floats (a lower bound on log2 of every
+ * sum; what was taken off every base-2 logit of a one-sweep step).  0: steps of this problem are of one kind.
+ */
+size_t fs_small_last_step_offset(const fs_small_problem* problem, int item, int prob);
+
+/*
  * The standard potentials of the solve that left `workspace` behind, each into memory of its own.
  * pots: a HOST array of 8 device pointers, NULL where not wanted: f, f before the extrapolation
  * ([items, n]), g, g before it ([items, m]), and with self_terms likewise those of (x, x) and of (y, y)

@@ -244,6 +244,51 @@ def test_one_sweep_steps_whose_sums_need_a_shift(n, m, d, eps, rho, mass, n_iter
                     rho_x=rho, rho_y=rho)
 
 
+# ... and that a shift of either sign was taken off the last step's logits (small sums: units that end at coarse products, and
+# every logit; large bounds: an eps that falls to a tenth from one step to the next).  Want: double precision.
+@pytest.mark.parametrize("n,m,d,scale,rho,mass,kw,sign", [
+    (4513, 4481, 20, 0.5, None, 1.3, dict(eps=0.003, entries=2, extrapolate=True), -1),
+    (4513, 4481, 20, 0.5, 0.1, 1.0, dict(eps=0.005, entries=4, extrapolate=True), -1),
+    (4513, 4481, 36, 0.5, None, 1.0, dict(blur=0.1, scaling=0.2, extrapolate=True), -1),
+    (4513, 4481, 36, 0.5, None, 1.0, dict(blur=0.1, scaling=0.3, cut=5, extrapolate=False), 1),
+    (4513, 4481, 36, 0.1, None, 1.0, dict(blur=0.1, scaling=0.25, cut=5, extrapolate=False), 1),
+    (4513, 4481, 36, 0.5, 0.7, 1.0, dict(blur=0.1, scaling=0.3, cut=4, extrapolate=False), 1)])
+def test_shifts_of_one_sweep_steps(n, m, d, scale, rho, mass, kw, sign):
+    import ctypes
+
+    from flash_sinkhorn_amd import _lib, _small
+    from flash_sinkhorn_amd.kernels._common import epsilon_schedule, max_diameter
+    x, y, a, b = inputs(n + d, n, m, d, scale=scale, y_shift=0.2)
+    X, Y, A, B = dev(x, y, a, (mass * b).astype(b.dtype))
+    eps = [kw["eps"]] * kw["entries"] if "eps" in kw else epsilon_schedule(
+        max_diameter(X, Y), kw["blur"], kw["scaling"])[:kw.get("cut")]
+    s = _small.solve(*_small.points(X, Y), A, B, items=1, cost_scale=1.0, rho_x=rho, rho_y=rho, normalize=False, self_terms=0,
+                     want_values=False, want_loss=False, keep=True, **kw)
+    at = _lib.lib().fs_small_last_step_offset(ctypes.byref(s.problem()), 0, 0)
+    words = s.ws[at:at + 20].cpu().numpy()
+    assert words[:4].view(np.int32)[0] == 1 and np.sign(words[16:].view(np.float32)[0]) == sign
+
+    U, V = X.double(), Y.double()
+    cost = (U * U).sum(1)[:, None] + (V * V).sum(1) - 2.0 * U @ V.T
+    la, lb = A.double().log()[:, None], B.double().log()
+    f, g = torch.zeros(n, 1, device="cuda").double(), torch.zeros(m, device="cuda").double()
+
+    def halves(e):
+        damp = 1.0 if rho is None else 1.0 / (1.0 + e / rho)
+        return (-e * damp * torch.logsumexp((g - cost) / e + lb, 1, keepdim=True),
+                -e * damp * torch.logsumexp((f - cost) / e + la, 0))
+    f, g = halves(eps[0])
+    for e in eps:
+        new = halves(e)
+        f, g = 0.5 * (f + new[0]), 0.5 * (g + new[1])
+    if kw["extrapolate"]:
+        f, g = halves(eps[-1])
+    # (four steps' worth of 2^-21 of the largest cost each)
+    off = 4.0 * 2.0 ** -21 * float(cost.max())
+    for got, want in ((s.potentials("f")[0], f[:, 0]), (s.potentials("g")[0], g)):
+        assert float((got.double() - want).abs().max()) < off
+
+
 # a whole schedule on these kernels (planes written behind every step), as long as it is
 def test_one_sweep_steps_of_a_full_schedule():
     from flash_sinkhorn_amd.kernels import sinkhorn_flashstyle_symmetric as solve
