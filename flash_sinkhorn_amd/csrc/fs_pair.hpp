@@ -195,7 +195,8 @@ __device__ __forceinline__ float pair_value(unsigned k) {
 // <= rho x - (rho - 1) log2 b_min  (and the other way round for rho < 1).  The biases count the
 // weights from the largest of their side (so that logits are small where eps is large, and what a
 // matrix product rounds off them is too).  Every sum has to lie in [2^-84, 2^120] once all logits are
-// shifted by one number: then no exponential overflows, and what is lost below 2^-126 is less
+// shifted by one number: then no exponential overflows (kappa f is up to 6e7 units, where a float's step is 4 and a
+// logit's rounding as much: see the merge), and what is lost below 2^-126 is less
 // than 2^-26 of a sum with 65,536 terms.  Before the first step the potentials are minus the norms,
 // so e_ij = -C_ij / eps >= -bound / eps.
 // By every lane of a wavefront with the same result; `set`: which of the three sets to read.
@@ -1688,7 +1689,11 @@ __global__ __launch_bounds__(1024) void pair_merge_kernel(PairArgsPtr args, int 
     const float2(&all)[4][64] = sh[quarter];
     float lse;
     if (sweep) {
-      lse = small_log2((all[0][lane].y + all[1][lane].y) + (all[2][lane].y + all[3][lane].y), others + mode.shift) - r;
+      // (fp32 holds every sum, by eight units from the bounds; where potentials of some 10^7 units cancel, logits and bounds are
+      // off by rounding themselves: what that takes past the range ends there, no further off than its logits are, and a
+      // potential stays a number.  NaN stays.)
+      const float sum = (all[0][lane].y + all[1][lane].y) + (all[2][lane].y + all[3][lane].y);
+      lse = small_log2(sum > 3.4e38f ? 3.4e38f : (sum < 1.2e-38f ? 1.2e-38f : sum), others + mode.shift) - r;
     } else {
       float M = kNegBig, s = 0.f;
 #pragma unroll

@@ -289,6 +289,31 @@ def test_shifts_of_one_sweep_steps(n, m, d, scale, rho, mass, kw, sign):
         assert float((got.double() - want).abs().max()) < off
 
 
+# ... of clouds so far from zero that a float's step at their potentials is 2 to 4 base-2 units: every cost is the same, so the
+# bounds are as tight as they come, a few units below what fp32 holds
+@pytest.mark.parametrize("rho", [None, 3.0])
+@pytest.mark.parametrize("far,units", [(30.0, 200.0), (100.0, 600.0), (100.0, 1500.0), (250.0, 1000.0)])
+def test_shifts_far_from_zero(far, units, rho):
+    import ctypes
+
+    from flash_sinkhorn_amd import _lib, _small
+    n, m, d = 4500, 4480, 16
+    per_unit = (2.8e7 - units) / (d * far * far)  # base-2 units per unit of cost
+    x, y = torch.full((n, d), far, device="cuda"), torch.full((m, d), far - (units / per_unit / d) ** 0.5, device="cuda")
+    a, b = torch.full((n,), 1 / n, device="cuda"), torch.full((m,), 1 / m, device="cuda")
+    cost, eps = float(((x[0] - y[0]).double() ** 2).sum()), 1.0 / (per_unit * np.log(2.0))
+    s = _small.solve(x, y, a, b, items=1, eps=eps, entries=1, cost_scale=1.0, rho_x=rho, rho_y=rho, normalize=False,
+                     self_terms=0, want_values=False, extrapolate=False, want_loss=False, keep=True)
+    at = _lib.lib().fs_small_last_step_offset(ctypes.byref(s.problem()), 0, 0)
+    words = s.ws[at:at + 20].cpu().numpy()
+    assert words[:4].view(np.int32)[0] == 1 and words[16:].view(np.float32)[0] != 0.0
+    damp = 1.0 if rho is None else 1.0 / (1.0 + eps / rho)
+    first = damp * cost
+    want = 0.5 * first + 0.5 * damp * (cost - first)
+    for which in "fg":  # (two steps; the logits of each are off by 2^-21 of the largest product, as everywhere)
+        assert float((s.potentials(which)[0] - want).abs().max()) < 2.0 ** -19 * 2 * d * far * far
+
+
 # a whole schedule on these kernels (planes written behind every step), as long as it is
 def test_one_sweep_steps_of_a_full_schedule():
     from flash_sinkhorn_amd.kernels import sinkhorn_flashstyle_symmetric as solve
