@@ -89,6 +89,7 @@ _SIGNATURES = {
     "fs_change": (ctypes.c_int, [_P, _P, _I, _P, _P, _I, _P, _P]),
 }
 EXPORTED_SYMBOLS = tuple(_SIGNATURES)
+VERSION = 2  # FS_VERSION of the header that these signatures and the structs beside them were written for
 
 
 def build(verbose: bool = False, force: bool = False) -> str:
@@ -113,6 +114,9 @@ def lib() -> ctypes.CDLL:
                 f"{LIB_PATH} is missing: build it with `make -C {CSRC_DIR}` "
                 "(flash_sinkhorn_amd has no non-HIP code path).")
         handle = ctypes.CDLL(LIB_PATH)
+        if handle.fs_version() != VERSION:
+            raise RuntimeError(f"{LIB_PATH} has interface {handle.fs_version()}, this package {VERSION}: build it again "
+                               f"with `make -C {CSRC_DIR}`.")
         for name, (res, args) in _SIGNATURES.items():
             fn = getattr(handle, name)
             fn.restype = res

@@ -1396,7 +1396,7 @@ using namespace fs;
 
 extern "C" {
 
-int fs_version(void) { return 1; }
+int fs_version(void) { return FS_VERSION; }
 
 const char* fs_error_string(int code) {
   switch (code) {

@@ -125,6 +125,10 @@ extern "C" {
 #define FS_OP_MAT5 5
 #define FS_OP_C_TRANSFORM 6
 
+/* Raised where a struct of this header or the meaning of an argument changes: a program built against another number must not
+ * call the rest (structs carry no size; fields that it does not know would be read behind its own).  Zero a struct before it is
+ * filled in: zero is every field's default. */
+#define FS_VERSION 2
 int fs_version(void);
 const char* fs_error_string(int code);
 

@@ -25,6 +25,16 @@ def test_library_exports_every_declared_symbol():
     assert _lib.lib().fs_error_string(-4) == b"workspace too small"
 
 
+# structs carry no size: a library of another layout is not called
+def test_a_library_of_another_interface_is_refused(monkeypatch):
+    header = open(os.path.join(ROOT, "include", "flash_sinkhorn_hip.h")).read()
+    assert int(re.search(r"#define FS_VERSION (\d+)", header).group(1)) == _lib.VERSION == _lib.lib().fs_version() > 1
+    monkeypatch.setattr(_lib, "_lib", None)
+    monkeypatch.setattr(_lib, "VERSION", 1)
+    with pytest.raises(RuntimeError, match="interface"):
+        _lib.lib()
+
+
 def test_c_abi_rejects_bad_arguments_before_any_launch():
     L = _lib.lib()
     fake = 0x1000  # never dereferenced: every call below fails validation on the host
