@@ -152,7 +152,8 @@ __global__ __launch_bounds__(512) void dense_prep_kernel(const SmallArgs a, cons
 
 // One operand's tile stream and C = A B^T: a workgroup of WR x WC wavefronts owns 32 WR RB rows and
 // 32 WC CB columns; per 16-column step both operands' blocks come into one of ST LDS stages by
-// direct global -> LDS loads of 1 KiB per wavefront, ST - 1 steps ahead, one barrier per step.
+// direct global -> LDS loads of 1 KiB per wavefront: with four stages three steps ahead and a barrier per step, with eight six
+// steps ahead and a barrier per two (dense_gemm_tile).
 // Bound by the matrix pipe: RB CB 3 MFMAs per wavefront and step against 2 (RB + CB) LDS reads.
 // LDS reads are written out by hand (the compiler would have each wait for the loads in flight).
 struct DenseGemmArgs {

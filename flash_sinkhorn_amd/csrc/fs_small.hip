@@ -48,7 +48,7 @@ bool use_pair(const fs_small_problem* p) {
 bool use_dense(const fs_small_problem* p) { return p->d > kSmallMaxD; }
 
 // Narrower rows whose products are formed once and kept for the steps of a solve (dense_rows_kernel).  A workgroup
-// of small_step_kernel reads the planes of all keys for 32 rows, 2, 4, 8 or 16 bytes a logit by the padded width, from the
+// of small_step_kernel reads the planes of all keys for 32 rows, 2, 4, 6, 8, 12 or 16 bytes a logit by the padded width, from the
 // caches; a kept product is 4.  `read`: the bytes of a step, which come from the last-level cache, against the narrower
 // planes.  Potentials after 50 steps at a fixed eps, and after a schedule of 14, planes -> products, us:
 //   d = 64:  256 points 243 -> 196, 91 -> 94; 1,000: 370 -> 238, 131 -> 102; 2,048 (32 MiB): 553 -> 395, 187 -> 152;

@@ -59,8 +59,6 @@ def test_schedules_of_every_length(n, m, d, cut):
         assert rel_err(f, wf) < POT and rel_err(g, wg) < POT
 
 
-# ---- wide rows, one launch per step (up to 1e7 products and 4,096 keys): one and two rows a wavefront, pieces
-# of 1,024 keys, and the sizes just past the line ----
 # lengths of schedules, from boxes whose farthest corner lies in one block of rows and one column of either cloud (up to
 # 64 blocks, sixteen threads a column or as many as 256 hold)
 @pytest.mark.parametrize("n,m,d", [(2, 3, 1), (40, 33, 2), (300, 65, 3), (513, 290, 15), (260, 545, 16), (1100, 2049, 17),
@@ -118,6 +116,8 @@ def test_losses_from_their_potentials(n, m, reach, debias):
     assert abs(float(got) - float(want)) < 3e-6 * abs(float(cost(a, x, b, y)))
 
 
+# ---- wide rows, one launch per step (up to 1e7 products and 4,096 keys): one and two rows a wavefront, pieces
+# of 1,024 keys, and the sizes just past the line ----
 @pytest.mark.parametrize("n,m,d", [(1, 1, 129), (5, 300, 130), (1023, 1025, 200), (1024, 1025, 140),
                                    (2400, 4096, 129), (30, 4097, 129), (2441, 4096, 131)])
 def test_wide_steps_of_one_launch(n, m, d):
