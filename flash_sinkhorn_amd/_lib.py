@@ -39,6 +39,7 @@ TILE_SKIP = os.environ.get("FLASH_SINKHORN_TILE_SKIP", "1") != "0"
 # once the potentials move little from step to step (FS_FLAG_NO_SWEEP switches that off)
 SWEEP = os.environ.get("FLASH_SINKHORN_SWEEP", "1") != "0"
 _lib: Optional[ctypes.CDLL] = None
+_native = None
 
 _P = ctypes.c_void_p
 _I = ctypes.c_int64
@@ -127,18 +128,21 @@ def lib() -> ctypes.CDLL:
 
 def native():
     """The module built against PyTorch, beside the library (csrc/host)."""
-    try:
-        from flash_sinkhorn_amd import _native as module
-    except ImportError as e:
-        raise RuntimeError(f"flash_sinkhorn_amd._native is missing or does not load ({e}): build it with "
-                           f"`make -C {CSRC_DIR}`.") from e
-    return module
+    global _native
+    if _native is None:
+        try:
+            from flash_sinkhorn_amd import _native as module
+        except ImportError as e:
+            raise RuntimeError(f"flash_sinkhorn_amd._native is missing or does not load ({e}): build it with "
+                               f"`make -C {CSRC_DIR}`.") from e
+        _native = module
+    return _native
 
 
 def ordinary(*tensors: torch.Tensor) -> bool:
     """Whether these carry nothing that only tensor operations pass on: no tangents, no transform of functorch, no
     subclass."""
-    return native().ordinary(list(tensors))
+    return native().ordinary(tensors)
 
 
 def check(code: int, what: str) -> None:
