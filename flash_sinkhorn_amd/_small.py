@@ -125,6 +125,12 @@ def _size_ok(n: int, m: int, d: int, fixed: bool, self_terms: int, stops: bool,
     and 12 columns:
       50,000: 6.1 / 5.6, 7.3 / 10.3, 5.9 / 5.7 | 8.9 / 8.1, 12.0 / 16.8, 7.4 / 8.4 | 24.0 / 25.1, 42.6 / 60.1, 16.2 / 26.4
       65,000: 9.6 / 7.9, 11.7 / 15.7, 9.1 / 7.9 | 13.9 / 11.0, 19.5 / 26.1, 11.1 / 11.4 | 36.5 / 32.4, 71.9 / 95.6, 23.2 / 32.8
+    and 40 columns, whose planes are 48 wide here and 64 there, so that the line is too high for 33 .. 48 of them (it stands where
+    64 columns have it):
+      32,000: 3.1 / 4.5, 4.8 / 5.8, 3.9 / 5.7 | 4.1 / 6.1, 8.2 / 9.0, 4.7 / 8.1 | 10.1 / 17.0, 30.0 / 30.6, 10.1 / 24.1
+      40,000: 4.6 / 5.5, 7.3 / 7.5, 5.8 / 7.0 | 5.9 / 7.4, 9.9 / 11.5, 6.9 / 9.7 | 14.5 / 19.7, 29.0 / 38.1, 14.2 / 27.7
+      50,000: 6.6 / 7.8, 10.4 / 10.7, 8.5 / 10.0 | 8.2 / 10.0, 14.4 / 15.7, 9.8 / 13.1 | 18.8 / 24.6, 40.2 / 50.0, 19.1 / 34.4
+      65,000: 10.8 / 11.2, 17.1 / 15.2, 13.5 / 14.4 | 13.1 / 13.9, 23.2 / 21.9, 15.4 / 18.5 | 28.2 / 31.3, 61.3 / 67.4, 27.7 / 46.1
     With self problems these kernels were faster in all of 160 settings from 26,000 to 60,000 rows (60,000 x 64, 10
     steps: 18.5 / 20.0, 45,000: 10.7 / 12.7), and so they are on schedules (60,000 x 64: 20.6 / 26.3).
 
@@ -309,9 +315,11 @@ def solver_problem(x, y, a, b, allow_tf32: bool, fixed: bool, stops: bool,
 
 def alternating_problem(x, y, a, b, allow_tf32: bool) -> bool:
     """Whether ``sinkhorn_flashstyle_alternating`` may hand its clouds and weights to ``solve``: a
-    half-update is one launch of the small kernels, faster than the streaming kernels' two and
-    what PyTorch does around them up to 1.4e8 logits (12,000 x 12,000 x 16: 44 against 48 us a
-    half-update; 6,206 x 5,067 x 37: 25 against 35), 6.5e7 on 33 .. 64 columns, 3.6e7 on more."""
+    half-update is one launch of the small kernels, the streaming kernels' two.  Up to 1.4e8 logits, 6.5e7 on 33 .. 64
+    columns, 3.6e7 on more; 40 iterations here / there, us a half-update: 8,000 x 3 16 / 23, 24 columns 21 / 26, 9,000 x 16
+    33 / 30, 11,000 x 32 48 / 42, 12,000 x 16 42 / 39; 6,206 x 5,067 x 37 18 / 26, 8,000 x 40 27 / 33, x 60 33 / 35, 9,000 x 40
+    50 / 47; 5,000 x 80 26 / 39, 6,000 x 80 35 / 42, x 128 40 / 44.  (The last third of the range on up to 32 columns has been the
+    streaming kernels' since what stands in front of their loop is one launch: 10 % of a solve there.)"""
     n, m, d = x.shape[0], y.shape[0], x.shape[-1]
     return (solver_problem(x, y, a, b, allow_tf32, True, False, any_size=True)
             and n * m <= (140_000_000 if d <= 32 else 65_000_000 if d <= 64 else 36_000_000))

@@ -54,6 +54,10 @@ bool use_dense(const fs_small_problem* p) { return p->d > kSmallMaxD; }
 //   d = 64:  256 points 243 -> 196, 91 -> 94; 1,000: 370 -> 238, 131 -> 102; 2,048 (32 MiB): 553 -> 395, 187 -> 152;
 //            2,500 (49 MiB): 657 -> 712, 177 -> 201; with self problems 1,000 (16 MiB): 388 -> 306, 110 -> 101;
 //            1,500 (35 MiB): 477 -> 507, 137 -> 159
+//   d = 48 (planes of 48 columns): 1,000: 334 -> 244, 110 -> 94; 2,048: 504 -> 401, 153 -> 138
+//   d = 96 (planes of 96): 256: 282 -> 207, 103 -> 97; 1,000: 448 -> 248, 149 -> 104; 2,000: 725 -> 411, 226 -> 155; 3,000: 1,000 ->
+//            860, 310 -> 295; 4,000: 1,370 -> 1,345, 411 -> 411; with self problems 1,000: 461 -> 308, 154 -> 120; 2,000: 840 -> 750,
+//            248 -> 260; 2,500: 1,557 -> 1,092, 478 -> 370
 //   d = 128: 256: 320 -> 201, 110 -> 96; 1,000: 563 -> 246, 175 -> 104; 3,000 (70 MiB): 1,143 -> 849, 344 -> 290; 4,000
 //            (125 MiB): 1,639 -> 1,447, 413 -> 391 (d = 100: 401 -> 417); with self problems 2,500 (98 MiB): 1,957 -> 1,083
 //   d = 32, fixed eps: 512: 233 -> 200; 1,000 (8 MiB): 295 -> 236; 1,500 (18 MiB): 359 -> 345; its schedules 85 -> 86 and
