@@ -92,8 +92,9 @@ def _max_change(f, g, prev_f, prev_g) -> float:
 
 
 def _starts_plain(x, y, a, b) -> bool:
-    """Whether a solve may start from ``_row_start``, which neither gradients nor tangents pass through."""
-    return (x.shape[0] > 0 and y.shape[0] > 0 and _lib.ordinary(x, y, a, b)
+    """Whether a solve may start from ``_row_start``, which neither gradients nor tangents pass through and which sees no
+    shapes (weights of another one are refused by the launchers)."""
+    return (x.shape[0] > 0 and y.shape[0] > 0 and a.ndim == 1 and b.ndim == 1 and _lib.ordinary(x, y, a, b)
             and not (torch.is_grad_enabled() and any(t.requires_grad for t in (x, y, a, b))))
 
 

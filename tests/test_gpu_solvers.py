@@ -1472,6 +1472,18 @@ def test_largest_change(n, m):
     assert _largest_change(p, q[1:], p, q[1:]) == 0.0 if m > 1 else True
 
 
+# weights with a column of their own: refused by the launchers, whoever forms their logarithms
+@pytest.mark.parametrize("of_x", [True, False])
+def test_weights_of_two_dimensions_are_refused(of_x):
+    from flash_sinkhorn_amd.kernels import sinkhorn_flashstyle_alternating, sinkhorn_flashstyle_symmetric
+    X, Y, A, B = dev(*inputs(4, 33, 20, 6))
+    A, B = (A[:, None], B) if of_x else (A, B[:, None])
+    with pytest.raises(ValueError, match="1D"):
+        sinkhorn_flashstyle_alternating(X, Y, A, B, eps=0.1, n_iters=2, ott_convention=True)
+    with pytest.raises(ValueError, match="1D"):
+        sinkhorn_flashstyle_symmetric(X, Y, A, B, use_epsilon_scaling=False, eps=0.1, n_iters=2, fused=False)
+
+
 # Tangents (forward-mode differentiation) go through the tensor operations around the kernels: of a potential or a c-transform
 # there is that of cost_scale |x|^2, whatever the sizes.
 def test_tangents_of_squared_norms():
